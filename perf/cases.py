@@ -15,6 +15,7 @@ recurrent state) that earlier steps would have left are random and
 depend on the seed alone.
 """
 
+import gc
 import json
 import math
 import os
@@ -496,6 +497,9 @@ def prepare(case, seed):
     runner, sched = llm.runner, llm.scheduler
     runner.model.load_weights(weights.checkpoint())
     if not case["prompts"]:
+        # a graph must not be destroyed while another one is captured:
+        # engines that are no longer used go first
+        gc.collect()
         runner.graph_runner = GraphRunner(runner)
         runner.graph_runner.capture_all()
     greedy = SamplingParams(temperature=0.0, ignore_eos=True,
