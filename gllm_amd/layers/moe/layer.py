@@ -33,7 +33,8 @@ class FusedMoE(nn.Module):
         act_limit), u = clamp(up, +-act_limit), act = g * sigmoid(
         act_alpha g) * (u + 1).
         ``fp32_routing_weights``: keep the routing weights in fp32 up to
-        the weighted sum instead of rounding them to the model dtype."""
+        the weighted sum in the segment loop too, instead of rounding them
+        to the model dtype (the grouped GEMMs always take them in fp32)."""
         super().__init__()
         assert activation in ("silu_glu", "relu2", "swiglu_clamp")
         self.activation = activation
@@ -125,8 +126,6 @@ class FusedMoE(nn.Module):
         from gllm_amd.parallel import get_dp_size
         if self.use_ep and get_dp_size() > 1:
             return self._forward_dp(x, weights, ids)
-        if not self.fp32_routing_weights:
-            weights = weights.to(x.dtype)
         out = self._expert_loop(x, weights, ids)
         if self.use_ep:
             from gllm_amd.parallel.state import ep_all_reduce
@@ -208,6 +207,8 @@ class FusedMoE(nn.Module):
                 return ops.fused_moe_int4(
                     x.contiguous(), w13c, w13sb, w2c, w2sb, weights, ids,
                     expert_start=self.expert_start)
+        if not self.fp32_routing_weights:
+            weights = weights.to(x.dtype)
         T = x.shape[0]
         out = torch.zeros_like(x)
         acc = torch.zeros(x.shape, dtype=torch.float32, device=x.device) \

@@ -188,6 +188,21 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
 
 # --------------------------------------------------------------- moe
 def topk_softmax(gating: torch.Tensor, topk: int, renormalize: bool = True):
+    """MoE routing: softmax over all experts, then the top k (weights
+    fp32 [T, k] in descending order, ids int32 [T, k]). Logits of up to
+    512 experts on the GPU take one wave-per-row kernel (ties go to the
+    lower index)."""
+    if (gating.is_cuda and gating.dim() == 2 and gating.shape[1] <= 512
+            and 0 < topk <= min(64, gating.shape[1])
+            and gating.dtype in (torch.float32, torch.bfloat16,
+                                 torch.float16) and has_moe_kernels()):
+        gating = gating.contiguous()
+        weights = torch.empty(gating.shape[0], topk, dtype=torch.float32,
+                              device=gating.device)
+        ids = torch.empty(gating.shape[0], topk, dtype=torch.int32,
+                          device=gating.device)
+        _gpu_kernels().softmax_topk_rows(weights, ids, gating, renormalize)
+        return weights, ids
     return torch_ref.topk_softmax(gating, topk, renormalize)
 
 
@@ -230,59 +245,74 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     alpha): min(g, limit) * sigmoid(alpha g) * (clamp(u) + 1)).
 
     Reference fused_experts_impl (fused_moe_triton/fused_moe.py:779):
-    align -> GEMM1 -> silu_and_mul -> GEMM2 (weighted scatter) -> sum.
+    align -> GEMM1 + activation -> GEMM2 (weighted scatter) -> sum.
     Fully device-resident and hipGraph-safe (no host syncs; grids are
     sized by upper bound and gated on the device-side block count).
     Returns the PARTIAL output for this rank's expert shard (callers
     run their TP/EP all-reduce on top).
     """
     T, K = x.shape
-    E_local, two_i, _ = w13.shape
+    E_local, rows13, _ = w13.shape
+    inter = w2.shape[2]
     topk = topk_ids.shape[1]
     n_pairs = T * topk
-    # tile heuristic: match block_m to the expected rows per expert so
-    # decode doesn't re-stream expert weights per m-block; large dense
-    # batches use the wide-BN prefill variant (gemm code 164 = BM 64 x
-    # BN 256 — quarters the A-tile re-reads that dominate prefill)
-    rpe = n_pairs / max(1, E_local)
-    if n_pairs >= 4096:
-        align_m, gemm_m = 64, 164
-    elif rpe < 12:
-        align_m = gemm_m = 16
-    elif rpe < 40:
-        align_m = gemm_m = 32
-    else:
-        align_m = gemm_m = 64
-    cap = n_pairs + E_local * (align_m - 1) + 1
-    max_blocks = (n_pairs + align_m - 1) // align_m + E_local
     dev = x.device
     k = _gpu_kernels()
-    ids32 = topk_ids.int().contiguous()
-    sorted_ids = torch.empty(cap, dtype=torch.int32, device=dev)
-    expert_blocks = torch.empty(max_blocks, dtype=torch.int32, device=dev)
-    n_post = torch.empty(1, dtype=torch.int32, device=dev)
-    k.moe_align(ids32, E_local, expert_start, align_m, sorted_ids,
-                expert_blocks, n_post)
-    rows_pad = cap - 1 + align_m  # >= n_post_pad upper bound
-    inter1 = torch.empty(rows_pad, two_i, dtype=x.dtype, device=dev)
-    k.moe_gemm(inter1, x, w13, sorted_ids, expert_blocks, n_post, None,
-               n_pairs, topk, gemm_m, False)
-    if activation == "relu2":
-        act = relu2(inter1)
-    elif activation == "swiglu_clamp":
-        act = clamp_swiglu(inter1, *act_args)
+    tw = topk_weights.float().contiguous()
+    pair_out = torch.empty(n_pairs, K, dtype=x.dtype, device=dev)
+    rpe = n_pairs / max(1, E_local)
+    if K % 64 == 0 and inter % 64 == 0:
+        # row block by the rows per expert: while an expert's weights are
+        # the cost, one block holds the rows of all but the most popular
+        # experts (csrc/moe_tiled.hip has times on both sides of each line)
+        block_m = (32 if rpe <= 12 else 64 if rpe <= 40
+                   else 128 if rpe <= 128 else 256)
+        ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
+                                          block_m)
+        act = torch.empty(rows, inter, dtype=x.dtype, device=dev)
+        code = {"silu_glu": 1, "swiglu_clamp": 2, "relu2": 3}[activation]
+        limit, alpha = act_args if activation == "swiglu_clamp" \
+            else (0.0, 0.0)
+        k.moe_gemm_tiled(act, x, w13, *tables, None, n_pairs, topk, block_m,
+                         code, limit, alpha)
+        k.moe_gemm_tiled(pair_out, act, w2, *tables, tw, n_pairs, topk,
+                         block_m, 0, 0.0, 0.0)
     else:
-        act = silu_and_mul(inter1)
-    # zero-filled: pairs routed to non-local experts (EP shards) or to
-    # the DP padding id -1 are dropped by the align kernel and must
-    # contribute zeros
-    pair_out = x.new_zeros(n_pairs, K)
-    k.moe_gemm(pair_out, act, w2, sorted_ids, expert_blocks, n_post,
-               topk_weights.float().contiguous(), n_pairs, topk, gemm_m,
-               True)
+        block_m = 16 if rpe < 12 else 32 if rpe < 40 else 64
+        ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
+                                          block_m)
+        inter1 = torch.empty(rows, rows13, dtype=x.dtype, device=dev)
+        k.moe_gemm(inter1, x, w13, *tables, None, n_pairs, topk, block_m,
+                   False)
+        if activation == "relu2":
+            act = relu2(inter1)
+        elif activation == "swiglu_clamp":
+            act = clamp_swiglu(inter1, *act_args)
+        else:
+            act = silu_and_mul(inter1)
+        k.moe_gemm(pair_out, act, w2, *tables, tw, n_pairs, topk, block_m,
+                   True)
     out = torch.empty(T, K, dtype=x.dtype, device=dev)
-    k.moe_sum(out, pair_out, topk)
+    k.moe_sum(out, pair_out, ids32, expert_start, E_local, topk)
     return out
+
+
+def _moe_tables(topk_ids: torch.Tensor, E_local: int, expert_start: int,
+                block_m: int):
+    """Sort the (token, expert) pairs by expert in blocks of ``block_m``
+    rows: (int32 ids, (sorted_ids, expert_blocks, n_post), rows of a
+    sorted buffer). Pairs of other ranks' experts, or of id -1, are in
+    no block."""
+    n_pairs = topk_ids.numel()
+    dev = topk_ids.device
+    cap = n_pairs + E_local * (block_m - 1) + 1
+    max_blocks = (n_pairs + block_m - 1) // block_m + E_local
+    ids32 = topk_ids.int().contiguous()
+    tables = (torch.empty(cap, dtype=torch.int32, device=dev),
+              torch.empty(max_blocks, dtype=torch.int32, device=dev),
+              torch.empty(1, dtype=torch.int32, device=dev))
+    _gpu_kernels().moe_align(ids32, E_local, expert_start, block_m, *tables)
+    return ids32, tables, cap - 1 + block_m
 
 
 # --------------------------------------------------------------- fp8
@@ -422,33 +452,24 @@ def fused_moe_fp8(x: torch.Tensor, w13: torch.Tensor, w13_scale,
         align_m = gemm_m = 32
     else:
         align_m = gemm_m = 64
-    cap = n_pairs + E_local * (align_m - 1) + 1
-    max_blocks = (n_pairs + align_m - 1) // align_m + E_local
     dev = x.device
     k = _gpu_kernels()
-    ids32 = topk_ids.int().contiguous()
-    sorted_ids = torch.empty(cap, dtype=torch.int32, device=dev)
-    expert_blocks = torch.empty(max_blocks, dtype=torch.int32, device=dev)
-    n_post = torch.empty(1, dtype=torch.int32, device=dev)
-    k.moe_align(ids32, E_local, expert_start, align_m, sorted_ids,
-                expert_blocks, n_post)
-    rows_pad = cap - 1 + align_m
+    ids32, tables, rows_pad = _moe_tables(topk_ids, E_local, expert_start,
+                                          align_m)
     aq, as_ = per_token_group_quant_fp8(x.contiguous())
     inter1 = torch.empty(rows_pad, two_i, dtype=x.dtype, device=dev)
     k.moe_gemm_fp8(inter1, aq.view(torch.uint8), as_,
                    w13.view(torch.uint8), w13_scale.contiguous(),
-                   sorted_ids, expert_blocks, n_post, None, n_pairs, topk,
-                   gemm_m, False)
+                   *tables, None, n_pairs, topk, gemm_m, False)
     act = silu_and_mul(inter1)
     actq, act_s = per_token_group_quant_fp8(act)
-    pair_out = x.new_zeros(n_pairs, K)
+    pair_out = torch.empty(n_pairs, K, dtype=x.dtype, device=dev)
     k.moe_gemm_fp8(pair_out, actq.view(torch.uint8), act_s,
-                   w2.view(torch.uint8), w2_scale.contiguous(),
-                   sorted_ids, expert_blocks, n_post,
+                   w2.view(torch.uint8), w2_scale.contiguous(), *tables,
                    topk_weights.float().contiguous(), n_pairs, topk,
                    gemm_m, True)
     out = torch.empty(T, K, dtype=x.dtype, device=dev)
-    k.moe_sum(out, pair_out, topk)
+    k.moe_sum(out, pair_out, ids32, expert_start, E_local, topk)
     return out
 
 
@@ -558,29 +579,20 @@ def fused_moe_int4(x: torch.Tensor, w13_c, w13_sb, w2_c, w2_sb,
     n_pairs = T * topk
     rpe = n_pairs / max(1, E_local)
     block_m = 16 if rpe < 12 else (32 if rpe < 40 else 64)
-    cap = n_pairs + E_local * (block_m - 1) + 1
-    max_blocks = (n_pairs + block_m - 1) // block_m + E_local
     dev = x.device
     k = _gpu_kernels()
-    ids32 = topk_ids.int().contiguous()
-    sorted_ids = torch.empty(cap, dtype=torch.int32, device=dev)
-    expert_blocks = torch.empty(max_blocks, dtype=torch.int32, device=dev)
-    n_post = torch.empty(1, dtype=torch.int32, device=dev)
-    k.moe_align(ids32, E_local, expert_start, block_m, sorted_ids,
-                expert_blocks, n_post)
-    rows_pad = cap - 1 + block_m
+    ids32, tables, rows_pad = _moe_tables(topk_ids, E_local, expert_start,
+                                          block_m)
     inter1 = torch.empty(rows_pad, two_i, dtype=x.dtype, device=dev)
-    k.moe_gemm_int4(inter1, x.contiguous(), w13_c, w13_sb, sorted_ids,
-                    expert_blocks, n_post, None, n_pairs, topk, block_m,
-                    False)
+    k.moe_gemm_int4(inter1, x.contiguous(), w13_c, w13_sb, *tables, None,
+                    n_pairs, topk, block_m, False)
     act = silu_and_mul(inter1)
-    pair_out = x.new_zeros(n_pairs, K)
-    k.moe_gemm_int4(pair_out, act, w2_c, w2_sb, sorted_ids,
-                    expert_blocks, n_post,
+    pair_out = torch.empty(n_pairs, K, dtype=x.dtype, device=dev)
+    k.moe_gemm_int4(pair_out, act, w2_c, w2_sb, *tables,
                     topk_weights.float().contiguous(), n_pairs, topk,
                     block_m, True)
     out = torch.empty(T, K, dtype=x.dtype, device=dev)
-    k.moe_sum(out, pair_out, topk)
+    k.moe_sum(out, pair_out, ids32, expert_start, E_local, topk)
     return out
 
 

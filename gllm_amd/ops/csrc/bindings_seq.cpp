@@ -184,7 +184,16 @@ void moe_gemm(torch::Tensor C, torch::Tensor A, torch::Tensor W,
               torch::Tensor n_post_pad,
               c10::optional<torch::Tensor> topk_weights, long n_pairs,
               long topk, long block_m, bool scatter);
-void moe_sum(torch::Tensor out, torch::Tensor pair_out, long topk);
+void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
+                    torch::Tensor sorted_ids, torch::Tensor expert_blocks,
+                    torch::Tensor n_post_pad,
+                    c10::optional<torch::Tensor> topk_weights, long n_pairs,
+                    long topk, long block_m, long act, double limit,
+                    double alpha);
+void moe_sum(torch::Tensor out, torch::Tensor pair_out, torch::Tensor ids,
+             long expert_start, long E_local, long topk);
+void softmax_topk_rows(torch::Tensor weights, torch::Tensor ids,
+                       torch::Tensor logits, bool renorm);
 void topk_softmax_rows(torch::Tensor weights, torch::Tensor ids,
                        torch::Tensor logits);
 
@@ -263,6 +272,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d]) * x[d:]");
   m.def("moe_align", &moe_align, "device-side moe_align_block_size");
   m.def("moe_gemm", &moe_gemm, "grouped MFMA GEMM over sorted pairs");
+  m.def("moe_gemm_tiled", &moe_gemm_tiled,
+        "grouped MFMA GEMM of wide tiles, activation in the epilogue");
+  m.def("softmax_topk_rows", &softmax_topk_rows,
+        "softmax over all experts, then top-k");
   m.def("moe_sum", &moe_sum, "sum pair outputs over topk");
   m.def("topk_softmax_rows", &topk_softmax_rows,
         "top-k of router logits, softmax over the chosen");
