@@ -8,21 +8,33 @@
 // of that row (zero-copy view — each KV byte is read exactly once for
 // ALL heads, and the PV B-fragments read straight out of the K tile).
 //
-// MI355X-native design: a (token, head) pair is a GEMM row — q flattens
-// to [T*H, 576] rows tiled 64 per workgroup; the causal mask depends
-// only on the row's token, so one kernel serves decode (1 token x 128
-// heads = 2 row tiles), chunked prefill, prefix hits and mixed batches.
-// Decode split-KVs over blockIdx.z with an fp32 LSE merge.
+// MI355X-native design: a (token, head) pair is a GEMM row; the causal mask
+// depends only on the row's token, so one kernel serves decode, chunked
+// prefill, prefix hits and mixed batches. Decode splits the keys over
+// blockIdx.z with an fp32 LSE merge.
 //
-// v2 execution structure (v1 ran 1 wave/SIMD and was latency-bound at
-// ~300 GB/s KV): 512 threads = 8 waves at 2 waves/SIMD. Wave w owns
-// row group w%4 (16 rows) and V half w/4 (256 dims) — the o
-// accumulator halves to 64 VGPRs so two waves co-reside per SIMD; the
-// QK^T S-tile is computed twice per row group (MFMA is not the bound).
-// K tiles stream through a 3-slot LDS ring via global_load_lds issued
-// by waves 0-3 with counted s_waitcnt vmcnt BEFORE the barrier (the
-// proven skinny-GEMM pipeline): consumers see landed tiles at barrier
-// release without ever waiting a vm counter of their own.
+// A workgroup of four waves takes R row tiles of 16 and walks tiles of 64
+// keys. A key tile sits in LDS once, as nine column blocks of [64 keys][128
+// B] whose 16 B units are permuted by key & 7 (the layout both reads below
+// want), in a ring of two filled by global_load_lds while the other tile is
+// worked on (147 KB: one workgroup per CU). Scores are K Q^T and the output
+// is O^T = V^T P^T, so a lane holds keys, then dims, of ONE row; V is read
+// transposed out of the key tile (ds_read_tr16_b64).
+//  * R = 1 (decode, up to 16 heads): wave w scores keys 16 w .. + 15, the
+//    row maxima and the weights pass through LDS, then wave w owns dims
+//    128 w .. + 127 of the output. Every key byte is read from LDS once for
+//    the scores and once for the output.
+//  * R = 4 (prompts, more heads): wave w scores row tile w against all 64
+//    keys; the output is split by dims as above, so V is read once for 64
+//    rows instead of once per row tile.
+// R = 1 is bound by memory, R = 4 by LDS reads (K 295 KB + V 64 KB + P 32 KB
+// a tile against 2176 cycles of products). The kernel before this one read V
+// element by element (eight 2 B reads a fragment) and chose the splits by
+// the batch's lengths, which a captured launch does not have: one split.
+// 128 requests of 16 heads at 512 to 1536 keys (151 MB): 52 + 6 us, 282 us
+// before. Prompts of 4096 tokens in four, 16 heads: 257 us (535 us).
+// 512 workgroups as the aim of the splits: twice the CUs, so that requests
+// of unequal lengths even out.
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -33,25 +45,39 @@ typedef __attribute__((ext_vector_type(4))) float mfma_f4;
 
 namespace {
 
-constexpr int BLOCK = 512;    // 8 waves
-constexpr int BQ = 64;        // flattened (token, head) rows per workgroup
-constexpr int BKV = 32;       // kv tokens per ring slot
-constexpr int RING = 3;
+typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
+
+constexpr int BLOCK = 256;    // 4 waves
+constexpr int BKV = 64;       // keys of a tile
 constexpr int DK = 576;       // latent dims (kv_lora 512 + rope 64)
 constexpr int DV = 512;
-constexpr int KT = DK / 32;   // QK^T k-steps (18)
-constexpr int NTW = 16;       // PV 16-wide n tiles per wave (256 dims)
-constexpr int NF = BKV / 16;  // score fragments per wave (2)
-constexpr int ROW_B = DK * 2; // K row bytes (1152)
-constexpr int TILE_B = BKV * ROW_B;          // 36864
-constexpr int GL_PER_WAVE = TILE_B / 1024 / 4;  // 9 (waves 0-3 stage)
-constexpr int PT_STRIDE = BKV + 8;
+constexpr int KT = DK / 32;   // score k-steps (18)
+constexpr int NT = DV / 4 / 16;  // 16-dim output tiles of a wave (8)
+constexpr int ROW_B = DK * 2;
+constexpr int CB = ROW_B / 128;  // column blocks (9)
+constexpr int CB_B = BKV * 128;
+constexpr int TILE_B = CB * CB_B;
+constexpr int P_ROW = BKV * 2 + 16;  // bytes of a weight row
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr int SPLIT_TARGET = 512;  // workgroups that a decode batch aims at
 
-DEV_INLINE int kswz(int row, int byte_off) {
-  return byte_off ^ ((row & 7) << 4);
+union MlaFrag {
+  mfma_bf8 v;
+  shortx4 h[2];
+};
+
+DEV_INLINE short bf16_bits(float v) {
+  return __builtin_bit_cast(short, __float2bfloat16(v));
 }
 
-template <bool SPLIT>
+// LDS writes of all waves are visible; loads to LDS stay in flight
+DEV_INLINE void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int R, bool SPLIT>
 __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     __hip_bfloat16 *__restrict__ out,      // [T, H, DV] (SPLIT: unused)
     float *__restrict__ partial_out,       // [S, TH, DV] (SPLIT only)
@@ -63,240 +89,249 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     const int *__restrict__ qsl,           // [B+1]
     int max_pages, int page_size, int H, float scale, int num_splits,
     long th_total) {
-  const int tile = blockIdx.x;
+  constexpr int BQ = R * 16;
+  constexpr int NF = R == 1 ? 1 : 4;  // score fragments of a wave
+  // the last row tiles see the most keys: they start first
+  const int tile = gridDim.x - 1 - blockIdx.x;
   const int b = blockIdx.y;
   const int split = blockIdx.z;
-
   const int q_start = qsl[b];
   const int q_len = qsl[b + 1] - q_start;
   const int rows = q_len * H;
-  const int tid = threadIdx.x;
   if (tile * BQ >= rows) return;
   const int seq_len = seq_lens[b];
   const int past = seq_len - q_len;
-
+  const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
   const int l16 = lane & 15;
   const int lhi = lane >> 4;
-  const int rg = wave & 3;        // row group (16 rows)
-  const int vhalf = wave >> 2;    // V half (256 dims)
 
-  // causal kv bound for this row tile, then the split's share of it
+  // causal bound of this row tile, then the split's share of it
   const int last_tok = min(rows - 1, (tile + 1) * BQ - 1) / H;
   const int kv_hi_all = min(seq_len, past + last_tok + 1);
   const int split_len =
       ((kv_hi_all + BKV - 1) / BKV + num_splits - 1) / num_splits * BKV;
   const int kv_lo = split * split_len;
   const int kv_hi = min(kv_lo + split_len, kv_hi_all);
-
-  const long row_base = (long)q_start * H + (long)tile * BQ;
-
-  if (kv_lo >= kv_hi) {
-    if (SPLIT) {
-      for (int r = tid; r < BQ; r += BLOCK) {
-        if (tile * BQ + r < rows)
-          partial_lse[(long)split * th_total + row_base + r] = -INFINITY;
-      }
-    }
+  const long row0 = (long)q_start * H + (long)tile * BQ;
+  const int rows_here = min(BQ, rows - tile * BQ);
+  if (kv_lo >= kv_hi) {  // an empty split: the merge skips it
+    if (SPLIT && tid < rows_here)
+      partial_lse[(long)split * th_total + row0 + tid] = -INFINITY;
     return;
   }
 
-  __shared__ __attribute__((aligned(16))) char k_ring[RING * TILE_B];
-  __shared__ __hip_bfloat16 p_tile[8][16 * PT_STRIDE];
+  __shared__ __attribute__((aligned(16))) char ring[2 * TILE_B];
+  __shared__ __attribute__((aligned(16))) char p_tile[BQ * P_ROW];
+  __shared__ float s_a[4][16], s_b[4][16], s_m[4][16];
 
-  // ---- Q fragments (A-operand): row = rg*16 + l16 ----
-  const int frow = tile * BQ + rg * 16 + l16;
-  const bool row_valid = frow < rows;
-  mfma_bf8 qfrag[KT];
+  // query fragments: column l16 = row, dims kt * 32 + lhi * 8
+  const int my_tile = R == 1 ? 0 : wave;
+  const int my_row = my_tile * 16 + l16;
+  mfma_bf8 qf[KT];
   {
     const __hip_bfloat16 *qp =
-        q + ((long)q_start * H + frow) * DK + lhi * 8;
+        q + (row0 + min(my_row, rows_here - 1)) * DK + lhi * 8;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      if (row_valid)
-        qfrag[kt] = *reinterpret_cast<const mfma_bf8 *>(qp + kt * 32);
-      else
-        qfrag[kt] = mfma_bf8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
+    for (int kt = 0; kt < KT; ++kt)
+      qf[kt] = *reinterpret_cast<const mfma_bf8 *>(qp + kt * 32);
   }
+  // keys this lane's row sees: below vis (none for a row past the end)
+  const int vis = my_row < rows_here
+                      ? min(seq_len, past + (tile * BQ + my_row) / H + 1)
+                      : 0;
+  const float qscale = scale * LOG2E;
 
-  float m_run[4], l_run[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) { m_run[r] = -INFINITY; l_run[r] = 0.f; }
-  mfma_f4 o_acc[NTW];
-#pragma unroll
-  for (int nt = 0; nt < NTW; ++nt) o_acc[nt] = mfma_f4{0, 0, 0, 0};
-
+  // ---- staging: wave w brings keys 16 w .. + 15 as 2 x 9 units of
+  // [8 keys][128 B]; rows of the next tile are looked up a tile ahead
   const int *bt = block_table + (long)b * max_pages;
-
-  // ---- glds staging (waves 0-3): 9 chunks of 1 KiB per wave ----
-  auto stage = [&](int kt_idx, int slot) {
-    const int kv0 = kv_lo + kt_idx * BKV;
-    char *base = k_ring + slot * TILE_B;
+  const int s_key = wave * 16 + (lane >> 3);
+  const int s_col = ((lane & 7) ^ (lane >> 3)) * 16;
+  int page[2];
+  auto key_of = [&](int k0, int g) {
+    return min(k0 + s_key + g * 8, seq_len - 1);
+  };
+  auto look_up = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < GL_PER_WAVE; ++j) {
-      const int p = (wave * GL_PER_WAVE + j) * 1024 + lane * 16;
-      const int row = p / ROW_B;
-      const int col = kswz(row, p % ROW_B);
-      const int tok = kv0 + row;
-      // clamp to a valid cache row; masked later by the score mask
-      const int ctok = min(tok, seq_len - 1);
-      const long crow =
-          (long)bt[ctok / page_size] * page_size + ctok % page_size;
-      // aux=2 (nt): each latent row is streamed once per split —
-      // non-temporal lands faster and leaves L2 to shared data
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const unsigned int *>(
-              reinterpret_cast<const char *>(kc) + crow * ROW_B + col),
-          reinterpret_cast<unsigned int *>(
-              base + (wave * GL_PER_WAVE + j) * 1024),
-          16, 0, 2);
-    }
+    for (int g = 0; g < 2; ++g) page[g] = bt[key_of(k0, g) / page_size];
+  };
+  auto stage = [&](int k0, int slot) {
+    const char *src[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      src[g] = reinterpret_cast<const char *>(kc) +
+               ((long)page[g] * page_size + key_of(k0, g) % page_size) *
+                   ROW_B + s_col;
+    char *dst = ring + slot * TILE_B + wave * 2048;
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const unsigned int *>(src[g] + c * 128),
+            reinterpret_cast<unsigned int *>(dst + c * CB_B + g * 1024), 16,
+            0, R == 1 ? 2 : 0);
   };
 
-  const int nkt = (kv_hi - kv_lo + BKV - 1) / BKV;
-  const int pre = min(RING - 1, nkt);
-  if (wave < 4)
-    for (int t = 0; t < pre; ++t) stage(t, t % RING);
+  float m_run = -INFINITY, l_run = 0.f;
+  mfma_f4 o[R][NT];
+#pragma unroll
+  for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) o[rt][nt] = mfma_f4{0, 0, 0, 0};
+  const int tr_row = lhi * 4 + (l16 >> 2), tr_col = (l16 & 3) * 8;
 
-  for (int kt_i = 0; kt_i < nkt; ++kt_i) {
-    const int kv0 = kv_lo + kt_i * BKV;
-    const int slot = kt_i % RING;
-    if (wave < 4) {
-      if (kt_i + RING - 1 < nkt)
-        stage(kt_i + RING - 1, (kt_i + RING - 1) % RING);
-      const int ahead = min(nkt - 1 - kt_i, RING - 1);
-      if (ahead >= 2) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * GL_PER_WAVE)
-                     : "memory");
-      } else if (ahead == 1) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(1 * GL_PER_WAVE)
-                     : "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
+  look_up(kv_lo);
+  stage(kv_lo, 0);
+  if (kv_lo + BKV < kv_hi) look_up(kv_lo + BKV);
+  int slot = 0;
+  for (int k0 = kv_lo; k0 < kv_hi; k0 += BKV, slot ^= 1) {
+    // the tile is there; the other slot and P are free
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (k0 + BKV < kv_hi) {
+      stage(k0 + BKV, slot ^ 1);
+      if (k0 + 2 * BKV < kv_hi) look_up(k0 + 2 * BKV);
     }
-    __syncthreads();  // stagers waited first -> tile kt_i is landed
+    const char *kt_base = ring + slot * TILE_B;
 
-    const char *ktile = k_ring + slot * TILE_B;
-
-    // ---------- QK^T: S[16 rows x 32 tokens] ----------
-    mfma_f4 s_frag[NF];
+    // ---- scores: fragment f = keys (R == 1 ? wave : f) * 16 + lhi * 4 + r
+    mfma_f4 s[NF][2];
 #pragma unroll
-    for (int f = 0; f < NF; ++f) s_frag[f] = mfma_f4{0, 0, 0, 0};
-    __builtin_amdgcn_s_setprio(1);
+    for (int f = 0; f < NF; ++f)
+      s[f][0] = s[f][1] = mfma_f4{0, 0, 0, 0};
+    const int krow = (R == 1 ? wave * 16 : 0) + l16;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        const int krow = f * 16 + l16;
-        mfma_bf8 bfrag = *reinterpret_cast<const mfma_bf8 *>(
-            ktile + krow * ROW_B + kswz(krow, (kt * 32 + lhi * 8) * 2));
-        s_frag[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            qfrag[kt], bfrag, s_frag[f], 0, 0, 0);
+        const mfma_bf8 kf = *reinterpret_cast<const mfma_bf8 *>(
+            kt_base + (kt >> 1) * CB_B + (krow + f * 16) * 128 +
+            (((kt & 1) * 64 + lhi * 16) ^ ((krow & 7) << 4)));
+        // (one fragment: two chains)
+        s[f][NF == 1 ? kt & 1 : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            kf, qf[kt], s[f][NF == 1 ? kt & 1 : 0], 0, 0, 0);
       }
-    }
-    __builtin_amdgcn_s_setprio(0);
-
-    // ---------- mask + online softmax (rows lhi*4+r) ----------
-    float p_vals[NF][4];
-    float alpha[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = tile * BQ + rg * 16 + lhi * 4 + r;
-      const int qpos = past + rr / H;
-      float sv[NF];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        const int kvp = kv0 + f * 16 + l16;
-        float s = s_frag[f][r] * scale;
-        if (rr >= rows || kvp > qpos || kvp >= seq_len) s = -INFINITY;
-        sv[f] = s;
-        mx = fmaxf(mx, s);
-      }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      const float m_new = fmaxf(m_run[r], mx);
-      float psum = 0.f;
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        const float p = (sv[f] == -INFINITY || m_new == -INFINITY)
-                            ? 0.f : __expf(sv[f] - m_new);
-        p_vals[f][r] = p;
-        psum += p;
-      }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        psum += __shfl_xor(psum, off, 64);
-      alpha[r] = (m_run[r] == -INFINITY || m_new == -INFINITY)
-                     ? 0.f : __expf(m_run[r] - m_new);
-      l_run[r] = l_run[r] * alpha[r] + psum;
-      m_run[r] = m_new;
-    }
-#pragma unroll
-    for (int nt = 0; nt < NTW; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o_acc[nt][r] *= alpha[r];
-
-    // ---------- P -> LDS bounce -> A fragment ----------
-    __hip_bfloat16 *pw = p_tile[wave];
+    float mx = -INFINITY;
+    float sv[NF][4];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        pw[(lhi * 4 + r) * PT_STRIDE + f * 16 + l16] =
-            __float2bfloat16(p_vals[f][r]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    mfma_bf8 pfrag = *reinterpret_cast<const mfma_bf8 *>(
-        &pw[l16 * PT_STRIDE + lhi * 8]);
-
-    // ---------- PV: o += P[16x32] x V[32 x 256-half] ----------
-    // B-fragments gather from the K tile (V = first 512 dims of the
-    // row): lane l reads tokens lhi*8+j at dim vhalf*256 + nt*16 + l16
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) {
-      const int dim = vhalf * 256 + nt * 16 + l16;
-      mfma_bf8 vfrag;
-      __hip_bfloat16 *ve = reinterpret_cast<__hip_bfloat16 *>(&vfrag);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int vrow = lhi * 8 + j;
-        ve[j] = *reinterpret_cast<const __hip_bfloat16 *>(
-            ktile + vrow * ROW_B + kswz(vrow, dim * 2));
+      for (int r = 0; r < 4; ++r) {
+        const int key = k0 + (R == 1 ? wave : f) * 16 + lhi * 4 + r;
+        const float x = (s[f][0][r] + s[f][1][r]) * qscale;
+        sv[f][r] = key < vis ? x : -INFINITY;
+        mx = fmaxf(mx, sv[f][r]);
       }
-      o_acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          pfrag, vfrag, o_acc[nt], 0, 0, 0);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (R == 1) {
+      if (lhi == 0) s_a[wave][l16] = mx;
+      lds_barrier();
+#pragma unroll
+      for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_a[w][l16]);
     }
-    __builtin_amdgcn_s_setprio(0);
-    __syncthreads();  // everyone done with this ring slot
+    // (a row may see nothing yet: a finite maximum keeps its weights at 0)
+    const float m_new = fmaxf(fmaxf(m_run, mx), -1e30f);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      shortx4 p;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(sv[f][r] - m_new);
+        sum += e;
+        p[r] = bf16_bits(e);
+      }
+      *reinterpret_cast<shortx4 *>(
+          p_tile + my_row * P_ROW +
+          ((R == 1 ? wave : f) * 16 + lhi * 4) * 2) = p;
+    }
+    l_run = l_run * alpha + sum;  // this lane's keys
+    if (R > 1 && lhi == 0) s_a[wave][l16] = alpha;
+    lds_barrier();
+
+    // ---- output dims wave * 128 + nt * 16 .. of every row tile
+    float al[R];
+#pragma unroll
+    for (int rt = 0; rt < R; ++rt) al[rt] = R == 1 ? alpha : s_a[rt][l16];
+#pragma unroll
+    for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[rt][nt][r] *= al[rt];
+#pragma unroll
+    for (int kk = 0; kk < BKV / 32; ++kk) {
+      MlaFrag pf[R];
+#pragma unroll
+      for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+          pf[rt].h[half] = *reinterpret_cast<const shortx4 *>(
+              p_tile + (rt * 16 + l16) * P_ROW +
+              (kk * 32 + half * 16 + lhi * 4) * 2);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        MlaFrag vf;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const int row = kk * 32 + half * 16 + tr_row;
+          vf.h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_shortx4 *)(kt_base + (wave * 2 + (nt >> 2)) * CB_B +
+                              row * 128 +
+                              (((nt & 3) * 32 + tr_col) ^
+                               ((row & 7) << 4))));
+        }
+#pragma unroll
+        for (int rt = 0; rt < R; ++rt)
+          o[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              vf.v, pf[rt].v, o[rt][nt], 0, 0, 0);
+      }
+    }
   }
 
-  // ---------- epilogue ----------
+  // ---- join the sums, write (lane: row l16, four neighbouring dims)
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (lhi == 0) {
+    s_b[wave][l16] = l_run;
+    s_m[wave][l16] = m_run;
+  }
+  __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int rr = tile * BQ + rg * 16 + lhi * 4 + r;
-    if (rr >= rows) continue;
-    const float l = l_run[r];
-    const float inv_l = (l > 0.f) ? 1.f / l : 0.f;
-    const long orow = row_base - tile * BQ + rr;
+  for (int rt = 0; rt < R; ++rt) {
+    const int row = rt * 16 + l16;
+    if (row >= rows_here) continue;
+    const float l = R == 1 ? s_b[0][l16] + s_b[1][l16] + s_b[2][l16] +
+                                 s_b[3][l16]
+                           : s_b[rt][l16];
+    const float m = s_m[rt][l16];
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const long at = row0 + row;
     if (SPLIT) {
-      float *op = partial_out +
-          ((long)split * th_total + orow) * DV + vhalf * 256;
+      float *op = partial_out + ((long)split * th_total + at) * DV +
+                  wave * 128 + lhi * 4;
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt)
-        op[nt * 16 + l16] = o_acc[nt][r] * inv_l;
-      if (l16 == 0 && vhalf == 0)
-        partial_lse[(long)split * th_total + orow] =
-            (l > 0.f) ? m_run[r] + __logf(l) : -INFINITY;
+      for (int nt = 0; nt < NT; ++nt)
+        *reinterpret_cast<floatx4 *>(op + nt * 16) =
+            floatx4{o[rt][nt][0] * inv, o[rt][nt][1] * inv,
+                    o[rt][nt][2] * inv, o[rt][nt][3] * inv};
+      if (wave == 0 && lhi == 0)
+        partial_lse[(long)split * th_total + at] =
+            l > 0.f ? m / LOG2E + __logf(l) : -INFINITY;
     } else {
-      __hip_bfloat16 *op = out + orow * DV + vhalf * 256;
+      __hip_bfloat16 *op = out + at * DV + wave * 128 + lhi * 4;
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt)
-        op[nt * 16 + l16] = __float2bfloat16(o_acc[nt][r] * inv_l);
+      for (int nt = 0; nt < NT; ++nt) {
+        shortx4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = bf16_bits(o[rt][nt][r] * inv);
+        *reinterpret_cast<shortx4 *>(op + nt * 16) = v;
+      }
     }
   }
 }
@@ -361,50 +396,59 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
   if (T == 0) return;
   const int H = q.size(1);
   const int B = seq_lens.size(0);
+  TORCH_CHECK(block_table.stride(1) == 1 && block_table.size(0) >= B &&
+              query_start_loc.scalar_type() == at::kInt &&
+              query_start_loc.numel() == B + 1);
+  TORCH_CHECK(k_cache.is_contiguous() &&
+              reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0);
+  const int R = max_query_len * H <= 16 ? 1 : 4;
+  const int BQ = R * 16;
   const int tiles = (int)((max_query_len * H + BQ - 1) / BQ);
   const long th_total = T * H;
   auto stream = at::cuda::getCurrentCUDAStream();
 
-  // split-KV only for pure-decode batches (uniform kv ranges)
+  // split-KV only for pure-decode batches (uniform kv ranges). The count
+  // depends on the batch size and the pool only: a captured launch serves
+  // every length, an empty split costs a few hundred cycles.
   int splits = 1;
   if (max_query_len == 1) {
-    const long kv_tiles = (max_seq_len + BKV - 1) / BKV;
-    while (splits < 16 && (long)B * tiles * splits < 640 &&
-           splits * 2 <= kv_tiles)
+    const long max_len = (long)k_cache.size(0) * k_cache.size(1);
+    while (splits < 32 && (long)B * tiles * splits < SPLIT_TARGET &&
+           splits * 2 <= (max_len + BKV - 1) / BKV)
       splits *= 2;
   }
-
+  torch::Tensor partial, lse;
+  float *po = nullptr, *pl = nullptr;
+  if (splits > 1) {
+    auto opts = q.options().dtype(at::kFloat);
+    partial = torch::empty({splits, th_total, (long)DV}, opts);
+    lse = torch::empty({splits, th_total}, opts);
+    po = partial.data_ptr<float>();
+    pl = lse.data_ptr<float>();
+  }
+#define RUN(RT, SPLIT)                                                       \
+  hipLaunchKernelGGL((mla_attention_kernel<RT, SPLIT>),                      \
+                     dim3(tiles, B, splits), dim3(BLOCK), 0, stream,         \
+                     (__hip_bfloat16 *)out.data_ptr(), po, pl,               \
+                     (const __hip_bfloat16 *)q.data_ptr(),                   \
+                     (const __hip_bfloat16 *)k_cache.data_ptr(),             \
+                     block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),  \
+                     query_start_loc.data_ptr<int>(),                        \
+                     (int)block_table.stride(0), (int)k_cache.size(1), H,    \
+                     (float)scale, splits, th_total)
   if (splits == 1) {
-    hipLaunchKernelGGL((mla_attention_kernel<false>), dim3(tiles, B, 1),
-                       dim3(BLOCK), 0, stream,
-                       (__hip_bfloat16 *)out.data_ptr(), nullptr, nullptr,
-                       (const __hip_bfloat16 *)q.data_ptr(),
-                       (const __hip_bfloat16 *)k_cache.data_ptr(),
-                       block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
-                       query_start_loc.data_ptr<int>(),
-                       (int)block_table.size(1), (int)k_cache.size(1), H,
-                       (float)scale, 1, th_total);
+    if (R == 1) RUN(1, false); else RUN(4, false);
     HIP_CHECK_KERNEL();
     return;
   }
-  auto opts = q.options().dtype(at::kFloat);
-  auto partial = torch::empty({splits, th_total, (long)DV}, opts);
-  auto lse = torch::empty({splits, th_total}, opts);
-  hipLaunchKernelGGL((mla_attention_kernel<true>), dim3(tiles, B, splits),
-                     dim3(BLOCK), 0, stream, nullptr,
-                     partial.data_ptr<float>(), lse.data_ptr<float>(),
-                     (const __hip_bfloat16 *)q.data_ptr(),
-                     (const __hip_bfloat16 *)k_cache.data_ptr(),
-                     block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
-                     query_start_loc.data_ptr<int>(),
-                     (int)block_table.size(1), (int)k_cache.size(1), H,
-                     (float)scale, splits, th_total);
+  if (R == 1) RUN(1, true); else RUN(4, true);
+#undef RUN
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((mla_merge_kernel), dim3((unsigned)th_total),
                      dim3(256), 0, stream,
-                     (__hip_bfloat16 *)out.data_ptr(),
-                     partial.data_ptr<float>(), lse.data_ptr<float>(),
-                     splits, th_total);
+                     (__hip_bfloat16 *)out.data_ptr(), po, pl, splits,
+                     th_total);
   HIP_CHECK_KERNEL();
 }
 

@@ -1,0 +1,84 @@
+"""Latent attention against fp64 at the edges of its row and key tiles."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(q_lens, ctx, H, page=16, seed=0):
+    torch.manual_seed(seed)
+    lens = [c + n for c, n in zip(ctx, q_lens)]
+    need = [-(-n // page) for n in lens]
+    pages = torch.randperm(sum(need) + 3)
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n].int()
+        at += n
+    cache = torch.randn(sum(need) + 3, page, 1, 576).bfloat16()
+    q = torch.randn(sum(q_lens), H, 576).bfloat16()
+    qsl = torch.tensor([0] + q_lens).cumsum(0).int()
+    return q, cache, table, torch.tensor(lens).int(), qsl
+
+
+def _ref(q, cache, table, lens, qsl, scale):
+    out = torch.empty(q.shape[0], q.shape[1], 512, dtype=torch.float64)
+    for i, n in enumerate(lens.tolist()):
+        a, b = int(qsl[i]), int(qsl[i + 1])
+        k = cache[table[i].long()].reshape(-1, 576)[:n].double()
+        s = q[a:b].double() @ k.t() * scale           # [n, H, keys]
+        pos = torch.arange(n - (b - a), n)
+        hide = torch.arange(n)[None] > pos[:, None]
+        s = s.masked_fill(hide[:, None], -float("inf"))
+        out[a:b] = s.softmax(-1) @ k[:, :512]
+    return out
+
+
+@pytest.mark.parametrize("q_lens,ctx,H,page", [
+    ([1], [0], 16, 16),                    # one key
+    ([1, 1, 1], [63, 64, 65], 16, 16),     # edges of a key tile
+    ([1] * 5, [127, 1000, 1, 300, 64], 5, 16),
+    ([1, 1], [200, 2000], 17, 16),         # more rows than one tile
+    ([1, 1], [70, 500], 128, 16),
+    ([1] * 600, [40] * 600, 16, 16),       # no split
+    ([70, 1, 3], [0, 130, 64], 16, 16),    # portions beside a decode
+    ([33], [100], 5, 48),                  # page size not a power of two
+    ([64, 65], [0, 0], 16, 1),
+])
+def test_mla_attention_tiles(q_lens, ctx, H, page):
+    from gllm_amd import ops
+    args = _case(q_lens, ctx, H, page)
+    scale = 192 ** -0.5
+    ref = _ref(*args, scale)
+    q, cache, table, lens, qsl = (t.cuda() for t in args)
+    out = ops.mla_paged_attention(q, cache, cache[..., :512], table, lens,
+                                  qsl, scale)
+    # weights and the result are rounded to bf16 (2^-9 each)
+    err = (out.cpu().double() - ref).norm() / ref.norm()
+    assert err < 3 * 2 ** -9, err
+
+
+def test_mla_decode_captured_serves_longer_batches():
+    """The split count does not depend on the lengths seen at capture."""
+    from gllm_amd import ops
+    scale = 192 ** -0.5
+    q, cache, table, lens, qsl = (
+        t.cuda() for t in _case([1] * 4, [5, 900, 64, 300], 16))
+    short = torch.ones_like(lens)
+    run = lambda: ops.mla_paged_attention(  # noqa: E731
+        q, cache, cache[..., :512], table, buf, qsl, scale,
+        seq_lens_cpu=[1] * 4, query_start_loc_cpu=[0, 1, 2, 3, 4])
+    buf = short.clone()
+    run()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = run()
+    for want in (lens, short, lens):
+        buf.copy_(want)
+        eager = ops.mla_paged_attention(q, cache, cache[..., :512], table,
+                                        want, qsl, scale)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
