@@ -127,10 +127,24 @@ class MLAAttention(nn.Module):
         else:
             q_resid = None
             q = self.q_proj(hidden)
+        kv_a = self.kv_a_proj_with_mqa(hidden)
+        if self.absorbed and not fctx.is_profile_run:
+            cos_sin = self.rotary_emb.cos_sin_cache
+            k_cache = fctx.k_caches[self.layer_idx]
+            w_kvb, norm = self.kv_b_proj.weight, self.kv_a_layernorm
+            if (self.rotary_emb.is_neox and cos_sin.device == q.device
+                    and self.kv_lora_rank == 512
+                    and ops.mla_absorbed_ok(q, kv_a, w_kvb, norm.weight,
+                                            k_cache, cos_sin, self.qk_nope,
+                                            self.v_dim)):
+                qf = ops.mla_queries(q, kv_a, norm.weight, norm.eps,
+                                     positions, cos_sin, w_kvb, k_cache,
+                                     fctx.slot_mapping)
+                out_lat = self._attend(qf, positions, hidden, q_resid, fctx)
+                return self.o_proj(ops.mla_values(out_lat, w_kvb))
         q = q.view(T, H, self.qk_dim)
         q_nope, q_pe = q.split([self.qk_nope, self.qk_rope], dim=-1)
 
-        kv_a = self.kv_a_proj_with_mqa(hidden)
         c_kv, k_pe = kv_a.split([self.kv_lora_rank, self.qk_rope], dim=-1)
         c_kv = self.kv_a_layernorm(c_kv.contiguous())
 
@@ -165,6 +179,17 @@ class MLAAttention(nn.Module):
             query_start_loc_cpu=fctx.host_qsl())
         return self.o_proj(out.reshape(T, -1))
 
+    def _attend(self, qf, positions, hidden, q_resid, fctx):
+        """Latent attention of the query rows [T, H, lora + rope] over
+        this layer's cache (v = view of its first lora dims)."""
+        topk_pos = self._dsa_select(positions, hidden, q_resid, fctx)
+        return ops.mla_paged_attention(
+            qf, fctx.k_caches[self.layer_idx], fctx.v_caches[self.layer_idx],
+            fctx.block_table, fctx.seq_lens, fctx.query_start_loc,
+            self.scale, topk_positions=topk_pos,
+            seq_lens_cpu=fctx.host_seq_lens(),
+            query_start_loc_cpu=fctx.host_qsl())
+
     def _forward_absorbed(self, positions, hidden, q_resid, q_nope, q_pe,
                           c_kv, k_pe, fctx):
         T, H = q_nope.shape[0], self.num_heads
@@ -178,16 +203,10 @@ class MLAAttention(nn.Module):
         qf = torch.cat([q_lat, q_pe], dim=-1).contiguous()  # [T,H,l+r]
         k_lat = torch.cat([c_kv, k_pe], dim=-1).unsqueeze(1)  # [T,1,l+r]
         k_cache = fctx.k_caches[self.layer_idx]   # [P,page,1,lora+rope]
-        v_cache = fctx.v_caches[self.layer_idx]   # VIEW: [..., :lora]
         # write the latent row once (the v view aliases its first lora
         # dims, so caching k fills both)
         ops.cache_latent(k_lat.contiguous(), k_cache, fctx.slot_mapping)
-        topk_pos = self._dsa_select(positions, hidden, q_resid, fctx)
-        out_lat = ops.mla_paged_attention(
-            qf, k_cache, v_cache, fctx.block_table, fctx.seq_lens,
-            fctx.query_start_loc, self.scale, topk_positions=topk_pos,
-            seq_lens_cpu=fctx.host_seq_lens(),
-            query_start_loc_cpu=fctx.host_qsl())
+        out_lat = self._attend(qf, positions, hidden, q_resid, fctx)
         # out[t,h,v] = sum_l out_lat[t,h,l] * W_UV[h,v,l]
         out = torch.einsum("thl,hvl->thv", out_lat.float(),
                            w_uv.float()).to(out_lat.dtype)

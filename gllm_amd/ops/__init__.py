@@ -640,6 +640,40 @@ def cache_latent(k, k_cache, slot_mapping):
     k_cache[pages, offs] = k.to(k_cache.dtype)
 
 
+def mla_absorbed_ok(q: torch.Tensor, kv: torch.Tensor, w_kvb: torch.Tensor,
+                    norm_w: torch.Tensor, k_cache: torch.Tensor,
+                    cos_sin: torch.Tensor, nope: int, vdim: int) -> bool:
+    """Whether ``mla_queries`` / ``mla_values`` take this layer: bf16 on
+    the GPU with the latent 512 + 64, 128 unrotated query and 128 value
+    dims a head (the sizes of every released checkpoint)."""
+    return (q.is_cuda and q.dtype == torch.bfloat16
+            and kv.dtype == torch.bfloat16 and w_kvb.dtype == torch.bfloat16
+            and k_cache.dtype == torch.bfloat16 and k_cache.is_contiguous()
+            and kv.shape[1] == 576 and k_cache.shape[-1] == 576
+            and w_kvb.dim() == 2 and w_kvb.shape[1] == 512
+            and w_kvb.is_contiguous() and nope == 128 and vdim == 128
+            and norm_w.dtype in (torch.bfloat16, torch.float32)
+            and cos_sin.dtype == torch.float32 and cos_sin.shape[-1] == 64
+            and q.stride(1) == 1 and q.stride(0) % 8 == 0
+            and kv.stride(1) == 1 and kv.stride(0) % 8 == 0
+            and all(t.data_ptr() % 16 == 0
+                    for t in (q, kv, w_kvb, norm_w, k_cache)))
+
+
+def mla_queries(q, kv, norm_w, eps, positions, cos_sin, w_kvb, k_cache,
+                slot_mapping):
+    """Norm and rotate the latent rows ``kv`` [T, 576] into their cache
+    slots; return the absorbed query rows [T, H, 576] of ``q`` [T, H *
+    192] (rotate-half on the last 64 dims of a head)."""
+    return _gpu_kernels().mla_queries(q, kv, norm_w, eps, positions, cos_sin,
+                                      w_kvb, k_cache, slot_mapping)
+
+
+def mla_values(o_lat, w_kvb):
+    """Per-head values [T, H * 128] of the weighted latents [T, H, 512]."""
+    return _gpu_kernels().mla_values(o_lat, w_kvb)
+
+
 _MLA_GPU_WARNED = False
 
 
@@ -658,17 +692,15 @@ def mla_paged_attention(q, k_cache, v_cache, block_table, seq_lens,
             and q.shape[-1] == 576 and v_cache.shape[-1] == 512
             and q.dtype == torch.bfloat16):
         qsl_h = query_start_loc_cpu or query_start_loc.tolist()
-        lens_h = seq_lens_cpu or seq_lens.tolist()
-        max_q = max((qsl_h[i + 1] - qsl_h[i] for i in range(len(lens_h))),
-                    default=1)
-        max_s = max(lens_h, default=1)
+        max_q = max((qsl_h[i + 1] - qsl_h[i]
+                     for i in range(len(qsl_h) - 1)), default=1)
         T, H = q.shape[0], q.shape[1]
         out = torch.empty(T, H, 512, dtype=q.dtype, device=q.device)
         qsl_i = query_start_loc.int() \
             if query_start_loc.dtype != torch.int32 else query_start_loc
         _gpu_kernels().mla_paged_attention(
             out, q.contiguous(), k_cache, block_table, seq_lens, qsl_i,
-            max_q, scale, max_s)
+            max_q, scale)
         return out
     if q.is_cuda and not _MLA_GPU_WARNED:
         from gllm_amd.logger import logger

@@ -383,7 +383,7 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
                          torch::Tensor k_cache, torch::Tensor block_table,
                          torch::Tensor seq_lens,
                          torch::Tensor query_start_loc, long max_query_len,
-                         double scale, long max_seq_len) {
+                         double scale) {
   TORCH_CHECK(q.scalar_type() == at::kBFloat16, "mla attn: bf16 only");
   TORCH_CHECK(q.is_contiguous() && out.is_contiguous());
   TORCH_CHECK(q.size(2) == DK, "mla attn: latent dim must be ", DK);

@@ -51,7 +51,13 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
                          torch::Tensor k_cache, torch::Tensor block_table,
                          torch::Tensor seq_lens,
                          torch::Tensor query_start_loc, long max_query_len,
-                         double scale, long max_seq_len);
+                         double scale);
+torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
+                          torch::Tensor norm_w, double eps,
+                          torch::Tensor positions, torch::Tensor cos_sin,
+                          torch::Tensor w_kvb, torch::Tensor k_cache,
+                          torch::Tensor slots);
+torch::Tensor mla_values(torch::Tensor o_lat, torch::Tensor w_kvb);
 void cache_latent(torch::Tensor k, torch::Tensor k_cache,
                   torch::Tensor slot_mapping);
 void moe_align(torch::Tensor topk_ids, long E_local, long expert_start,
@@ -144,6 +150,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "decode-regime weight-streaming GEMM (M<=256)");
   m.def("mla_paged_attention", &mla_paged_attention,
         "absorbed-MLA varlen attention over the 576-dim latent cache");
+  m.def("mla_queries", &mla_queries,
+        "latent cache rows and absorbed, rotated query rows");
+  m.def("mla_values", &mla_values, "per-head values of the weighted latent");
   m.def("cache_latent", &cache_latent,
         "scatter the per-token latent row into the paged cache");
   m.def("moe_align", &moe_align,

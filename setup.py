@@ -39,7 +39,8 @@ SEQ_SOURCES = ["bindings_seq.cpp", "layernorm.hip", "hyper.hip",
                "skinny_gemm.hip"]
 CORE_SOURCES = ["bindings.cpp", "norm.hip", "elementwise.hip",
                 "attention_decode.hip", "attention_prefill.hip",
-                "attention_mla.hip", "moe.hip", "moe_tiled.hip", "fp8.hip",
+                "attention_mla.hip", "mla_proj.hip", "moe.hip",
+                "moe_tiled.hip", "fp8.hip",
                 "gdn.hip", "int4.hip", "skinny_gemm.hip", "sampling.hip",
                 "custom_ar.hip"]
 

@@ -82,3 +82,53 @@ def test_mla_decode_captured_serves_longer_batches():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("T,H,strided,wdtype", [
+    (1, 16, False, torch.bfloat16), (64, 3, True, torch.float32),
+    (65, 16, False, torch.float32), (130, 128, True, torch.bfloat16)])
+def test_mla_queries_and_values(T, H, strided, wdtype):
+    """Latent rows, absorbed queries and per-head values against fp64."""
+    from gllm_amd import ops
+    torch.manual_seed(T)
+    wide = 8 if strided else 0        # rows of a wider projection
+    q = torch.randn(T, H * 192 + wide, device="cuda").bfloat16()[
+        :, :H * 192]
+    kv = torch.randn(T, 576 + wide, device="cuda").bfloat16()[:, :576]
+    norm = (1 + 0.1 * torch.randn(512, device="cuda")).to(wdtype)
+    w = (torch.randn(H * 256, 512, device="cuda") * 512 ** -0.5).bfloat16()
+    pos = torch.randint(0, 4096, (T,), device="cuda")
+    ang = torch.arange(4096).double()[:, None] * 10000.0 ** (
+        -torch.arange(0, 64, 2).double() / 64)
+    cs = torch.cat([ang.cos(), ang.sin()], -1).float().cuda()
+    cache = torch.zeros(T // 16 + 2, 16, 1, 576, device="cuda").bfloat16()
+    slots = torch.randperm(cache.shape[0] * 16, device="cuda")[:T]
+    assert ops.mla_absorbed_ok(q, kv, w, norm, cache, cs, 128, 128)
+    qf = ops.mla_queries(q, kv, norm, 1e-6, pos, cs, w, cache, slots)
+
+    def turn(x):
+        c, s = cs[pos].double().chunk(2, -1)
+        if x.dim() == 3:
+            c, s = c[:, None], s[:, None]
+        a, b = x.chunk(2, -1)
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+    q64, kv64 = q.double().view(T, H, 192), kv.double()
+    wv = w.double().view(H, 256, 512)
+    lat = torch.matmul(q64[..., :128].transpose(0, 1).contiguous(),
+                       wv[:, :128].contiguous()).transpose(0, 1)
+    want = torch.cat([lat, turn(q64[..., 128:])], -1)
+    c = kv64[:, :512]
+    c = c * (c.square().mean(-1, keepdim=True) + 1e-6).rsqrt() * norm.double()
+    row = torch.cat([c, turn(kv64[:, 512:])], -1)
+    got = cache.view(-1, 576)[slots].double()
+    values = ops.mla_values(qf[..., :512].contiguous(), w)
+    vref = torch.matmul(
+        qf[..., :512].double().transpose(0, 1).contiguous(),
+        wv[:, 128:].transpose(1, 2).contiguous()).transpose(0, 1)
+    # one bf16 rounding of the result each
+    for a, b in ((qf.double(), want), (got, row),
+                 (values.double().view(T, H, 128), vref)):
+        assert (a - b).norm() / b.norm() < 2 ** -8
+    untouched = torch.ones(cache.shape[0] * 16, dtype=torch.bool)
+    untouched[slots.cpu()] = False
+    assert not cache.view(-1, 576)[untouched.cuda()].any()
