@@ -38,13 +38,21 @@ class Attention(nn.Module):
             # (reference layers/attention.py:112-116): skip attention math,
             # return a same-shape tensor.
             return q.reshape(T, -1)
-        k_cache = fctx.k_caches[self.layer_idx]
-        v_cache = fctx.v_caches[self.layer_idx]
-        ops.reshape_and_cache(k, v, k_cache, v_cache, fctx.slot_mapping)
+        ops.reshape_and_cache(k, v, fctx.k_caches[self.layer_idx],
+                              fctx.v_caches[self.layer_idx],
+                              fctx.slot_mapping)
+        return self.attend(q, fctx)
+
+    def attend(self, q: torch.Tensor, fctx: ForwardContext) -> torch.Tensor:
+        """Attention of the (rotated) queries over the cache, which holds
+        this batch's keys and values already."""
+        T = q.shape[0]
+        if q.dim() == 2:
+            q = q.unflatten(-1, (self.num_heads, self.head_dim))
         out = ops.paged_attention(
-            q, k_cache, v_cache, fctx.block_table, fctx.seq_lens,
-            fctx.query_start_loc, self.scale,
-            max_query_len=fctx.max_query_len,
+            q, fctx.k_caches[self.layer_idx], fctx.v_caches[self.layer_idx],
+            fctx.block_table, fctx.seq_lens, fctx.query_start_loc,
+            self.scale, max_query_len=fctx.max_query_len,
             sliding_window=self.sliding_window)
         return out.reshape(T, -1)
 

@@ -14,6 +14,10 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(hidden_size))
         self.eps = eps
 
+    def scale(self) -> torch.Tensor:
+        """What the normed row is multiplied by."""
+        return self.weight
+
     def forward(self, x: torch.Tensor,
                 residual: Optional[torch.Tensor] = None):
         if residual is not None:
@@ -33,7 +37,7 @@ class GemmaRMSNorm(nn.Module):
         self.eps = eps
         self._w1 = None
 
-    def _scale(self):
+    def scale(self) -> torch.Tensor:
         if self._w1 is None or self._w1.device != self.weight.device:
             self._w1 = (self.weight + 1.0).contiguous()
         return self._w1
@@ -41,9 +45,9 @@ class GemmaRMSNorm(nn.Module):
     def forward(self, x: torch.Tensor,
                 residual: Optional[torch.Tensor] = None):
         if residual is not None:
-            return ops.fused_add_rmsnorm(x, residual, self._scale(),
+            return ops.fused_add_rmsnorm(x, residual, self.scale(),
                                          self.eps)
-        return ops.rmsnorm(x, self._scale(), self.eps)
+        return ops.rmsnorm(x, self.scale(), self.eps)
 
 
 class LayerNorm(nn.Module):

@@ -108,6 +108,11 @@ class LinearBase(nn.Module):
             w = self._w_dq
         return ops.linear(x, w, bias)
 
+    @property
+    def is_plain(self) -> bool:
+        """Unquantized weights (the fused few-row forms take them)."""
+        return self.fp8_block is None and self.int4_cfg is None
+
     def _bias32(self):
         """fp32 bias cached once (the skinny epilogues add fp32)."""
         if self.bias is None:
@@ -226,6 +231,13 @@ class MergedColumnParallelLinear(LinearBase):
     def forward(self, x):
         return self._gemm(x, self.bias)
 
+    def forward_silu(self, x):
+        """silu(gate) * up of a gate | up projection."""
+        if self.is_plain and self.bias is None and x.is_cuda \
+                and x.dim() == 2:
+            return ops.linear_silu(x, self.weight)
+        return ops.silu_and_mul(self(x))
+
 
 class PackedLinear(LinearBase):
     """Several projections of one input as one GEMM, each block of output
@@ -297,9 +309,13 @@ class QKVParallelLinear(LinearBase):
         param.data.narrow(0, offset, size).copy_(
             loaded.narrow(0, src_rank * size, size))
 
+    def project(self, x):
+        """The merged q | k | v rows."""
+        return self._gemm(x, self.bias)
+
     def forward(self, x):
-        out = self._gemm(x, self.bias)
-        return out.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
+        return self.project(x).split(
+            [self.q_size, self.kv_size, self.kv_size], dim=-1)
 
 
 class RowParallelLinear(LinearBase):
@@ -323,6 +339,16 @@ class RowParallelLinear(LinearBase):
     @staticmethod
     def _load_b(param, loaded):
         param.data.copy_(loaded)
+
+    def forward_add_norm(self, x, residual, norm):
+        """(norm(residual + self(x)), that sum): one kernel behind the
+        product where nothing has to be reduced over ranks first."""
+        if (self.is_plain and self.bias is None and x.is_cuda
+                and x.dim() == 2
+                and (get_tp_size() == 1 or not self.reduce_results)):
+            return ops.linear_add_rmsnorm(x, self.weight, residual,
+                                          norm.scale(), norm.eps)
+        return norm(self(x), residual)
 
     def forward(self, x):
         out = self._gemm(x)

@@ -119,6 +119,15 @@ class MLAAttention(nn.Module):
         return w[:, :self.qk_nope, :], w[:, self.qk_nope:, :]
 
     def forward(self, positions, hidden, fctx: ForwardContext):
+        return self.o_proj(self.heads(positions, hidden, fctx))
+
+    def forward_add_norm(self, positions, hidden, residual, norm, fctx):
+        """(norm(residual + self(...)), that sum)."""
+        return self.o_proj.forward_add_norm(
+            self.heads(positions, hidden, fctx), residual, norm)
+
+    def heads(self, positions, hidden, fctx: ForwardContext):
+        """The heads' outputs [T, heads * v_dim], before o_proj."""
         T = hidden.shape[0]
         H = self.num_heads
         if self.q_lora_rank:
@@ -141,7 +150,7 @@ class MLAAttention(nn.Module):
                                      positions, cos_sin, w_kvb, k_cache,
                                      fctx.slot_mapping)
                 out_lat = self._attend(qf, positions, hidden, q_resid, fctx)
-                return self.o_proj(ops.mla_values(out_lat, w_kvb))
+                return ops.mla_values(out_lat, w_kvb)
         q = q.view(T, H, self.qk_dim)
         q_nope, q_pe = q.split([self.qk_nope, self.qk_rope], dim=-1)
 
@@ -177,7 +186,7 @@ class MLAAttention(nn.Module):
             fctx.query_start_loc, self.scale, topk_positions=topk_pos,
             seq_lens_cpu=fctx.host_seq_lens(),
             query_start_loc_cpu=fctx.host_qsl())
-        return self.o_proj(out.reshape(T, -1))
+        return out.reshape(T, -1)
 
     def _attend(self, qf, positions, hidden, q_resid, fctx):
         """Latent attention of the query rows [T, H, lora + rope] over
@@ -210,7 +219,7 @@ class MLAAttention(nn.Module):
         # out[t,h,v] = sum_l out_lat[t,h,l] * W_UV[h,v,l]
         out = torch.einsum("thl,hvl->thv", out_lat.float(),
                            w_uv.float()).to(out_lat.dtype)
-        return self.o_proj(out.reshape(T, -1))
+        return out.reshape(T, -1)
 
 
 class DeepseekMoE(nn.Module):
@@ -257,7 +266,8 @@ class DeepseekMoE(nn.Module):
         else:
             w, ids = ops.topk_softmax(logits, self.top_k,
                                       renormalize=self.norm_topk)
-        return w * self.routed_scaling, ids
+        return (w if self.routed_scaling == 1.0
+                else w * self.routed_scaling), ids
 
     def forward(self, x):
         logits = self.gate(x)
@@ -289,16 +299,22 @@ class DeepseekDecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(cfg.hidden_size, eps)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
-    def forward(self, positions, hidden, residual, fctx):
+    def forward(self, positions, hidden, residual, fctx, normed=False,
+                next_norm=None):
+        """``normed`` / ``next_norm``: see llama_family's
+        DenseDecoderLayer."""
         if residual is None:
             residual = hidden
             hidden = self.input_layernorm(hidden)
-        else:
+        elif not normed:
             hidden, residual = self.input_layernorm(hidden, residual)
-        hidden = self.self_attn(positions, hidden, fctx)
-        hidden, residual = self.post_attention_layernorm(hidden, residual)
-        hidden = self.mlp(hidden)
-        return hidden, residual
+        hidden, residual = self.self_attn.forward_add_norm(
+            positions, hidden, residual, self.post_attention_layernorm, fctx)
+        if next_norm is None:
+            return self.mlp(hidden), residual
+        if isinstance(self.mlp, DenseMLP):
+            return self.mlp.forward_add_norm(hidden, residual, next_norm)
+        return next_norm(self.mlp(hidden), residual)
 
 
 class DeepseekV2ForCausalLM(nn.Module):
@@ -359,11 +375,20 @@ class DeepseekV2ForCausalLM(nn.Module):
                     0, fctx.mm_rows,
                     fctx.mm_embeds.to(hidden_states.dtype))
             residual = None
-        for layer in self.layers:
+        normed = False
+        for li, layer in enumerate(self.layers):
+            nxt = None      # the norm behind this layer
+            if li + 1 < len(self.layers):
+                nxt = self.layers[li + 1].input_layernorm
+            elif self.is_last_stage:
+                nxt = self.norm
             hidden_states, residual = layer(positions, hidden_states,
-                                            residual, fctx)
+                                            residual, fctx, normed=normed,
+                                            next_norm=nxt)
+            normed = nxt is not None
         if self.is_last_stage:
-            hidden_states, _ = self.norm(hidden_states, residual)
+            if not normed:
+                hidden_states, _ = self.norm(hidden_states, residual)
             return hidden_states, None
         return hidden_states, residual
 

@@ -127,8 +127,15 @@ class GatedDeltaNet(nn.Module):
             off += size
 
     def forward(self, hidden: torch.Tensor, fctx: ForwardContext):
+        heads = self.heads(hidden, fctx)
+        return torch.zeros_like(hidden) if heads is None \
+            else self.out_proj(heads)
+
+    def heads(self, hidden: torch.Tensor, fctx: ForwardContext):
+        """The gated heads [T, value_dim] before out_proj; None in a
+        profile run (no state to work on)."""
         if fctx.is_profile_run or fctx.ssm_pool is None:
-            return torch.zeros_like(hidden)
+            return None
         T = hidden.shape[0]
         k_tp = self.tp_k_heads * self.head_k_dim
         v_tp = self.tp_v * self.head_v_dim
@@ -184,7 +191,7 @@ class GatedDeltaNet(nn.Module):
                 o.reshape(T * self.tp_v, self.head_v_dim),
                 z.reshape(T * self.tp_v, self.head_v_dim).contiguous(),
                 self.norm_weight, self.eps)
-            return self.out_proj(gated.reshape(T, -1))
+            return gated.reshape(T, -1)
 
         qsl = fctx.host_qsl()
         # ---- GPU mixed/prefill path: conv stays per segment (cheap),
@@ -257,7 +264,7 @@ class GatedDeltaNet(nn.Module):
             out_core.reshape(T * self.tp_v, self.head_v_dim),
             z.reshape(T * self.tp_v, self.head_v_dim),
             self.norm_weight, self.eps)
-        return self.out_proj(gated.reshape(T, -1))
+        return gated.reshape(T, -1)
 
 
 class HybridFullAttention(nn.Module):
@@ -301,6 +308,10 @@ class HybridFullAttention(nn.Module):
                               self.head_dim ** -0.5)
 
     def forward(self, positions, hidden, fctx):
+        return self.o_proj(self.heads(positions, hidden, fctx))
+
+    def heads(self, positions, hidden, fctx):
+        """The heads' outputs [T, heads * head_dim], before o_proj."""
         qg, k, v = self.qkv_proj(hidden)
         T = hidden.shape[0]
         if self.gate:
@@ -319,7 +330,7 @@ class HybridFullAttention(nn.Module):
         o = self.attn(q, k, v, fctx)
         if gate is not None:
             o = o * torch.sigmoid(gate.float()).to(o.dtype)
-        return self.o_proj(o)
+        return o
 
 
 class HybridDecoderLayer(nn.Module):
@@ -339,19 +350,31 @@ class HybridDecoderLayer(nn.Module):
         self.input_layernorm = GemmaRMSNorm(cfg.hidden_size, eps)
         self.post_attention_layernorm = GemmaRMSNorm(cfg.hidden_size, eps)
 
-    def forward(self, positions, hidden, residual, fctx):
+    def forward(self, positions, hidden, residual, fctx, normed=False,
+                next_norm=None):
+        """``normed`` / ``next_norm``: see llama_family's
+        DenseDecoderLayer."""
         if residual is None:
             residual = hidden
             hidden = self.input_layernorm(hidden)
-        else:
+        elif not normed:
             hidden, residual = self.input_layernorm(hidden, residual)
         if self.layer_type == "linear_attention":
-            hidden = self.linear_attn(hidden, fctx)
+            heads, proj = (self.linear_attn.heads(hidden, fctx),
+                           self.linear_attn.out_proj)
         else:
-            hidden = self.self_attn(positions, hidden, fctx)
-        hidden, residual = self.post_attention_layernorm(hidden, residual)
-        hidden = self.mlp(hidden)
-        return hidden, residual
+            heads, proj = (self.self_attn.heads(positions, hidden, fctx),
+                           self.self_attn.o_proj)
+        norm = self.post_attention_layernorm
+        if heads is None:       # profile run: a mixer without its state
+            hidden, residual = norm(torch.zeros_like(hidden), residual)
+        else:
+            hidden, residual = proj.forward_add_norm(heads, residual, norm)
+        if next_norm is None:
+            return self.mlp(hidden), residual
+        if isinstance(self.mlp, DenseMLP):
+            return self.mlp.forward_add_norm(hidden, residual, next_norm)
+        return next_norm(self.mlp(hidden), residual)
 
 
 class Qwen3_5ForCausalLM(nn.Module):
@@ -458,9 +481,20 @@ class Qwen3_5ForCausalLM(nn.Module):
                     fctx.mm_embeds.to(hidden_states.dtype))
             residual = None
         ds = getattr(fctx, "mm_deepstack", None)
+        normed = False
         for li, layer in enumerate(self.layers):
+            # the norm behind this layer (deepstack adds to the layer's
+            # own output in between)
+            nxt = None
+            if ds is None:
+                if li + 1 < len(self.layers):
+                    nxt = self.layers[li + 1].input_layernorm
+                elif self.is_last_stage:
+                    nxt = self.norm
             hidden_states, residual = layer(positions, hidden_states,
-                                            residual, fctx)
+                                            residual, fctx, normed=normed,
+                                            next_norm=nxt)
+            normed = nxt is not None
             if ds is not None:
                 # deepstack level li ADDED at the image rows after
                 # decoder layer li (reference qwen3_5.py:795-812 —
@@ -472,7 +506,8 @@ class Qwen3_5ForCausalLM(nn.Module):
                         0, fctx.mm_rows,
                         ds[:, g * H:(g + 1) * H].to(hidden_states.dtype))
         if self.is_last_stage:
-            hidden_states, _ = self.norm(hidden_states, residual)
+            if not normed:
+                hidden_states, _ = self.norm(hidden_states, residual)
             return hidden_states, None
         return hidden_states, residual
 

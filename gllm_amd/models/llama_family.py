@@ -16,6 +16,7 @@ from typing import Iterable, List, Optional, Tuple
 import torch
 import torch.nn as nn
 
+from gllm_amd import ops
 from gllm_amd.layers.activation import SiluAndMul
 from gllm_amd.layers.attention import Attention
 from gllm_amd.layers.embedding import ParallelLMHead, VocabParallelEmbedding
@@ -37,7 +38,12 @@ class DenseMLP(nn.Module):
         self.act_fn = SiluAndMul()
 
     def forward(self, x):
-        return self.down_proj(self.act_fn(self.gate_up_proj(x)))
+        return self.down_proj(self.gate_up_proj.forward_silu(x))
+
+    def forward_add_norm(self, x, residual, norm):
+        """(norm(residual + self(x)), that sum)."""
+        return self.down_proj.forward_add_norm(
+            self.gate_up_proj.forward_silu(x), residual, norm)
 
 
 class DenseAttention(nn.Module):
@@ -75,7 +81,24 @@ class DenseAttention(nn.Module):
             self.head_dim, self.head_dim ** -0.5,
             sliding_window=self.sliding_window)
 
-    def forward(self, positions, hidden, fctx: ForwardContext):
+    def heads(self, positions, hidden, fctx: ForwardContext):
+        """The heads' outputs [T, heads * head_dim], before o_proj."""
+        if (not (self.qk_norm or fctx.is_profile_run) and hidden.is_cuda
+                and positions.dim() == 1):
+            attn, rope = self.attn, self.rotary_emb
+            k_cache = fctx.k_caches[attn.layer_idx]
+            v_cache = fctx.v_caches[attn.layer_idx]
+            if (hidden.dtype == torch.bfloat16 and ops.qkv_rope_cache_ok(
+                    k_cache, v_cache, rope.cos_sin_cache, rope.is_neox)):
+                proj, bias = self.qkv_proj, self.qkv_proj.bias
+                src = ops.qkv_parts(hidden, proj.weight, bias) \
+                    if proj.is_plain else None
+                if src is None:
+                    src, bias = proj.project(hidden), None
+                q = ops.qkv_rope_cache(src, bias, positions,
+                                       rope.cos_sin_cache, k_cache, v_cache,
+                                       fctx.slot_mapping, attn.num_heads)
+                return attn.attend(q, fctx)
         q, k, v = self.qkv_proj(hidden)
         if self.qk_norm:
             T = q.shape[0]
@@ -84,8 +107,15 @@ class DenseAttention(nn.Module):
             k = self.k_norm(
                 k.contiguous().view(T, -1, self.head_dim)).view(T, -1)
         q, k = self.rotary_emb(positions, q, k)
-        o = self.attn(q, k, v, fctx)
-        return self.o_proj(o)
+        return self.attn(q, k, v, fctx)
+
+    def forward(self, positions, hidden, fctx: ForwardContext):
+        return self.o_proj(self.heads(positions, hidden, fctx))
+
+    def forward_add_norm(self, positions, hidden, residual, norm, fctx):
+        """(norm(residual + self(...)), that sum)."""
+        return self.o_proj.forward_add_norm(
+            self.heads(positions, hidden, fctx), residual, norm)
 
 
 class DenseDecoderLayer(nn.Module):
@@ -100,16 +130,21 @@ class DenseDecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(cfg.hidden_size, eps)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
-    def forward(self, positions, hidden, residual, fctx):
+    def forward(self, positions, hidden, residual, fctx, normed=False,
+                next_norm=None):
+        """``normed``: hidden is this layer's normed input already (the
+        layer before was given this layer's input norm as ``next_norm``,
+        and normed its own output with it)."""
         if residual is None:
             residual = hidden
             hidden = self.input_layernorm(hidden)
-        else:
+        elif not normed:
             hidden, residual = self.input_layernorm(hidden, residual)
-        hidden = self.self_attn(positions, hidden, fctx)
-        hidden, residual = self.post_attention_layernorm(hidden, residual)
-        hidden = self.mlp(hidden)
-        return hidden, residual
+        hidden, residual = self.self_attn.forward_add_norm(
+            positions, hidden, residual, self.post_attention_layernorm, fctx)
+        if next_norm is not None:
+            return self.mlp.forward_add_norm(hidden, residual, next_norm)
+        return self.mlp(hidden), residual
 
 
 class LlamaFamilyForCausalLM(nn.Module):
@@ -175,9 +210,20 @@ class LlamaFamilyForCausalLM(nn.Module):
                     fctx.mm_embeds.to(hidden_states.dtype))
             residual = None
         ds = getattr(fctx, "mm_deepstack", None)
+        normed = False
         for li, layer in enumerate(self.layers):
+            # the norm behind this layer: the next layer's, or the final
+            # one (deepstack adds to the layer's own output in between)
+            nxt = None
+            if ds is None:
+                if li + 1 < len(self.layers):
+                    nxt = self.layers[li + 1].input_layernorm
+                elif self.is_last_stage:
+                    nxt = self.norm
             hidden_states, residual = layer(positions, hidden_states,
-                                            residual, fctx)
+                                            residual, fctx, normed=normed,
+                                            next_norm=nxt)
+            normed = nxt is not None
             if ds is not None:
                 # Qwen3-VL deepstack: level li of the multiscale vision
                 # features is ADDED at the image rows after decoder
@@ -189,7 +235,8 @@ class LlamaFamilyForCausalLM(nn.Module):
                         0, fctx.mm_rows,
                         ds[:, g * H:(g + 1) * H].to(hidden_states.dtype))
         if self.is_last_stage:
-            hidden_states, _ = self.norm(hidden_states, residual)
+            if not normed:
+                hidden_states, _ = self.norm(hidden_states, residual)
             return hidden_states, None
         return hidden_states, residual
 

@@ -68,16 +68,21 @@ class MoEDecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(cfg.hidden_size, eps)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
-    def forward(self, positions, hidden, residual, fctx):
+    def forward(self, positions, hidden, residual, fctx, normed=False,
+                next_norm=None):
+        """``normed`` / ``next_norm``: see DenseDecoderLayer."""
         if residual is None:
             residual = hidden
             hidden = self.input_layernorm(hidden)
-        else:
+        elif not normed:
             hidden, residual = self.input_layernorm(hidden, residual)
-        hidden = self.self_attn(positions, hidden, fctx)
-        hidden, residual = self.post_attention_layernorm(hidden, residual)
-        hidden = self.mlp(hidden)
-        return hidden, residual
+        hidden, residual = self.self_attn.forward_add_norm(
+            positions, hidden, residual, self.post_attention_layernorm, fctx)
+        if next_norm is None:
+            return self.mlp(hidden), residual
+        if isinstance(self.mlp, DenseMLP):
+            return self.mlp.forward_add_norm(hidden, residual, next_norm)
+        return next_norm(self.mlp(hidden), residual)
 
 
 class MoEFamilyForCausalLM(LlamaFamilyForCausalLM):

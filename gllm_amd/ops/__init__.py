@@ -714,19 +714,7 @@ def mla_paged_attention(q, k_cache, v_cache, block_table, seq_lens,
 
 
 # --------------------------------------------------------------- gemm
-_SKINNY_WS: dict = {}
 SKINNY_MAX_M = 256
-
-
-def _skinny_splitk(M: int, N: int, K: int) -> int:
-    # v2 kernel grid is (N/64, splitk) — M-blocks live INSIDE one
-    # workgroup, so the fill target counts only N tiles
-    n_wg = -(-N // 64)
-    s = 1
-    while s < 16 and n_wg * s < 512 and (K // (s * 2)) >= 64:
-        s *= 2
-    k_slice = ((-(-K // s)) + 63) // 64 * 64
-    return -(-K // k_slice)
 
 
 def _quant_splitk(N: int, K: int, bk: int) -> int:
@@ -742,63 +730,123 @@ def _quant_splitk(N: int, K: int, bk: int) -> int:
     return -(-K // k_slice)
 
 
+def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """bf16 operands as csrc/stream_gemm.hip reads them: 16 B aligned
+    rows, K a multiple of 64, N of 8."""
+    return (x.is_cuda and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
+            and x.is_contiguous() and w.is_contiguous()
+            and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _plain_bias(bias, N: int) -> bool:
+    return bias is None or (bias.dtype == torch.bfloat16
+                            and bias.is_contiguous() and bias.numel() == N)
+
+
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out = x @ w.T via the gfx950 weight-streaming kernel (M<=256-ish)."""
-    import os
-    M, K = x.shape
-    N = w.shape[0]
-    splitk = int(os.environ.get("SK_SPLITK", "0")) or \
-        _skinny_splitk(M, N, K)
-    need = splitk * M * N
-    key = x.device.index or 0
-    ws = _SKINNY_WS.get(key)
-    if ws is None or ws.numel() < need:
-        if torch.cuda.is_current_stream_capturing():
-            # growing the cached workspace mid-capture would free the
-            # buffer an earlier-captured graph writes (the r1 replay
-            # fault class); warmup must size it first
-            raise RuntimeError(
-                "skinny_gemm workspace grown during graph capture — "
-                "run an eager warmup at the largest bucket first")
-        ws = torch.empty(need, dtype=torch.float32, device=x.device)
-        _SKINNY_WS[key] = ws
-    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-    _gpu_kernels().skinny_gemm(out, x, w, None, ws, splitk)
-    if bias is not None:
-        out += bias
-    return out
+    """out = x @ w.T (+ bias) via the gfx950 weight-streaming kernel (at
+    most 256 rows)."""
+    if not _rows_ok(x, w):
+        import torch.nn.functional as F
+        return F.linear(x, w, bias)
+    if not _plain_bias(bias, w.shape[0]):
+        return _gpu_kernels().stream_gemm(x, w, None) + bias
+    return _gpu_kernels().stream_gemm(x, w, bias)
 
 
 def _use_skinny(M: int, N: int, K: int) -> bool:
-    """Measured dispatch rule (scripts/gemm_sweep.py on MI355X r01):
-    the skinny kernel beats hipBLASLt on K-deep reductions at any decode
-    M (down_proj: 1.9 -> 4.1 TB/s) and on every N<=8k shape once M>64
-    (library tiles collapse to ~1.1-1.6 TB/s there); the library keeps
-    wide-N shapes (gate_up, lm_head) and small-M small-K projections."""
+    """Measured against hipBLASLt (us, stream / library): up to 64 rows
+    the stream wins wherever the product is more than a few workgroups (64
+    x 5120 x 5120 20.6 / 24.6, 64 x 38016 x 5120 83 / 89, 64 x 5120 x 27648
+    63 / 159); above that the library is level or better on wide weights
+    (96 x 28672 x 4096 57.6 / 55.6, 256 x 38016 x 5120 139 / 109) and
+    worse on the rest (256 x 7168 x 5120 40 / 54, 256 x 5120 x 27648 110 /
+    266)."""
     import os
     if os.environ.get("GLLM_DISABLE_SKINNY"):
         return False
     max_m = int(os.environ.get("GLLM_SKINNY_MAX_M", "0")) or SKINNY_MAX_M
-    if K % 64 != 0 or N < 1024 or M > max_m:
+    if K % 64 != 0 or N < 512 or M > max_m or M == 0:
         return False
-    # MB>=2 under capture: r1 faulted with dynamic LDS; the kernel now
-    # uses static LDS and captures cleanly
-    if K >= 2 * N:
-        return True
-    return M > 64 and N <= 8192
+    return M <= 64 or N < 16384
+
+
+def _streams(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return _rows_ok(x, w) and _use_skinny(x.shape[0], w.shape[0],
+                                          w.shape[1])
 
 
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """GEMM dispatch: the skinny weight-streaming kernel where measured
-    faster, hipBLASLt otherwise."""
+    """GEMM dispatch: the weight-streaming kernel where measured faster,
+    hipBLASLt otherwise."""
     import torch.nn.functional as F
-    if (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2
-            and x.is_contiguous()
-            and _use_skinny(x.shape[0], w.shape[0], w.shape[1])):
+    if _streams(x, w) and _plain_bias(bias, w.shape[0]):
         return skinny_gemm(x, w, bias)
     return F.linear(x, w, bias)
+
+
+def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ w_gate.T) * (x @ w_up.T), w = gate rows over up rows. Few
+    rows: one kernel, the [rows, 2 ff] product is never written (above 64
+    rows it is level with the library's product and saves the second
+    kernel: 256 x 55296 x 5120 149 us against 154 + 9)."""
+    if (_rows_ok(x, w) and w.shape[0] % 16 == 0 and w.shape[0] >= 512
+            and _use_skinny(x.shape[0], 512, w.shape[1])):
+        return _gpu_kernels().stream_gemm_gated(x, w)
+    return silu_and_mul(linear(x, w))
+
+
+def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
+                       residual: torch.Tensor, norm_w: torch.Tensor,
+                       eps: float):
+    """residual += x @ w.T; (rmsnorm(residual), residual). Few rows: the
+    split product's parts are summed, added and normed by one kernel."""
+    if (_streams(x, w) and w.shape[0] <= 8192
+            and residual.dtype == torch.bfloat16
+            and residual.is_contiguous()
+            and residual.data_ptr() % 16 == 0
+            and norm_w.dtype in (torch.bfloat16, torch.float32)):
+        return _gpu_kernels().stream_add_norm(x, w, residual, norm_w,
+                                              eps), residual
+    return fused_add_rmsnorm(linear(x, w), residual, norm_w, eps)
+
+
+def qkv_parts(x: torch.Tensor, w: torch.Tensor,
+              bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """The fp32 parts [S, M, N] of x @ w.T for ``qkv_rope_cache``, or None
+    where the library's product is the better one."""
+    if _streams(x, w) and _plain_bias(bias, w.shape[0]):
+        return _gpu_kernels().stream_parts(x, w)
+    return None
+
+
+def qkv_rope_cache_ok(k_cache: torch.Tensor, v_cache: torch.Tensor,
+                      cos_sin: torch.Tensor, is_neox: bool) -> bool:
+    return (is_neox and k_cache.is_cuda and k_cache.dim() == 4
+            and k_cache.dtype == torch.bfloat16
+            and v_cache.dtype == torch.bfloat16
+            and v_cache.shape == k_cache.shape and k_cache.is_contiguous()
+            and v_cache.is_contiguous() and k_cache.shape[3] % 8 == 0
+            and cos_sin.device == k_cache.device
+            and cos_sin.dtype == torch.float32 and cos_sin.is_contiguous()
+            and cos_sin.shape[-1] % 8 == 0
+            and cos_sin.shape[-1] <= k_cache.shape[3])
+
+
+def qkv_rope_cache(src: torch.Tensor, bias, positions: torch.Tensor,
+                   cos_sin: torch.Tensor, k_cache: torch.Tensor,
+                   v_cache: torch.Tensor, slot_mapping: torch.Tensor,
+                   num_heads: int) -> torch.Tensor:
+    """From a merged q|k|v projection (bf16 rows, or the fp32 parts of
+    ``qkv_parts``): add the bias, rotate queries and keys, write keys and
+    values to their cache slots, return the queries [M, heads * D]. One
+    kernel for a bias, a rotation, a scatter and their copies."""
+    return _gpu_kernels().qkv_finish(src, bias, positions, cos_sin, k_cache,
+                                     v_cache, slot_mapping, num_heads)
 
 
 # --------------------------------------------------------------- layer norm

@@ -17,9 +17,17 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_table, torch::Tensor seq_lens,
                             double scale, long sliding_window);
-void skinny_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                 c10::optional<torch::Tensor> bias,
-                 torch::Tensor workspace, long splitk);
+torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
+                          c10::optional<torch::Tensor> bias);
+torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
+torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w);
+torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
+                              torch::Tensor residual, torch::Tensor norm_w,
+                              double eps);
+torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, long Hq);
 void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor k_cache, torch::Tensor v_cache,
                              torch::Tensor block_table,
@@ -146,8 +154,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attention_decode", &window_attention_decode,
         "split-KV decode kernels with window + kept first + sink + gate; "
         "false = geometry not instantiated");
-  m.def("skinny_gemm", &skinny_gemm,
-        "decode-regime weight-streaming GEMM (M<=256)");
+  m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
+  m.def("stream_gemm_gated", &stream_gemm_gated,
+        "silu(x w_gate^T) * (x w_up^T) for at most 256 rows");
+  m.def("stream_parts", &stream_parts, "fp32 parts of x w^T");
+  m.def("stream_add_norm", &stream_add_norm,
+        "residual += x w^T; RMS norm of it");
+  m.def("qkv_finish", &qkv_finish,
+        "bias, rotation, keys and values to the cache; queries");
   m.def("mla_paged_attention", &mla_paged_attention,
         "absorbed-MLA varlen attention over the 576-dim latent cache");
   m.def("mla_queries", &mla_queries,

@@ -170,11 +170,19 @@ void sigmoid_group_topk(torch::Tensor weights, torch::Tensor ids,
                         torch::Tensor logits,
                         c10::optional<torch::Tensor> correction,
                         long n_group, long keep, double scale);
-// shared with the full extension (skinny_gemm.hip, moe.hip,
+// shared with the full extension (stream_gemm.hip, moe.hip,
 // elementwise.hip): what ops.linear / FusedMoE dispatch to in bf16
-void skinny_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                 c10::optional<torch::Tensor> bias,
-                 torch::Tensor workspace, long splitk);
+torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
+                          c10::optional<torch::Tensor> bias);
+torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
+torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w);
+torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
+                              torch::Tensor residual, torch::Tensor norm_w,
+                              double eps);
+torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, long Hq);
 void silu_and_mul(torch::Tensor out, torch::Tensor x);
 void moe_align(torch::Tensor topk_ids, long E_local, long expert_start,
                long block_m, torch::Tensor sorted_ids,
@@ -267,8 +275,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tanh_rows", &tanh_rows, "tanh over strided rows");
   m.def("sigmoid_group_topk", &sigmoid_group_topk,
         "sigmoid router with correction and group limits");
-  m.def("skinny_gemm", &skinny_gemm,
-        "decode-regime weight-streaming GEMM (M<=256)");
+  m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
+  m.def("stream_gemm_gated", &stream_gemm_gated,
+        "silu(x w_gate^T) * (x w_up^T) for at most 256 rows");
+  m.def("stream_parts", &stream_parts, "fp32 parts of x w^T");
+  m.def("stream_add_norm", &stream_add_norm,
+        "residual += x w^T; RMS norm of it");
+  m.def("qkv_finish", &qkv_finish,
+        "bias, rotation, keys and values to the cache; queries");
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d]) * x[d:]");
   m.def("moe_align", &moe_align, "device-side moe_align_block_size");
   m.def("moe_gemm", &moe_gemm, "grouped MFMA GEMM over sorted pairs");

@@ -1,0 +1,589 @@
+// Products of few rows (M <= 256) with a weight matrix: x [M, K] W[N, K]^T,
+// bf16 in, fp32 sums (K a multiple of 64).
+//
+// Bound by the weights' bytes, so the job is to keep them coming: 16 B
+// global -> LDS loads (non-temporal: a weight row is used by one workgroup)
+// into a ring that holds several 64-column stages in flight, two workgroups
+// per CU where LDS allows. LDS rows are 128 B with their 16 B units permuted
+// by row & 7, so fragment reads fall on all banks; products are W x^T, so a
+// lane ends with four neighbouring columns of one row.
+//
+// A weight with few 64-row tiles is also split along K, into about 512
+// workgroups in all; the fp32 parts [S, M, N] are then summed by whatever
+// comes next, in the order of S:
+//   stream_gemm           bias, bf16
+//   stream_add_norm       residual += sum, RMS norm of it (attention and
+//                         feed-forward outputs)
+//   qkv_finish            bias, rotation, keys and values to their cache
+//                         slots, queries out
+// and a gated feed-forward (gate and up rows of W alternate in the staged
+// tile) leaves silu(gate) * up straight from the sums.
+// (us against hipBLASLt and against the kernel before this one, which split
+// K into up to 16 and summed the parts one load at a time:) 5120 x 27648, 64
+// rows 63 for 159 and 79, 256 rows 110 for 266 and 160; 7168 x 5120, 1 row
+// 16.4 for 24; 28672 x 4096 gated, 1 row 39 for 61 + 5. Weights come at 4.0
+// to 6.6 TB/s from 35 MB on, below that the launch and the ring's first
+// stages are most of the time (2048 x 2048: 5 + 3 us).
+
+#include <torch/extension.h>
+#include <ATen/cuda/CUDAContext.h>
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 st_bf8;
+typedef __attribute__((ext_vector_type(4))) float st_f4;
+
+namespace {
+
+constexpr int BK = 64;
+constexpr int ROW_B = BK * 2;  // LDS row bytes
+constexpr int MAX_SPLIT = 16;
+
+enum Form { GATED = 0, PLAIN = 1, PART = 2 };
+
+// AUX 2: non-temporal
+template <int AUX>
+DEV_INLINE void glds16(const __hip_bfloat16 *gsrc, char *lds_ptr) {
+  __builtin_amdgcn_global_load_lds(
+      reinterpret_cast<const unsigned int *>(gsrc),
+      reinterpret_cast<unsigned int *>(lds_ptr), 16, 0, AUX);
+}
+
+DEV_INLINE short to_bf16(float v) {
+  return __builtin_bit_cast(short, __float2bfloat16(v));
+}
+
+// wait until at most AHEAD stages of LD loads are on their way
+template <int AHEAD, int LD>
+DEV_INLINE void wait_stages(int ahead) {
+  if (ahead >= AHEAD)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(AHEAD * LD) : "memory");
+  else if constexpr (AHEAD > 0)
+    wait_stages<AHEAD - 1, LD>(ahead);
+}
+
+// WM x WN waves share a BM x BN tile; a ring of ST stages of BK columns
+template <int BM, int BN, int WM, int WN, int ST, int FORM>
+__global__ __launch_bounds__(WM *WN * 64) void stream_gemm_kernel(
+    void *__restrict__ C,  // bf16 [M, N or N / 2], PART: fp32 [S, M, N]
+    const __hip_bfloat16 *__restrict__ A, long lda,
+    const __hip_bfloat16 *__restrict__ W,  // [N, K]
+    const __hip_bfloat16 *__restrict__ bias, int M, int N, int K,
+    int k_slice, int nbm, int nbn) {
+  constexpr int THREADS = WM * WN * 64;
+  constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
+  constexpr int A_B = BM * ROW_B, STAGE = A_B + BN * ROW_B;
+  constexpr int A_UNITS = A_B / 1024, B_UNITS = BN * ROW_B / 1024;
+  constexpr int WAVES = WM * WN;
+  // BM = 16: two waves bring the rows, the other two only weights
+  constexpr int AL = (A_UNITS + WAVES - 1) / WAVES;
+  constexpr int BL = B_UNITS / WAVES;
+  static_assert(BL * WAVES == B_UNITS, "whole loads");
+  static_assert(A_UNITS % WAVES == 0 || A_UNITS < WAVES, "whole loads");
+  __shared__ __attribute__((aligned(16))) char smem[ST * STAGE];
+
+  // eight dies take workgroups in turn: each gets a contiguous run of tiles,
+  // row blocks fastest (they share weights)
+  const int total = nbm * nbn;
+  const int pid = blockIdx.x, xcd = pid & 7, per = total >> 3;
+  const int t = xcd * per + min(xcd, total & 7) + (pid >> 3);
+  const int mb = t % nbm, nb = t / nbm;
+  const int z = blockIdx.y;
+  const int k0 = z * k_slice;
+  const int nkt = min(K - k0, k_slice) / BK;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int l16 = lane & 15, lhi = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  const int NC = FORM == GATED ? N >> 1 : N;  // columns of C
+
+  // sources: unit u of 1 KB = 8 rows, lane = row u * 8 + lane / 8
+  const int sub = lane >> 3, col = ((lane & 7) ^ sub) * 8;
+  const bool a_wave = A_UNITS >= WAVES || wave < A_UNITS;
+  const __hip_bfloat16 *asrc[AL], *bsrc[BL];
+#pragma unroll
+  for (int j = 0; j < AL; ++j) {
+    const int row = min((j * WAVES + wave) * 8 + sub, BM - 1);
+    asrc[j] = A + (long)min(mb * BM + row, M - 1) * lda + k0 + col;
+  }
+#pragma unroll
+  for (int j = 0; j < BL; ++j) {
+    const int row = (j * WAVES + wave) * 8 + sub;
+    int n;
+    if (FORM == GATED) {  // 16 gate rows, their 16 up rows, the next 16
+      const int c = min(nb * (BN / 2) + (row >> 5) * 16 + (row & 15), NC - 1);
+      n = (row & 16) ? NC + c : c;
+    } else {
+      n = min(nb * BN + row, N - 1);
+    }
+    bsrc[j] = W + (long)n * K + k0 + col;
+  }
+  auto stage = [&](int slot) {
+    char *base = smem + slot * STAGE + wave * 1024;
+    if (a_wave) {
+#pragma unroll
+      for (int j = 0; j < AL; ++j) {
+        glds16<0>(asrc[j], base + j * WAVES * 1024);
+        asrc[j] += BK;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < BL; ++j) {
+      glds16<2>(bsrc[j], base + A_B + j * WAVES * 1024);
+      bsrc[j] += BK;
+    }
+  };
+  st_f4 acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = st_f4{0, 0, 0, 0};
+
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i)
+    if (i < nkt) stage(i);
+  int cur = 0, nxt = ST - 1;
+  for (int kt = 0; kt < nkt; ++kt) {
+    // this wave's loads of stage kt have landed, later ones may fly
+    const int ahead = min(nkt - 1 - kt, ST - 2);
+    if (a_wave) wait_stages<ST - 2, AL + BL>(ahead);
+    else wait_stages<ST - 2, BL>(ahead);
+    // everybody's are there, and stage kt - 1 (the slot that the next one
+    // takes) has been read
+    __builtin_amdgcn_s_barrier();
+    if (kt + ST - 1 < nkt) stage(nxt);
+    const char *ab = smem + cur * STAGE + (wm * MT * 16 + l16) * ROW_B;
+    const char *bb = smem + cur * STAGE + A_B + (wn * NT * 16 + l16) * ROW_B;
+#pragma unroll
+    for (int ks = 0; ks < BK / 32; ++ks) {
+      const int off = ((ks * 4 + lhi) ^ (l16 & 7)) << 4;
+      st_bf8 bf[NT], af[MT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        bf[n] = *reinterpret_cast<const st_bf8 *>(bb + n * 16 * ROW_B + off);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        af[m] = *reinterpret_cast<const st_bf8 *>(ab + m * 16 * ROW_B + off);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              bf[n], af[m], acc[n][m], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    cur = cur + 1 == ST ? 0 : cur + 1;
+    nxt = nxt + 1 == ST ? 0 : nxt + 1;
+  }
+
+  // lane: row l16 of each row tile, columns lhi * 4 + r
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = mb * BM + (wm * MT + m) * 16 + l16;
+    if (row >= M) continue;
+#pragma unroll
+    for (int n = 0; n < NT; n += FORM == GATED ? 2 : 1) {
+      const int tile = wn * NT + n;
+      const int c = nb * (FORM == GATED ? BN / 2 : BN) +
+                    tile * (FORM == GATED ? 8 : 16) + lhi * 4;
+      if (c >= NC) continue;
+      if (FORM == PART) {
+        *reinterpret_cast<st_f4 *>((float *)C + ((long)z * M + row) * N + c) =
+            acc[n][m];
+        continue;
+      }
+      shortx4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[n][m][r];
+        if (FORM == GATED)
+          v = v / (1.f + __expf(-v)) * acc[n + (NT > 1 ? 1 : 0)][m][r];
+        else if (bias)
+          v += __bfloat162float(bias[c + r]);
+        o[r] = to_bf16(v);
+      }
+      *reinterpret_cast<shortx4 *>((__hip_bfloat16 *)C + (long)row * NC + c) =
+          o;
+    }
+  }
+}
+
+// sum of the S parts of four columns; loads of eight parts in flight
+DEV_INLINE st_f4 part_sum(const float *p, long stride, int S) {
+  st_f4 v = *reinterpret_cast<const st_f4 *>(p);
+  int s = 1;
+  for (; s + 8 <= S; s += 8) {
+    st_f4 b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      b[i] = *reinterpret_cast<const st_f4 *>(p + (s + i) * stride);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v += b[i];
+  }
+  st_f4 b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    b[i] = *reinterpret_cast<const st_f4 *>(p + min(s + i, S - 1) * stride);
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (s + i < S) v += b[i];
+  return v;
+}
+
+__global__ __launch_bounds__(256) void stream_sum_kernel(
+    __hip_bfloat16 *__restrict__ out, const float *__restrict__ part,
+    const __hip_bfloat16 *__restrict__ bias, long MN, int N, int S) {
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= MN) return;
+  const st_f4 v = part_sum(part + i, MN, S);
+  const int n = i % N;
+  shortx4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    o[r] = to_bf16(v[r] + (bias ? __bfloat162float(bias[n + r]) : 0.f));
+  *reinterpret_cast<shortx4 *>(out + i) = o;
+}
+
+// A workgroup per row: residual += sum of the parts (rounded as stored),
+// out = RMS norm of the stored residual. V x 4 columns per thread.
+template <int V, typename TW>
+__global__ __launch_bounds__(512) void stream_add_norm_kernel(
+    __hip_bfloat16 *__restrict__ out, __hip_bfloat16 *__restrict__ residual,
+    const float *__restrict__ part, const TW *__restrict__ w, float eps,
+    int M, int N, int S) {
+  __shared__ float red[8];
+  const long row = blockIdx.x;
+  const long MN = (long)M * N;
+  float x[V][4], ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const int c = (j * 512 + threadIdx.x) * 4;
+    if (c >= N) continue;
+    const st_f4 v = part_sum(part + row * N + c, MN, S);
+    __hip_bfloat16 *rp = residual + row * N + c;
+    const shortx4 old = *reinterpret_cast<const shortx4 *>(rp);
+    shortx4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      o[r] = to_bf16(v[r] + __bfloat162float(__builtin_bit_cast(
+                                __hip_bfloat16, (short)old[r])));
+      x[j][r] =
+          __bfloat162float(__builtin_bit_cast(__hip_bfloat16, (short)o[r]));
+      ss += x[j][r] * x[j][r];
+    }
+    *reinterpret_cast<shortx4 *>(rp) = o;
+  }
+  ss = block_reduce_sum<512>(ss, red);
+  const float inv = rsqrtf(ss / N + eps);
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const int c = (j * 512 + threadIdx.x) * 4;
+    if (c >= N) continue;
+    shortx4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      o[r] = to_bf16(x[j][r] * inv * ScalarOps<TW>::to_f32(w[c + r]));
+    *reinterpret_cast<shortx4 *>(out + row * N + c) = o;
+  }
+}
+
+// A workgroup per token, a thread per 8 columns of a head: 4 + 4 columns of
+// a rotated pair block, or 8 plain ones. PARTS: src is fp32 [S, M, N].
+template <bool PARTS>
+__global__ __launch_bounds__(256) void qkv_finish_kernel(
+    __hip_bfloat16 *__restrict__ q_out, __hip_bfloat16 *__restrict__ k_cache,
+    __hip_bfloat16 *__restrict__ v_cache, const void *__restrict__ src,
+    long src_stride, const __hip_bfloat16 *__restrict__ bias,
+    const long *__restrict__ positions, const float *__restrict__ cos_sin,
+    const long *__restrict__ slots, int M, int S, int Hq, int Hkv, int D,
+    int rot) {
+  const long t = blockIdx.x;
+  const int N = (Hq + 2 * Hkv) * D, per = D / 8;
+  const float *cs = cos_sin + positions[t] * rot;
+  const long slot = slots[t];
+  auto load4 = [&](int c, float *o) {
+    if (PARTS) {
+      const st_f4 v =
+          part_sum((const float *)src + t * N + c, (long)M * N, S);
+      o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
+    } else {
+      const shortx4 v = *reinterpret_cast<const shortx4 *>(
+          (const __hip_bfloat16 *)src + t * src_stride + c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = __bfloat162float(
+            __builtin_bit_cast(__hip_bfloat16, (short)v[r]));
+    }
+    if (bias) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] += __bfloat162float(bias[c + r]);
+    }
+  };
+  for (int i = threadIdx.x; i < (Hq + 2 * Hkv) * per; i += blockDim.x) {
+    const int h = i / per, u = i % per;
+    const bool turned = h < Hq + Hkv && u < rot / 8;
+    // first columns of the two groups of four
+    const int d1 = turned ? u * 4 : u * 8;
+    const int d2 = turned ? rot / 2 + u * 4 : u * 8 + 4;
+    float a[4], b[4];
+    load4(h * D + d1, a);
+    load4(h * D + d2, b);
+    if (turned) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float c = cs[d1 + r], s = cs[rot / 2 + d1 + r];
+        const float x = a[r], y = b[r];
+        a[r] = x * c - y * s;
+        b[r] = y * c + x * s;
+      }
+    }
+    __hip_bfloat16 *dst;
+    if (h < Hq) dst = q_out + (t * Hq + h) * D;
+    else if (h < Hq + Hkv) dst = k_cache + (slot * Hkv + (h - Hq)) * D;
+    else dst = v_cache + (slot * Hkv + (h - Hq - Hkv)) * D;
+    shortx4 o1, o2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      o1[r] = to_bf16(a[r]);
+      o2[r] = to_bf16(b[r]);
+    }
+    *reinterpret_cast<shortx4 *>(dst + d1) = o1;
+    *reinterpret_cast<shortx4 *>(dst + d2) = o2;
+  }
+}
+
+bool aligned16(const torch::Tensor &t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+struct Plan {
+  int bm, bn, nbm, nbn, splits, k_slice;
+};
+
+// The tile by the rows and by how wide the weight is (us, M x N x K, each
+// against its neighbour):
+//  * up to 64 rows 64 columns, two workgroups per CU: 16 x 7168 x 5120 18.2
+//    (128 columns 19.1), 64 x 28672 x 4096 47.6 (50.7); from 36000 columns
+//    on, where rows would be staged too often, 256: 64 x 55296 x 5120 93
+//    (64 columns 129, 128 columns 106), 24 rows 86 (98).
+//  * up to 128 rows: below 8192 columns two row blocks of 64, 128 x 7168 x
+//    5120 28.9 (128 x 64 tiles 31.6); K at least 2 N: 128 x 128, 128 x 5120
+//    x 27648 75 (128 x 64 80); from 36000 columns 128 x 256, 128 x 55296 x
+//    5120 105 (128 x 128 128); else 128 x 64.
+//  * up to 256 rows: K at least 2 N or 16384 columns and more: 256 x 128,
+//    256 x 5120 x 27648 110 (128 x 128 118), 256 x 28672 x 4096 68 (128 x 64
+//    90); gated and 36000 columns 256 x 256, 149 (256 x 128 175); else 128 x
+//    64, 256 x 7168 x 5120 40 (128 x 128 42).
+// K is split into about 384 workgroups where there are fewer than 160 tiles
+// (5120 x 27648, 16 rows: 5 splits 50.8, 13 splits 52.9; 7168 x 5120: 4
+// splits 18.2, 7 splits 19.6; 11008 x 2048 at 172 tiles: none 11.2, two
+// 13.4), into two from there to 288 tiles if K is long, each part at least
+// four stages long.
+Plan plan_for(int M, int N, int K, bool gated) {
+  Plan p;
+  const bool wide = N >= 36000, deep = K >= 2 * N;
+  p.bn = 64;
+  if (M <= 64) {
+    p.bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    if (wide && p.bm > 16) p.bn = 256;
+  } else if (M <= 128) {
+    p.bm = wide || deep || N >= 8192 ? 128 : 64;
+    p.bn = wide ? 256 : deep ? 128 : 64;
+  } else {
+    p.bm = deep || N >= 16384 ? 256 : 128;
+    p.bn = p.bm == 128 ? 64 : gated && wide ? 256 : 128;
+  }
+  p.nbm = (M + p.bm - 1) / p.bm;
+  p.nbn = (N + p.bn - 1) / p.bn;
+  const int tiles = p.nbm * p.nbn, stages = K / BK;
+  int s = 1;
+  if (!gated) {
+    if (tiles < 160) s = (384 + tiles - 1) / tiles;
+    else if (tiles < 288 && stages >= 128) s = 2;
+    s = std::max(1, std::min(std::min(s, MAX_SPLIT), stages / 4));
+  }
+  const int per = (stages + s - 1) / s;
+  p.k_slice = per * BK;
+  p.splits = (stages + per - 1) / per;
+  return p;
+}
+
+void check_operands(const torch::Tensor &x, const torch::Tensor &w) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16 && x.dim() == 2 &&
+              w.dim() == 2 && x.size(1) == w.size(1));
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+              w.is_contiguous() && aligned16(x) && aligned16(w),
+              "stream_gemm: 16 B aligned rows");
+  TORCH_CHECK(w.size(1) % BK == 0 && w.size(1) > 0 && w.size(0) % 8 == 0,
+              "stream_gemm: K a multiple of 64, N of 8");
+  TORCH_CHECK(x.size(0) <= 256, "stream_gemm: at most 256 rows");
+}
+
+template <int FORM>
+void launch(const Plan &p, void *C, const torch::Tensor &x,
+            const torch::Tensor &w, const void *bias) {
+  const int M = x.size(0), N = w.size(0), K = w.size(1);
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define RUN(BM, BN, WM, WN, ST)                                              \
+  hipLaunchKernelGGL((stream_gemm_kernel<BM, BN, WM, WN, ST, FORM>),         \
+                     dim3(p.nbm * p.nbn, p.splits), dim3((WM) * (WN) * 64),  \
+                     0, stream, C, (const __hip_bfloat16 *)x.data_ptr(),     \
+                     x.size(0) > 1 ? (long)x.stride(0) : 0L,                 \
+                     (const __hip_bfloat16 *)w.data_ptr(),                   \
+                     (const __hip_bfloat16 *)bias, M, N, K, p.k_slice,       \
+                     p.nbm, p.nbn)
+  // (a wave needs a gate and an up tile, so 16 columns are too few)
+  if (p.bm == 16) RUN(16, 64, 1, FORM == GATED ? 2 : 4, 8);
+  else if (p.bm == 32 && p.bn == 64) RUN(32, 64, 1, 2, 6);
+  else if (p.bm == 32) RUN(32, 256, 1, 4, 4);
+  else if (p.bm == 64 && p.bn == 64) RUN(64, 64, 2, 2, 5);
+  else if (p.bm == 64) RUN(64, 256, 2, 4, 3);
+  else if (p.bm == 128 && p.bn == 64) RUN(128, 64, 2, 2, 3);
+  else if (p.bm == 128 && p.bn == 128) RUN(128, 128, 2, 2, 2);
+  else if (p.bm == 128) RUN(128, 256, 2, 4, 3);
+  else if (p.bn == 128) RUN(256, 128, 4, 2, 3);
+  else if constexpr (FORM == GATED) RUN(256, 256, 2, 4, 2);
+  else TORCH_CHECK(false, "stream_gemm: no such tile");
+#undef RUN
+  HIP_CHECK_KERNEL();
+}
+
+const void *bias_ptr(const c10::optional<torch::Tensor> &bias, long N) {
+  if (!bias.has_value()) return nullptr;
+  TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+              bias->numel() == N, "bias: bf16 [N]");
+  return bias->data_ptr();
+}
+
+}  // namespace
+
+// the fp32 parts [S, M, N] of x w^T
+torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w) {
+  check_operands(x, w);
+  const long M = x.size(0), N = w.size(0);
+  TORCH_CHECK(M > 0);
+  const Plan p = plan_for(M, N, w.size(1), false);
+  auto part = torch::empty({(long)p.splits, M, N},
+                           x.options().dtype(at::kFloat));
+  launch<PART>(p, part.data_ptr(), x, w, nullptr);
+  return part;
+}
+
+torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
+                          c10::optional<torch::Tensor> bias) {
+  check_operands(x, w);
+  const long M = x.size(0), N = w.size(0);
+  const void *bp = bias_ptr(bias, N);
+  auto out = torch::empty({M, N}, x.options());
+  if (M == 0) return out;
+  const Plan p = plan_for(M, N, w.size(1), false);
+  if (p.splits == 1) {
+    launch<PLAIN>(p, out.data_ptr(), x, w, bp);
+    return out;
+  }
+  auto part = torch::empty({(long)p.splits, M, N},
+                           x.options().dtype(at::kFloat));
+  launch<PART>(p, part.data_ptr(), x, w, nullptr);
+  auto stream = at::cuda::getCurrentCUDAStream();
+  hipLaunchKernelGGL(stream_sum_kernel, dim3((M * N / 4 + 255) / 256),
+                     dim3(256), 0, stream, (__hip_bfloat16 *)out.data_ptr(),
+                     part.data_ptr<float>(), (const __hip_bfloat16 *)bp,
+                     M * N, (int)N, p.splits);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+// silu(x w_gate^T) * (x w_up^T), w = gate rows, up rows
+torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w) {
+  check_operands(x, w);
+  const long M = x.size(0), N = w.size(0);
+  TORCH_CHECK(N % 16 == 0);
+  auto out = torch::empty({M, N / 2}, x.options());
+  if (M == 0) return out;
+  launch<GATED>(plan_for(M, N, w.size(1), true), out.data_ptr(), x, w,
+                nullptr);
+  return out;
+}
+
+// residual (bf16 [M, N], in place) += x w^T; returns its RMS norm
+torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
+                              torch::Tensor residual, torch::Tensor norm_w,
+                              double eps) {
+  auto part = stream_parts(x, w);
+  const int S = part.size(0), M = part.size(1), N = part.size(2);
+  TORCH_CHECK(residual.scalar_type() == at::kBFloat16 &&
+              residual.is_contiguous() && residual.numel() == (long)M * N &&
+              aligned16(residual));
+  TORCH_CHECK(norm_w.is_contiguous() && norm_w.numel() == N &&
+              N <= 512 * 4 * 4, "stream_add_norm: at most 8192 columns");
+  auto out = torch::empty({(long)M, (long)N}, x.options());
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define RUN(V, TW)                                                           \
+  hipLaunchKernelGGL((stream_add_norm_kernel<V, TW>), dim3(M), dim3(512), 0, \
+                     stream, (__hip_bfloat16 *)out.data_ptr(),               \
+                     (__hip_bfloat16 *)residual.data_ptr(),                  \
+                     part.data_ptr<float>(), (const TW *)norm_w.data_ptr(),  \
+                     (float)eps, M, N, S)
+#define COLS(TW)                                                             \
+  do {                                                                       \
+    if (N <= 2048) RUN(1, TW);                                               \
+    else if (N <= 4096) RUN(2, TW);                                          \
+    else if (N <= 6144) RUN(3, TW);                                          \
+    else RUN(4, TW);                                                         \
+  } while (0)
+  if (norm_w.scalar_type() == at::kFloat) COLS(float);
+  else if (norm_w.scalar_type() == at::kBFloat16) COLS(__hip_bfloat16);
+  else TORCH_CHECK(false, "norm_w: fp32 or bf16");
+#undef COLS
+#undef RUN
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+// src: bf16 rows [M, (Hq + 2 Hkv) D] (a row view is fine) or the fp32 parts
+// of the same. Rotates (rotate-half on the first `rot` dims) queries and
+// keys, writes keys and values to their slots, returns the queries.
+torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, long Hq) {
+  const bool parts = src.dim() == 3;
+  const long M = src.size(parts ? 1 : 0), N = src.size(parts ? 2 : 1);
+  const int Hkv = k_cache.size(2), D = k_cache.size(3);
+  const int rot = cos_sin.size(-1);
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.is_contiguous() &&
+              v_cache.is_contiguous() && v_cache.sizes() == k_cache.sizes() &&
+              k_cache.scalar_type() == at::kBFloat16 &&
+              v_cache.scalar_type() == at::kBFloat16 && aligned16(k_cache) &&
+              aligned16(v_cache));
+  TORCH_CHECK(N == (Hq + 2L * Hkv) * D && D % 8 == 0 && rot % 8 == 0 &&
+              rot <= D && Hq > 0);
+  TORCH_CHECK(src.is_cuda() && aligned16(src) &&
+              (parts ? src.is_contiguous() &&
+                           src.scalar_type() == at::kFloat
+                     : src.scalar_type() == at::kBFloat16 &&
+                           src.stride(1) == 1 && src.stride(0) % 8 == 0));
+  TORCH_CHECK(positions.scalar_type() == at::kLong &&
+              positions.is_contiguous() && positions.numel() == M &&
+              slots.scalar_type() == at::kLong && slots.is_contiguous() &&
+              slots.numel() == M);
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat &&
+              cos_sin.is_contiguous());
+  const void *bp = bias_ptr(bias, N);
+  auto q = torch::empty({M, Hq * D}, k_cache.options());
+  if (M == 0) return q;
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define RUN(P)                                                               \
+  hipLaunchKernelGGL((qkv_finish_kernel<P>), dim3(M), dim3(256), 0, stream,  \
+                     (__hip_bfloat16 *)q.data_ptr(),                         \
+                     (__hip_bfloat16 *)k_cache.data_ptr(),                   \
+                     (__hip_bfloat16 *)v_cache.data_ptr(), src.data_ptr(),   \
+                     parts ? 0L : (long)src.stride(0),                       \
+                     (const __hip_bfloat16 *)bp, positions.data_ptr<long>(), \
+                     cos_sin.data_ptr<float>(), slots.data_ptr<long>(),      \
+                     (int)M, parts ? (int)src.size(0) : 1, (int)Hq, Hkv, D,  \
+                     rot)
+  if (parts) RUN(true); else RUN(false);
+#undef RUN
+  HIP_CHECK_KERNEL();
+  return q;
+}

@@ -9,7 +9,7 @@ repo snapshots without a site-packages install:
 * ``gllm_amd._kernels_seq``  the dtype-generic sequence-mixer kernels
   (norms over an fp32 residual, windowed sink attention, talking-heads
   and latent attention, varlen delta rules, outer-product recurrences)
-  plus the grouped MoE GEMM, activations and skinny GEMM that the
+  plus the grouped MoE GEMM, activations and the few-row GEMM that the
   linear / MoE layers dispatch to — the only native code the config-driven decoder families need, so a
   fresh checkout can serve one without compiling the rest.
 
@@ -36,12 +36,12 @@ SEQ_SOURCES = ["bindings_seq.cpp", "layernorm.hip", "hyper.hip",
                "attention_talking.hip", "attention_latent.hip",
                "attention_prefill.hip", "attention_decode.hip",
                "delta_rule.hip", "moe.hip", "moe_tiled.hip", "elementwise.hip",
-               "skinny_gemm.hip"]
+               "stream_gemm.hip"]
 CORE_SOURCES = ["bindings.cpp", "norm.hip", "elementwise.hip",
                 "attention_decode.hip", "attention_prefill.hip",
                 "attention_mla.hip", "mla_proj.hip", "moe.hip",
                 "moe_tiled.hip", "fp8.hip",
-                "gdn.hip", "int4.hip", "skinny_gemm.hip", "sampling.hip",
+                "gdn.hip", "int4.hip", "stream_gemm.hip", "sampling.hip",
                 "custom_ar.hip"]
 
 
