@@ -201,6 +201,16 @@ class Sampler(torch.nn.Module):
         return SamplerOutput(next_tokens, chosen, topv, topi)
 
 
+def upload(values, dtype, device) -> torch.Tensor:
+    """A list as a tensor on ``device``, without waiting for the device:
+    through pinned memory, which the allocator keeps until the copy is
+    done."""
+    t = torch.tensor(values, dtype=dtype)
+    if torch.device(device).type != "cuda":
+        return t.to(device)
+    return t.pin_memory().to(device, non_blocking=True)
+
+
 def build_sampling_metadata(items, device,
                             penalty_pool=None) -> SamplingMetadata:
     """Build metadata from the scheduled batch items (one row per item).
@@ -209,7 +219,7 @@ def build_sampling_metadata(items, device,
     slots (seeded from the prompt on first use, updated on-GPU after
     every sample); the host token-row fallback covers pool exhaustion."""
     temps, tps, tks, mps, pens, gens = [], [], [], [], [], []
-    rows: List[torch.Tensor] = []
+    rows = {}               # row -> token history (no mask slot)
     slots: List[int] = []
     sample_rows: List[int] = []
     max_lp = 0
@@ -254,13 +264,8 @@ def build_sampling_metadata(items, device,
                 slot = penalty_pool.ensure(it.seq)
             if slot < 0:
                 need_rows = True
-                rows.append(torch.tensor(it.seq.token_ids,
-                                         dtype=torch.long, device=device))
-            else:
-                rows.append(torch.empty(0, dtype=torch.long,
-                                        device=device))
-        else:
-            rows.append(torch.empty(0, dtype=torch.long, device=device))
+                rows[i] = torch.tensor(it.seq.token_ids, dtype=torch.long,
+                                       device=device)
         slots.append(slot)
         pres = getattr(sp, "presence_penalty", 0.0) or 0.0
         freq = getattr(sp, "frequency_penalty", 0.0) or 0.0
@@ -278,16 +283,20 @@ def build_sampling_metadata(items, device,
         else:
             gens.append(None)
     all_greedy = all(t == 0.0 for t in temps)
+    # a greedy batch reads none of the per-row numbers on the device
+    where = "cpu" if all_greedy and not any_pen else device
     return SamplingMetadata(
-        temperatures=torch.tensor(temps, dtype=torch.float32, device=device),
-        top_ps=torch.tensor(tps, dtype=torch.float32, device=device),
-        top_ks=torch.tensor(tks, dtype=torch.int32, device=device),
-        min_ps=torch.tensor(mps, dtype=torch.float32, device=device),
-        penalties=torch.tensor(pens, dtype=torch.float32, device=device),
+        temperatures=upload(temps, torch.float32, where),
+        top_ps=upload(tps, torch.float32, where),
+        top_ks=upload(tks, torch.int32, where),
+        min_ps=upload(mps, torch.float32, where),
+        penalties=upload(pens, torch.float32, where),
         all_greedy=all_greedy, any_penalty=any_pen,
-        token_id_rows=rows if need_rows else None,
+        token_id_rows=[rows.get(i, torch.empty(0, dtype=torch.long,
+                                               device=device))
+                       for i in range(len(slots))] if need_rows else None,
         penalty_pool=penalty_pool if any_pen else None,
-        penalty_slots=torch.tensor(slots, dtype=torch.long, device=device)
+        penalty_slots=upload(slots, torch.long, device)
         if any_pen else None,
         sample_rows=sample_rows,
         pres_freq_rows=pres_freq or None,

@@ -597,6 +597,17 @@ def fused_moe_int4(x: torch.Tensor, w13_c, w13_sb, w2_c, w2_sb,
 
 
 # --------------------------------------------------------------- sampling
+def resolve_tokens(tokens: torch.Tensor, ring: torch.Tensor) -> torch.Tensor:
+    """Negative token ids are places in ``ring`` (id -1 - i: its i-th
+    entry) of tokens sampled by an earlier step."""
+    if (tokens.is_cuda and tokens.dtype == torch.long
+            and tokens.is_contiguous() and has_moe_kernels()):
+        return _gpu_kernels().resolve_tokens(tokens, ring)
+    flat = ring.view(-1)
+    idx = (-tokens - 1).clamp_min(0)
+    return torch.where(tokens < 0, flat[idx], tokens)
+
+
 def topk_topp_filter(probs: torch.Tensor, top_ks: torch.Tensor,
                      top_ps: torch.Tensor,
                      min_ps: Optional[torch.Tensor] = None):

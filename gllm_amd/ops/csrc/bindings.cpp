@@ -17,6 +17,7 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_table, torch::Tensor seq_lens,
                             double scale, long sliding_window);
+torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
@@ -154,6 +155,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attention_decode", &window_attention_decode,
         "split-KV decode kernels with window + kept first + sink + gate; "
         "false = geometry not instantiated");
+  m.def("resolve_tokens", &resolve_tokens,
+        "token ids with places in the ring of sampled tokens");
   m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
   m.def("stream_gemm_gated", &stream_gemm_gated,
         "silu(x w_gate^T) * (x w_up^T) for at most 256 rows");

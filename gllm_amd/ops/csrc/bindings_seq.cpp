@@ -172,6 +172,7 @@ void sigmoid_group_topk(torch::Tensor weights, torch::Tensor ids,
                         long n_group, long keep, double scale);
 // shared with the full extension (stream_gemm.hip, moe.hip,
 // elementwise.hip): what ops.linear / FusedMoE dispatch to in bf16
+torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
@@ -275,6 +276,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tanh_rows", &tanh_rows, "tanh over strided rows");
   m.def("sigmoid_group_topk", &sigmoid_group_topk,
         "sigmoid router with correction and group limits");
+  m.def("resolve_tokens", &resolve_tokens,
+        "token ids with places in the ring of sampled tokens");
   m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
   m.def("stream_gemm_gated", &stream_gemm_gated,
         "silu(x w_gate^T) * (x w_up^T) for at most 256 rows");

@@ -713,3 +713,34 @@ void tanh_rows(torch::Tensor out, torch::Tensor x) {
 #undef RUN
   HIP_CHECK_KERNEL();
 }
+
+// ------------------------------------------------------------------
+// Token ids of a step that was launched before the one ahead of it ended:
+// a negative id -1 - i stands for entry i of the ring of sampled tokens.
+// One launch for a negation, a clamp, a gather, a comparison and a select.
+namespace {
+
+__global__ void resolve_tokens_kernel(long *__restrict__ out,
+                                      const long *__restrict__ tokens,
+                                      const long *__restrict__ ring, long n) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const long t = tokens[i];
+  out[i] = t < 0 ? ring[-t - 1] : t;
+}
+
+}  // namespace
+
+torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring) {
+  TORCH_CHECK(tokens.scalar_type() == at::kLong && tokens.is_contiguous() &&
+              ring.scalar_type() == at::kLong && ring.is_contiguous());
+  auto out = torch::empty_like(tokens);
+  const long n = tokens.numel();
+  if (n == 0) return out;
+  auto stream = at::cuda::getCurrentCUDAStream();
+  hipLaunchKernelGGL(resolve_tokens_kernel, dim3((n + 255) / 256), dim3(256),
+                     0, stream, out.data_ptr<long>(),
+                     tokens.data_ptr<long>(), ring.data_ptr<long>(), n);
+  HIP_CHECK_KERNEL();
+  return out;
+}

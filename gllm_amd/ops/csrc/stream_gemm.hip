@@ -285,8 +285,9 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
   }
 }
 
-// A workgroup per token, a thread per 8 columns of a head: 4 + 4 columns of
-// a rotated pair block, or 8 plain ones. PARTS: src is fp32 [S, M, N].
+// Workgroups along the columns of a token, a thread per 8 columns of a head:
+// 4 + 4 columns of a rotated pair block, or 8 plain ones. PARTS: src is fp32
+// [S, M, N].
 template <bool PARTS>
 __global__ __launch_bounds__(256) void qkv_finish_kernel(
     __hip_bfloat16 *__restrict__ q_out, __hip_bfloat16 *__restrict__ k_cache,
@@ -317,7 +318,8 @@ __global__ __launch_bounds__(256) void qkv_finish_kernel(
       for (int r = 0; r < 4; ++r) o[r] += __bfloat162float(bias[c + r]);
     }
   };
-  for (int i = threadIdx.x; i < (Hq + 2 * Hkv) * per; i += blockDim.x) {
+  const int i = blockIdx.y * 256 + threadIdx.x;
+  if (i < (Hq + 2 * Hkv) * per) {
     const int h = i / per, u = i % per;
     const bool turned = h < Hq + Hkv && u < rot / 8;
     // first columns of the two groups of four
@@ -573,7 +575,8 @@ torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
   if (M == 0) return q;
   auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(P)                                                               \
-  hipLaunchKernelGGL((qkv_finish_kernel<P>), dim3(M), dim3(256), 0, stream,  \
+  hipLaunchKernelGGL((qkv_finish_kernel<P>),                                 \
+                     dim3(M, (N / 8 + 255) / 256), dim3(256), 0, stream,     \
                      (__hip_bfloat16 *)q.data_ptr(),                         \
                      (__hip_bfloat16 *)k_cache.data_ptr(),                   \
                      (__hip_bfloat16 *)v_cache.data_ptr(), src.data_ptr(),   \

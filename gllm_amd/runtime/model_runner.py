@@ -13,7 +13,8 @@ from gllm_amd.config import EngineConfig
 from gllm_amd.core.kv_cache import (KVCacheSpec, MemoryManager,
                                     PrefixMemoryManager)
 from gllm_amd.core.scheduler import ScheduledBatch
-from gllm_amd.layers.sampler import Sampler, build_sampling_metadata
+from gllm_amd.layers.sampler import (Sampler, build_sampling_metadata,
+                                     upload)
 from gllm_amd.logger import logger
 from gllm_amd.models.loader import load_hf_config, load_model
 from gllm_amd.runtime.batch_builder import BatchBuilder
@@ -413,11 +414,9 @@ class ModelRunner:
         if getattr(self.model, "wants_state_tensors", False):
             # ragged state kernels read slots / carried-state flags on
             # the device
-            fctx.ssm_slots_t = torch.tensor(
-                slots, dtype=torch.long).to(self.device, non_blocking=True)
-            fctx.ssm_has_init_t = torch.tensor(
-                has_init, dtype=torch.int32).to(self.device,
-                                                non_blocking=True)
+            fctx.ssm_slots_t = upload(slots, torch.long, self.device)
+            fctx.ssm_has_init_t = upload(has_init, torch.int32,
+                                         self.device)
 
     def _attach_mm(self, batch, fctx) -> None:
         """Collect vision-embedding rows for this batch's prefill chunks
@@ -454,9 +453,8 @@ class ModelRunner:
     def resolve_tokens(self, tokens: torch.Tensor) -> torch.Tensor:
         """Replace negative placeholder ids with sampled tokens from the
         ring (overlap mode)."""
-        ring_flat = self.token_ring.view(-1)
-        idx = (-tokens - 1).clamp_min(0)
-        return torch.where(tokens < 0, ring_flat[idx], tokens)
+        from gllm_amd import ops
+        return ops.resolve_tokens(tokens, self.token_ring)
 
     def _prompt_logprobs(self, batch: ScheduledBatch, hidden, fctx):
         """Prompt logprobs (reference model_runner.py:1700-1807): for
