@@ -53,7 +53,8 @@ class Attention(nn.Module):
             q, fctx.k_caches[self.layer_idx], fctx.v_caches[self.layer_idx],
             fctx.block_table, fctx.seq_lens, fctx.query_start_loc,
             self.scale, max_query_len=fctx.max_query_len,
-            sliding_window=self.sliding_window)
+            sliding_window=self.sliding_window,
+            single_rows=fctx.single_rows)
         return out.reshape(T, -1)
 
 

@@ -167,7 +167,11 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
                     seq_lens: torch.Tensor, query_start_loc: torch.Tensor,
                     scale: float, max_query_len: int = 1,
                     out: Optional[torch.Tensor] = None,
-                    sliding_window: int = 0) -> torch.Tensor:
+                    sliding_window: int = 0,
+                    single_rows: int = 0) -> torch.Tensor:
+    """``single_rows``: how many of the sequences bring one query row
+    beside longer portions, if the caller knows (those then go through
+    the decode kernel)."""
     if q.is_cuda:
         kern = _gpu_kernels()
         if out is None:
@@ -175,11 +179,18 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
         if max_query_len == 1:
             kern.paged_attention_decode(
                 out, q, k_cache, v_cache, block_table, seq_lens, scale,
-                sliding_window)
+                sliding_window, None)
         else:
+            qsl = query_start_loc.int()
+            split = single_rows > 0 and kern.decode_rows_ok(
+                k_cache, v_cache, q.shape[1])
+            if split:
+                kern.paged_attention_decode(
+                    out, q, k_cache, v_cache, block_table, seq_lens, scale,
+                    sliding_window, qsl)
             kern.paged_attention_prefill(
-                out, q, k_cache, v_cache, block_table, seq_lens,
-                query_start_loc.int(), max_query_len, scale, sliding_window)
+                out, q, k_cache, v_cache, block_table, seq_lens, qsl,
+                max_query_len, scale, sliding_window, split)
         return out
     return torch_ref.paged_attention(q, k_cache, v_cache, block_table,
                                      seq_lens, query_start_loc, scale,

@@ -16,6 +16,11 @@
 //   they stand. At the end the waves join through LDS.
 //   Split partials written fp32 + LSE; merge kernel combines splits and
 //   converts to bf16 (reference semantics: merge_state / split-KV decode).
+//   One split writes the result itself.
+//   A mixed batch sends the sequences that bring one query row here: the
+//   prefill kernel would spend a 128-row tile per head on each (37 such
+//   rows of ~1024 keys, 40 heads, beside 4096 prompt tokens: 683 us a layer
+//   there, 43 + 5 us here, and 193 for the prompts that remain).
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -53,7 +58,14 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     int max_pages, int page_size, int num_kv_heads, int G, int Dr, int Dvr,
     float scale, int num_splits, long q_stride, int window, int keep_first,
     float softcap, const float *__restrict__ bias, int bias_len,
-    float temp_coef, int temp_every) {
+    float temp_coef, int temp_every,
+    // rows of a mixed batch: [B + 1]; sequences of other than one query row
+    // are left alone
+    const int *__restrict__ qsl,
+    // one split: the result itself, bf16 [rows, Hq * Dvr]
+    __hip_bfloat16 *__restrict__ out, long out_stride, int sink,
+    const float *__restrict__ sinks, const __hip_bfloat16 *__restrict__ gate,
+    long gate_stride) {
   constexpr int KT = D / 32, NT = DV / 16;
   constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
   constexpr int VROW = DV * 2;             // LDS row bytes
@@ -63,6 +75,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const int split = blockIdx.z;
   const int Hq = num_kv_heads * G;
   const int seq_len = seq_lens[b];
+  const int row = qsl ? qsl[b] : b;  // of q and of the result
+  if (qsl && qsl[b + 1] - row != 1) return;
   const int w_begin = (window > 0) ? max(0, seq_len - window) : 0;
   // this split's share of the visible keys, whole tiles
   const int tiles = (seq_len - w_begin + TK - 1) / TK;
@@ -82,7 +96,13 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const long lse0 = (long)split * gridDim.x * Hq + (long)b * Hq + kvh * G;
   if (t0 >= t1) {
     // empty split: publish -inf lse so the merge ignores it
-    if (tid < G) partial_lse[lse0 + tid] = -INFINITY;
+    if (out) {
+      for (int i = tid; i < G * Dvr; i += BLOCK)
+        out[row * out_stride + (long)kvh * G * Dvr + i] =
+            __float2bfloat16(0.f);
+    } else if (tid < G) {
+      partial_lse[lse0 + tid] = -INFINITY;
+    }
     return;
   }
   // a patch per wave: its V tile, later its output (as many bytes)
@@ -96,7 +116,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     qf[kt] = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
     if (l16 < G && kt * 32 + lhi * 8 < Dr)
       qf[kt] = *reinterpret_cast<const dec_bf8 *>(
-          q + (long)b * q_stride + (kvh * G + l16) * Dr + kt * 32 + lhi * 8);
+          q + (long)row * q_stride + (kvh * G + l16) * Dr + kt * 32 +
+          lhi * 8);
   }
   const int *bt = block_table + (long)b * max_pages;
   const shortx8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -109,7 +130,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   auto key_of = [&](int k0) { return min(k0 + (lane & 31), t1 - 1); };
   auto look_up = [&](int k0) { page_id = bt[key_of(k0) / page_size]; };
   auto load = [&](int k0) {
-    const int row = page_id * page_size + key_of(k0) % page_size;
+    const int krow = page_id * page_size + key_of(k0) % page_size;
     // a table entry per key of this lane (before K and V: loads return in
     // order)
     if (brow) {
@@ -124,7 +145,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     for (int f = 0; f < 2; ++f) {
       const __hip_bfloat16 *kp =
           k_cache +
-          ((long)__shfl(row, f * 16 + l16, 64) * num_kv_heads + kvh) * Dr +
+          ((long)__shfl(krow, f * 16 + l16, 64) * num_kv_heads + kvh) * Dr +
           lhi * 8;
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
@@ -137,7 +158,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     for (int j = 0; j < VU; ++j) {
       const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 8;
       const __hip_bfloat16 *vp =
-          v_cache + ((long)__shfl(row, r, 64) * num_kv_heads + kvh) * Dvr + c;
+          v_cache + ((long)__shfl(krow, r, 64) * num_kv_heads + kvh) * Dvr + c;
       vn[j] = c < Dvr ? __builtin_nontemporal_load(
                             reinterpret_cast<const shortx8 *>(vp))
                       : zero;
@@ -264,6 +285,18 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
       l += e * s_l[w][h];
       acc += e * reinterpret_cast<const float *>(patch[w])[at];
     }
+    if (out) {  // the only split
+      if (sinks || sink)
+        l += __builtin_amdgcn_exp2f(
+            (sinks ? sinks[kvh * G + h] : 0.f) * LOG2E - m);
+      const long col = (long)(kvh * G + h) * Dvr + d;
+      float res = acc / l;
+      if (gate)
+        res *= 1.f / (1.f + __expf(-__bfloat162float(
+                                 gate[row * gate_stride + col])));
+      out[row * out_stride + col] = __float2bfloat16(res);
+      continue;
+    }
     partial_out[(lse0 + h) * Dvr + d] = acc / l;
     if (d == 0) partial_lse[lse0 + h] = m / LOG2E + __logf(l);
   }
@@ -278,8 +311,10 @@ __global__ void decode_merge_kernel(
     const float *__restrict__ partial_lse,  // [S, B, Hq]
     int num_splits, int Hq, int sink,
     const __hip_bfloat16 *__restrict__ gate, long gate_stride,
-    const float *__restrict__ sinks) {
+    const float *__restrict__ sinks, const int *__restrict__ qsl) {
   const int b = blockIdx.x, h = blockIdx.y;
+  const int row = qsl ? qsl[b] : b;
+  if (qsl && qsl[b + 1] - row != 1) return;
   const int d = threadIdx.x, D = blockDim.x;
   const int B = gridDim.x;
   // sink: one more "partial" with lse 0 (or the head's learned score)
@@ -300,10 +335,10 @@ __global__ void decode_merge_kernel(
   float res = denom > 0.f ? o / denom : 0.f;
   if (gate != nullptr) {
     const float z =
-        __bfloat162float(gate[(long)b * gate_stride + (long)h * D + d]);
+        __bfloat162float(gate[(long)row * gate_stride + (long)h * D + d]);
     res *= 1.f / (1.f + __expf(-z));
   }
-  out[(long)b * out_stride + (long)h * D + d] = __float2bfloat16(res);
+  out[(long)row * out_stride + (long)h * D + d] = __float2bfloat16(res);
 }
 
 bool decode_shape_ok(const torch::Tensor &k_cache,
@@ -325,8 +360,9 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                    const void *gate = nullptr, long gate_stride = 0,
                    const float *sinks = nullptr, float softcap = 0.f,
                    const float *bias = nullptr, int bias_len = 0,
-                   float temp_coef = 0.f, int temp_every = 0) {
-  const int B = q.size(0), Hkv = k_cache.size(2), Hq = Hkv * G;
+                   float temp_coef = 0.f, int temp_every = 0,
+                   const int *qsl = nullptr) {
+  const int B = seq_lens.size(0), Hkv = k_cache.size(2), Hq = Hkv * G;
   const int D = k_cache.size(3), Dv = v_cache.size(3);
   // the longest sequence the pool can hold bounds the useful splits; the
   // count depends on the batch size only (a captured launch serves every
@@ -336,21 +372,34 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
     const char *e = getenv("GLLM_DECODE_SPLITS");
     return e ? atoi(e) : 0;
   }();
+  // (two workgroups fit a CU; requests are unequal, so twice that many even
+  // out better: 64 requests of 512 to 1536 keys, 8 heads, 62 us in two
+  // splits, 69 us in one; 24 of 2700 to 8100 115 us in eight, 121 in four)
   int splits = 1;
-  while (splits < 16 && B * Hkv * splits < 512 &&
+  while (splits < 16 && B * Hkv * splits < 1024 &&
          splits * 2 <= (max_seq_len + 127) / 128)
     splits *= 2;
   if (splits_env > 0) splits = splits_env;
   auto opts = q.options().dtype(at::kFloat);
   // + 1: the kept-first segment of a windowed layer
   const int zdim = splits + ((keep_first > 0 && window > 0) ? 1 : 0);
-  auto partial = torch::empty({zdim, B, Hq, Dv}, opts);
-  auto lse = torch::empty({zdim, B, Hq}, opts);
+  const long out_stride =
+      out.dim() == 2 ? (long)out.stride(0) : (long)Hq * Dv;
+  // one split writes the result itself
+  torch::Tensor partial, lse;
+  float *po = nullptr, *pl = nullptr;
+  auto *direct = (__hip_bfloat16 *)out.data_ptr();
+  if (zdim > 1) {
+    partial = torch::empty({zdim, B, Hq, Dv}, opts);
+    lse = torch::empty({zdim, B, Hq}, opts);
+    po = partial.data_ptr<float>();
+    pl = lse.data_ptr<float>();
+    direct = nullptr;
+  }
   auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(DT, DVT)                                                         \
   hipLaunchKernelGGL((paged_decode_kernel<DT, DVT>), dim3(B, Hkv, zdim),     \
-                     dim3(BLOCK), 0, stream, partial.data_ptr<float>(),      \
-                     lse.data_ptr<float>(),                                  \
+                     dim3(BLOCK), 0, stream, po, pl,                         \
                      (const __hip_bfloat16 *)q.data_ptr(),                   \
                      (const __hip_bfloat16 *)k_cache.data_ptr(),             \
                      (const __hip_bfloat16 *)v_cache.data_ptr(),             \
@@ -358,17 +407,17 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      (int)block_table.stride(0), (int)k_cache.size(1), Hkv,  \
                      G, D, Dv, scale, splits, (long)q.stride(0), window,     \
                      keep_first, softcap, bias, bias_len, temp_coef,         \
-                     temp_every)
+                     temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
+                     sinks, (const __hip_bfloat16 *)gate, gate_stride)
   if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
 #undef RUN
   HIP_CHECK_KERNEL();
+  if (zdim == 1) return;
   hipLaunchKernelGGL(decode_merge_kernel, dim3(B, Hq), dim3(Dv), 0, stream,
-                     (__hip_bfloat16 *)out.data_ptr(),
-                     out.dim() == 2 ? (long)out.stride(0) : (long)Hq * Dv,
-                     partial.data_ptr<float>(), lse.data_ptr<float>(), zdim,
-                     Hq, sink ? 1 : 0, (const __hip_bfloat16 *)gate,
-                     gate_stride, sinks);
+                     (__hip_bfloat16 *)out.data_ptr(), out_stride, po, pl,
+                     zdim, Hq, sink ? 1 : 0, (const __hip_bfloat16 *)gate,
+                     gate_stride, sinks, qsl);
   HIP_CHECK_KERNEL();
 }
 
@@ -377,7 +426,8 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_table, torch::Tensor seq_lens,
-                            double scale, long sliding_window) {
+                            double scale, long sliding_window,
+                            c10::optional<torch::Tensor> query_start_loc) {
   TORCH_CHECK(q.scalar_type() == at::kBFloat16, "decode attn: bf16 only");
   TORCH_CHECK(out.is_contiguous());
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2),
@@ -391,8 +441,28 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
               decode_shape_ok(k_cache, v_cache, Hq / Hkv),
               "paged_attention_decode: unsupported head_dim=", q.size(2),
               " group=", Hq / Hkv);
+  const int *qsl = nullptr;
+  if (query_start_loc.has_value()) {
+    TORCH_CHECK(query_start_loc->scalar_type() == at::kInt &&
+                query_start_loc->is_contiguous() &&
+                query_start_loc->numel() == seq_lens.numel() + 1);
+    qsl = query_start_loc->data_ptr<int>();
+  } else {
+    TORCH_CHECK(seq_lens.numel() == q.size(0), "one query row per sequence");
+  }
+  TORCH_CHECK(block_table.size(0) >= seq_lens.numel());
   launch_decode(out, q, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
-                (float)scale, (int)sliding_window);
+                (float)scale, (int)sliding_window, 0, false, nullptr, 0,
+                nullptr, 0.f, nullptr, 0, 0.f, 0, qsl);
+}
+
+// whether the decode kernel takes heads of this geometry (a mixed batch
+// sends its one-row sequences there)
+bool decode_rows_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq) {
+  const long Hkv = k_cache.size(2);
+  return k_cache.is_contiguous() && v_cache.is_contiguous() &&
+         Hkv > 0 && Hq % Hkv == 0 &&
+         decode_shape_ok(k_cache, v_cache, Hq / Hkv);
 }
 
 // Windowed-sink form of the split-KV decode kernels: one decode token per

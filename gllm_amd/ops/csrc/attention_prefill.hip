@@ -83,7 +83,9 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_prefill_kernel(
     // EXT: head sizes; bias [Hq, bias_len] (nullptr: none), entry
     // min(i - j, bias_len - 1) added to the scaled score
     int Dr_, int Dvr_, const float *__restrict__ bias, int bias_len,
-    float temp_coef, int temp_every, int vec_out) {
+    float temp_coef, int temp_every, int vec_out,
+    // sequences of fewer query rows are served elsewhere
+    int min_rows) {
   const int Dr = EXT ? Dr_ : D, Dvr = EXT ? Dvr_ : DV;
   const int tile = blockIdx.x;
   const int b = blockIdx.y;
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_prefill_kernel(
 
   const int q_start = qsl[b];
   const int q_len = qsl[b + 1] - q_start;
-  if (tile * BQ >= q_len) return;
+  if (tile * BQ >= q_len || q_len < min_rows) return;
   const int seq_len = seq_lens[b];
   const int past = seq_len - q_len;
 
@@ -444,7 +446,7 @@ void launch_prefill(torch::Tensor &out, torch::Tensor &q, int Hq,
                     long gate_stride, const float *sinks = nullptr,
                     float softcap = 0.f, const float *bias = nullptr,
                     int bias_len = 0, float temp_coef = 0.f,
-                    int temp_every = 0) {
+                    int temp_every = 0, int min_rows = 1) {
   const int Hkv = k_cache.size(2);
   const int D = k_cache.size(3), Dv = v_cache.size(3);
   const int B = seq_lens.size(0);
@@ -477,7 +479,7 @@ void launch_prefill(torch::Tensor &out, torch::Tensor &q, int Hq,
                      (int)keep_first, sink ? 1 : 0,                          \
                      (const __hip_bfloat16 *)gate, gate_stride, sinks,       \
                      softcap, D, Dv, bias, bias_len, temp_coef, temp_every,  \
-                     vec_out)
+                     vec_out, min_rows)
   if (!ext && D == 128) RUN(128, 128, false);
   else if (!ext && D == 64) RUN(64, 64, false);
   else if (D % 8 == 0 && Dv % 8 == 0 && D <= 128 && Dv <= 128) {
@@ -499,7 +501,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor seq_lens,
                              torch::Tensor query_start_loc,
                              long max_query_len, double scale,
-                             long sliding_window) {
+                             long sliding_window, bool skip_single) {
   TORCH_CHECK(q.scalar_type() == at::kBFloat16, "prefill attn: bf16 only");
   TORCH_CHECK(out.is_contiguous());
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == q.size(2),
@@ -507,7 +509,8 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
   if (q.size(0) == 0) return;
   launch_prefill(out, q, q.size(1), q.stride(0), k_cache, v_cache,
                  block_table, seq_lens, query_start_loc, max_query_len,
-                 scale, sliding_window, 0, false, nullptr, 0);
+                 scale, sliding_window, 0, false, nullptr, 0, nullptr, 0.f,
+                 nullptr, 0, 0.f, 0, skip_single ? 2 : 1);
 }
 
 // Windowed-sink form of the same MFMA kernel: q [T, H*D] (row-strided

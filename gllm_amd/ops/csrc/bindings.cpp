@@ -16,7 +16,9 @@ void reshape_and_cache(torch::Tensor k, torch::Tensor v,
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             torch::Tensor k_cache, torch::Tensor v_cache,
                             torch::Tensor block_table, torch::Tensor seq_lens,
-                            double scale, long sliding_window);
+                            double scale, long sliding_window,
+                            c10::optional<torch::Tensor> query_start_loc);
+bool decode_rows_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq);
 torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
@@ -35,7 +37,7 @@ void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor seq_lens,
                              torch::Tensor query_start_loc,
                              long max_query_len, double scale,
-                             long sliding_window);
+                             long sliding_window, bool skip_single);
 void window_attention_mfma(torch::Tensor out, torch::Tensor q,
                            c10::optional<torch::Tensor> gate,
                            torch::Tensor k_cache, torch::Tensor v_cache,
@@ -148,6 +150,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "scatter K/V into paged cache");
   m.def("paged_attention_decode", &paged_attention_decode,
         "split-KV paged decode attention");
+  m.def("decode_rows_ok", &decode_rows_ok,
+        "the decode kernel takes these heads");
   m.def("paged_attention_prefill", &paged_attention_prefill,
         "varlen MFMA paged prefill attention");
   m.def("window_attention_mfma", &window_attention_mfma,

@@ -91,6 +91,8 @@ class BatchBuilder:
             v_caches=v_caches,
         )
         fctx.has_placeholders = has_ph
+        if max_q > 1:
+            fctx.single_rows = int((lens == 1).sum())
         fctx.seq_lens_cpu = seq_lens.tolist()
         fctx.query_start_loc_cpu = qsl.tolist()
         if need_logits:

@@ -22,6 +22,9 @@ class ForwardContext:
     query_start_loc: torch.Tensor    # [B+1] int32
     max_query_len: int               # 1 => pure decode
     max_seq_len: int
+    # sequences of this batch that bring one query row beside portions of
+    # more (0: unknown or none)
+    single_rows: int = dataclasses.field(default=0, kw_only=True)
     # --- KV cache (this stage's layers) ---
     k_caches: List[torch.Tensor]     # per local layer [pages, page, Hkv, D]
     v_caches: List[torch.Tensor]
