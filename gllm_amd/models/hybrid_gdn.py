@@ -27,6 +27,7 @@ from gllm_amd.layers.layernorm import GemmaRMSNorm, RMSNorm
 from gllm_amd.layers.linear import (ColumnParallelLinear,
                                     MergedColumnParallelLinear,
                                     QKVParallelLinear, RowParallelLinear)
+from gllm_amd.layers.recurrent import state_rows
 from gllm_amd.layers.rotary import get_rope
 from gllm_amd.models.llama_family import DenseMLP
 from gllm_amd.ops import gdn_ref
@@ -143,11 +144,24 @@ class GatedDeltaNet(nn.Module):
         ba = self.in_proj_ba(hidden)
         q, k, v, z = qkvz.split([k_tp, k_tp, v_tp, v_tp], dim=-1)
         b, a = ba.split([self.tp_v, self.tp_v], dim=-1)
-        mixed = torch.cat([q, k, v], dim=-1)         # [T, conv_dim/tp]
 
         pool = fctx.ssm_pool
         conv_states = pool.conv_state[self.ssm_layer_id]
         ssm_states = pool.ssm_state[self.ssm_layer_id]
+        from gllm_amd import ops as _ops
+        if _ops.gdn_rows_ok(qkvz, ba, self.conv1d_weight, conv_states,
+                            ssm_states, self.norm_weight, self.head_k_dim,
+                            self.head_v_dim):
+            slots_t, init_t = state_rows(fctx, T, hidden.device)
+            carried = fctx.ssm_slots_dev is not None or (
+                fctx.max_query_len == 1 and T == len(fctx.ssm_slots)
+                and all(fctx.ssm_has_init))
+            return _ops.gdn_rows(
+                qkvz, ba, self.conv1d_weight, self.A_log, self.dt_bias,
+                self.norm_weight, self.eps, conv_states, ssm_states, slots_t,
+                init_t, fctx.query_start_loc, fctx.max_query_len, carried,
+                self.tp_k_heads, self.scale)
+        mixed = torch.cat([q, k, v], dim=-1)         # [T, conv_dim/tp]
         g_all, beta_all = gdn_ref.gdn_gating(self.A_log, a, b, self.dt_bias)
 
         out_core = torch.empty(T, self.tp_v, self.head_v_dim,
@@ -159,7 +173,6 @@ class GatedDeltaNet(nn.Module):
         # single-token step with carried state -> one conv-update launch
         # + one fused recurrent launch for the whole batch (the per-seq
         # loop below costs ~8 launches PER SEQUENCE)
-        from gllm_amd import ops as _ops
         graph_path = fctx.ssm_slots_dev is not None
         if (hidden.is_cuda and self.head_k_dim == 128
                 and self.conv1d_weight.shape[1] == 4
@@ -382,6 +395,9 @@ class Qwen3_5ForCausalLM(nn.Module):
     reference qwen3_5_moe.py) is config-driven — layers with
     ``num_experts > 1`` (minus ``mlp_only_layers`` /
     ``decoder_sparse_step`` exceptions) get a routed MoE MLP."""
+
+    # the ragged state kernels read slots and flags on the device
+    wants_state_tensors = True
 
     @staticmethod
     def _is_sparse_layer(cfg, global_idx: int) -> bool:

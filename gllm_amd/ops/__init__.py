@@ -512,11 +512,10 @@ def gdn_decode(qn: torch.Tensor, kn: torch.Tensor, v: torch.Tensor,
 def gdn_chunk_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       g: torch.Tensor, beta: torch.Tensor,
                       states: torch.Tensor, scale: float) -> torch.Tensor:
-    """Fused WY chunk-parallel gated delta rule over a padded batch
-    (one launch per layer; replaces ~25 torch launches per 256-token
-    chunk). q/k [B, T, Hk, 128], v [B, T, Hv, 128], g/beta [B, T, Hv]
-    fp32, states [B, Hv, 128, 128] fp32 updated IN PLACE. Falls back
-    to the torch oracle off-GPU or for non-128 head dims."""
+    """WY chunk-parallel gated delta rule over a padded batch. q/k [B, T,
+    Hk, 128], v [B, T, Hv, 128], g/beta [B, T, Hv] fp32, states [B, Hv,
+    128, 128] fp32 updated IN PLACE. Falls back to the torch oracle
+    off-GPU or for non-128 head dims."""
     B, T, Hk, Dk = q.shape
     Hv, Dv = v.shape[2], v.shape[3]
     if not (q.is_cuda and has_kernels() and Dk == 128 and Dv == 128
@@ -524,22 +523,54 @@ def gdn_chunk_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         from gllm_amd.ops import gdn_ref
         return gdn_ref.gated_delta_rule_chunked_batched(
             q, k, v, g, beta, scale, states)
-    Tp = (T + 63) // 64 * 64
-    if Tp != T:  # zero padding rows carry g = 0, beta = 0 -> inert
-        pad = (0, 0, 0, 0, 0, Tp - T)
-        q = torch.nn.functional.pad(q, pad)
-        k = torch.nn.functional.pad(k, pad)
-        v = torch.nn.functional.pad(v, pad)
-        g = torch.nn.functional.pad(g, (0, 0, 0, Tp - T))
-        beta = torch.nn.functional.pad(beta, (0, 0, 0, Tp - T))
-    o = torch.empty(B, Tp, Hv, Dv, dtype=torch.bfloat16, device=q.device)
+    o = torch.empty(B, T, Hv, Dv, dtype=torch.bfloat16, device=q.device)
     _gpu_kernels().gdn_chunk_prefill(
         o, q.to(torch.bfloat16).contiguous(),
         k.to(torch.bfloat16).contiguous(),
         v.to(torch.bfloat16).contiguous(),
         g.float().contiguous(), beta.float().contiguous(),
         states, float(scale))
-    return o[:, :T]
+    return o
+
+
+def gdn_rows_ok(qkvz: torch.Tensor, ba: torch.Tensor, conv_w: torch.Tensor,
+                conv_state: torch.Tensor, state: torch.Tensor,
+                norm_w: torch.Tensor, Dk: int, Dv: int) -> bool:
+    """Whether ``gdn_rows`` takes this layer: bf16 on the GPU, heads of
+    128, up to 8 taps."""
+    return (qkvz.is_cuda and has_kernels() and _load_seq_kernels() is not None
+            and all(t.dtype == torch.bfloat16 for t in
+                    (qkvz, ba, conv_w, conv_state, norm_w))
+            and state.dtype == torch.float32 and state.is_contiguous()
+            and conv_state.is_contiguous() and conv_w.is_contiguous()
+            and Dk == 128 and Dv == 128 and conv_w.shape[1] <= 8
+            and qkvz.stride(1) == 1 and qkvz.stride(0) % 8 == 0
+            and qkvz.data_ptr() % 16 == 0 and norm_w.data_ptr() % 16 == 0)
+
+
+def gdn_rows(qkvz: torch.Tensor, ba: torch.Tensor, conv_w: torch.Tensor,
+             A_log: torch.Tensor, dt_bias: torch.Tensor,
+             norm_w: torch.Tensor, eps: float, conv_state: torch.Tensor,
+             state: torch.Tensor, slots: torch.Tensor,
+             has_init: torch.Tensor, query_start_loc: torch.Tensor,
+             max_query_len: int, carried: bool, Hk: int,
+             scale: float) -> torch.Tensor:
+    """A gated-delta layer between its projections over a ragged batch:
+    short convolution, unit q and k, gates, recurrence (state in place),
+    gated norm. qkvz rows are q | k | v | z, ba rows b | a; ``carried``:
+    every sequence is one token on carried state. Returns [T, Hv * 128]."""
+    k = _gpu_kernels()
+    conv_dim = conv_w.shape[0]
+    conv = causal_conv_silu(qkvz[:, :conv_dim], conv_w, conv_state, slots,
+                            has_init, query_start_loc,
+                            max_query_len=max_query_len)
+    A, dt = A_log.float(), dt_bias.float()
+    if carried:
+        o = k.gdn_step(conv, ba, A, dt, state, slots, Hk, scale)
+    else:
+        o = k.gdn_varlen(conv, ba, A, dt, state, slots, has_init,
+                         query_start_loc, Hk, max_query_len, scale)
+    return k.gdn_gate(o, qkvz[:, conv_dim:], norm_w, eps)
 
 
 def rmsnorm_gated(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,

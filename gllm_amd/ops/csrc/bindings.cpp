@@ -117,6 +117,17 @@ void gdn_conv_update(torch::Tensor out, torch::Tensor x,
 void gdn_chunk_prefill(torch::Tensor o, torch::Tensor q, torch::Tensor k,
                        torch::Tensor v, torch::Tensor g, torch::Tensor beta,
                        torch::Tensor states, double scale);
+torch::Tensor gdn_varlen(torch::Tensor conv, torch::Tensor ba,
+                         torch::Tensor A_log, torch::Tensor dt_bias,
+                         torch::Tensor states, torch::Tensor slots,
+                         torch::Tensor has_init, torch::Tensor qsl, long Hk,
+                         long max_len, double scale);
+torch::Tensor gdn_step(torch::Tensor conv, torch::Tensor ba,
+                       torch::Tensor A_log, torch::Tensor dt_bias,
+                       torch::Tensor states, torch::Tensor slots, long Hk,
+                       double scale);
+torch::Tensor gdn_gate(torch::Tensor o, torch::Tensor z, torch::Tensor w,
+                       double eps);
 void gdn_decode(torch::Tensor o, torch::Tensor qn, torch::Tensor kn,
                 torch::Tensor v, torch::Tensor g, torch::Tensor beta,
                 torch::Tensor state, torch::Tensor slots);
@@ -199,6 +210,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "batched causal-conv1d decode step w/ state roll");
   m.def("gdn_chunk_prefill", &gdn_chunk_prefill,
         "fused WY chunk-parallel gated delta rule prefill");
+  m.def("gdn_varlen", &gdn_varlen,
+        "ragged chunk-parallel gated delta rule");
+  m.def("gdn_step", &gdn_step,
+        "one token per sequence from the convolved projection");
+  m.def("gdn_gate", &gdn_gate, "rmsnorm(o) * w * silu(z) per head");
   m.def("gdn_decode", &gdn_decode,
         "batched fused recurrent gated-delta-rule decode step");
   m.def("rmsnorm_gated", &rmsnorm_gated, "rmsnorm(x)*w*silu(z)");
