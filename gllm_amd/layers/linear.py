@@ -54,21 +54,12 @@ class LinearBase(nn.Module):
         resident cache — prefill is compute-bound and bursty). CPU and
         int4 keep the dequant path."""
         w = self.weight
+        if not self.is_plain and self._native(x):
+            op = self._few_rows(x)
+            if op is not None:
+                return ops.quant_rows(x, op, self._bias32())
+            return self._prefill_quant(x, bias)
         if self.fp8_block is not None:
-            native = (x.is_cuda and x.dim() == 2
-                      and x.dtype == torch.bfloat16
-                      and x.shape[1] % 128 == 0
-                      and self.fp8_block == (128, 128)
-                      and ops.has_kernels())
-            if native:
-                # measured crossover (profiles/): the weight-streaming
-                # skinny wins only at M <= 64; above that the bf16
-                # shadow + library GEMM is faster (M=256 gate_up:
-                # 329 us skinny vs ~103 us library)
-                if x.shape[0] <= 64:
-                    return ops.fp8_linear(x, w, self.weight_scale_inv,
-                                          self._bias32())
-                return self._prefill_quant(x, bias)
             from gllm_amd.layers.quantization.fp8 import dequant_block_fp8
             if x.is_cuda:
                 wd = dequant_block_fp8(w, self.weight_scale_inv,
@@ -80,25 +71,6 @@ class LinearBase(nn.Module):
                     x.dtype).to(x.device)
             w = self._w_dq
         elif self.int4_cfg is not None:
-            native = (x.is_cuda and x.dim() == 2
-                      and x.dtype == torch.bfloat16
-                      and x.shape[1] % 256 == 0
-                      and self.int4_cfg[1] == 128 and ops.has_kernels())
-            if native:
-                # packed-nibble streaming GEMMs (one-time canonical
-                # repack; sbt = transposed (scale,bias) for the skinny)
-                if getattr(self, "_i4_canon", None) is None:
-                    from gllm_amd.layers.quantization.int4 import \
-                        repack_canonical
-                    wq4, sb, grp = repack_canonical(self)
-                    sbt = sb.permute(1, 2, 0).contiguous()
-                    self._i4_canon = (wq4.to(x.device), sb.to(x.device),
-                                      sbt.to(x.device), grp)
-                wq4, sb, sbt, grp = self._i4_canon
-                if x.shape[0] <= 64:
-                    return ops.int4_linear(x, wq4, sbt, grp,
-                                           self._bias32())
-                return self._prefill_quant(x, bias)
             if x.is_cuda:
                 from gllm_amd.layers.quantization.int4 import dequant_layer
                 return ops.linear(x, dequant_layer(self, x.dtype), bias)
@@ -112,6 +84,40 @@ class LinearBase(nn.Module):
     def is_plain(self) -> bool:
         """Unquantized weights (the fused few-row forms take them)."""
         return self.fp8_block is None and self.int4_cfg is None
+
+    def _native(self, x) -> bool:
+        """Whether the quantized weight is used as it is stored."""
+        if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
+                and ops.has_kernels()):
+            return False
+        if self.fp8_block is not None:
+            return self.fp8_block == (128, 128) and x.shape[1] % 128 == 0
+        return self.int4_cfg[1] == 128 and x.shape[1] % 256 == 0
+
+    def _few_rows(self, x):
+        """The quantized weight as ``ops.quant_rows`` takes it, None above
+        64 rows: there the bf16 copy and the library's product are the
+        faster ones (256 rows, gate_up: 103 us against 329)."""
+        if self.int4_cfg is not None:
+            # one-time canonical repack; sbt = transposed (scale, bias)
+            if getattr(self, "_i4_canon", None) is None:
+                from gllm_amd.layers.quantization.int4 import \
+                    repack_canonical
+                wq4, sb, grp = repack_canonical(self)
+                sbt = sb.permute(1, 2, 0).contiguous()
+                self._i4_canon = (wq4.to(x.device), sb.to(x.device),
+                                  sbt.to(x.device), grp)
+            wq4, _, sbt, _ = self._i4_canon
+            return ("int4", wq4, sbt) if x.shape[0] <= 64 else None
+        return ("fp8", self.weight, self.weight_scale_inv) \
+            if x.shape[0] <= 64 else None
+
+    def _fused_op(self, x):
+        """``_few_rows`` where a fused form may take this layer, else
+        None."""
+        if self.is_plain or x.shape[0] == 0 or not self._native(x):
+            return None
+        return self._few_rows(x)
 
     def _bias32(self):
         """fp32 bias cached once (the skinny epilogues add fp32)."""
@@ -236,6 +242,10 @@ class MergedColumnParallelLinear(LinearBase):
         if self.is_plain and self.bias is None and x.is_cuda \
                 and x.dim() == 2:
             return ops.linear_silu(x, self.weight)
+        if self.bias is None:
+            op = self._fused_op(x)
+            if op is not None:
+                return ops.quant_silu(x, op)
         return ops.silu_and_mul(self(x))
 
 
@@ -313,6 +323,18 @@ class QKVParallelLinear(LinearBase):
         """The merged q | k | v rows."""
         return self._gemm(x, self.bias)
 
+    def parts(self, x):
+        """The fp32 parts of the merged rows without the bias, for
+        ``ops.qkv_rope_cache``, which adds it; None where ``project`` is
+        the better one."""
+        if self.is_plain:
+            return ops.qkv_parts(x, self.weight, self.bias)
+        op = self._fused_op(x)
+        if op is None or not ops.plain_bias(
+                self.bias, self.q_size + 2 * self.kv_size):
+            return None
+        return ops.quant_parts(x, op)
+
     def forward(self, x):
         return self.project(x).split(
             [self.q_size, self.kv_size, self.kv_size], dim=-1)
@@ -343,11 +365,15 @@ class RowParallelLinear(LinearBase):
     def forward_add_norm(self, x, residual, norm):
         """(norm(residual + self(x)), that sum): one kernel behind the
         product where nothing has to be reduced over ranks first."""
-        if (self.is_plain and self.bias is None and x.is_cuda
-                and x.dim() == 2
+        if (self.bias is None and x.is_cuda and x.dim() == 2
                 and (get_tp_size() == 1 or not self.reduce_results)):
-            return ops.linear_add_rmsnorm(x, self.weight, residual,
-                                          norm.scale(), norm.eps)
+            if self.is_plain:
+                return ops.linear_add_rmsnorm(x, self.weight, residual,
+                                              norm.scale(), norm.eps)
+            op = self._fused_op(x)
+            if op is not None:
+                return ops.quant_add_rmsnorm(x, op, residual, norm.scale(),
+                                             norm.eps)
         return norm(self(x), residual)
 
     def forward(self, x):

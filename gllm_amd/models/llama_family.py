@@ -91,13 +91,13 @@ class DenseAttention(nn.Module):
             if (hidden.dtype == torch.bfloat16 and ops.qkv_rope_cache_ok(
                     k_cache, v_cache, rope.cos_sin_cache, rope.is_neox)):
                 proj, bias = self.qkv_proj, self.qkv_proj.bias
-                src = ops.qkv_parts(hidden, proj.weight, bias) \
-                    if proj.is_plain else None
+                src = proj.parts(hidden)
                 if src is None:
                     src, bias = proj.project(hidden), None
                 q = ops.qkv_rope_cache(src, bias, positions,
                                        rope.cos_sin_cache, k_cache, v_cache,
-                                       fctx.slot_mapping, attn.num_heads)
+                                       fctx.slot_mapping, attn.num_heads,
+                                       rounded=proj.fp8_block is not None)
                 return attn.attend(q, fctx)
         q, k, v = self.qkv_proj(hidden)
         if self.qk_norm:

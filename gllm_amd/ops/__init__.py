@@ -349,33 +349,83 @@ def per_token_group_quant_fp8(x: torch.Tensor, group: int = 128,
     return q, scales
 
 
-_FP8_WS: dict = {}
+def _quant_splitk(N: int, K: int, bk: int) -> int:
+    """Parts along K of an fp8 product: the deepest power of two that
+    leaves at least 8 stages of ``bk`` per part and at most 1024
+    workgroups of 64 columns (us, 64 rows: 7168 x 5120 4 parts 16.7, 3
+    17.6; 4096 x 14336 8 parts 18.3; 5120 x 27648 8 parts 38, 10 38)."""
+    n_wg = -(-N // 64)
+    s = 1
+    while (s < 16 and n_wg * (s * 2) <= 1024
+           and (K // bk) // (s * 2) >= 8):
+        s *= 2
+    k_slice = ((-(-K // s)) + bk - 1) // bk * bk
+    return -(-K // k_slice)
+
+
+def _quant_gemm(x: torch.Tensor, kind: str, w: torch.Tensor,
+                ws: torch.Tensor, bias, form: int) -> torch.Tensor:
+    splits = _quant_splitk(w.shape[0], x.shape[1], 128) \
+        if kind == "fp8" else 0
+    return _gpu_kernels().quant_gemm(*_quant_operands(x, kind, w, ws), bias,
+                                     form, splits)
+
+
+def _quant_operands(x: torch.Tensor, kind: str, w: torch.Tensor,
+                    ws: torch.Tensor):
+    """(rows, their scales, weight bytes, weight scales) as
+    csrc/quant_gemm.hip takes them; ``kind`` "fp8" (w [N, K] e4m3, ws fp32
+    per 128 x 128 block; the rows are quantized per 128 columns) or "int4"
+    (w [N, K / 2] packed, ws [K / 128, 2, N])."""
+    if kind == "fp8":
+        xq, _, xs = per_token_group_quant_fp8(x, transposed=True)
+        return xq.view(torch.uint8), xs, w.view(torch.uint8), ws.contiguous()
+    x = x.contiguous()
+    return (x.clone() if x.data_ptr() % 16 else x), None, w, ws
+
+
+def quant_rows(x: torch.Tensor, op, bias: Optional[torch.Tensor] = None):
+    """x @ dequant(w).T (+ bias) for at most 256 rows; ``op`` = (kind, w,
+    scales)."""
+    return _quant_gemm(
+        x, *op, bias.float().contiguous() if bias is not None else None, 1)
+
+
+def quant_silu(x: torch.Tensor, op) -> torch.Tensor:
+    """silu(x @ w_gate.T) * (x @ w_up.T), w = gate rows over up rows. The
+    one-kernel form cannot split K, so it is for weights with tiles enough
+    without (28672 x 4096, 1 row, int4: 25 us against 20 + the second
+    kernel's 5)."""
+    N = op[1].shape[0]
+    if N % 32 == 0 and N >= 16384:
+        return _quant_gemm(x, *op, None, 0)
+    return silu_and_mul(quant_rows(x, op))
+
+
+def quant_parts(x: torch.Tensor, op) -> Optional[torch.Tensor]:
+    """The fp32 parts [S, M, N] of x @ dequant(w).T, or None for an N that
+    their readers do not take."""
+    if op[1].shape[0] % 8:
+        return None
+    return _quant_gemm(x, *op, None, 2)
+
+
+def quant_add_rmsnorm(x: torch.Tensor, op, residual: torch.Tensor,
+                      norm_w: torch.Tensor, eps: float):
+    """residual += x @ dequant(w).T; (rmsnorm(residual), residual)."""
+    if _norm_parts_ok(op[1].shape[0], residual, norm_w):
+        return _gpu_kernels().parts_add_norm(quant_parts(x, op), residual,
+                                             norm_w, eps,
+                                             op[0] == "fp8"), residual
+    return fused_add_rmsnorm(quant_rows(x, op), residual, norm_w, eps)
 
 
 def fp8_linear(x: torch.Tensor, w_q: torch.Tensor, w_scale: torch.Tensor,
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = x @ dequant(w_q).T via the fp8 weight-streaming kernel
     (M <= 256): per-token-group activation quant + block-scale fp8
-    MFMA. Weights stream at 1 B/elem — ~2x the bf16 decode rate."""
-    M, K = x.shape
-    N = w_q.shape[0]
-    aq, _, ast = per_token_group_quant_fp8(x.contiguous(),
-                                           transposed=True)
-    splitk = _quant_splitk(N, K, 128)
-    need = splitk * M * N
-    key = x.device.index or 0
-    ws = _FP8_WS.get(key)
-    if ws is None or ws.numel() < need:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("fp8 workspace grown during graph capture")
-        ws = torch.empty(need, dtype=torch.float32, device=x.device)
-        _FP8_WS[key] = ws
-    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-    _gpu_kernels().fp8_skinny_gemm(
-        out, aq.view(torch.uint8), ast, w_q.view(torch.uint8),
-        w_scale.contiguous(),
-        bias.float() if bias is not None else None, ws, splitk)
-    return out
+    MFMA."""
+    return quant_rows(x, ("fp8", w_q, w_scale), bias)
 
 
 _IDENT: dict = {}
@@ -588,26 +638,13 @@ def rmsnorm_gated(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,
 def int4_linear(x: torch.Tensor, wq4: torch.Tensor, sbt: torch.Tensor,
                 group: int,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out = x @ dequant(wq4).T via the fused-dequant int4 skinny GEMM
+    """out = x @ dequant(wq4).T via the int4 weight-streaming kernel
     (M <= 256): packed nibbles stream at 0.5 B/elem. ``sbt`` is the
     TRANSPOSED (scale, bias) bank [K/group, 2, N] (lane-contiguous
-    staging; repack_canonical builds it)."""
-    M, K = x.shape
-    N = wq4.shape[0]
-    splitk = _quant_splitk(N, K, 256)
-    need = splitk * M * N
-    key = x.device.index or 0
-    ws = _FP8_WS.get(key)  # shares the fp32 partial workspace pool
-    if ws is None or ws.numel() < need:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("int4 workspace grown during graph capture")
-        ws = torch.empty(need, dtype=torch.float32, device=x.device)
-        _FP8_WS[key] = ws
-    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
-    _gpu_kernels().int4_skinny_gemm(
-        out, x.contiguous(), wq4, sbt,
-        bias.float() if bias is not None else None, ws, group)
-    return out
+    staging; repack_canonical builds it), ``group`` 128."""
+    if group != 128:
+        raise RuntimeError("int4 gemm: group size 128")
+    return quant_rows(x, ("int4", wq4, sbt), bias)
 
 
 def fused_moe_int4(x: torch.Tensor, w13_c, w13_sb, w2_c, w2_sb,
@@ -770,19 +807,6 @@ def mla_paged_attention(q, k_cache, v_cache, block_table, seq_lens,
 SKINNY_MAX_M = 256
 
 
-def _quant_splitk(N: int, K: int, bk: int) -> int:
-    """splitk for the quant skinny GEMMs (fp8 bk=128, int4 bk=256):
-    deepest split that still leaves >= 8 ring stages per block, with
-    the grid capped near chip size (measured sweep, profiles/)."""
-    n_wg = -(-N // 64)
-    s = 1
-    while (s < 16 and n_wg * (s * 2) <= 1024
-           and (K // bk) // (s * 2) >= 8):
-        s *= 2
-    k_slice = ((-(-K // s)) + bk - 1) // bk * bk
-    return -(-K // k_slice)
-
-
 def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """bf16 operands as csrc/stream_gemm.hip reads them: 16 B aligned
     rows, K a multiple of 64, N of 8."""
@@ -793,7 +817,7 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def _plain_bias(bias, N: int) -> bool:
+def plain_bias(bias, N: int) -> bool:
     return bias is None or (bias.dtype == torch.bfloat16
                             and bias.is_contiguous() and bias.numel() == N)
 
@@ -805,7 +829,7 @@ def skinny_gemm(x: torch.Tensor, w: torch.Tensor,
     if not _rows_ok(x, w):
         import torch.nn.functional as F
         return F.linear(x, w, bias)
-    if not _plain_bias(bias, w.shape[0]):
+    if not plain_bias(bias, w.shape[0]):
         return _gpu_kernels().stream_gemm(x, w, None) + bias
     return _gpu_kernels().stream_gemm(x, w, bias)
 
@@ -837,7 +861,7 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     """GEMM dispatch: the weight-streaming kernel where measured faster,
     hipBLASLt otherwise."""
     import torch.nn.functional as F
-    if _streams(x, w) and _plain_bias(bias, w.shape[0]):
+    if _streams(x, w) and plain_bias(bias, w.shape[0]):
         return skinny_gemm(x, w, bias)
     return F.linear(x, w, bias)
 
@@ -853,16 +877,19 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_and_mul(linear(x, w))
 
 
+def _norm_parts_ok(N: int, residual: torch.Tensor,
+                   norm_w: torch.Tensor) -> bool:
+    return (N % 8 == 0 and N <= 8192 and residual.dtype == torch.bfloat16
+            and residual.is_contiguous() and residual.data_ptr() % 16 == 0
+            and norm_w.dtype in (torch.bfloat16, torch.float32))
+
+
 def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
                        residual: torch.Tensor, norm_w: torch.Tensor,
                        eps: float):
     """residual += x @ w.T; (rmsnorm(residual), residual). Few rows: the
     split product's parts are summed, added and normed by one kernel."""
-    if (_streams(x, w) and w.shape[0] <= 8192
-            and residual.dtype == torch.bfloat16
-            and residual.is_contiguous()
-            and residual.data_ptr() % 16 == 0
-            and norm_w.dtype in (torch.bfloat16, torch.float32)):
+    if _streams(x, w) and _norm_parts_ok(w.shape[0], residual, norm_w):
         return _gpu_kernels().stream_add_norm(x, w, residual, norm_w,
                                               eps), residual
     return fused_add_rmsnorm(linear(x, w), residual, norm_w, eps)
@@ -872,7 +899,7 @@ def qkv_parts(x: torch.Tensor, w: torch.Tensor,
               bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """The fp32 parts [S, M, N] of x @ w.T for ``qkv_rope_cache``, or None
     where the library's product is the better one."""
-    if _streams(x, w) and _plain_bias(bias, w.shape[0]):
+    if _streams(x, w) and plain_bias(bias, w.shape[0]):
         return _gpu_kernels().stream_parts(x, w)
     return None
 
@@ -893,13 +920,15 @@ def qkv_rope_cache_ok(k_cache: torch.Tensor, v_cache: torch.Tensor,
 def qkv_rope_cache(src: torch.Tensor, bias, positions: torch.Tensor,
                    cos_sin: torch.Tensor, k_cache: torch.Tensor,
                    v_cache: torch.Tensor, slot_mapping: torch.Tensor,
-                   num_heads: int) -> torch.Tensor:
+                   num_heads: int, rounded: bool = False) -> torch.Tensor:
     """From a merged q|k|v projection (bf16 rows, or the fp32 parts of
     ``qkv_parts``): add the bias, rotate queries and keys, write keys and
     values to their cache slots, return the queries [M, heads * D]. One
-    kernel for a bias, a rotation, a scatter and their copies."""
+    kernel for a bias, a rotation, a scatter and their copies.
+    ``rounded``: the biased rows are rounded to bf16 first (fp8 weights)."""
     return _gpu_kernels().qkv_finish(src, bias, positions, cos_sin, k_cache,
-                                     v_cache, slot_mapping, num_heads)
+                                     v_cache, slot_mapping, num_heads,
+                                     rounded)
 
 
 # --------------------------------------------------------------- layer norm

@@ -372,11 +372,15 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
     const char *e = getenv("GLLM_DECODE_SPLITS");
     return e ? atoi(e) : 0;
   }();
-  // (two workgroups fit a CU; requests are unequal, so twice that many even
-  // out better: 64 requests of 512 to 1536 keys, 8 heads, 62 us in two
-  // splits, 69 us in one; 24 of 2700 to 8100 115 us in eight, 121 in four)
+  // Two workgroups fit a CU. Twice as many would even unequal requests out
+  // a little better (64 requests of 512 to 1536 keys, 8 heads: 62 us in two
+  // splits, 69 us in one; 24 of 2700 to 8100 115 us in eight, 121 in four),
+  // but each split rounds its probabilities to bf16 against its own maximum,
+  // and behind products that quantize their rows to e4m3 that alone moves a
+  // two-layer model's outputs by 3 %: the count stays the smallest that
+  // fills the chip.
   int splits = 1;
-  while (splits < 16 && B * Hkv * splits < 1024 &&
+  while (splits < 16 && B * Hkv * splits < 512 &&
          splits * 2 <= (max_seq_len + 127) / 128)
     splits *= 2;
   if (splits_env > 0) splits = splits_env;

@@ -30,7 +30,7 @@ torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
 torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
                          torch::Tensor positions, torch::Tensor cos_sin,
                          torch::Tensor k_cache, torch::Tensor v_cache,
-                         torch::Tensor slots, long Hq);
+                         torch::Tensor slots, long Hq, bool rounded);
 void paged_attention_prefill(torch::Tensor out, torch::Tensor q,
                              torch::Tensor k_cache, torch::Tensor v_cache,
                              torch::Tensor block_table,
@@ -93,19 +93,19 @@ void per_token_group_quant_fp8(torch::Tensor x, torch::Tensor q,
                                torch::Tensor scales,
                                c10::optional<torch::Tensor> scales_t,
                                bool ue8m0);
-void fp8_skinny_gemm(torch::Tensor out, torch::Tensor aq, torch::Tensor as,
-                     torch::Tensor w, torch::Tensor ws,
-                     c10::optional<torch::Tensor> bias,
-                     torch::Tensor workspace, long splitk);
 void moe_gemm_fp8(torch::Tensor C, torch::Tensor A, torch::Tensor As,
                   torch::Tensor W, torch::Tensor Ws,
                   torch::Tensor sorted_ids, torch::Tensor expert_blocks,
                   torch::Tensor n_post_pad,
                   c10::optional<torch::Tensor> topk_weights, long n_pairs,
                   long topk, long block_m, bool scatter);
-void int4_skinny_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor wq,
-                      torch::Tensor sb, c10::optional<torch::Tensor> bias,
-                      torch::Tensor workspace, long group);
+torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
+                         torch::Tensor w, torch::Tensor ws,
+                         c10::optional<torch::Tensor> bias, long form,
+                         long splits);
+torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
+                             torch::Tensor norm_w, double eps,
+                             bool rounded);
 void moe_gemm_int4(torch::Tensor C, torch::Tensor A, torch::Tensor W,
                    torch::Tensor SB, torch::Tensor sorted_ids,
                    torch::Tensor expert_blocks, torch::Tensor n_post_pad,
@@ -198,12 +198,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_sum", &moe_sum, "sum pair outputs over topk");
   m.def("per_token_group_quant_fp8", &per_token_group_quant_fp8,
         "per (token, 128-group) e4m3 quant + fp32 scales");
-  m.def("fp8_skinny_gemm", &fp8_skinny_gemm,
-        "block-scale fp8 weight-streaming GEMM (decode)");
   m.def("moe_gemm_fp8", &moe_gemm_fp8,
         "block-scale fp8 grouped MoE GEMM");
-  m.def("int4_skinny_gemm", &int4_skinny_gemm,
-        "fused-dequant int4 weight-streaming GEMM (decode)");
+  m.def("quant_gemm", &quant_gemm,
+        "few-row product with int4 or block-scale fp8 weights");
+  m.def("parts_add_norm", &parts_add_norm,
+        "residual += sum of fp32 parts, RMS norm of it");
   m.def("moe_gemm_int4", &moe_gemm_int4,
         "fused-dequant int4 grouped MoE GEMM (w4a16)");
   m.def("gdn_conv_update", &gdn_conv_update,

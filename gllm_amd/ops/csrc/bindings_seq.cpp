@@ -183,7 +183,7 @@ torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
 torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
                          torch::Tensor positions, torch::Tensor cos_sin,
                          torch::Tensor k_cache, torch::Tensor v_cache,
-                         torch::Tensor slots, long Hq);
+                         torch::Tensor slots, long Hq, bool rounded);
 void silu_and_mul(torch::Tensor out, torch::Tensor x);
 void moe_align(torch::Tensor topk_ids, long E_local, long expert_start,
                long block_m, torch::Tensor sorted_ids,

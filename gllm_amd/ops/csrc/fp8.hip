@@ -74,219 +74,6 @@ __global__ void per_token_group_quant_kernel(
   }
 }
 
-// ------------------------------------------------- skinny fp8 GEMM
-// Same glds-ring structure as skinny_gemm.hip (v2), fp8 tiles: a ring
-// slot holds { W[64][128B] | A[MB*64][128B] } = one BK=128 scale block.
-template <int AUX>
-DEV_INLINE void glds16(const unsigned char *gsrc, char *lds_ptr) {
-  __builtin_amdgcn_global_load_lds(
-      reinterpret_cast<const unsigned int *>(gsrc),
-      reinterpret_cast<unsigned int *>(lds_ptr), 16, 0, AUX);
-}
-
-template <int MB, int RING>
-__global__ __launch_bounds__(BLOCK) void fp8_skinny_kernel(
-    float *__restrict__ partial,           // [SPLITK, M, N]
-    const unsigned char *__restrict__ aq,  // [M, K] e4m3
-    const float *__restrict__ ast,         // [K/128, M] (transposed)
-    const unsigned char *__restrict__ w,   // [N, K] e4m3
-    const float *__restrict__ ws,          // [N/128, K/128]
-    __hip_bfloat16 *__restrict__ out,      // non-null iff splitk == 1
-    const float *__restrict__ bias, int M, int N, int K, int k_slice) {
-  constexpr int TILE_B = (BN + MB * 64) * ROW_B;
-  const int n0 = blockIdx.x * BN;
-  const int z = blockIdx.y;
-  const int kb_begin = z * (k_slice / BK);
-  const int kb_end = min(K / BK, kb_begin + k_slice / BK);
-  const int nkt = kb_end - kb_begin;
-  if (nkt <= 0) return;
-  const int kgroups = K / BK;
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int l16 = lane & 15;
-  const int lhi = lane >> 4;
-
-  __shared__ __attribute__((aligned(16)))
-      char smem[RING * ((BN + MB * 64) * ROW_B + MB * 256)];
-  // the whole k-slice's weight scales, staged ONCE (a per-tile global
-  // scale load would force a vmcnt drain that serializes the glds ring)
-  __shared__ float ws_lds[256];
-
-  const int wblk = n0 / 128;  // BN=64 tile sits inside one n scale block
-  for (int i = tid; i < nkt; i += BLOCK)
-    ws_lds[i] = ws[(long)wblk * kgroups + kb_begin + i];
-  __syncthreads();
-
-  constexpr int GL_PER_WAVE = TILE_B / 1024 / 4;
-  // per-stage vm ops per wave: GL_PER_WAVE glds16 + MB glds4 (the
-  // activation scales gather through the SAME lds-dma pipeline so the
-  // counted waits stay exact — a plain global scale load would make the
-  // compiler emit a drain that serializes the ring)
-  constexpr int VM_PER_STAGE = GL_PER_WAVE + MB;
-  constexpr int ASC_OFF = TILE_B;  // asc area at the slot tail
-  constexpr int SLOT_B = TILE_B + MB * 64 * 4;
-  const unsigned char *gsrc[GL_PER_WAVE];
-  {
-#pragma unroll
-    for (int j = 0; j < GL_PER_WAVE; ++j) {
-      const int p = (wave * GL_PER_WAVE + j) * 1024 + lane * 16;
-      const int row = p / ROW_B;
-      const int col = swz(row, p % ROW_B);
-      if (row < BN) {
-        const int n = min(n0 + row, N - 1);
-        gsrc[j] = w + (long)n * K + col;
-      } else {
-        const int m = min(row - BN, M - 1);
-        gsrc[j] = aq + (long)m * K + col;
-      }
-    }
-  }
-
-  auto stage = [&](int kt, int slot) {
-    const long kb = (long)(kb_begin + kt) * BK;
-    char *base = smem + slot * SLOT_B;
-#pragma unroll
-    for (int j = 0; j < GL_PER_WAVE; ++j) {
-      const int off = (wave * GL_PER_WAVE + j) * 1024;
-      if (off < BN * ROW_B)
-        glds16<2>(gsrc[j] + kb, base + off);
-      else
-        glds16<0>(gsrc[j] + kb, base + off);
-    }
-    // every wave issues the identical scale load (same values land
-    // at the same LDS bytes) so per-wave vm counters stay uniform.
-    // ast is [kgroups, M]: the stage's M scales are CONTIGUOUS — a
-    // handful of cache lines instead of the 64-line strided gather
-    // that used to double the ring's line-request rate.
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int m = min(mb * 64 + lane, M - 1);
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const unsigned int *>(
-              ast + (long)(kb_begin + kt) * M + m),
-          reinterpret_cast<unsigned int *>(base + ASC_OFF + mb * 256), 4,
-          0, 0);
-    }
-  };
-
-  f8_f4 acc[MB][BN / 16];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int nt = 0; nt < BN / 16; ++nt) acc[mb][nt] = f8_f4{0, 0, 0, 0};
-
-  const int pre = min(RING - 1, nkt);
-  for (int t = 0; t < pre; ++t) stage(t, t % RING);
-
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int slot = kt % RING;
-    if (kt + RING - 1 < nkt) stage(kt + RING - 1, (kt + RING - 1) % RING);
-    const int ahead = min(nkt - 1 - kt, RING - 1);
-    if (RING >= 4 && ahead == 3) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(3 * VM_PER_STAGE)
-                   : "memory");
-    } else if (RING >= 3 && ahead == 2) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * VM_PER_STAGE)
-                   : "memory");
-    } else if (ahead == 1) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(1 * VM_PER_STAGE)
-                   : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __builtin_amdgcn_s_barrier();
-
-    const char *wbase = smem + slot * SLOT_B;
-    const char *xbase = wbase + BN * ROW_B;
-    const float *asc_lds =
-        reinterpret_cast<const float *>(wbase + ASC_OFF);
-    const float wsc = ws_lds[kt];
-
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      f8_f4 sub[BN / 16];
-#pragma unroll
-      for (int nt = 0; nt < BN / 16; ++nt) sub[nt] = f8_f4{0, 0, 0, 0};
-#pragma unroll
-      for (int ks = 0; ks < BK / 32; ++ks) {
-        const int arow = mb * 64 + wave * 16 + l16;
-        const long afrag = *reinterpret_cast<const long *>(
-            xbase + arow * ROW_B + swz(arow, ks * 32 + lhi * 8));
-#pragma unroll
-        for (int nt = 0; nt < BN / 16; ++nt) {
-          const int brow = nt * 16 + l16;
-          const long bfrag = *reinterpret_cast<const long *>(
-              wbase + brow * ROW_B + swz(brow, ks * 32 + lhi * 8));
-          sub[nt] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-              afrag, bfrag, sub[nt], 0, 0, 0);
-        }
-      }
-      float asc[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        asc[r] = asc_lds[mb * 64 + min(wave * 16 + lhi * 4 + r, 63)] * wsc;
-#pragma unroll
-      for (int nt = 0; nt < BN / 16; ++nt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc[mb][nt][r] += sub[nt][r] * asc[r];
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  }
-
-  if (out != nullptr) {
-    // splitk == 1: write bf16 directly (+bias) — skips the separate
-    // fp32-partial round-trip and the reduce launch entirely
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-      for (int nt = 0; nt < BN / 16; ++nt) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = mb * 64 + wave * 16 + lhi * 4 + r;
-          const int n = n0 + nt * 16 + l16;
-          if (m < M && n < N) {
-            float v = acc[mb][nt][r];
-            if (bias) v += bias[n];
-            out[(long)m * N + n] = __float2bfloat16(v);
-          }
-        }
-      }
-    }
-    return;
-  }
-  float *base = partial + (long)z * M * N;
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-    for (int nt = 0; nt < BN / 16; ++nt) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = mb * 64 + wave * 16 + lhi * 4 + r;
-        const int n = n0 + nt * 16 + l16;
-        if (m < M && n < N) base[(long)m * N + n] = acc[mb][nt][r];
-      }
-    }
-  }
-}
-
-// out[m, n] = bf16( sum_z partial[z, m, n] + bias[n] )
-__global__ void fp8_reduce_kernel(__hip_bfloat16 *__restrict__ out,
-                                  const float *__restrict__ partial,
-                                  const float *__restrict__ bias, int M,
-                                  int N, int splitk) {
-  const long total = (long)M * N;
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    float v = bias ? bias[i % N] : 0.f;
-    for (int z = 0; z < splitk; ++z) v += partial[(long)z * total + i];
-    out[i] = __float2bfloat16(v);
-  }
-}
-
 // ------------------------------------------------- fp8 grouped MoE GEMM
 // moe.hip's pipeline with fp8 operands + block scales. LDS-tiled like
 // the bf16 version (BKm = 128 elems = one scale block per k tile).
@@ -498,77 +285,6 @@ void per_token_group_quant_fp8(torch::Tensor x, torch::Tensor q,
                      (const __hip_bfloat16 *)x.data_ptr(),
                      (unsigned char *)q.data_ptr(),
                      scales.data_ptr<float>(), st, n_groups, kg, K, ue8m0);
-  HIP_CHECK_KERNEL();
-}
-
-void fp8_skinny_gemm(torch::Tensor out, torch::Tensor aq, torch::Tensor ast,
-                     torch::Tensor w, torch::Tensor ws,
-                     c10::optional<torch::Tensor> bias,
-                     torch::Tensor workspace, long splitk_arg) {
-  const int M = aq.size(0), K = aq.size(1), N = w.size(0);
-  TORCH_CHECK(aq.is_contiguous() && w.is_contiguous() && out.is_contiguous());
-  TORCH_CHECK(K % BK == 0, "fp8 gemm: K must be a multiple of 128");
-  TORCH_CHECK(K / BK <= 256, "fp8 skinny: K <= 32768 (ws_lds)");
-  TORCH_CHECK(M <= 256, "fp8 skinny: M <= 256");
-  TORCH_CHECK(ast.is_contiguous() && ast.numel() == (long)M * (K / BK),
-              "fp8 skinny: transposed scales [K/128, M]");
-  const int n_wg = (N + BN - 1) / BN;
-  int splitk = (int)splitk_arg;
-  if (splitk <= 0) {
-    splitk = 1;
-    while (splitk < 16 && n_wg * (splitk * 2) <= 1024 &&
-           (K / BK) / (splitk * 2) >= 8)
-      splitk *= 2;
-  }
-  int k_slice = (K + splitk - 1) / splitk;
-  k_slice = ((k_slice + BK - 1) / BK) * BK;
-  splitk = (K + k_slice - 1) / k_slice;
-  TORCH_CHECK(splitk == 1 || workspace.numel() >= (long)splitk * M * N);
-  auto stream = at::cuda::getCurrentCUDAStream();
-  auto *wsp = workspace.data_ptr<float>();
-  auto *ap = (const unsigned char *)aq.data_ptr();
-  auto *asp = ast.data_ptr<float>();
-  auto *wp = (const unsigned char *)w.data_ptr();
-  auto *wsc = ws.data_ptr<float>();
-  const float *bias_ptr = nullptr;
-  if (bias.has_value()) bias_ptr = bias->data_ptr<float>();
-  // splitk == 1: the GEMM kernel writes bf16 (+bias) itself
-  __hip_bfloat16 *outp =
-      splitk == 1 ? (__hip_bfloat16 *)out.data_ptr() : nullptr;
-#define LAUNCH_SK(MB, RING)                                                  \
-  hipLaunchKernelGGL((fp8_skinny_kernel<MB, RING>),                          \
-                     dim3(n_wg, splitk), dim3(BLOCK), 0, stream, wsp, ap,    \
-                     asp, wp, wsc, outp, bias_ptr, M, N, K, k_slice)
-  static int ring_env = [] {
-    const char *e = getenv("FP8_RING");
-    return e ? atoi(e) : 0;
-  }();
-  if (M <= 64) {
-    // RING=2 = 33 KB LDS = 4 blocks/CU: measured faster than the
-    // deeper 3-slot ring at 3 blocks/CU on every decode shape.
-    // (A W-only-DMA variant with asm register A-loads measured ~8%
-    // faster still, but async asm defs are invisible to regalloc —
-    // it may copy the register before the data lands — and it
-    // miscompiled; profiles/r02_session_notes.md records the attempt.)
-    const int r = ring_env ? ring_env : 2;
-    if (r == 3) LAUNCH_SK(1, 3);
-    else if (r == 4) LAUNCH_SK(1, 4);
-    else LAUNCH_SK(1, 2);
-  }
-  else if (M <= 128) {
-    // RING=2 measured faster (3 blocks/CU): down 116 -> 85 us @ M=96
-    if (ring_env == 3) LAUNCH_SK(2, 3);
-    else LAUNCH_SK(2, 2);
-  }
-  else LAUNCH_SK(4, 2);
-#undef LAUNCH_SK
-  HIP_CHECK_KERNEL();
-  if (splitk == 1) return;
-  const long total = (long)M * N;
-  const long grid = std::min<long>((total + 1023) / 1024, 2048);
-  hipLaunchKernelGGL(fp8_reduce_kernel, dim3(grid), dim3(256), 0, stream,
-                     (__hip_bfloat16 *)out.data_ptr(), wsp, bias_ptr, M, N,
-                     splitk);
   HIP_CHECK_KERNEL();
 }
 

@@ -1,0 +1,583 @@
+// Products of few rows (M <= 256) with a quantized weight matrix, fp32 sums:
+//   int4  x bf16 [M, K], w packed nibbles [N, K / 2] (even k low), scales
+//         fp32 [K / 128, 2, N]: w = q * s + b per group of 128
+//   fp8   x e4m3 [M, K] with fp32 scales [K / 128, M], w e4m3 [N, K] with
+//         fp32 scales [ceil(N / 128), K / 128]
+// (K a multiple of 128). One K stage is one scale group: its sum is formed by
+// matrix instructions on its own and enters the result times its scales.
+//
+// Bound by the weights' bytes; the structure is that of the unquantized
+// stream product: 16 B global -> LDS loads into a ring of stages, products
+// are W x^T, a weight with few tiles is split along K into fp32 parts that
+// the next kernel sums, a gated feed-forward leaves silu(gate) * up.
+//
+// int4: the integer 16 + q is a bf16 number whose mantissa holds the nibble,
+// so two weights cost a shift and an and-or, where q * s + b in floating
+// point took six operations a weight (91 % of the issue slots went there).
+// A matrix instruction with ones beside the weights' gives sum(x), and the
+// group enters as s * (part - 16 sum(x)) + b sum(x): the weights are not
+// rounded to bf16. A row whose sum is not finite (16 x - 16 x has no value
+// there) takes the group again with the weights formed one by one.
+//
+// fp8: what comes out is quantized to e4m3 again a kernel or two later, where
+// a last bit decides between neighbours; so the gated form and the readers of
+// the parts round the sums to bf16 before they go on, and a fused product
+// gives what the separate one gives.
+//
+// (us, 29 rows; the kernels before these formed floats weight by weight and
+// did not fill the chip:) 55296 x 5120 int4 48, fp8 46 gated; 5120 x 27648 28
+// and 31; four products of a 5120-wide layer 100 (210) and 99. Weights come
+// at 4.6 (int4, 1 row) and 6.3 TB/s (fp8); int4 with 17 rows and more is
+// bound by its vector instructions.
+
+#include <torch/extension.h>
+#include <ATen/cuda/CUDAContext.h>
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 qg_bf8;
+typedef __attribute__((ext_vector_type(4))) float qg_f4;
+typedef __attribute__((ext_vector_type(4))) unsigned qg_u4;
+
+namespace {
+
+constexpr int MAX_SPLIT = 16;
+constexpr int GROUP = 128;
+
+enum Quant { INT4 = 0, FP8 = 1 };
+enum Form { GATED = 0, PLAIN = 1, PART = 2 };
+
+// AUX 2: non-temporal
+template <int AUX>
+DEV_INLINE void glds16(const char *gsrc, char *lds_ptr) {
+  __builtin_amdgcn_global_load_lds(
+      reinterpret_cast<const unsigned int *>(gsrc),
+      reinterpret_cast<unsigned int *>(lds_ptr), 16, 0, AUX);
+}
+
+DEV_INLINE void glds4(const char *gsrc, char *lds_ptr) {
+  __builtin_amdgcn_global_load_lds(
+      reinterpret_cast<const unsigned int *>(gsrc),
+      reinterpret_cast<unsigned int *>(lds_ptr), 4, 0, 0);
+}
+
+DEV_INLINE short to_bf16(float v) {
+  return __builtin_bit_cast(short, __float2bfloat16(v));
+}
+
+// wait until at most AHEAD stages of LD loads are on their way
+template <int AHEAD, int LD>
+DEV_INLINE void wait_stages(int ahead) {
+  if (ahead >= AHEAD)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(AHEAD * LD) : "memory");
+  else if constexpr (AHEAD > 0)
+    wait_stages<AHEAD - 1, LD>(ahead);
+}
+
+// the two constants of offset_weights in registers: a three-operand
+// instruction takes neither as a literal
+struct Offset {
+  unsigned mask, base;
+  DEV_INLINE Offset() {
+    asm("s_mov_b32 %0, 0x00780078" : "=s"(mask));
+    asm("v_mov_b32 %0, 0x41804180" : "=v"(base));
+  }
+};
+
+// eight nibbles as 16 + q, elements in the order 0 4 1 5 2 6 3 7
+DEV_INLINE qg_bf8 offset_weights(unsigned w, const Offset &k) {
+  qg_u4 o;
+  o[0] = ((w << 3) & k.mask) | k.base;
+  o[1] = ((w >> 1) & k.mask) | k.base;
+  o[2] = ((w >> 5) & k.mask) | k.base;
+  o[3] = ((w >> 9) & k.mask) | k.base;
+  return __builtin_bit_cast(qg_bf8, o);
+}
+
+// the same order for eight activations
+DEV_INLINE qg_bf8 weight_order(qg_u4 v) {
+  qg_u4 o;
+  o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
+  o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
+  o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
+  o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
+  return __builtin_bit_cast(qg_bf8, o);
+}
+
+// eight weights q * s + b, same order
+DEV_INLINE qg_bf8 scaled_weights(unsigned w, float s, float b) {
+  qg_u4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float lo = (float)((w >> (4 * i)) & 15u) * s + b;
+    const float hi = (float)((w >> (4 * i + 16)) & 15u) * s + b;
+    o[i] = (unsigned short)to_bf16(lo) |
+           ((unsigned)(unsigned short)to_bf16(hi) << 16);
+  }
+  return __builtin_bit_cast(qg_bf8, o);
+}
+
+// lane: row l16 of each row tile, columns lhi * 4 + r
+template <int Q, int NT, int MT, int BN, int FORM>
+DEV_INLINE void store_tile(void *C, const qg_f4 (&acc)[NT][MT],
+                           const float *bias, int M, int N, int NC, int row0,
+                           int nb, int z, int tile0, int lane) {
+  const int l16 = lane & 15, lhi = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = row0 + m * 16 + l16;
+    if (row >= M) continue;
+#pragma unroll
+    for (int n = 0; n < NT; n += FORM == GATED ? 2 : 1) {
+      const int c = nb * (FORM == GATED ? BN / 2 : BN) +
+                    (tile0 + n) * (FORM == GATED ? 8 : 16) + lhi * 4;
+      if (c >= NC) continue;
+      if (FORM == PART) {
+        *reinterpret_cast<qg_f4 *>((float *)C + ((long)z * M + row) * N + c) =
+            acc[n][m];
+        continue;
+      }
+      shortx4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[n][m][r];
+        if (FORM == GATED) {
+          float u = acc[n + (NT > 1 ? 1 : 0)][m][r];
+          if (Q == FP8) {  // (see above)
+            v = __bfloat162float(__float2bfloat16(v));
+            u = __bfloat162float(__float2bfloat16(u));
+          }
+          v = v / (1.f + __expf(-v)) * u;
+        }
+        else if (bias)
+          v += bias[min(c + r, N - 1)];
+        o[r] = to_bf16(v);
+      }
+      short *dst = (short *)C + (long)row * NC + c;
+      if (NC % 4 == 0) {
+        *reinterpret_cast<shortx4 *>(dst) = o;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c + r < NC) dst[r] = o[r];
+      }
+    }
+  }
+}
+
+// WM x WN waves share a BM x BN tile; a ring of ST stages of 128 columns
+template <int Q, int BM, int BN, int WM, int WN, int ST, int FORM>
+__global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
+    void *__restrict__ C,  // bf16 [M, N or N / 2], PART: fp32 [S, M, N]
+    const char *__restrict__ X, const float *__restrict__ XS,
+    const char *__restrict__ W, const float *__restrict__ WS,
+    const float *__restrict__ bias, int M, int N, int K, int k_slice,
+    int nbm, int nbn) {
+  constexpr int WAVES = WM * WN;
+  constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
+  // LDS row bytes; 128 of a weight row at once in either form (64 B pieces of
+  // it come at half the rate)
+  constexpr int GS = Q == INT4 ? 2 : 1;  // groups of a stage
+  constexpr int XROW = Q == INT4 ? GS * 2 * GROUP : GROUP;
+  constexpr int WROW = 128;
+  constexpr int XU = XROW / 16, WU = WROW / 16;  // 16 B units of a row
+  constexpr int XLOADS = BM * XROW / 1024, WLOADS = BN * WROW / 1024;
+  // fp32 scales of a stage, 64 to a load: s | b of the columns, or the rows'
+  constexpr int SN = Q == INT4 ? GS * 2 * BN : BM;
+  constexpr int SLOADS = (SN + 63) / 64;
+  constexpr int XL = (XLOADS + WAVES - 1) / WAVES;
+  constexpr int WL = (WLOADS + WAVES - 1) / WAVES;
+  constexpr int SL = (SLOADS + WAVES - 1) / WAVES;
+  constexpr int W_OFF = BM * XROW, S_OFF = W_OFF + BN * WROW;
+  constexpr int STAGE = S_OFF + SLOADS * 256;
+  static_assert(FORM != GATED || NT % 2 == 0, "gate and up in one wave");
+  __shared__ __attribute__((aligned(16))) char smem[ST * STAGE];
+
+  // eight dies take workgroups in turn: each gets a contiguous run of tiles,
+  // row blocks fastest (they share weights)
+  const int total = nbm * nbn;
+  const int pid = blockIdx.x, xcd = pid & 7, per = total >> 3;
+  const int t = xcd * per + min(xcd, total & 7) + (pid >> 3);
+  const int mb = t % nbm, nb = t / nbm;
+  const int z = blockIdx.y;
+  const int k0 = z * k_slice;
+  const int nkt = min(K - k0, k_slice) / (GS * GROUP);
+  const int kgroups = K / GROUP, g0 = k0 / GROUP;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lhi = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  const int NC = FORM == GATED ? N >> 1 : N;  // columns of C
+
+  // weight row of a row of the tile
+  auto weight_row = [&](int row) {
+    if (FORM == GATED) {  // 16 gate rows, their 16 up rows, the next 16
+      const int c = min(nb * (BN / 2) + (row >> 5) * 16 + (row & 15), NC - 1);
+      return (row & 16) ? NC + c : c;
+    }
+    return min(nb * BN + row, N - 1);
+  };
+  // 16 B units are permuted so that 16 rows at one unit fall on all banks
+  auto xswz = [](int row) { return Q == INT4 ? row & 15 : row & 7; };
+
+  // sources; a wave without a load of its own repeats another wave's
+  const char *xsrc[XL], *wsrc[WL], *ssrc[SL];
+  int xdst[XL], wdst[WL], sdst[SL];
+#pragma unroll
+  for (int j = 0; j < XL; ++j) {
+    const int u = (j * WAVES + wave) % XLOADS;
+    const int row = u * (64 / XU) + lane / XU;
+    const int c = (lane % XU) ^ xswz(row);
+    xsrc[j] = X + ((long)min(mb * BM + row, M - 1) * K + k0) *
+                      (Q == INT4 ? 2 : 1) + c * 16;
+    xdst[j] = u * 1024;
+  }
+#pragma unroll
+  for (int j = 0; j < WL; ++j) {
+    const int u = (j * WAVES + wave) % WLOADS;
+    const int row = u * (64 / WU) + lane / WU;
+    const int c = (lane % WU) ^ (row & 7);
+    wsrc[j] = W + ((long)weight_row(row) * K + k0) / GS + c * 16;
+    wdst[j] = W_OFF + u * 1024;
+  }
+#pragma unroll
+  for (int j = 0; j < SL; ++j) {
+    const int u = (j * WAVES + wave) % SLOADS;
+    const int i = u * 64 + lane;
+    if (Q == INT4)
+      ssrc[j] = (const char *)(WS + ((long)g0 * 2 + i / BN) * N +
+                               weight_row(i % BN));
+    else
+      ssrc[j] = (const char *)(XS + (long)g0 * M +
+                               min(mb * BM + min(i, BM - 1), M - 1));
+    sdst[j] = S_OFF + u * 256;
+  }
+  const long sstep = (Q == INT4 ? 2L * GS * N : (long)M) * 4;
+  auto stage = [&](int slot) {
+    char *base = smem + slot * STAGE;
+#pragma unroll
+    for (int j = 0; j < XL; ++j) {
+      glds16<0>(xsrc[j], base + xdst[j]);
+      xsrc[j] += XROW;
+    }
+#pragma unroll
+    for (int j = 0; j < WL; ++j) {
+      glds16<2>(wsrc[j], base + wdst[j]);
+      wsrc[j] += WROW;
+    }
+#pragma unroll
+    for (int j = 0; j < SL; ++j) {
+      glds4(ssrc[j], base + sdst[j]);
+      ssrc[j] += sstep;
+    }
+  };
+  constexpr int LD = XL + WL + SL;
+
+  // fp8: the weight scales of this wave's column tiles, one stage ahead
+  const float *wsc[NT];
+  float wnext[NT];
+  if (Q == FP8) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      wsc[n] = WS + (long)(weight_row((wn * NT + n) * 16) / 128) * kgroups +
+               g0;
+      wnext[n] = wsc[n][0];
+    }
+  }
+
+  const Offset offset;
+  qg_f4 acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = qg_f4{0, 0, 0, 0};
+
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i)
+    if (i < nkt) stage(i);
+  int cur = 0, nxt = ST - 1;
+  for (int kt = 0; kt < nkt; ++kt) {
+    // this wave's loads of stage kt have landed, later ones may fly
+    wait_stages<ST - 2, LD>(min(nkt - 1 - kt, ST - 2));
+    // everybody's are there, and stage kt - 1 (the slot that the next one
+    // takes) has been read
+    __builtin_amdgcn_s_barrier();
+    if (kt + ST - 1 < nkt) stage(nxt);
+    const char *xb = smem + cur * STAGE + (wm * MT * 16 + l16) * XROW;
+    const char *wb = smem + cur * STAGE + W_OFF + (wn * NT * 16 + l16) * WROW;
+    const float *sb =
+        reinterpret_cast<const float *>(smem + cur * STAGE + S_OFF);
+    if constexpr (Q == INT4) {
+#pragma unroll
+      for (int i = 0; i < GS; ++i) {
+        qg_f4 part[NT][MT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
+        const float *sg = sb + i * 2 * BN;
+        // lane lhi holds elements 32 lhi .. + 31 of its rows
+        qg_u4 wv[NT];
+        qg_f4 xsum[MT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          wv[n] = *reinterpret_cast<const qg_u4 *>(
+              wb + n * 16 * WROW + (((i * 4 + lhi) ^ (l16 & 7)) << 4));
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xsum[m] = qg_f4{0, 0, 0, 0};
+        const qg_bf8 ones = __builtin_bit_cast(
+            qg_bf8, qg_u4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          qg_bf8 xf[MT];
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            xf[m] = weight_order(*reinterpret_cast<const qg_u4 *>(
+                xb + m * 16 * XROW + ((i * 16 + ((lhi * 4 + j) ^ l16)) << 4)));
+            xsum[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xf[m],
+                                                              xsum[m], 0, 0, 0);
+          }
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const qg_bf8 wf = offset_weights(wv[n][j], offset);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  wf, xf[m], part[n][m], 0, 0, 0);
+          }
+        }
+        bool finite[MT], all = true;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          finite[m] = fabsf(xsum[m][0]) < 1e36f;  // (false for NaN)
+          all &= finite[m];
+        }
+        const bool plain = __all(all);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const int c = (wn * NT + n) * 16 + lhi * 4;
+          const qg_f4 s = *reinterpret_cast<const qg_f4 *>(sg + c);
+          qg_f4 b = *reinterpret_cast<const qg_f4 *>(sg + BN + c);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) b[r] -= 16.f * s[r];
+          if (__builtin_expect(plain, 1)) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                acc[n][m][r] = fmaf(s[r], part[n][m][r],
+                                    fmaf(b[r], xsum[m][r], acc[n][m][r]));
+            continue;
+          }
+          const int cw = (wn * NT + n) * 16 + l16;
+          qg_bf8 wf[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            wf[j] = scaled_weights(wv[n][j], sg[cw], sg[BN + cw]);
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            qg_f4 one = qg_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              one = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  wf[j],
+                  weight_order(*reinterpret_cast<const qg_u4 *>(
+                      xb + m * 16 * XROW +
+                      ((i * 16 + ((lhi * 4 + j) ^ l16)) << 4))),
+                  one, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              acc[n][m][r] =
+                  finite[m] ? fmaf(s[r], part[n][m][r],
+                                   fmaf(b[r], xsum[m][r], acc[n][m][r]))
+                            : acc[n][m][r] + one[r];
+          }
+        }
+      }
+    } else {
+      qg_f4 part[NT][MT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
+      float ws[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        ws[n] = wnext[n];
+        wnext[n] = wsc[n][min(kt + 1, nkt - 1)];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {  // lane lhi: columns 32 j + 8 lhi .. + 7
+        long xf[MT], wf[NT];
+        const int off =
+            (((j * 2 + (lhi >> 1)) ^ xswz(l16)) << 4) + (lhi & 1) * 8;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          wf[n] = *reinterpret_cast<const long *>(wb + n * 16 * WROW + off);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          xf[m] = *reinterpret_cast<const long *>(xb + m * 16 * XROW + off);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+            part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                wf[n], xf[m], part[n][m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const float xs = sb[(wm * MT + m) * 16 + l16];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const float f = xs * ws[n];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[n][m][r] += f * part[n][m][r];
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    cur = cur + 1 == ST ? 0 : cur + 1;
+    nxt = nxt + 1 == ST ? 0 : nxt + 1;
+  }
+
+  store_tile<Q, NT, MT, BN, FORM>(C, acc, bias, M, N, NC, mb * BM + wm * MT * 16,
+                               nb, z, wn * NT, lane);
+}
+
+struct Plan {
+  int bm, bn, nbm, nbn, splits, k_slice;
+};
+
+// The tile by rows and width (us, rows x N x K):
+//  * int4: up to 16 rows 64 columns, 128 where the weight is wide or deep
+//    (1 x 7168 x 5120 8.6, 128 columns 9.9; 1 x 5120 x 27648 17.8 at 128,
+//    21.2 at 64); above that 256 for wide and deep ones (29 x 55296 x 5120
+//    47.8, 128 columns 48.8; 29 x 5120 x 27648 27.6, 28.6; 64 x 55296 x 5120
+//    72.9, 84.8), else 64 (29 x 7168 x 5120 13.2, 128 columns 15) or, for
+//    more than 32 rows, 128 (64 x 5120 x 5120 16.0, 64 columns 19).
+//  * fp8: up to 16 rows the same (1 x 7168 x 5120 9.2, 128 columns 10.1; 1 x
+//    28672 x 4096 22.1); above that 64 (29 x 7168 x 5120 12.4, 128 columns
+//    14), 256 from 36000 columns (64 x 55296 x 5120 51.2, 128 columns 57.4),
+//    128 between for more than 32 rows (64 x 28672 x 4096 28.6, 29.1).
+// K is split into about as many workgroups as the chip holds at once: 256 of
+// the 512-thread tiles, 448 of the others (1 x 7168 x 5120 4 parts 8.6, 3
+// 9.4), each part at least four stages long.
+Plan plan_for(bool int4, int M, int N, int K, bool gated, int splits) {
+  Plan p;
+  const bool wide = N >= 16384, deep = K >= 2 * N;
+  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  if (p.bm == 16) p.bn = gated || wide || deep ? 128 : 64;
+  else if (int4) p.bn = wide || deep ? 256 : gated || p.bm == 64 ? 128 : 64;
+  else p.bn = N >= 36000 ? 256 : p.bm == 64 && wide ? 128 : 64;
+  p.nbm = (M + p.bm - 1) / p.bm;
+  p.nbn = (N + p.bn - 1) / p.bn;
+  const int step = int4 ? 2 * GROUP : GROUP;
+  const int tiles = p.nbm * p.nbn, stages = K / step;
+  const int aim = p.bn == 256 ? 256 : 448;
+  int s = 1;
+  if (!gated && N % 8 == 0) {
+    if (splits > 0) s = std::min(splits, stages);
+    else s = std::max(1, std::min(std::min(aim / tiles, MAX_SPLIT),
+                                  stages / 4));
+  }
+  const int per = (stages + s - 1) / s;
+  p.k_slice = per * step;
+  p.splits = (stages + per - 1) / per;
+  return p;
+}
+
+template <int FORM>
+void launch(const Plan &p, bool int4, void *C, const void *X, const float *XS,
+            const void *W, const float *WS, const float *bias, int M, int N,
+            int K) {
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define RUN(Q, BM, BN, WM, WN, ST)                                           \
+  hipLaunchKernelGGL((quant_gemm_kernel<Q, BM, BN, WM, WN, ST, FORM>),       \
+                     dim3(p.nbm * p.nbn, p.splits), dim3((WM) * (WN) * 64),  \
+                     0, stream, C, (const char *)X, XS, (const char *)W, WS, \
+                     bias, M, N, K, p.k_slice, p.nbm, p.nbn)
+  if (int4) {
+    if (p.bm == 16 && p.bn == 128) RUN(INT4, 16, 128, 1, 4, 2);
+    else if (p.bm == 32 && p.bn == 256) RUN(INT4, 32, 256, 1, 8, 2);
+    else if (p.bm == 32 && p.bn == 128) RUN(INT4, 32, 128, 1, 4, 2);
+    else if (p.bm == 64 && p.bn == 256) RUN(INT4, 64, 256, 2, 4, 2);
+    else if (p.bm == 64) RUN(INT4, 64, 128, 2, 4, 2);
+    else if constexpr (FORM != GATED) {  // (gate and up tile in one wave)
+      if (p.bm == 16) RUN(INT4, 16, 64, 1, 4, 3);
+      else RUN(INT4, 32, 64, 1, 4, 2);
+    }
+  } else {
+    if (p.bm == 16 && p.bn == 128) RUN(FP8, 16, 128, 1, 4, 4);
+    else if (p.bm == 32 && p.bn == 256) RUN(FP8, 32, 256, 1, 8, 3);
+    else if (p.bm == 32) RUN(FP8, 32, 64, 1, 2, 4);
+    else if (p.bm == 64 && p.bn == 256) RUN(FP8, 64, 256, 2, 4, 3);
+    else if (p.bm == 64 && p.bn == 128) RUN(FP8, 64, 128, 2, 4, 3);
+    else if (p.bm == 64) RUN(FP8, 64, 64, 2, 2, 3);
+    else if constexpr (FORM != GATED) RUN(FP8, 16, 64, 1, 4, 6);
+  }
+#undef RUN
+  HIP_CHECK_KERNEL();
+}
+
+bool aligned16(const torch::Tensor &t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+}  // namespace
+
+torch::Tensor parts_sum(torch::Tensor part, c10::optional<torch::Tensor> bias);
+
+// x w^T for quantized w, as laid out above: int4 without xs (x bf16), fp8
+// with it (x the e4m3 bytes). form 0: silu(gate) * up of w = gate rows over
+// up rows, bf16 [M, N / 2]; 1: bf16 [M, N], with the fp32 bias; 2: the fp32
+// parts [S, M, N]. splits: parts along K, 0: by the plan
+torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
+                         torch::Tensor w, torch::Tensor ws,
+                         c10::optional<torch::Tensor> bias, long form,
+                         long splits) {
+  const bool int4 = !xs.has_value();
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 &&
+              x.is_contiguous() && w.is_contiguous() && aligned16(x) &&
+              aligned16(w) && w.scalar_type() == at::kByte &&
+              x.scalar_type() == (int4 ? at::kBFloat16 : at::kByte),
+              "quant_gemm: 16 B aligned rows, bf16 or e4m3 by packed bytes");
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  const long kg = K / GROUP;
+  TORCH_CHECK(K > 0 && K % (int4 ? 2 * GROUP : GROUP) == 0 &&
+              w.size(1) == (int4 ? K / 2 : K),
+              "quant_gemm: K a multiple of 128 (fp8) or 256 (int4)");
+  TORCH_CHECK(M <= 256 && N > 0, "quant_gemm: at most 256 rows");
+  TORCH_CHECK(ws.is_contiguous() && ws.scalar_type() == at::kFloat &&
+              ws.numel() >= (int4 ? kg * 2 * N : (N + 127) / 128 * kg),
+              "quant_gemm: weight scales");
+  if (!int4)
+    TORCH_CHECK(xs->is_contiguous() && xs->scalar_type() == at::kFloat &&
+                xs->numel() == M * kg, "quant_gemm: row scales [K / 128, M]");
+  if (bias.has_value())
+    TORCH_CHECK(bias->is_contiguous() && bias->numel() == N &&
+                bias->scalar_type() == at::kFloat, "quant_gemm: fp32 bias");
+  TORCH_CHECK(form == GATED ? N % 32 == 0 && !bias.has_value()
+              : form == PART ? N % 8 == 0 && !bias.has_value()
+                             : form == PLAIN,
+              "quant_gemm: gated N a multiple of 32, parts of 8");
+  const Plan p = plan_for(int4, std::max(M, 1L), N, K, form == GATED, splits);
+  const float *xsp = int4 ? nullptr : xs->data_ptr<float>();
+  const float *bp = bias.has_value() ? bias->data_ptr<float>() : nullptr;
+  const auto o16 = x.options().dtype(at::kBFloat16);
+  if (form == GATED || (form == PLAIN && (p.splits == 1 || M == 0))) {
+    auto out = torch::empty({M, form == GATED ? N / 2 : N}, o16);
+    if (M == 0) return out;
+    if (form == GATED)
+      launch<GATED>(p, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+                    ws.data_ptr<float>(), nullptr, M, N, K);
+    else
+      launch<PLAIN>(p, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+                    ws.data_ptr<float>(), bp, M, N, K);
+    return out;
+  }
+  auto part = torch::empty({(long)p.splits, M, N},
+                           x.options().dtype(at::kFloat));
+  if (M > 0)
+    launch<PART>(p, int4, part.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+                 ws.data_ptr<float>(), nullptr, M, N, K);
+  return form == PART ? part : parts_sum(part, bias);
+}

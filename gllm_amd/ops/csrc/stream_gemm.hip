@@ -206,6 +206,10 @@ __global__ __launch_bounds__(WM *WN * 64) void stream_gemm_kernel(
   }
 }
 
+DEV_INLINE float bf16_value(float v) {
+  return __bfloat162float(__float2bfloat16(v));
+}
+
 // sum of the S parts of four columns; loads of eight parts in flight
 DEV_INLINE st_f4 part_sum(const float *p, long stride, int S) {
   st_f4 v = *reinterpret_cast<const st_f4 *>(p);
@@ -228,9 +232,10 @@ DEV_INLINE st_f4 part_sum(const float *p, long stride, int S) {
   return v;
 }
 
+template <typename TB>
 __global__ __launch_bounds__(256) void stream_sum_kernel(
     __hip_bfloat16 *__restrict__ out, const float *__restrict__ part,
-    const __hip_bfloat16 *__restrict__ bias, long MN, int N, int S) {
+    const TB *__restrict__ bias, long MN, int N, int S) {
   const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
   const st_f4 v = part_sum(part + i, MN, S);
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(256) void stream_sum_kernel(
   shortx4 o;
 #pragma unroll
   for (int r = 0; r < 4; ++r)
-    o[r] = to_bf16(v[r] + (bias ? __bfloat162float(bias[n + r]) : 0.f));
+    o[r] = to_bf16(v[r] + (bias ? ScalarOps<TB>::to_f32(bias[n + r]) : 0.f));
   *reinterpret_cast<shortx4 *>(out + i) = o;
 }
 
@@ -248,7 +253,7 @@ template <int V, typename TW>
 __global__ __launch_bounds__(512) void stream_add_norm_kernel(
     __hip_bfloat16 *__restrict__ out, __hip_bfloat16 *__restrict__ residual,
     const float *__restrict__ part, const TW *__restrict__ w, float eps,
-    int M, int N, int S) {
+    int M, int N, int S, int rounded) {
   __shared__ float red[8];
   const long row = blockIdx.x;
   const long MN = (long)M * N;
@@ -257,7 +262,11 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
   for (int j = 0; j < V; ++j) {
     const int c = (j * 512 + threadIdx.x) * 4;
     if (c >= N) continue;
-    const st_f4 v = part_sum(part + row * N + c, MN, S);
+    st_f4 v = part_sum(part + row * N + c, MN, S);
+    if (rounded) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = bf16_value(v[r]);
+    }
     __hip_bfloat16 *rp = residual + row * N + c;
     const shortx4 old = *reinterpret_cast<const shortx4 *>(rp);
     shortx4 o;
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(256) void qkv_finish_kernel(
     long src_stride, const __hip_bfloat16 *__restrict__ bias,
     const long *__restrict__ positions, const float *__restrict__ cos_sin,
     const long *__restrict__ slots, int M, int S, int Hq, int Hkv, int D,
-    int rot) {
+    int rot, int rounded) {
   const long t = blockIdx.x;
   const int N = (Hq + 2 * Hkv) * D, per = D / 8;
   const float *cs = cos_sin + positions[t] * rot;
@@ -316,6 +325,10 @@ __global__ __launch_bounds__(256) void qkv_finish_kernel(
     if (bias) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] += __bfloat162float(bias[c + r]);
+    }
+    if (rounded) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = bf16_value(o[r]);
     }
   };
   const int i = blockIdx.y * 256 + threadIdx.x;
@@ -470,6 +483,32 @@ torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w) {
   return part;
 }
 
+// bf16 sum of fp32 parts [S, M, N] (N a multiple of 8) and a bias (bf16 or
+// fp32)
+torch::Tensor parts_sum(torch::Tensor part,
+                        c10::optional<torch::Tensor> bias) {
+  TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.is_contiguous() &&
+              part.scalar_type() == at::kFloat && part.size(2) % 8 == 0 &&
+              aligned16(part));
+  const int S = part.size(0);
+  const long M = part.size(1), N = part.size(2);
+  auto out = torch::empty({M, N}, part.options().dtype(at::kBFloat16));
+  if (M * N == 0) return out;
+  const bool wide = bias.has_value() && bias->scalar_type() == at::kFloat;
+  TORCH_CHECK(!wide || (bias->is_contiguous() && bias->numel() == N));
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define RUN(TB, BP)                                                          \
+  hipLaunchKernelGGL((stream_sum_kernel<TB>), dim3((M * N / 4 + 255) / 256), \
+                     dim3(256), 0, stream, (__hip_bfloat16 *)out.data_ptr(), \
+                     part.data_ptr<float>(), (const TB *)(BP), M * N,        \
+                     (int)N, S)
+  if (wide) RUN(float, bias->data_ptr());
+  else RUN(__hip_bfloat16, bias_ptr(bias, N));
+#undef RUN
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias) {
   check_operands(x, w);
@@ -482,16 +521,7 @@ torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
     launch<PLAIN>(p, out.data_ptr(), x, w, bp);
     return out;
   }
-  auto part = torch::empty({(long)p.splits, M, N},
-                           x.options().dtype(at::kFloat));
-  launch<PART>(p, part.data_ptr(), x, w, nullptr);
-  auto stream = at::cuda::getCurrentCUDAStream();
-  hipLaunchKernelGGL(stream_sum_kernel, dim3((M * N / 4 + 255) / 256),
-                     dim3(256), 0, stream, (__hip_bfloat16 *)out.data_ptr(),
-                     part.data_ptr<float>(), (const __hip_bfloat16 *)bp,
-                     M * N, (int)N, p.splits);
-  HIP_CHECK_KERNEL();
-  return out;
+  return parts_sum(stream_parts(x, w), bias);
 }
 
 // silu(x w_gate^T) * (x w_up^T), w = gate rows, up rows
@@ -506,25 +536,29 @@ torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w) {
   return out;
 }
 
-// residual (bf16 [M, N], in place) += x w^T; returns its RMS norm
-torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
-                              torch::Tensor residual, torch::Tensor norm_w,
-                              double eps) {
-  auto part = stream_parts(x, w);
+// residual (bf16 [M, N], in place) += the sum of the fp32 parts [S, M, N]
+// (rounded: rounded to bf16 first); returns its RMS norm
+torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
+                             torch::Tensor norm_w, double eps,
+                             bool rounded) {
+  TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.is_contiguous() &&
+              part.scalar_type() == at::kFloat && part.size(2) % 8 == 0 &&
+              aligned16(part));
   const int S = part.size(0), M = part.size(1), N = part.size(2);
   TORCH_CHECK(residual.scalar_type() == at::kBFloat16 &&
               residual.is_contiguous() && residual.numel() == (long)M * N &&
               aligned16(residual));
   TORCH_CHECK(norm_w.is_contiguous() && norm_w.numel() == N &&
               N <= 512 * 4 * 4, "stream_add_norm: at most 8192 columns");
-  auto out = torch::empty({(long)M, (long)N}, x.options());
+  auto out = torch::empty({(long)M, (long)N}, residual.options());
+  if (M == 0) return out;
   auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(V, TW)                                                           \
   hipLaunchKernelGGL((stream_add_norm_kernel<V, TW>), dim3(M), dim3(512), 0, \
                      stream, (__hip_bfloat16 *)out.data_ptr(),               \
                      (__hip_bfloat16 *)residual.data_ptr(),                  \
                      part.data_ptr<float>(), (const TW *)norm_w.data_ptr(),  \
-                     (float)eps, M, N, S)
+                     (float)eps, M, N, S, (int)rounded)
 #define COLS(TW)                                                             \
   do {                                                                       \
     if (N <= 2048) RUN(1, TW);                                               \
@@ -541,13 +575,20 @@ torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
   return out;
 }
 
+// residual (bf16 [M, N], in place) += x w^T; returns its RMS norm
+torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
+                              torch::Tensor residual, torch::Tensor norm_w,
+                              double eps) {
+  return parts_add_norm(stream_parts(x, w), residual, norm_w, eps, false);
+}
+
 // src: bf16 rows [M, (Hq + 2 Hkv) D] (a row view is fine) or the fp32 parts
-// of the same. Rotates (rotate-half on the first `rot` dims) queries and
+// of the same (rounded: rounded to bf16, with the bias, first). Rotates (rotate-half on the first `rot` dims) queries and
 // keys, writes keys and values to their slots, returns the queries.
 torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
                          torch::Tensor positions, torch::Tensor cos_sin,
                          torch::Tensor k_cache, torch::Tensor v_cache,
-                         torch::Tensor slots, long Hq) {
+                         torch::Tensor slots, long Hq, bool rounded) {
   const bool parts = src.dim() == 3;
   const long M = src.size(parts ? 1 : 0), N = src.size(parts ? 2 : 1);
   const int Hkv = k_cache.size(2), D = k_cache.size(3);
@@ -584,7 +625,7 @@ torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
                      (const __hip_bfloat16 *)bp, positions.data_ptr<long>(), \
                      cos_sin.data_ptr<float>(), slots.data_ptr<long>(),      \
                      (int)M, parts ? (int)src.size(0) : 1, (int)Hq, Hkv, D,  \
-                     rot)
+                     rot, (int)rounded)
   if (parts) RUN(true); else RUN(false);
 #undef RUN
   HIP_CHECK_KERNEL();

@@ -41,7 +41,8 @@ CORE_SOURCES = ["bindings.cpp", "norm.hip", "elementwise.hip",
                 "attention_decode.hip", "attention_prefill.hip",
                 "attention_mla.hip", "mla_proj.hip", "moe.hip",
                 "moe_tiled.hip", "fp8.hip",
-                "gdn.hip", "int4.hip", "stream_gemm.hip", "sampling.hip",
+                "gdn.hip", "int4.hip", "quant_gemm.hip", "stream_gemm.hip",
+                "sampling.hip",
                 "custom_ar.hip"]
 
 
