@@ -8,9 +8,10 @@
 
 namespace {
 
-template <typename T, int BLOCK>
+// (TW: the weight's own type, T or fp32)
+template <typename T, typename TW, int BLOCK>
 __global__ void rmsnorm_kernel(T *__restrict__ out, const T *__restrict__ in,
-                               const T *__restrict__ weight, float eps,
+                               const TW *__restrict__ weight, float eps,
                                int hidden) {
   __shared__ float red[BLOCK / WAVE_SIZE];
   const int row = blockIdx.x;
@@ -31,10 +32,9 @@ __global__ void rmsnorm_kernel(T *__restrict__ out, const T *__restrict__ in,
 
   for (int i = threadIdx.x; i < nvec; i += BLOCK) {
     shortx8 p = reinterpret_cast<const shortx8 *>(x)[i];
-    shortx8 w = reinterpret_cast<const shortx8 *>(weight)[i];
     float v[8], wv[8];
     unpack8<T>(p, v);
-    unpack8<T>(w, wv);
+    ld8<TW>(weight + i * 8, wv);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = v[j] * inv * wv[j];
     reinterpret_cast<shortx8 *>(o)[i] = pack8<T>(v);
@@ -44,10 +44,10 @@ __global__ void rmsnorm_kernel(T *__restrict__ out, const T *__restrict__ in,
 // residual += x; x = rmsnorm(residual) — both in place.
 // The summed row is staged in LDS (bf16, exactly what was stored to
 // residual) so the normalize pass re-reads LDS instead of HBM.
-template <typename T, int BLOCK>
+template <typename T, typename TW, int BLOCK>
 __global__ void fused_add_rmsnorm_kernel(T *__restrict__ x,
                                          T *__restrict__ residual,
-                                         const T *__restrict__ weight,
+                                         const TW *__restrict__ weight,
                                          float eps, int hidden) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T *srow = reinterpret_cast<T *>(smem_raw);
@@ -81,10 +81,9 @@ __global__ void fused_add_rmsnorm_kernel(T *__restrict__ x,
 
   for (int i = threadIdx.x; i < nvec; i += BLOCK) {
     shortx8 p = reinterpret_cast<const shortx8 *>(srow)[i];
-    shortx8 w = reinterpret_cast<const shortx8 *>(weight)[i];
     float v[8], wv[8];
     unpack8<T>(p, v);
-    unpack8<T>(w, wv);
+    ld8<TW>(weight + i * 8, wv);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = v[j] * inv * wv[j];
     reinterpret_cast<shortx8 *>(xr)[i] = pack8<T>(v);
@@ -107,6 +106,19 @@ __global__ void fused_add_rmsnorm_kernel(T *__restrict__ x,
     }                                                                       \
   } while (0)
 
+namespace {
+
+// true: the weight is fp32 (a third type is converted to it), false: of the
+// rows' type
+bool wide_weight(torch::Tensor &weight, const torch::Tensor &x, int hidden) {
+  TORCH_CHECK(weight.numel() >= hidden && weight.is_contiguous());
+  if (weight.scalar_type() == x.scalar_type()) return false;
+  weight = weight.to(at::kFloat);
+  return true;
+}
+
+}  // namespace
+
 void rmsnorm(torch::Tensor out, torch::Tensor in, torch::Tensor weight,
              double eps) {
   const int hidden = in.size(-1);
@@ -115,14 +127,16 @@ void rmsnorm(torch::Tensor out, torch::Tensor in, torch::Tensor weight,
   TORCH_CHECK(in.is_contiguous() && out.is_contiguous());
   constexpr int BLOCK = 256;
   auto stream = at::cuda::getCurrentCUDAStream();
+  const bool wide = wide_weight(weight, in, hidden);
+#define RUN(TW)                                                              \
+  hipLaunchKernelGGL((rmsnorm_kernel<scalar_t, TW, BLOCK>), dim3(rows),      \
+                     dim3(BLOCK), 0, stream, (scalar_t *)out.data_ptr(),     \
+                     (const scalar_t *)in.data_ptr(),                        \
+                     (const TW *)weight.data_ptr(), (float)eps, hidden)
   DISPATCH_16BIT(in, "rmsnorm", {
-    hipLaunchKernelGGL((rmsnorm_kernel<scalar_t, BLOCK>), dim3(rows),
-                       dim3(BLOCK), 0, stream,
-                       (scalar_t *)out.data_ptr(),
-                       (const scalar_t *)in.data_ptr(),
-                       (const scalar_t *)weight.data_ptr(), (float)eps,
-                       hidden);
+    if (wide) RUN(float); else RUN(scalar_t);
   });
+#undef RUN
   HIP_CHECK_KERNEL();
 }
 
@@ -135,13 +149,16 @@ void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
   constexpr int BLOCK = 256;
   const int lds = hidden * x.element_size();
   auto stream = at::cuda::getCurrentCUDAStream();
+  const bool wide = wide_weight(weight, x, hidden);
+#define RUN(TW)                                                              \
+  hipLaunchKernelGGL((fused_add_rmsnorm_kernel<scalar_t, TW, BLOCK>),        \
+                     dim3(rows), dim3(BLOCK), lds, stream,                   \
+                     (scalar_t *)x.data_ptr(),                               \
+                     (scalar_t *)residual.data_ptr(),                        \
+                     (const TW *)weight.data_ptr(), (float)eps, hidden)
   DISPATCH_16BIT(x, "fused_add_rmsnorm", {
-    hipLaunchKernelGGL((fused_add_rmsnorm_kernel<scalar_t, BLOCK>),
-                       dim3(rows), dim3(BLOCK), lds, stream,
-                       (scalar_t *)x.data_ptr(),
-                       (scalar_t *)residual.data_ptr(),
-                       (const scalar_t *)weight.data_ptr(), (float)eps,
-                       hidden);
+    if (wide) RUN(float); else RUN(scalar_t);
   });
+#undef RUN
   HIP_CHECK_KERNEL();
 }
