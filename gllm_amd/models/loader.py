@@ -118,17 +118,19 @@ def _flatten_text_config(cfg):
 
 def _normalize_rope(cfg):
     """transformers >= 5 renamed rope_scaling -> rope_parameters (with
-    rope_theta folded in); the model classes read the classic names."""
-    if getattr(cfg, "rope_scaling", None) is None:
-        rp = getattr(cfg, "rope_parameters", None)
-        if isinstance(rp, dict) and rp:
-            try:
-                cfg.rope_scaling = dict(rp)
-                if rp.get("rope_theta") is not None and \
-                        getattr(cfg, "rope_theta", None) is None:
-                    cfg.rope_theta = rp["rope_theta"]
-            except Exception:  # frozen config object
-                pass
+    rope_theta folded in, and rope_scaling an alias of it); the model
+    classes read the classic names."""
+    rp = getattr(cfg, "rope_parameters", None)
+    if not isinstance(rp, dict) or not rp:
+        return cfg
+    try:
+        if getattr(cfg, "rope_scaling", None) is None:
+            cfg.rope_scaling = dict(rp)
+        if rp.get("rope_theta") is not None and \
+                getattr(cfg, "rope_theta", None) is None:
+            cfg.rope_theta = rp["rope_theta"]
+    except Exception:  # frozen config object
+        pass
     return cfg
 
 
