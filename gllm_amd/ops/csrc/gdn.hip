@@ -134,37 +134,100 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 
 
 // ------------------------------------------------- chunked WY prefill
-// Chunk-parallel gated delta rule (WY form) over a ragged batch, all in fp32
-// (V_MFMA_F32_16X16X4_F32), in two kernels:
+// Chunk-parallel gated delta rule (WY form) over a ragged batch, in two
+// kernels (t, i: rows of a chunk; k, q: the unit keys and queries):
 //
 //   local   one workgroup per (64-token chunk, v-head), all chunks at once:
-//           unit keys, A = strict tril(beta_t exp(b_t - b_i) k_t k_i), and
-//           X = (I + A)^-1 [beta B k | beta v] by blocks of 16 rows (their
-//           inverses by substitution, the rest as products), att =
+//           A = strict tril(beta_t exp(b_t - b_i) k_t k_i), T = (I + A)^-1 by
+//           blocks of 16 rows, X = T [beta B k | beta v] and att =
 //           tril(exp(b_t - b_i) q_t k_i). b is the running log decay.
 //   carry   one workgroup per (sequence, v-head, DVS value columns), chunk
 //           after chunk: U = X_v - X_k S^T, o = B q S^T + att U,
 //           S = B_last S + (exp(b_last - b) U)^T k, with its columns of S in
-//           accumulators and LDS and the next chunk's operands on their way
-//           into registers.
-// Only what needs the state is serial: 224 matrix instructions a wave and
-// chunk at 32 columns. One kernel that did all of it chunk after chunk, a
-// workgroup per (sequence, head, 64 columns) and the substitution on one
-// wave, took 922 us for 4096 tokens in four prompts, 16 heads of 128; these
-// take 212 (local; five rounds of workgroups, one per CU by its LDS) and
-// 200 us (carry; the serial chain of the longest prompt, 3 us of matrix
-// instructions a chunk). X and att are 168 MB of traffic, 34 us.
+//           accumulators and the next chunk's operands on their way into
+//           registers.
+//
+// Keys, queries and values are bf16 and enter the matrix instructions as they
+// are, their norms as fp32 factors of the sums; an fp32 operand (T, X_k, att,
+// U, S) is the sum of three bf16 numbers, 24 bits in all, and a product of
+// two such takes the six partial products above 2^-24. That is 3 (6)
+// instructions of 16 cycles for 32 terms where fp32 ones take 8 of 32.
+// Accumulation, T and the state stay fp32. Error of the state against 64
+// bits, 64 to 1500 tokens, weak and strong decay: 1.1e-7 to 5.2e-7 (1.7e-7 to
+// 5.3e-7 with fp32 instructions, mean 2.5e-7 against 2.9e-7).
+// 4096 tokens in four prompts, 16 heads of 128: 60 + 150 us (212 + 200 with
+// fp32 instructions throughout and the triangular system solved column strip
+// by column strip; 922 for one kernel that did all of it chunk after chunk on
+// a workgroup per sequence, head and 64 columns). local is bound by its
+// stores (X, att: 105 MB); carry by the serial chain of the longest prompt, a
+// chunk's operands arriving (110 KB a workgroup) and two barriers.
 typedef __attribute__((ext_vector_type(4))) float gdn_f4;
+typedef __attribute__((ext_vector_type(8))) __bf16 gdn_bf8;
+typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
+
+union GdnFrag {
+  gdn_bf8 v;
+  shortx8 s;
+  shortx4 h[2];
+};
 
 constexpr int C = 64;     // tokens of a chunk
 constexpr int D = 128;    // key and value size of a head
-constexpr int KS = 132;   // LDS row of 128 floats: rows 4 banks apart
-constexpr int AS = 68;    // of 64 floats
-constexpr int XS = 272;   // of 256 floats: rows 16 banks apart
-constexpr int US = 48;    // of 32 floats
+constexpr int AS = 68;    // LDS row of 64 floats: rows 4 banks apart
+constexpr int KB = 144;   // of 128 bf16, for transposed reads: 8 banks
+constexpr int SB = 136;   // of 128 bf16: 4 banks
+constexpr int UB = 72;    // of 64 bf16
 
 DEV_INLINE gdn_f4 mma4(float a, float b, gdn_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+DEV_INLINE gdn_f4 mma32(const GdnFrag &a, const GdnFrag &b, gdn_f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, c, 0, 0, 0);
+}
+
+DEV_INLINE gdn_f4 mma6(const GdnFrag (&a)[3], const GdnFrag (&b)[3],
+                       gdn_f4 c) {
+  c = mma32(a[2], b[0], c);
+  c = mma32(a[0], b[2], c);
+  c = mma32(a[1], b[1], c);
+  c = mma32(a[1], b[0], c);
+  c = mma32(a[0], b[1], c);
+  return mma32(a[0], b[0], c);
+}
+
+// x as a sum of three bf16 numbers
+DEV_INLINE void split3(float x, short &h, short &m, short &l) {
+  const __hip_bfloat16 a = __float2bfloat16(x);
+  x -= __bfloat162float(a);
+  const __hip_bfloat16 b = __float2bfloat16(x);
+  x -= __bfloat162float(b);
+  h = __builtin_bit_cast(short, a);
+  m = __builtin_bit_cast(short, b);
+  l = __builtin_bit_cast(short, __float2bfloat16(x));
+}
+
+DEV_INLINE void split3(gdn_f4 x, shortx4 (&p)[3]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    short h, m, l;
+    split3(x[r], h, m, l);
+    p[0][r] = h;
+    p[1][r] = m;
+    p[2][r] = l;
+  }
+}
+
+// fragment of the transpose of an LDS tile with rows of `ld`: lane l16 is
+// column col0 + l16, elements rows row0 + 4 lhi + 0..3 and + 16
+DEV_INLINE void read_tr(GdnFrag &f, const short *tile, int ld, int row0,
+                        int col0, int l16, int lhi) {
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+    f.h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_shortx4 *)(tile +
+                        (row0 + half * 16 + lhi * 4 + (l16 >> 2)) * ld +
+                        col0 + (l16 & 3) * 4));
 }
 
 DEV_INLINE float sigmoid_f(float x) { return 1.f / (1.f + __expf(-x)); }
@@ -189,10 +252,11 @@ struct Gates {
   }
 };
 
-__global__ __launch_bounds__(256) void gdn_local_kernel(
-    float *__restrict__ wk, float *__restrict__ u0,  // X_k, X_v [T, Hv, D]
-    float *__restrict__ att,                         // [T, Hv, C]
-    float *__restrict__ scal,                        // [3, T, Hv]: b, 1/|k|, scale/|q|
+__global__ __launch_bounds__(512) void gdn_local_kernel(
+    short *__restrict__ wk,    // X_k, bf16 [3, T, Hv, D]
+    float *__restrict__ u0,    // X_v [T, Hv, D]
+    short *__restrict__ att,   // bf16 [3, T, Hv, C]
+    float *__restrict__ scal,  // [3, T, Hv]: b, 1/|k|, scale/|q|
     const __hip_bfloat16 *__restrict__ q, const __hip_bfloat16 *__restrict__ k,
     const __hip_bfloat16 *__restrict__ v, long qk_stride, long v_stride,
     Gates gates, const int *__restrict__ qsl, long T, int Hk, int Hv,
@@ -204,40 +268,42 @@ __global__ __launch_bounds__(256) void gdn_local_kernel(
   const int hk = h / (Hv / Hk);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, lhi = lane >> 4;
-  __shared__ float Kt[C * KS];
-  __shared__ float X[C * XS];     // q first, the solution afterwards
-  __shared__ float Am[C * AS];
-  __shared__ float Di[4][16 * 20];
-  __shared__ float bb[C], btv[C];
-  float *Qt = X;
+  __shared__ __attribute__((aligned(16))) short Kt[C * KB], Vt[C * KB];
+  __shared__ __attribute__((aligned(16))) float Am[C * AS], Tm[C * AS];
+  __shared__ __attribute__((aligned(16))) float bb[C], btv[C], rkv[C],
+      rqv[C], ck[C];
 
-  // ---- 16 rows of a wave: unit keys and queries
-  unsigned kr[16], qr[16];
+  // ---- keys and values to LDS (rows past the end: the last one, factors
+  // 0), norms of keys and queries: 16 lanes per row
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int t = wave * 16 + r;
-    const long row = (long)(start + min(t, len - 1)) * qk_stride + hk * D;
-    kr[r] = reinterpret_cast<const unsigned *>(k + row)[lane];
-    qr[r] = reinterpret_cast<const unsigned *>(q + row)[lane];
-  }
+  for (int j = 0; j < 2; ++j) {
+    const int u = j * 512 + tid, t = u >> 4, c = (u & 15) * 8;
+    const long row = start + min(t, len - 1);
+    const shortx8 kr = *reinterpret_cast<const shortx8 *>(
+        k + row * qk_stride + hk * D + c);
+    const shortx8 qr = *reinterpret_cast<const shortx8 *>(
+        q + row * qk_stride + hk * D + c);
+    *reinterpret_cast<shortx8 *>(Vt + t * KB + c) =
+        *reinterpret_cast<const shortx8 *>(v + row * v_stride + h * D + c);
+    *reinterpret_cast<shortx8 *>(Kt + t * KB + c) = kr;
+    float kf[8], qf[8], nk = 0.f, nq = 0.f;
+    unpack8<__hip_bfloat16>(kr, kf);
+    unpack8<__hip_bfloat16>(qr, qf);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int t = wave * 16 + r;
-    float k0 = __uint_as_float(kr[r] << 16);
-    float k1 = __uint_as_float(kr[r] & 0xffff0000u);
-    float q0 = __uint_as_float(qr[r] << 16);
-    float q1 = __uint_as_float(qr[r] & 0xffff0000u);
+    for (int e = 0; e < 8; ++e) {
+      nk += kf[e] * kf[e];
+      nq += qf[e] * qf[e];
+    }
     const float live = t < len ? 1.f : 0.f;
-    const float rk = live * rsqrtf(wave_reduce_sum(k0 * k0 + k1 * k1) + 1e-6f);
-    const float rq =
-        live * rsqrtf(wave_reduce_sum(q0 * q0 + q1 * q1) + 1e-6f) * scale;
-    *reinterpret_cast<floatx2 *>(Kt + t * KS + lane * 2) =
-        floatx2{k0 * rk, k1 * rk};
-    *reinterpret_cast<floatx2 *>(Qt + t * KS + lane * 2) =
-        floatx2{q0 * rq, q1 * rq};
-    if (lane == 0 && t < len) {
-      scal[(T + start + t) * Hv + h] = rk;
-      scal[(2 * T + start + t) * Hv + h] = rq;
+    const float rk = live * rsqrtf(lanes_sum<16>(nk) + 1e-6f);
+    const float rq = live * rsqrtf(lanes_sum<16>(nq) + 1e-6f) * scale;
+    if (c == 0) {
+      rkv[t] = rk;
+      rqv[t] = rq;
+      if (t < len) {
+        scal[(T + row) * Hv + h] = rk;
+        scal[(2 * T + row) * Hv + h] = rq;
+      }
     }
   }
   if (wave == 0) {  // running log decay
@@ -253,45 +319,57 @@ __global__ __launch_bounds__(256) void gdn_local_kernel(
     if (lane < len) scal[(long)(start + lane) * Hv + h] = gv;
   }
   __syncthreads();
+  if (tid < C) ck[tid] = btv[tid] * __expf(bb[tid]) * rkv[tid];
 
-  // ---- rows 16 w .. + 15 of A and att (blocks on and below the diagonal)
-  for (int it = 0; it <= wave; ++it) {
-    gdn_f4 a = {0, 0, 0, 0}, s = {0, 0, 0, 0};
-#pragma unroll 8
-    for (int ks = 0; ks < D / 4; ++ks) {
-      const float ki = Kt[(it * 16 + l16) * KS + ks * 4 + lhi];
-      a = mma4(Kt[(wave * 16 + l16) * KS + ks * 4 + lhi], ki, a);
-      s = mma4(Qt[(wave * 16 + l16) * KS + ks * 4 + lhi], ki, s);
+  // ---- blocks on and below the diagonal of A and att, a wave each
+  for (int blk = wave; blk < 12; blk += 8) {
+    // 0..9: (R, I) row by row; 10, 11: (0, 1) and (2, 3), zero
+    int R = blk < 1 ? 0 : blk < 3 ? 1 : blk < 6 ? 2 : 3;
+    int I = blk - R * (R + 1) / 2;
+    if (blk >= 10) {
+      R = (blk - 10) * 2;
+      I = R + 1;
     }
-    const int i = it * 16 + l16;
+    gdn_f4 a = {0, 0, 0, 0}, s = {0, 0, 0, 0};
+    if (blk < 10) {
+      const long qrow = start + min(R * 16 + l16, len - 1);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        GdnFrag ki, kt, qt;
+        const int c = ks * 32 + lhi * 8;
+        ki.s = *reinterpret_cast<const shortx8 *>(Kt + (I * 16 + l16) * KB + c);
+        kt.s = *reinterpret_cast<const shortx8 *>(Kt + (R * 16 + l16) * KB + c);
+        qt.s = *reinterpret_cast<const shortx8 *>(q + qrow * qk_stride +
+                                                  hk * D + c);
+        a = mma32(kt, ki, a);  // lane: i = l16, t = 4 lhi + r
+        s = mma32(ki, qt, s);  // lane: t = l16, i = 4 lhi + r
+      }
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int t = wave * 16 + lhi * 4 + r;
-      const float d = i <= t ? __expf(bb[t] - bb[i]) : 0.f;
-      Am[t * AS + i] = i < t ? btv[t] * d * a[r] : 0.f;
-      if (t < len) att[((long)(start + t) * Hv + h) * C + i] = d * s[r];
+      const int t = R * 16 + lhi * 4 + r, i = I * 16 + l16;
+      const float d = i < t ? __expf(bb[t] - bb[i]) : 0.f;
+      Am[t * AS + i] = i < t ? btv[t] * d * rkv[t] * rkv[i] * a[r] : 0.f;
+      if (blk >= 10) Tm[t * AS + i] = 0.f;
+    }
+    const int t = R * 16 + l16, i0 = I * 16 + lhi * 4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      s[r] = i0 + r <= t ? __expf(bb[t] - bb[i0 + r]) * rqv[t] *
+                               rkv[i0 + r] * s[r]
+                         : 0.f;
+    if (t < len) {
+      shortx4 p[3];
+      split3(s, p);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        *reinterpret_cast<shortx4 *>(
+            att + ((j * T + start + t) * Hv + h) * C + i0) = p[j];
     }
   }
-  // right hand sides: waves 0, 1 the keys' columns, 2, 3 the values'
-  gdn_f4 x[4][4];
-  const int c0 = (wave & 1) * 64;
-#pragma unroll
-  for (int R = 0; R < 4; ++R)
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = R * 16 + lhi * 4 + r, c = c0 + n * 16 + l16;
-        if (wave < 2) {
-          x[R][n][r] = btv[t] * __expf(bb[t]) * Kt[t * KS + c];
-        } else {
-          const float vv = __bfloat162float(
-              v[(long)(start + min(t, len - 1)) * v_stride + h * D + c]);
-          x[R][n][r] = btv[t] * vv;  // (rows past the end: beta 0)
-        }
-      }
-  __syncthreads();  // A is there; q is not needed any more
-  {  // inverse of this wave's diagonal block, a column per lane
+  __syncthreads();
+  // ---- T: inverses of the diagonal blocks, a column per lane
+  if (wave < 4) {
     float y[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -303,47 +381,88 @@ __global__ __launch_bounds__(256) void gdn_local_kernel(
     }
     if (lhi == 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) Di[wave][i * 20 + l16] = y[i];
+      for (int i = 0; i < 16; ++i)
+        Tm[(wave * 16 + i) * AS + wave * 16 + l16] = y[i];
     }
   }
   __syncthreads();
-  float *xw = X + wave * 64;  // this wave's columns
-  float *dst = wave < 2 ? wk : u0;
-#pragma unroll
-  for (int R = 0; R < 4; ++R) {
-    for (int ks = 0; ks < R * 4; ++ks) {
-      const float a = -Am[(R * 16 + l16) * AS + ks * 4 + lhi];
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-        x[R][n] = mma4(a, xw[(ks * 4 + lhi) * XS + n * 16 + l16], x[R][n]);
-    }
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
+  // then the blocks below it: T_RI = -T_RR sum_J A_RJ T_JI
+  for (int d = 1; d < 4; ++d) {
+    const int I = wave, R = I + d;
+    gdn_f4 y = {0, 0, 0, 0};
+    if (R < 4) {
+      for (int c = I * 16; c < R * 16; c += 4)
+        y = mma4(Am[(R * 16 + l16) * AS + c + lhi],
+                 Tm[(c + lhi) * AS + I * 16 + l16], y);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        xw[(R * 16 + lhi * 4 + r) * XS + n * 16 + l16] = x[R][n][r];
-    __syncthreads();
-    gdn_f4 y[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) y[n] = gdn_f4{0, 0, 0, 0};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float a = Di[R][l16 * 20 + ks * 4 + lhi];
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-        y[n] = mma4(a, xw[(R * 16 + ks * 4 + lhi) * XS + n * 16 + l16], y[n]);
+        Tm[(R * 16 + lhi * 4 + r) * AS + I * 16 + l16] = y[r];
     }
     __syncthreads();
+    if (R < 4) {
+      y = gdn_f4{0, 0, 0, 0};
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = R * 16 + lhi * 4 + r;
-        xw[t * XS + n * 16 + l16] = y[n][r];
-        if (t < len)
-          dst[((long)(start + t) * Hv + h) * D + c0 + n * 16 + l16] = y[n][r];
-      }
+      for (int c = 0; c < 16; c += 4)
+        y = mma4(-Tm[(R * 16 + l16) * AS + R * 16 + c + lhi],
+                 Tm[(R * 16 + c + lhi) * AS + I * 16 + l16], y);
+    }
     __syncthreads();
+    if (R < 4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Tm[(R * 16 + lhi * 4 + r) * AS + I * 16 + l16] = y[r];
+    }
+    __syncthreads();
+  }
+  // ---- X, transposed: waves 0..3 the keys' columns, 4..7 the values'
+  const short *src = wave < 4 ? Kt : Vt;
+  const float *fac = wave < 4 ? ck : btv;
+  const int c0 = (wave & 3) * 32;
+  GdnFrag cols[2][2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      read_tr(cols[kk][n], src, KB, kk * 32, c0 + n * 16, l16, lhi);
+#pragma unroll
+  for (int R = 0; R < 4; ++R) {
+    gdn_f4 x[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int kk = 0; kk <= R / 2; ++kk) {
+      GdnFrag tf[3];
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int i = kk * 32 + half * 16 + lhi * 4;
+        gdn_f4 tv = *reinterpret_cast<const gdn_f4 *>(
+            Tm + (R * 16 + l16) * AS + i);
+        tv *= *reinterpret_cast<const gdn_f4 *>(fac + i);
+        shortx4 p[3];
+        split3(tv, p);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) tf[j].h[half] = p[j];
+      }
+#pragma unroll
+      for (int j = 2; j >= 0; --j)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) x[n] = mma32(cols[kk][n], tf[j], x[n]);
+    }
+    const int t = R * 16 + l16;
+    if (t >= len) continue;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int c = c0 + n * 16 + lhi * 4;
+      if (wave < 4) {
+        shortx4 p[3];
+        split3(x[n], p);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          *reinterpret_cast<shortx4 *>(
+              wk + ((j * T + start + t) * Hv + h) * D + c) = p[j];
+      } else {
+        *reinterpret_cast<gdn_f4 *>(
+            u0 + ((long)(start + t) * Hv + h) * D + c) = x[n];
+      }
+    }
   }
 }
 
@@ -352,8 +471,8 @@ template <int DVS>
 __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     __hip_bfloat16 *__restrict__ o,  // [T, Hv, D]
     float *__restrict__ states,      // [slots, Hv, D, D], in place
-    const float *__restrict__ wk, const float *__restrict__ u0,
-    const float *__restrict__ att, const float *__restrict__ scal,
+    const short *__restrict__ wk, const float *__restrict__ u0,
+    const short *__restrict__ att, const float *__restrict__ scal,
     const __hip_bfloat16 *__restrict__ q, const __hip_bfloat16 *__restrict__ k,
     long qk_stride, const long *__restrict__ slots,
     const int *__restrict__ has_init, const int *__restrict__ qsl, long T,
@@ -363,56 +482,82 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
   const int begin = qsl[seq], end = qsl[seq + 1];
   if (begin >= end) return;
   const int hk = h / (Hv / Hk);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lhi = lane >> 4;
-  __shared__ float Ws[C * KS], Ks[C * KS], Qs[C * KS], At[C * AS];
-  __shared__ float Ss[DVS * KS], Us[C * US];
-  __shared__ float bb[C];
+  __shared__ __attribute__((aligned(16))) short Kt[2][C * KB];
+  __shared__ __attribute__((aligned(16))) short Sp[3][DVS * SB];
+  // U and, for the state, exp(b_last - b) U / |k|; rows are value columns
+  __shared__ __attribute__((aligned(16))) short Up[6][DVS * UB];
+  __shared__ float sc[2][3][C];  // b, 1/|k|, scale/|q|
 
-  // S rows (values) vt * 16 + lhi * 4 + r, columns (keys) of this wave's
-  // two tiles
+  // S transposed: lane value column vt * 16 + l16, keys (wave * 2 + dt) * 16
+  // + lhi * 4 + r
   float *sg = states + ((slots[seq] * Hv + h) * D + z * DVS) * D;
   gdn_f4 s[VT][2];
   const bool init = has_init[seq] != 0;
+  auto put_state = [&]() {
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) {
+        shortx4 p[3];
+        split3(s[vt][dt], p);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          *reinterpret_cast<shortx4 *>(
+              Sp[j] + (vt * 16 + l16) * SB + (wave * 2 + dt) * 16 +
+              lhi * 4) = p[j];
+      }
+  };
 #pragma unroll
   for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int vr = vt * 16 + lhi * 4 + r, d = (wave * 2 + dt) * 16 + l16;
-        s[vt][dt][r] = init ? sg[(long)vr * D + d] : 0.f;
-        Ss[vr * KS + d] = s[vt][dt][r];
-      }
+      s[vt][dt] = init ? *reinterpret_cast<const gdn_f4 *>(
+                             sg + (long)(vt * 16 + l16) * D +
+                             (wave * 2 + dt) * 16 + lhi * 4)
+                       : gdn_f4{0, 0, 0, 0};
+  put_state();
 
   // operands of a chunk, on their way in registers
-  floatx4 wr[8], ar[4];
-  shortx8 kr[4], qr[4];
-  float rk[4], rq[4], ur[VT][4], br;
+  shortx8 wr[4][3], ar[2][3], qr[4], kr[4];
+  float ur[VT][4], sr;
   auto fetch = [&](int start) {
     const int len = min(C, end - start);
+    {
+      const int t = wave * 16 + l16;
+      const bool live = t < len;
+      const long row = start + min(t, len - 1);
+      const shortx8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int u = j * 256 + tid, row = u >> 5, c = (u & 31) * 4;
-      wr[j] = row < len ? *reinterpret_cast<const floatx4 *>(
-                              wk + ((long)(start + row) * Hv + h) * D + c)
-                        : floatx4{0, 0, 0, 0};
+      for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          wr[ks][j] = live ? *reinterpret_cast<const shortx8 *>(
+                                 wk + ((j * T + row) * Hv + h) * D + ks * 32 +
+                                 lhi * 8)
+                           : zero;
+        qr[ks] = *reinterpret_cast<const shortx8 *>(
+            q + row * qk_stride + hk * D + ks * 32 + lhi * 8);
+      }
+      // (blocks past the diagonal's pair are never written, nor read)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          ar[kk][j] = live && kk <= wave / 2
+                          ? *reinterpret_cast<const shortx8 *>(
+                                att + ((j * T + row) * Hv + h) * C + kk * 32 +
+                                lhi * 8)
+                          : zero;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int u = j * 256 + tid, row = u >> 4, c = u & 15;
-      const bool live = row < len;
-      const long t = start + min(row, len - 1);
-      // (columns above the diagonal block are never read)
-      ar[j] = live ? *reinterpret_cast<const floatx4 *>(
-                         att + (t * Hv + h) * C + c * 4)
-                   : floatx4{0, 0, 0, 0};
-      kr[j] = *reinterpret_cast<const shortx8 *>(k + t * qk_stride + hk * D +
-                                                 c * 8);
-      qr[j] = *reinterpret_cast<const shortx8 *>(q + t * qk_stride + hk * D +
-                                                 c * 8);
-      rk[j] = live ? scal[(T + t) * Hv + h] : 0.f;
-      rq[j] = live ? scal[(2 * T + t) * Hv + h] : 0.f;
+      const int u = j * 256 + tid;
+      kr[j] = *reinterpret_cast<const shortx8 *>(
+          k + (long)(start + min(u >> 4, len - 1)) * qk_stride + hk * D +
+          (u & 15) * 8);
     }
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
@@ -423,68 +568,94 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
                                  vt * 16 + l16]
                             : 0.f;
       }
-    br = scal[(long)(start + min(lane, len - 1)) * Hv + h];
+    sr = scal[(min(wave, 2) * T + start + min(lane, len - 1)) * Hv + h];
   };
-  fetch(begin);
-  for (int start = begin; start < end; start += C) {
-    const int len = min(C, end - start);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int u = j * 256 + tid;
-      *reinterpret_cast<floatx4 *>(Ws + (u >> 5) * KS + (u & 31) * 4) = wr[j];
-    }
+  auto put_keys = [&](int buf) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int u = j * 256 + tid, row = u >> 4, c = u & 15;
-      *reinterpret_cast<floatx4 *>(At + row * AS + c * 4) = ar[j];
-      float kf[8], qf[8];
-      unpack8<__hip_bfloat16>(kr[j], kf);
-      unpack8<__hip_bfloat16>(qr[j], qf);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        kf[e] *= rk[j];
-        qf[e] *= rq[j];
-      }
-      st8<float>(Ks + row * KS + c * 8, kf);
-      st8<float>(Qs + row * KS + c * 8, qf);
+      const int u = j * 256 + tid;
+      *reinterpret_cast<shortx8 *>(Kt[buf] + (u >> 4) * KB + (u & 15) * 8) =
+          kr[j];
     }
-    if (wave == 0) bb[lane] = br;
+    if (wave < 3) sc[buf][wave][lane] = sr;
+  };
+  fetch(begin);
+  put_keys(0);
+  __syncthreads();
+  int cur = 0;
+  for (int start = begin; start < end; start += C) {
+    const int len = min(C, end - start);
+    GdnFrag w[4][3], at[2][3], qf[4];
     gdn_f4 u[VT];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) w[ks][j].s = wr[ks][j];
+      qf[ks].s = qr[ks];
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) at[kk][j].s = ar[kk][j];
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
       u[vt] = gdn_f4{ur[vt][0], ur[vt][1], ur[vt][2], ur[vt][3]};
-    __syncthreads();
     if (start + C < end) fetch(start + C);
 
-    // ---- U = X_v - X_k S^T and B q S^T, rows 16 w ..
-    gdn_f4 qs[VT];
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt) qs[vt] = gdn_f4{0, 0, 0, 0};
-#pragma unroll 8
-    for (int ks = 0; ks < D / 4; ++ks) {
-      const float w = -Ws[(wave * 16 + l16) * KS + ks * 4 + lhi];
-      const float qv = Qs[(wave * 16 + l16) * KS + ks * 4 + lhi];
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        const float sv = Ss[(vt * 16 + l16) * KS + ks * 4 + lhi];
-        u[vt] = mma4(w, sv, u[vt]);
-        qs[vt] = mma4(qv, sv, qs[vt]);
-      }
-    }
+    // ---- U = X_v - X_k S^T and q S^T, rows 16 w ..
+    gdn_f4 xs[VT], qs[VT];
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
+      xs[vt] = qs[vt] = gdn_f4{0, 0, 0, 0};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        Us[(wave * 16 + lhi * 4 + r) * US + vt * 16 + l16] = u[vt][r];
-        qs[vt][r] *= __expf(bb[wave * 16 + lhi * 4 + r]);
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        GdnFrag sf[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          sf[j].s = *reinterpret_cast<const shortx8 *>(
+              Sp[j] + (vt * 16 + l16) * SB + ks * 32 + lhi * 8);
+        xs[vt] = mma6(w[ks], sf, xs[vt]);
+#pragma unroll
+        for (int j = 2; j >= 0; --j) qs[vt] = mma32(qf[ks], sf[j], qs[vt]);
       }
-    __syncthreads();
-    // ---- o = that + att U (columns up to the diagonal block)
-    for (int ks = 0; ks < (wave + 1) * 4; ++ks) {
-      const float a = At[(wave * 16 + l16) * AS + ks * 4 + lhi];
+    const float last = sc[cur][0][len - 1];
+    gdn_f4 wc, eb;
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-        qs[vt] = mma4(a, Us[(ks * 4 + lhi) * US + vt * 16 + l16], qs[vt]);
+    for (int r = 0; r < 4; ++r) {
+      const int t = wave * 16 + lhi * 4 + r;
+      wc[r] = __expf(last - sc[cur][0][t]) * sc[cur][1][t];
+      eb[r] = __expf(sc[cur][0][t]) * sc[cur][2][t];
+    }
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) {
+      u[vt] -= xs[vt];
+      qs[vt] *= eb;
+      shortx4 p[3], pw[3];
+      split3(u[vt], p);
+      split3(u[vt] * wc, pw);
+      const int at_u = (vt * 16 + l16) * UB + wave * 16 + lhi * 4;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        *reinterpret_cast<shortx4 *>(Up[j] + at_u) = p[j];
+        *reinterpret_cast<shortx4 *>(Up[3 + j] + at_u) = pw[j];
+      }
+    }
+    __syncthreads();
+    // ---- o = B q S^T + att U
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      if (kk > wave / 2) continue;
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        GdnFrag uf[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          uf[j].s = *reinterpret_cast<const shortx8 *>(
+              Up[j] + (vt * 16 + l16) * UB + kk * 32 + lhi * 8);
+        qs[vt] = mma6(at[kk], uf, qs[vt]);
+      }
     }
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
@@ -496,47 +667,43 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
               __float2bfloat16(qs[vt][r]);
       }
     // ---- S = B_last S + (exp(b_last - b) U)^T k
-    const float last = bb[len - 1], keep = __expf(last);
+    const float keep = __expf(last);
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
+      for (int dt = 0; dt < 2; ++dt) s[vt][dt] *= keep;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[vt][dt][r] *= keep;
-#pragma unroll 4
-    for (int ks = 0; ks < C / 4; ++ks) {
-      const int t = ks * 4 + lhi;
-      const float wc = __expf(last - bb[t]);
-      float kv[2];
+    for (int kk = 0; kk < 2; ++kk) {
+      GdnFrag kf[2];
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt)
-        kv[dt] = Ks[t * KS + (wave * 2 + dt) * 16 + l16];
+        read_tr(kf[dt], Kt[cur], KB, kk * 32, (wave * 2 + dt) * 16, l16, lhi);
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        const float uv = wc * Us[t * US + vt * 16 + l16];
+      for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
-        for (int dt = 0; dt < 2; ++dt)
-          s[vt][dt] = mma4(uv, kv[dt], s[vt][dt]);
-      }
+        for (int j = 2; j >= 0; --j) {
+          GdnFrag uf;
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+            uf.h[half] = *reinterpret_cast<const shortx4 *>(
+                Up[3 + j] + (vt * 16 + l16) * UB + kk * 32 + half * 16 +
+                lhi * 4);
+#pragma unroll
+          for (int dt = 0; dt < 2; ++dt)
+            s[vt][dt] = mma32(kf[dt], uf, s[vt][dt]);
+        }
     }
-    __syncthreads();  // everybody is done with this chunk's operands and S
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          Ss[(vt * 16 + lhi * 4 + r) * KS + (wave * 2 + dt) * 16 + l16] =
-              s[vt][dt][r];
+    put_state();
+    if (start + C < end) put_keys(cur ^ 1);
+    cur ^= 1;
+    __syncthreads();  // S is there, this chunk's U and keys have been read
   }
 #pragma unroll
   for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sg[(long)(vt * 16 + lhi * 4 + r) * D + (wave * 2 + dt) * 16 + l16] =
-            s[vt][dt][r];
+      *reinterpret_cast<gdn_f4 *>(sg + (long)(vt * 16 + l16) * D +
+                                  (wave * 2 + dt) * 16 + lhi * 4) = s[vt][dt];
 }
 
 // ------------------------------------------------- one token per sequence
@@ -696,14 +863,15 @@ void run_chunks(torch::Tensor &o, const void *q, const void *k,
                 const int *has_init, const int *qsl, long T, int B,
                 int max_len, int Hk, int Hv, double scale) {
   auto opts = states.options();
-  auto wk = torch::empty({T, (long)Hv, (long)D}, opts);
+  auto bf = opts.dtype(at::kBFloat16);
+  auto wk = torch::empty({3, T, (long)Hv, (long)D}, bf);
   auto u0 = torch::empty({T, (long)Hv, (long)D}, opts);
-  auto att = torch::empty({T, (long)Hv, (long)C}, opts);
+  auto att = torch::empty({3, T, (long)Hv, (long)C}, bf);
   auto scal = torch::empty({3, T, (long)Hv}, opts);
   auto stream = at::cuda::getCurrentCUDAStream();
   hipLaunchKernelGGL(gdn_local_kernel, dim3((max_len + C - 1) / C, B, Hv),
-                     dim3(256), 0, stream, wk.data_ptr<float>(),
-                     u0.data_ptr<float>(), att.data_ptr<float>(),
+                     dim3(512), 0, stream, (short *)wk.data_ptr(),
+                     u0.data_ptr<float>(), (short *)att.data_ptr(),
                      scal.data_ptr<float>(), (const __hip_bfloat16 *)q,
                      (const __hip_bfloat16 *)k, (const __hip_bfloat16 *)v,
                      qk_stride, v_stride, gates, qsl, T, Hk, Hv,
@@ -712,8 +880,8 @@ void run_chunks(torch::Tensor &o, const void *q, const void *k,
 #define RUN(DVS)                                                             \
   hipLaunchKernelGGL((gdn_carry_kernel<DVS>), dim3(B, Hv, D / DVS),          \
                      dim3(256), 0, stream, (__hip_bfloat16 *)o.data_ptr(),   \
-                     states.data_ptr<float>(), wk.data_ptr<float>(),         \
-                     u0.data_ptr<float>(), att.data_ptr<float>(),            \
+                     states.data_ptr<float>(), (const short *)wk.data_ptr(), \
+                     u0.data_ptr<float>(), (const short *)att.data_ptr(),    \
                      scal.data_ptr<float>(), (const __hip_bfloat16 *)q,      \
                      (const __hip_bfloat16 *)k, qk_stride, slots, has_init,  \
                      qsl, T, Hk, Hv)

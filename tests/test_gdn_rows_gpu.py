@@ -83,6 +83,7 @@ def test_gdn_rows(lens, init, Hk, Hv):
         assert over.max() <= 1, [(i, float(x)) for i, x in enumerate(
             over.view(T, Hv, D).amax((1, 2))) if x > 1]
         rows = torch.tensor(slots)
+        # (three bf16 numbers hold an fp32 one to 2^-24: 32-bit sums)
         err = (s.cpu().double() - ref_state)[rows].abs().max()
         assert err <= 1e-5 * ref_state.abs().max().clamp(min=1)
         rest = torch.tensor([i for i in range(B + 2) if i not in slots])
