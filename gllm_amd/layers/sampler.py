@@ -10,6 +10,7 @@ from typing import List, Optional
 
 import torch
 
+from gllm_amd import ops
 from gllm_amd.ops import torch_ref
 
 
@@ -60,7 +61,7 @@ class Sampler(torch.nn.Module):
         if meta.bias_rows or meta.allowed_rows or meta.ban_rows:
             logits = self._apply_row_adjust(logits, meta)
         if meta.all_greedy:
-            next_tokens = logits.argmax(dim=-1)
+            next_tokens = ops.greedy_argmax(logits)
             return self._with_logprobs(logits, next_tokens, meta)
 
         logits = logits.float()
@@ -70,7 +71,6 @@ class Sampler(torch.nn.Module):
         if probs.is_cuda:
             # fused sorting-free radix-select kernel (in-place),
             # replaces the [B, V] sort composite below
-            from gllm_amd import ops
             if ops.has_kernels():
                 probs = probs.contiguous()
                 ops.topk_topp_filter(probs, meta.top_ks,

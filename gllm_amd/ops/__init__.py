@@ -687,6 +687,17 @@ def resolve_tokens(tokens: torch.Tensor, ring: torch.Tensor) -> torch.Tensor:
     return torch.where(tokens < 0, flat[idx], tokens)
 
 
+def greedy_argmax(logits: torch.Tensor) -> torch.Tensor:
+    """logits.argmax(-1) of [B, V]: the first of equals, a NaN as the
+    largest. (The kernel is in the core module only.)"""
+    if (logits.is_cuda and logits.dim() == 2 and logits.is_contiguous()
+            and logits.dtype in (torch.bfloat16, torch.float32)
+            and 0 < logits.shape[1] < 2 ** 30
+            and _load_kernels() is not None):
+        return _gpu_kernels().greedy_argmax(logits)
+    return logits.argmax(dim=-1)
+
+
 def topk_topp_filter(probs: torch.Tensor, top_ks: torch.Tensor,
                      top_ps: torch.Tensor,
                      min_ps: Optional[torch.Tensor] = None):

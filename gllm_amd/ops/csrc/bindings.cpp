@@ -136,6 +136,7 @@ void rmsnorm_gated(torch::Tensor out, torch::Tensor x, torch::Tensor z,
 void apply_repetition_penalty(torch::Tensor logits, torch::Tensor pool,
                               torch::Tensor slots,
                               torch::Tensor penalties);
+torch::Tensor greedy_argmax(torch::Tensor logits);
 void topk_topp_filter(torch::Tensor probs, torch::Tensor top_ks,
                       torch::Tensor top_ps,
                       c10::optional<torch::Tensor> min_ps);
@@ -220,6 +221,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_gated", &rmsnorm_gated, "rmsnorm(x)*w*silu(z)");
   m.def("apply_repetition_penalty", &apply_repetition_penalty,
         "scaling penalty vs persistent seen-token mask pool");
+  m.def("greedy_argmax", &greedy_argmax, "first largest value of each row");
   m.def("topk_topp_filter", &topk_topp_filter,
         "fused sorting-free top-k/top-p/min-p filter + renormalize");
   m.def("car_alloc", &car_alloc, "alloc hipIpc-shared AR buffer");
