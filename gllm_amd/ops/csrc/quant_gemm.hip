@@ -16,8 +16,11 @@
 // point took six operations a weight (91 % of the issue slots went there).
 // A matrix instruction with ones beside the weights' gives sum(x), and the
 // group enters as s * (part - 16 sum(x)) + b sum(x): the weights are not
-// rounded to bf16. A row whose sum is not finite (16 x - 16 x has no value
-// there) takes the group again with the weights formed one by one.
+// rounded to bf16. The terms of that form are up to 31 |x|, and 16 x - 16 x
+// has no value for an infinite x: a workgroup that ends with a result that is
+// not finite walks its weights once more, formed one by one (as bf16), for
+// those results. The results themselves are looked at, once: a row's sum may
+// be small where its terms are past 32 bits.
 //
 // fp8: what comes out is quantized to e4m3 again a kernel or two later, where
 // a last bit decides between neighbours; so the gated form and the readers of
@@ -25,13 +28,15 @@
 // gives what the separate one gives.
 //
 // (us, 29 rows; the kernels before these formed floats weight by weight and
-// did not fill the chip:) 55296 x 5120 int4 48, fp8 46 gated; 5120 x 27648 28
-// and 31; four products of a 5120-wide layer 100 (210) and 99. Weights come
-// at 4.6 (int4, 1 row) and 6.3 TB/s (fp8); int4 with 17 rows and more is
-// bound by its vector instructions.
+// did not fill the chip:) 55296 x 5120 int4 45, fp8 46 gated; 5120 x 27648 25
+// and 31; four products of a 5120-wide layer 89 (210) and 99. Weights come
+// at 4.1 (int4, 1 row) and 6.3 TB/s (fp8); int4 with 17 rows and more is
+// bound by its vector instructions. (int4 with a look at each group's row sum
+// in the loop: 49 and 26.)
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
+#include <type_traits>
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 qg_bf8;
@@ -286,157 +291,188 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
 
   const Offset offset;
   qg_f4 acc[NT][MT];
+  // One walk over the stages of this workgroup; FORMED (int4): the weights
+  // are formed one by one.
+  auto walk = [&](auto formed) {
+    constexpr bool FORMED = decltype(formed)::value;
 #pragma unroll
-  for (int n = 0; n < NT; ++n)
+    for (int n = 0; n < NT; ++n)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[n][m] = qg_f4{0, 0, 0, 0};
+      for (int m = 0; m < MT; ++m) acc[n][m] = qg_f4{0, 0, 0, 0};
 
 #pragma unroll
-  for (int i = 0; i < ST - 1; ++i)
-    if (i < nkt) stage(i);
-  int cur = 0, nxt = ST - 1;
-  for (int kt = 0; kt < nkt; ++kt) {
-    // this wave's loads of stage kt have landed, later ones may fly
-    wait_stages<ST - 2, LD>(min(nkt - 1 - kt, ST - 2));
-    // everybody's are there, and stage kt - 1 (the slot that the next one
-    // takes) has been read
-    __builtin_amdgcn_s_barrier();
-    if (kt + ST - 1 < nkt) stage(nxt);
-    const char *xb = smem + cur * STAGE + (wm * MT * 16 + l16) * XROW;
-    const char *wb = smem + cur * STAGE + W_OFF + (wn * NT * 16 + l16) * WROW;
-    const float *sb =
-        reinterpret_cast<const float *>(smem + cur * STAGE + S_OFF);
-    if constexpr (Q == INT4) {
+    for (int i = 0; i < ST - 1; ++i)
+      if (i < nkt) stage(i);
+    int cur = 0, nxt = ST - 1;
+    for (int kt = 0; kt < nkt; ++kt) {
+      // this wave's loads of stage kt have landed, later ones may fly
+      wait_stages<ST - 2, LD>(min(nkt - 1 - kt, ST - 2));
+      // everybody's are there, and stage kt - 1 (the slot that the next one
+      // takes) has been read
+      __builtin_amdgcn_s_barrier();
+      if (kt + ST - 1 < nkt) stage(nxt);
+      const char *xb = smem + cur * STAGE + (wm * MT * 16 + l16) * XROW;
+      const char *wb =
+          smem + cur * STAGE + W_OFF + (wn * NT * 16 + l16) * WROW;
+      const float *sb =
+          reinterpret_cast<const float *>(smem + cur * STAGE + S_OFF);
+      if constexpr (Q == INT4) {
 #pragma unroll
-      for (int i = 0; i < GS; ++i) {
-        qg_f4 part[NT][MT];
+        for (int i = 0; i < GS; ++i) {
+          qg_f4 part[NT][MT];
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
+          for (int n = 0; n < NT; ++n)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
-        const float *sg = sb + i * 2 * BN;
-        // lane lhi holds elements 32 lhi .. + 31 of its rows
-        qg_u4 wv[NT];
-        qg_f4 xsum[MT];
+            for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
+          const float *sg = sb + i * 2 * BN;
+          // lane lhi holds elements 32 lhi .. + 31 of its rows
+          qg_u4 wv[NT];
+          qg_f4 xsum[MT];
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-          wv[n] = *reinterpret_cast<const qg_u4 *>(
-              wb + n * 16 * WROW + (((i * 4 + lhi) ^ (l16 & 7)) << 4));
+          for (int n = 0; n < NT; ++n)
+            wv[n] = *reinterpret_cast<const qg_u4 *>(
+                wb + n * 16 * WROW + (((i * 4 + lhi) ^ (l16 & 7)) << 4));
 #pragma unroll
-        for (int m = 0; m < MT; ++m) xsum[m] = qg_f4{0, 0, 0, 0};
-        const qg_bf8 ones = __builtin_bit_cast(
-            qg_bf8, qg_u4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+          for (int m = 0; m < MT; ++m) xsum[m] = qg_f4{0, 0, 0, 0};
+          const qg_bf8 ones = __builtin_bit_cast(
+              qg_bf8,
+              qg_u4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          qg_bf8 xf[MT];
+          for (int j = 0; j < 4; ++j) {
+            qg_bf8 xf[MT];
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            xf[m] = weight_order(*reinterpret_cast<const qg_u4 *>(
-                xb + m * 16 * XROW + ((i * 16 + ((lhi * 4 + j) ^ l16)) << 4)));
-            xsum[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xf[m],
-                                                              xsum[m], 0, 0, 0);
+            for (int m = 0; m < MT; ++m) {
+              xf[m] = weight_order(*reinterpret_cast<const qg_u4 *>(
+                  xb + m * 16 * XROW +
+                  ((i * 16 + ((lhi * 4 + j) ^ l16)) << 4)));
+              if (!FORMED)
+                xsum[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    ones, xf[m], xsum[m], 0, 0, 0);
+            }
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+              const int cw = (wn * NT + n) * 16 + l16;
+              const qg_bf8 wf = FORMED ? scaled_weights(wv[n][j], sg[cw],
+                                                        sg[BN + cw])
+                                       : offset_weights(wv[n][j], offset);
+#pragma unroll
+              for (int m = 0; m < MT; ++m)
+                part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    wf, xf[m], part[n][m], 0, 0, 0);
+            }
           }
 #pragma unroll
           for (int n = 0; n < NT; ++n) {
-            const qg_bf8 wf = offset_weights(wv[n][j], offset);
+            if (FORMED) {
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
-              part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  wf, xf[m], part[n][m], 0, 0, 0);
-          }
-        }
-        bool finite[MT], all = true;
+              for (int m = 0; m < MT; ++m) acc[n][m] += part[n][m];
+              continue;
+            }
+            const int c = (wn * NT + n) * 16 + lhi * 4;
+            const qg_f4 s = *reinterpret_cast<const qg_f4 *>(sg + c);
+            qg_f4 b = *reinterpret_cast<const qg_f4 *>(sg + BN + c);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          finite[m] = fabsf(xsum[m][0]) < 1e36f;  // (false for NaN)
-          all &= finite[m];
-        }
-        const bool plain = __all(all);
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          const int c = (wn * NT + n) * 16 + lhi * 4;
-          const qg_f4 s = *reinterpret_cast<const qg_f4 *>(sg + c);
-          qg_f4 b = *reinterpret_cast<const qg_f4 *>(sg + BN + c);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) b[r] -= 16.f * s[r];
-          if (__builtin_expect(plain, 1)) {
+            for (int r = 0; r < 4; ++r) b[r] -= 16.f * s[r];
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
               for (int r = 0; r < 4; ++r)
                 acc[n][m][r] = fmaf(s[r], part[n][m][r],
                                     fmaf(b[r], xsum[m][r], acc[n][m][r]));
-            continue;
           }
-          const int cw = (wn * NT + n) * 16 + l16;
-          qg_bf8 wf[4];
+        }
+      } else {
+        qg_f4 part[NT][MT];
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            wf[j] = scaled_weights(wv[n][j], sg[cw], sg[BN + cw]);
+        for (int n = 0; n < NT; ++n)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            qg_f4 one = qg_f4{0, 0, 0, 0};
+          for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
+        float ws[NT];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              one = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  wf[j],
-                  weight_order(*reinterpret_cast<const qg_u4 *>(
-                      xb + m * 16 * XROW +
-                      ((i * 16 + ((lhi * 4 + j) ^ l16)) << 4))),
-                  one, 0, 0, 0);
+        for (int n = 0; n < NT; ++n) {
+          ws[n] = wnext[n];
+          wnext[n] = wsc[n][min(kt + 1, nkt - 1)];
+        }
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              acc[n][m][r] =
-                  finite[m] ? fmaf(s[r], part[n][m][r],
-                                   fmaf(b[r], xsum[m][r], acc[n][m][r]))
-                            : acc[n][m][r] + one[r];
+        for (int j = 0; j < 4; ++j) {  // lane lhi: columns 32 j + 8 lhi .. + 7
+          long xf[MT], wf[NT];
+          const int off =
+              (((j * 2 + (lhi >> 1)) ^ xswz(l16)) << 4) + (lhi & 1) * 8;
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+            wf[n] = *reinterpret_cast<const long *>(wb + n * 16 * WROW + off);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            xf[m] = *reinterpret_cast<const long *>(xb + m * 16 * XROW + off);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+              part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                  wf[n], xf[m], part[n][m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const float xs = sb[(wm * MT + m) * 16 + l16];
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const float f = xs * ws[n];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[n][m][r] += f * part[n][m][r];
           }
         }
       }
-    } else {
-      qg_f4 part[NT][MT];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      cur = cur + 1 == ST ? 0 : cur + 1;
+      nxt = nxt + 1 == ST ? 0 : nxt + 1;
+    }
+  };
+  walk(std::false_type{});
+
+  if constexpr (Q == INT4) {
+    // (16 + q) x or its sum past 32 bits leaves an infinity or a NaN, and
+    // neither goes away again
+    bool finite = true;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          finite &= fabsf(acc[n][m][r]) < INFINITY;  // (false for NaN)
+    // (the flags lie in the ring: with a second array in LDS the compiler
+    // waits for the ring's loads before each of its reads)
+    int *again = reinterpret_cast<int *>(smem);
+    __syncthreads();  // the ring has been read
+    const bool mine = __any(!finite);
+    if (lane == 0) again[wave] = mine;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) any |= again[w];
+    __syncthreads();
+    if (__builtin_expect(any, 0)) {
+      qg_f4 first[NT][MT];
 #pragma unroll
       for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) part[n][m] = qg_f4{0, 0, 0, 0};
-      float ws[NT];
+        for (int m = 0; m < MT; ++m) first[n][m] = acc[n][m];
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        ws[n] = wnext[n];
-        wnext[n] = wsc[n][min(kt + 1, nkt - 1)];
-      }
+      for (int j = 0; j < XL; ++j) xsrc[j] -= (long)nkt * XROW;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {  // lane lhi: columns 32 j + 8 lhi .. + 7
-        long xf[MT], wf[NT];
-        const int off =
-            (((j * 2 + (lhi >> 1)) ^ xswz(l16)) << 4) + (lhi & 1) * 8;
+      for (int j = 0; j < WL; ++j) wsrc[j] -= (long)nkt * WROW;
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-          wf[n] = *reinterpret_cast<const long *>(wb + n * 16 * WROW + off);
+      for (int j = 0; j < SL; ++j) ssrc[j] -= nkt * sstep;
+      walk(std::true_type{});
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-          xf[m] = *reinterpret_cast<const long *>(xb + m * 16 * XROW + off);
+      for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-          for (int n = 0; n < NT; ++n)
-            part[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-                wf[n], xf[m], part[n][m], 0, 0, 0);
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const float xs = sb[(wm * MT + m) * 16 + l16];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          const float f = xs * ws[n];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[n][m][r] += f * part[n][m][r];
-        }
-      }
+          for (int r = 0; r < 4; ++r)
+            if (fabsf(first[n][m][r]) < INFINITY)
+              acc[n][m][r] = first[n][m][r];
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    cur = cur + 1 == ST ? 0 : cur + 1;
-    nxt = nxt + 1 == ST ? 0 : nxt + 1;
   }
 
   store_tile<Q, NT, MT, BN, FORM>(C, acc, bias, M, N, NC, mb * BM + wm * MT * 16,
@@ -449,18 +485,18 @@ struct Plan {
 
 // The tile by rows and width (us, rows x N x K):
 //  * int4: up to 16 rows 64 columns, 128 where the weight is wide or deep
-//    (1 x 7168 x 5120 8.6, 128 columns 9.9; 1 x 5120 x 27648 17.8 at 128,
-//    21.2 at 64); above that 256 for wide and deep ones (29 x 55296 x 5120
-//    47.8, 128 columns 48.8; 29 x 5120 x 27648 27.6, 28.6; 64 x 55296 x 5120
-//    72.9, 84.8), else 64 (29 x 7168 x 5120 13.2, 128 columns 15) or, for
-//    more than 32 rows, 128 (64 x 5120 x 5120 16.0, 64 columns 19).
+//    (1 x 7168 x 5120 7.7, 128 columns 8.9; 1 x 5120 x 27648 18.9 at 128,
+//    22.1 at 64); above that 256 for wide and deep ones (29 x 55296 x 5120
+//    44.7, 128 columns 46.3; 29 x 5120 x 27648 24.5, 26.1; 64 x 55296 x 5120
+//    68.3, 79.2), else 64 (29 x 7168 x 5120 10.0, 128 columns 12.6) or, for
+//    more than 32 rows, 128 (64 x 5120 x 5120 12.1, 64 columns 16.6).
 //  * fp8: up to 16 rows the same (1 x 7168 x 5120 9.2, 128 columns 10.1; 1 x
 //    28672 x 4096 22.1); above that 64 (29 x 7168 x 5120 12.4, 128 columns
 //    14), 256 from 36000 columns (64 x 55296 x 5120 51.2, 128 columns 57.4),
 //    128 between for more than 32 rows (64 x 28672 x 4096 28.6, 29.1).
 // K is split into about as many workgroups as the chip holds at once: 256 of
-// the 512-thread tiles, 448 of the others (1 x 7168 x 5120 4 parts 8.6, 3
-// 9.4), each part at least four stages long.
+// the 512-thread tiles, 448 of the others (1 x 7168 x 5120 4 parts 7.4, 3
+// 8.3), each part at least four stages long.
 Plan plan_for(bool int4, int M, int N, int K, bool gated, int splits) {
   Plan p;
   const bool wide = N >= 16384, deep = K >= 2 * N;

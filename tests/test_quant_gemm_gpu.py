@@ -119,6 +119,38 @@ def test_int4_rows_that_are_not_finite():
     assert torch.equal(out[6][w6.abs() > 1e-6] > 0, w6[w6.abs() > 1e-6] > 0)
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 272, 512), (20, 272, 512),
+                                   (29, 16640, 256), (40, 1040, 768)])
+def test_int4_large_values_that_cancel(M, N, K):
+    """The sum of a group's activations may be small where the terms of the
+    offset form are past 32 bits."""
+    from gllm_amd import ops
+    x, op, _, _ = make("int4", M, N, K)
+    x[2] = 0
+    x[2, 10], x[2, 11] = 2e37, -2e37
+    x[3, 128:256:2], x[3, 129:256:2] = 3e36, -3e36
+    q = torch.stack([op[1].cpu() & 15, op[1].cpu() >> 4], -1).view(N, K)
+    s, b = (op[2][:, i].cpu().t().repeat_interleave(128, 1).double()
+            for i in (0, 1))
+    w = q.double() * s + b
+    ref, size = (a @ v.t() for a, v in (
+        (x.cpu().double(), w), (x.cpu().double().abs(), w.abs())))
+    rest = [i for i in range(M) if i not in (2, 3)]
+    for out in (ops.quant_rows(x, op), ops.quant_parts(x, op).sum(0)):
+        out = out.cpu().double()
+        close(out[rest], ref[rest], size[rest])
+        # (these rows may take weights rounded to bf16)
+        assert ((out - ref).abs() <= 2 ** -7 * size)[2:4].all()
+    # gate and up of a size that silu and their product leave finite
+    small = (op[0], op[1], op[2] * 1e-30)
+    g, u = (ref * 1e-30).split(N // 2, 1)
+    want = torch.nn.functional.silu(g) * u
+    sg, su = (size * 1e-30).split(N // 2, 1)
+    out = ops.quant_silu(x, small).cpu().double()
+    err = 2 ** -6 * (sg * u.abs() + g.abs() * su + want.abs()) + 1e-30
+    assert ((out - want).abs() <= err)[2:4].all()
+
+
 def test_refusals():
     from gllm_amd import ops
     x, op, _, _ = make("int4", 4, 64, 256)
