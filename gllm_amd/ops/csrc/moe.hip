@@ -371,6 +371,31 @@ namespace {
 
 constexpr int TK_MAXJ = 8;  // logits per lane: E <= 64 * TK_MAXJ
 
+// Order of floats as unsigned numbers, for picks on which all lanes of a
+// wave agree whatever the values are (with a NaN, comparisons of the floats
+// themselves leave lanes with different picks): 0 is no candidate, a NaN
+// stands behind every number, -0 equals 0.
+DEV_INLINE unsigned pick_key(float v) {
+  if (v != v) return 1u;
+  const unsigned u = __float_as_uint(v + 0.f);
+  return u & 0x80000000u ? ~u : u | 0x80000000u;
+}
+
+DEV_INLINE float key_value(unsigned k) {
+  return __uint_as_float(k == 1u ? 0x7fc00000u
+                         : k & 0x80000000u ? k ^ 0x80000000u : ~k);
+}
+
+// the wave's largest key, the lower index of equals
+DEV_INLINE void wave_pick(unsigned &key, int &idx) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned ok = __shfl_xor(key, off, 64);
+    const int oi = __shfl_xor(idx, off, 64);
+    if (ok > key || (ok == key && oi < idx)) { key = ok; idx = oi; }
+  }
+}
+
 __global__ __launch_bounds__(256) void topk_softmax_rows_kernel(
     float *__restrict__ weights, int *__restrict__ ids,
     const float *__restrict__ logits, long rows, int E, int k) {
@@ -378,39 +403,27 @@ __global__ __launch_bounds__(256) void topk_softmax_rows_kernel(
   const int lane = threadIdx.x & 63;
   if (r >= rows) return;
   const float *row = logits + r * E;
-  float v[TK_MAXJ];
+  unsigned key[TK_MAXJ];
 #pragma unroll
   for (int j = 0; j < TK_MAXJ; ++j) {
     const int e = lane + 64 * j;
-    v[j] = e < E ? row[e] : -INFINITY;
+    key[j] = e < E ? pick_key(row[e]) : 0u;
   }
   unsigned taken = 0;
   float my_val = -INFINITY;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    float best = -INFINITY;
-    int bidx = 0x7fffffff;
+    unsigned best = 0;
+    int bidx = 0;
 #pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j) {
-      const int e = lane + 64 * j;
-      if (e < E && !(taken >> j & 1u) && (bidx == 0x7fffffff || v[j] > best)) {
-        best = v[j];
-        bidx = e;
+    for (int j = 0; j < TK_MAXJ; ++j)
+      if (!(taken >> j & 1u) && key[j] > best) {
+        best = key[j];
+        bidx = lane + 64 * j;
       }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const int oi = __shfl_xor(bidx, off, 64);
-      // an exhausted lane (no index) loses; a NaN never beats a number
-      const bool take = oi != 0x7fffffff &&
-                        (bidx == 0x7fffffff || ov > best ||
-                         (ov == best && oi < bidx) ||
-                         (best != best && ov == ov));
-      if (take) { best = ov; bidx = oi; }
-    }
+    wave_pick(best, bidx);
     if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
-    if (lane == it) { my_val = best; my_idx = bidx; }
+    if (lane == it) { my_val = key_value(best); my_idx = bidx; }
   }
   const float top = __shfl(my_val, 0, 64);  // the first pick is the largest
   const float p = lane < k ? expf(my_val - top) : 0.f;
@@ -443,39 +456,30 @@ __global__ __launch_bounds__(256) void softmax_topk_rows_kernel(
   }
   mx = wave_reduce_max(mx);
   float sum = 0.f;
+  unsigned key[TK_MAXJ];
 #pragma unroll
   for (int j = 0; j < TK_MAXJ; ++j) {
-    const int e = lane + 64 * j;
-    v[j] = e < E ? expf(v[j] - mx) : -INFINITY;
-    if (e < E) sum += v[j];
+    const bool live = lane + 64 * j < E;
+    const float p = expf(v[j] - mx);
+    key[j] = live ? pick_key(p) : 0u;
+    if (live) sum += p;
   }
   sum = wave_reduce_sum(sum);
   unsigned taken = 0;
   float my_val = 0.f;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    float best = -INFINITY;
-    int bidx = 0x7fffffff;
+    unsigned best = 0;
+    int bidx = 0;
 #pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j) {
-      const int e = lane + 64 * j;
-      if (e < E && !(taken >> j & 1u) && (bidx == 0x7fffffff || v[j] > best)) {
-        best = v[j];
-        bidx = e;
+    for (int j = 0; j < TK_MAXJ; ++j)
+      if (!(taken >> j & 1u) && key[j] > best) {
+        best = key[j];
+        bidx = lane + 64 * j;
       }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const int oi = __shfl_xor(bidx, off, 64);
-      const bool take = oi != 0x7fffffff &&
-                        (bidx == 0x7fffffff || ov > best ||
-                         (ov == best && oi < bidx) ||
-                         (best != best && ov == ov));
-      if (take) { best = ov; bidx = oi; }
-    }
+    wave_pick(best, bidx);
     if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
-    if (lane == it) { my_val = best / sum; my_idx = bidx; }
+    if (lane == it) { my_val = key_value(best) / sum; my_idx = bidx; }
   }
   if (renorm) my_val /= wave_reduce_sum(lane < k ? my_val : 0.f);
   if (lane < k) {
@@ -504,16 +508,15 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
   float *crow = sg_lds + (size_t)wave * (E + n_group);
   float *gsc = crow + E;
   const float *row = logits + r * E;
-  float s[TK_MAXJ], c[TK_MAXJ];
+  float c[TK_MAXJ];
 #pragma unroll
   for (int j = 0; j < TK_MAXJ; ++j) {
     const int e = lane + 64 * j;
     if (e < E) {
-      s[j] = 1.0f / (1.0f + expf(-row[e]));
-      c[j] = s[j] + (correction ? correction[e] : 0.f);
+      c[j] = 1.0f / (1.0f + expf(-row[e])) +
+             (correction ? correction[e] : 0.f);
       crow[e] = c[j];
     } else {
-      s[j] = 0.f;
       c[j] = -INFINITY;
     }
   }
@@ -547,36 +550,27 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
       }
     }
   }
+  unsigned key[TK_MAXJ];
+#pragma unroll
+  for (int j = 0; j < TK_MAXJ; ++j)
+    key[j] = lane + 64 * j < E ? pick_key(c[j]) : 0u;
   unsigned taken = 0;
-  float my_w = 0.f;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    float best = -INFINITY, bs = 0.f;
-    int bidx = 0x7fffffff;
+    unsigned best = 0;
+    int bidx = 0;
 #pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j) {
-      const int e = lane + 64 * j;
-      if (e < E && !(taken >> j & 1u) && (bidx == 0x7fffffff || c[j] > best)) {
-        best = c[j];
-        bs = s[j];
-        bidx = e;
+    for (int j = 0; j < TK_MAXJ; ++j)
+      if (!(taken >> j & 1u) && key[j] > best) {
+        best = key[j];
+        bidx = lane + 64 * j;
       }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const float os = __shfl_xor(bs, off, 64);
-      const int oi = __shfl_xor(bidx, off, 64);
-      const bool take = oi != 0x7fffffff &&
-                        (bidx == 0x7fffffff || ov > best ||
-                         (ov == best && oi < bidx) ||
-                         (best != best && ov == ov));
-      if (take) { best = ov; bs = os; bidx = oi; }
-    }
+    wave_pick(best, bidx);
     if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
-    if (lane == it) { my_w = bs; my_idx = bidx; }
+    if (lane == it) my_idx = bidx;
   }
-  const float sum = wave_reduce_sum(lane < k ? my_w : 0.f);
+  const float my_w = lane < k ? 1.0f / (1.0f + expf(-row[my_idx])) : 0.f;
+  const float sum = wave_reduce_sum(my_w);
   if (lane < k) {
     weights[r * k + lane] = my_w / (sum + 1e-20f) * scale;
     ids[r * k + lane] = my_idx;

@@ -103,3 +103,28 @@ def test_softmax_topk(rows, E, k, dtype, renorm):
     assert torch.equal(ids, rids) and w.dtype == torch.float32
     # fp32 exponentials and sums of at most 512 terms
     assert torch.allclose(w, rw.float(), rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("E,k", [(8, 2), (64, 6), (100, 64)])
+def test_softmax_topk_rows_that_are_not_finite(E, k):
+    """Whatever the logits, the ids are k different experts; rows beside
+    them are as ever."""
+    from gllm_amd import ops
+    from gllm_amd.ops import torch_ref
+    torch.manual_seed(E)
+    x = torch.stack([torch.randperm(E) for _ in range(9)]).float()
+    ref, rids = torch_ref.topk_softmax(x.double(), k)
+    x[0] = float("nan")
+    x[2, 1], x[2, E - 1] = float("nan"), float("nan")
+    x[4, 0], x[4, E // 2] = float("inf"), float("inf")
+    x[6] = float("-inf")
+    w, ids = ops.topk_softmax(x.cuda(), k)
+    for out in (ids, ops.topk_then_softmax(x.cuda(), k)[1],
+                ops.sigmoid_group_topk(x.cuda(), None, k)[1]):
+        for row in out.tolist():
+            assert len(set(row)) == k and 0 <= min(row) and max(row) < E
+    good = [1, 3, 5, 7, 8]
+    assert torch.equal(ids.cpu()[good], rids[good])
+    assert torch.allclose(w.cpu()[good], ref[good].float(), rtol=1e-5,
+                          atol=1e-9)
+    assert w[[0, 2, 4, 6]].isnan().all()
