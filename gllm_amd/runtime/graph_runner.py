@@ -17,6 +17,8 @@ per-row numbers travel in one copy (they were six, 4 us each on the
 device), the block table in a second.
 """
 
+import contextlib
+import gc
 from typing import Dict, List, Optional
 
 import numpy as np
@@ -27,6 +29,22 @@ from gllm_amd.runtime.forward_context import ForwardContext
 
 STAGES = 4  # steps that may be staged ahead of the device
 DECODE_BUCKETS = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512]
+
+
+@contextlib.contextmanager
+def _collector_held():
+    """A graph that is destroyed while another one is captured ends the
+    process, and the graphs of an engine that is no longer used go when the
+    cyclic collector runs (its parts refer to each other): they go now, and
+    the collector waits."""
+    enabled = gc.isenabled()
+    gc.disable()
+    try:
+        gc.collect()
+        yield
+    finally:
+        if enabled:
+            gc.enable()
 
 
 class GraphRunner:
@@ -121,6 +139,15 @@ class GraphRunner:
         pool = torch.cuda.graphs.graph_pool_handle()
         stream = torch.cuda.Stream()
         torch.cuda.synchronize()
+        with _collector_held():
+            self._capture_buckets(pool, stream)
+        torch.cuda.synchronize()
+        self.captured = True
+        logger.info("hipGraph capture done: %d decode buckets (max bs %d)",
+                    len(self.graphs), self.max_bs)
+
+    def _capture_buckets(self, pool, stream):
+        runner = self.runner
         # capture largest first so the shared pool is sized once
         for bs in reversed(self.buckets):
             fctx = self._fctx_for(bs)
@@ -138,10 +165,6 @@ class GraphRunner:
                 hidden, _ = runner.model(ids, pos, fctx)
             self.graphs[bs] = g
             self.hidden_out[bs] = hidden
-        torch.cuda.synchronize()
-        self.captured = True
-        logger.info("hipGraph capture done: %d decode buckets (max bs %d)",
-                    len(self.graphs), self.max_bs)
 
     # ------------------------------------------------------------------
     def can_replay(self, batch) -> bool:
