@@ -35,12 +35,10 @@ DECODE_BUCKETS = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512]
 def _collector_held():
     """A graph that is destroyed while another one is captured ends the
     process, and the graphs of an engine that is no longer used go when the
-    cyclic collector runs (its parts refer to each other): they go now, and
-    the collector waits."""
+    cyclic collector runs (its parts refer to each other): it waits."""
     enabled = gc.isenabled()
     gc.disable()
     try:
-        gc.collect()
         yield
     finally:
         if enabled:
