@@ -65,6 +65,73 @@ def test_steps_staged_ahead_match_eager(tmp_path):
         assert err < 0.02, err
 
 
+@pytest.mark.parametrize("rows,pages", [(1, 2048), (3, 5), (500, 2047),
+                                        (512, 2048)])
+def test_staging_waits_for_its_own_copies_only(rows, pages):
+    """With the device far behind, STAGES steps are staged at once and the
+    next one only when the first one's copies are done; every step sees its
+    own numbers."""
+    from types import SimpleNamespace
+
+    from gllm_amd.runtime.graph_runner import STAGES, GraphRunner
+    runner = GraphRunner(SimpleNamespace(
+        config=SimpleNamespace(device="cuda:0", max_graph_bs=512,
+                               model_max_length=32768, page_size=16),
+        num_kv_pages_total=5000, ssm_pool=None))
+    steps = STAGES + 2
+    torch.manual_seed(rows)
+
+    def items(step):
+        out = []
+        for i in range(rows):
+            n = pages if i == rows // 2 else 1 + (i + step) % 3
+            table = torch.randint(0, 4999, (n,)).tolist()
+            start = n * 16 - 1 - (i + step) % 16
+            out.append(SimpleNamespace(start=start, seq=SimpleNamespace(
+                token_ids={start: 7 * i + step}, page_table=table,
+                mrope_positions=None)))
+        return out
+    work = [items(s) for s in range(steps)]
+    seen = torch.zeros(steps, *runner.block_table.shape, dtype=torch.int32,
+                       device="cuda")
+    nums = torch.zeros(steps, runner.flat.numel(), dtype=torch.long,
+                       device="cuda")
+
+    def stage(s):
+        bs = runner._stage(work[s])
+        seen[s].copy_(runner.block_table)
+        nums[s].copy_(runner.flat)
+        return bs
+    for s in range(steps):              # (what is set up once)
+        bs = stage(s)
+    torch.cuda.synchronize()
+    seen.zero_()
+    a = torch.ones(8192, 8192, device="cuda").bfloat16()
+    behind = torch.cuda.Event()
+    for _ in range(300):                # about 0.2 s
+        torch.mm(a, a)
+    behind.record()
+    for s in range(steps):
+        stage(s)
+        assert behind.query() == (s >= STAGES), s
+    torch.cuda.synchronize()
+    B = runner.max_bs
+    for s in range(steps):
+        ids, pos, slots = nums[s, :3 * B].view(3, B).cpu()
+        lens = nums[s, 4 * B:].view(torch.int32)[:B].cpu()
+        for i, it in enumerate(work[s]):
+            t = it.seq.page_table
+            assert int(ids[i]) == 7 * i + s and int(pos[i]) == it.start
+            assert int(lens[i]) == it.start + 1
+            assert int(slots[i]) == t[it.start // 16] * 16 + it.start % 16
+        got = seen[s].cpu()
+        for i, it in enumerate(work[s]):
+            t = it.seq.page_table
+            assert got[i, :len(t)].tolist() == t
+        for i in range(rows, bs):       # padding: the scratch page
+            assert int(got[i, 0]) == 4999 and int(lens[i]) == 1
+
+
 @pytest.mark.parametrize("n", [1, 255, 257])
 def test_resolve_tokens(n):
     from gllm_amd import ops
