@@ -362,7 +362,9 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                    const float *bias = nullptr, int bias_len = 0,
                    float temp_coef = 0.f, int temp_every = 0,
                    const int *qsl = nullptr) {
-  const int B = seq_lens.size(0), Hkv = k_cache.size(2), Hq = Hkv * G;
+  // (lengths past a step's own rows are not looked at)
+  const int B = qsl ? seq_lens.size(0) : q.size(0);
+  const int Hkv = k_cache.size(2), Hq = Hkv * G;
   const int D = k_cache.size(3), Dv = v_cache.size(3);
   // the longest sequence the pool can hold bounds the useful splits; the
   // count depends on the batch size only (a captured launch serves every
@@ -452,9 +454,9 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                 query_start_loc->numel() == seq_lens.numel() + 1);
     qsl = query_start_loc->data_ptr<int>();
   } else {
-    TORCH_CHECK(seq_lens.numel() == q.size(0), "one query row per sequence");
+    TORCH_CHECK(seq_lens.numel() >= q.size(0), "a length per query row");
   }
-  TORCH_CHECK(block_table.size(0) >= seq_lens.numel());
+  TORCH_CHECK(block_table.size(0) >= (qsl ? seq_lens.numel() : q.size(0)));
   launch_decode(out, q, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
                 (float)scale, (int)sliding_window, 0, false, nullptr, 0,
                 nullptr, 0.f, nullptr, 0, 0.f, 0, qsl);

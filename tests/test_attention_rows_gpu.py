@@ -91,3 +91,20 @@ def test_unsplit_decode(B, Hkv):
         # the split form rounds its weights against another maximum
         err = (whole.double() - parts.double()).norm() / parts.double().norm()
         assert err < 3 * 2 ** -9, err
+
+
+def test_decode_reads_as_many_lengths_as_rows():
+    """A step's tables may be longer than the step (buffers of a larger
+    batch): the first rows count."""
+    from gllm_amd import ops
+    q, kc, vc, table, lens, qsl = _case([1] * 5, [3, 200, 64, 17, 90], 8, 2,
+                                        128)
+    ref = ops.paged_attention(q, kc, vc, table, lens, qsl, 0.1)
+    for n in (1, 3):
+        for t in (table, table[:n]):
+            out = ops.paged_attention(q[:n], kc, vc, t, lens, qsl, 0.1)
+            # (the splits follow the rows)
+            err = (out - ref[:n]).float().norm() / ref[:n].float().norm()
+            assert err < 3 * 2 ** -9, err
+    with pytest.raises(RuntimeError):           # lengths for fewer rows
+        ops.paged_attention(q, kc, vc, table, lens[:4], qsl, 0.1)
