@@ -794,7 +794,7 @@ def mla_paged_attention(q, k_cache, v_cache, block_table, seq_lens,
             and q.dtype == torch.bfloat16):
         qsl_h = query_start_loc_cpu or query_start_loc.tolist()
         max_q = max((qsl_h[i + 1] - qsl_h[i]
-                     for i in range(len(qsl_h) - 1)), default=1)
+                     for i in range(seq_lens.shape[0])), default=1)
         T, H = q.shape[0], q.shape[1]
         out = torch.empty(T, H, 512, dtype=q.dtype, device=q.device)
         qsl_i = query_start_loc.int() \

@@ -398,7 +398,7 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
   const int B = seq_lens.size(0);
   TORCH_CHECK(block_table.stride(1) == 1 && block_table.size(0) >= B &&
               query_start_loc.scalar_type() == at::kInt &&
-              query_start_loc.numel() == B + 1);
+              query_start_loc.numel() >= B + 1);
   TORCH_CHECK(k_cache.is_contiguous() &&
               reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0);

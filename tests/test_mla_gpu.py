@@ -59,6 +59,19 @@ def test_mla_attention_tiles(q_lens, ctx, H, page):
     assert err < 3 * 2 ** -9, err
 
 
+def test_mla_attention_reads_as_many_offsets_as_lengths():
+    """Offsets past the sequences' own (buffers of a larger batch) are not
+    looked at."""
+    from gllm_amd import ops
+    q, cache, table, lens, qsl = (
+        t.cuda() for t in _case([1, 1, 1, 9], [5, 900, 64, 0], 16))
+    want = ops.mla_paged_attention(q[:3], cache, cache[..., :512], table[:3],
+                                   lens[:3], qsl[:4], 0.1)
+    out = ops.mla_paged_attention(q[:3], cache, cache[..., :512], table[:3],
+                                  lens[:3], qsl, 0.1)
+    assert torch.equal(out, want)
+
+
 def test_mla_decode_captured_serves_longer_batches():
     """The split count does not depend on the lengths seen at capture."""
     from gllm_amd import ops
