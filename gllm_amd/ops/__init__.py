@@ -272,7 +272,10 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     tw = topk_weights.float().contiguous()
     pair_out = torch.empty(n_pairs, K, dtype=x.dtype, device=dev)
     rpe = n_pairs / max(1, E_local)
-    if K % 64 == 0 and inter % 64 == 0:
+    # (the wide tiles come to LDS in units of 16 B)
+    x = x.clone() if x.data_ptr() % 16 else x
+    if (K % 64 == 0 and inter % 64 == 0
+            and w13.data_ptr() % 16 == 0 and w2.data_ptr() % 16 == 0):
         # row block by the rows per expert: while an expert's weights are
         # the cost, one block holds the rows of all but the most popular
         # experts (csrc/moe_tiled.hip has times on both sides of each line)
@@ -281,7 +284,7 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
                                           block_m)
         act = torch.empty(rows, inter, dtype=x.dtype, device=dev)
-        code = {"silu_glu": 1, "swiglu_clamp": 2, "relu2": 3}[activation]
+        code = {"swiglu_clamp": 2, "relu2": 3}.get(activation, 1)
         limit, alpha = act_args if activation == "swiglu_clamp" \
             else (0.0, 0.0)
         k.moe_gemm_tiled(act, x, w13, *tables, None, n_pairs, topk, block_m,

@@ -128,3 +128,27 @@ def test_softmax_topk_rows_that_are_not_finite(E, k):
     assert torch.allclose(w.cpu()[good], ref[good].float(), rtol=1e-5,
                           atol=1e-9)
     assert w[[0, 2, 4, 6]].isnan().all()
+
+
+@pytest.mark.parametrize("which", ["x", "w13", "w2", "activation"])
+def test_fused_moe_takes_what_the_general_form_takes(which):
+    """Operands that do not start on 16 bytes, and a gated activation by
+    another name."""
+    from gllm_amd import ops
+    torch.manual_seed(3)
+    T, E, H, I = 40, 8, 128, 192
+    arg = {"x": torch.randn(T, H, device="cuda").bfloat16(),
+           "w13": (torch.randn(E, 2 * I, H, device="cuda") * 0.1).bfloat16(),
+           "w2": (torch.randn(E, H, I, device="cuda") * 0.1).bfloat16()}
+    weights, ids = ops.topk_softmax(torch.randn(T, E, device="cuda"), 2)
+    ref = _ref(arg["x"], arg["w13"], arg["w2"], weights, ids, 0, "", ())
+    kind = "silu_glu"
+    if which == "activation":
+        kind = "silu"
+    else:
+        t = arg[which]
+        buf = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        arg[which] = buf[4:4 + t.numel()].view(t.shape).copy_(t)
+    out = ops.fused_moe(arg["x"], arg["w13"], arg["w2"], weights, ids,
+                        activation=kind)
+    assert (out.double() - ref).norm() / ref.norm() < 4 * 2 ** -9
