@@ -839,13 +839,23 @@ def plain_bias(bias, N: int) -> bool:
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = x @ w.T (+ bias) via the gfx950 weight-streaming kernel (at
-    most 256 rows)."""
-    if not _rows_ok(x, w):
-        import torch.nn.functional as F
-        return F.linear(x, w, bias)
-    if not plain_bias(bias, w.shape[0]):
-        return _gpu_kernels().stream_gemm(x, w, None) + bias
-    return _gpu_kernels().stream_gemm(x, w, bias)
+    most 256 rows; an N or an address off its units goes to the library). A
+    bias of another type is added to the bf16 product."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and x.is_contiguous()
+            and w.is_contiguous() and w.shape[1] % 64 == 0
+            and x.shape[0] <= 256):
+        raise RuntimeError("skinny_gemm: contiguous bf16 on the GPU, K a "
+                           "multiple of 64, at most 256 rows")
+    if _rows_ok(x, w):
+        run = _gpu_kernels().stream_gemm
+    else:
+        run = torch.nn.functional.linear
+    if plain_bias(bias, w.shape[0]):
+        return run(x, w, bias)
+    out = run(x, w, None)
+    out += bias
+    return out
 
 
 def _use_skinny(M: int, N: int, K: int) -> bool:
@@ -875,7 +885,7 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     """GEMM dispatch: the weight-streaming kernel where measured faster,
     hipBLASLt otherwise."""
     import torch.nn.functional as F
-    if _streams(x, w) and plain_bias(bias, w.shape[0]):
+    if _streams(x, w):
         return skinny_gemm(x, w, bias)
     return F.linear(x, w, bias)
 

@@ -101,3 +101,23 @@ def test_qkv_rope_cache(M, Hq, Hkv, D, rot, K, parts):
     free[slots] = False
     assert not kc.view(-1, Hkv, D)[free].any()
     assert not vc.view(-1, Hkv, D)[free].any()
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 4096), (100, 2056, 128)])
+def test_bias_of_another_type(M, N, K):
+    """An fp32 bias is added to the bf16 product; the result stays bf16."""
+    from gllm_amd import ops
+    x, w, ref = _operands(M, N, K)
+    bias = torch.randn(N, device="cuda")
+    for f in (ops.skinny_gemm, ops.linear):
+        out = f(x, w, bias)
+        assert out.dtype == torch.bfloat16
+        # two roundings
+        _close(out, ref + bias.double(), 2 ** -7)
+    # an N that the kernel does not take
+    _close(ops.skinny_gemm(x, w[:N - 3], bias[:N - 3]),
+           ref[:, :N - 3] + bias[:N - 3].double(), 2 ** -7)
+    for bad in ((x.float(), w.float()), (x.t(), w[:, :M].contiguous()),
+                (x.repeat(300, 1), w)):
+        with pytest.raises(RuntimeError):
+            ops.skinny_gemm(*bad)
