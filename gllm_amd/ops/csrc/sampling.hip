@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
+#include "common.h"
 
 namespace {
 
@@ -331,5 +332,6 @@ torch::Tensor greedy_argmax(torch::Tensor logits) {
             out.data_ptr<long>(), (const unsigned short *)logits.data_ptr(),
             V, wide);
   }
+  HIP_CHECK_KERNEL();
   return out;
 }
