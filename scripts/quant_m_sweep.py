@@ -1,4 +1,5 @@
-"""fp8 skinny at M in {96, 128, 192, 256} per ring (FP8_RING env)."""
+"""The fp8 few-row product above 64 rows, where the layers use the library's
+(both sides of that line: scripts/gemm_sweep.py)."""
 import os
 import sys
 import time

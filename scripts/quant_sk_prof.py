@@ -4,6 +4,7 @@ Times each Qwen2.5-32B decode shape through the public ops wrappers
 (quant + GEMM + reduce end to end) and prints actual-weight-byte TB/s.
 
     python scripts/quant_sk_prof.py fp8|int4 [shape] [iters]
+    python scripts/quant_sk_prof.py sweep      # fp8, parts along K
 
 Under rocprofv3 PMC (single shape keeps the counter file small):
     rocprofv3 --pmc SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_WAIT_INST_ANY \
@@ -73,7 +74,7 @@ def main():
 
 
 def splitk_sweep():
-    """Direct fp8_skinny_gemm calls with explicit splitk values."""
+    """The fp8 product alone (its fp32 parts) with explicit parts along K."""
     from gllm_amd.layers.quantization import fp8 as qfp8
     from gllm_amd.ops import _gpu_kernels, per_token_group_quant_fp8
     k = _gpu_kernels()
@@ -85,22 +86,13 @@ def splitk_sweep():
         wq, ws = wq.cuda().view(torch.uint8), ws.cuda().contiguous()
         aq, _, ast = per_token_group_quant_fp8(x, transposed=True)
         aq = aq.view(torch.uint8)
-        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
-        for sk in (1, 2, 4, 8, 16):
-            if (K // sk) % 128:
-                continue
-            wsb = torch.empty(sk * M * N, dtype=torch.float32,
-                              device="cuda")
-            try:
-                k.fp8_skinny_gemm(out, aq, ast, wq, ws, None, wsb, sk)
-            except RuntimeError as e:
-                print(f"{name} sk={sk}: {e}")
-                continue
+        for sk in (1, 2, 3, 4, 8, 16):
+            for _ in range(3):
+                k.quant_gemm(aq, ast, wq, ws, None, 2, sk)
             torch.cuda.synchronize()
-            import time
             t0 = time.time()
             for _ in range(30):
-                k.fp8_skinny_gemm(out, aq, ast, wq, ws, None, wsb, sk)
+                k.quant_gemm(aq, ast, wq, ws, None, 2, sk)
             torch.cuda.synchronize()
             dt = (time.time() - t0) / 30
             print(f"{name:8s} splitk={sk:2d} {dt*1e6:7.1f} us "
