@@ -128,7 +128,7 @@ class LinearBase(nn.Module):
         return self._bias_f32
 
     def _prefill_quant(self, x, bias):
-        """Quantized prefill (M > 256), three modes via
+        """Quantized rows above 64, three modes via
         GLLM_QUANT_PREFILL:
 
         - "cache" (default): dequantize ONCE into a resident bf16 copy

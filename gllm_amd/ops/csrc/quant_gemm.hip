@@ -492,8 +492,10 @@ struct Plan {
 //    more than 32 rows, 128 (64 x 5120 x 5120 12.1, 64 columns 16.6).
 //  * fp8: up to 16 rows the same (1 x 7168 x 5120 9.2, 128 columns 10.1; 1 x
 //    28672 x 4096 22.1); above that 64 (29 x 7168 x 5120 12.4, 128 columns
-//    14), 256 from 36000 columns (64 x 55296 x 5120 51.2, 128 columns 57.4),
-//    128 between for more than 32 rows (64 x 28672 x 4096 28.6, 29.1).
+//    14), 256 from 36000 columns (64 x 55296 x 5120 51.2, 128 columns 57.4;
+//    gated K 5120, 64 rows, 128 / 256 columns: 32768 34 / 52, 34816 52 / 49,
+//    38912 53 / 50; with 24 rows level there, 39 / 40), 128 between for more
+//    than 32 rows (64 x 28672 x 4096 28.6, 29.1).
 // K is split into about as many workgroups as the chip holds at once: 256 of
 // the 512-thread tiles, 448 of the others (1 x 7168 x 5120 4 parts 7.4, 3
 // 8.3), each part at least four stages long.

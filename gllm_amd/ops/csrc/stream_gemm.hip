@@ -8,9 +8,9 @@
 // by row & 7, so fragment reads fall on all banks; products are W x^T, so a
 // lane ends with four neighbouring columns of one row.
 //
-// A weight with few 64-row tiles is also split along K, into about 512
-// workgroups in all; the fp32 parts [S, M, N] are then summed by whatever
-// comes next, in the order of S:
+// A weight with few tiles is also split along K (plan_for: into about 384
+// workgroups below 160 tiles, into two parts up to 288 if K is long); the fp32
+// parts [S, M, N] are then summed by whatever comes next, in the order of S:
 //   stream_gemm           bias, bf16
 //   stream_add_norm       residual += sum, RMS norm of it (attention and
 //                         feed-forward outputs)
@@ -387,6 +387,12 @@ struct Plan {
 //    256 x 5120 x 27648 110 (128 x 128 118), 256 x 28672 x 4096 68 (128 x 64
 //    90); gated and 36000 columns 256 x 256, 149 (256 x 128 175); else 128 x
 //    64, 256 x 7168 x 5120 40 (128 x 128 42).
+// The lines in between (K 5120, gated, us, narrow / wide tile): 32768 columns
+// are 512 tiles of 64, two per CU, and the last that the chip holds at once:
+// 64 rows 68 / 81, 128 rows 88 / 96, 256 rows 96 / 132; 36864: 93 / 84, 123 /
+// 98, 157 / 134 (24 rows 90 / 80). From 64 rows on the wide tile is the faster
+// one from there already (34816: 92 / 83, 122 / 97, 155 / 133), 24 rows not
+// yet (74 / 80).
 // K is split into about 384 workgroups where there are fewer than 160 tiles
 // (5120 x 27648, 16 rows: 5 splits 50.8, 13 splits 52.9; 7168 x 5120: 4
 // splits 18.2, 7 splits 19.6; 11008 x 2048 at 172 tiles: none 11.2, two
