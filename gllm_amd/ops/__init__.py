@@ -281,6 +281,10 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
         # experts (csrc/moe_tiled.hip has times on both sides of each line)
         block_m = (32 if rpe <= 12 else 64 if rpe <= 40
                    else 128 if rpe <= 128 else 256)
+        if block_m == 256 and max(
+                T * K, (n_pairs + E_local * 255 + 256) * inter, n_pairs * K,
+                rows13 * K, K * inter) >= 1 << 30:
+            block_m = 128  # (256-row blocks take operands below 2 GiB)
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
                                           block_m)
         act = torch.empty(rows, inter, dtype=x.dtype, device=dev)
@@ -880,13 +884,42 @@ def _streams(x: torch.Tensor, w: torch.Tensor) -> bool:
                                           w.shape[1])
 
 
+def _tile_fits(M: int, N: int, K: int, gated: bool) -> bool:
+    """Sizes that csrc/tile_gemm.hip takes (more rows than the streaming
+    kernel's)."""
+    return (M > SKINNY_MAX_M and K % 64 == 0 and N <= 1 << 20
+            and K <= 1 << 21 and M <= 1 << 24
+            and ((M + 127) // 128) * (N // 256 + 2) < 1 << 24
+            and (not gated or N * K < 1 << 30))
+
+
+def _use_tile(M: int, N: int, K: int) -> bool:
+    """Plain products for csrc/tile_gemm.hip: long K, where hipBLASLt keeps
+    whole tiles and leaves CUs idle or falls to small ones, from 0.5 to 1.65
+    PFLOP/s with no order in M (us, library / tile): 4133 x 5120 x 27648
+    1448 / 810, 5000 x 5120 x 27648 1667 / 1013, 600 x 2048 x 10944 54 / 38,
+    4100 x 4096 x 14336 725 / 347 but 4096 x 4096 x 14336 286 / 311. The
+    library goes on where a tile's step of 1.33 us says less than 1.2
+    PFLOP/s (2800 x 4096 x 14336 236 / 291), and with shorter K, where it
+    is mostly 5 % ahead (4133 x 7168 x 5120 202 / 216)."""
+    if K < 3 * N or not _tile_fits(M, N, K, False):
+        return False
+    us = 1.33 * _gpu_kernels().tile_gemm_cost(M, N, K, False)
+    return us * 1.2e9 < 2.0 * M * N * K
+
+
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """GEMM dispatch: the weight-streaming kernel where measured faster,
-    hipBLASLt otherwise."""
+    """GEMM dispatch: the weight-streaming kernel for few rows, the tile
+    kernel for many rows and long K, where measured faster; hipBLASLt
+    otherwise."""
     import torch.nn.functional as F
     if _streams(x, w):
         return skinny_gemm(x, w, bias)
+    if (x.dim() == 2 and _use_tile(x.shape[0], w.shape[0], w.shape[1])
+            and _rows_ok(x, w) and plain_bias(bias, w.shape[0])
+            and (bias is None or bias.data_ptr() % 16 == 0)):
+        return _gpu_kernels().tile_gemm(x, w, bias, False)
     return F.linear(x, w, bias)
 
 
@@ -894,10 +927,17 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ w_gate.T) * (x @ w_up.T), w = gate rows over up rows. Few
     rows: one kernel, the [rows, 2 ff] product is never written (above 64
     rows it is level with the library's product and saves the second
-    kernel: 256 x 55296 x 5120 149 us against 154 + 9)."""
-    if (_rows_ok(x, w) and w.shape[0] % 16 == 0 and w.shape[0] >= 512
-            and _use_skinny(x.shape[0], 512, w.shape[1])):
-        return _gpu_kernels().stream_gemm_gated(x, w)
+    kernel: 256 x 55296 x 5120 149 us against 154 + 9). Many rows: the tile
+    kernel, again one (us, library and second kernel / tile: 512 x 5632 x
+    2048 27 / 26, 512 x 55296 x 5120 288 / 237, 4133 x 55296 x 5120 1960 /
+    1700, 8192 x 28672 x 4096 1388 / 1304; wide weights need 384 rows: 333 x
+    55296 x 5120 217 / 270)."""
+    if (_rows_ok(x, w) and w.shape[0] % 16 == 0 and w.shape[0] >= 512):
+        M, (N, K) = x.shape[0], w.shape
+        if _use_skinny(M, 512, K):
+            return _gpu_kernels().stream_gemm_gated(x, w)
+        if _tile_fits(M, N, K, True) and (M >= 384 or N < 16384):
+            return _gpu_kernels().tile_gemm(x, w, None, True)
     return silu_and_mul(linear(x, w))
 
 

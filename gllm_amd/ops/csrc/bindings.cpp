@@ -23,6 +23,9 @@ torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
+torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w,
+                        c10::optional<torch::Tensor> bias, bool gated);
+double tile_gemm_cost(long M, long N, long K, bool gated);
 torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w);
 torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
                               torch::Tensor residual, torch::Tensor norm_w,
@@ -174,6 +177,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("resolve_tokens", &resolve_tokens,
         "token ids with places in the ring of sampled tokens");
   m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
+  m.def("tile_gemm", &tile_gemm, "x w^T + bias, or its gated form");
+  m.def("tile_gemm_cost", &tile_gemm_cost,
+        "cost of a tile_gemm in steps of one tile");
   m.def("stream_gemm_gated", &stream_gemm_gated,
         "silu(x w_gate^T) * (x w_up^T) for at most 256 rows");
   m.def("stream_parts", &stream_parts, "fp32 parts of x w^T");

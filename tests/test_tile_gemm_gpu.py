@@ -1,0 +1,81 @@
+"""Many-row products on 256-row tiles against fp64, at the edges of their
+tiles, row blocks, splits along K and of the dispatch."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K,bias,gated", [
+    (1, 8, 64, False, False),            # one stage, one row, one unit
+    (257, 264, 128, True, False),        # a row and 8 columns into a tile
+    (128, 512, 320, False, False),       # a whole half block
+    (129, 248, 192, True, False),
+    (385, 1040, 64, False, True),        # half block last, ragged columns
+    (300, 16, 128, False, True),
+    (2049, 1024, 640, True, False),      # many tiles of one row more
+    (640, 4096, 4160, True, False),      # split along K
+    (700, 4112, 4160, False, True),
+    (4133, 2048, 1088, False, False),    # whole tiles, then split ones
+])
+def test_tile_gemm(M, N, K, bias, gated):
+    from gllm_amd import ops
+    k = ops._gpu_kernels()
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    b = torch.randn(N, device="cuda").bfloat16() if bias else None
+    out = k.tile_gemm(x, w, b, gated)
+    y = x.double() @ w.double().t()
+    if bias:
+        y = y + b.double()
+    if gated:
+        g, u = y.chunk(2, dim=-1)
+        y = torch.nn.functional.silu(g) * u
+    assert out.shape == y.shape and torch.isfinite(out).all()
+    # one rounding to bf16 of fp32 sums; exponentials to a few 2^-23
+    err = ((out.double() - y).abs() / y.abs().clamp_min(
+        y.square().mean().sqrt())).max()
+    assert err < 1.1 * 2 ** -8, err
+    assert torch.equal(out, k.tile_gemm(x, w, b, gated))
+
+
+def test_rows_past_the_last_are_left_alone():
+    """Infinities and NaN in one row stay in it."""
+    from gllm_amd import ops
+    x = torch.randn(390, 192, device="cuda").bfloat16()
+    w = torch.randn(520, 192, device="cuda").bfloat16()
+    clean = ops._gpu_kernels().tile_gemm(x, w, None, False)
+    x[17], x[388] = float("inf"), float("nan")
+    out = ops._gpu_kernels().tile_gemm(x, w, None, False)
+    keep = torch.ones(390, dtype=torch.bool)
+    keep[17] = keep[388] = False
+    assert torch.equal(out[keep], clean[keep])
+    assert out[388].isnan().all() and not out[17].isfinite().any()
+
+
+@pytest.mark.parametrize("M", [256, 257, 384, 500])
+def test_dispatch(M):
+    """The same numbers whichever kernel a row count is sent to."""
+    from gllm_amd import ops
+    torch.manual_seed(M)
+    x = torch.randn(M, 3072, device="cuda").bfloat16()
+    w = (torch.randn(1024, 3072, device="cuda") * 3072 ** -0.5).bfloat16()
+    b = torch.randn(1024, device="cuda").bfloat16()
+    ref = x.double() @ w.double().t()
+    for out, y in ((ops.linear(x, w, b), ref + b.double()),
+                   (ops.linear(x, w), ref)):
+        assert ((out.double() - y).norm() / y.norm()) < 2 ** -8
+    # a bias of another type, off 16 bytes or a strided view: refused or
+    # taken as before
+    off = torch.cat([b[:1], b])[1:]
+    assert torch.allclose(ops.linear(x, w, off).float(),
+                          ops.linear(x, w, b).float(), atol=0.05)
+    half = ops.linear(x[:, ::2], w[:, ::2])
+    y = x[:, ::2].double() @ w[:, ::2].double().t()
+    assert ((half.double() - y).norm() / y.norm()) < 2 ** -8
+    g, u = ref.chunk(2, dim=-1)
+    y = torch.nn.functional.silu(g) * u
+    out = ops.linear_silu(x, w)
+    assert ((out.double() - y).norm() / y.norm()) < 2 ** -7
