@@ -916,9 +916,9 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     import torch.nn.functional as F
     if _streams(x, w):
         return skinny_gemm(x, w, bias)
-    if (x.dim() == 2 and _use_tile(x.shape[0], w.shape[0], w.shape[1])
-            and _rows_ok(x, w) and plain_bias(bias, w.shape[0])
-            and (bias is None or bias.data_ptr() % 16 == 0)):
+    if (_rows_ok(x, w) and plain_bias(bias, w.shape[0])
+            and (bias is None or bias.data_ptr() % 16 == 0)
+            and _use_tile(x.shape[0], w.shape[0], w.shape[1])):
         return _gpu_kernels().tile_gemm(x, w, bias, False)
     return F.linear(x, w, bias)
 
