@@ -2,9 +2,19 @@
 //
 // Memory-bound: the job is to stream each sequence's K/V pages once at
 // near-HBM rate. Structure:
-//   grid = (B, Hkv, num_splits), block = 256 threads (4 waves). A workgroup
+//   grid = B * Hkv * splits, block = 256 threads (4 waves). A workgroup
 //   serves the whole GQA group (up to 16 query heads) of one kv head over
 //   a share of the keys, so K/V bytes are read once for all its heads.
+//   Up to two rounds of workgroups, heads are the fastest index (the eight
+//   dies take workgroups in turn, so with 8 heads each die gets a share of
+//   every sequence), then splits, and sequences come longest first
+//   (sequence_at), so what starts last is short. More rounds even out by
+//   themselves, and finding the sequence costs each workgroup about 1 us:
+//   there sequences are the fastest index, as they come. (us, 512 to 1536
+//   keys unless said, sequences fastest / this: 64 sequences 69 / 58, 128 of
+//   1024 to 3072 keys 203 / 188, 24 of 2700 to 8100 in four splits 123 / 105,
+//   37 in two 40 / 38; 256 sequences 189 / 188 and 10 more in a step; heads
+//   fastest alone 62, 219, 120, 44, 206.)
 //   Its waves work on their own: wave w takes the 32-key tiles w, w + 4,
 //   ... of the share, with a softmax state of its own and no barrier in the
 //   loop; the next tile's K and V are in registers while this one is
@@ -44,6 +54,53 @@ union DecFrag {
   __hip_bfloat16 e[8];
 };
 
+constexpr int ORDERED = 1024;  // workgroups at most: two rounds
+
+// The sequence whose visible keys come `rank`th, the most first, to within a
+// sixteenth of the most (equal ones by number); every wave finds it by
+// itself. B <= ORDERED.
+DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
+                           const int *qsl) {
+  if (B == 1) return rank;
+  const int lane = threadIdx.x & 63;
+  constexpr int PER = ORDERED / 64;
+  int keys[PER], most = 1;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int b = i * 64 + lane;
+    keys[i] = -1;
+    if (i * 64 < B && b < B) {
+      keys[i] = max(seq_lens[b], 0);
+      if (window > 0) keys[i] = min(keys[i], window);
+      if (qsl && qsl[b + 1] - qsl[b] != 1) keys[i] = 0;
+      most = max(most, keys[i]);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    most = max(most, __shfl_xor(most, off, 64));
+  const float unit = 15.999f / most;
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    keys[i] = keys[i] < 0 ? -1 : (int)(keys[i] * unit);
+  for (int k = 15; k >= 0; --k) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (i * 64 >= B) break;
+      const unsigned long long m = __ballot(keys[i] == k);
+      const int n = __popcll(m);
+      if (rank < n) {
+        const int before = __builtin_amdgcn_mbcnt_hi(
+            (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        return i * 64 +
+               __ffsll(__ballot(keys[i] == k && before == rank)) - 1;
+      }
+      rank -= n;
+    }
+  }
+  return 0;  // (not reached: every key is in 0 .. 15)
+}
+
 // Head sizes Dr <= D, Dvr <= DV (multiples of 8; D, DV 64 or 128): columns
 // beyond a head are zero. G query heads per kv head, rows of the products
 // beyond G are zero. Optional bias by distance and query temperature.
@@ -65,14 +122,24 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     // one split: the result itself, bf16 [rows, Hq * Dvr]
     __hip_bfloat16 *__restrict__ out, long out_stride, int sink,
     const float *__restrict__ sinks, const __hip_bfloat16 *__restrict__ gate,
-    long gate_stride) {
+    long gate_stride, int B, int zdim) {
   constexpr int KT = D / 32, NT = DV / 16;
   constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
   constexpr int VROW = DV * 2;             // LDS row bytes
   constexpr int VMASK = (DV / 8 - 1) & 15;
-  const int b = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int split = blockIdx.z;
+  int b, kvh, split;  // (zdim: splits, and the kept-first segment)
+  if (gridDim.x <= ORDERED) {
+    const int rest = blockIdx.x / num_kv_heads;
+    kvh = blockIdx.x - rest * num_kv_heads;
+    split = rest % zdim;
+    b = __builtin_amdgcn_readfirstlane(
+        sequence_at(rest / zdim, B, seq_lens, window, qsl));
+  } else {
+    const int rest = blockIdx.x / B;
+    b = blockIdx.x - rest * B;
+    kvh = rest % num_kv_heads;
+    split = rest / num_kv_heads;
+  }
   const int Hq = num_kv_heads * G;
   const int seq_len = seq_lens[b];
   const int row = qsl ? qsl[b] : b;  // of q and of the result
@@ -93,7 +160,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const int lane = tid & 63;
   const int l16 = lane & 15;
   const int lhi = lane >> 4;
-  const long lse0 = (long)split * gridDim.x * Hq + (long)b * Hq + kvh * G;
+  const long lse0 = (long)split * B * Hq + (long)b * Hq + kvh * G;
   if (t0 >= t1) {
     // empty split: publish -inf lse so the merge ignores it
     if (out) {
@@ -406,7 +473,7 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
   }
   auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(DT, DVT)                                                         \
-  hipLaunchKernelGGL((paged_decode_kernel<DT, DVT>), dim3(B, Hkv, zdim),     \
+  hipLaunchKernelGGL((paged_decode_kernel<DT, DVT>), dim3(B * Hkv * zdim),   \
                      dim3(BLOCK), 0, stream, po, pl,                         \
                      (const __hip_bfloat16 *)q.data_ptr(),                   \
                      (const __hip_bfloat16 *)k_cache.data_ptr(),             \
@@ -416,7 +483,8 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      G, D, Dv, scale, splits, (long)q.stride(0), window,     \
                      keep_first, softcap, bias, bias_len, temp_coef,         \
                      temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
-                     sinks, (const __hip_bfloat16 *)gate, gate_stride)
+                     sinks, (const __hip_bfloat16 *)gate, gate_stride, B,    \
+                     zdim)
   if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
 #undef RUN
