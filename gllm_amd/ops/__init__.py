@@ -931,9 +931,15 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     kernel, again one (us, library and second kernel / tile: 512 x 5632 x
     2048 27 / 26, 512 x 55296 x 5120 288 / 237, 4133 x 55296 x 5120 1960 /
     1700, 8192 x 28672 x 4096 1388 / 1304; wide weights need 384 rows: 333 x
-    55296 x 5120 217 / 270)."""
+    55296 x 5120 217 / 270). One block of rows on very wide weights too
+    (stream / tile: 256 x 55296 x 5120 152 / 137, 192 rows 150 / 129, 128
+    rows 116 / 116; 256 x 28672 x 4096 67 / 80)."""
     if (_rows_ok(x, w) and w.shape[0] % 16 == 0 and w.shape[0] >= 512):
         M, (N, K) = x.shape[0], w.shape
+        # one row block and a round of 192 to 256 column blocks
+        if (128 < M <= 256 and 49152 <= N <= 65536 and 4096 <= K < 16384
+                and _use_skinny(M, 512, K)):
+            return _gpu_kernels().tile_gemm(x, w, None, True)
         if _use_skinny(M, 512, K):
             return _gpu_kernels().stream_gemm_gated(x, w)
         if _tile_fits(M, N, K, True) and (M >= 384 or N < 16384):

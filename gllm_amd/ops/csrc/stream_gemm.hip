@@ -23,11 +23,14 @@
 // rows 63 for 159 and 79, 256 rows 110 for 266 and 160; 7168 x 5120, 1 row
 // 16.4 for 24; 28672 x 4096 gated, 1 row 39 for 61 + 5. Weights come at 4.0
 // to 6.6 TB/s from 35 MB on, below that the launch and the ring's first
-// stages are most of the time (2048 x 2048: 5 + 3 us).
+// stages are most of the time (2048 x 2048: 5 + 3 us). Parts of large weights
+// with more than 64 rows (32 if K is long) come from tile_gemm.hip, where 256
+// columns share their rows (tile_parts_plan has both sides of the line).
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
+#include "tile_gemm.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 st_bf8;
 typedef __attribute__((ext_vector_type(4))) float st_f4;
@@ -482,6 +485,15 @@ torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w) {
   check_operands(x, w);
   const long M = x.size(0), N = w.size(0);
   TORCH_CHECK(M > 0);
+  int bm, splits;
+  tile_parts_plan(M, N, w.size(1), &bm, &splits);
+  if (splits > 0 && x.is_contiguous()) {
+    auto part = torch::empty({(long)splits, M, N},
+                             x.options().dtype(at::kFloat));
+    tile_parts(part.data_ptr<float>(), x.data_ptr(), w.data_ptr(), M, N,
+               w.size(1), bm, splits);
+    return part;
+  }
   const Plan p = plan_for(M, N, w.size(1), false);
   auto part = torch::empty({(long)p.splits, M, N},
                            x.options().dtype(at::kFloat));

@@ -1,5 +1,5 @@
-// Grouped products on 256-row blocks (tile_gemm.hip), called by
-// moe_gemm_tiled.
+// tile_gemm.hip: grouped products on 256-row blocks, called by
+// moe_gemm_tiled; split products of few rows, called by stream_parts.
 #pragma once
 
 void tile_gemm_grouped(void *C, const void *A, const void *W,
@@ -8,3 +8,8 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
                        long max_blocks, long n_pairs, long topk, long Nd,
                        long K, long a_rows, int act, float limit,
                        float alpha);
+
+// x [M, K] w [N, K]^T of at most 256 rows as fp32 parts [splits, M, N]
+void tile_parts_plan(long M, long N, long K, int *bm, int *splits);
+void tile_parts(float *part, const void *x, const void *w, long M, long N,
+                long K, int bm, int splits);

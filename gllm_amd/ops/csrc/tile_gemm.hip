@@ -5,6 +5,7 @@
 //   gated    out = f(x W_gate^T)(x W_up^T), W = gate rows over up rows: the
 //            [M, N] product is never written
 //   scatter  out[pair] = w[pair] * act W^T (grouped)
+//   parts    fp32 [S, M, N] of at most 256 rows, each part over a share of K
 //
 // Bound by the matrix cores' power and clock where it is fed well: 4096 x
 // 4096 x 16384 runs at 1550 TFLOP/s on normal data and 1830 on zeros. What
@@ -61,7 +62,7 @@ constexpr int BK = 64;
 constexpr int ROW_B = BK * 2;      // LDS row bytes
 constexpr int SLOT = 256 * ROW_B;  // a stage of one operand
 
-enum Form { PLAIN = 0, GATED = 1, SCATTER = 2 };
+enum Form { PLAIN = 0, GATED = 1, SCATTER = 2, PARTS = 3 };
 enum Act { NONE = 0, SILU = 1, CLAMP = 2, RELU2 = 3 };
 
 struct Args {
@@ -199,6 +200,10 @@ DEV_INLINE int table_at(const int *p, int i) {
   return ((const __attribute__((address_space(4))) int *)p)[i];
 }
 
+DEV_INLINE __amdgpu_buffer_rsrc_t bytes_of(float *p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, bytes, 0x00020000);
+}
+
 template <int V> struct Int { static constexpr int value = V; };
 
 // f(Int<0>), f(Int<1>), ... f(Int<N - 1>)
@@ -253,7 +258,9 @@ DEV_INLINE shortx8 results(const float *g, const float *u, float scale,
   return o;
 }
 
-template <int FORM, int ACT, bool GROUPED, bool BIAS>
+// ONCE: a weight row is read by one workgroup (non-temporal loads leave the
+// L2 to x)
+template <int FORM, int ACT, bool GROUPED, bool BIAS, bool ONCE = false>
 __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   // two stages of x, then three of W
   __shared__ __attribute__((aligned(16))) char smem[5 * SLOT];
@@ -374,6 +381,11 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         r, (lds_void *)(slot + wave * 1024 + j * 4096), 16, v, lso, 0, 0);
   };
+  auto load_w = [&](char *slot, int v, int j) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rw, (lds_void *)(slot + wave * 1024 + j * 4096), 16, v, lso, 0,
+        ONCE ? 2 : 0);
+  };
 
   tg_bf8 fa[2][8], fb[2][8];  // fragments of 32 columns
   const int off = (lhi ^ (l16 & 7)) << 4;
@@ -396,7 +408,7 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
     advance();
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      load(rw, sw + s * SLOT, vw[j], j);
+      load_w(sw + s * SLOT, vw[j], j);
       load(ra, smem + s * SLOT, va[j], j);
     }
   }
@@ -452,7 +464,7 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
           }
           if (i % LD == LD / 2 && i / LD < 8) {
             ORDER;
-            load(rw, sw + wn2, vw[i / LD], i / LD);
+            load_w(sw + wn2, vw[i / LD], i / LD);
             ORDER;
           }
           Sum<i>::add(fb[0][i & 7], fa[0][i >> 3]);
@@ -500,6 +512,25 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
       int x16 = l16, xhi = lhi;  // addresses are formed here, not above
       asm volatile("" : "+v"(x16), "+v"(xhi));
       const int r0 = wm * MT * 16 + x16;  // row of the tile
+      if (FORM == PARTS) {
+        // (a row is N * 4 bytes; rows and columns outside are not stored)
+        const int s = RFL(it.part / R);
+        const int rows = RFL(min(P.bm, P.M - it.mb * P.bm));
+        const auto rc = bytes_of(
+            P.part + ((long)s * P.M + it.mb * P.bm) * P.N, rows * P.N * 4);
+        const int c0 = it.nb * 256 + wn * 128 + xhi * 8;
+        repeat<P1>([&](auto at) {
+          constexpr int i = decltype(at)::value, n = i & 7, m = i >> 3;
+          constexpr int dc = (n >> 1) * 32 + (n & 1) * 4;
+          ORDER;
+          const bool used = r0 + m * 16 < rows && c0 + dc < P.N;
+          __builtin_amdgcn_raw_buffer_store_b128(
+              __builtin_bit_cast(tg_u4, Sum<i>::get()), rc,
+              used ? ((r0 + m * 16) * P.N + c0 + dc) * 4 : 0x7ffffff0, 0, 0);
+        });
+        stores = P1;
+        return;
+      }
       if (!GROUPED && it.part >= 0) {
         float *p = P.part + (long)it.part * 65536 + r0 * 256 + wn * 128 +
                    xhi * 8;
@@ -749,7 +780,10 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w,
   auto stream = at::cuda::getCurrentCUDAStream();
   // (whole multiples of eight: as many workgroups as tiles on each die)
   const dim3 grid(std::min((items + 7) / 8 * 8, cus)), block(256);
-  if (gated)
+  if (gated && p.nbm == 1)  // (256 x 55296 x 5120 137 us, 151 without)
+    hipLaunchKernelGGL((tile_gemm_kernel<GATED, SILU, false, false, true>),
+                       grid, block, 0, stream, P);
+  else if (gated)
     hipLaunchKernelGGL((tile_gemm_kernel<GATED, SILU, false, false>), grid,
                        block, 0, stream, P);
   else if (P.bias)
@@ -769,6 +803,68 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w,
     HIP_CHECK_KERNEL();
   }
   return out;
+}
+
+// Row block and splits of few rows (at most 256), 0 splits where the
+// streaming kernel's ring is the better one. A round of workgroups at most.
+// Rows beyond 128 are one block while the parts are at most 0.4 of the
+// weight's bytes, else two of 128 rows with half the splits (us with the norm
+// that sums the parts, one / two: 256 x 5120 x 27648 81 / 95, 256 x 5120 x
+// 5120 44 / 36, 256 x 4096 x 14336 57 / 51, 136 x 7168 x 5120 37 / 38).
+// Against the stream (stream / this): 256 x 5120 x 27648 113 / 81, 256 x 7168
+// x 5120 48 / 42, 256 x 5120 x 5120 45 / 36, 160 x 6144 x 4096 37 / 31, 96 x
+// 5120 x 5120 31 / 28, 128 x 4096 x 14336 44 / 39; below 24 M weights its
+// short parts lose (256 x 4096 x 4096 28 / 28, 256 x 6144 x 2048 25 / 27).
+// Up to 64 rows only long streams gain: 64 x 5120 x 27648 73 / 63, 40 x 10240
+// x 8192 42 / 38, but 64 x 4096 x 14336 37 / 37, 64 x 7168 x 5120 28 / 31.
+void tile_parts_plan(long M, long N, long K, int *bm, int *splits) {
+  *splits = 0;
+  *bm = M > 128 ? 256 : 128;
+  const long weights = N * K, nbn = (N + 255) / 256;
+  const int cus = compute_units(), nkt = K / BK;
+  if (M <= 32 || M > 256 || nbn > cus || N > (1 << 20) || K > (1 << 21) ||
+      weights < (M > 64 ? 24L << 20 : 72L << 20) || (M <= 64 && K < 8192))
+    return;
+  auto most = [&](int blocks) {
+    return (int)std::min<long>(std::min<long>(cus / (nbn * blocks), nkt / 4),
+                               16);
+  };
+  int s = most(1);
+  if (M > 128 && 5 * s * M > K && most(2) > 0) {
+    *bm = 128;
+    s = most(2);
+  }
+  *splits = s;
+}
+
+// The fp32 parts [S, M, N] of x w^T, each over a share of K (operands checked
+// by stream_parts; sizes as tile_parts_plan takes them).
+void tile_parts(float *part, const void *x, const void *w, long M, long N,
+                long K, int bm, int splits) {
+  Args P{};
+  P.A = (const __hip_bfloat16 *)x;
+  P.W = (const __hip_bfloat16 *)w;
+  P.part = part;
+  P.M = M;
+  P.N = N;
+  P.K = K;
+  P.bm = bm;
+  P.nbm = (M + bm - 1) / bm;
+  P.nbn = (N + 255) / 256;
+  P.whole = 0;
+  P.splits = splits;
+  P.group = P.nbm;
+  set_divisors(P);
+  const int items = P.nbm * P.nbn * splits;
+  const dim3 grid(std::min((items + 7) / 8 * 8, compute_units())), block(256);
+  auto stream = at::cuda::getCurrentCUDAStream();
+  if (P.nbm == 1)
+    hipLaunchKernelGGL((tile_gemm_kernel<PARTS, NONE, false, false, true>),
+                       grid, block, 0, stream, P);
+  else
+    hipLaunchKernelGGL((tile_gemm_kernel<PARTS, NONE, false, false>), grid,
+                       block, 0, stream, P);
+  HIP_CHECK_KERNEL();
 }
 
 // The grouped forms over blocks of 256 rows (operands checked by

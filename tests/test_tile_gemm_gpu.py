@@ -79,3 +79,34 @@ def test_dispatch(M):
     y = torch.nn.functional.silu(g) * u
     out = ops.linear_silu(x, w)
     assert ((out.double() - y).norm() / y.norm()) < 2 ** -7
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (32, 9216, 8192),        # the stream's last row count
+    (33, 9216, 8192), (64, 9216, 8192),    # long streams
+    (65, 5128, 5120), (128, 5120, 5120),   # half a block, ragged columns
+    (129, 5128, 5120), (256, 5120, 5120),  # two blocks of 128 rows
+    (129, 9208, 8192), (200, 5120, 27648),  # one block
+])
+@pytest.mark.parametrize("gated", [False, True])
+def test_few_rows(M, N, K, gated):
+    """Parts of wide weights, and the gated form on very wide ones."""
+    from gllm_amd import ops
+    if gated:
+        N, K = {5120: 65536, 5128: 49152}.get(N, 49168), 4096
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    y = x.double() @ w.double().t()
+    if gated:
+        g, u = y.chunk(2, dim=-1)
+        y = torch.nn.functional.silu(g) * u
+        out = ops.linear_silu(x, w).double()
+        bound = 1.1 * 2 ** -8   # one rounding to bf16
+    else:
+        part = ops._gpu_kernels().stream_parts(x, w)
+        assert part.shape[1:] == (M, N)
+        out = part.double().sum(0)
+        bound = 2 ** -23 * K ** 0.5  # fp32 sums: a rounding per 32 columns
+    err = (out - y).abs() / y.abs().clamp_min(y.square().mean().sqrt())
+    assert err.max() < bound, err.max()
