@@ -16,6 +16,10 @@
 // load's source address. Tiles that no row of a wave can see are skipped
 // by that wave; tiles every row sees wholly skip the mask.
 //
+// Plain causal attention of 64 or 128 dims goes to attention_causal.hip: the
+// options that this kernel can carry are selects in every tile, 60 % of its
+// instructions.
+//
 // Capability parity: flash_attn_with_kvcache varlen semantics
 // (reference layers/attention.py:77-141) — one kernel serves chunked
 // prefill, mixed prefill+decode batches, prefix-cache hits and sliding
@@ -24,6 +28,7 @@
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
+#include "attention_causal.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 mfma_bf8;
 typedef __attribute__((ext_vector_type(4))) float mfma_f4;
@@ -461,6 +466,17 @@ void launch_prefill(torch::Tensor &out, torch::Tensor &q, int Hq,
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 &&
       (!gate || (gate_stride % 4 == 0 &&
                  reinterpret_cast<uintptr_t>(gate) % 8 == 0)) ? 1 : 0;
+  // nothing but causal softmax (us, here / there: see attention_causal.hip)
+  if (!ext && vec_out && window <= 0 && !sink && !sinks && !gate &&
+      softcap == 0.f && causal_prefill_ok(D, Dv, (float)scale)) {
+    causal_prefill(out.data_ptr(), out_stride, q.data_ptr(), q_stride,
+                   k_cache.data_ptr(), v_cache.data_ptr(),
+                   block_table.data_ptr<int>(), block_table.stride(0),
+                   k_cache.size(1), seq_lens.data_ptr<int>(),
+                   query_start_loc.data_ptr<int>(), B, q.size(0),
+                   max_query_len, Hq, Hkv, D, (float)scale, min_rows);
+    return;
+  }
   const size_t lds =
       bias && bias_len <= BIAS_LDS
           ? (bias_len + 2 * BIAS_PAD) * sizeof(float) : 0;

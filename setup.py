@@ -34,13 +34,14 @@ CXX_FLAGS = ["-O3", "-std=c++17"]
 SEQ_SOURCES = ["bindings_seq.cpp", "layernorm.hip", "hyper.hip",
                "mingru.hip", "linear_scan.hip", "attention_window.hip",
                "attention_talking.hip", "attention_latent.hip",
-               "attention_prefill.hip", "attention_decode.hip",
-               "delta_rule.hip", "moe.hip", "moe_tiled.hip", "tile_gemm.hip",
-               "elementwise.hip", "stream_gemm.hip"]
+               "attention_prefill.hip", "attention_causal.hip",
+               "attention_decode.hip", "delta_rule.hip", "moe.hip",
+               "moe_tiled.hip", "tile_gemm.hip", "elementwise.hip",
+               "stream_gemm.hip"]
 CORE_SOURCES = ["bindings.cpp", "norm.hip", "elementwise.hip",
                 "attention_decode.hip", "attention_prefill.hip",
-                "attention_mla.hip", "mla_proj.hip", "moe.hip",
-                "moe_tiled.hip", "tile_gemm.hip", "fp8.hip",
+                "attention_causal.hip", "attention_mla.hip", "mla_proj.hip",
+                "moe.hip", "moe_tiled.hip", "tile_gemm.hip", "fp8.hip",
                 "gdn.hip", "int4.hip", "quant_gemm.hip", "stream_gemm.hip",
                 "sampling.hip",
                 "custom_ar.hip"]
