@@ -146,6 +146,10 @@ class MLAAttention(nn.Module):
                     and ops.mla_absorbed_ok(q, kv_a, w_kvb, norm.weight,
                                             k_cache, cos_sin, self.qk_nope,
                                             self.v_dim)):
+                first = self._prompts_from(fctx)
+                if first < fctx.seq_lens.shape[0]:
+                    return self._with_prompts(first, positions, hidden,
+                                              q_resid, q, kv_a, fctx)
                 qf = ops.mla_queries(q, kv_a, norm.weight, norm.eps,
                                      positions, cos_sin, w_kvb, k_cache,
                                      fctx.slot_mapping)
@@ -187,6 +191,46 @@ class MLAAttention(nn.Module):
             seq_lens_cpu=fctx.host_seq_lens(),
             query_start_loc_cpu=fctx.host_qsl())
         return out.reshape(T, -1)
+
+    def _prompts_from(self, fctx):
+        """First sequence that attends in the per-head form (all of them
+        from there on are whole prompts)."""
+        if type(self)._dsa_select is not MLAAttention._dsa_select:
+            return fctx.seq_lens.shape[0]  # (selected positions only)
+        return fctx.prompts_from()
+
+    def _with_prompts(self, first, positions, hidden, q_resid, q, kv_a,
+                      fctx):
+        """``heads`` of a batch whose sequences from ``first`` on are whole
+        prompts: those per head, what comes before them absorbed."""
+        qsl = fctx.host_qsl()
+        row, end = qsl[first], qsl[fctx.seq_lens.shape[0]]
+        w_kvb, norm = self.kv_b_proj.weight, self.kv_a_layernorm
+        cos_sin = self.rotary_emb.cos_sin_cache
+        k_cache = fctx.k_caches[self.layer_idx]
+        slots, starts = fctx.slot_mapping, fctx.query_start_loc
+        out = q.new_empty(q.shape[0], self.num_heads * self.v_dim)
+        if row > 0:
+            qf = ops.mla_queries(q[:row], kv_a[:row], norm.weight, norm.eps,
+                                 positions[:row], cos_sin, w_kvb, k_cache,
+                                 slots[:row])
+            lat = ops.mla_paged_attention(
+                qf, k_cache, fctx.v_caches[self.layer_idx],
+                fctx.block_table[:first], fctx.seq_lens[:first],
+                starts[:first + 1], self.scale,
+                seq_lens_cpu=fctx.host_seq_lens()[:first],
+                query_start_loc_cpu=qsl[:first + 1])
+            out[:row] = ops.mla_values(lat, w_kvb)
+        lens = [b - a for a, b in zip(qsl[first:], qsl[first + 1:])]
+        starts = starts[first:] if starts.dtype == torch.int32 \
+            else starts[first:].int()
+        if row > 0:
+            starts = starts - row
+        ops.mla_prompts(q[row:end], kv_a[row:end], norm.weight, norm.eps,
+                        positions[row:end], cos_sin, w_kvb, k_cache,
+                        slots[row:end], starts, max(lens), self.scale,
+                        out[row:end])
+        return out
 
     def _attend(self, qf, positions, hidden, q_resid, fctx):
         """Latent attention of the query rows [T, H, lora + rope] over

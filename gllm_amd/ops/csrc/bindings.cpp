@@ -72,6 +72,13 @@ torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
                           torch::Tensor w_kvb, torch::Tensor k_cache,
                           torch::Tensor slots);
 torch::Tensor mla_values(torch::Tensor o_lat, torch::Tensor w_kvb);
+std::vector<torch::Tensor> mla_prompt_rows(
+    torch::Tensor q, torch::Tensor kv, torch::Tensor norm_w, double eps,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor k_cache,
+    torch::Tensor slots);
+void mla_prompts(torch::Tensor out, torch::Tensor q, torch::Tensor kv,
+                 torch::Tensor pe, torch::Tensor query_start_loc,
+                 long max_query_len, double scale);
 void cache_latent(torch::Tensor k, torch::Tensor k_cache,
                   torch::Tensor slot_mapping);
 void moe_align(torch::Tensor topk_ids, long E_local, long expert_start,
@@ -191,6 +198,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "absorbed-MLA varlen attention over the 576-dim latent cache");
   m.def("mla_queries", &mla_queries,
         "latent cache rows and absorbed, rotated query rows");
+  m.def("mla_prompt_rows", &mla_prompt_rows,
+        "normed and rotated latent rows of prompts, queries in place");
+  m.def("mla_prompts", &mla_prompts, "per-head attention of whole prompts");
   m.def("mla_values", &mla_values, "per-head values of the weighted latent");
   m.def("cache_latent", &cache_latent,
         "scatter the per-token latent row into the paged cache");

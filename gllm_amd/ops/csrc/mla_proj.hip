@@ -60,12 +60,15 @@ DEV_INLINE void rotate8(const __hip_bfloat16 *src, __hip_bfloat16 *dst,
   st8<__hip_bfloat16>(dst + 32 + d, y);
 }
 
-// 4 waves: wave 0 the latent row, waves 1 to 3 the queries
-template <typename TW>
+// 4 waves: wave 0 the latent row, waves 1 to 3 the queries. PROMPT: the latent
+// goes to lat and pe too, and the queries are turned where they are.
+template <typename TW, bool PROMPT>
 __global__ __launch_bounds__(256) void mla_prepare_kernel(
     __hip_bfloat16 *__restrict__ qf,        // [T, H, DK] (dims LORA..)
+    __hip_bfloat16 *__restrict__ lat,       // [T, LORA]
+    __hip_bfloat16 *__restrict__ pe,        // [T, ROPE]
     __hip_bfloat16 *__restrict__ k_cache,   // [slots, DK]
-    const __hip_bfloat16 *__restrict__ q, long q_stride,
+    __hip_bfloat16 *q, long q_stride,
     const __hip_bfloat16 *__restrict__ kv, long kv_stride,
     const TW *__restrict__ norm_w, float eps,
     const long *__restrict__ positions, const float *__restrict__ cos_sin,
@@ -85,13 +88,16 @@ __global__ __launch_bounds__(256) void mla_prepare_kernel(
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = x[i] * inv * w[i];
     st8<__hip_bfloat16>(dst + lane * 8, x);
+    if (PROMPT) st8<__hip_bfloat16>(lat + t * LORA + lane * 8, x);
     if (lane < 4) rotate8(row + LORA, dst + LORA, cs, lane * 8);
+    if (PROMPT && lane < 4) rotate8(row + LORA, pe + t * ROPE, cs, lane * 8);
     return;
   }
   for (int i = threadIdx.x - 64; i < H * 4; i += 192) {
     const int h = i >> 2;
-    rotate8(q + t * q_stride + h * QD + NOPE,
-            qf + (t * H + h) * (long)DK + LORA, cs, (i & 3) * 8);
+    __hip_bfloat16 *src = q + t * q_stride + h * QD + NOPE;
+    rotate8(src, PROMPT ? src : qf + (t * H + h) * (long)DK + LORA, cs,
+            (i & 3) * 8);
   }
 }
 
@@ -201,28 +207,21 @@ void check16(const torch::Tensor &t, const char *what) {
               reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, what);
 }
 
-}  // namespace
-
-// q [T, H * 192], kv [T, 576] (row views allowed), norm_w [512] fp32 or
-// bf16, w_kvb [H * 256, 512]; writes the cache rows of `slots`, returns the
-// query rows [T, H, 576].
-torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
-                          torch::Tensor norm_w, double eps,
-                          torch::Tensor positions, torch::Tensor cos_sin,
-                          torch::Tensor w_kvb, torch::Tensor k_cache,
-                          torch::Tensor slots) {
+// What mla_queries and mla_prompt_rows take: q [T, H * 192], kv [T, 576] (row
+// views allowed), norm_w [512] fp32 or bf16
+void check_rows(const torch::Tensor &q, const torch::Tensor &kv,
+                const torch::Tensor &norm_w, const torch::Tensor &positions,
+                const torch::Tensor &cos_sin, const torch::Tensor &k_cache,
+                const torch::Tensor &slots) {
   const long T = q.size(0);
   check16(q, "q: bf16, 16 B aligned");
   check16(kv, "kv: bf16, 16 B aligned");
-  check16(w_kvb, "w_kvb: bf16, 16 B aligned");
   check16(k_cache, "k_cache: bf16, 16 B aligned");
   const int H = q.size(1) / QD;
   TORCH_CHECK(q.dim() == 2 && q.size(1) == (long)H * QD && H > 0 &&
               q.stride(1) == 1 && q.stride(0) % 8 == 0);
   TORCH_CHECK(kv.dim() == 2 && kv.size(0) == T && kv.size(1) == DK &&
               kv.stride(1) == 1 && kv.stride(0) % 8 == 0);
-  TORCH_CHECK(w_kvb.is_contiguous() && w_kvb.size(0) == (long)H * WROWS &&
-              w_kvb.size(1) == LORA);
   TORCH_CHECK(k_cache.is_contiguous() && k_cache.size(-1) == DK);
   TORCH_CHECK(positions.scalar_type() == at::kLong &&
               positions.is_contiguous() && positions.numel() == T);
@@ -231,32 +230,82 @@ torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
   TORCH_CHECK(cos_sin.scalar_type() == at::kFloat &&
               cos_sin.is_contiguous() && cos_sin.size(-1) == ROPE);
   TORCH_CHECK(norm_w.is_contiguous() && norm_w.numel() == LORA &&
-              reinterpret_cast<uintptr_t>(norm_w.data_ptr()) % 16 == 0);
-  auto qf = torch::empty({T, (long)H, (long)DK}, q.options());
-  if (T == 0) return qf;
+              reinterpret_cast<uintptr_t>(norm_w.data_ptr()) % 16 == 0 &&
+              (norm_w.scalar_type() == at::kFloat ||
+               norm_w.scalar_type() == at::kBFloat16),
+              "norm_w: fp32 or bf16");
+}
+
+// qf: the query rows of the absorbed form, nullptr for prompts
+void prepare(void *qf, void *lat, void *pe, torch::Tensor &q,
+             const torch::Tensor &kv, const torch::Tensor &norm_w, float eps,
+             const torch::Tensor &positions, const torch::Tensor &cos_sin,
+             const torch::Tensor &k_cache, const torch::Tensor &slots) {
+  const long T = q.size(0);
   auto stream = at::cuda::getCurrentCUDAStream();
-#define PREP(TW)                                                             \
-  hipLaunchKernelGGL((mla_prepare_kernel<TW>), dim3(T), dim3(256), 0, stream,\
-                     (__hip_bfloat16 *)qf.data_ptr(),                        \
+#define PREP(TW, PROMPT)                                                     \
+  hipLaunchKernelGGL((mla_prepare_kernel<TW, PROMPT>), dim3(T), dim3(256),   \
+                     0, stream, (__hip_bfloat16 *)qf, (__hip_bfloat16 *)lat, \
+                     (__hip_bfloat16 *)pe,                                   \
                      (__hip_bfloat16 *)k_cache.data_ptr(),                   \
-                     (const __hip_bfloat16 *)q.data_ptr(),                   \
-                     (long)q.stride(0),                                      \
+                     (__hip_bfloat16 *)q.data_ptr(), (long)q.stride(0),      \
                      (const __hip_bfloat16 *)kv.data_ptr(),                  \
-                     (long)kv.stride(0), (const TW *)norm_w.data_ptr(),      \
-                     (float)eps, positions.data_ptr<long>(),                 \
-                     cos_sin.data_ptr<float>(), slots.data_ptr<long>(), H)
-  if (norm_w.scalar_type() == at::kFloat) PREP(float);
-  else if (norm_w.scalar_type() == at::kBFloat16) PREP(__hip_bfloat16);
-  else TORCH_CHECK(false, "norm_w: fp32 or bf16");
+                     (long)kv.stride(0), (const TW *)norm_w.data_ptr(), eps, \
+                     positions.data_ptr<long>(), cos_sin.data_ptr<float>(),  \
+                     slots.data_ptr<long>(), (int)(q.size(1) / QD))
+  const bool wide = norm_w.scalar_type() == at::kFloat;
+  if (qf && wide) PREP(float, false);
+  else if (qf) PREP(__hip_bfloat16, false);
+  else if (wide) PREP(float, true);
+  else PREP(__hip_bfloat16, true);
 #undef PREP
   HIP_CHECK_KERNEL();
+}
+
+}  // namespace
+
+// w_kvb [H * 256, 512]; writes the cache rows of `slots`, returns the query
+// rows [T, H, 576].
+torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
+                          torch::Tensor norm_w, double eps,
+                          torch::Tensor positions, torch::Tensor cos_sin,
+                          torch::Tensor w_kvb, torch::Tensor k_cache,
+                          torch::Tensor slots) {
+  check_rows(q, kv, norm_w, positions, cos_sin, k_cache, slots);
+  const long T = q.size(0);
+  const int H = q.size(1) / QD;
+  check16(w_kvb, "w_kvb: bf16, 16 B aligned");
+  TORCH_CHECK(w_kvb.is_contiguous() && w_kvb.size(0) == (long)H * WROWS &&
+              w_kvb.size(1) == LORA);
+  auto qf = torch::empty({T, (long)H, (long)DK}, q.options());
+  if (T == 0) return qf;
+  prepare(qf.data_ptr(), nullptr, nullptr, q, kv, norm_w, (float)eps,
+          positions, cos_sin, k_cache, slots);
   hipLaunchKernelGGL(mla_absorb_kernel,
                      dim3((T + TOK - 1) / TOK, H, LORA / CHUNK), dim3(256),
-                     0, stream, (__hip_bfloat16 *)qf.data_ptr(),
+                     0, at::cuda::getCurrentCUDAStream(),
+                     (__hip_bfloat16 *)qf.data_ptr(),
                      (const __hip_bfloat16 *)q.data_ptr(), (long)q.stride(0),
                      (const __hip_bfloat16 *)w_kvb.data_ptr(), (int)T, H);
   HIP_CHECK_KERNEL();
   return qf;
+}
+
+// Rows of prompts: turns the rotated parts of q in place, writes the cache
+// rows of `slots`, returns the normed latents [T, 512] and the shared rotated
+// key parts [T, 64].
+std::vector<torch::Tensor> mla_prompt_rows(
+    torch::Tensor q, torch::Tensor kv, torch::Tensor norm_w, double eps,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor k_cache,
+    torch::Tensor slots) {
+  check_rows(q, kv, norm_w, positions, cos_sin, k_cache, slots);
+  const long T = q.size(0);
+  auto lat = torch::empty({T, (long)LORA}, q.options());
+  auto pe = torch::empty({T, (long)ROPE}, q.options());
+  if (T > 0)
+    prepare(nullptr, lat.data_ptr(), pe.data_ptr(), q, kv, norm_w,
+            (float)eps, positions, cos_sin, k_cache, slots);
+  return {lat, pe};
 }
 
 // o_lat [T, H, 512] -> [T, H * 128]

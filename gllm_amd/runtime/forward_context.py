@@ -63,6 +63,22 @@ class ForwardContext:
     seq_lens_cpu: Optional[List[int]] = None
     query_start_loc_cpu: Optional[List[int]] = None
 
+    _prompts_from: Optional[int] = dataclasses.field(default=None,
+                                                     kw_only=True)
+
+    def prompts_from(self) -> int:
+        """The first sequence from which on all are whole prompts: two rows
+        or more and nothing in the cache (their number if there are none)."""
+        if self._prompts_from is None:
+            s = self.seq_lens.shape[0]
+            if self.max_query_len > 1:
+                qsl, lens = self.host_qsl(), self.host_seq_lens()
+                while s > 0 and lens[s - 1] > 1 and \
+                        lens[s - 1] == qsl[s] - qsl[s - 1]:
+                    s -= 1
+            self._prompts_from = s
+        return self._prompts_from
+
     @property
     def is_pure_decode(self) -> bool:
         return self.max_query_len == 1
