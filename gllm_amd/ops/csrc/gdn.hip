@@ -155,8 +155,9 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // Accumulation, T and the state stay fp32. Error of the state against 64
 // bits, 64 to 1500 tokens, weak and strong decay: 1.1e-7 to 5.2e-7 (1.7e-7 to
 // 5.3e-7 with fp32 instructions, mean 2.5e-7 against 2.9e-7).
-// 4096 tokens in four prompts, 16 heads of 128: 60 + 150 us (212 + 200 with
-// fp32 instructions throughout and the triangular system solved column strip
+// 4096 tokens in four prompts, 16 heads of 128: 59 + 127 us (carry 145 with a
+// 64-bit address and a branch for each load, with stores inside the wait for
+// the next chunk's operands, and one sum after the other; 212 + 200 with fp32 instructions throughout and the triangular system solved column strip
 // by column strip; 922 for one kernel that did all of it chunk after chunk on
 // a workgroup per sequence, head and 64 columns). local is bound by its
 // stores (X, att: 105 MB); carry by the serial chain of the longest prompt, a
@@ -186,15 +187,8 @@ DEV_INLINE gdn_f4 mma32(const GdnFrag &a, const GdnFrag &b, gdn_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, c, 0, 0, 0);
 }
 
-DEV_INLINE gdn_f4 mma6(const GdnFrag (&a)[3], const GdnFrag (&b)[3],
-                       gdn_f4 c) {
-  c = mma32(a[2], b[0], c);
-  c = mma32(a[0], b[2], c);
-  c = mma32(a[1], b[1], c);
-  c = mma32(a[1], b[0], c);
-  c = mma32(a[0], b[1], c);
-  return mma32(a[0], b[0], c);
-}
+// terms of a product of two numbers of three parts each, small ones first
+constexpr int TERM_A[6] = {2, 0, 1, 1, 0, 0}, TERM_B[6] = {0, 2, 1, 0, 1, 0};
 
 // x as a sum of three bf16 numbers
 DEV_INLINE void split3(float x, short &h, short &m, short &l) {
@@ -466,6 +460,12 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
   }
 }
 
+// bytes from p on
+template <typename T_>
+DEV_INLINE __amdgpu_buffer_rsrc_t rows_of(const T_ *p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, bytes, 0x00020000);
+}
+
 // DVS value columns of a (sequence, head)
 template <int DVS>
 __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
@@ -521,53 +521,58 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
   put_state();
 
   // operands of a chunk, on their way in registers
-  shortx8 wr[4][3], ar[2][3], qr[4], kr[4];
+  shortx8 wr[4][3], ar[2][3] = {}, qr[4], kr[4];
   float ur[VT][4], sr;
+  // Rows of a chunk by descriptors that end with it (what lies past is zero):
+  // addresses are a lane's fixed offsets, where 64 bits and a branch for each
+  // load were a third of the loop's instructions.
+  const int row_b = Hv * D * 2, key_b = (int)qk_stride * 2;
+  const int w_at = (wave * 16 + l16) * row_b + lhi * 16;
+  const int a_at = (wave * 16 + l16) * (Hv * C * 2) + lhi * 16;
+  const int q_at = (wave * 16 + l16) * key_b + lhi * 16;
+  const int k_at = (tid >> 4) * key_b + (tid & 15) * 16;
+  const int u_at = (wave * 16 + lhi * 4) * (row_b * 2) + l16 * 4;
+  auto load16 = [](__amdgpu_buffer_rsrc_t r, int at) {
+    return __builtin_bit_cast(
+        shortx8, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+  };
   auto fetch = [&](int start) {
     const int len = min(C, end - start);
-    {
-      const int t = wave * 16 + l16;
-      const bool live = t < len;
-      const long row = start + min(t, len - 1);
-      const shortx8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const __amdgpu_buffer_rsrc_t rq =
+        rows_of(q + start * qk_stride + hk * D, (len - 1) * key_b + D * 2);
+    const __amdgpu_buffer_rsrc_t rk =
+        rows_of(k + start * qk_stride + hk * D, (len - 1) * key_b + D * 2);
+    const __amdgpu_buffer_rsrc_t ru =
+        rows_of(u0 + ((long)start * Hv + h) * D + z * DVS,
+                (len - 1) * row_b * 2 + DVS * 4);
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+    for (int j = 0; j < 3; ++j) {
+      const __amdgpu_buffer_rsrc_t rw =
+          rows_of(wk + ((j * T + start) * Hv + h) * D,
+                  (len - 1) * row_b + D * 2);
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          wr[ks][j] = live ? *reinterpret_cast<const shortx8 *>(
-                                 wk + ((j * T + row) * Hv + h) * D + ks * 32 +
-                                 lhi * 8)
-                           : zero;
-        qr[ks] = *reinterpret_cast<const shortx8 *>(
-            q + row * qk_stride + hk * D + ks * 32 + lhi * 8);
-      }
+      for (int ks = 0; ks < 4; ++ks) wr[ks][j] = load16(rw, w_at + ks * 64);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qr[ks] = load16(rq, q_at + ks * 64);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const __amdgpu_buffer_rsrc_t ra =
+          rows_of(att + ((j * T + start) * Hv + h) * C,
+                  ((len - 1) * Hv + 1) * C * 2);
+      ar[0][j] = load16(ra, a_at);
       // (blocks past the diagonal's pair are never written, nor read)
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          ar[kk][j] = live && kk <= wave / 2
-                          ? *reinterpret_cast<const shortx8 *>(
-                                att + ((j * T + row) * Hv + h) * C + kk * 32 +
-                                lhi * 8)
-                          : zero;
+      if (wave >= 2) ar[1][j] = load16(ra, a_at + 64);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int u = j * 256 + tid;
-      kr[j] = *reinterpret_cast<const shortx8 *>(
-          k + (long)(start + min(u >> 4, len - 1)) * qk_stride + hk * D +
-          (u & 15) * 8);
-    }
+    for (int j = 0; j < 4; ++j) kr[j] = load16(rk, k_at + j * 16 * key_b);
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = wave * 16 + lhi * 4 + r;
-        ur[vt][r] = t < len ? u0[((long)(start + t) * Hv + h) * D + z * DVS +
-                                 vt * 16 + l16]
-                            : 0.f;
-      }
+      for (int r = 0; r < 4; ++r)
+        ur[vt][r] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(
+                       ru, u_at + r * row_b * 2 + vt * 64, 0, 0));
     sr = scal[(min(wave, 2) * T + start + min(lane, len - 1)) * Hv + h];
   };
   auto put_keys = [&](int buf) {
@@ -607,19 +612,34 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
       xs[vt] = qs[vt] = gdn_f4{0, 0, 0, 0};
+    // (one wave per SIMD: nothing else hides the latency of a chain of
+    // products or of an LDS read, so the sums take turns and fragments are
+    // read a step ahead)
+    GdnFrag sf[2][VT][3];
+    auto read_state = [&](int ks) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        GdnFrag sf[3];
+      for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          sf[j].s = *reinterpret_cast<const shortx8 *>(
+          sf[ks & 1][vt][j].s = *reinterpret_cast<const shortx8 *>(
               Sp[j] + (vt * 16 + l16) * SB + ks * 32 + lhi * 8);
-        xs[vt] = mma6(w[ks], sf, xs[vt]);
+    };
+    read_state(0);
 #pragma unroll
-        for (int j = 2; j >= 0; --j) qs[vt] = mma32(qf[ks], sf[j], qs[vt]);
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) read_state(ks + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) {
+          xs[vt] = mma32(w[ks][TERM_A[i]], sf[ks & 1][vt][TERM_B[i]], xs[vt]);
+          if (i % 2 == vt)
+            qs[vt] = mma32(qf[ks], sf[ks & 1][vt][2 - i / 2], qs[vt]);
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const float last = sc[cur][0][len - 1];
     gdn_f4 wc, eb;
 #pragma unroll
@@ -644,28 +664,53 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     }
     __syncthreads();
     // ---- o = B q S^T + att U
+    GdnFrag uf[2][VT][3], kf[2][2], wf[2][VT][3];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          uf[kk][vt][j].s = *reinterpret_cast<const shortx8 *>(
+              Up[j] + (vt * 16 + l16) * UB + kk * 32 + lhi * 8);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {  // the state's, for below
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+        read_tr(kf[kk][dt], Kt[cur], KB, kk * 32, (wave * 2 + dt) * 16, l16,
+                lhi);
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+            wf[kk][vt][j].h[half] = *reinterpret_cast<const shortx4 *>(
+                Up[3 + j] + (vt * 16 + l16) * UB + kk * 32 + half * 16 +
+                lhi * 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       if (kk > wave / 2) continue;
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        GdnFrag uf[3];
+      for (int i = 0; i < 6; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          uf[j].s = *reinterpret_cast<const shortx8 *>(
-              Up[j] + (vt * 16 + l16) * UB + kk * 32 + lhi * 8);
-        qs[vt] = mma6(at[kk], uf, qs[vt]);
-      }
+        for (int vt = 0; vt < VT; ++vt)
+          qs[vt] = mma32(at[kk][TERM_A[i]], uf[kk][vt][TERM_B[i]], qs[vt]);
     }
+    // (rows past the end fall outside: with a branch around each store the
+    // wait for the next chunk's operands would be one for these stores too)
+    const __amdgpu_buffer_rsrc_t ro =
+        rows_of(o + ((long)start * Hv + h) * D + z * DVS,
+                (len - 1) * row_b + DVS * 2);
 #pragma unroll
     for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = wave * 16 + lhi * 4 + r;
-        if (t < len)
-          o[((long)(start + t) * Hv + h) * D + z * DVS + vt * 16 + l16] =
-              __float2bfloat16(qs[vt][r]);
-      }
+      for (int r = 0; r < 4; ++r)
+        __builtin_amdgcn_raw_buffer_store_b16(
+            __builtin_bit_cast(short, __float2bfloat16(qs[vt][r])), ro,
+            (wave * 16 + lhi * 4 + r) * row_b + l16 * 2 + vt * 32, 0, 0);
     // ---- S = B_last S + (exp(b_last - b) U)^T k
     const float keep = __expf(last);
 #pragma unroll
@@ -673,26 +718,14 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt) s[vt][dt] *= keep;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      GdnFrag kf[2];
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-        read_tr(kf[dt], Kt[cur], KB, kk * 32, (wave * 2 + dt) * 16, l16, lhi);
+      for (int j = 2; j >= 0; --j)
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int j = 2; j >= 0; --j) {
-          GdnFrag uf;
-#pragma unroll
-          for (int half = 0; half < 2; ++half)
-            uf.h[half] = *reinterpret_cast<const shortx4 *>(
-                Up[3 + j] + (vt * 16 + l16) * UB + kk * 32 + half * 16 +
-                lhi * 4);
+        for (int vt = 0; vt < VT; ++vt)
 #pragma unroll
           for (int dt = 0; dt < 2; ++dt)
-            s[vt][dt] = mma32(kf[dt], uf, s[vt][dt]);
-        }
-    }
+            s[vt][dt] = mma32(kf[kk][dt], wf[kk][vt][j], s[vt][dt]);
     put_state();
     if (start + C < end) put_keys(cur ^ 1);
     cur ^= 1;
