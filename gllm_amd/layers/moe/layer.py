@@ -134,6 +134,36 @@ class FusedMoE(nn.Module):
             out = tensor_parallel_all_reduce(out)
         return out
 
+    def routed_add_norm(self, x: torch.Tensor, weights: torch.Tensor,
+                        ids: torch.Tensor, shared: Optional[torch.Tensor],
+                        residual: torch.Tensor, norm):
+        """(norm(residual + (forward_routed(...) + shared)), that sum): one
+        kernel behind the experts where nothing has to be reduced over
+        ranks first."""
+        one_rank = (get_ep_size() if self.use_ep else get_tp_size()) == 1
+        if (one_rank and self._grouped(x)
+                and ops.moe_add_norm_ok(x, shared, residual, norm.scale())):
+            out = ops.fused_moe(
+                x.contiguous(), self.w13_weight, self.w2_weight, weights,
+                ids, expert_start=self.expert_start,
+                num_global_experts=self.num_experts,
+                activation=self.activation, act_args=self.act_args,
+                add_norm=(shared, residual, norm.scale(), norm.eps))
+            return out, residual
+        out = self.forward_routed(x, weights, ids)
+        if shared is not None:
+            out = out + shared
+        return norm(out, residual)
+
+    def _grouped(self, x: torch.Tensor) -> bool:
+        """Unquantized experts for the grouped bf16 product (it loads
+        8-element vectors along K; odd widths take the segment loop)."""
+        return (x.is_cuda and x.dtype == torch.bfloat16
+                and ops.has_moe_kernels() and self.int4_packed is None
+                and self.fp8_block is None and self.int4_cfg is None
+                and x.shape[1] % 8 == 0
+                and self.intermediate_per_rank % 8 == 0)
+
     def _expert_loop(self, x: torch.Tensor, weights: torch.Tensor,
                      ids: torch.Tensor) -> torch.Tensor:
         """Local expert shard over the (possibly DP-gathered) batch;
@@ -174,11 +204,7 @@ class FusedMoE(nn.Module):
                     x.contiguous(), w13s, w2s, weights, ids,
                     expert_start=self.expert_start,
                     num_global_experts=self.num_experts)
-            if (self.fp8_block is None and self.int4_cfg is None
-                    and x.shape[1] % 8 == 0
-                    and self.intermediate_per_rank % 8 == 0):
-                # (the grouped GEMM loads 8-element bf16 vectors along
-                # K; odd widths take the segment loop below)
+            if self._grouped(x):
                 return ops.fused_moe(
                     x.contiguous(), self.w13_weight, self.w2_weight,
                     weights, ids, expert_start=self.expert_start,

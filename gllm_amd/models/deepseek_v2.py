@@ -321,6 +321,14 @@ class DeepseekMoE(nn.Module):
             out = out + self.shared_experts(x)
         return out
 
+    def forward_add_norm(self, x, residual, norm):
+        """(norm(residual + self(x)), that sum)."""
+        weights, ids = self._route(self.gate(x))
+        shared = None if self.shared_experts is None \
+            else self.shared_experts(x)
+        return self.experts.routed_add_norm(x, weights, ids, shared,
+                                            residual, norm)
+
 
 class DeepseekDecoderLayer(nn.Module):
     def __init__(self, cfg, engine_config, layer_idx, global_idx,
@@ -356,9 +364,7 @@ class DeepseekDecoderLayer(nn.Module):
             positions, hidden, residual, self.post_attention_layernorm, fctx)
         if next_norm is None:
             return self.mlp(hidden), residual
-        if isinstance(self.mlp, DenseMLP):
-            return self.mlp.forward_add_norm(hidden, residual, next_norm)
-        return next_norm(self.mlp(hidden), residual)
+        return self.mlp.forward_add_norm(hidden, residual, next_norm)
 
 
 class DeepseekV2ForCausalLM(nn.Module):

@@ -11,6 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from gllm_amd import ops
 from gllm_amd.layers.activation import SiluAndMul
 from gllm_amd.layers.embedding import ParallelLMHead, VocabParallelEmbedding
 from gllm_amd.layers.layernorm import RMSNorm
@@ -52,6 +53,17 @@ class MoEBlock(nn.Module):
             out = out + shared * g
         return out
 
+    def forward_add_norm(self, x, residual, norm):
+        """(norm(residual + self(x)), that sum)."""
+        weights, ids = ops.topk_softmax(self.gate(x), self.experts.top_k,
+                                        self.experts.renormalize)
+        shared = None
+        if self.shared_expert is not None:
+            g = torch.sigmoid(self.shared_expert_gate(x).float()).to(x.dtype)
+            shared = self.shared_expert(x) * g
+        return self.experts.routed_add_norm(x, weights, ids, shared,
+                                            residual, norm)
+
 
 class MoEDecoderLayer(nn.Module):
     def __init__(self, cfg, engine_config, layer_idx, *, qkv_bias, qk_norm,
@@ -80,9 +92,7 @@ class MoEDecoderLayer(nn.Module):
             positions, hidden, residual, self.post_attention_layernorm, fctx)
         if next_norm is None:
             return self.mlp(hidden), residual
-        if isinstance(self.mlp, DenseMLP):
-            return self.mlp.forward_add_norm(hidden, residual, next_norm)
-        return next_norm(self.mlp(hidden), residual)
+        return self.mlp.forward_add_norm(hidden, residual, next_norm)
 
 
 class MoEFamilyForCausalLM(LlamaFamilyForCausalLM):

@@ -248,7 +248,8 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
               expert_start: int = 0,
               num_global_experts: Optional[int] = None,
               activation: str = "silu_glu",
-              act_args: tuple = ()) -> torch.Tensor:
+              act_args: tuple = (),
+              add_norm: Optional[tuple] = None) -> torch.Tensor:
     """Grouped-GEMM fused MoE on the gfx950 kernels (GPU, bf16).
     ``activation``: "silu_glu" (w13 = gate | up rows), "relu2"
     (ungated experts, w13 = up rows only, act = max(z, 0)^2) or
@@ -260,7 +261,10 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     Fully device-resident and hipGraph-safe (no host syncs; grids are
     sized by upper bound and gated on the device-side block count).
     Returns the PARTIAL output for this rank's expert shard (callers
-    run their TP/EP all-reduce on top).
+    run their TP/EP all-reduce on top). ``add_norm`` = (shared or None,
+    residual, norm weight, eps): the output (+ shared) is added to the
+    residual, in place, and the norm of that is returned (one kernel; see
+    ``moe_add_norm_ok``).
     """
     T, K = x.shape
     E_local, rows13, _ = w13.shape
@@ -310,9 +314,25 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
             act = silu_and_mul(inter1)
         k.moe_gemm(pair_out, act, w2, *tables, tw, n_pairs, topk, block_m,
                    True)
+    if add_norm is not None:
+        return k.moe_sum_norm(pair_out, ids32, expert_start, E_local, topk,
+                              *add_norm)
     out = torch.empty(T, K, dtype=x.dtype, device=dev)
     k.moe_sum(out, pair_out, ids32, expert_start, E_local, topk)
     return out
+
+
+def moe_add_norm_ok(x: torch.Tensor, shared: Optional[torch.Tensor],
+                    residual: torch.Tensor, norm_w: torch.Tensor) -> bool:
+    """Whether ``fused_moe`` takes ``add_norm`` of these."""
+    rows = [residual] + ([] if shared is None else [shared])
+    return (x.is_cuda and x.dim() == 2 and x.shape[1] % 8 == 0
+            and x.shape[1] <= 8192
+            and all(t.dtype == torch.bfloat16 and t.shape == x.shape
+                    and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in rows)
+            and norm_w.dtype in (torch.bfloat16, torch.float32)
+            and norm_w.is_contiguous() and norm_w.data_ptr() % 16 == 0)
 
 
 def _moe_tables(topk_ids: torch.Tensor, E_local: int, expert_start: int,

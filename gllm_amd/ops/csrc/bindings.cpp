@@ -95,6 +95,11 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
                     c10::optional<torch::Tensor> topk_weights, long n_pairs,
                     long topk, long block_m, long act, double limit,
                     double alpha);
+torch::Tensor moe_sum_norm(torch::Tensor pair_out, torch::Tensor ids,
+                           long expert_start, long E_local, long topk,
+                           c10::optional<torch::Tensor> shared,
+                           torch::Tensor residual, torch::Tensor norm_w,
+                           double eps);
 void moe_sum(torch::Tensor out, torch::Tensor pair_out, torch::Tensor ids,
              long expert_start, long E_local, long topk);
 void softmax_topk_rows(torch::Tensor weights, torch::Tensor ids,
@@ -212,6 +217,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "grouped MFMA GEMM of wide tiles, activation in the epilogue");
   m.def("softmax_topk_rows", &softmax_topk_rows,
         "softmax over all experts, then top-k");
+  m.def("moe_sum_norm", &moe_sum_norm,
+        "pair outputs over topk (+ shared), residual and RMS norm");
   m.def("moe_sum", &moe_sum, "sum pair outputs over topk");
   m.def("per_token_group_quant_fp8", &per_token_group_quant_fp8,
         "per (token, 128-group) e4m3 quant + fp32 scales");

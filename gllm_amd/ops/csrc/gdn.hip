@@ -157,9 +157,10 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // 5.3e-7 with fp32 instructions, mean 2.5e-7 against 2.9e-7).
 // 4096 tokens in four prompts, 16 heads of 128: 59 + 127 us (carry 145 with a
 // 64-bit address and a branch for each load, with stores inside the wait for
-// the next chunk's operands, and one sum after the other; 212 + 200 with fp32 instructions throughout and the triangular system solved column strip
-// by column strip; 922 for one kernel that did all of it chunk after chunk on
-// a workgroup per sequence, head and 64 columns). local is bound by its
+// the next chunk's operands, and one sum after the other; 212 + 200 with fp32
+// instructions throughout and the triangular system solved column strip by
+// column strip; 922 for one kernel that did all of it chunk after chunk on a
+// workgroup per sequence, head and 64 columns). local is bound by its
 // stores (X, att: 105 MB); carry by the serial chain of the longest prompt, a
 // chunk's operands arriving (110 KB a workgroup) and two barriers.
 typedef __attribute__((ext_vector_type(4))) float gdn_f4;
