@@ -82,6 +82,8 @@ class MLAAttention(nn.Module):
                 hidden, self.total_heads * self.qk_dim, params_dtype=dtype)
         self.kv_a_proj_with_mqa = ReplicatedLinear(
             hidden, self.kv_lora_rank + self.qk_rope, params_dtype=dtype)
+        if not self.q_lora_rank:
+            self._lay_together()
         self.kv_a_layernorm = RMSNorm(self.kv_lora_rank,
                                       getattr(cfg, "rms_norm_eps", 1e-6))
         self.kv_b_proj = ColumnParallelLinear(
@@ -105,6 +107,30 @@ class MLAAttention(nn.Module):
         self.rotary_emb = get_rope(self.qk_rope, self.qk_rope, max_pos,
                                    getattr(cfg, "rope_theta", 10000.0),
                                    is_neox=True, rope_scaling=rope_scaling)
+
+    def _lay_together(self):
+        """The rows of kv_a_proj's weight behind those of q_proj's."""
+        a, b = self.q_proj.weight, self.kv_a_proj_with_mqa.weight
+        rows = torch.cat([a.data, b.data])
+        a.data, b.data = rows[:a.shape[0]], rows[a.shape[0]:]
+
+    def _queries_and_latents(self, hidden):
+        """q_proj(hidden), kv_a_proj_with_mqa(hidden): one product where
+        the weights still lie together (us, two / one: 4096 rows 48 + 24 /
+        66, 128 rows 29 / 15)."""
+        qp, kp = self.q_proj, self.kv_a_proj_with_mqa
+        a, b = qp.weight, kp.weight
+        if (hidden.is_cuda and qp.is_plain and kp.is_plain
+                and qp.bias is None and kp.bias is None
+                and a.dtype == b.dtype == hidden.dtype
+                and a.is_contiguous() and b.is_contiguous()
+                and a.untyped_storage().data_ptr()
+                == b.untyped_storage().data_ptr()
+                and b.storage_offset() == a.storage_offset() + a.numel()):
+            w = a.as_strided((a.shape[0] + b.shape[0], a.shape[1]),
+                             (a.shape[1], 1))
+            return ops.linear(hidden, w).split([a.shape[0], b.shape[0]], -1)
+        return qp(hidden), kp(hidden)
 
     def _dsa_select(self, positions, hidden, q_resid, fctx):
         """DSA hook (DeepSeek-V3.2): per-query top-k token positions, or
@@ -133,10 +159,10 @@ class MLAAttention(nn.Module):
         if self.q_lora_rank:
             q_resid = self.q_a_layernorm(self.q_a_proj(hidden))
             q = self.q_b_proj(q_resid)
+            kv_a = self.kv_a_proj_with_mqa(hidden)
         else:
             q_resid = None
-            q = self.q_proj(hidden)
-        kv_a = self.kv_a_proj_with_mqa(hidden)
+            q, kv_a = self._queries_and_latents(hidden)
         if self.absorbed and not fctx.is_profile_run:
             cos_sin = self.rotary_emb.cos_sin_cache
             k_cache = fctx.k_caches[self.layer_idx]
