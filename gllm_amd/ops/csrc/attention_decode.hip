@@ -5,12 +5,14 @@
 //   grid = B * Hkv * splits, block = 256 threads (4 waves). A workgroup
 //   serves the whole GQA group (up to 16 query heads) of one kv head over
 //   a share of the keys, so K/V bytes are read once for all its heads.
-//   Up to two rounds of workgroups, heads are the fastest index (the eight
-//   dies take workgroups in turn, so with 8 heads each die gets a share of
-//   every sequence), then splits, and sequences come longest first
-//   (sequence_at), so what starts last is short. More rounds even out by
-//   themselves, and finding the sequence costs each workgroup about 1 us:
-//   there sequences are the fastest index, as they come. (us, 512 to 1536
+//   From 257 workgroups to two rounds of them, if a sequence has more than
+//   1024 keys, heads are the fastest index (the eight dies take workgroups in
+//   turn, so with 8 heads each die gets a share of every sequence), then
+//   splits, and sequences come longest first (sequence_at), so what starts
+//   last is short. More rounds even out by themselves, a workgroup per CU
+//   starts at once in any order, and finding the sequence costs each
+//   workgroup 1 to 3 us, more than short sequences give back: there sequences
+//   are the fastest index, as they come. (us, 512 to 1536
 //   keys unless said, sequences fastest / this: 64 sequences 69 / 58, 128 of
 //   1024 to 3072 keys 203 / 188, 24 of 2700 to 8100 in four splits 123 / 105,
 //   37 in two 40 / 38; 256 sequences 189 / 188 and 10 more in a step; heads
@@ -55,13 +57,14 @@ union DecFrag {
 };
 
 constexpr int ORDERED = 1024;  // workgroups at most: two rounds
+constexpr int ALONE = 256;     // a CU each: all start at once, in any order
+constexpr int SHORT = 1024;    // keys: below, order gives less than it takes
 
 // The sequence whose visible keys come `rank`th, the most first, to within a
 // sixteenth of the most (equal ones by number); every wave finds it by
 // itself. B <= ORDERED.
 DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
                            const int *qsl) {
-  if (B == 1) return rank;
   const int lane = threadIdx.x & 63;
   constexpr int PER = ORDERED / 64;
   int keys[PER], most = 1;
@@ -127,21 +130,25 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
   constexpr int VROW = DV * 2;             // LDS row bytes
   constexpr int VMASK = (DV / 8 - 1) & 15;
-  int b, kvh, split;  // (zdim: splits, and the kept-first segment)
-  if (gridDim.x <= ORDERED) {
-    const int rest = blockIdx.x / num_kv_heads;
-    kvh = blockIdx.x - rest * num_kv_heads;
-    split = rest % zdim;
-    b = __builtin_amdgcn_readfirstlane(
-        sequence_at(rest / zdim, B, seq_lens, window, qsl));
-  } else {
-    const int rest = blockIdx.x / B;
-    b = blockIdx.x - rest * B;
-    kvh = rest % num_kv_heads;
-    split = rest / num_kv_heads;
+  // (zdim: splits, and the kept-first segment)
+  const int rest = blockIdx.x / B;
+  int b = blockIdx.x - rest * B, kvh = rest % num_kv_heads;
+  int split = rest / num_kv_heads;
+  int seq_len = seq_lens[b];
+  if (B > 1 && gridDim.x > ALONE && gridDim.x <= ORDERED) {
+    bool order = false;
+    for (int i = threadIdx.x & 63; i < B; i += 64)
+      order |= seq_lens[i] > SHORT;
+    if (__any(order)) {
+      const int of_heads = blockIdx.x / num_kv_heads;
+      kvh = blockIdx.x - of_heads * num_kv_heads;
+      split = of_heads % zdim;
+      b = __builtin_amdgcn_readfirstlane(
+          sequence_at(of_heads / zdim, B, seq_lens, window, qsl));
+      seq_len = seq_lens[b];
+    }
   }
   const int Hq = num_kv_heads * G;
-  const int seq_len = seq_lens[b];
   const int row = qsl ? qsl[b] : b;  // of q and of the result
   if (qsl && qsl[b + 1] - row != 1) return;
   const int w_begin = (window > 0) ? max(0, seq_len - window) : 0;
