@@ -44,7 +44,7 @@ constexpr int WAVES = 4, BLOCK = 64 * WAVES;
 constexpr int RG = 2;                // groups of 16 rows per wave
 constexpr int BQ = 16 * RG * WAVES;  // rows of a workgroup
 constexpr int BKV = 64, NF = BKV / 16;
-constexpr int LISTED = 256;          // sequences whose tiles are counted
+constexpr int LISTED = 256;          // sequences of a launch at most
 constexpr float LOG2E = 1.4426950408889634f;
 
 struct Args {
@@ -58,7 +58,7 @@ struct Args {
   long max_pages;
   int page_size;
   const int *seq_lens, *qsl;
-  int B, Hq, Hkv, q_tiles, min_rows;
+  int B, Hq, Hkv, min_rows;
   float scale;  // times log2 e
 };
 
@@ -80,12 +80,6 @@ DEV_INLINE int swz(int row, int off) {
 // The `rank`th tile of 128 rows, last tiles of the longest sequences first;
 // every wave finds it by itself. False past the end.
 DEV_INLINE bool tile_at(int rank, const Args &P, int &b, int &tile) {
-  if (P.B > LISTED) {
-    b = rank % P.B;
-    tile = P.q_tiles - 1 - rank / P.B;
-    const int n = P.qsl[b + 1] - P.qsl[b];
-    return tile >= 0 && tile * BQ < n && n >= P.min_rows;
-  }
   const int lane = threadIdx.x & 63;
   constexpr int PER = LISTED / 64;
   int n[PER], most = 0;
@@ -398,15 +392,23 @@ __global__ __launch_bounds__(BLOCK, 2) void causal_kernel(const Args P) {
 }
 
 template <int D, int DV, bool PAGED>
-void launch(Args &P, long T, long max_query_len) {
-  P.q_tiles = (max_query_len + BQ - 1) / BQ;
-  // tiles at most (B > LISTED: tiles of every sequence)
-  long ranks = (long)P.q_tiles * P.B;
-  if (P.B <= LISTED) ranks = std::min(ranks, T / BQ + P.B);
-  if (ranks <= 0) return;
-  hipLaunchKernelGGL((causal_kernel<D, DV, PAGED>), dim3(ranks * P.Hq),
-                     dim3(BLOCK), 0, at::cuda::getCurrentCUDAStream(), P);
-  HIP_CHECK_KERNEL();
+void launch(Args P, long T, long max_query_len) {
+  const long q_tiles = (max_query_len + BQ - 1) / BQ;
+  auto stream = at::cuda::getCurrentCUDAStream();
+  for (int left = P.B; left > 0; left -= LISTED) {
+    P.B = std::min(left, LISTED);
+    // tiles at most
+    const long ranks = std::min(q_tiles * P.B, T / BQ + P.B);
+    if (ranks <= 0) return;
+    hipLaunchKernelGGL((causal_kernel<D, DV, PAGED>), dim3(ranks * P.Hq),
+                       dim3(BLOCK), 0, stream, P);
+    HIP_CHECK_KERNEL();
+    P.qsl += P.B;
+    if (PAGED) {
+      P.seq_lens += P.B;
+      P.block_table += P.B * P.max_pages;
+    }
+  }
 }
 
 }  // namespace

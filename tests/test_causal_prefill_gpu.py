@@ -30,8 +30,8 @@ def _check(out, ref):
     ([63, 64, 65, 31, 33], [0, 0, 0, 0, 0], 5, 1, 64, 16),
     ([300, 2, 16], [1, 64, 500], 16, 2, 128, 16),   # cached prefixes
     ([1, 1, 200], [700, 0, 0], 10, 2, 128, 48),     # rows that decode
-    ([3] * 256, [0] * 256, 2, 1, 64, 16),           # sequences counted
-    ([3] * 256 + [140], [5] * 257, 2, 1, 64, 1),    # not counted
+    ([3] * 256, [0] * 256, 2, 1, 64, 16),           # one launch
+    ([3] * 256 + [140], [5] * 257, 2, 1, 64, 1),    # two
     ([1100], [0], 3, 3, 128, 16),
 ])
 @pytest.mark.parametrize("single", [False, True])
