@@ -43,7 +43,8 @@ __global__ void rmsnorm_kernel(T *__restrict__ out, const T *__restrict__ in,
 
 // Rows of at most 8 L values (heads): L lanes each, the row in registers. A
 // workgroup per row leaves most of its lanes idle (65536 rows of 128 42 us,
-// this 7.7; 8192 rows 7.1 and 4.0; 4096 of 512 5.7 and 4.4). Sums in the order of the kernel above.
+// this 7.7; 8192 rows 7.1 and 4.0; 4096 of 512 5.7 and 4.4). Sums in the
+// order of the kernel above.
 template <typename T, typename TW, int L>
 __global__ __launch_bounds__(256) void rmsnorm_short_kernel(
     T *__restrict__ out, const T *__restrict__ in,
