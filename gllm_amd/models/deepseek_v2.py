@@ -229,12 +229,13 @@ class MLAAttention(nn.Module):
                       fctx):
         """``heads`` of a batch whose sequences from ``first`` on are whole
         prompts: those per head, what comes before them absorbed."""
-        qsl = fctx.host_qsl()
-        row, end = qsl[first], qsl[fctx.seq_lens.shape[0]]
+        n = fctx.seq_lens.shape[0]  # (a buffer of offsets may be longer)
+        qsl, starts = fctx.host_qsl()[:n + 1], fctx.query_start_loc[:n + 1]
+        row, end = qsl[first], qsl[n]
         w_kvb, norm = self.kv_b_proj.weight, self.kv_a_layernorm
         cos_sin = self.rotary_emb.cos_sin_cache
         k_cache = fctx.k_caches[self.layer_idx]
-        slots, starts = fctx.slot_mapping, fctx.query_start_loc
+        slots = fctx.slot_mapping
         out = q.new_empty(q.shape[0], self.num_heads * self.v_dim)
         if row > 0:
             qf = ops.mla_queries(q[:row], kv_a[:row], norm.weight, norm.eps,
