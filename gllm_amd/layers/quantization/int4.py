@@ -297,6 +297,13 @@ def convert_model_to_int4(model, quant_config: dict) -> int:
         if name.rsplit(".", 1)[-1] in _QUANT_SUFFIXES:
             convert_linear_to_int4(mod, method, group)
             n += 1
+    # a dense weight that lay together with a converted one would keep that
+    # one's rows in memory
+    for mod in model.modules():
+        if isinstance(mod, LinearBase) and mod.is_plain:
+            w = mod.weight
+            if w.untyped_storage().nbytes() > w.numel() * w.element_size():
+                w.data = w.data.clone()
     return n
 
 

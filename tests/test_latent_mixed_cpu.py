@@ -66,3 +66,19 @@ def test_longer_offsets(monkeypatch, extra):
                     "rows": (17, 17, tail, tail, 17),
                     "front": ([6, 8], [0, 1, 2], [6, 8], [0, 1, 2], 2)}
     assert (out[:2] == 1).all() and (out[2:] == 2).all()
+
+
+def test_converted_rows_are_freed():
+    """q_proj's dense rows go with its conversion although kv_a_proj's, which
+    stay, were laid behind them."""
+    from gllm_amd.layers.quantization.int4 import convert_model_to_int4
+    for quantized in (False, True):
+        layer = _layer()
+        if quantized:
+            convert_model_to_int4(torch.nn.ModuleDict({"attn": layer}),
+                                  {"quant_method": "gptq", "group_size": 64})
+        w = layer.kv_a_proj_with_mqa.weight
+        assert w.shape == (576, 64)
+        own = w.numel() * w.element_size()
+        assert w.untyped_storage().nbytes() == (
+            own if quantized else own + 192 * 64 * 4)
