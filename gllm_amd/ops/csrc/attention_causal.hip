@@ -9,14 +9,15 @@
 // Bound by the vector instructions of the softmax and the LDS reads of K and
 // V, about level with each other and with the products (1100, 1000 and 1000
 // clocks of a tile's 64 keys x 128 rows, two workgroups per CU), so:
-//  * a weight is one multiply-add, one exponential and half a conversion; the
-//    masked tiles are a branch of their own (as selects the mask and the cap
-//    that the general kernel can carry made 60 % of its instructions);
-//  * the weights' sum is a product with ones, of the weights as they are
-//    rounded: a large weight's rounding cancels (error against 64 bits, 1000
-//    normal rows: 0.00198, 0.00200 with the sum of fp32 weights). Counting
-//    weights from a maximum that may lag behind by 2^8 would save 3 % and
-//    cost precision, since then the largest weight is rounded too (0.00203);
+//  * a weight is one multiply-add, one exponential, one addition and half a
+//    conversion; the masked tiles are a branch of their own (as selects the
+//    mask and the cap that the general kernel can carry made 60 % of its
+//    instructions);
+//  * the weights' sum is that of the fp32 weights, a lane's four at a time (a
+//    product of the rounded weights with ones is 0 to 2.5 % faster, 4096 rows
+//    209.6 for 212.6 us, but drops 16 bits of each). Counting weights from a
+//    maximum that may lag behind by 2^8 would save 3 % and round the largest
+//    weight too (error against 64 bits 0.00203 for 0.00200);
 //  * the row maximum joins lane groups by swapping lanes, not through LDS;
 //  * heavy tiles start first: workgroups are numbered by tile from the last
 //    one on, only over tiles that exist, heads fastest with the heads of a kv
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(BLOCK, 2) void causal_kernel(const Args P) {
   const bool busy = row0 < q_len;
   ca_bf8 qf[RG][KT];
   float m_run[RG];
-  ca_f4 l_run[RG];  // (four times the same number)
+  ca_f4 l_run[RG];  // of this lane's keys; lanes join at the end
   ca_f4 o_acc[RG][NT];
 #pragma unroll
   for (int g = 0; g < RG; ++g) {
@@ -258,9 +259,6 @@ __global__ __launch_bounds__(BLOCK, 2) void causal_kernel(const Args P) {
 
   const int tr_row = lhi * 4 + (l16 >> 2), tr_col = (l16 & 3) * 8;
   const float scale = P.scale;
-  CaFrag ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones.e[i] = __float2bfloat16(1.f);
   for (int it = 0; it < nkt; ++it) {
     const int kv0 = it * BKV;
     // every wave's loads of this tile have landed; and every wave is done
@@ -339,20 +337,18 @@ __global__ __launch_bounds__(BLOCK, 2) void causal_kernel(const Args P) {
 #pragma unroll
       for (int f = 0; f < NF; ++f)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          pf[g][f >> 1].e[(f & 1) * 4 + r] = __float2bfloat16(
-              __builtin_amdgcn_exp2f(__builtin_fmaf(s[g][f][r], scale,
-                                                    -base)));
+        for (int r = 0; r < 4; ++r) {
+          const float p = __builtin_amdgcn_exp2f(
+              __builtin_fmaf(s[g][f][r], scale, -base));
+          l_run[g][r] += p;
+          pf[g][f >> 1].e[(f & 1) * 4 + r] = __float2bfloat16(p);
+        }
     }
 
     // ---------- O^T += V^T P^T ----------
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int ks = 0; ks < BKV / 32; ++ks) {
-#pragma unroll
-      for (int g = 0; g < RG; ++g)
-        l_run[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            ones.v, pf[g][ks].v, l_run[g], 0, 0, 0);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         CaFrag vf;
@@ -374,7 +370,9 @@ __global__ __launch_bounds__(BLOCK, 2) void causal_kernel(const Args P) {
   // ---------- lane = one query, 4 columns of each column tile ----------
 #pragma unroll
   for (int g = 0; g < RG; ++g) {
-    const float l = l_run[g][0];
+    float l = (l_run[g][0] + l_run[g][1]) + (l_run[g][2] + l_run[g][3]);
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
     const int qrow = row0 + g * 16 + l16;
     if (qrow >= q_len) continue;
     const float inv_l = l > 0.f ? 1.f / l : 0.f;

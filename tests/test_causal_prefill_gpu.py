@@ -81,3 +81,29 @@ def test_scores_far_apart():
     out = ops.paged_attention(q.cuda(), k.cuda(), v.cuda(), table, qsl[1:],
                               qsl, 0.5, n)
     _check(out.view(ref.shape), ref)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_weights_are_summed_in_32_bits(D):
+    """One key of weight 1 and value 1, the others of one weight w a row and
+    value 0: the result is 1 / (1 + n w), off by its own rounding only."""
+    from gllm_amd import ops
+    rows, past = 500, 300
+    n = rows + past
+    k = torch.zeros(n // 16, 16, 1, D)
+    k[0, 0, 0, 0] = 1.0
+    v = torch.zeros_like(k)
+    v[0, 0] = 1.0
+    q = torch.zeros(rows, 1, D)
+    q[:, 0, 0] = torch.linspace(0.5, 6, rows)
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    ref = _attend(q.double(), k.view(n, 1, D).double(),
+                  v.view(n, 1, D).double(), 1.0)
+    table = torch.arange(n // 16, dtype=torch.int32)[None].cuda()
+    out = ops.paged_attention(
+        q.cuda(), k.cuda(), v.cuda(), table,
+        torch.tensor([n], dtype=torch.int32).cuda(),
+        torch.tensor([0, rows], dtype=torch.int32).cuda(), 1.0, rows)
+    err = (out.view(ref.shape).cpu().double() / ref - 1).abs().max()
+    # half a step of the 8 bits of a bf16; rounded weights add as much again
+    assert err < 2 ** -8 * 1.01, err
