@@ -285,10 +285,6 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
         # experts (csrc/moe_tiled.hip has times on both sides of each line)
         block_m = (32 if rpe <= 12 else 64 if rpe <= 40
                    else 128 if rpe <= 128 else 256)
-        if block_m == 256 and max(
-                T * K, (n_pairs + E_local * 255 + 256) * inter, n_pairs * K,
-                rows13 * K, K * inter) >= 1 << 30:
-            block_m = 128  # (256-row blocks take operands below 2 GiB)
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
                                           block_m)
         act = torch.empty(rows, inter, dtype=x.dtype, device=dev)

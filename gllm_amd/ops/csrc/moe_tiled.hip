@@ -26,7 +26,10 @@
 //    have more, 64 rows take 2732 us for a step of four layers, 32 rows
 //    2875 us; at 24 the two are within 3 %, at 32 64 rows take 299 + 184 us
 //    against 375 + 230 us.
-//  * many rows: the matrix cores. Blocks of 256 rows go to tile_gemm.hip.
+//  * many rows: the matrix cores. Blocks of 256 rows go to tile_gemm.hip,
+//    which takes operands below 2 GiB (8 experts of 4096 x 14336, 10000 rows:
+//    1910 + 990 us); for larger ones 256 x 256 tiles on eight waves of 128 x
+//    64, one workgroup each (2226 + 1177 us).
 //  * between (40 to 128 rows per expert): 128 x 128 tiles on four waves;
 //    64 rows per expert 375 + 192 us against 442 + 251 us (64 x 128) and
 //    475 + 379 us (256 x 256); 192 rows 287 + 182 us against 226 + 163 us
@@ -90,7 +93,7 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
   if (pid >= total) return;
   const int xcd = pid & 7, per = total >> 3;
   const int t = xcd * per + min(xcd, total & 7) + (pid >> 3);
-  constexpr int GM = 8;  // row blocks of a group
+  constexpr int GM = BM >= 256 ? 4 : 8;  // row blocks of a group
   const int grp = t / (GM * nbn), in_g = t - grp * GM * nbn;
   const int gm = min(GM, nblk - grp * GM);
   const int mb = grp * GM + in_g % gm, nb = in_g / gm;
@@ -284,7 +287,8 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
                 topk_weights->numel() >= n_pairs);
     tw = topk_weights->data_ptr<float>();
   }
-  if (block_m == 256) {
+  if (block_m == 256 &&
+      tile_gemm_grouped_ok(A.numel(), n_pairs, Nd, K, (int)act)) {
     tile_gemm_grouped(C.data_ptr(), A.data_ptr(), W.data_ptr(),
                       sorted_ids.data_ptr<int>(),
                       expert_blocks.data_ptr<int>(),
@@ -316,6 +320,7 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
   if (block_m == 32) FORMS(32, 128, 1, 4, 4, 2);
   else if (block_m == 64) FORMS(64, 128, 1, 4, 3, 2);
   else if (block_m == 128) FORMS(128, 128, 2, 2, 3, 0);
+  else if (block_m == 256) FORMS(256, 256, 2, 4, 2, 0);
   else TORCH_CHECK(false, "moe_gemm_tiled: block_m must be 32/64/128/256");
 #undef FORMS
 #undef RUN

@@ -2,6 +2,8 @@
 // moe_gemm_tiled; split products of few rows, called by stream_parts.
 #pragma once
 
+bool tile_gemm_grouped_ok(long a_numel, long n_pairs, long Nd, long K,
+                          int act);
 void tile_gemm_grouped(void *C, const void *A, const void *W,
                        const int *sorted_ids, const int *expert_blocks,
                        const int *n_post_pad, const float *topk_w,

@@ -867,8 +867,16 @@ void tile_parts(float *part, const void *x, const void *w, long M, long N,
   HIP_CHECK_KERNEL();
 }
 
+// Offsets into A, into an expert's weights and, for scatter, into C are 32
+// bits.
+bool tile_gemm_grouped_ok(long a_numel, long n_pairs, long Nd, long K,
+                          int act) {
+  return a_numel < (1L << 30) && Nd * K < (1L << 30) &&
+         (act != NONE || n_pairs * Nd < (1L << 30));
+}
+
 // The grouped forms over blocks of 256 rows (operands checked by
-// moe_gemm_tiled; act as there).
+// moe_gemm_tiled, sizes by tile_gemm_grouped_ok; act as there).
 void tile_gemm_grouped(void *C, const void *A, const void *W,
                        const int *sorted_ids, const int *expert_blocks,
                        const int *n_post_pad, const float *topk_w,
@@ -876,9 +884,6 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
                        long K, long a_rows, int act, float limit,
                        float alpha) {
   const bool gated = act == SILU || act == CLAMP;
-  TORCH_CHECK(a_rows * K < (1L << 30) && Nd * K < (1L << 30) &&
-                  (act != NONE || n_pairs * Nd < (1L << 30)),
-              "moe_gemm_tiled: 256-row blocks take operands below 2 GiB");
   Args P{};
   P.C = (__hip_bfloat16 *)C;
   P.A = (const __hip_bfloat16 *)A;
@@ -903,8 +908,8 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
   const dim3 grid(
       std::min<long>((max_blocks * P.nbn + 7) / 8 * 8, compute_units()));
 #define RUN(FORM, ACT)                                                       \
-  hipLaunchKernelGGL((tile_gemm_kernel<FORM, ACT, true, false>), grid, dim3(256),   \
-                     0, stream, P)
+  hipLaunchKernelGGL((tile_gemm_kernel<FORM, ACT, true, false>), grid,       \
+                     dim3(256), 0, stream, P)
   if (act == NONE) RUN(SCATTER, NONE);
   else if (act == SILU) RUN(GATED, SILU);
   else if (act == CLAMP) RUN(GATED, CLAMP);
