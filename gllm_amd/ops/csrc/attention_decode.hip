@@ -5,18 +5,22 @@
 //   grid = B * Hkv * splits, block = 256 threads (4 waves). A workgroup
 //   serves the whole GQA group (up to 16 query heads) of one kv head over
 //   a share of the keys, so K/V bytes are read once for all its heads.
-//   From 257 workgroups to two rounds of them, if a sequence has more than
-//   1024 keys, heads are the fastest index (the eight dies take workgroups in
-//   turn, so with 8 heads each die gets a share of every sequence), then
-//   splits, and sequences come longest first (sequence_at), so what starts
-//   last is short. More rounds even out by themselves, a workgroup per CU
-//   starts at once in any order, and finding the sequence costs each
-//   workgroup 1 to 3 us, more than short sequences give back: there sequences
-//   are the fastest index, as they come. (us, 512 to 1536
-//   keys unless said, sequences fastest / this: 64 sequences 69 / 58, 128 of
-//   1024 to 3072 keys 203 / 188, 24 of 2700 to 8100 in four splits 123 / 105,
-//   37 in two 40 / 38; 256 sequences 189 / 188 and 10 more in a step; heads
-//   fastest alone 62, 219, 120, 44, 206.)
+//   From 257 workgroups to two rounds of them, if a sequence gives each of
+//   its workgroups more than 1024 keys of 128 + 128 values and lengths differ,
+//   heads are the fastest index (the eight dies take workgroups in turn, so
+//   with 8 heads each die gets a share of every sequence), then splits, and
+//   sequences come longest first (sequence_at), so what starts last is short.
+//   More rounds even out by themselves, and a workgroup per CU starts at once
+//   in any order. Finding the sequence costs each workgroup 1 to 3 us, more
+//   than short shares give back, and heads fastest is the slower one for equal
+//   lengths: there sequences are the fastest index, as they come. (us, 32
+//   heads on 8 of 128, sequences fastest / this: 64 sequences of 512 to 1536
+//   keys 68 / 61, 128 of 1024 to 3072 218 / 197, 24 of 2700 to 8100 in four
+//   splits 138 / 124, 100 of 1 to 4000 179 / 153. Where it is not done, as
+//   they come / in order: 128 of 2048 179 / 193, 33 of 1100 in two splits 39 /
+//   46, 100 of 700 to 1000 71 / 78; one head, 33 of 10 to 1100 in sixteen
+//   splits 18.5 / 25.4; 14 heads on 2 of 64, 64 of 512 to 1536 14.5 / 17.2,
+//   400 of 100 to 1500 39 / 42; 64 of 1600 to 2048 would gain, 96 / 91.)
 //   Its waves work on their own: wave w takes the 32-key tiles w, w + 4,
 //   ... of the share, with a softmax state of its own and no barrier in the
 //   loop; the next tile's K and V are in registers while this one is
@@ -58,10 +62,12 @@ union DecFrag {
 
 constexpr int ORDERED = 1024;  // workgroups at most: two rounds
 constexpr int ALONE = 256;     // a CU each: all start at once, in any order
-constexpr int SHORT = 1024;    // keys: below, order gives less than it takes
+constexpr int SHARE = 1024 * 256;  // values of K and V a workgroup: up to
+                                   // here, order gives less than it takes
 
 // The sequence whose visible keys come `rank`th, the most first, to within a
-// sixteenth of the most (equal ones by number); every wave finds it by
+// sixteenth of the most (equal ones by number); -1 if half of them have more
+// than seven eighths of the most: too alike to gain. Every wave finds it by
 // itself. B <= ORDERED.
 DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
                            const int *qsl) {
@@ -82,6 +88,13 @@ DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     most = max(most, __shfl_xor(most, off, 64));
+  int alike = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    if (i * 64 >= B) break;
+    alike += __popcll(__ballot(keys[i] > most - (most >> 3)));
+  }
+  if (2 * alike >= B) return -1;
   const float unit = 15.999f / most;
 #pragma unroll
   for (int i = 0; i < PER; ++i)
@@ -125,7 +138,9 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     // one split: the result itself, bf16 [rows, Hq * Dvr]
     __hip_bfloat16 *__restrict__ out, long out_stride, int sink,
     const float *__restrict__ sinks, const __hip_bfloat16 *__restrict__ gate,
-    long gate_stride, int B, int zdim) {
+    long gate_stride, int B, int zdim,
+    // keys from which on the order of sequences matters
+    int order_above) {
   constexpr int KT = D / 32, NT = DV / 16;
   constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
   constexpr int VROW = DV * 2;             // LDS row bytes
@@ -137,15 +152,24 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   int seq_len = seq_lens[b];
   if (B > 1 && gridDim.x > ALONE && gridDim.x <= ORDERED) {
     bool order = false;
-    for (int i = threadIdx.x & 63; i < B; i += 64)
-      order |= seq_lens[i] > SHORT;
+    if (window <= 0 || window > order_above)
+      for (int i = threadIdx.x & 63; i < B; i += 256) {  // loads in fours
+        int n = seq_lens[i];
+#pragma unroll
+        for (int j = 1; j < 4; ++j)
+          n = max(n, seq_lens[min(i + j * 64, B - 1)]);
+        order |= n > order_above;
+      }
     if (__any(order)) {
       const int of_heads = blockIdx.x / num_kv_heads;
-      kvh = blockIdx.x - of_heads * num_kv_heads;
-      split = of_heads % zdim;
-      b = __builtin_amdgcn_readfirstlane(
+      const int s = __builtin_amdgcn_readfirstlane(
           sequence_at(of_heads / zdim, B, seq_lens, window, qsl));
-      seq_len = seq_lens[b];
+      if (s >= 0) {
+        b = s;
+        kvh = blockIdx.x - of_heads * num_kv_heads;
+        split = of_heads % zdim;
+        seq_len = seq_lens[b];
+      }
     }
   }
   const int Hq = num_kv_heads * G;
@@ -491,7 +515,7 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      keep_first, softcap, bias, bias_len, temp_coef,         \
                      temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
                      sinks, (const __hip_bfloat16 *)gate, gate_stride, B,    \
-                     zdim)
+                     zdim, SHARE / (D + Dv) * splits)
   if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
 #undef RUN
