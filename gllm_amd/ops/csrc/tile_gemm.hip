@@ -814,22 +814,30 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w,
 // Against the stream (stream / this): 256 x 5120 x 27648 113 / 81, 256 x 7168
 // x 5120 48 / 42, 256 x 5120 x 5120 45 / 36, 160 x 6144 x 4096 37 / 31, 96 x
 // 5120 x 5120 31 / 28, 128 x 4096 x 14336 44 / 39; below 24 M weights its
-// short parts lose (256 x 4096 x 4096 28 / 28, 256 x 6144 x 2048 25 / 27).
-// Up to 64 rows only long streams gain: 64 x 5120 x 27648 73 / 63, 40 x 10240
-// x 8192 42 / 38, but 64 x 4096 x 14336 37 / 37, 64 x 7168 x 5120 28 / 31.
+// short parts lose (256 x 4096 x 4096 28 / 28, 256 x 6144 x 2048 25 / 27), up
+// to 128 rows those of K below 4608 (128 x 6144 x 4096 27.7 / 29.6, 96 x 7680
+// x 3840 28 / 31, 128 x 8192 x 3584 25 / 31). Up to 64 rows only long streams
+// gain: 64 x 5120 x 27648 73 / 63, 40 x 10240 x 8192 42 / 38, but 64 x 4096 x
+// 14336 37 / 37, 64 x 7168 x 5120 28 / 31. Few columns leave CUs idle with 16
+// parts, the most (256 x 1024 x 28672 38 / 52, 160 x 2048 x 16384 28 / 35): it
+// takes 160 workgroups for a block of rows (256 x 2560 x 12800 51 / 37), 200
+// for half a one (96 x 3072 x 12288 with 192 29.6 / 31.9, 96 x 3584 x 8192
+// with 224 27.6 / 26.4).
 void tile_parts_plan(long M, long N, long K, int *bm, int *splits) {
   *splits = 0;
   *bm = M > 128 ? 256 : 128;
   const long weights = N * K, nbn = (N + 255) / 256;
   const int cus = compute_units(), nkt = K / BK;
   if (M <= 32 || M > 256 || nbn > cus || N > (1 << 20) || K > (1 << 21) ||
-      weights < (M > 64 ? 24L << 20 : 72L << 20) || (M <= 64 && K < 8192))
+      weights < (M > 64 ? 24L : 72L) << 20 ||
+      K < (M > 128 ? 0 : M > 64 ? 4608 : 8192))
     return;
   auto most = [&](int blocks) {
     return (int)std::min<long>(std::min<long>(cus / (nbn * blocks), nkt / 4),
                                16);
   };
   int s = most(1);
+  if (nbn * s * 32 < cus * (M > 128 ? 20 : 25)) return;
   if (M > 128 && 5 * s * M > K && most(2) > 0) {
     *bm = 128;
     s = most(2);

@@ -110,3 +110,29 @@ def test_few_rows(M, N, K, gated):
         bound = 2 ** -23 * K ** 0.5  # fp32 sums: a rounding per 32 columns
     err = (out - y).abs() / y.abs().clamp_min(y.square().mean().sqrt())
     assert err.max() < bound, err.max()
+
+
+@pytest.mark.parametrize("M,N,K,stream", [
+    (256, 1024, 28736, True), (160, 2048, 16448, True),  # CUs would idle
+    (256, 2560, 12864, False),
+    (96, 3072, 12352, True), (96, 3584, 8256, False),
+    (128, 6144, 4096, True), (128, 8192, 3584, True),    # short parts
+    (128, 5120, 5120, False), (136, 6144, 4096, False),
+])
+def test_lines_of_parts(M, N, K, stream):
+    """Sizes whose parts come from the stream kernel: as many as for rows
+    that are apart in memory, which only that kernel takes."""
+    from gllm_amd import ops
+    k = ops._gpu_kernels()
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K + 8, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    apart, part = k.stream_parts(x, w), k.stream_parts(x.contiguous(), w)
+    if stream:
+        assert torch.equal(apart, part)
+    else:
+        assert apart.shape != part.shape or not torch.equal(apart, part)
+    y = x.double() @ w.double().t()
+    err = (part.double().sum(0) - y).abs() / y.abs().clamp_min(
+        y.square().mean().sqrt())
+    assert err.max() < 2 ** -23 * K ** 0.5  # fp32 sums
