@@ -32,6 +32,8 @@ def _check(out, ref):
     ([1, 1, 200], [700, 0, 0], 10, 2, 128, 48),     # rows that decode
     ([3] * 256, [0] * 256, 2, 1, 64, 16),           # one launch
     ([3] * 256 + [140], [5] * 257, 2, 1, 64, 1),    # two
+    ([5] * 300 + [1] * 5, [2] * 305, 2, 1, 64, 16),  # a tile each, one launch
+    ([128, 1, 127, 1], [0, 9, 70, 0], 4, 2, 128, 16),
     ([1100], [0], 3, 3, 128, 16),
 ])
 @pytest.mark.parametrize("single", [False, True])
