@@ -951,7 +951,10 @@ def linear(x: torch.Tensor, w: torch.Tensor,
         return skinny_gemm(x, w, bias)
     if (_rows_ok(x, w) and plain_bias(bias, w.shape[0])
             and (bias is None or bias.data_ptr() % 16 == 0)
-            and _use_tile(x.shape[0], w.shape[0], w.shape[1])):
+            and _use_tile(x.shape[0], w.shape[0], w.shape[1])
+            and not (torch.is_grad_enabled()  # (the library's has one)
+                     and any(t is not None and t.requires_grad
+                             for t in (x, w, bias)))):
         return _gpu_kernels().tile_gemm(x, w, bias, False)
     return F.linear(x, w, bias)
 

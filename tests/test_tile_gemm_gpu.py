@@ -136,3 +136,23 @@ def test_lines_of_parts(M, N, K, stream):
     err = (part.double().sum(0) - y).abs() / y.abs().clamp_min(
         y.square().mean().sqrt())
     assert err.max() < 2 ** -23 * K ** 0.5  # fp32 sums
+
+
+def test_long_contractions_have_gradients():
+    from gllm_amd import ops
+    torch.manual_seed(0)
+    M, N, K = 4096, 1024, 17408
+    assert ops._use_tile(M, N, K)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    g = torch.randn(M, N, device="cuda").bfloat16()
+    for operand in (x, w):
+        operand.requires_grad_()
+        out = ops.linear(x, w)
+        ref = torch.nn.functional.linear(x, w)
+        got, want = (torch.autograd.grad(o, operand, g)[0]
+                     for o in (out, ref))
+        assert torch.equal(got, want)
+        with torch.no_grad():
+            assert not ops.linear(x, w).requires_grad
+        operand.requires_grad_(False)
