@@ -12,6 +12,7 @@ through here. Dispatch rule:
   which double as the numerics oracle for the HIP kernels.
 """
 
+import functools
 from typing import Optional
 
 import torch
@@ -903,11 +904,12 @@ def _use_skinny(M: int, N: int, K: int) -> bool:
     (96 x 28672 x 4096 57.6 / 55.6, 256 x 38016 x 5120 139 / 109) and
     worse on the rest (256 x 7168 x 5120 40 / 54, 256 x 5120 x 27648 110 /
     266)."""
+    if K % 64 != 0 or N < 512 or M > SKINNY_MAX_M or M == 0:
+        return False
     import os
     if os.environ.get("GLLM_DISABLE_SKINNY"):
         return False
-    max_m = int(os.environ.get("GLLM_SKINNY_MAX_M", "0")) or SKINNY_MAX_M
-    if K % 64 != 0 or N < 512 or M > max_m or M == 0:
+    if M > (int(os.environ.get("GLLM_SKINNY_MAX_M", "0")) or SKINNY_MAX_M):
         return False
     return M <= 64 or N < 16384
 
@@ -926,16 +928,34 @@ def _tile_fits(M: int, N: int, K: int, gated: bool) -> bool:
             and (not gated or N * K < 1 << 30))
 
 
+@functools.lru_cache(maxsize=None)
+def _compute_units() -> int:
+    return torch.cuda.get_device_properties(
+        torch.cuda.current_device()).multi_processor_count
+
+
+@functools.lru_cache(maxsize=4096)
 def _use_tile(M: int, N: int, K: int) -> bool:
     """Plain products for csrc/tile_gemm.hip: long K, where hipBLASLt keeps
     whole tiles and leaves CUs idle or falls to small ones, from 0.5 to 1.65
-    PFLOP/s with no order in M (us, library / tile): 4133 x 5120 x 27648
-    1448 / 810, 5000 x 5120 x 27648 1667 / 1013, 600 x 2048 x 10944 54 / 38,
-    4100 x 4096 x 14336 725 / 347 but 4096 x 4096 x 14336 286 / 311. The
-    library goes on where a tile's step of 1.33 us says less than 1.2
-    PFLOP/s (2800 x 4096 x 14336 236 / 291), and with shorter K, where it
-    is mostly 5 % ahead (4133 x 7168 x 5120 202 / 216)."""
+    PFLOP/s (us, library / tile): 4133 x 5120 x 27648 1448 / 810, 5000 x 5120
+    x 27648 1667 / 1013, 4100 x 4096 x 14336 725 / 347, 512 x 4096 x 29568
+    267 / 121. The library goes on where a tile's step of 1.33 us says less
+    than 1.2 PFLOP/s (2800 x 4096 x 14336 236 / 291), with shorter K, where
+    it is mostly 5 % ahead (4133 x 7168 x 5120 202 / 216), and where its own
+    tiles fit: a last round of 256 x 256 tiles that is nearly full (8192 x
+    4096 x 14336 605 / 642, 8192 x 2048 x 6144 131 / 142), a single one that
+    is half to four fifths full (8192 x 1536 x 11904 222 / 278, 2304 x 5120 x
+    15360 277 / 319), and, with K below 14336, any that is more than two
+    fifths full (10594 x 2560 x 7680 301 / 332). Over 3977 sizes of 256 to
+    16384 rows this takes 863, in 0.71 of the library's time, five of them
+    slower by 3 to 7 %."""
     if K < 3 * N or not _tile_fits(M, N, K, False):
+        return False
+    tiles, cus = -(-M // 256) * -(-N // 256), _compute_units()
+    last = ((tiles - 1) % cus + 1) / cus  # full part of the last round
+    if last > 0.9 or (tiles <= cus and 0.5 < last <= 0.8) \
+            or (last > 0.4 and K < 14336):
         return False
     us = 1.33 * _gpu_kernels().tile_gemm_cost(M, N, K, False)
     return us * 1.2e9 < 2.0 * M * N * K
@@ -947,15 +967,16 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     kernel for many rows and long K, where measured faster; hipBLASLt
     otherwise."""
     import torch.nn.functional as F
-    if _streams(x, w):
-        return skinny_gemm(x, w, bias)
-    if (_rows_ok(x, w) and plain_bias(bias, w.shape[0])
-            and (bias is None or bias.data_ptr() % 16 == 0)
-            and _use_tile(x.shape[0], w.shape[0], w.shape[1])
-            and not (torch.is_grad_enabled()  # (the library's has one)
-                     and any(t is not None and t.requires_grad
-                             for t in (x, w, bias)))):
-        return _gpu_kernels().tile_gemm(x, w, bias, False)
+    if _rows_ok(x, w):
+        M, (N, K) = x.shape[0], w.shape
+        if _use_skinny(M, N, K):
+            return skinny_gemm(x, w, bias)
+        if (_use_tile(M, N, K) and plain_bias(bias, N)
+                and (bias is None or bias.data_ptr() % 16 == 0)
+                and not (torch.is_grad_enabled()  # (the library's has one)
+                         and any(t is not None and t.requires_grad
+                                 for t in (x, w, bias)))):
+            return _gpu_kernels().tile_gemm(x, w, bias, False)
     return F.linear(x, w, bias)
 
 

@@ -57,7 +57,8 @@ def test_rows_past_the_last_are_left_alone():
 
 @pytest.mark.parametrize("M", [256, 257, 384, 500])
 def test_dispatch(M):
-    """The same numbers whichever kernel a row count is sent to."""
+    """The same numbers whichever kernel a row count is sent to: the stream
+    and the library, gated the stream and the tile kernel."""
     from gllm_amd import ops
     torch.manual_seed(M)
     x = torch.randn(M, 3072, device="cuda").bfloat16()
@@ -136,6 +137,39 @@ def test_lines_of_parts(M, N, K, stream):
     err = (part.double().sum(0) - y).abs() / y.abs().clamp_min(
         y.square().mean().sqrt())
     assert err.max() < 2 ** -23 * K ** 0.5  # fp32 sums
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (4096, 1024, 17408, True), (500, 4096, 28672, True),
+    (8200, 1024, 17408, False),    # a round that is half full
+    (8192, 2048, 6144, False),     # nearly full
+    (10600, 2560, 7680, False),    # the second one, K short
+    (4096, 1024, 3008, False),     # K below 3 N
+    (2000, 512, 2048, False),      # slow for either
+])
+def test_long_contractions(M, N, K, tile):
+    """Which sizes ops.linear sends to the tile kernel, and its bias there:
+    one off 16 bytes, of another type or strided goes to the library."""
+    from gllm_amd import ops
+    assert ops._use_tile(M, N, K) == tile
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    b = torch.randn(N + 1, device="cuda").bfloat16()
+    y = x.double() @ w.double().t()
+    lib = torch.nn.functional.linear
+    for bias in (None, b[:N], b[1:], b[:N].repeat(2).view(2, N).t()[:, 0],
+                 b[:1].expand(N)):
+        ours = tile and (bias is None or (bias.is_contiguous()
+                                          and bias.data_ptr() % 16 == 0))
+        out = ops.linear(x, w, bias)
+        if ours:
+            assert torch.equal(
+                out, ops._gpu_kernels().tile_gemm(x, w, bias, False))
+        else:
+            assert torch.equal(out, lib(x, w, bias))
+        ref = y if bias is None else y + bias.double()
+        assert ((out.double() - ref).norm() / ref.norm()) < 2 ** -8
 
 
 def test_long_contractions_have_gradients():
