@@ -961,6 +961,54 @@ def _use_tile(M: int, N: int, K: int) -> bool:
     return us * 1.2e9 < 2.0 * M * N * K
 
 
+@functools.lru_cache(maxsize=4096)
+def _use_tile_gated(M: int, N: int, K: int) -> bool:
+    """Gated products for csrc/tile_gemm.hip (us, library and the second
+    kernel or, up to 256 rows, stream / tile).
+    More than 256 rows: the tile kernel (512 x 5632 x 2048 31 / 26, 700 x
+    55296 x 5120 415 / 342, 4133 x 55296 x 5120 1971 / 1750, 4133 x 9728 x
+    2560 265 / 193), where hipBLASLt's tiles do not fit better:
+      half a row block is left, of few of them (384 x 55296 x 5120 218 / 260,
+      1152 x 43008 x 3840 332 / 367);
+      a single round of tiles, less than 25 / 32 full (512 x 9728 x 2560 41 /
+      46, 768 x 16384 x 11136 223 / 269);
+      a second one, half full (714 x 32768 x 2560 126 / 142) or, with short
+      K, less than a third (1242 x 16384 x 1536 75 / 81).
+    With short K the second kernel weighs more, so a single round or an
+    estimate (as in ``_use_tile``) of 1.1 PFLOP/s is enough, and so are few
+    tiles of any K, where the library does not split it. Below 384 rows wide
+    weights stay with the library (333 x 55296 x 5120 217 / 270). Over 3827
+    sizes of 257 to 9000 rows this takes 1995, in 0.84 of the time, three of
+    them slower by 4 %.
+    One block of rows: weights of a round of tiles that is at least 25 / 32
+    full, for K of 1024 to 14336 (256 x 51200 x 1024 34 / 32, 256 x 51200 x
+    4096 119 / 104, 129 x 61440 x 14336 426 / 341; 256 x 49152 x 8192 223 /
+    233, 256 x 28672 x 4096 67 / 80)."""
+    if not (K % 64 == 0 and N <= 1 << 20 and M <= 1 << 24
+            and N * K < 1 << 30):
+        return False
+    cus, cols = _compute_units(), -(-N // 256)
+    if M <= SKINNY_MAX_M:
+        return 128 < M and 25 * cus <= 32 * cols <= 32 * cus and K >= 1024
+    if not _tile_fits(M, N, K, True) or (M < 384 and N >= 16384):
+        return False
+    tiles = -(-M // 256) * cols
+    if tiles <= 20:
+        return True
+    if K <= 2048:
+        us = 1.33 * _gpu_kernels().tile_gemm_cost(M, N, K, True)
+        if tiles <= cus or us * 1.1e9 < 2.0 * M * N * K:
+            return True
+    if 0 < M % 256 <= 128 and M < 1600:
+        return False
+    if tiles <= cus:
+        return 32 * tiles > 25 * cus
+    if tiles <= 2 * cus:
+        last = tiles / cus - 1
+        return not 0.47 < last < 0.53 and (K > 2048 or last > 1 / 3)
+    return True
+
+
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """GEMM dispatch: the weight-streaming kernel for few rows, the tile
@@ -984,23 +1032,16 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ w_gate.T) * (x @ w_up.T), w = gate rows over up rows. Few
     rows: one kernel, the [rows, 2 ff] product is never written (above 64
     rows it is level with the library's product and saves the second
-    kernel: 256 x 55296 x 5120 149 us against 154 + 9). Many rows: the tile
-    kernel, again one (us, library and second kernel / tile: 512 x 5632 x
-    2048 27 / 26, 512 x 55296 x 5120 288 / 237, 4133 x 55296 x 5120 1960 /
-    1700, 8192 x 28672 x 4096 1388 / 1304; wide weights need 384 rows: 333 x
-    55296 x 5120 217 / 270). One block of rows on very wide weights too
-    (stream / tile: 256 x 55296 x 5120 152 / 137, 192 rows 150 / 129, 128
-    rows 116 / 116; 256 x 28672 x 4096 67 / 80)."""
+    kernel: 256 x 55296 x 5120 149 us against 154 + 9). Many rows, and one
+    block of them on very wide weights: the tile kernel, again one, where it
+    is the faster (see ``_use_tile_gated``)."""
     if (_rows_ok(x, w) and w.shape[0] % 16 == 0 and w.shape[0] >= 512):
         M, (N, K) = x.shape[0], w.shape
-        # one row block and a round of 192 to 256 column blocks
-        if (128 < M <= 256 and 49152 <= N <= 65536 and 4096 <= K < 16384
-                and _use_skinny(M, 512, K)):
+        few = _use_skinny(M, 512, K)
+        if (few or M > SKINNY_MAX_M) and _use_tile_gated(M, N, K):
             return _gpu_kernels().tile_gemm(x, w, None, True)
-        if _use_skinny(M, 512, K):
+        if few:
             return _gpu_kernels().stream_gemm_gated(x, w)
-        if _tile_fits(M, N, K, True) and (M >= 384 or N < 16384):
-            return _gpu_kernels().tile_gemm(x, w, None, True)
     return silu_and_mul(linear(x, w))
 
 

@@ -190,3 +190,39 @@ def test_long_contractions_have_gradients():
         with torch.no_grad():
             assert not ops.linear(x, w).requires_grad
         operand.requires_grad_(False)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (128, 55296, 4096, False), (129, 55296, 4096, True),
+    (256, 51200, 1024, True), (256, 51184, 1088, True),
+    (256, 50944, 1024, False), (200, 65536, 1024, True),
+    (200, 65552, 1024, False),               # more than a round
+    (200, 51200, 960, False),
+    (300, 5632, 2048, True), (300, 16384, 2048, False),
+    (257, 2048, 4096, True),                 # few tiles
+    (512, 9728, 2560, False), (768, 16384, 11136, False),  # part of a round
+    (1000, 13312, 2560, True),
+    (384, 55296, 5120, False), (512, 55296, 5120, True),   # half row blocks
+    (1152, 43008, 3840, False), (1664, 43008, 3840, True),
+    (714, 32768, 2560, False), (700, 37888, 3584, True),   # second rounds
+    (1242, 16384, 1536, False), (1242, 21888, 2048, True),
+])
+def test_lines_of_gated(M, N, K, tile):
+    """Which sizes ops.linear_silu sends to the tile kernel; up to 256 rows
+    the others are the stream's, above the library's."""
+    from gllm_amd import ops
+    assert ops._use_tile_gated(M, N, K) == tile
+    k = ops._gpu_kernels()
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    if tile:
+        ref = k.tile_gemm(x, w, None, True)
+    elif M <= 256:
+        ref = k.stream_gemm_gated(x, w)
+    else:
+        ref = ops.silu_and_mul(torch.nn.functional.linear(x, w))
+    assert torch.equal(ops.linear_silu(x, w), ref)
+    g, u = (x[:3].double() @ w.double().t()).chunk(2, dim=-1)
+    y = torch.nn.functional.silu(g) * u
+    assert ((ref[:3].double() - y).norm() / y.norm()) < 2 ** -7
