@@ -223,7 +223,7 @@ class MLAAttention(nn.Module):
         from there on are whole prompts)."""
         if type(self)._dsa_select is not MLAAttention._dsa_select:
             return fctx.seq_lens.shape[0]  # (selected positions only)
-        return fctx.prompts_from()
+        return fctx.per_head_from(self.num_heads)
 
     def _with_prompts(self, first, positions, hidden, q_resid, q, kv_a,
                       fctx):

@@ -65,6 +65,8 @@ class ForwardContext:
 
     _prompts_from: Optional[int] = dataclasses.field(default=None,
                                                      kw_only=True)
+    _per_head_from: Optional[tuple] = dataclasses.field(default=None,
+                                                        kw_only=True)
 
     def prompts_from(self) -> int:
         """The first sequence from which on all are whole prompts: two rows
@@ -78,6 +80,37 @@ class ForwardContext:
                     s -= 1
             self._prompts_from = s
         return self._prompts_from
+
+    def per_head_from(self, heads: int) -> int:
+        """The first sequence from which on latent attention of ``heads``
+        heads takes the per-head form, which only whole prompts can (their
+        number where the absorbed form of everything is the faster one; us
+        of an attention layer of 16 heads, absorbed / the two forms):
+        prompts of 8 rows and more on average (64 of 8 55 / 41, 300 of 2 72
+        / 86); behind decode rows if one of those has 512 keys, for which the
+        absorbed form of a mixed batch is one long chain (16 of 1000 keys and
+        32 rows 114 / 80, of 200 keys 52 / 72), or if the mixed batch's tiles
+        fill the chip (64 of 200 keys and 192 rows 152 / 86); behind portions
+        of prompts, which stay absorbed, if there is much to save (256 rows
+        after 2000 and 64 rows 250 / 281, 2048 rows 413 / 367)."""
+        if self._per_head_from is None or self._per_head_from[0] != heads:
+            self._per_head_from = (heads, self._choose_per_head(heads))
+        return self._per_head_from[1]
+
+    def _choose_per_head(self, heads: int) -> int:
+        n, s = self.seq_lens.shape[0], self.prompts_from()
+        if s == n:
+            return n
+        qsl, lens = self.host_qsl(), self.host_seq_lens()
+        rows = qsl[n] - qsl[s]
+        if rows < 8 * (n - s):
+            return n
+        if qsl[s] > s:
+            return s if rows * heads >= 32768 else n
+        if s > 0 and max(lens[:s]) < 512 \
+                and n * max(lens[s:n]) * heads < 65536:
+            return n
+        return s
 
     @property
     def is_pure_decode(self) -> bool:

@@ -82,3 +82,29 @@ def test_converted_rows_are_freed():
         own = w.numel() * w.element_size()
         assert w.untyped_storage().nbytes() == (
             own if quantized else own + 192 * 64 * 4)
+
+
+@pytest.mark.parametrize("rows,past,heads,prompts,per_head", [
+    ([8], [0], 16, 0, 0), ([7], [0], 16, 0, 1),
+    ([1], [0], 16, 1, 1), ([1], [30], 16, 1, 1),     # decode rows
+    ([2] * 300, [0] * 300, 16, 0, 300), ([8] * 64, [0] * 64, 16, 0, 0),
+    ([9, 1], [0, 0], 16, 2, 2),            # a prompt of one row ends the tail
+    ([40, 40], [0, 16], 16, 2, 2),         # so does a cached prefix
+    ([1] * 16 + [32], [510] * 16 + [0], 16, 16, 17),  # 511 keys
+    ([1] * 16 + [32], [511] + [9] * 15 + [0], 16, 16, 16),
+    ([1] * 64 + [63], [200] * 64 + [0], 16, 64, 65),  # tiles of the mixed
+    ([1] * 64 + [64], [200] * 64 + [0], 16, 64, 64),
+    ([1] * 64 + [63], [200] * 64 + [0], 32, 64, 64),
+    ([1, 256, 2047], [900, 2000, 0], 16, 2, 3),       # behind a portion
+    ([1, 256, 2048], [900, 2000, 0], 16, 2, 2),
+    ([1, 256, 256], [900, 2000, 0], 128, 2, 2),
+    ([0, 12], [5, 0], 16, 1, 2),
+])
+def test_forms(rows, past, heads, prompts, per_head):
+    """Where whole prompts begin, and from where on they attend per head."""
+    for extra in ((), (sum(rows), 9 + sum(rows))):
+        fctx = _context(rows, past, extra)
+        assert fctx.prompts_from() == prompts
+        assert fctx.per_head_from(heads) == per_head
+        assert fctx.per_head_from(heads) == per_head  # (kept)
+        assert _layer()._prompts_from(fctx) == fctx.per_head_from(1)
