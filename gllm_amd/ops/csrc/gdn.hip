@@ -479,6 +479,7 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     const int *__restrict__ has_init, const int *__restrict__ qsl, long T,
     int Hk, int Hv) {
   constexpr int VT = DVS / 16;
+  static_assert(VT <= 2, "q S^T: a term of each column tile in turn, below");
   const int seq = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
   const int begin = qsl[seq], end = qsl[seq + 1];
   if (begin >= end) return;
