@@ -5,22 +5,23 @@
 //   grid = B * Hkv * splits, block = 256 threads (4 waves). A workgroup
 //   serves the whole GQA group (up to 16 query heads) of one kv head over
 //   a share of the keys, so K/V bytes are read once for all its heads.
-//   From 257 workgroups to two rounds of them, if a sequence gives each of
-//   its workgroups more than 1024 keys of 128 + 128 values and lengths differ,
-//   heads are the fastest index (the eight dies take workgroups in turn, so
-//   with 8 heads each die gets a share of every sequence), then splits, and
-//   sequences come longest first (sequence_at), so what starts last is short.
-//   More rounds even out by themselves, and a workgroup per CU starts at once
-//   in any order. Finding the sequence costs each workgroup 1 to 3 us, more
-//   than short shares give back, and heads fastest is the slower one for equal
-//   lengths: there sequences are the fastest index, as they come. (us, 32
-//   heads on 8 of 128, sequences fastest / this: 64 sequences of 512 to 1536
-//   keys 68 / 61, 128 of 1024 to 3072 218 / 197, 24 of 2700 to 8100 in four
-//   splits 138 / 124, 100 of 1 to 4000 179 / 153. Where it is not done, as
-//   they come / in order: 128 of 2048 179 / 193, 33 of 1100 in two splits 39 /
-//   46, 100 of 700 to 1000 71 / 78; one head, 33 of 10 to 1100 in sixteen
-//   splits 18.5 / 25.4; 14 heads on 2 of 64, 64 of 512 to 1536 14.5 / 17.2,
-//   400 of 100 to 1500 39 / 42; 64 of 1600 to 2048 would gain, 96 / 91.)
+//   From 257 workgroups to two rounds of them, if a sequence gives each of its
+//   workgroups more than 1024 keys of 128 + 128 values (700 in a round of at
+//   most 64 sequences) and lengths differ, heads are the fastest index (the
+//   eight dies take workgroups in turn, so with 8 heads each die gets a share
+//   of every sequence), then splits, and sequences come longest first
+//   (sequence_at), so what starts last is short. More rounds even out by
+//   themselves, and a workgroup per CU starts at once in any order. Finding
+//   the sequence costs each workgroup 1 to 3 us, more than short shares give
+//   back, and heads fastest is the slower one for equal lengths: there
+//   sequences are the fastest index, as they come. (us, 32 heads on 8 of 128,
+//   sequences fastest / this: 64 sequences of 512 to 1536 keys 68 / 61, 128 of
+//   1024 to 3072 218 / 197, 24 of 2700 to 8100 in four splits 138 / 124, 100
+//   of 1 to 4000 179 / 153, 32 of 10 to 1500 in two 35 / 30. Where it is not
+//   done, as they come / in order: 128 of 2048 179 / 193, 33 of 1100 in two
+//   splits 39 / 46, 100 of 700 to 1000 71 / 78; one head, 33 of 10 to 1100 in
+//   sixteen splits 18.5 / 25.4; 14 heads on 2 of 64, 64 of 512 to 1536 14.5 /
+//   17.2, 400 of 100 to 1500 39 / 42; 64 of 1600 to 2048 would gain, 96 / 91.)
 //   Its waves work on their own: wave w takes the 32-key tiles w, w + 4,
 //   ... of the share, with a softmax state of its own and no barrier in the
 //   loop; the next tile's K and V are in registers while this one is
@@ -62,8 +63,9 @@ union DecFrag {
 
 constexpr int ORDERED = 1024;  // workgroups at most: two rounds
 constexpr int ALONE = 256;     // a CU each: all start at once, in any order
-constexpr int SHARE = 1024 * 256;  // values of K and V a workgroup: up to
-                                   // here, order gives less than it takes
+// Values of K and V a workgroup: up to here, order gives less than it takes.
+// (FEW: a round of workgroups of at most 64 sequences, found the fastest)
+constexpr int SHARE = 1024 * 256, SHARE_FEW = 700 * 256;
 
 // The sequence whose visible keys come `rank`th, the most first, to within a
 // sixteenth of the most (equal ones by number); -1 if half of them have more
@@ -502,6 +504,8 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
     pl = lse.data_ptr<float>();
     direct = nullptr;
   }
+  const bool few = B <= 64 && B * Hkv * zdim <= ORDERED / 2;
+  const int order_above = (few ? SHARE_FEW : SHARE) / (D + Dv) * splits;
   auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(DT, DVT)                                                         \
   hipLaunchKernelGGL((paged_decode_kernel<DT, DVT>), dim3(B * Hkv * zdim),   \
@@ -515,7 +519,7 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      keep_first, softcap, bias, bias_len, temp_coef,         \
                      temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
                      sinks, (const __hip_bfloat16 *)gate, gate_stride, B,    \
-                     zdim, SHARE / (D + Dv) * splits)
+                     zdim, order_above)
   if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
 #undef RUN

@@ -56,8 +56,9 @@ def _in_order(n, Hkv, D, pool):
         splits *= 2
     most = max(n)
     alike = sum(x > most - most // 8 for x in n)
+    share = 700 if B <= 64 and B * Hkv * splits <= 512 else 1024
     return splits, (256 < B * Hkv * splits <= 1024 and 2 * alike < B
-                    and most > 1024 * 128 // D * splits)
+                    and most > share * 256 // (2 * D) * splits)
 
 
 @pytest.mark.parametrize("B,Hkv,D,splits,lens,order", [
@@ -67,6 +68,8 @@ def _in_order(n, Hkv, D, pool):
     (1024, 1, 128, 1, "wide", True),    # the most sequences
     (400, 2, 64, 1, "wide", True),
     (37, 8, 128, 2, "wide", True), (24, 8, 128, 4, "wide", True),
+    (64, 8, 128, 1, "shorter", True), (65, 8, 128, 1, "shorter", False),
+    (32, 8, 128, 2, "shorter", True),
     (96, 4, 128, 2, "zeros", True),
     (40, 8, 128, 2, "one long", True),
     (64, 8, 128, 1, "alike", False), (64, 8, 128, 1, "half alike", False),
@@ -78,7 +81,8 @@ def test_long_sequences(B, Hkv, D, splits, lens, order):
     from gllm_amd import ops
     from gllm_amd.ops import torch_ref
     torch.manual_seed(B + Hkv)
-    G, page, most = 2, 16, 1100 * splits * 128 // D
+    G, page = 2, 16
+    most = (750 if lens == "shorter" else 1100) * splits * 128 // D
     n = torch.randint(1, most // 3, (B,))
     longs = torch.randperm(B)[:1 if lens == "one long" else max(2, B // 16)]
     n[longs] = torch.randint(most // 2, most, longs.shape)
