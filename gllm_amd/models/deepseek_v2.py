@@ -116,8 +116,10 @@ class MLAAttention(nn.Module):
 
     def _queries_and_latents(self, hidden):
         """q_proj(hidden), kv_a_proj_with_mqa(hidden): one product where
-        the weights still lie together (us, two / one: 4096 rows 48 + 24 /
-        66, 128 rows 29 / 15)."""
+        the weights still lie together and it is a round of tiles at most
+        (us, two / one, width 2048: 16 heads, 128 rows 31 / 15, 4096 rows 63
+        / 59; beyond, the 576 columns cost the library its even tiles: 8 heads,
+        8192 rows 73 / 81, 128 heads, 2048 rows 163 / 226)."""
         qp, kp = self.q_proj, self.kv_a_proj_with_mqa
         a, b = qp.weight, kp.weight
         if (hidden.is_cuda and qp.is_plain and kp.is_plain
@@ -126,7 +128,9 @@ class MLAAttention(nn.Module):
                 and a.is_contiguous() and b.is_contiguous()
                 and a.untyped_storage().data_ptr()
                 == b.untyped_storage().data_ptr()
-                and b.storage_offset() == a.storage_offset() + a.numel()):
+                and b.storage_offset() == a.storage_offset() + a.numel()
+                and ops.one_round(hidden.shape[0],
+                                  a.shape[0] + b.shape[0])):
             w = a.as_strided((a.shape[0] + b.shape[0], a.shape[1]),
                              (a.shape[1], 1))
             return ops.linear(hidden, w).split([a.shape[0], b.shape[0]], -1)

@@ -934,6 +934,11 @@ def _compute_units() -> int:
         torch.cuda.current_device()).multi_processor_count
 
 
+def one_round(M: int, N: int) -> bool:
+    """Whether an M x N product is a round of 256 x 256 tiles at most."""
+    return -(-M // 256) * -(-N // 256) <= _compute_units()
+
+
 @functools.lru_cache(maxsize=4096)
 def _use_tile(M: int, N: int, K: int) -> bool:
     """Plain products for csrc/tile_gemm.hip: long K, where hipBLASLt keeps

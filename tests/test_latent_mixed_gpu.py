@@ -140,6 +140,14 @@ def test_one_product_for_two():
         assert q.stride(0) == kv.stride(0) == 16 * 192 + 576
         for a, b in zip((q, kv), parts):  # sums in another order
             assert (a.double() - b.double()).norm() / b.norm() < 2 ** -8
+    for M, one in ((4352, True), (4353, False)):  # 255 tiles, 270
+        x = torch.randn(M, HIDDEN, device=DEV).bfloat16()
+        with torch.no_grad():
+            q, kv = layer._queries_and_latents(x)
+            parts = layer.q_proj(x), layer.kv_a_proj_with_mqa(x)
+        assert q.is_contiguous() != one
+        for a, b in zip((q, kv), parts):
+            assert (a.double() - b.double()).norm() / b.norm() < 2 ** -8
     b = layer.kv_a_proj_with_mqa.weight
     b.data = b.data.clone()               # apart: two products
     with torch.no_grad():
