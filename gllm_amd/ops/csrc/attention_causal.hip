@@ -27,10 +27,10 @@
 // The structure is the general kernel's: four waves of 32 rows, scores K Q^T
 // so that a lane holds 16 keys of one query, O^T = V^T P^T with V read
 // transposed, K and V in two LDS slots of 64 keys. (us, general kernel / this;
-// 128 wide: 5 prompts of 4096 rows, 40 heads on 8, 157 / 79; 7 of 5000, 32 on
-// 8, 140 / 68; 4 of 2048 435 / 171; one of 8192 1375 / 568, 968 TFLOP/s; 512
-// rows after 8192 346 / 228; 32 of 128 rows 33 / 27; 64 wide, 2 of 2048, 32
-// heads 163 / 59.)
+// 128 wide: 5 prompts of 4096 rows in all, 40 heads on 8, 145 / 77; 7 of 5000
+// in all, 32 on 8, 145 / 65; 4 of 2048 441 / 178; one of 8192 1387 / 588, 935
+// TFLOP/s; 512 rows after 8192 347 / 233; 40 heads, 32 of 128 rows 41 / 32; 64
+// wide, 2 of 2048, 32 heads 164 / 58.)
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
