@@ -951,16 +951,16 @@ def _use_tile(M: int, N: int, K: int) -> bool:
     tiles fit: a last round of 256 x 256 tiles that is nearly full (8192 x
     4096 x 14336 605 / 642, 8192 x 2048 x 6144 131 / 142), a single one that
     is half to four fifths full (8192 x 1536 x 11904 222 / 278, 2304 x 5120 x
-    15360 277 / 319), and, with K below 14336, any that is more than two
-    fifths full (10594 x 2560 x 7680 301 / 332). Over 3977 sizes of 256 to
-    16384 rows this takes 863, in 0.71 of the library's time, five of them
-    slower by 3 to 7 %."""
+    15360 277 / 319), and, with K below 14336, any that is more than half
+    full, below 9600 two fifths (10594 x 2560 x 7680 301 / 332; 4096 x 2048 x
+    10944 154 / 142). Over 3977 sizes of 256 to 16384 rows this takes 915, in
+    0.72 of the library's time, five of them slower by 3 to 7 %."""
     if K < 3 * N or not _tile_fits(M, N, K, False):
         return False
     tiles, cus = -(-M // 256) * -(-N // 256), _compute_units()
     last = ((tiles - 1) % cus + 1) / cus  # full part of the last round
     if last > 0.9 or (tiles <= cus and 0.5 < last <= 0.8) \
-            or (last > 0.4 and K < 14336):
+            or K < (0 if last <= 0.4 else 9600 if last <= 0.5 else 14336):
         return False
     us = 1.33 * _gpu_kernels().tile_gemm_cost(M, N, K, False)
     return us * 1.2e9 < 2.0 * M * N * K

@@ -142,6 +142,7 @@ def test_lines_of_parts(M, N, K, stream):
 @pytest.mark.parametrize("M,N,K,tile", [
     (4096, 1024, 17408, True), (500, 4096, 28672, True),
     (8200, 1024, 17408, False),    # a round that is half full
+    (4096, 2048, 10944, True), (4096, 2048, 9472, False),
     (8192, 2048, 6144, False),     # nearly full
     (10600, 2560, 7680, False),    # the second one, K short
     (4096, 1024, 3008, False),     # K below 3 N
