@@ -547,34 +547,52 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     const __amdgpu_buffer_rsrc_t ru =
         rows_of(u0 + ((long)start * Hv + h) * D + z * DVS,
                 (len - 1) * row_b * 2 + DVS * 4);
+    if (wave * 16 >= len) {
+      // no row of this wave (64 prompts of 16 rows, 16 heads: 118 us, 126
+      // with loads that all fall outside)
+      const shortx8 none = {};
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const __amdgpu_buffer_rsrc_t rw =
-          rows_of(wk + ((j * T + start) * Hv + h) * D,
-                  (len - 1) * row_b + D * 2);
+      for (int j = 0; j < 3; ++j) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) wr[ks][j] = load16(rw, w_at + ks * 64);
-    }
+        for (int ks = 0; ks < 4; ++ks) wr[ks][j] = none;
+        ar[0][j] = ar[1][j] = none;
+      }
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) qr[ks] = load16(rq, q_at + ks * 64);
+      for (int ks = 0; ks < 4; ++ks) qr[ks] = none;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const __amdgpu_buffer_rsrc_t ra =
-          rows_of(att + ((j * T + start) * Hv + h) * C,
-                  ((len - 1) * Hv + 1) * C * 2);
-      ar[0][j] = load16(ra, a_at);
-      // (blocks past the diagonal's pair are never written, nor read)
-      if (wave >= 2) ar[1][j] = load16(ra, a_at + 64);
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ur[vt][r] = 0.f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const __amdgpu_buffer_rsrc_t rw =
+            rows_of(wk + ((j * T + start) * Hv + h) * D,
+                    (len - 1) * row_b + D * 2);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) wr[ks][j] = load16(rw, w_at + ks * 64);
+      }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) qr[ks] = load16(rq, q_at + ks * 64);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const __amdgpu_buffer_rsrc_t ra =
+            rows_of(att + ((j * T + start) * Hv + h) * C,
+                    ((len - 1) * Hv + 1) * C * 2);
+        ar[0][j] = load16(ra, a_at);
+        // (blocks past the diagonal's pair are never written, nor read)
+        if (wave >= 2) ar[1][j] = load16(ra, a_at + 64);
+      }
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          ur[vt][r] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(
+                         ru, u_at + r * row_b * 2 + vt * 64, 0, 0));
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) kr[j] = load16(rk, k_at + j * 16 * key_b);
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ur[vt][r] = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(
-                       ru, u_at + r * row_b * 2 + vt * 64, 0, 0));
     sr = scal[(min(wave, 2) * T + start + min(lane, len - 1)) * Hv + h];
   };
   auto put_keys = [&](int buf) {
