@@ -30,10 +30,11 @@
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
+#include "qkv_rows.h"
 #include "tile_gemm.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 st_bf8;
-typedef __attribute__((ext_vector_type(4))) float st_f4;
+typedef part_f4 st_f4;
 
 namespace {
 
@@ -49,10 +50,6 @@ DEV_INLINE void glds16(const __hip_bfloat16 *gsrc, char *lds_ptr) {
   __builtin_amdgcn_global_load_lds(
       reinterpret_cast<const unsigned int *>(gsrc),
       reinterpret_cast<unsigned int *>(lds_ptr), 16, 0, AUX);
-}
-
-DEV_INLINE short to_bf16(float v) {
-  return __builtin_bit_cast(short, __float2bfloat16(v));
 }
 
 // wait until at most AHEAD stages of LD loads are on their way
@@ -209,39 +206,15 @@ __global__ __launch_bounds__(WM *WN * 64) void stream_gemm_kernel(
   }
 }
 
-DEV_INLINE float bf16_value(float v) {
-  return __bfloat162float(__float2bfloat16(v));
-}
-
-// sum of the S parts of four columns; loads of eight parts in flight
-DEV_INLINE st_f4 part_sum(const float *p, long stride, int S) {
-  st_f4 v = *reinterpret_cast<const st_f4 *>(p);
-  int s = 1;
-  for (; s + 8 <= S; s += 8) {
-    st_f4 b[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      b[i] = *reinterpret_cast<const st_f4 *>(p + (s + i) * stride);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v += b[i];
-  }
-  st_f4 b[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    b[i] = *reinterpret_cast<const st_f4 *>(p + min(s + i, S - 1) * stride);
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    if (s + i < S) v += b[i];
-  return v;
-}
-
 template <typename TB>
 __global__ __launch_bounds__(256) void stream_sum_kernel(
     __hip_bfloat16 *__restrict__ out, const float *__restrict__ part,
     const TB *__restrict__ bias, long MN, int N, int S) {
   const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
-  const st_f4 v = part_sum(part + i, MN, S);
+  st_f4 sum[1];
+  part_sums<1>({part + i}, MN, S, sum);
+  const st_f4 v = sum[0];
   const int n = i % N;
   shortx4 o;
 #pragma unroll
@@ -251,7 +224,10 @@ __global__ __launch_bounds__(256) void stream_sum_kernel(
 }
 
 // A workgroup per row: residual += sum of the parts (rounded as stored),
-// out = RMS norm of the stored residual. V x 4 columns per thread.
+// out = RMS norm of the stored residual. V x 4 columns per thread. Bound by
+// one chain of memory latencies: with all loads ahead of the sums, and each
+// part read once, 64 x 5120 in four parts takes 5.7 us (7.6 with the groups
+// of columns in turn), 256 x 5120 in six 10.4 (11.1), 1 x 4096 4.5 (4.8).
 template <int V, typename TW>
 __global__ __launch_bounds__(512) void stream_add_norm_kernel(
     __hip_bfloat16 *__restrict__ out, __hip_bfloat16 *__restrict__ residual,
@@ -260,28 +236,40 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
   __shared__ float red[8];
   const long row = blockIdx.x;
   const long MN = (long)M * N;
+  // every load goes out before the first sum (columns past the row's end
+  // repeat its last four)
+  const float *p[V];
+  shortx4 old[V];
+  float wv[V][4];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const int c = min((j * 512 + (int)threadIdx.x) * 4, N - 4);
+    p[j] = part + row * N + c;
+    old[j] = *reinterpret_cast<const shortx4 *>(residual + row * N + c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wv[j][r] = ScalarOps<TW>::to_f32(w[c + r]);
+  }
+  st_f4 v[V];
+  part_sums<V>(p, MN, S, v);
   float x[V][4], ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
     const int c = (j * 512 + threadIdx.x) * 4;
-    if (c >= N) continue;
-    st_f4 v = part_sum(part + row * N + c, MN, S);
     if (rounded) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = bf16_value(v[r]);
+      for (int r = 0; r < 4; ++r) v[j][r] = bf16_value(v[j][r]);
     }
-    __hip_bfloat16 *rp = residual + row * N + c;
-    const shortx4 old = *reinterpret_cast<const shortx4 *>(rp);
     shortx4 o;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      o[r] = to_bf16(v[r] + __bfloat162float(__builtin_bit_cast(
-                                __hip_bfloat16, (short)old[r])));
+      o[r] = to_bf16(v[j][r] + __bfloat162float(__builtin_bit_cast(
+                                   __hip_bfloat16, (short)old[j][r])));
       x[j][r] =
           __bfloat162float(__builtin_bit_cast(__hip_bfloat16, (short)o[r]));
-      ss += x[j][r] * x[j][r];
+      if (c < N) ss += x[j][r] * x[j][r];
     }
-    *reinterpret_cast<shortx4 *>(rp) = o;
+    if (c < N)
+      *reinterpret_cast<shortx4 *>(residual + row * N + c) = o;
   }
   ss = block_reduce_sum<512>(ss, red);
   const float inv = rsqrtf(ss / N + eps);
@@ -291,81 +279,31 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
     if (c >= N) continue;
     shortx4 o;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      o[r] = to_bf16(x[j][r] * inv * ScalarOps<TW>::to_f32(w[c + r]));
+    for (int r = 0; r < 4; ++r) o[r] = to_bf16(x[j][r] * inv * wv[j][r]);
     *reinterpret_cast<shortx4 *>(out + row * N + c) = o;
   }
 }
 
-// Workgroups along the columns of a token, a thread per 8 columns of a head:
-// 4 + 4 columns of a rotated pair block, or 8 plain ones. PARTS: src is fp32
-// [S, M, N].
+// Workgroups along the columns of a token, a thread per unit. PARTS: the rows
+// are fp32 parts [S, M, N].
 template <bool PARTS>
 __global__ __launch_bounds__(256) void qkv_finish_kernel(
     __hip_bfloat16 *__restrict__ q_out, __hip_bfloat16 *__restrict__ k_cache,
-    __hip_bfloat16 *__restrict__ v_cache, const void *__restrict__ src,
-    long src_stride, const __hip_bfloat16 *__restrict__ bias,
-    const long *__restrict__ positions, const float *__restrict__ cos_sin,
-    const long *__restrict__ slots, int M, int S, int Hq, int Hkv, int D,
-    int rot, int rounded) {
+    __hip_bfloat16 *__restrict__ v_cache, const QkvRows rows,
+    const long *__restrict__ slots, int Hq, int Hkv, int D) {
   const long t = blockIdx.x;
-  const int N = (Hq + 2 * Hkv) * D, per = D / 8;
-  const float *cs = cos_sin + positions[t] * rot;
   const long slot = slots[t];
-  auto load4 = [&](int c, float *o) {
-    if (PARTS) {
-      const st_f4 v =
-          part_sum((const float *)src + t * N + c, (long)M * N, S);
-      o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
-    } else {
-      const shortx4 v = *reinterpret_cast<const shortx4 *>(
-          (const __hip_bfloat16 *)src + t * src_stride + c);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        o[r] = __bfloat162float(
-            __builtin_bit_cast(__hip_bfloat16, (short)v[r]));
-    }
-    if (bias) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] += __bfloat162float(bias[c + r]);
-    }
-    if (rounded) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = bf16_value(o[r]);
-    }
-  };
-  const int i = blockIdx.y * 256 + threadIdx.x;
-  if (i < (Hq + 2 * Hkv) * per) {
-    const int h = i / per, u = i % per;
-    const bool turned = h < Hq + Hkv && u < rot / 8;
-    // first columns of the two groups of four
-    const int d1 = turned ? u * 4 : u * 8;
-    const int d2 = turned ? rot / 2 + u * 4 : u * 8 + 4;
-    float a[4], b[4];
-    load4(h * D + d1, a);
-    load4(h * D + d2, b);
-    if (turned) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float c = cs[d1 + r], s = cs[rot / 2 + d1 + r];
-        const float x = a[r], y = b[r];
-        a[r] = x * c - y * s;
-        b[r] = y * c + x * s;
-      }
-    }
-    __hip_bfloat16 *dst;
-    if (h < Hq) dst = q_out + (t * Hq + h) * D;
-    else if (h < Hq + Hkv) dst = k_cache + (slot * Hkv + (h - Hq)) * D;
-    else dst = v_cache + (slot * Hkv + (h - Hq - Hkv)) * D;
-    shortx4 o1, o2;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      o1[r] = to_bf16(a[r]);
-      o2[r] = to_bf16(b[r]);
-    }
-    *reinterpret_cast<shortx4 *>(dst + d1) = o1;
-    *reinterpret_cast<shortx4 *>(dst + d2) = o2;
-  }
+  const int i = blockIdx.y * 256 + threadIdx.x, per = D / 8;
+  if (i >= (Hq + 2 * Hkv) * per) return;
+  const int h = i / per;
+  const QkvUnit x =
+      qkv_unit<PARTS>(rows, t, h, i % per, h < Hq + Hkv, Hq + 2 * Hkv, D);
+  __hip_bfloat16 *dst;
+  if (h < Hq) dst = q_out + (t * Hq + h) * D;
+  else if (h < Hq + Hkv) dst = k_cache + (slot * Hkv + (h - Hq)) * D;
+  else dst = v_cache + (slot * Hkv + (h - Hq - Hkv)) * D;
+  *reinterpret_cast<shortx4 *>(dst + x.d1) = x.o1;
+  *reinterpret_cast<shortx4 *>(dst + x.d2) = x.o2;
 }
 
 bool aligned16(const torch::Tensor &t) {
@@ -633,17 +571,22 @@ torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
   auto q = torch::empty({M, Hq * D}, k_cache.options());
   if (M == 0) return q;
   auto stream = at::cuda::getCurrentCUDAStream();
+  const QkvRows rows{src.data_ptr(),
+                     parts ? 0L : (long)src.stride(0),
+                     (const __hip_bfloat16 *)bp,
+                     positions.data_ptr<long>(),
+                     cos_sin.data_ptr<float>(),
+                     (int)M,
+                     parts ? (int)src.size(0) : 1,
+                     rot,
+                     (int)rounded};
 #define RUN(P)                                                               \
   hipLaunchKernelGGL((qkv_finish_kernel<P>),                                 \
                      dim3(M, (N / 8 + 255) / 256), dim3(256), 0, stream,     \
                      (__hip_bfloat16 *)q.data_ptr(),                         \
                      (__hip_bfloat16 *)k_cache.data_ptr(),                   \
-                     (__hip_bfloat16 *)v_cache.data_ptr(), src.data_ptr(),   \
-                     parts ? 0L : (long)src.stride(0),                       \
-                     (const __hip_bfloat16 *)bp, positions.data_ptr<long>(), \
-                     cos_sin.data_ptr<float>(), slots.data_ptr<long>(),      \
-                     (int)M, parts ? (int)src.size(0) : 1, (int)Hq, Hkv, D,  \
-                     rot, (int)rounded)
+                     (__hip_bfloat16 *)v_cache.data_ptr(), rows,             \
+                     slots.data_ptr<long>(), (int)Hq, Hkv, D)
   if (parts) RUN(true); else RUN(false);
 #undef RUN
   HIP_CHECK_KERNEL();
