@@ -94,6 +94,15 @@ class DenseAttention(nn.Module):
                 src = proj.parts(hidden)
                 if src is None:
                     src, bias = proj.project(hidden), None
+                elif fctx.is_pure_decode and ops.qkv_decode_ok(
+                        src, k_cache, attn.num_heads):
+                    return ops.qkv_decode(
+                        src, bias, positions, rope.cos_sin_cache, k_cache,
+                        v_cache, fctx.slot_mapping, fctx.block_table,
+                        fctx.seq_lens,
+                        fctx.arrivals(attn.num_kv_heads), attn.num_heads,
+                        attn.scale, attn.sliding_window,
+                        rounded=proj.fp8_block is not None)
                 q = ops.qkv_rope_cache(src, bias, positions,
                                        rope.cos_sin_cache, k_cache, v_cache,
                                        fctx.slot_mapping, attn.num_heads,

@@ -1104,6 +1104,32 @@ def qkv_rope_cache(src: torch.Tensor, bias, positions: torch.Tensor,
                                      rounded)
 
 
+def qkv_decode_ok(parts: torch.Tensor, k_cache: torch.Tensor,
+                  num_heads: int) -> bool:
+    """Whether ``qkv_decode`` takes these rows and heads (with caches that
+    ``qkv_rope_cache_ok`` takes) and is the faster form."""
+    return parts.dim() == 3 and _gpu_kernels().qkv_decode_ok(
+        k_cache, k_cache, num_heads, parts.shape[1])
+
+
+def qkv_decode(parts: torch.Tensor, bias, positions: torch.Tensor,
+               cos_sin: torch.Tensor, k_cache: torch.Tensor,
+               v_cache: torch.Tensor, slot_mapping: torch.Tensor,
+               block_table: torch.Tensor, seq_lens: torch.Tensor,
+               arrived: torch.Tensor, num_heads: int, scale: float,
+               sliding_window: int = 0,
+               rounded: bool = False) -> torch.Tensor:
+    """``qkv_rope_cache`` and the decode attention behind it, one token per
+    sequence, as one kernel; the heads' outputs [B, heads * D]. Each slot is
+    the last of its sequence. ``arrived``: int32 zeros, one per sequence and
+    kv head, that are zeros again behind the launch (launches that may run
+    at the same time need their own)."""
+    return _gpu_kernels().qkv_decode(
+        parts, bias, positions, cos_sin, k_cache, v_cache, slot_mapping,
+        block_table, seq_lens, arrived, num_heads, scale, sliding_window,
+        rounded)
+
+
 # --------------------------------------------------------------- layer norm
 def layernorm_f32(x: torch.Tensor, w: torch.Tensor, b, eps: float,
                   dtype) -> torch.Tensor:

@@ -43,6 +43,7 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <cstdlib>
 #include "common.h"
+#include "qkv_rows.h"
 
 namespace {
 
@@ -119,10 +120,66 @@ DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
   return 0;  // (not reached: every key is in 0 .. 15)
 }
 
+// What an instance that starts from the projection takes beside the caches.
+struct NewRows {
+  QkvRows rows;                    // q | k | v of each sequence's new token
+  __hip_bfloat16 *k_cache, *v_cache;
+  const long *slots;               // [B] where its key and value go
+  int *arrived;                    // [B, Hkv] zeros, left as zeros
+};
+
+// partials pass from one workgroup to another within a launch: written
+// through to where every die reads them
+DEV_INLINE void publish(float *p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// sum_s w_s o_s, w the softmax of the splits' scores (and of `sink`, which has
+// no value); scores of -inf take no part. AGENT: published by this launch
+template <bool AGENT>
+DEV_INLINE float merged(const float *o, long o_stride, const float *lse,
+                        long lse_stride, int n, float sink) {
+  auto at = [](const float *p) {
+    return AGENT ? __hip_atomic_load(p, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT)
+                 : *p;
+  };
+  // (sixteen splits, the most that the launcher chooses, are read at once)
+  float x[16], v[16], mx = sink;
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+    if (s < n) {
+      x[s] = at(lse + s * lse_stride);
+      v[s] = at(o + s * o_stride);
+    }
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+    if (s < n) mx = fmaxf(mx, x[s]);
+  for (int s = 16; s < n; ++s) mx = fmaxf(mx, at(lse + s * lse_stride));
+  float denom = sink == -INFINITY ? 0.f : __expf(sink - mx), sum = 0.f;
+  auto join = [&](float score, float value) {
+    if (score == -INFINITY) return;  // (its values are not written)
+    const float w = __expf(score - mx);
+    denom += w;
+    sum += w * value;
+  };
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+    if (s < n) join(x[s], v[s]);
+  for (int s = 16; s < n; ++s)
+    join(at(lse + s * lse_stride), at(o + s * o_stride));
+  return denom > 0.f ? sum / denom : 0.f;
+}
+
 // Head sizes Dr <= D, Dvr <= DV (multiples of 8; D, DV 64 or 128): columns
 // beyond a head are zero. G query heads per kv head, rows of the products
 // beyond G are zero. Optional bias by distance and query temperature.
-template <int D, int DV>
+// FRESH: the step from the projection's rows in one launch. Each workgroup
+// forms its heads' queries and the new key and value (in LDS; the first
+// split's workgroup stores them to the caches), and the last of a sequence's
+// workgroups to end joins their partials. (No bias, cap, gate, sink or
+// temperature; one query row per sequence.)
+template <int D, int DV, bool FRESH = false>
 __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     float *__restrict__ partial_out,  // [S, B, Hq, Dvr]
     float *__restrict__ partial_lse,  // [S, B, Hq]
@@ -142,11 +199,19 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     const float *__restrict__ sinks, const __hip_bfloat16 *__restrict__ gate,
     long gate_stride, int B, int zdim,
     // keys from which on the order of sequences matters
-    int order_above) {
+    int order_above, const NewRows fresh) {
   constexpr int KT = D / 32, NT = DV / 16;
   constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
   constexpr int VROW = DV * 2;             // LDS row bytes
   constexpr int VMASK = (DV / 8 - 1) & 15;
+  if constexpr (FRESH) {
+    softcap = temp_coef = 0.f;
+    bias = sinks = nullptr;
+    gate = nullptr;
+    qsl = nullptr;
+    keep_first = sink = 0;
+    zdim = num_splits;
+  }
   // (zdim: splits, and the kept-first segment)
   const int rest = blockIdx.x / B;
   int b = blockIdx.x - rest * B, kvh = rest % num_kv_heads;
@@ -194,7 +259,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const int l16 = lane & 15;
   const int lhi = lane >> 4;
   const long lse0 = (long)split * B * Hq + (long)b * Hq + kvh * G;
-  if (t0 >= t1) {
+  if (FRESH && t0 >= t1 && split > 0) return;
+  if (!FRESH && t0 >= t1) {
     // empty split: publish -inf lse so the merge ignores it
     if (out) {
       for (int i = tid; i < G * Dvr; i += BLOCK)
@@ -209,16 +275,6 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   __shared__ __attribute__((aligned(16))) char patch[WAVES][TK * VROW];
   __shared__ float s_m[WAVES][16], s_l[WAVES][16];
 
-  // query fragments: column l16 = head, dims kt * 32 + lhi * 8
-  dec_bf8 qf[KT];
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt) {
-    qf[kt] = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (l16 < G && kt * 32 + lhi * 8 < Dr)
-      qf[kt] = *reinterpret_cast<const dec_bf8 *>(
-          q + (long)row * q_stride + (kvh * G + l16) * Dr + kt * 32 +
-          lhi * 8);
-  }
   const int *bt = block_table + (long)b * max_pages;
   const shortx8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const float *brow =
@@ -281,6 +337,47 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     load(k0);
     if (k0 + WAVES * TK < t1) look_up(k0 + WAVES * TK);
   }
+  // FRESH: the new rows are formed while the first tiles arrive
+  __shared__ __attribute__((aligned(16))) short
+      own[FRESH ? (16 + 2) * D : 8];  // G queries, the key, the value
+  if constexpr (FRESH) {
+    const int per = Dr / 8;
+    for (int i = tid; i < (G + 2) * per; i += BLOCK) {
+      const int h = i / per;
+      const int col = h < G ? kvh * G + h : Hq + kvh + (h - G) * num_kv_heads;
+      const QkvUnit x = qkv_unit<true>(fresh.rows, b, col, i - h * per,
+                                       h <= G, Hq + 2 * num_kv_heads, Dr);
+      *reinterpret_cast<shortx4 *>(own + h * D + x.d1) = x.o1;
+      *reinterpret_cast<shortx4 *>(own + h * D + x.d2) = x.o2;
+      if (h >= G && split == 0) {
+        __hip_bfloat16 *dst =
+            (h == G ? fresh.k_cache : fresh.v_cache) +
+            (fresh.slots[b] * num_kv_heads + kvh) * Dr;
+        *reinterpret_cast<shortx4 *>(dst + x.d1) = x.o1;
+        *reinterpret_cast<shortx4 *>(dst + x.d2) = x.o2;
+      }
+    }
+    __syncthreads();
+    if (t0 >= t1) {  // (a sequence without keys)
+      for (int i = tid; i < G * Dvr; i += BLOCK)
+        out[row * out_stride + (long)kvh * G * Dvr + i] =
+            __float2bfloat16(0.f);
+      return;
+    }
+  }
+  // query fragments: column l16 = head, dims kt * 32 + lhi * 8
+  dec_bf8 qf[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    qf[kt] = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (l16 < G && kt * 32 + lhi * 8 < Dr)
+      qf[kt] =
+          FRESH ? *reinterpret_cast<const dec_bf8 *>(own + l16 * D + kt * 32 +
+                                                     lhi * 8)
+                : *reinterpret_cast<const dec_bf8 *>(
+                      q + (long)row * q_stride + (kvh * G + l16) * Dr +
+                      kt * 32 + lhi * 8);
+  }
   for (; k0 < t1; k0 += WAVES * TK) {
     DecFrag kf[2][KT];
     float bv[8];
@@ -291,6 +388,24 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
         *reinterpret_cast<shortx8 *>(&kf[f][kt]) = kn[f][kt];
+    if (FRESH && k0 + TK >= seq_len) {
+      // the new token's row comes from LDS, and so does what stands behind
+      // it in the tile (the cache's row may not be written yet)
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+          if (k0 + f * 16 + l16 >= seq_len - 1 && kt * 32 + lhi * 8 < Dr)
+            *reinterpret_cast<shortx8 *>(&kf[f][kt]) =
+                *reinterpret_cast<const shortx8 *>(own + G * D + kt * 32 +
+                                                   lhi * 8);
+#pragma unroll
+      for (int j = 0; j < VU; ++j) {
+        const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 8;
+        if (k0 + r >= seq_len - 1 && c < Dvr)
+          vn[j] = *reinterpret_cast<const shortx8 *>(own + (G + 1) * D + c);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < VU; ++j) {
       const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 16;
@@ -372,6 +487,8 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) mo[(nt * 4 + r) * 64 + lane] = o[nt][r];
   __syncthreads();
+  // workgroups that have keys of this sequence (one: it writes the result)
+  const int live = (tiles * TK + split_len - 1) / split_len;
   for (int idx = tid; idx < G * Dvr; idx += BLOCK) {
     const int h = idx / Dvr, d = idx % Dvr;
     const int at = ((d >> 4) * 4 + (d & 3)) * 64 + ((d >> 2) & 3) * 16 + h;
@@ -385,7 +502,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
       l += e * s_l[w][h];
       acc += e * reinterpret_cast<const float *>(patch[w])[at];
     }
-    if (out) {  // the only split
+    if (FRESH ? live == 1 : out != nullptr) {  // the only split
       if (sinks || sink)
         l += __builtin_amdgcn_exp2f(
             (sinks ? sinks[kvh * G + h] : 0.f) * LOG2E - m);
@@ -397,8 +514,43 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
       out[row * out_stride + col] = __float2bfloat16(res);
       continue;
     }
-    partial_out[(lse0 + h) * Dvr + d] = acc / l;
-    if (d == 0) partial_lse[lse0 + h] = m / LOG2E + __logf(l);
+    const float lse = m / LOG2E + __logf(l);
+    if constexpr (FRESH) {
+      publish(&partial_out[(lse0 + h) * Dvr + d], acc / l);
+      if (d == 0) publish(&partial_lse[lse0 + h], lse);
+    } else {
+      partial_out[(lse0 + h) * Dvr + d] = acc / l;
+      if (d == 0) partial_lse[lse0 + h] = lse;
+    }
+  }
+  if constexpr (FRESH) {
+    if (live == 1) return;
+    // Every wave's partials are where all dies see them before the count
+    // goes up, and they are read there (a fence here would empty the L2 that
+    // the other workgroups' keys pass through: 24 of 5400 keys in four splits
+    // 30 us a launch).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int *last = reinterpret_cast<int *>(&s_m[0][0]);
+    if (tid == 0) {
+      int *at = fresh.arrived + b * num_kv_heads + kvh;
+      const int before = __hip_atomic_fetch_add(at, 1, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+      *last = before == live - 1;
+      if (before == live - 1)
+        __hip_atomic_store(at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*last) return;
+    const long of_split = (long)B * Hq;
+    for (int idx = tid; idx < G * Dvr; idx += BLOCK) {
+      const int h = idx / Dvr, d = idx % Dvr;
+      const long at = (long)b * Hq + kvh * G + h;
+      out[row * out_stride + (long)(kvh * G + h) * Dvr + d] =
+          __float2bfloat16(merged<true>(partial_out + at * Dvr + d,
+                                  of_split * Dvr, partial_lse + at, of_split,
+                                  live, -INFINITY));
+    }
   }
 }
 
@@ -417,22 +569,12 @@ __global__ void decode_merge_kernel(
   if (qsl && qsl[b + 1] - row != 1) return;
   const int d = threadIdx.x, D = blockDim.x;
   const int B = gridDim.x;
-  // sink: one more "partial" with lse 0 (or the head's learned score)
-  // and no value
-  const float sk = sinks ? sinks[h] : 0.f;
-  sink = sink || sinks != nullptr;
-  float mx = sink ? sk : -INFINITY;
-  for (int s = 0; s < num_splits; ++s)
-    mx = fmaxf(mx, partial_lse[((long)s * B + b) * Hq + h]);
-  float denom = sink ? __expf(sk - mx) : 0.f, o = 0.f;
-  for (int s = 0; s < num_splits; ++s) {
-    const float lse = partial_lse[((long)s * B + b) * Hq + h];
-    if (lse == -INFINITY) continue;
-    const float w = __expf(lse - mx);
-    denom += w;
-    o += w * partial_out[(((long)s * B + b) * Hq + h) * D + d];
-  }
-  float res = denom > 0.f ? o / denom : 0.f;
+  // sink: one more "partial" with lse 0 (or the head's learned score) and no
+  // value
+  const long at = (long)b * Hq + h, of_split = (long)B * Hq;
+  float res = merged<false>(partial_out + at * D + d, of_split * D, partial_lse + at,
+                     of_split, num_splits,
+                     sinks ? sinks[h] : sink ? 0.f : -INFINITY);
   if (gate != nullptr) {
     const float z =
         __bfloat162float(gate[(long)row * gate_stride + (long)h * D + d]);
@@ -452,20 +594,9 @@ bool decode_shape_ok(const torch::Tensor &k_cache,
          reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 16 == 0;
 }
 
-void launch_decode(torch::Tensor &out, const torch::Tensor &q,
-                   const torch::Tensor &k_cache, const torch::Tensor &v_cache,
-                   const torch::Tensor &block_table,
-                   const torch::Tensor &seq_lens, int G, float scale,
-                   int window, int keep_first = 0, bool sink = false,
-                   const void *gate = nullptr, long gate_stride = 0,
-                   const float *sinks = nullptr, float softcap = 0.f,
-                   const float *bias = nullptr, int bias_len = 0,
-                   float temp_coef = 0.f, int temp_every = 0,
-                   const int *qsl = nullptr) {
-  // (lengths past a step's own rows are not looked at)
-  const int B = qsl ? seq_lens.size(0) : q.size(0);
-  const int Hkv = k_cache.size(2), Hq = Hkv * G;
-  const int D = k_cache.size(3), Dv = v_cache.size(3);
+// Workgroups that share the keys of one sequence and kv head.
+int splits_for(const torch::Tensor &k_cache, long B) {
+  const long Hkv = k_cache.size(2);
   // the longest sequence the pool can hold bounds the useful splits; the
   // count depends on the batch size only (a captured launch serves every
   // length)
@@ -488,6 +619,26 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
          splits * 2 <= (max_seq_len + 127) / 128)
     splits *= 2;
   if (splits_env > 0) splits = splits_env;
+  return splits;
+}
+
+void launch_decode(torch::Tensor &out, const torch::Tensor &q,
+                   const torch::Tensor &k_cache, const torch::Tensor &v_cache,
+                   const torch::Tensor &block_table,
+                   const torch::Tensor &seq_lens, int G, float scale,
+                   int window, int keep_first = 0, bool sink = false,
+                   const void *gate = nullptr, long gate_stride = 0,
+                   const float *sinks = nullptr, float softcap = 0.f,
+                   const float *bias = nullptr, int bias_len = 0,
+                   float temp_coef = 0.f, int temp_every = 0,
+                   const int *qsl = nullptr,
+                   const NewRows *fresh = nullptr) {
+  // (lengths past a step's own rows are not looked at; q: the result's
+  // tensor where the rows are fresh)
+  const int B = qsl ? seq_lens.size(0) : q.size(0);
+  const int Hkv = k_cache.size(2), Hq = Hkv * G;
+  const int D = k_cache.size(3), Dv = v_cache.size(3);
+  const int splits = splits_for(k_cache, B);
   auto opts = q.options().dtype(at::kFloat);
   // + 1: the kept-first segment of a windowed layer
   const int zdim = splits + ((keep_first > 0 && window > 0) ? 1 : 0);
@@ -502,14 +653,14 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
     lse = torch::empty({zdim, B, Hq}, opts);
     po = partial.data_ptr<float>();
     pl = lse.data_ptr<float>();
-    direct = nullptr;
+    if (!fresh) direct = nullptr;
   }
   const bool few = B <= 64 && B * Hkv * zdim <= ORDERED / 2;
   const int order_above = (few ? SHARE_FEW : SHARE) / (D + Dv) * splits;
   auto stream = at::cuda::getCurrentCUDAStream();
-#define RUN(DT, DVT)                                                         \
-  hipLaunchKernelGGL((paged_decode_kernel<DT, DVT>), dim3(B * Hkv * zdim),   \
-                     dim3(BLOCK), 0, stream, po, pl,                         \
+#define RUN(...)                                                             \
+  hipLaunchKernelGGL((paged_decode_kernel<__VA_ARGS__>),                     \
+                     dim3(B * Hkv * zdim), dim3(BLOCK), 0, stream, po, pl,   \
                      (const __hip_bfloat16 *)q.data_ptr(),                   \
                      (const __hip_bfloat16 *)k_cache.data_ptr(),             \
                      (const __hip_bfloat16 *)v_cache.data_ptr(),             \
@@ -519,12 +670,13 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      keep_first, softcap, bias, bias_len, temp_coef,         \
                      temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
                      sinks, (const __hip_bfloat16 *)gate, gate_stride, B,    \
-                     zdim, order_above)
-  if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
+                     zdim, order_above, fresh ? *fresh : NewRows{})
+  if (fresh) { if (D <= 64) RUN(64, 64, true); else RUN(128, 128, true); }
+  else if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
 #undef RUN
   HIP_CHECK_KERNEL();
-  if (zdim == 1) return;
+  if (zdim == 1 || fresh) return;
   hipLaunchKernelGGL(decode_merge_kernel, dim3(B, Hq), dim3(Dv), 0, stream,
                      (__hip_bfloat16 *)out.data_ptr(), out_stride, po, pl,
                      zdim, Hq, sink ? 1 : 0, (const __hip_bfloat16 *)gate,
@@ -565,6 +717,88 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
   launch_decode(out, q, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
                 (float)scale, (int)sliding_window, 0, false, nullptr, 0,
                 nullptr, 0.f, nullptr, 0, 0.f, 0, qsl);
+}
+
+bool decode_rows_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq);
+
+// One decode token per sequence from the fp32 parts [S, B, (Hq + 2 Hkv) D] of
+// the merged q | k | v projection: bias, rotation (rotate-half on the first
+// rot columns), keys and values to their slots, which must be the last of
+// their sequence's (block table, length), and attention, in one launch;
+// bf16 [B, Hq * D]. rounded: the biased rows are rounded to bf16 first.
+// arrived: int32 zeros, one per sequence and kv head, left as zeros; launches
+// that may overlap need their own.
+torch::Tensor qkv_decode(torch::Tensor parts,
+                         c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, torch::Tensor block_table,
+                         torch::Tensor seq_lens, torch::Tensor arrived,
+                         long Hq, double scale, long sliding_window,
+                         bool rounded) {
+  const long B = parts.size(1), Hkv = k_cache.size(2), D = k_cache.size(3);
+  const int rot = cos_sin.size(-1);
+  TORCH_CHECK(parts.is_cuda() && parts.dim() == 3 && parts.is_contiguous() &&
+              parts.scalar_type() == at::kFloat &&
+              reinterpret_cast<uintptr_t>(parts.data_ptr()) % 16 == 0 &&
+              parts.size(2) == (Hq + 2 * Hkv) * D,
+              "qkv_decode: fp32 parts [S, B, (Hq + 2 Hkv) D]");
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.is_contiguous() &&
+              v_cache.is_contiguous() && v_cache.sizes() == k_cache.sizes() &&
+              k_cache.scalar_type() == at::kBFloat16 &&
+              v_cache.scalar_type() == at::kBFloat16 && Hq > 0 &&
+              Hq % Hkv == 0 && decode_shape_ok(k_cache, v_cache, Hq / Hkv),
+              "qkv_decode: unsupported head_dim=", D, " group=", Hq / Hkv);
+  TORCH_CHECK(rot % 8 == 0 && rot <= D &&
+              cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous());
+  TORCH_CHECK(positions.scalar_type() == at::kLong &&
+              positions.is_contiguous() && positions.numel() == B &&
+              slots.scalar_type() == at::kLong && slots.is_contiguous() &&
+              slots.numel() == B);
+  TORCH_CHECK(block_table.scalar_type() == at::kInt &&
+              block_table.size(0) >= B && block_table.stride(1) == 1 &&
+              seq_lens.scalar_type() == at::kInt &&
+              seq_lens.is_contiguous() && seq_lens.numel() >= B);
+  TORCH_CHECK(arrived.is_cuda() && arrived.scalar_type() == at::kInt &&
+              arrived.is_contiguous() && arrived.numel() >= B * Hkv,
+              "qkv_decode: a zero per sequence and kv head");
+  const __hip_bfloat16 *bp = nullptr;
+  if (bias.has_value()) {
+    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 &&
+                bias->is_contiguous() && bias->numel() == parts.size(2));
+    bp = (const __hip_bfloat16 *)bias->data_ptr();
+  }
+  auto out = torch::empty({B, Hq * D}, k_cache.options());
+  if (B == 0) return out;
+  const NewRows fresh{{parts.data_ptr(), 0L, bp, positions.data_ptr<long>(),
+                       cos_sin.data_ptr<float>(), (int)B,
+                       (int)parts.size(0), rot, (int)rounded},
+                      (__hip_bfloat16 *)k_cache.data_ptr(),
+                      (__hip_bfloat16 *)v_cache.data_ptr(),
+                      slots.data_ptr<long>(), arrived.data_ptr<int>()};
+  launch_decode(out, out, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
+                (float)scale, (int)sliding_window, 0, false, nullptr, 0,
+                nullptr, 0.f, nullptr, 0, 0.f, 0, nullptr, &fresh);
+  return out;
+}
+
+// Whether qkv_decode takes heads of this geometry, and is the faster form: its
+// rows cost each workgroup a few us, which pays while all of them are on the
+// chip at once (in two rounds if none waits for another's partials). (us of an
+// attention step, 40 heads on 8 of 128, two kernels or
+// three / this one: 1 sequence of 600 keys 13.2 / 12.6, 2 of 2400 19.8 / 17.5,
+// 16 of 340 to 880 21.4 / 20.1, 32 of 520 to 1500 41.5 / 39.5, 64 of them 64.4
+// / 61.4, 128 112.5 / 109.3, 64 of 150 to 450 27.8 / 25.7; 14 on 2 of 64, 64 of
+// 520 to 1500 18.7 / 16.9. Beyond: 48 of 520 to 1500 in two splits 60.4 / 61.6, 24 of 2700 to
+// 7900 in four 117.9 / 122.6, 256 of 150 to 450 74.6 / 77.9.)
+bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
+                   long B) {
+  const long Hkv = k_cache.size(2);
+  const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+  const int splits = splits_for(k_cache, B);
+  return decode_rows_ok(k_cache, v_cache, Hq) &&
+         k_cache.sizes() == v_cache.sizes() &&
+         B * Hkv * splits <= (splits > 1 ? 2L : 4L) * cus;
 }
 
 // whether the decode kernel takes heads of this geometry (a mixed batch

@@ -30,6 +30,16 @@ torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w);
 torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
                               torch::Tensor residual, torch::Tensor norm_w,
                               double eps);
+bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
+                   long B);
+torch::Tensor qkv_decode(torch::Tensor parts,
+                         c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, torch::Tensor block_table,
+                         torch::Tensor seq_lens, torch::Tensor arrived,
+                         long Hq, double scale, long sliding_window,
+                         bool rounded);
 torch::Tensor qkv_finish(torch::Tensor src, c10::optional<torch::Tensor> bias,
                          torch::Tensor positions, torch::Tensor cos_sin,
                          torch::Tensor k_cache, torch::Tensor v_cache,
@@ -197,6 +207,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_parts", &stream_parts, "fp32 parts of x w^T");
   m.def("stream_add_norm", &stream_add_norm,
         "residual += x w^T; RMS norm of it");
+  m.def("qkv_decode_ok", &qkv_decode_ok);
+  m.def("qkv_decode", &qkv_decode,
+        "bias, rotation, cache and decode attention of projection parts");
   m.def("qkv_finish", &qkv_finish,
         "bias, rotation, keys and values to the cache; queries");
   m.def("mla_paged_attention", &mla_paged_attention,

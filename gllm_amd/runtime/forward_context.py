@@ -68,6 +68,19 @@ class ForwardContext:
     _per_head_from: Optional[tuple] = dataclasses.field(default=None,
                                                         kw_only=True)
 
+    _arrivals: Optional[torch.Tensor] = dataclasses.field(default=None,
+                                                          kw_only=True)
+
+    def arrivals(self, kv_heads: int) -> torch.Tensor:
+        """Zeros that this forward's split decode attention counts its
+        workgroups in and leaves as zeros (its layers follow one another; a
+        captured forward keeps its own)."""
+        n = self.seq_lens.shape[0] * kv_heads
+        if self._arrivals is None or self._arrivals.numel() < n:
+            self._arrivals = torch.zeros(n, dtype=torch.int32,
+                                         device=self.seq_lens.device)
+        return self._arrivals
+
     def prompts_from(self) -> int:
         """The first sequence from which on all are whole prompts: two rows
         or more and nothing in the cache (their number if there are none)."""

@@ -56,6 +56,8 @@ class GraphRunner:
         self.buckets = [b for b in DECODE_BUCKETS if b <= cfg.max_graph_bs]
         self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self.hidden_out: Dict[int, torch.Tensor] = {}
+        # (what a captured forward counts in must live as long as its graph)
+        self.contexts: Dict[int, ForwardContext] = {}
         self.captured = False
         self.max_bs = self.buckets[-1]
         max_len = cfg.model_max_length or 32768
@@ -165,6 +167,7 @@ class GraphRunner:
                 hidden, _ = runner.model(ids, pos, fctx)
             self.graphs[bs] = g
             self.hidden_out[bs] = hidden
+            self.contexts[bs] = fctx
 
     # ------------------------------------------------------------------
     def can_replay(self, batch) -> bool:
