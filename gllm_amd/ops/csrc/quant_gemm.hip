@@ -27,12 +27,21 @@
 // the parts round the sums to bf16 before they go on, and a fused product
 // gives what the separate one gives.
 //
+// int4 with 17 rows and more is bound by what its waves do in turn: a stage's
+// LDS reads, vector instructions (unpacking 7 per 8 weights, reordering the
+// rows 4 per 8 values, scales) and products are 0.5, 0.75 and 0.5 us, and the
+// stage takes 2. With a group per wave of a pair (WK) the rows are read,
+// reordered and summed by half as many waves. (us, 29 rows, 8 waves along the
+// columns / this: 55296 x 5120 gated 45.9 / 41.1, 5120 x 27648 26.1 / 22.5,
+// 7168 x 5120 10.3 / 9.3; 64 rows 67.5 / 58.9, 38.1 / 34.5, 22.7 / 21.7; 1 row
+// 37.2 / 32.3, 19.2 / 17.8. Sixteen waves 40.8 / 23.2; three stages 42.2 /
+// 23.9.)
+//
 // (us, 29 rows; the kernels before these formed floats weight by weight and
-// did not fill the chip:) 55296 x 5120 int4 45, fp8 46 gated; 5120 x 27648 25
-// and 31; four products of a 5120-wide layer 89 (210) and 99. Weights come
-// at 4.1 (int4, 1 row) and 6.3 TB/s (fp8); int4 with 17 rows and more is
-// bound by its vector instructions. (int4 with a look at each group's row sum
-// in the loop: 49 and 26.)
+// did not fill the chip:) fp8 55296 x 5120 gated 46, 5120 x 27648 31; four
+// products of a 5120-wide layer 99, int4 81 (210). Weights come at 4.5 (int4,
+// 1 row) and 6.3 TB/s (fp8). (int4 with a look at each group's row sum in the
+// loop takes 7 % longer.)
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -169,15 +178,19 @@ DEV_INLINE void store_tile(void *C, const qg_f4 (&acc)[NT][MT],
   }
 }
 
-// WM x WN waves share a BM x BN tile; a ring of ST stages of 128 columns
-template <int Q, int BM, int BN, int WM, int WN, int ST, int FORM>
-__global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
+// WM x WN waves share a BM x BN tile; a ring of ST stages of 128 columns (256
+// for int4). WK 2 (int4): as many waves again, each of a pair takes one of a
+// stage's two groups and twice the columns, and their sums are joined at the
+// end: the rows, which every wave reads, reorders and sums for itself, are
+// then half the work.
+template <int Q, int BM, int BN, int WM, int WN, int ST, int FORM, int WK = 1>
+__global__ __launch_bounds__(WM *WN *WK * 64, 2) void quant_gemm_kernel(
     void *__restrict__ C,  // bf16 [M, N or N / 2], PART: fp32 [S, M, N]
     const char *__restrict__ X, const float *__restrict__ XS,
     const char *__restrict__ W, const float *__restrict__ WS,
     const float *__restrict__ bias, int M, int N, int K, int k_slice,
     int nbm, int nbn) {
-  constexpr int WAVES = WM * WN;
+  constexpr int WAVES = WM * WN * WK;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
   // LDS row bytes; 128 of a weight row at once in either form (64 B pieces of
   // it come at half the rate)
@@ -195,6 +208,8 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
   constexpr int W_OFF = BM * XROW, S_OFF = W_OFF + BN * WROW;
   constexpr int STAGE = S_OFF + SLOADS * 256;
   static_assert(FORM != GATED || NT % 2 == 0, "gate and up in one wave");
+  static_assert(WK == 1 || (Q == INT4 && WK == GS), "a group per wave");
+  static_assert(WK == 1 || WM * WN * NT * MT * 1024 <= ST * STAGE, "sums");
   __shared__ __attribute__((aligned(16))) char smem[ST * STAGE];
 
   // eight dies take workgroups in turn: each gets a contiguous run of tiles,
@@ -210,7 +225,7 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lhi = lane >> 4;
-  const int wm = wave / WN, wn = wave % WN;
+  const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
   const int NC = FORM == GATED ? N >> 1 : N;  // columns of C
 
   // weight row of a row of the tile
@@ -318,7 +333,8 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
           reinterpret_cast<const float *>(smem + cur * STAGE + S_OFF);
       if constexpr (Q == INT4) {
 #pragma unroll
-        for (int i = 0; i < GS; ++i) {
+        for (int g = 0; g < GS / WK; ++g) {
+          const int i = WK > 1 ? wk : g;
           qg_f4 part[NT][MT];
 #pragma unroll
           for (int n = 0; n < NT; ++n)
@@ -427,7 +443,29 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
       nxt = nxt + 1 == ST ? 0 : nxt + 1;
     }
   };
+  // The first wave of a pair ends with both sums.
+  auto join = [&]() {
+    if constexpr (WK > 1) {
+      qg_f4 *sums = reinterpret_cast<qg_f4 *>(smem) +
+                    (wave % (WM * WN)) * NT * MT * 64 + lane;
+      __syncthreads();  // the ring has been read
+      if (wk > 0) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) sums[(n * MT + m) * 64] = acc[n][m];
+      }
+      __syncthreads();
+      if (wk == 0) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[n][m] += sums[(n * MT + m) * 64];
+      }
+    }
+  };
   walk(std::false_type{});
+  join();
 
   if constexpr (Q == INT4) {
     // (16 + q) x or its sum past 32 bits leaves an infinity or a NaN, and
@@ -444,7 +482,7 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
     // waits for the ring's loads before each of its reads)
     int *again = reinterpret_cast<int *>(smem);
     __syncthreads();  // the ring has been read
-    const bool mine = __any(!finite);
+    const bool mine = wk == 0 && __any(!finite);
     if (lane == 0) again[wave] = mine;
     __syncthreads();
     int any = 0;
@@ -464,6 +502,7 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
 #pragma unroll
       for (int j = 0; j < SL; ++j) ssrc[j] -= nkt * sstep;
       walk(std::true_type{});
+      join();
 #pragma unroll
       for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -475,6 +514,7 @@ __global__ __launch_bounds__(WM *WN * 64, 2) void quant_gemm_kernel(
     }
   }
 
+  if (WK > 1 && wk > 0) return;
   store_tile<Q, NT, MT, BN, FORM>(C, acc, bias, M, N, NC, mb * BM + wm * MT * 16,
                                nb, z, wn * NT, lane);
 }
@@ -486,10 +526,13 @@ struct Plan {
 // The tile by rows and width (us, rows x N x K):
 //  * int4: up to 16 rows 64 columns, 128 where the weight is wide or deep
 //    (1 x 7168 x 5120 7.7, 128 columns 8.9; 1 x 5120 x 27648 18.9 at 128,
-//    22.1 at 64); above that 256 for wide and deep ones (29 x 55296 x 5120
-//    44.7, 128 columns 46.3; 29 x 5120 x 27648 24.5, 26.1; 64 x 55296 x 5120
-//    68.3, 79.2), else 64 (29 x 7168 x 5120 10.0, 128 columns 12.6) or, for
-//    more than 32 rows, 128 (64 x 5120 x 5120 12.1, 64 columns 16.6).
+//    22.1 at 64); above that 256 for wide and deep ones (29 x 5120 x 27648
+//    22.5, 128 columns 24.5; 64 x 28672 x 4096 31.1, 35.2), else 64 (29 x 7168
+//    x 5120 10.0, 128 columns 12.6) or, for more than 32 rows, 128 (64 x 5120
+//    x 5120 12.1, 64 columns 16.6). A gated product cannot split K: 128
+//    columns up to a tile per CU (K 4096, 32 and 64 rows, 128 / 256 columns:
+//    22016 23 / 31, 30 / 46; 32768 24 / 31, 31 / 46), 256 beyond (36864 31 /
+//    31, 56 / 46; 45056 32 / 31, 56 / 47).
 //  * fp8: up to 16 rows the same (1 x 7168 x 5120 9.2, 128 columns 10.1; 1 x
 //    28672 x 4096 22.1); above that 64 (29 x 7168 x 5120 12.4, 128 columns
 //    14), 256 from 36000 columns (64 x 55296 x 5120 51.2, 128 columns 57.4;
@@ -504,7 +547,8 @@ Plan plan_for(bool int4, int M, int N, int K, bool gated, int splits) {
   const bool wide = N >= 16384, deep = K >= 2 * N;
   p.bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   if (p.bm == 16) p.bn = gated || wide || deep ? 128 : 64;
-  else if (int4) p.bn = wide || deep ? 256 : gated || p.bm == 64 ? 128 : 64;
+  else if (int4 && gated) p.bn = N > 32768 ? 256 : 128;
+  else if (int4) p.bn = wide || deep ? 256 : p.bm == 64 ? 128 : 64;
   else p.bn = N >= 36000 ? 256 : p.bm == 64 && wide ? 128 : 64;
   p.nbm = (M + p.bm - 1) / p.bm;
   p.nbn = (N + p.bn - 1) / p.bn;
@@ -528,29 +572,30 @@ void launch(const Plan &p, bool int4, void *C, const void *X, const float *XS,
             const void *W, const float *WS, const float *bias, int M, int N,
             int K) {
   auto stream = at::cuda::getCurrentCUDAStream();
-#define RUN(Q, BM, BN, WM, WN, ST)                                           \
-  hipLaunchKernelGGL((quant_gemm_kernel<Q, BM, BN, WM, WN, ST, FORM>),       \
-                     dim3(p.nbm * p.nbn, p.splits), dim3((WM) * (WN) * 64),  \
-                     0, stream, C, (const char *)X, XS, (const char *)W, WS, \
-                     bias, M, N, K, p.k_slice, p.nbm, p.nbn)
+#define RUN(Q, BM, BN, WM, WN, ST, WK)                                       \
+  hipLaunchKernelGGL((quant_gemm_kernel<Q, BM, BN, WM, WN, ST, FORM, WK>),   \
+                     dim3(p.nbm * p.nbn, p.splits),                          \
+                     dim3((WM) * (WN) * (WK) * 64), 0, stream, C,            \
+                     (const char *)X, XS, (const char *)W, WS, bias, M, N,   \
+                     K, p.k_slice, p.nbm, p.nbn)
   if (int4) {
-    if (p.bm == 16 && p.bn == 128) RUN(INT4, 16, 128, 1, 4, 2);
-    else if (p.bm == 32 && p.bn == 256) RUN(INT4, 32, 256, 1, 8, 2);
-    else if (p.bm == 32 && p.bn == 128) RUN(INT4, 32, 128, 1, 4, 2);
-    else if (p.bm == 64 && p.bn == 256) RUN(INT4, 64, 256, 2, 4, 2);
-    else if (p.bm == 64) RUN(INT4, 64, 128, 2, 4, 2);
+    if (p.bm == 16 && p.bn == 128) RUN(INT4, 16, 128, 1, 2, 2, 2);
+    else if (p.bm == 32 && p.bn == 256) RUN(INT4, 32, 256, 1, 4, 2, 2);
+    else if (p.bm == 32 && p.bn == 128) RUN(INT4, 32, 128, 1, 2, 2, 2);
+    else if (p.bm == 64 && p.bn == 256) RUN(INT4, 64, 256, 1, 4, 2, 2);
+    else if (p.bm == 64) RUN(INT4, 64, 128, 2, 2, 2, 2);
     else if constexpr (FORM != GATED) {  // (gate and up tile in one wave)
-      if (p.bm == 16) RUN(INT4, 16, 64, 1, 4, 3);
-      else RUN(INT4, 32, 64, 1, 4, 2);
+      if (p.bm == 16) RUN(INT4, 16, 64, 1, 2, 2, 2);
+      else RUN(INT4, 32, 64, 1, 2, 2, 2);
     }
   } else {
-    if (p.bm == 16 && p.bn == 128) RUN(FP8, 16, 128, 1, 4, 4);
-    else if (p.bm == 32 && p.bn == 256) RUN(FP8, 32, 256, 1, 8, 3);
-    else if (p.bm == 32) RUN(FP8, 32, 64, 1, 2, 4);
-    else if (p.bm == 64 && p.bn == 256) RUN(FP8, 64, 256, 2, 4, 3);
-    else if (p.bm == 64 && p.bn == 128) RUN(FP8, 64, 128, 2, 4, 3);
-    else if (p.bm == 64) RUN(FP8, 64, 64, 2, 2, 3);
-    else if constexpr (FORM != GATED) RUN(FP8, 16, 64, 1, 4, 6);
+    if (p.bm == 16 && p.bn == 128) RUN(FP8, 16, 128, 1, 4, 4, 1);
+    else if (p.bm == 32 && p.bn == 256) RUN(FP8, 32, 256, 1, 8, 3, 1);
+    else if (p.bm == 32) RUN(FP8, 32, 64, 1, 2, 4, 1);
+    else if (p.bm == 64 && p.bn == 256) RUN(FP8, 64, 256, 2, 4, 3, 1);
+    else if (p.bm == 64 && p.bn == 128) RUN(FP8, 64, 128, 2, 4, 3, 1);
+    else if (p.bm == 64) RUN(FP8, 64, 64, 2, 2, 3, 1);
+    else if constexpr (FORM != GATED) RUN(FP8, 16, 64, 1, 4, 6, 1);
   }
 #undef RUN
   HIP_CHECK_KERNEL();
