@@ -54,11 +54,12 @@ class LinearBase(nn.Module):
         resident cache — prefill is compute-bound and bursty). CPU and
         int4 keep the dequant path."""
         w = self.weight
-        if not self.is_plain and self._native(x):
-            op = self._few_rows(x)
+        if not self.is_plain and self._native(ops.plain_rows(x)):
+            op = self._few_rows(ops.plain_rows(x))
             if op is not None:
                 return ops.quant_rows(x, op, self._bias32())
-            return self._prefill_quant(x, bias)
+            return self._prefill_quant(ops.plain_rows(x), bias)
+        x = ops.plain_rows(x)
         if self.fp8_block is not None:
             from gllm_amd.layers.quantization.fp8 import dequant_block_fp8
             if x.is_cuda:
@@ -115,9 +116,20 @@ class LinearBase(nn.Module):
     def _fused_op(self, x):
         """``_few_rows`` where a fused form may take this layer, else
         None."""
+        x = ops.plain_rows(x)
         if self.is_plain or x.shape[0] == 0 or not self._native(x):
             return None
         return self._few_rows(x)
+
+    def takes_fp8(self, rows) -> bool:
+        """Whether this layer quantizes as many rows to e4m3 as ``rows``
+        has: what forms them may then hand them over as
+        ``ops.Fp8Rows``."""
+        rows = ops.plain_rows(rows)
+        return (self.fp8_block == (128, 128) and rows.is_cuda
+                and rows.dim() == 2 and rows.dtype == torch.bfloat16
+                and 0 < rows.shape[0] <= 64
+                and self.weight.shape[1] % 128 == 0 and ops.has_kernels())
 
     def _bias32(self):
         """fp32 bias cached once (the skinny epilogues add fp32)."""
@@ -237,15 +249,16 @@ class MergedColumnParallelLinear(LinearBase):
     def forward(self, x):
         return self._gemm(x, self.bias)
 
-    def forward_silu(self, x):
-        """silu(gate) * up of a gate | up projection."""
+    def forward_silu(self, x, fp8=False):
+        """silu(gate) * up of a gate | up projection; ``fp8``: as
+        ``ops.Fp8Rows`` where the product can leave them."""
         if self.is_plain and self.bias is None and x.is_cuda \
                 and x.dim() == 2:
             return ops.linear_silu(x, self.weight)
         if self.bias is None:
             op = self._fused_op(x)
             if op is not None:
-                return ops.quant_silu(x, op)
+                return ops.quant_silu(x, op, fp8)
         return ops.silu_and_mul(self(x))
 
 
@@ -362,10 +375,12 @@ class RowParallelLinear(LinearBase):
     def _load_b(param, loaded):
         param.data.copy_(loaded)
 
-    def forward_add_norm(self, x, residual, norm):
+    def forward_add_norm(self, x, residual, norm, fp8=False):
         """(norm(residual + self(x)), that sum): one kernel behind the
-        product where nothing has to be reduced over ranks first."""
-        if (self.bias is None and x.is_cuda and x.dim() == 2
+        product where nothing has to be reduced over ranks first. ``fp8``:
+        the norm as ``ops.Fp8Rows`` where that kernel can leave them."""
+        rows = ops.plain_rows(x)
+        if (self.bias is None and rows.is_cuda and rows.dim() == 2
                 and (get_tp_size() == 1 or not self.reduce_results)):
             if self.is_plain:
                 return ops.linear_add_rmsnorm(x, self.weight, residual,
@@ -373,7 +388,7 @@ class RowParallelLinear(LinearBase):
             op = self._fused_op(x)
             if op is not None:
                 return ops.quant_add_rmsnorm(x, op, residual, norm.scale(),
-                                             norm.eps)
+                                             norm.eps, fp8)
         return norm(self(x), residual)
 
     def forward(self, x):

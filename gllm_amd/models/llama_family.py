@@ -40,10 +40,13 @@ class DenseMLP(nn.Module):
     def forward(self, x):
         return self.down_proj(self.gate_up_proj.forward_silu(x))
 
-    def forward_add_norm(self, x, residual, norm):
-        """(norm(residual + self(x)), that sum)."""
-        return self.down_proj.forward_add_norm(
-            self.gate_up_proj.forward_silu(x), residual, norm)
+    def forward_add_norm(self, x, residual, norm, fp8=False):
+        """(norm(residual + self(x)), that sum); ``fp8``: see
+        RowParallelLinear."""
+        down = self.down_proj
+        return down.forward_add_norm(
+            self.gate_up_proj.forward_silu(x, down.takes_fp8(x)), residual,
+            norm, fp8)
 
 
 class DenseAttention(nn.Module):
@@ -83,6 +86,7 @@ class DenseAttention(nn.Module):
 
     def heads(self, positions, hidden, fctx: ForwardContext):
         """The heads' outputs [T, heads * head_dim], before o_proj."""
+        rows, hidden = hidden, ops.plain_rows(hidden)
         if (not (self.qk_norm or fctx.is_profile_run) and hidden.is_cuda
                 and positions.dim() == 1):
             attn, rope = self.attn, self.rotary_emb
@@ -91,9 +95,9 @@ class DenseAttention(nn.Module):
             if (hidden.dtype == torch.bfloat16 and ops.qkv_rope_cache_ok(
                     k_cache, v_cache, rope.cos_sin_cache, rope.is_neox)):
                 proj, bias = self.qkv_proj, self.qkv_proj.bias
-                src = proj.parts(hidden)
+                src = proj.parts(rows)
                 if src is None:
-                    src, bias = proj.project(hidden), None
+                    src, bias = proj.project(rows), None
                 elif fctx.is_pure_decode and ops.qkv_decode_ok(
                         src, k_cache, attn.num_heads):
                     return ops.qkv_decode(
@@ -102,7 +106,8 @@ class DenseAttention(nn.Module):
                         fctx.seq_lens,
                         fctx.arrivals(attn.num_kv_heads), attn.num_heads,
                         attn.scale, attn.sliding_window,
-                        rounded=proj.fp8_block is not None)
+                        rounded=proj.fp8_block is not None,
+                        fp8=self.o_proj.takes_fp8(hidden))
                 q = ops.qkv_rope_cache(src, bias, positions,
                                        rope.cos_sin_cache, k_cache, v_cache,
                                        fctx.slot_mapping, attn.num_heads,
@@ -121,10 +126,12 @@ class DenseAttention(nn.Module):
     def forward(self, positions, hidden, fctx: ForwardContext):
         return self.o_proj(self.heads(positions, hidden, fctx))
 
-    def forward_add_norm(self, positions, hidden, residual, norm, fctx):
-        """(norm(residual + self(...)), that sum)."""
+    def forward_add_norm(self, positions, hidden, residual, norm, fctx,
+                         fp8=False):
+        """(norm(residual + self(...)), that sum); ``fp8``: see
+        RowParallelLinear."""
         return self.o_proj.forward_add_norm(
-            self.heads(positions, hidden, fctx), residual, norm)
+            self.heads(positions, hidden, fctx), residual, norm, fp8)
 
 
 class DenseDecoderLayer(nn.Module):
@@ -140,19 +147,22 @@ class DenseDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, positions, hidden, residual, fctx, normed=False,
-                next_norm=None):
+                next_norm=None, next_fp8=False):
         """``normed``: hidden is this layer's normed input already (the
         layer before was given this layer's input norm as ``next_norm``,
-        and normed its own output with it)."""
+        and normed its own output with it). ``next_fp8``: what reads
+        ``next_norm``'s output takes it as ``ops.Fp8Rows``."""
         if residual is None:
             residual = hidden
             hidden = self.input_layernorm(hidden)
         elif not normed:
             hidden, residual = self.input_layernorm(hidden, residual)
         hidden, residual = self.self_attn.forward_add_norm(
-            positions, hidden, residual, self.post_attention_layernorm, fctx)
+            positions, hidden, residual, self.post_attention_layernorm, fctx,
+            self.mlp.gate_up_proj.takes_fp8(residual))
         if next_norm is not None:
-            return self.mlp.forward_add_norm(hidden, residual, next_norm)
+            return self.mlp.forward_add_norm(hidden, residual, next_norm,
+                                             next_fp8)
         return self.mlp(hidden), residual
 
 
@@ -223,15 +233,19 @@ class LlamaFamilyForCausalLM(nn.Module):
         for li, layer in enumerate(self.layers):
             # the norm behind this layer: the next layer's, or the final
             # one (deepstack adds to the layer's own output in between)
-            nxt = None
+            nxt, more = None, {}
             if ds is None:
                 if li + 1 < len(self.layers):
                     nxt = self.layers[li + 1].input_layernorm
+                    if isinstance(layer, DenseDecoderLayer):
+                        more["next_fp8"] = self.layers[
+                            li + 1].self_attn.qkv_proj.takes_fp8(
+                                hidden_states)
                 elif self.is_last_stage:
                     nxt = self.norm
             hidden_states, residual = layer(positions, hidden_states,
                                             residual, fctx, normed=normed,
-                                            next_norm=nxt)
+                                            next_norm=nxt, **more)
             normed = nxt is not None
             if ds is not None:
                 # Qwen3-VL deepstack: level li of the multiscale vision

@@ -13,7 +13,7 @@ through here. Dispatch rule:
 """
 
 import functools
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -389,18 +389,34 @@ def _quant_splitk(N: int, K: int, bk: int) -> int:
 
 def _quant_gemm(x: torch.Tensor, kind: str, w: torch.Tensor,
                 ws: torch.Tensor, bias, form: int) -> torch.Tensor:
-    splits = _quant_splitk(w.shape[0], x.shape[1], 128) \
+    splits = _quant_splitk(w.shape[0], plain_rows(x).shape[1], 128) \
         if kind == "fp8" else 0
     return _gpu_kernels().quant_gemm(*_quant_operands(x, kind, w, ws), bias,
                                      form, splits)
 
 
-def _quant_operands(x: torch.Tensor, kind: str, w: torch.Tensor,
-                    ws: torch.Tensor):
+class Fp8Rows(NamedTuple):
+    """bf16 rows with the e4m3 bytes and scales [columns / 128, rows] that
+    an fp8 product takes of them, from the kernel that formed the rows
+    (``per_token_group_quant_fp8`` would give the same)."""
+    x: torch.Tensor
+    q: torch.Tensor
+    scales: torch.Tensor
+
+
+def plain_rows(x):
+    """The tensor of rows that may be ``Fp8Rows``."""
+    return x.x if isinstance(x, Fp8Rows) else x
+
+
+def _quant_operands(x, kind: str, w: torch.Tensor, ws: torch.Tensor):
     """(rows, their scales, weight bytes, weight scales) as
     csrc/quant_gemm.hip takes them; ``kind`` "fp8" (w [N, K] e4m3, ws fp32
     per 128 x 128 block; the rows are quantized per 128 columns) or "int4"
     (w [N, K / 2] packed, ws [K / 128, 2, N])."""
+    if kind == "fp8" and isinstance(x, Fp8Rows):
+        return x.q, x.scales, w.view(torch.uint8), ws.contiguous()
+    x = plain_rows(x)
     if kind == "fp8":
         xq, _, xs = per_token_group_quant_fp8(x, transposed=True)
         return xq.view(torch.uint8), xs, w.view(torch.uint8), ws.contiguous()
@@ -415,13 +431,18 @@ def quant_rows(x: torch.Tensor, op, bias: Optional[torch.Tensor] = None):
         x, *op, bias.float().contiguous() if bias is not None else None, 1)
 
 
-def quant_silu(x: torch.Tensor, op) -> torch.Tensor:
+def quant_silu(x, op, fp8: bool = False):
     """silu(x @ w_gate.T) * (x @ w_up.T), w = gate rows over up rows. The
     one-kernel form cannot split K, so it is for weights with tiles enough
     without (28672 x 4096, 1 row, int4: 25 us against 20 + the second
-    kernel's 5)."""
+    kernel's 5). ``fp8``: as ``Fp8Rows`` where the product can leave
+    them."""
     N = op[1].shape[0]
     if N % 32 == 0 and N >= 16384:
+        if fp8 and op[0] == "fp8":
+            out = _gpu_kernels().quant_gemm_gated_fp8(
+                *_quant_operands(x, *op))
+            return Fp8Rows(*out) if len(out) == 3 else out[0]
         return _quant_gemm(x, *op, None, 0)
     return silu_and_mul(quant_rows(x, op))
 
@@ -434,10 +455,15 @@ def quant_parts(x: torch.Tensor, op) -> Optional[torch.Tensor]:
     return _quant_gemm(x, *op, None, 2)
 
 
-def quant_add_rmsnorm(x: torch.Tensor, op, residual: torch.Tensor,
-                      norm_w: torch.Tensor, eps: float):
-    """residual += x @ dequant(w).T; (rmsnorm(residual), residual)."""
+def quant_add_rmsnorm(x, op, residual: torch.Tensor, norm_w: torch.Tensor,
+                      eps: float, fp8: bool = False):
+    """residual += x @ dequant(w).T; (rmsnorm(residual), residual).
+    ``fp8``: the norm as ``Fp8Rows`` where its kernel can leave them."""
     if _norm_parts_ok(op[1].shape[0], residual, norm_w):
+        if fp8 and op[1].shape[0] % 128 == 0:
+            return Fp8Rows(*_gpu_kernels().parts_add_norm_fp8(
+                quant_parts(x, op), residual, norm_w, eps,
+                op[0] == "fp8")), residual
         return _gpu_kernels().parts_add_norm(quant_parts(x, op), residual,
                                              norm_w, eps,
                                              op[0] == "fp8"), residual
@@ -1117,17 +1143,20 @@ def qkv_decode(parts: torch.Tensor, bias, positions: torch.Tensor,
                v_cache: torch.Tensor, slot_mapping: torch.Tensor,
                block_table: torch.Tensor, seq_lens: torch.Tensor,
                arrived: torch.Tensor, num_heads: int, scale: float,
-               sliding_window: int = 0,
-               rounded: bool = False) -> torch.Tensor:
+               sliding_window: int = 0, rounded: bool = False,
+               fp8: bool = False):
     """``qkv_rope_cache`` and the decode attention behind it, one token per
     sequence, as one kernel; the heads' outputs [B, heads * D]. Each slot is
     the last of its sequence. ``arrived``: int32 zeros, one per sequence and
     kv head, that are zeros again behind the launch (launches that may run
-    at the same time need their own)."""
-    return _gpu_kernels().qkv_decode(
-        parts, bias, positions, cos_sin, k_cache, v_cache, slot_mapping,
-        block_table, seq_lens, arrived, num_heads, scale, sliding_window,
-        rounded)
+    at the same time need their own). ``fp8``: as ``Fp8Rows`` where a head
+    is a group of 128."""
+    args = (parts, bias, positions, cos_sin, k_cache, v_cache, slot_mapping,
+            block_table, seq_lens, arrived, num_heads, scale, sliding_window,
+            rounded)
+    if fp8 and k_cache.shape[3] == 128:
+        return Fp8Rows(*_gpu_kernels().qkv_decode_fp8(*args))
+    return _gpu_kernels().qkv_decode(*args)
 
 
 # --------------------------------------------------------------- layer norm

@@ -43,6 +43,7 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <cstdlib>
 #include "common.h"
+#include "fp8_rows.h"
 #include "qkv_rows.h"
 
 namespace {
@@ -126,6 +127,7 @@ struct NewRows {
   __hip_bfloat16 *k_cache, *v_cache;
   const long *slots;               // [B] where its key and value go
   int *arrived;                    // [B, Hkv] zeros, left as zeros
+  Fp8Out fp8;                      // the result's e4m3 rows (heads of 128)
 };
 
 // partials pass from one workgroup to another within a launch: written
@@ -359,9 +361,15 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     }
     __syncthreads();
     if (t0 >= t1) {  // (a sequence without keys)
-      for (int i = tid; i < G * Dvr; i += BLOCK)
+      for (int i = tid; i < G * Dvr; i += BLOCK) {
         out[row * out_stride + (long)kvh * G * Dvr + i] =
             __float2bfloat16(0.f);
+        if (fresh.fp8.q)
+          fresh.fp8.q[row * (long)Hq * Dvr + kvh * G * Dvr + i] = 0;
+        if (fresh.fp8.q && i % 128 == 0)
+          fresh.fp8.scales[(long)(kvh * G + i / 128) * B + row] =
+              fp8_scale(0.f);
+      }
       return;
     }
   }
@@ -487,6 +495,34 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) mo[(nt * 4 + r) * 64 + lane] = o[nt][r];
   __syncthreads();
+  // FRESH: what is written, in LDS for its e4m3 form (a head is a group)
+  auto keep = [&](int idx, __hip_bfloat16 v) {
+    if (FRESH && fresh.fp8.q) own[idx] = __builtin_bit_cast(short, v);
+  };
+  auto write_fp8 = [&]() {
+    if constexpr (FRESH && DV == 128) {
+      if (!fresh.fp8.q) return;
+      __syncthreads();
+      for (int h = wave; h < G; h += WAVES) {
+        float v[2], amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          v[i] = __bfloat162float(
+              __builtin_bit_cast(__hip_bfloat16, own[h * 128 + lane * 2 + i]));
+          amax = fmaxf(amax, fabsf(v[i]));
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+          amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        const float scale = fp8_scale(amax), inv = 1.f / scale;
+        const long head = kvh * G + h;
+        *reinterpret_cast<unsigned short *>(
+            fresh.fp8.q + ((long)row * Hq + head) * 128 + lane * 2) =
+            fp8_byte(v[0] * inv) | fp8_byte(v[1] * inv) << 8;
+        if (lane == 0) fresh.fp8.scales[head * B + row] = scale;
+      }
+    }
+  };
   // workgroups that have keys of this sequence (one: it writes the result)
   const int live = (tiles * TK + split_len - 1) / split_len;
   for (int idx = tid; idx < G * Dvr; idx += BLOCK) {
@@ -511,7 +547,9 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
       if (gate)
         res *= 1.f / (1.f + __expf(-__bfloat162float(
                                  gate[row * gate_stride + col])));
-      out[row * out_stride + col] = __float2bfloat16(res);
+      const __hip_bfloat16 r = __float2bfloat16(res);
+      out[row * out_stride + col] = r;
+      keep(idx, r);
       continue;
     }
     const float lse = m / LOG2E + __logf(l);
@@ -524,7 +562,10 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     }
   }
   if constexpr (FRESH) {
-    if (live == 1) return;
+    if (live == 1) {
+      write_fp8();
+      return;
+    }
     // Every wave's partials are where all dies see them before the count
     // goes up, and they are read there (a fence here would empty the L2 that
     // the other workgroups' keys pass through: 24 of 5400 keys in four splits
@@ -546,11 +587,13 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     for (int idx = tid; idx < G * Dvr; idx += BLOCK) {
       const int h = idx / Dvr, d = idx % Dvr;
       const long at = (long)b * Hq + kvh * G + h;
-      out[row * out_stride + (long)(kvh * G + h) * Dvr + d] =
-          __float2bfloat16(merged<true>(partial_out + at * Dvr + d,
-                                  of_split * Dvr, partial_lse + at, of_split,
-                                  live, -INFINITY));
+      const __hip_bfloat16 r = __float2bfloat16(
+          merged<true>(partial_out + at * Dvr + d, of_split * Dvr,
+                       partial_lse + at, of_split, live, -INFINITY));
+      out[row * out_stride + (long)(kvh * G + h) * Dvr + d] = r;
+      keep(idx, r);
     }
+    write_fp8();
   }
 }
 
@@ -728,14 +771,12 @@ bool decode_rows_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq);
 // bf16 [B, Hq * D]. rounded: the biased rows are rounded to bf16 first.
 // arrived: int32 zeros, one per sequence and kv head, left as zeros; launches
 // that may overlap need their own.
-torch::Tensor qkv_decode(torch::Tensor parts,
-                         c10::optional<torch::Tensor> bias,
-                         torch::Tensor positions, torch::Tensor cos_sin,
-                         torch::Tensor k_cache, torch::Tensor v_cache,
-                         torch::Tensor slots, torch::Tensor block_table,
-                         torch::Tensor seq_lens, torch::Tensor arrived,
-                         long Hq, double scale, long sliding_window,
-                         bool rounded) {
+static torch::Tensor decode_rows(
+    torch::Tensor parts, c10::optional<torch::Tensor> bias,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor k_cache,
+    torch::Tensor v_cache, torch::Tensor slots, torch::Tensor block_table,
+    torch::Tensor seq_lens, torch::Tensor arrived, long Hq, double scale,
+    long sliding_window, bool rounded, const Fp8Out &fp8) {
   const long B = parts.size(1), Hkv = k_cache.size(2), D = k_cache.size(3);
   const int rot = cos_sin.size(-1);
   TORCH_CHECK(parts.is_cuda() && parts.dim() == 3 && parts.is_contiguous() &&
@@ -775,11 +816,44 @@ torch::Tensor qkv_decode(torch::Tensor parts,
                        (int)parts.size(0), rot, (int)rounded},
                       (__hip_bfloat16 *)k_cache.data_ptr(),
                       (__hip_bfloat16 *)v_cache.data_ptr(),
-                      slots.data_ptr<long>(), arrived.data_ptr<int>()};
+                      slots.data_ptr<long>(), arrived.data_ptr<int>(), fp8};
   launch_decode(out, out, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
                 (float)scale, (int)sliding_window, 0, false, nullptr, 0,
                 nullptr, 0.f, nullptr, 0, 0.f, 0, nullptr, &fresh);
   return out;
+}
+
+torch::Tensor qkv_decode(torch::Tensor parts,
+                         c10::optional<torch::Tensor> bias,
+                         torch::Tensor positions, torch::Tensor cos_sin,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor slots, torch::Tensor block_table,
+                         torch::Tensor seq_lens, torch::Tensor arrived,
+                         long Hq, double scale, long sliding_window,
+                         bool rounded) {
+  return decode_rows(parts, bias, positions, cos_sin, k_cache, v_cache, slots,
+                     block_table, seq_lens, arrived, Hq, scale,
+                     sliding_window, rounded, Fp8Out{});
+}
+
+// ... with the result's e4m3 rows (heads of 128): {bf16, bytes, scales}
+std::vector<torch::Tensor> qkv_decode_fp8(
+    torch::Tensor parts, c10::optional<torch::Tensor> bias,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor k_cache,
+    torch::Tensor v_cache, torch::Tensor slots, torch::Tensor block_table,
+    torch::Tensor seq_lens, torch::Tensor arrived, long Hq, double scale,
+    long sliding_window, bool rounded) {
+  TORCH_CHECK(parts.dim() == 3 && k_cache.dim() == 4 && k_cache.size(3) == 128,
+              "qkv_decode_fp8: heads of 128");
+  const long B = parts.size(1);
+  auto q = torch::empty({B, Hq * 128}, k_cache.options().dtype(at::kByte));
+  auto st = torch::empty({Hq, B}, k_cache.options().dtype(at::kFloat));
+  auto out = decode_rows(parts, bias, positions, cos_sin, k_cache, v_cache,
+                         slots, block_table, seq_lens, arrived, Hq, scale,
+                         sliding_window, rounded,
+                         Fp8Out{q.data_ptr<unsigned char>(),
+                                st.data_ptr<float>()});
+  return {out, q, st};
 }
 
 // Whether qkv_decode takes heads of this geometry, and is the faster form: its

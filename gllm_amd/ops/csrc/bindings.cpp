@@ -128,6 +128,20 @@ torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
                          torch::Tensor w, torch::Tensor ws,
                          c10::optional<torch::Tensor> bias, long form,
                          long splits);
+std::vector<torch::Tensor> quant_gemm_gated_fp8(torch::Tensor x,
+                                                torch::Tensor xs,
+                                                torch::Tensor w,
+                                                torch::Tensor ws);
+std::vector<torch::Tensor> parts_add_norm_fp8(torch::Tensor part,
+                                              torch::Tensor residual,
+                                              torch::Tensor norm_w,
+                                              double eps, bool rounded);
+std::vector<torch::Tensor> qkv_decode_fp8(
+    torch::Tensor parts, c10::optional<torch::Tensor> bias,
+    torch::Tensor positions, torch::Tensor cos_sin, torch::Tensor k_cache,
+    torch::Tensor v_cache, torch::Tensor slots, torch::Tensor block_table,
+    torch::Tensor seq_lens, torch::Tensor arrived, long Hq, double scale,
+    long sliding_window, bool rounded);
 torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
                              torch::Tensor norm_w, double eps,
                              bool rounded);
@@ -239,6 +253,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "block-scale fp8 grouped MoE GEMM");
   m.def("quant_gemm", &quant_gemm,
         "few-row product with int4 or block-scale fp8 weights");
+  m.def("quant_gemm_gated_fp8", &quant_gemm_gated_fp8,
+        "gated fp8 product with its e4m3 rows");
+  m.def("parts_add_norm_fp8", &parts_add_norm_fp8,
+        "parts_add_norm with its e4m3 rows");
+  m.def("qkv_decode_fp8", &qkv_decode_fp8,
+        "qkv_decode with its e4m3 rows");
   m.def("parts_add_norm", &parts_add_norm,
         "residual += sum of fp32 parts, RMS norm of it");
   m.def("moe_gemm_int4", &moe_gemm_int4,

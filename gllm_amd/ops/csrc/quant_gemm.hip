@@ -47,6 +47,7 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <type_traits>
 #include "common.h"
+#include "fp8_rows.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 qg_bf8;
 typedef __attribute__((ext_vector_type(4))) float qg_f4;
@@ -178,6 +179,56 @@ DEV_INLINE void store_tile(void *C, const qg_f4 (&acc)[NT][MT],
   }
 }
 
+// The e4m3 rows of a gated tile of 256 columns, which leaves 128, a group, of
+// each row; `most` (LDS): [WN][BM].
+template <int NT, int MT, int WN, int BM>
+DEV_INLINE void store_fp8(const Fp8Out &out, const qg_f4 (&acc)[NT][MT],
+                          float *most, int M, int NC, int row0, int wrow0,
+                          int nb, int wn, int lane) {
+  const int l16 = lane & 15, lhi = lane >> 4;
+  float v[NT / 2][MT][4], amax[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    amax[m] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; n += 2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // (as store_tile forms and rounds them)
+        const float g = __bfloat162float(__float2bfloat16(acc[n][m][r]));
+        const float u = __bfloat162float(__float2bfloat16(acc[n + 1][m][r]));
+        const float x = __bfloat162float(
+            __float2bfloat16(g / (1.f + __expf(-g)) * u));
+        v[n / 2][m][r] = x;
+        amax[m] = fmaxf(amax[m], fabsf(x));
+      }
+    amax[m] = fmaxf(amax[m], __shfl_xor(amax[m], 16, 64));
+    amax[m] = fmaxf(amax[m], __shfl_xor(amax[m], 32, 64));
+  }
+  __syncthreads();  // the ring has been read
+  if (lhi == 0) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) most[wn * BM + wrow0 + m * 16 + l16] = amax[m];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = row0 + m * 16 + l16;
+    float a = 0.f;
+#pragma unroll
+    for (int w = 0; w < WN; ++w)
+      a = fmaxf(a, most[w * BM + wrow0 + m * 16 + l16]);
+    if (row >= M) continue;
+    const float scale = fp8_scale(a), inv = 1.f / scale;
+#pragma unroll
+    for (int n = 0; n < NT / 2; ++n)
+      *reinterpret_cast<unsigned *>(
+          out.q + (long)row * NC + nb * 128 + (wn * NT / 2 + n) * 16 +
+          lhi * 4) = fp8_bytes(v[n][m], inv);
+    if (wn == 0 && lhi == 0) out.scales[(long)nb * M + row] = scale;
+  }
+}
+
 // WM x WN waves share a BM x BN tile; a ring of ST stages of 128 columns (256
 // for int4). WK 2 (int4): as many waves again, each of a pair takes one of a
 // stage's two groups and twice the columns, and their sums are joined at the
@@ -189,7 +240,7 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void quant_gemm_kernel(
     const char *__restrict__ X, const float *__restrict__ XS,
     const char *__restrict__ W, const float *__restrict__ WS,
     const float *__restrict__ bias, int M, int N, int K, int k_slice,
-    int nbm, int nbn) {
+    int nbm, int nbn, const Fp8Out fp8) {
   constexpr int WAVES = WM * WN * WK;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
   // LDS row bytes; 128 of a weight row at once in either form (64 B pieces of
@@ -514,6 +565,12 @@ __global__ __launch_bounds__(WM *WN *WK * 64, 2) void quant_gemm_kernel(
     }
   }
 
+  if constexpr (Q == FP8 && FORM == GATED && BN == 256) {
+    if (fp8.q)
+      store_fp8<NT, MT, WN, BM>(fp8, acc, reinterpret_cast<float *>(smem), M,
+                                NC, mb * BM + wm * MT * 16, wm * MT * 16, nb,
+                                wn, lane);
+  }
   if (WK > 1 && wk > 0) return;
   store_tile<Q, NT, MT, BN, FORM>(C, acc, bias, M, N, NC, mb * BM + wm * MT * 16,
                                nb, z, wn * NT, lane);
@@ -568,7 +625,7 @@ Plan plan_for(bool int4, int M, int N, int K, bool gated, int splits) {
 }
 
 template <int FORM>
-void launch(const Plan &p, bool int4, void *C, const void *X, const float *XS,
+void launch(const Plan &p, const Fp8Out &fp8, bool int4, void *C, const void *X, const float *XS,
             const void *W, const float *WS, const float *bias, int M, int N,
             int K) {
   auto stream = at::cuda::getCurrentCUDAStream();
@@ -577,7 +634,7 @@ void launch(const Plan &p, bool int4, void *C, const void *X, const float *XS,
                      dim3(p.nbm * p.nbn, p.splits),                          \
                      dim3((WM) * (WN) * (WK) * 64), 0, stream, C,            \
                      (const char *)X, XS, (const char *)W, WS, bias, M, N,   \
-                     K, p.k_slice, p.nbm, p.nbn)
+                     K, p.k_slice, p.nbm, p.nbn, fp8)
   if (int4) {
     if (p.bm == 16 && p.bn == 128) RUN(INT4, 16, 128, 1, 2, 2, 2);
     else if (p.bm == 32 && p.bn == 256) RUN(INT4, 32, 256, 1, 4, 2, 2);
@@ -613,10 +670,10 @@ torch::Tensor parts_sum(torch::Tensor part, c10::optional<torch::Tensor> bias);
 // with it (x the e4m3 bytes). form 0: silu(gate) * up of w = gate rows over
 // up rows, bf16 [M, N / 2]; 1: bf16 [M, N], with the fp32 bias; 2: the fp32
 // parts [S, M, N]. splits: parts along K, 0: by the plan
-torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
-                         torch::Tensor w, torch::Tensor ws,
-                         c10::optional<torch::Tensor> bias, long form,
-                         long splits) {
+static torch::Tensor product(torch::Tensor x, c10::optional<torch::Tensor> xs,
+                             torch::Tensor w, torch::Tensor ws,
+                             c10::optional<torch::Tensor> bias, long form,
+                             long splits, const Fp8Out &fp8) {
   const bool int4 = !xs.has_value();
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && w.dim() == 2 &&
               x.is_contiguous() && w.is_contiguous() && aligned16(x) &&
@@ -650,17 +707,43 @@ torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
     auto out = torch::empty({M, form == GATED ? N / 2 : N}, o16);
     if (M == 0) return out;
     if (form == GATED)
-      launch<GATED>(p, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+      launch<GATED>(p, fp8, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
                     ws.data_ptr<float>(), nullptr, M, N, K);
     else
-      launch<PLAIN>(p, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+      launch<PLAIN>(p, fp8, int4, out.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
                     ws.data_ptr<float>(), bp, M, N, K);
     return out;
   }
   auto part = torch::empty({(long)p.splits, M, N},
                            x.options().dtype(at::kFloat));
   if (M > 0)
-    launch<PART>(p, int4, part.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
+    launch<PART>(p, fp8, int4, part.data_ptr(), x.data_ptr(), xsp, w.data_ptr(),
                  ws.data_ptr<float>(), nullptr, M, N, K);
   return form == PART ? part : parts_sum(part, bias);
+}
+
+torch::Tensor quant_gemm(torch::Tensor x, c10::optional<torch::Tensor> xs,
+                         torch::Tensor w, torch::Tensor ws,
+                         c10::optional<torch::Tensor> bias, long form,
+                         long splits) {
+  return product(x, xs, w, ws, bias, form, splits, Fp8Out{});
+}
+
+// Form 0 of fp8 with the result's e4m3 rows, {bf16, bytes, scales}, where a
+// tile holds whole groups of 128 columns; else {bf16}.
+std::vector<torch::Tensor> quant_gemm_gated_fp8(torch::Tensor x,
+                                                torch::Tensor xs,
+                                                torch::Tensor w,
+                                                torch::Tensor ws) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2);
+  const long M = x.size(0), N = w.size(0);
+  if (N % 256 ||
+      plan_for(false, std::max(M, 1L), N, x.size(1), true, 0).bn != 256)
+    return {product(x, xs, w, ws, c10::nullopt, GATED, 0, Fp8Out{})};
+  auto q = torch::empty({M, N / 2}, x.options());
+  auto st = torch::empty({N / 256, M}, xs.options());
+  auto out = product(x, xs, w, ws, c10::nullopt, GATED, 0,
+                     Fp8Out{q.data_ptr<unsigned char>(),
+                            st.data_ptr<float>()});
+  return {out, q, st};
 }

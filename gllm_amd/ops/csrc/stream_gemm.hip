@@ -30,6 +30,7 @@
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
+#include "fp8_rows.h"
 #include "qkv_rows.h"
 #include "tile_gemm.h"
 
@@ -228,11 +229,12 @@ __global__ __launch_bounds__(256) void stream_sum_kernel(
 // one chain of memory latencies: with all loads ahead of the sums, and each
 // part read once, 64 x 5120 in four parts takes 5.7 us (7.6 with the groups
 // of columns in turn), 256 x 5120 in six 10.4 (11.1), 1 x 4096 4.5 (4.8).
-template <int V, typename TW>
+// FP8 (N a multiple of 128): the result's e4m3 rows too.
+template <int V, typename TW, bool FP8>
 __global__ __launch_bounds__(512) void stream_add_norm_kernel(
     __hip_bfloat16 *__restrict__ out, __hip_bfloat16 *__restrict__ residual,
     const float *__restrict__ part, const TW *__restrict__ w, float eps,
-    int M, int N, int S, int rounded) {
+    int M, int N, int S, int rounded, const Fp8Out fp8) {
   __shared__ float red[8];
   const long row = blockIdx.x;
   const long MN = (long)M * N;
@@ -281,6 +283,22 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) o[r] = to_bf16(x[j][r] * inv * wv[j][r]);
     *reinterpret_cast<shortx4 *>(out + row * N + c) = o;
+    if constexpr (FP8) {  // a group is the columns of 32 lanes
+      float v8[4], amax = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v8[r] =
+            __bfloat162float(__builtin_bit_cast(__hip_bfloat16, (short)o[r]));
+        amax = fmaxf(amax, fabsf(v8[r]));
+      }
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1)
+        amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+      const float scale = fp8_scale(amax);
+      *reinterpret_cast<unsigned *>(fp8.q + row * N + c) =
+          fp8_bytes(v8, 1.f / scale);
+      if ((threadIdx.x & 31) == 0) fp8.scales[(long)(c >> 7) * M + row] = scale;
+    }
   }
 }
 
@@ -494,9 +512,9 @@ torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w) {
 
 // residual (bf16 [M, N], in place) += the sum of the fp32 parts [S, M, N]
 // (rounded: rounded to bf16 first); returns its RMS norm
-torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
-                             torch::Tensor norm_w, double eps,
-                             bool rounded) {
+static torch::Tensor add_norm(torch::Tensor part, torch::Tensor residual,
+                              torch::Tensor norm_w, double eps, bool rounded,
+                              const Fp8Out &fp8) {
   TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.is_contiguous() &&
               part.scalar_type() == at::kFloat && part.size(2) % 8 == 0 &&
               aligned16(part));
@@ -509,26 +527,54 @@ torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
   auto out = torch::empty({(long)M, (long)N}, residual.options());
   if (M == 0) return out;
   auto stream = at::cuda::getCurrentCUDAStream();
-#define RUN(V, TW)                                                           \
-  hipLaunchKernelGGL((stream_add_norm_kernel<V, TW>), dim3(M), dim3(512), 0, \
-                     stream, (__hip_bfloat16 *)out.data_ptr(),               \
+#define RUN(V, TW, FP8)                                                      \
+  hipLaunchKernelGGL((stream_add_norm_kernel<V, TW, FP8>), dim3(M),          \
+                     dim3(512), 0, stream, (__hip_bfloat16 *)out.data_ptr(), \
                      (__hip_bfloat16 *)residual.data_ptr(),                  \
                      part.data_ptr<float>(), (const TW *)norm_w.data_ptr(),  \
-                     (float)eps, M, N, S, (int)rounded)
-#define COLS(TW)                                                             \
+                     (float)eps, M, N, S, (int)rounded, fp8)
+#define COLS(TW, FP8)                                                        \
   do {                                                                       \
-    if (N <= 2048) RUN(1, TW);                                               \
-    else if (N <= 4096) RUN(2, TW);                                          \
-    else if (N <= 6144) RUN(3, TW);                                          \
-    else RUN(4, TW);                                                         \
+    if (N <= 2048) RUN(1, TW, FP8);                                          \
+    else if (N <= 4096) RUN(2, TW, FP8);                                     \
+    else if (N <= 6144) RUN(3, TW, FP8);                                     \
+    else RUN(4, TW, FP8);                                                    \
   } while (0)
-  if (norm_w.scalar_type() == at::kFloat) COLS(float);
-  else if (norm_w.scalar_type() == at::kBFloat16) COLS(__hip_bfloat16);
+#define WEIGHTS(TW)                                                          \
+  do {                                                                       \
+    if (fp8.q) COLS(TW, true);                                               \
+    else COLS(TW, false);                                                    \
+  } while (0)
+  if (norm_w.scalar_type() == at::kFloat) WEIGHTS(float);
+  else if (norm_w.scalar_type() == at::kBFloat16) WEIGHTS(__hip_bfloat16);
   else TORCH_CHECK(false, "norm_w: fp32 or bf16");
+#undef WEIGHTS
 #undef COLS
 #undef RUN
   HIP_CHECK_KERNEL();
   return out;
+}
+
+torch::Tensor parts_add_norm(torch::Tensor part, torch::Tensor residual,
+                             torch::Tensor norm_w, double eps,
+                             bool rounded) {
+  return add_norm(part, residual, norm_w, eps, rounded, Fp8Out{});
+}
+
+// ... with its e4m3 rows (N a multiple of 128): {bf16, bytes, scales}
+std::vector<torch::Tensor> parts_add_norm_fp8(torch::Tensor part,
+                                              torch::Tensor residual,
+                                              torch::Tensor norm_w,
+                                              double eps, bool rounded) {
+  TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.size(2) % 128 == 0,
+              "parts_add_norm_fp8: columns a multiple of 128");
+  const long M = part.size(1), N = part.size(2);
+  auto q = torch::empty({M, N}, part.options().dtype(at::kByte));
+  auto st = torch::empty({N / 128, M}, part.options());
+  auto out = add_norm(part, residual, norm_w, eps, rounded,
+                      Fp8Out{q.data_ptr<unsigned char>(),
+                             st.data_ptr<float>()});
+  return {out, q, st};
 }
 
 // residual (bf16 [M, N], in place) += x w^T; returns its RMS norm
