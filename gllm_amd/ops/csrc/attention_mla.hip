@@ -13,28 +13,24 @@
 // prefill, prefix hits and mixed batches. Decode splits the keys over
 // blockIdx.z with an fp32 LSE merge.
 //
-// A workgroup of four waves takes R row tiles of 16 and walks tiles of 64
-// keys. A key tile sits in LDS once, as nine column blocks of [64 keys][128
-// B] whose 16 B units are permuted by key & 7 (the layout both reads below
-// want), in a ring of two filled by global_load_lds while the other tile is
-// worked on (147 KB: one workgroup per CU). Scores are K Q^T and the output
-// is O^T = V^T P^T, so a lane holds keys, then dims, of ONE row; V is read
-// transposed out of the key tile (ds_read_tr16_b64).
-//  * R = 1 (decode, up to 16 heads): wave w scores keys 16 w .. + 15, the
-//    row maxima and the weights pass through LDS, then wave w owns dims
-//    128 w .. + 127 of the output. Every key byte is read from LDS once for
-//    the scores and once for the output.
-//  * R = 4 (prompts, more heads): wave w scores row tile w against all 64
-//    keys; the output is split by dims as above, so V is read once for 64
-//    rows instead of once per row tile.
-// R = 1 is bound by memory, R = 4 by LDS reads (K 295 KB + V 64 KB + P 32 KB
-// a tile against 2176 cycles of products). The kernel before this one read V
-// element by element (eight 2 B reads a fragment) and chose the splits by
-// the batch's lengths, which a captured launch does not have: one split.
-// 128 requests of 16 heads at 512 to 1536 keys (151 MB): 52 + 6 us, 282 us
-// before. Prompts of 4096 tokens in four, 16 heads: 257 us (535 us).
-// 512 workgroups as the aim of the splits: twice the CUs, so that requests
-// of unequal lengths even out.
+// A key tile sits in LDS once, as nine column blocks of [keys][128 B] whose 16
+// B units are permuted by key & 7 (the layout both reads below want), in a
+// ring of two filled by global_load_lds while the other tile is worked on.
+// Scores are K Q^T and the output is O^T = V^T P^T, so a lane holds keys, then
+// dims, of ONE row; V is read transposed out of the key tile
+// (ds_read_tr16_b64).
+//  * up to 16 rows (decode): mla_decode_kernel, bound by memory.
+//  * prompts, more heads: a workgroup of four waves takes R = 4 row tiles of
+//    16 and walks tiles of 64 keys (147 KB: one workgroup per CU). Wave w
+//    scores row tile w against all 64 keys; the output is split by dims, so V
+//    is read once for 64 rows instead of once per row tile. Bound by LDS reads
+//    (K 295 KB + V 64 KB + P 32 KB a tile against 2176 cycles of products).
+// 128 requests of 16 heads at 512 to 1536 keys (151 MB), us: element by
+// element and in one split 282; in tiles of 64 keys, one workgroup per CU, 52
+// + 6; of 32 keys, two per CU, 37 + 6. Prompts of 4096 tokens in four, 16
+// heads: 257 (535 element by element).
+// 512 workgroups as the aim of the splits: twice the CUs, so that all are on
+// the chip at once.
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -90,7 +86,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     int max_pages, int page_size, int H, float scale, int num_splits,
     long th_total) {
   constexpr int BQ = R * 16;
-  constexpr int NF = R == 1 ? 1 : 4;  // score fragments of a wave
+  constexpr int NF = 4;  // score fragments of a wave
   // the last row tiles see the most keys: they start first
   const int tile = gridDim.x - 1 - blockIdx.x;
   const int b = blockIdx.y;
@@ -127,8 +123,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
   __shared__ float s_a[4][16], s_b[4][16], s_m[4][16];
 
   // query fragments: column l16 = row, dims kt * 32 + lhi * 8
-  const int my_tile = R == 1 ? 0 : wave;
-  const int my_row = my_tile * 16 + l16;
+  const int my_row = wave * 16 + l16;
   mfma_bf8 qf[KT];
   {
     const __hip_bfloat16 *qp =
@@ -171,7 +166,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
         __builtin_amdgcn_global_load_lds(
             reinterpret_cast<const unsigned int *>(src[g] + c * 128),
             reinterpret_cast<unsigned int *>(dst + c * CB_B + g * 1024), 16,
-            0, R == 1 ? 2 : 0);
+            0, 0);
   };
 
   float m_run = -INFINITY, l_run = 0.f;
@@ -196,22 +191,19 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     }
     const char *kt_base = ring + slot * TILE_B;
 
-    // ---- scores: fragment f = keys (R == 1 ? wave : f) * 16 + lhi * 4 + r
-    mfma_f4 s[NF][2];
+    // ---- scores: fragment f = keys f * 16 + lhi * 4 + r
+    mfma_f4 s[NF];
 #pragma unroll
-    for (int f = 0; f < NF; ++f)
-      s[f][0] = s[f][1] = mfma_f4{0, 0, 0, 0};
-    const int krow = (R == 1 ? wave * 16 : 0) + l16;
+    for (int f = 0; f < NF; ++f) s[f] = mfma_f4{0, 0, 0, 0};
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const mfma_bf8 kf = *reinterpret_cast<const mfma_bf8 *>(
-            kt_base + (kt >> 1) * CB_B + (krow + f * 16) * 128 +
-            (((kt & 1) * 64 + lhi * 16) ^ ((krow & 7) << 4)));
-        // (one fragment: two chains)
-        s[f][NF == 1 ? kt & 1 : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            kf, qf[kt], s[f][NF == 1 ? kt & 1 : 0], 0, 0, 0);
+            kt_base + (kt >> 1) * CB_B + (l16 + f * 16) * 128 +
+            (((kt & 1) * 64 + lhi * 16) ^ ((l16 & 7) << 4)));
+        s[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[kt], s[f], 0, 0,
+                                                       0);
       }
     float mx = -INFINITY;
     float sv[NF][4];
@@ -219,19 +211,13 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int key = k0 + (R == 1 ? wave : f) * 16 + lhi * 4 + r;
-        const float x = (s[f][0][r] + s[f][1][r]) * qscale;
+        const int key = k0 + f * 16 + lhi * 4 + r;
+        const float x = s[f][r] * qscale;
         sv[f][r] = key < vis ? x : -INFINITY;
         mx = fmaxf(mx, sv[f][r]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (R == 1) {
-      if (lhi == 0) s_a[wave][l16] = mx;
-      lds_barrier();
-#pragma unroll
-      for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_a[w][l16]);
-    }
     // (a row may see nothing yet: a finite maximum keeps its weights at 0)
     const float m_new = fmaxf(fmaxf(m_run, mx), -1e30f);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -247,17 +233,16 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
         p[r] = bf16_bits(e);
       }
       *reinterpret_cast<shortx4 *>(
-          p_tile + my_row * P_ROW +
-          ((R == 1 ? wave : f) * 16 + lhi * 4) * 2) = p;
+          p_tile + my_row * P_ROW + (f * 16 + lhi * 4) * 2) = p;
     }
     l_run = l_run * alpha + sum;  // this lane's keys
-    if (R > 1 && lhi == 0) s_a[wave][l16] = alpha;
+    if (lhi == 0) s_a[wave][l16] = alpha;
     lds_barrier();
 
     // ---- output dims wave * 128 + nt * 16 .. of every row tile
     float al[R];
 #pragma unroll
-    for (int rt = 0; rt < R; ++rt) al[rt] = R == 1 ? alpha : s_a[rt][l16];
+    for (int rt = 0; rt < R; ++rt) al[rt] = s_a[rt][l16];
 #pragma unroll
     for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -306,9 +291,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
   for (int rt = 0; rt < R; ++rt) {
     const int row = rt * 16 + l16;
     if (row >= rows_here) continue;
-    const float l = R == 1 ? s_b[0][l16] + s_b[1][l16] + s_b[2][l16] +
-                                 s_b[3][l16]
-                           : s_b[rt][l16];
+    const float l = s_b[rt][l16];
     const float m = s_m[rt][l16];
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const long at = row0 + row;
@@ -332,6 +315,179 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
         for (int r = 0; r < 4; ++r) v[r] = bf16_bits(o[rt][nt][r] * inv);
         *reinterpret_cast<shortx4 *>(op + nt * 16) = v;
       }
+    }
+  }
+}
+
+// Up to 16 rows, decode: tiles of 32 keys in a ring of two, 78 KB, so that a
+// CU holds two workgroups and one's latencies are the other's work. Waves w
+// and w + 2 score keys 16 (w & 1) .. + 15, half of the dims each; the partial
+// scores pass through LDS, behind which every wave has all 32 keys' scores in
+// the layout that the second product takes: maxima, weights and sums stay in
+// registers. Wave w then owns dims 128 w .. + 127 of the output.
+template <bool SPLIT>
+__global__ __launch_bounds__(BLOCK, 2) void mla_decode_kernel(
+    __hip_bfloat16 *__restrict__ out, float *__restrict__ partial_out,
+    float *__restrict__ partial_lse, const __hip_bfloat16 *__restrict__ q,
+    const __hip_bfloat16 *__restrict__ kc,
+    const int *__restrict__ block_table, const int *__restrict__ seq_lens,
+    const int *__restrict__ qsl, int max_pages, int page_size, int H,
+    float scale, int num_splits, long th_total) {
+  constexpr int TK = 32, BLK_B = TK * 128, T_B = CB * BLK_B, HT = KT / 2;
+  const int b = blockIdx.y, split = blockIdx.z;
+  const int q_start = qsl[b];
+  const int q_len = qsl[b + 1] - q_start;
+  const int rows = min(q_len * H, 16);
+  if (rows <= 0) return;
+  const int seq_len = seq_lens[b], past = seq_len - q_len;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int l16 = lane & 15, lhi = lane >> 4;
+  // (shares of whole 64-key tiles)
+  const int split_len =
+      ((seq_len + BKV - 1) / BKV + num_splits - 1) / num_splits * BKV;
+  const int kv_lo = split * split_len;
+  const int kv_hi = min(kv_lo + split_len, seq_len);
+  const long row0 = (long)q_start * H;
+  if (kv_lo >= kv_hi) {  // an empty split: the merge skips it
+    if (SPLIT && tid < rows)
+      partial_lse[(long)split * th_total + row0 + tid] = -INFINITY;
+    return;
+  }
+  __shared__ __attribute__((aligned(16))) char ring[2 * T_B];
+  __shared__ mfma_f4 part[4][64];
+
+  // staging: wave w brings keys 8 w .. + 7 as nine units of [8 keys][128 B]
+  const int *bt = block_table + (long)b * max_pages;
+  const int s_key = wave * 8 + (lane >> 3);
+  const int s_col = ((lane & 7) ^ (lane >> 3)) * 16;
+  int page = 0;
+  auto key_of = [&](int k0) { return min(k0 + s_key, seq_len - 1); };
+  auto look_up = [&](int k0) { page = bt[key_of(k0) / page_size]; };
+  auto stage = [&](int k0, int slot) {
+    const char *src =
+        reinterpret_cast<const char *>(kc) +
+        ((long)page * page_size + key_of(k0) % page_size) * ROW_B + s_col;
+    char *dst = ring + slot * T_B + wave * 1024;
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const unsigned int *>(src + c * 128),
+          reinterpret_cast<unsigned int *>(dst + c * BLK_B), 16, 0, 2);
+  };
+  look_up(kv_lo);
+  stage(kv_lo, 0);
+  if (kv_lo + TK < kv_hi) look_up(kv_lo + TK);
+
+  // query fragments of this wave's half of the dims: column l16 = row
+  const int my_half = wave >> 1, my_keys = (wave & 1) * 16;
+  mfma_bf8 qf[HT];
+  {
+    const __hip_bfloat16 *qp =
+        q + (row0 + min(l16, rows - 1)) * DK + my_half * HT * 32 + lhi * 8;
+#pragma unroll
+    for (int i = 0; i < HT; ++i)
+      qf[i] = *reinterpret_cast<const mfma_bf8 *>(qp + i * 32);
+  }
+  const int vis = l16 < rows ? min(seq_len, past + l16 / H + 1) : 0;
+  const float qscale = scale * LOG2E;
+
+  float m_run = -INFINITY, l_run = 0.f;
+  mfma_f4 o[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) o[nt] = mfma_f4{0, 0, 0, 0};
+  const int tr_row = lhi * 4 + (l16 >> 2), tr_col = (l16 & 3) * 8;
+  int slot = 0;
+  for (int k0 = kv_lo; k0 < kv_hi; k0 += TK, slot ^= 1) {
+    // the tile is there; the other slot and the scores are free
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (k0 + TK < kv_hi) {
+      stage(k0 + TK, slot ^ 1);
+      if (k0 + 2 * TK < kv_hi) look_up(k0 + 2 * TK);
+    }
+    const char *base = ring + slot * T_B;
+    mfma_f4 s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};  // two chains
+    const int krow = my_keys + l16;
+#pragma unroll
+    for (int i = 0; i < HT; ++i) {
+      const int kt = my_half * HT + i;
+      const mfma_bf8 kf = *reinterpret_cast<const mfma_bf8 *>(
+          base + (kt >> 1) * BLK_B + krow * 128 +
+          (((kt & 1) * 64 + lhi * 16) ^ ((krow & 7) << 4)));
+      s[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[i], s[i & 1],
+                                                         0, 0, 0);
+    }
+    part[wave][lane] = s[0] + s[1];
+    lds_barrier();
+    // keys f * 16 + lhi * 4 + r of row l16
+    float sv[2][4], mx = -INFINITY;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      const mfma_f4 x = part[f][lane] + part[f + 2][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sv[f][r] = k0 + f * 16 + lhi * 4 + r < vis ? x[r] * qscale
+                                                   : -INFINITY;
+        mx = fmaxf(mx, sv[f][r]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    // (a row may see nothing yet: a finite maximum keeps its weights at 0)
+    const float m_new = fmaxf(fmaxf(m_run, mx), -1e30f);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    float sum = 0.f;
+    MlaFrag pf;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(sv[f][r] - m_new);
+        sum += e;
+        pf.h[f][r] = bf16_bits(e);
+      }
+    l_run = l_run * alpha + sum;  // this lane's keys
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      MlaFrag vf;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int row = half * 16 + tr_row;
+        vf.h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_shortx4 *)(base + (wave * 2 + (nt >> 2)) * BLK_B + row * 128 +
+                            (((nt & 3) * 32 + tr_col) ^ ((row & 7) << 4))));
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[nt][r] *= alpha;
+      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, o[nt], 0, 0,
+                                                      0);
+    }
+  }
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (l16 >= rows) return;
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  const long at = row0 + l16;
+  if (SPLIT) {
+    float *op = partial_out + ((long)split * th_total + at) * DV + wave * 128 +
+                lhi * 4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      *reinterpret_cast<floatx4 *>(op + nt * 16) =
+          floatx4{o[nt][0] * inv, o[nt][1] * inv, o[nt][2] * inv,
+                  o[nt][3] * inv};
+    if (wave == 0 && lhi == 0)
+      partial_lse[(long)split * th_total + at] =
+          l_run > 0.f ? m_run / LOG2E + __logf(l_run) : -INFINITY;
+  } else {
+    __hip_bfloat16 *op = out + at * DV + wave * 128 + lhi * 4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      shortx4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = bf16_bits(o[nt][r] * inv);
+      *reinterpret_cast<shortx4 *>(op + nt * 16) = v;
     }
   }
 }
@@ -427,10 +583,9 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
     po = partial.data_ptr<float>();
     pl = lse.data_ptr<float>();
   }
-#define RUN(RT, SPLIT)                                                       \
-  hipLaunchKernelGGL((mla_attention_kernel<RT, SPLIT>),                      \
-                     dim3(tiles, B, splits), dim3(BLOCK), 0, stream,         \
-                     (__hip_bfloat16 *)out.data_ptr(), po, pl,               \
+#define RUN(...)                                                             \
+  hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles, B, splits), dim3(BLOCK), 0,  \
+                     stream, (__hip_bfloat16 *)out.data_ptr(), po, pl,       \
                      (const __hip_bfloat16 *)q.data_ptr(),                   \
                      (const __hip_bfloat16 *)k_cache.data_ptr(),             \
                      block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),  \
@@ -438,11 +593,13 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
                      (int)block_table.stride(0), (int)k_cache.size(1), H,    \
                      (float)scale, splits, th_total)
   if (splits == 1) {
-    if (R == 1) RUN(1, false); else RUN(4, false);
+    if (R == 1) RUN(mla_decode_kernel<false>);
+    else RUN(mla_attention_kernel<4, false>);
     HIP_CHECK_KERNEL();
     return;
   }
-  if (R == 1) RUN(1, true); else RUN(4, true);
+  if (R == 1) RUN(mla_decode_kernel<true>);
+  else RUN(mla_attention_kernel<4, true>);
 #undef RUN
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((mla_merge_kernel), dim3((unsigned)th_total),

@@ -43,6 +43,9 @@ def _ref(q, cache, table, lens, qsl, scale):
     ([1, 1], [70, 500], 128, 16),
     ([1] * 600, [40] * 600, 16, 16),       # no split
     ([70, 1, 3], [0, 130, 64], 16, 16),    # portions beside a decode
+    ([1] * 7, [30, 31, 32, 94, 95, 96, 1500], 16, 16),  # 32 keys
+    ([2, 1, 2], [31, 33, 700], 8, 16),     # two rows a head
+    ([3] * 300, [64] * 300, 5, 16),        # the same, no split
     ([33], [100], 5, 48),                  # page size not a power of two
     ([64, 65], [0, 0], 16, 1),
 ])
