@@ -512,14 +512,41 @@ DEV_INLINE float key_value(unsigned k) {
                          : k & 0x80000000u ? k ^ 0x80000000u : ~k);
 }
 
-// the wave's largest key, the lower index of equals
-DEV_INLINE void wave_pick(unsigned &key, int &idx) {
+// the largest of the wave's keys
+DEV_INLINE unsigned wave_max_key(unsigned x) {
+#define STEP(CTRL, ROWS)                                                     \
+  x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS,    \
+                                                   0xf, false))
+  STEP(0x111, 0xf);  // row_shr 1, 2, 4, 8; then the rows before
+  STEP(0x112, 0xf);
+  STEP(0x114, 0xf);
+  STEP(0x118, 0xf);
+  STEP(0x142, 0xa);
+  STEP(0x143, 0xc);
+#undef STEP
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Takes the wave's largest key (lane: indexes lane + 64 j) out of the
+// candidates; its index, the lowest of equals. (us, eight of 128 experts, 128
+// rows 6.0, 8192 rows 13.1; with key and index passed from lane to lane 8.6 and
+// 17.2.)
+template <int J>
+DEV_INLINE int take_best(unsigned (&key)[J], unsigned &best) {
+  unsigned mine = key[0];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned ok = __shfl_xor(key, off, 64);
-    const int oi = __shfl_xor(idx, off, 64);
-    if (ok > key || (ok == key && oi < idx)) { key = ok; idx = oi; }
+  for (int j = 1; j < J; ++j) mine = max(mine, key[j]);
+  best = wave_max_key(mine);
+  int idx = -1;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const unsigned long long m = __ballot(key[j] == best);
+    if (idx < 0 && m) idx = 64 * j + __ffsll(m) - 1;
   }
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (idx == (int)(threadIdx.x & 63) + 64 * j) key[j] = 0u;
+  return idx;
 }
 
 __global__ __launch_bounds__(256) void topk_softmax_rows_kernel(
@@ -535,20 +562,11 @@ __global__ __launch_bounds__(256) void topk_softmax_rows_kernel(
     const int e = lane + 64 * j;
     key[j] = e < E ? pick_key(row[e]) : 0u;
   }
-  unsigned taken = 0;
   float my_val = -INFINITY;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    unsigned best = 0;
-    int bidx = 0;
-#pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j)
-      if (!(taken >> j & 1u) && key[j] > best) {
-        best = key[j];
-        bidx = lane + 64 * j;
-      }
-    wave_pick(best, bidx);
-    if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
+    unsigned best;
+    const int bidx = take_best(key, best);
     if (lane == it) { my_val = key_value(best); my_idx = bidx; }
   }
   const float top = __shfl(my_val, 0, 64);  // the first pick is the largest
@@ -564,8 +582,9 @@ __global__ __launch_bounds__(256) void topk_softmax_rows_kernel(
 // descending order (ties to the lower index); renorm: over their sum.
 // Bound by launches, not by work: it stands for a cast, a softmax, a top-k,
 // a sort, a sum, a division and a cast (8 experts: 64 tokens 5.3 us for 48,
-// 5000 tokens 7.8 us for 57). A wave per row, as above.
-template <typename T>
+// 5000 tokens 7.8 us for 57). A wave per row, as above, J experts per lane;
+// with one, a pick is a maximum over lanes and the first lane that has it.
+template <typename T, int J>
 __global__ __launch_bounds__(256) void softmax_topk_rows_kernel(
     float *__restrict__ weights, int *__restrict__ ids,
     const T *__restrict__ logits, long rows, int E, int k, bool renorm) {
@@ -573,38 +592,29 @@ __global__ __launch_bounds__(256) void softmax_topk_rows_kernel(
   const int lane = threadIdx.x & 63;
   if (r >= rows) return;
   const T *row = logits + r * E;
-  float v[TK_MAXJ], mx = -INFINITY;
+  float v[J], mx = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < TK_MAXJ; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int e = lane + 64 * j;
     v[j] = e < E ? ScalarOps<T>::to_f32(row[e]) : -INFINITY;
     mx = fmaxf(mx, v[j]);
   }
   mx = wave_reduce_max(mx);
   float sum = 0.f;
-  unsigned key[TK_MAXJ];
+  unsigned key[J];
 #pragma unroll
-  for (int j = 0; j < TK_MAXJ; ++j) {
+  for (int j = 0; j < J; ++j) {
     const bool live = lane + 64 * j < E;
     const float p = expf(v[j] - mx);
     key[j] = live ? pick_key(p) : 0u;
     if (live) sum += p;
   }
   sum = wave_reduce_sum(sum);
-  unsigned taken = 0;
   float my_val = 0.f;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    unsigned best = 0;
-    int bidx = 0;
-#pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j)
-      if (!(taken >> j & 1u) && key[j] > best) {
-        best = key[j];
-        bidx = lane + 64 * j;
-      }
-    wave_pick(best, bidx);
-    if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
+    unsigned best;
+    const int bidx = take_best(key, best);
     if (lane == it) { my_val = key_value(best) / sum; my_idx = bidx; }
   }
   if (renorm) my_val /= wave_reduce_sum(lane < k ? my_val : 0.f);
@@ -680,19 +690,10 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
 #pragma unroll
   for (int j = 0; j < TK_MAXJ; ++j)
     key[j] = lane + 64 * j < E ? pick_key(c[j]) : 0u;
-  unsigned taken = 0;
   int my_idx = 0;
   for (int it = 0; it < k; ++it) {
-    unsigned best = 0;
-    int bidx = 0;
-#pragma unroll
-    for (int j = 0; j < TK_MAXJ; ++j)
-      if (!(taken >> j & 1u) && key[j] > best) {
-        best = key[j];
-        bidx = lane + 64 * j;
-      }
-    wave_pick(best, bidx);
-    if ((bidx & 63) == lane) taken |= 1u << (bidx >> 6);
+    unsigned best;
+    const int bidx = take_best(key, best);
     if (lane == it) my_idx = bidx;
   }
   const float my_w = lane < k ? 1.0f / (1.0f + expf(-row[my_idx])) : 0.f;
@@ -761,16 +762,22 @@ void softmax_topk_rows(torch::Tensor weights, torch::Tensor ids,
               ", top <= min(64, experts)");
   if (rows == 0) return;
   auto stream = at::cuda::getCurrentCUDAStream();
-#define RUN(T)                                                               \
-  hipLaunchKernelGGL((softmax_topk_rows_kernel<T>), dim3((rows + 3) / 4),    \
+#define ROWS(T, J)                                                           \
+  hipLaunchKernelGGL((softmax_topk_rows_kernel<T, J>), dim3((rows + 3) / 4), \
                      dim3(256), 0, stream, weights.data_ptr<float>(),        \
                      ids.data_ptr<int>(), (const T *)logits.data_ptr(), rows,\
                      E, k, renorm)
+#define RUN(T)                                                               \
+  do {                                                                       \
+    if (E <= 64) ROWS(T, 1);                                                 \
+    else ROWS(T, TK_MAXJ);                                                   \
+  } while (0)
   if (logits.scalar_type() == at::kFloat) RUN(float);
   else if (logits.scalar_type() == at::kBFloat16) RUN(__hip_bfloat16);
   else if (logits.scalar_type() == at::kHalf) RUN(__half);
   else TORCH_CHECK(false, "softmax_topk_rows: fp32, bf16 or fp16 logits");
 #undef RUN
+#undef ROWS
   HIP_CHECK_KERNEL();
 }
 
