@@ -8,9 +8,8 @@
 // by row & 7, so fragment reads fall on all banks; products are W x^T, so a
 // lane ends with four neighbouring columns of one row.
 //
-// A weight with few tiles is also split along K (plan_for: into about 384
-// workgroups below 160 tiles, into two parts up to 288 if K is long); the fp32
-// parts [S, M, N] are then summed by whatever comes next, in the order of S:
+// A weight with few tiles is also split along K (plan_for: into one full round
+// of workgroups); the fp32 parts [S, M, N] are then summed by whatever comes next, in the order of S:
 //   stream_gemm           bias, bf16
 //   stream_add_norm       residual += sum, RMS norm of it (attention and
 //                         feed-forward outputs)
@@ -20,8 +19,8 @@
 // tile) leaves silu(gate) * up straight from the sums.
 // (us against hipBLASLt and against the kernel before this one, which split
 // K into up to 16 and summed the parts one load at a time:) 5120 x 27648, 64
-// rows 63 for 159 and 79, 256 rows 110 for 266 and 160; 7168 x 5120, 1 row
-// 16.4 for 24; 28672 x 4096 gated, 1 row 39 for 61 + 5. Weights come at 4.0
+// rows 60 for 159 and 79, 256 rows 83 for 266 and 160; 7168 x 5120, 1 row
+// 13.5 for 24; 28672 x 4096 gated, 1 row 40 for 61 + 5. Weights come at 4.2
 // to 6.6 TB/s from 35 MB on, below that the launch and the ring's first
 // stages are most of the time (2048 x 2048: 5 + 3 us). Parts of large weights
 // with more than 64 rows (32 if K is long) come from tile_gemm.hip, where 256
@@ -332,53 +331,94 @@ struct Plan {
   int bm, bn, nbm, nbn, splits, k_slice;
 };
 
-// The tile by the rows and by how wide the weight is (us, M x N x K, each
-// against its neighbour):
-//  * up to 64 rows 64 columns, two workgroups per CU: 16 x 7168 x 5120 18.2
-//    (128 columns 19.1), 64 x 28672 x 4096 47.6 (50.7); from 36000 columns
-//    on, where rows would be staged too often, 256: 64 x 55296 x 5120 93
-//    (64 columns 129, 128 columns 106), 24 rows 86 (98).
-//  * up to 128 rows: below 8192 columns two row blocks of 64, 128 x 7168 x
-//    5120 28.9 (128 x 64 tiles 31.6); K at least 2 N: 128 x 128, 128 x 5120
-//    x 27648 75 (128 x 64 80); from 36000 columns 128 x 256, 128 x 55296 x
-//    5120 105 (128 x 128 128); else 128 x 64.
-//  * up to 256 rows: K at least 2 N or 16384 columns and more: 256 x 128,
-//    256 x 5120 x 27648 110 (128 x 128 118), 256 x 28672 x 4096 68 (128 x 64
-//    90); gated and 36000 columns 256 x 256, 149 (256 x 128 175); else 128 x
-//    64, 256 x 7168 x 5120 40 (128 x 128 42).
-// The lines in between (K 5120, gated, us, narrow / wide tile): 32768 columns
-// are 512 tiles of 64, two per CU, and the last that the chip holds at once:
-// 64 rows 68 / 81, 128 rows 88 / 96, 256 rows 96 / 132; 36864: 93 / 84, 123 /
-// 98, 157 / 134 (24 rows 90 / 80). From 64 rows on the wide tile is the faster
-// one from there already (34816: 92 / 83, 122 / 97, 155 / 133), 24 rows not
-// yet (74 / 80).
-// K is split into about 384 workgroups where there are fewer than 160 tiles
-// (5120 x 27648, 16 rows: 5 splits 50.8, 13 splits 52.9; 7168 x 5120: 4
-// splits 18.2, 7 splits 19.6; 11008 x 2048 at 172 tiles: none 11.2, two
-// 13.4), into two from there to 288 tiles if K is long, each part at least
-// four stages long.
+// How full `slots` workgroups are with `tiles`, each split where they fit
+// more than once.
+double fill_of(int tiles, int slots) {
+  const int rounds = (tiles + slots - 1) / slots;
+  return tiles <= slots ? (double)(slots / tiles * tiles) / slots
+                        : (double)tiles / (rounds * slots);
+}
+
+// What a tile costs is the stages it has in flight and how evenly the tiles
+// fill the chip: a product runs in one round of workgroups that are all there
+// from the start (two a CU for 16 rows and for 64 columns, else one), split
+// along K into as many as fit that round. Rounding up instead (to about 384
+// workgroups of 64 columns) left a second round nearly empty or half the CUs
+// with twice the work. us in turn over weights that no cache holds, before /
+// now, with the norm or the bias behind them:
+//  * up to 64 rows, large weights: 128 columns. 1 x 6144 x 4096 11.8 / 10.0,
+//    64 x 5120 x 5120 23.2 / 20.2, 64 x 4096 x 14336 36.5 / 28.7, 1 x 8192 x
+//    8192 32.4 / 28.2. 64 columns stay where that is small (below 6 M values
+//    for 16 rows, 20 M above: 2048 x 2048 7.0 both) or where 64 columns fill
+//    nine tenths of 512 workgroups unsplit (32064 x 4096); 256 columns where
+//    they fill the chip better by a tenth: 64 x 19008 x 5120 60 / 44.
+//  * up to 128 rows 128 x 128 from 20 M values on, one row block in place of
+//    two of 64: 128 x 6144 x 4096 21.6 / 16.4, 19008 x 5120 79 / 60.
+//  * up to 256 rows, narrow: 128 columns, 64 rows below 12 M values: 256 x
+//    2048 x 2816 19.6 / 15.6, 160 x 4096 x 4096 26.3 / 22.7. Rounding up stays
+//    for 256 x 128 tiles (160 x 19008 x 5120 58; unsplit 74).
+//  * gated (not split): by whole rounds too, 128 columns where 64 leave the
+//    second round thin (64 x 22016 x 4096 44.5 / 38.2, 128 x 28672 x 4096 60 /
+//    50), 256 from 36000 columns on (one row: from 48000, 55296 x 5120 96 / 89;
+//    43008 x 4096 keeps 128 columns, 74 / 70).
+// 28 to 32 tiles take at most 8 splits, a workgroup a CU: 4096 x 4096 11.6
+// against 13.1 with 16, whose sums then cost more than the stages they save;
+// 40 tiles don't gain by a cap of 8 (5120 x 5120 15.7 / 16.6, K 27648 50 / 59).
+// Each part has four stages at least.
 Plan plan_for(int M, int N, int K, bool gated) {
   Plan p;
-  const bool wide = N >= 36000, deep = K >= 2 * N;
+  const long weights = (long)N * K;
+  const int tiles64 = (N + 63) / 64;
+  const bool even = tiles64 > 256 && (fill_of(tiles64, 512) >= 0.9 ||
+                                      (M <= 16 && tiles64 <= 512 &&
+                                       K < 4096));
+  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
   p.bn = 64;
-  if (M <= 64) {
-    p.bm = M <= 16 ? 16 : M <= 32 ? 32 : 64;
-    if (wide && p.bm > 16) p.bn = 256;
+  int slots = 512;
+  if (gated && M <= 64) {
+    if (N >= (p.bm == 16 ? 48000 : 36000)) p.bn = 256;
+    else if (N >= 16384 && !even &&
+             (p.bm == 64 ? N <= 32768 : fill_of(tiles64, 512) < 0.8))
+      p.bn = 128;
+  } else if (gated && M <= 128) {
+    p.bm = N >= 8192 ? 128 : 64;
+    p.bn = N >= 36000 ? 256 : N >= 16384 && N <= 32768 ? 128 : 64;
+  } else if (gated) {
+    p.bm = K >= 2 * N || N >= 16384 ? 256 : 128;
+    p.bn = p.bm == 128 ? 64 : N >= 36000 ? 256 : 128;
+  } else if (M <= 64) {
+    const bool small = weights < (p.bm == 16 ? 6L << 20 : 20L << 20);
+    if (!small && !even) {
+      p.bn = 128;
+      if (p.bm > 16) {
+        slots = 256;
+        if (N >= 8192 && fill_of((N + 255) / 256, 256) >
+                             fill_of((N + 127) / 128, 256) + 0.1)
+          p.bn = 256;
+      }
+    }
   } else if (M <= 128) {
-    p.bm = wide || deep || N >= 8192 ? 128 : 64;
-    p.bn = wide ? 256 : deep ? 128 : 64;
+    slots = 256;
+    p.bn = N >= 36000 ? 256 : weights >= (20L << 20) ? 128 : 64;
   } else {
-    p.bm = deep || N >= 16384 ? 256 : 128;
-    p.bn = p.bm == 128 ? 64 : gated && wide ? 256 : 128;
+    slots = 256;
+    if (N >= 16384 || (K >= 2 * N && N >= 5120)) {
+      p.bm = 256;
+      p.bn = 128;
+    } else if (N < 5120) {
+      p.bn = 128;
+      if (weights < (12L << 20)) p.bm = 64;
+    }
   }
   p.nbm = (M + p.bm - 1) / p.bm;
   p.nbn = (N + p.bn - 1) / p.bn;
   const int tiles = p.nbm * p.nbn, stages = K / BK;
   int s = 1;
   if (!gated) {
-    if (tiles < 160) s = (384 + tiles - 1) / tiles;
-    else if (tiles < 288 && stages >= 128) s = 2;
-    s = std::max(1, std::min(std::min(s, MAX_SPLIT), stages / 4));
+    s = std::min(slots / tiles, MAX_SPLIT);
+    if (p.bm == 256 && tiles < 160) s = (384 + tiles - 1) / tiles;
+    if (tiles >= 28 && tiles <= 32) s = std::min(s, 8);
+    s = std::max(1, std::min(s, stages / 4));
   }
   const int per = (stages + s - 1) / s;
   p.k_slice = per * BK;
@@ -411,17 +451,28 @@ void launch(const Plan &p, void *C, const torch::Tensor &x,
                      (const __hip_bfloat16 *)w.data_ptr(),                   \
                      (const __hip_bfloat16 *)bias, M, N, K, p.k_slice,       \
                      p.nbm, p.nbn)
-  // (a wave needs a gate and an up tile, so 16 columns are too few)
-  if (p.bm == 16) RUN(16, 64, 1, FORM == GATED ? 2 : 4, 8);
+  // (a wave needs a gate and an up tile, so 16 columns are too few; the last
+  // figure is the ring, as deep as one or two workgroups a CU leave room for)
+  if (p.bm == 16 && p.bn == 64) RUN(16, 64, 1, FORM == GATED ? 2 : 4, 8);
+  else if (p.bm == 16 && p.bn == 128) RUN(16, 128, 1, 4, 4);
   else if (p.bm == 32 && p.bn == 64) RUN(32, 64, 1, 2, 6);
-  else if (p.bm == 32) RUN(32, 256, 1, 4, 4);
+  else if (p.bm == 32 && p.bn == 128 && FORM == GATED) RUN(32, 128, 1, 4, 4);
+  else if (p.bm == 32 && p.bn == 128) RUN(32, 128, 1, 4, 7);
+  else if (p.bm == 32) RUN(32, 256, 1, 8, 4);
   else if (p.bm == 64 && p.bn == 64) RUN(64, 64, 2, 2, 5);
-  else if (p.bm == 64) RUN(64, 256, 2, 4, 3);
-  else if (p.bm == 128 && p.bn == 64) RUN(128, 64, 2, 2, 3);
-  else if (p.bm == 128 && p.bn == 128) RUN(128, 128, 2, 2, 2);
+  else if (p.bm == 64 && p.bn == 128) RUN(64, 128, 2, 4, 6);
+  else if (p.bm == 64) RUN(64, 256, 2, 4, 4);
+  else if (p.bm == 128 && p.bn == 64 && (FORM == GATED || x.size(0) > 128))
+    RUN(128, 64, 2, 2, 3);
+  else if (p.bm == 128 && p.bn == 64) {
+    if constexpr (FORM != GATED) RUN(128, 64, 2, 4, 6);
+  } else if (p.bm == 128 && p.bn == 128) RUN(128, 128, 2, 4, 5);
   else if (p.bm == 128) RUN(128, 256, 2, 4, 3);
-  else if (p.bn == 128) RUN(256, 128, 4, 2, 3);
-  else if constexpr (FORM == GATED) RUN(256, 256, 2, 4, 2);
+  else if (p.bm == 256 && p.bn == 128) RUN(256, 128, 4, 2, 3);
+  else if constexpr (FORM == GATED) {
+    if (p.bm == 16) RUN(16, 256, 1, 8, 4);
+    else RUN(256, 256, 2, 4, 2);
+  }
   else TORCH_CHECK(false, "stream_gemm: no such tile");
 #undef RUN
   HIP_CHECK_KERNEL();

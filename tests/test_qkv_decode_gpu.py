@@ -95,6 +95,7 @@ def test_replayed():
                               s["cos_sin"], s["k"], s["v"], s["slots"],
                               s["table"], s["lens"], arrived, 32, 128 ** -0.5)
     stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
     with torch.cuda.stream(stream):
         call()
     torch.cuda.synchronize()
