@@ -14,20 +14,25 @@
 //   themselves, and a workgroup per CU starts at once in any order. Finding
 //   the sequence costs each workgroup 1 to 3 us, more than short shares give
 //   back, and heads fastest is the slower one for equal lengths: there
-//   sequences are the fastest index, as they come. (us, 32 heads on 8 of 128,
-//   sequences fastest / this: 64 sequences of 512 to 1536 keys 68 / 61, 128 of
-//   1024 to 3072 218 / 197, 24 of 2700 to 8100 in four splits 138 / 124, 100
-//   of 1 to 4000 179 / 153, 32 of 10 to 1500 in two 35 / 30. Where it is not
-//   done, as they come / in order: 128 of 2048 179 / 193, 33 of 1100 in two
-//   splits 39 / 46, 100 of 700 to 1000 71 / 78; one head, 33 of 10 to 1100 in
-//   sixteen splits 18.5 / 25.4; 14 heads on 2 of 64, 64 of 512 to 1536 14.5 /
-//   17.2, 400 of 100 to 1500 39 / 42; 64 of 1600 to 2048 would gain, 96 / 91.)
+//   sequences are the fastest index, as they come. (us, with the keys' own
+//   step, 32 heads on 8 of 128, sequences fastest / this: 64 sequences of 512
+//   to 1536 keys 58 / 55, 128 of 1024 to 3072 182 / 176, 24 of 2700 to 8100 in
+//   four splits 116 / 106, 100 of 1 to 4000 149 / 143, 32 of 10 to 1500 in two
+//   32.6 / 31.6; 40 heads, 24 of 2700 to 7900 114 / 102. What finding out costs
+//   where it gives nothing: 24 of 5400 101.3 / 103.1, 128 of 520 to 1500 93.1 /
+//   96.2, 64 of 1600 to 2048 87.2 / 88.9.)
 //   Its waves work on their own: wave w takes the 32-key tiles w, w + 4,
 //   ... of the share, with a softmax state of its own and no barrier in the
-//   loop; the next tile's K and V are in registers while this one is
-//   worked on. K rows come from memory in operand layout (no LDS); V
-//   passes through a patch of LDS that belongs to the wave and is read
-//   transposed (ds_read_tr16_b64). Scores are K Q^T and the output is
+//   loop. K and V go straight to a patch of LDS that belongs to the wave, whole
+//   rows at a time, their 16 B units permuted by the row. As soon as a tile's K
+//   is in registers the next tile's takes its place, and so with V (read
+//   transposed, ds_read_tr16_b64): 16 KB a wave are on their way, 128 KB a CU,
+//   what two workgroups find room for. K by registers, in operand layout, costs
+//   a quarter of a row a lane group and the copies: the loads alone took 50 us
+//   so and 43 by whole rows (64 sequences of 1024 keys, 8 heads of 128; 41 at
+//   6.5 TB/s), the kernel 55 and 49 now; 256 of 1024 175 / 164, 24 of 5400 in
+//   four splits 104 / 96, 64 of 4096 201 / 178, 29 of 1024 in two 34 / 31.
+//   Scores are K Q^T and the output is
 //   O^T = V^T P^T, so a lane holds keys of ONE head: one softmax state per
 //   lane, and the weights are the right operand of the second product as
 //   they stand. At the end the waves join through LDS.
@@ -121,6 +126,24 @@ DEV_INLINE int sequence_at(int rank, int B, const int *seq_lens, int window,
   return 0;  // (not reached: every key is in 0 .. 15)
 }
 
+// global -> LDS, 16 B a lane, non-temporal (a cached row is read by one wave)
+DEV_INLINE void fetch16(const char *src, char *dst) {
+  __builtin_amdgcn_global_load_lds(
+      reinterpret_cast<const unsigned int *>(src),
+      reinterpret_cast<unsigned int *>(dst), 16, 0, 2);
+}
+
+DEV_INLINE void fetch4(const int *src, int *dst) {
+  __builtin_amdgcn_global_load_lds(
+      reinterpret_cast<const unsigned int *>(src),
+      reinterpret_cast<unsigned int *>(dst), 4, 0, 0);
+}
+
+template <int LEFT>
+DEV_INLINE void wait_loads() {  // until at most LEFT are on their way
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LEFT) : "memory");
+}
+
 // What an instance that starts from the projection takes beside the caches.
 struct NewRows {
   QkvRows rows;                    // q | k | v of each sequence's new token
@@ -203,9 +226,10 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     // keys from which on the order of sequences matters
     int order_above, const NewRows fresh) {
   constexpr int KT = D / 32, NT = DV / 16;
-  constexpr int VU = TK * (DV / 8) / 64;   // 16 B units of V per lane
-  constexpr int VROW = DV * 2;             // LDS row bytes
-  constexpr int VMASK = (DV / 8 - 1) & 15;
+  // 16 B units per lane, LDS row bytes, the rows that permute them
+  constexpr int KU = TK * (D / 8) / 64, VU = TK * (DV / 8) / 64;
+  constexpr int KROW = D * 2, VROW = DV * 2;
+  constexpr int KMASK = (D / 8 - 1) & 15, VMASK = (DV / 8 - 1) & 15;
   if constexpr (FRESH) {
     softcap = temp_coef = 0.f;
     bias = sinks = nullptr;
@@ -256,7 +280,7 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const int t1 = kept ? min(keep_first, w_begin)
                       : min(t0 + split_len, seq_len);
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int l16 = lane & 15;
   const int lhi = lane >> 4;
@@ -273,53 +297,61 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
     }
     return;
   }
-  // a patch per wave: its V tile, later its output (as many bytes)
-  __shared__ __attribute__((aligned(16))) char patch[WAVES][TK * VROW];
+  // a patch per wave: its V tile (later its output, as many bytes), its K tile
+  __shared__ __attribute__((aligned(16))) char
+      patch[WAVES][TK * (VROW + KROW)];
   __shared__ float s_m[WAVES][16], s_l[WAVES][16];
 
   const int *bt = block_table + (long)b * max_pages;
-  const shortx8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const float *brow =
       bias ? bias + (long)(kvh * G + min(l16, G - 1)) * bias_len : nullptr;
-  shortx8 kn[2][KT], vn[VU];
+  char *mine = patch[wave], *mine_k = mine + TK * VROW;
   float bn[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  // cache row of key lane & 31 of a tile, looked up a tile ahead
-  int page_id = 0;
-  auto key_of = [&](int k0) { return min(k0 + (lane & 31), t1 - 1); };
-  auto look_up = [&](int k0) { page_id = bt[key_of(k0) / page_size]; };
-  auto load = [&](int k0) {
-    const int krow = page_id * page_size + key_of(k0) % page_size;
-    // a table entry per key of this lane (before K and V: loads return in
-    // order)
+  // Cache row of key lane & 31 of a tile, its page looked up a tile ahead, into
+  // LDS like K and V: behind the next K and before the next V, so that the
+  // waits below can count what was issued behind what they need.
+  __shared__ int pages[WAVES][64];
+  int in_page = 0, krow = 0, rows[KU];
+  const unsigned k_bytes = num_kv_heads * Dr * 2;
+  const unsigned v_bytes = num_kv_heads * Dvr * 2;
+  const char *k_head = reinterpret_cast<const char *>(k_cache + kvh * Dr);
+  const char *v_head = reinterpret_cast<const char *>(v_cache + kvh * Dvr);
+  auto look_up = [&](int k0) {
+    const int key = min(k0 + (lane & 31), t1 - 1), page = key / page_size;
+    in_page = key - page * page_size;
+    fetch4(bt + page, pages[wave]);
+  };
+  // (columns beyond a head repeat its last unit)
+  auto load_k = [&](int k0) {
+    krow = pages[wave][lane] * page_size + in_page;
+    // a table entry per key of this lane
     if (brow) {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         bn[e] = brow[min(max(seq_len - 1 - (k0 + (e >> 2) * 16 + lhi * 4 +
                                             (e & 3)), 0), bias_len - 1)];
     }
-    // K: lane = key row l16 (+ 16), one 16 B unit per 32 dims; each row is
-    // read by exactly one wave: non-temporal
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
-      const __hip_bfloat16 *kp =
-          k_cache +
-          ((long)__shfl(krow, f * 16 + l16, 64) * num_kv_heads + kvh) * Dr +
-          lhi * 8;
+    for (int j = 0; j < KU; ++j)
+      rows[j] = __shfl(krow, (j * 64 + lane) / (D / 8), 64);
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-        kn[f][kt] = kt * 32 + lhi * 8 < Dr
-                        ? __builtin_nontemporal_load(
-                              reinterpret_cast<const shortx8 *>(kp + kt * 32))
-                        : zero;
+    for (int j = 0; j < KU; ++j) {
+      const int u = j * 64 + lane, r = u / (D / 8);
+      const int c = ((u % (D / 8)) ^ (r & KMASK)) * 8;
+      fetch16(k_head + (unsigned long)(unsigned)rows[j] * k_bytes +
+                  min(c, Dr - 8) * 2,
+              mine_k + j * 1024);
     }
+  };
+  auto load_v = [&]() {
 #pragma unroll
     for (int j = 0; j < VU; ++j) {
-      const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 8;
-      const __hip_bfloat16 *vp =
-          v_cache + ((long)__shfl(krow, r, 64) * num_kv_heads + kvh) * Dvr + c;
-      vn[j] = c < Dvr ? __builtin_nontemporal_load(
-                            reinterpret_cast<const shortx8 *>(vp))
-                      : zero;
+      const int u = j * 64 + lane, r = u / (DV / 8);
+      const int row = D == DV ? rows[j % KU] : __shfl(krow, r, 64);
+      const int c = ((u % (DV / 8)) ^ (r & VMASK)) * 8;
+      fetch16(v_head + (unsigned long)(unsigned)row * v_bytes +
+                  min(c, Dvr - 8) * 2,
+              mine + j * 1024);
     }
   };
   float qscale = scale * query_temp(seq_len - 1, temp_coef, temp_every);
@@ -330,14 +362,28 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   dec_f4 o[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) o[nt] = dec_f4{0, 0, 0, 0};
-  char *mine = patch[wave];
   const int tr_row = lhi * 4 + (l16 >> 2), tr_col = (l16 & 3) * 8;
 
+  // query fragments: column l16 = head, dims kt * 32 + lhi * 8
+  dec_bf8 qf[KT];
+  auto load_q = [&](const __hip_bfloat16 *heads, int stride) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      qf[kt] = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (l16 < G && kt * 32 + lhi * 8 < Dr)
+        qf[kt] = *reinterpret_cast<const dec_bf8 *>(heads + l16 * stride +
+                                                    kt * 32 + lhi * 8);
+    }
+  };
+  if constexpr (!FRESH)
+    load_q(q + (long)row * q_stride + (long)kvh * G * Dr, Dr);
   int k0 = t0 + wave * TK;
   if (k0 < t1) {
     look_up(k0);
-    load(k0);
-    if (k0 + WAVES * TK < t1) look_up(k0 + WAVES * TK);
+    wait_loads<0>();
+    load_k(k0);
+    look_up(k0 + WAVES * TK);
+    load_v();
   }
   // FRESH: the new rows are formed while the first tiles arrive
   __shared__ __attribute__((aligned(16))) short
@@ -373,29 +419,29 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
       return;
     }
   }
-  // query fragments: column l16 = head, dims kt * 32 + lhi * 8
-  dec_bf8 qf[KT];
+  if constexpr (FRESH) load_q(reinterpret_cast<const __hip_bfloat16 *>(own), D);
+  // (here, or each pass of the loop would wait for all that is on its way)
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt) {
-    qf[kt] = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (l16 < G && kt * 32 + lhi * 8 < Dr)
-      qf[kt] =
-          FRESH ? *reinterpret_cast<const dec_bf8 *>(own + l16 * D + kt * 32 +
-                                                     lhi * 8)
-                : *reinterpret_cast<const dec_bf8 *>(
-                      q + (long)row * q_stride + (kvh * G + l16) * Dr +
-                      kt * 32 + lhi * 8);
-  }
+  for (int kt = 0; kt < KT; ++kt) asm volatile("" : "+v"(qf[kt]));
   for (; k0 < t1; k0 += WAVES * TK) {
+    const bool more = k0 + WAVES * TK < t1;
     DecFrag kf[2][KT];
     float bv[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) bv[e] = bn[e] * LOG2E;
+    wait_loads<VU>();
 #pragma unroll
     for (int f = 0; f < 2; ++f)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
-        *reinterpret_cast<shortx8 *>(&kf[f][kt]) = kn[f][kt];
+        kf[f][kt].v = *reinterpret_cast<const dec_bf8 *>(
+            mine_k + (f * 16 + l16) * KROW +
+            ((kt * 64 + lhi * 16) ^ ((l16 & KMASK) << 4)));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) {
+      load_k(k0 + WAVES * TK);
+      look_up(k0 + 2 * WAVES * TK);
+    }
     if (FRESH && k0 + TK >= seq_len) {
       // the new token's row comes from LDS, and so does what stands behind
       // it in the tile (the cache's row may not be written yet)
@@ -404,25 +450,16 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
           if (k0 + f * 16 + l16 >= seq_len - 1 && kt * 32 + lhi * 8 < Dr)
-            *reinterpret_cast<shortx8 *>(&kf[f][kt]) =
-                *reinterpret_cast<const shortx8 *>(own + G * D + kt * 32 +
-                                                   lhi * 8);
-#pragma unroll
-      for (int j = 0; j < VU; ++j) {
-        const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 8;
-        if (k0 + r >= seq_len - 1 && c < Dvr)
-          vn[j] = *reinterpret_cast<const shortx8 *>(own + (G + 1) * D + c);
-      }
+            kf[f][kt].v = *reinterpret_cast<const dec_bf8 *>(
+                own + G * D + kt * 32 + lhi * 8);
     }
+    if (Dr < D) {
 #pragma unroll
-    for (int j = 0; j < VU; ++j) {
-      const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8) * 16;
-      *reinterpret_cast<shortx8 *>(mine + r * VROW +
-                                   (c ^ ((r & VMASK) << 4))) = vn[j];
-    }
-    if (k0 + WAVES * TK < t1) {
-      load(k0 + WAVES * TK);
-      if (k0 + 2 * WAVES * TK < t1) look_up(k0 + 2 * WAVES * TK);
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+          if (kt * 32 + lhi * 8 >= Dr)
+            kf[f][kt].v = dec_bf8{0, 0, 0, 0, 0, 0, 0, 0};
     }
 
     dec_f4 s[2];
@@ -466,19 +503,37 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
         pf.e[f * 4 + r] = __float2bfloat16(p);
       }
     l_run = l_run * alpha + sum;  // this lane's keys; joined at the end
+    if (more)
+      wait_loads<KU + 1>();
+    else
+      wait_loads<0>();
+    if (FRESH && k0 + TK >= seq_len) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      DecFrag vf;
+      for (int j = 0; j < VU; ++j) {
+        const int u = j * 64 + lane, r = u / (DV / 8), c = u % (DV / 8);
+        if (k0 + r >= seq_len - 1 && c * 8 < Dvr)
+          *reinterpret_cast<shortx8 *>(mine + r * VROW +
+                                       ((c ^ (r & VMASK)) << 4)) =
+              *reinterpret_cast<const shortx8 *>(own + (G + 1) * D + c * 8);
+      }
+    }
+    DecFrag vf[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int half = 0; half < 2; ++half)
-        vf.h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        vf[nt].h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (lds_shortx4 *)(mine + (half * 16 + tr_row) * VROW +
                             ((nt * 32 + tr_col) ^
                              ((tr_row & VMASK) << 4))));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) load_v();
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[nt][r] *= alpha;
-      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, o[nt], 0,
-                                                      0, 0);
+      o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[nt].v, pf.v, o[nt],
+                                                      0, 0, 0);
     }
   }
 
@@ -649,9 +704,8 @@ int splits_for(const torch::Tensor &k_cache, long B) {
     return e ? atoi(e) : 0;
   }();
   // Two workgroups fit a CU. Twice as many would even unequal requests out
-  // a little better (64 requests of 512 to 1536 keys, 8 heads: 62 us in two
-  // splits, 69 us in one; 24 of 2700 to 8100 115 us in eight, 121 in four)
-  // and are as exact: error against 64 bits 2.13e-3 in one split, 2.09e-3 in
+  // a little better (24 of 2700 to 7900 keys, 8 heads: 100 us in eight splits,
+  // 102 in four) and are as exact: error against 64 bits 2.13e-3 in one split, 2.09e-3 in
   // two; 2.15e-3 in four, 2.11e-3 in eight. But each split rounds its
   // probabilities to bf16 against its own maximum, so another count is
   // another result, and behind products that quantize their rows to e4m3 it
@@ -859,12 +913,13 @@ std::vector<torch::Tensor> qkv_decode_fp8(
 // Whether qkv_decode takes heads of this geometry, and is the faster form: its
 // rows cost each workgroup a few us, which pays while all of them are on the
 // chip at once (in two rounds if none waits for another's partials). (us of an
-// attention step, 40 heads on 8 of 128, two kernels or
-// three / this one: 1 sequence of 600 keys 13.2 / 12.6, 2 of 2400 19.8 / 17.5,
-// 16 of 340 to 880 21.4 / 20.1, 32 of 520 to 1500 41.5 / 39.5, 64 of them 64.4
-// / 61.4, 128 112.5 / 109.3, 64 of 150 to 450 27.8 / 25.7; 14 on 2 of 64, 64 of
-// 520 to 1500 18.7 / 16.9. Beyond: 48 of 520 to 1500 in two splits 60.4 / 61.6, 24 of 2700 to
-// 7900 in four 117.9 / 122.6, 256 of 150 to 450 74.6 / 77.9.)
+// attention step, 40 heads on 8 of 128, two kernels or three / this one: 1
+// sequence of 600 keys 13.9 / 12.8, 2 of 2400 19.4 / 18.1, 16 of 340 to 880
+// 19.4 / 18.9, 32 of 520 to 1500 36.5 / 34.6, 64 of them 54.8 / 51.5, 128 96.2
+// / 92.3, 64 of 150 to 450 24.3 / 21.8; 14 on 2 of 64, 64 of 520 to 1500 17.0 /
+// 15.5. Beyond: 48 of 520 to 1500 in two splits 50.0 / 50.6, 24 of 150 to 450
+// in four 21.6 / 24.2, of 2700 to 7900 101.9 / 102.1, 256 of 150 to 450 65.2 /
+// 67.1.)
 bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
                    long B) {
   const long Hkv = k_cache.size(2);
