@@ -95,23 +95,23 @@ class DenseAttention(nn.Module):
             if (hidden.dtype == torch.bfloat16 and ops.qkv_rope_cache_ok(
                     k_cache, v_cache, rope.cos_sin_cache, rope.is_neox)):
                 proj, bias = self.qkv_proj, self.qkv_proj.bias
-                src = proj.parts(rows)
+                src, rounded = proj.parts(rows), proj.fp8_block is not None
                 if src is None:
                     src, bias = proj.project(rows), None
                 elif fctx.is_pure_decode and ops.qkv_decode_ok(
-                        src, k_cache, attn.num_heads):
+                        src, k_cache, attn.num_heads, rounded):
                     return ops.qkv_decode(
                         src, bias, positions, rope.cos_sin_cache, k_cache,
                         v_cache, fctx.slot_mapping, fctx.block_table,
                         fctx.seq_lens,
                         fctx.arrivals(attn.num_kv_heads), attn.num_heads,
                         attn.scale, attn.sliding_window,
-                        rounded=proj.fp8_block is not None,
+                        rounded=rounded,
                         fp8=self.o_proj.takes_fp8(hidden))
                 q = ops.qkv_rope_cache(src, bias, positions,
                                        rope.cos_sin_cache, k_cache, v_cache,
                                        fctx.slot_mapping, attn.num_heads,
-                                       rounded=proj.fp8_block is not None)
+                                       rounded=rounded)
                 return attn.attend(q, fctx)
         q, k, v = self.qkv_proj(hidden)
         if self.qk_norm:

@@ -1131,11 +1131,11 @@ def qkv_rope_cache(src: torch.Tensor, bias, positions: torch.Tensor,
 
 
 def qkv_decode_ok(parts: torch.Tensor, k_cache: torch.Tensor,
-                  num_heads: int) -> bool:
+                  num_heads: int, rounded: bool = False) -> bool:
     """Whether ``qkv_decode`` takes these rows and heads (with caches that
     ``qkv_rope_cache_ok`` takes) and is the faster form."""
     return parts.dim() == 3 and _gpu_kernels().qkv_decode_ok(
-        k_cache, k_cache, num_heads, parts.shape[1])
+        k_cache, k_cache, num_heads, parts.shape[1], rounded)
 
 
 def qkv_decode(parts: torch.Tensor, bias, positions: torch.Tensor,

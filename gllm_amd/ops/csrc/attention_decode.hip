@@ -151,6 +151,8 @@ struct NewRows {
   const long *slots;               // [B] where its key and value go
   int *arrived;                    // [B, Hkv] zeros, left as zeros
   Fp8Out fp8;                      // the result's e4m3 rows (heads of 128)
+  // tiles up to which a sequence is not split, and a split's at least
+  int whole, least;
 };
 
 // partials pass from one workgroup to another within a launch: written
@@ -271,7 +273,10 @@ __global__ __launch_bounds__(BLOCK, 2) void paged_decode_kernel(
   const int w_begin = (window > 0) ? max(0, seq_len - window) : 0;
   // this split's share of the visible keys, whole tiles
   const int tiles = (seq_len - w_begin + TK - 1) / TK;
-  const int split_len = (tiles + num_splits - 1) / num_splits * TK;
+  const int even = (tiles + num_splits - 1) / num_splits;
+  const int split_len =
+      TK * (!FRESH ? even
+                   : tiles <= fresh.whole ? tiles : max(even, fresh.least));
   // split == num_splits (launched only when keep_first > 0) is the
   // kept-first segment [0, min(keep_first, w_begin)): tokens that stay
   // visible outside the window; its partial merges like any other
@@ -767,7 +772,23 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      keep_first, softcap, bias, bias_len, temp_coef,         \
                      temp_every, qsl, direct, out_stride, sink ? 1 : 0,      \
                      sinks, (const __hip_bfloat16 *)gate, gate_stride, B,    \
-                     zdim, order_above, fresh ? *fresh : NewRows{})
+                     zdim, order_above, rows)
+  // A split's rows, partials and the join take 3 us, as long as a wave takes
+  // for one or two tiles while most of the chip idles, for two to four in one
+  // round of workgroups and for six beside others (us, 40 heads on 8 of 128,
+  // every sequence over all splits / so: 4 of 520 to 1500 keys 17.7 / 15.2, 16
+  // of 150 to 450 15.8 / 12.8, 12 of them 22.6 / 12.6, 12 of 520 to 1500 28.4 /
+  // 21.2, 24 of 60 to 180 21.1 / 10.2, 31 of 150 to 450 25.8 / 14.7, 60 of 600
+  // 40.2 / 30.5, 9 of 5400 46.9 / 43.8; 24 of 2700 to 7900 102.5 / 102.8. 24
+  // tiles in one round: 8 of 520 to 1500 20.4 for 18.8; 16 beyond: 60 of 600
+  // 40.2). Rounded rows stand behind e4m3 products: there the count stays
+  // (splits_for).
+  NewRows rows = fresh ? *fresh : NewRows{};
+  if (fresh && !fresh->rows.rounded) {
+    const long all = (long)B * Hkv * splits;
+    rows.whole = all <= ALONE ? 8 : all <= 2 * ALONE ? 16 : 24;
+    rows.least = all <= ALONE ? 4 : all <= 2 * ALONE ? 8 : 24;
+  }
   if (fresh) { if (D <= 64) RUN(64, 64, true); else RUN(128, 128, true); }
   else if (D <= 64) { if (Dv <= 64) RUN(64, 64); else RUN(64, 128); }
   else { if (Dv <= 64) RUN(128, 64); else RUN(128, 128); }
@@ -870,7 +891,7 @@ static torch::Tensor decode_rows(
                        (int)parts.size(0), rot, (int)rounded},
                       (__hip_bfloat16 *)k_cache.data_ptr(),
                       (__hip_bfloat16 *)v_cache.data_ptr(),
-                      slots.data_ptr<long>(), arrived.data_ptr<int>(), fp8};
+                      slots.data_ptr<long>(), arrived.data_ptr<int>(), fp8, 0, 0};
   launch_decode(out, out, k_cache, v_cache, block_table, seq_lens, Hq / Hkv,
                 (float)scale, (int)sliding_window, 0, false, nullptr, 0,
                 nullptr, 0.f, nullptr, 0, 0.f, 0, nullptr, &fresh);
@@ -911,23 +932,23 @@ std::vector<torch::Tensor> qkv_decode_fp8(
 }
 
 // Whether qkv_decode takes heads of this geometry, and is the faster form: its
-// rows cost each workgroup a few us, which pays while all of them are on the
-// chip at once (in two rounds if none waits for another's partials). (us of an
-// attention step, 40 heads on 8 of 128, two kernels or three / this one: 1
-// sequence of 600 keys 13.9 / 12.8, 2 of 2400 19.4 / 18.1, 16 of 340 to 880
-// 19.4 / 18.9, 32 of 520 to 1500 36.5 / 34.6, 64 of them 54.8 / 51.5, 128 96.2
-// / 92.3, 64 of 150 to 450 24.3 / 21.8; 14 on 2 of 64, 64 of 520 to 1500 17.0 /
-// 15.5. Beyond: 48 of 520 to 1500 in two splits 50.0 / 50.6, 24 of 150 to 450
-// in four 21.6 / 24.2, of 2700 to 7900 101.9 / 102.1, 256 of 150 to 450 65.2 /
-// 67.1.)
+// rows cost each workgroup a few us, which pays in up to two rounds of
+// workgroups; rounded, with all sequences in all splits, in one if they are
+// split. (us of an attention step, 40 heads on 8 of 128, two kernels or three /
+// this one: 1 sequence of 600 keys 13.9 / 12.8, 2 of 2400 19.4 / 18.1, 16 of 340
+// to 880 19.4 / 18.9, 24 of 150 to 450 21.5 / 13.5, of 2700 to 7900 102.3 /
+// 102.8, 32 of 520 to 1500 36.5 / 34.6, 60 of them 56.1 / 58.1, of 150 to 450
+// 30.2 / 21.2, 64 of 520 to 1500 54.8 / 51.5, 128 96.2 / 92.3; 14 on 2 of 64, 64
+// of 520 to 1500 17.0 / 15.5. Beyond: 256 of 150 to 450 65.2 / 67.1. Rounded: 24
+// of 150 to 450 in four splits 21.6 / 24.2.)
 bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
-                   long B) {
+                   long B, bool rounded) {
   const long Hkv = k_cache.size(2);
   const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
   const int splits = splits_for(k_cache, B);
   return decode_rows_ok(k_cache, v_cache, Hq) &&
          k_cache.sizes() == v_cache.sizes() &&
-         B * Hkv * splits <= (splits > 1 ? 2L : 4L) * cus;
+         B * Hkv * splits <= (rounded && splits > 1 ? 2L : 4L) * cus;
 }
 
 // whether the decode kernel takes heads of this geometry (a mixed batch

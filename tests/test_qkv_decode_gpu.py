@@ -1,6 +1,7 @@
 """Decode attention straight from a projection's parts against the two
 kernels that it stands for: the same sums in the same order, so the same
-bits, in the caches too."""
+bits, in the caches too; rows that are not rounded may be split less, and
+then each form's weights are rounded to bf16 against another maximum."""
 
 import pytest
 import torch
@@ -68,6 +69,9 @@ CASES = [
     (40, 32, 8, 128, 128, 7, [1 + 97 * i for i in range(40)], 0),  # in order
     (9, 14, 2, 64, 64, 3, [300, 1, 17, 64, 65, 900, 2, 33, 500], 100),
     (2, 4, 4, 96, 96, 2, [48, 1025], 0),
+    # tiles up to which a sequence is not split, and a split's at least
+    (4, 8, 8, 64, 64, 2, [256, 257, 384, 4000], 0),
+    (12, 16, 8, 128, 128, 2, [768, 769, 1536, 1537, 40, 3000] * 2, 0),
 ]
 
 
@@ -78,8 +82,11 @@ def test_as_two_kernels(B, Hq, Hkv, D, rot, S, lens, window, rounded):
     arrived = torch.zeros(B * Hkv, dtype=torch.int32, device="cuda")
     for bias in (True, False):
         got, want = _both(s, Hq, D, window, rounded, bias, arrived)
-        for a, b in zip(got, want):
+        for a, b in zip(got[0 if rounded else 1:], want[0 if rounded else 1:]):
             assert torch.equal(a, b)
+        # weights and results of both forms, 2^-9 relative each
+        err = (got[0].double() - want[0].double()).norm()
+        assert err <= 2 ** -7 * want[0].double().norm()
         assert not arrived.any()
 
 
@@ -88,7 +95,7 @@ def test_replayed():
     from gllm_amd import ops
     s = _step(6, 32, 8, 128, 128, 6, [600, 1, 40, 1300, 33, 256])
     arrived = torch.zeros(48, dtype=torch.int32, device="cuda")
-    _, want = _both(s, 32, 128, 0, False, True, arrived)
+    want, _ = _both(s, 32, 128, 0, False, True, arrived)
 
     def call():
         return ops.qkv_decode(s["parts"], s["bias"], s["positions"],
