@@ -22,7 +22,7 @@ page tables: 0.13 ms for 64 requests of 64 pages, 0.5 ms for 256.
 
 import contextlib
 import gc
-from typing import Dict, List, Optional
+from typing import Dict, List, Optional, Tuple
 
 import numpy as np
 import torch
@@ -54,10 +54,11 @@ class GraphRunner:
         cfg = runner.config
         self.device = cfg.device
         self.buckets = [b for b in DECODE_BUCKETS if b <= cfg.max_graph_bs]
-        self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
+        # a graph and its forward's context: what a captured forward counts
+        # in must live as long as the graph
+        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph,
+                                     ForwardContext]] = {}
         self.hidden_out: Dict[int, torch.Tensor] = {}
-        # (what a captured forward counts in must live as long as its graph)
-        self.contexts: Dict[int, ForwardContext] = {}
         self.captured = False
         self.max_bs = self.buckets[-1]
         max_len = cfg.model_max_length or 32768
@@ -165,9 +166,8 @@ class GraphRunner:
             with torch.cuda.graph(g, pool=pool, stream=stream):
                 ids = runner.resolve_tokens(self.in_ids[:bs])
                 hidden, _ = runner.model(ids, pos, fctx)
-            self.graphs[bs] = g
+            self.graphs[bs] = g, fctx
             self.hidden_out[bs] = hidden
-            self.contexts[bs] = fctx
 
     # ------------------------------------------------------------------
     def can_replay(self, batch) -> bool:
@@ -247,7 +247,7 @@ class GraphRunner:
     def replay(self, batch):
         items = batch.items
         bs = self._stage(items)
-        self.graphs[bs].replay()
+        self.graphs[bs][0].replay()
         hidden = self.hidden_out[bs][:len(items)]
         fctx = self._fctx_for(bs)
         fctx.logits_indices = None  # hidden already one row per seq
