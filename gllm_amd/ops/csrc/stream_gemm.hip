@@ -341,27 +341,35 @@ double fill_of(int tiles, int slots) {
 
 // What a tile costs is the stages it has in flight and how evenly the tiles
 // fill the chip: a product runs in one round of workgroups that are all there
-// from the start (two a CU for 16 rows and for 64 columns, else one), split
+// from the start (two a CU for 16 rows, else one), split
 // along K into as many as fit that round. Rounding up instead (to about 384
 // workgroups of 64 columns) left a second round nearly empty or half the CUs
 // with twice the work. us in turn over weights that no cache holds, before /
 // now, with the norm or the bias behind them:
+//  * up to 64 rows, below 20 M values (6 M for 16 rows): 64 columns, a
+//    workgroup a CU while there are that few tiles. A second one doubles the
+//    parts and brings no weight sooner: 64 x 4096 x 4096 16.7 / 13.6, 32 x 3648
+//    x 2048 9.3 / 8.0, 64 x 2560 x 2560 13.3 / 10.9, 2048 x 2048 9.6 both.
 //  * up to 64 rows, large weights: 128 columns. 1 x 6144 x 4096 11.8 / 10.0,
 //    64 x 5120 x 5120 23.2 / 20.2, 64 x 4096 x 14336 36.5 / 28.7, 1 x 8192 x
-//    8192 32.4 / 28.2. 64 columns stay where that is small (below 6 M values
-//    for 16 rows, 20 M above: 2048 x 2048 7.0 both) or where 64 columns fill
+//    8192 32.4 / 28.2. 64 columns stay where they fill
 //    nine tenths of 512 workgroups unsplit (32064 x 4096); 256 columns where
 //    they fill the chip better by a tenth: 64 x 19008 x 5120 60 / 44.
 //  * up to 128 rows 128 x 128 from 20 M values on, one row block in place of
 //    two of 64: 128 x 6144 x 4096 21.6 / 16.4, 19008 x 5120 79 / 60.
-//  * up to 256 rows, narrow: 128 columns, 64 rows below 12 M values: 256 x
-//    2048 x 2816 19.6 / 15.6, 160 x 4096 x 4096 26.3 / 22.7. Rounding up stays
-//    for 256 x 128 tiles (160 x 19008 x 5120 58; unsplit 74).
+//    Below, two row blocks of 64 x 64 where they fill six tenths of the CUs
+//    (128 x 2048 x 2048 12.9 / 10.4, 128 x 5120 x 2048 15.2 / 12.1, 128 x 3648 x
+//    2048 13.8 / 11.5, 72 x 4096 x 4096 16.1 / 16.4), else 128 x 64: 128 x 4608
+//    x 3584 at 144 tiles 13.7, 64 x 64 over 15; 10000 x 1536 15.8, 18.3.
+//  * up to 256 rows, narrow: below 12 M values 64 x 64 where they fill two
+//    thirds of the CUs (256 x 2048 x 2048 14.3 / 12.4, 160 x 3648 x 2048 15.1 /
+//    11.9), else 128 x 64 (256 x 2560 x 2048 9.8 / 8.9); above 128 x 128.
+//    Rounding up stays for 256 x 128 tiles (160 x 19008 x 5120 58; unsplit 74).
 //  * gated (not split): by whole rounds too, 128 columns where 64 leave the
 //    second round thin (64 x 22016 x 4096 44.5 / 38.2, 128 x 28672 x 4096 60 /
 //    50), 256 from 36000 columns on (one row: from 48000, 55296 x 5120 96 / 89;
 //    43008 x 4096 keeps 128 columns, 74 / 70).
-// 28 to 32 tiles take at most 8 splits, a workgroup a CU: 4096 x 4096 11.6
+// 28 to 32 tiles take at most 8 splits, a workgroup a CU: 1 x 4096 x 4096 11.6
 // against 13.1 with 16, whose sums then cost more than the stages they save;
 // 40 tiles don't gain by a cap of 8 (5120 x 5120 15.7 / 16.6, K 27648 50 / 59).
 // Each part has four stages at least.
@@ -388,6 +396,7 @@ Plan plan_for(int M, int N, int K, bool gated) {
     p.bn = p.bm == 128 ? 64 : N >= 36000 ? 256 : 128;
   } else if (M <= 64) {
     const bool small = weights < (p.bm == 16 ? 6L << 20 : 20L << 20);
+    if (small && tiles64 <= 256) slots = 256;
     if (!small && !even) {
       p.bn = 128;
       if (p.bm > 16) {
@@ -400,14 +409,17 @@ Plan plan_for(int M, int N, int K, bool gated) {
   } else if (M <= 128) {
     slots = 256;
     p.bn = N >= 36000 ? 256 : weights >= (20L << 20) ? 128 : 64;
+    if (p.bn == 64 && tiles64 <= 128 && fill_of(2 * tiles64, 256) >= 0.6)
+      p.bm = 64;
   } else {
     slots = 256;
     if (N >= 16384 || (K >= 2 * N && N >= 5120)) {
       p.bm = 256;
       p.bn = 128;
     } else if (N < 5120) {
-      p.bn = 128;
-      if (weights < (12L << 20)) p.bm = 64;
+      const int tiles = (M + 63) / 64 * tiles64;
+      if (weights >= (12L << 20)) p.bn = 128;
+      else if (tiles <= 256 && fill_of(tiles, 256) >= 0.65) p.bm = 64;
     }
   }
   p.nbm = (M + p.bm - 1) / p.bm;

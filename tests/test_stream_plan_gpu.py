@@ -27,6 +27,8 @@ def _close(got, want):
     (32, 5128, 4160), (17, 18952, 1152),
     (64, 5128, 4160), (33, 18952, 1152),
     (128, 5128, 4160), (65, 1032, 1088),
+    (33, 4104, 4096), (24, 12296, 1024), (100, 2048, 2112), (72, 5128, 640),
+    (160, 2056, 1088), (256, 2568, 704), (129, 4104, 2048),
     (129, 1032, 1088), (256, 4104, 3136), (200, 5128, 10304)])
 def test_plain(M, N, K):
     from gllm_amd import ops
