@@ -6,7 +6,7 @@ read from a global.
 """
 
 import dataclasses
-from typing import List, Optional
+from typing import Dict, List, Optional
 
 import torch
 
@@ -68,18 +68,32 @@ class ForwardContext:
     _per_head_from: Optional[tuple] = dataclasses.field(default=None,
                                                         kw_only=True)
 
-    _arrivals: Optional[torch.Tensor] = dataclasses.field(default=None,
-                                                          kw_only=True)
+    # zeros of the owner of a captured forward, who keeps them as long as the
+    # graph (see arrivals)
+    arrived: Optional[torch.Tensor] = dataclasses.field(default=None,
+                                                        kw_only=True)
+    _arrivals: Dict[int, torch.Tensor] = dataclasses.field(
+        default_factory=dict, kw_only=True)
 
     def arrivals(self, kv_heads: int) -> torch.Tensor:
-        """Zeros that this forward's split decode attention counts its
-        workgroups in and leaves as zeros (its layers follow one another; a
-        captured forward keeps its own)."""
+        """Zeros that split decode attention counts its workgroups in and
+        leaves as zeros. The layers of a forward follow one another and share
+        them; forwards on two streams do not, and a graph may outlive this
+        context, so what a capture counts in is ``arrived`` or the graph's
+        own."""
         n = self.seq_lens.shape[0] * kv_heads
-        if self._arrivals is None or self._arrivals.numel() < n:
-            self._arrivals = torch.zeros(n, dtype=torch.int32,
-                                         device=self.seq_lens.device)
-        return self._arrivals
+        zeros = self.arrived
+        if zeros is not None and zeros.numel() >= n:
+            return zeros
+        if torch.cuda.is_current_stream_capturing():
+            return torch.zeros(n, dtype=torch.int32,
+                               device=self.seq_lens.device)
+        stream = torch.cuda.current_stream().cuda_stream
+        zeros = self._arrivals.get(stream)
+        if zeros is None or zeros.numel() < n:
+            zeros = self._arrivals[stream] = torch.zeros(
+                n, dtype=torch.int32, device=self.seq_lens.device)
+        return zeros
 
     def prompts_from(self) -> int:
         """The first sequence from which on all are whole prompts: two rows

@@ -22,7 +22,7 @@ page tables: 0.13 ms for 64 requests of 64 pages, 0.5 ms for 256.
 
 import contextlib
 import gc
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, Optional
 
 import numpy as np
 import torch
@@ -49,15 +49,16 @@ def _collector_held():
 
 
 class GraphRunner:
+    # what the captured forwards' decode attention counts in; the graphs are
+    # replayed one behind the other
+    arrived: Optional[torch.Tensor] = None
+
     def __init__(self, runner):
         self.runner = runner
         cfg = runner.config
         self.device = cfg.device
         self.buckets = [b for b in DECODE_BUCKETS if b <= cfg.max_graph_bs]
-        # a graph and its forward's context: what a captured forward counts
-        # in must live as long as the graph
-        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph,
-                                     ForwardContext]] = {}
+        self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self.hidden_out: Dict[int, torch.Tensor] = {}
         self.captured = False
         self.max_bs = self.buckets[-1]
@@ -123,7 +124,8 @@ class GraphRunner:
             query_start_loc=self.qsl[:bs + 1],
             max_query_len=1, max_seq_len=1,
             k_caches=self.runner.k_caches,
-            v_caches=self.runner.v_caches)
+            v_caches=self.runner.v_caches,
+            arrived=self.arrived)
         if self.ssm_slots_dev is not None:
             fctx.ssm_pool = self.runner.ssm_pool
             fctx.ssm_slots_dev = self.ssm_slots_dev[:bs]
@@ -139,6 +141,9 @@ class GraphRunner:
         base = self.dummy_page * runner.config.page_size
         ps = runner.config.page_size
         self.slots.copy_(base + torch.arange(self.max_bs) % ps)
+        heads = max((c.shape[2] for c in runner.k_caches
+                     if c is not None and c.dim() == 4), default=0)
+        self.arrived = self.seq_lens.new_zeros(self.max_bs * heads)
         pool = torch.cuda.graphs.graph_pool_handle()
         stream = torch.cuda.Stream()
         torch.cuda.synchronize()
@@ -166,7 +171,7 @@ class GraphRunner:
             with torch.cuda.graph(g, pool=pool, stream=stream):
                 ids = runner.resolve_tokens(self.in_ids[:bs])
                 hidden, _ = runner.model(ids, pos, fctx)
-            self.graphs[bs] = g, fctx
+            self.graphs[bs] = g
             self.hidden_out[bs] = hidden
 
     # ------------------------------------------------------------------
@@ -247,7 +252,7 @@ class GraphRunner:
     def replay(self, batch):
         items = batch.items
         bs = self._stage(items)
-        self.graphs[bs][0].replay()
+        self.graphs[bs].replay()
         hidden = self.hidden_out[bs][:len(items)]
         fctx = self._fctx_for(bs)
         fctx.logits_indices = None  # hidden already one row per seq
