@@ -113,7 +113,7 @@ class DenseAttention(nn.Module):
                                        fctx.slot_mapping, attn.num_heads,
                                        rounded=rounded)
                 return attn.attend(q, fctx)
-        q, k, v = self.qkv_proj(hidden)
+        q, k, v = self.qkv_proj(rows)
         if self.qk_norm:
             T = q.shape[0]
             q = self.q_norm(
