@@ -238,20 +238,22 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
   const long row = blockIdx.x;
   const long MN = (long)M * N;
   // every load goes out before the first sum (columns past the row's end
-  // repeat its last four)
-  const float *p[V];
-  shortx4 old[V];
-  float wv[V][4];
+  // repeat its last four; threads with none of their own load nothing)
+  shortx4 old[V] = {};
+  float wv[V][4] = {};
+  st_f4 v[V] = {};
+  if ((int)threadIdx.x * 4 < N) {
+    const float *p[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) {
-    const int c = min((j * 512 + (int)threadIdx.x) * 4, N - 4);
-    p[j] = part + row * N + c;
-    old[j] = *reinterpret_cast<const shortx4 *>(residual + row * N + c);
+    for (int j = 0; j < V; ++j) {
+      const int c = min((j * 512 + (int)threadIdx.x) * 4, N - 4);
+      p[j] = part + row * N + c;
+      old[j] = *reinterpret_cast<const shortx4 *>(residual + row * N + c);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) wv[j][r] = ScalarOps<TW>::to_f32(w[c + r]);
+      for (int r = 0; r < 4; ++r) wv[j][r] = ScalarOps<TW>::to_f32(w[c + r]);
+    }
+    part_sums<V>(p, MN, S, v);
   }
-  st_f4 v[V];
-  part_sums<V>(p, MN, S, v);
   float x[V][4], ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V; ++j) {
