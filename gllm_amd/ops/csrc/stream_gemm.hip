@@ -8,8 +8,9 @@
 // by row & 7, so fragment reads fall on all banks; products are W x^T, so a
 // lane ends with four neighbouring columns of one row.
 //
-// A weight with few tiles is also split along K (plan_for: into one full round
-// of workgroups); the fp32 parts [S, M, N] are then summed by whatever comes next, in the order of S:
+// A weight with few tiles is also split along K (parts_plan: into one full
+// round of workgroups); the fp32 parts [S, M, N] are then summed by whatever
+// comes next, in the order of S:
 //   stream_gemm           bias, bf16
 //   stream_add_norm       residual += sum, RMS norm of it (attention and
 //                         feed-forward outputs)
@@ -341,102 +342,170 @@ double fill_of(int tiles, int slots) {
                         : (double)tiles / (rounds * slots);
 }
 
-// What a tile costs is the stages it has in flight and how evenly the tiles
-// fill the chip: a product runs in one round of workgroups that are all there
-// from the start (two a CU for 16 rows, else one), split
-// along K into as many as fit that round. Rounding up instead (to about 384
-// workgroups of 64 columns) left a second round nearly empty or half the CUs
-// with twice the work. us in turn over weights that no cache holds, before /
-// now, with the norm or the bias behind them:
-//  * up to 64 rows, below 20 M values (6 M for 16 rows): 64 columns, a
-//    workgroup a CU while there are that few tiles. A second one doubles the
-//    parts and brings no weight sooner: 64 x 4096 x 4096 16.7 / 13.6, 32 x 3648
-//    x 2048 9.3 / 8.0, 64 x 2560 x 2560 13.3 / 10.9, 2048 x 2048 9.6 both.
-//  * up to 64 rows, large weights: 128 columns. 1 x 6144 x 4096 11.8 / 10.0,
-//    64 x 5120 x 5120 23.2 / 20.2, 64 x 4096 x 14336 36.5 / 28.7, 1 x 8192 x
-//    8192 32.4 / 28.2. 64 columns stay where they fill
-//    nine tenths of 512 workgroups unsplit (32064 x 4096); 256 columns where
-//    they fill the chip better by a tenth: 64 x 19008 x 5120 60 / 44.
-//  * up to 128 rows 128 x 128 from 20 M values on, one row block in place of
-//    two of 64: 128 x 6144 x 4096 21.6 / 16.4, 19008 x 5120 79 / 60.
-//    Below, two row blocks of 64 x 64 where they fill six tenths of the CUs
-//    (128 x 2048 x 2048 12.9 / 10.4, 128 x 5120 x 2048 15.2 / 12.1, 128 x 3648 x
-//    2048 13.8 / 11.5, 72 x 4096 x 4096 16.1 / 16.4), else 128 x 64: 128 x 4608
-//    x 3584 at 144 tiles 13.7, 64 x 64 over 15; 10000 x 1536 15.8, 18.3.
-//  * up to 256 rows, narrow: below 12 M values 64 x 64 where they fill two
-//    thirds of the CUs (256 x 2048 x 2048 14.3 / 12.4, 160 x 3648 x 2048 15.1 /
-//    11.9), else 128 x 64 (256 x 2560 x 2048 9.8 / 8.9); above 128 x 128.
-//    Rounding up stays for 256 x 128 tiles (160 x 19008 x 5120 58; unsplit 74).
-//  * gated (not split): by whole rounds too, 128 columns where 64 leave the
-//    second round thin (64 x 22016 x 4096 44.5 / 38.2, 128 x 28672 x 4096 60 /
-//    50), 256 from 36000 columns on (one row: from 48000, 55296 x 5120 96 / 89;
-//    43008 x 4096 keeps 128 columns, 74 / 70).
-// 28 to 32 tiles take at most 8 splits, a workgroup a CU: 1 x 4096 x 4096 11.6
-// against 13.1 with 16, whose sums then cost more than the stages they save;
-// 40 tiles don't gain by a cap of 8 (5120 x 5120 15.7 / 16.6, K 27648 50 / 59).
-// Each part has four stages at least.
-Plan plan_for(int M, int N, int K, bool gated) {
-  Plan p;
-  const long weights = (long)N * K;
-  const int tiles64 = (N + 63) / 64;
-  const bool even = tiles64 > 256 && (fill_of(tiles64, 512) >= 0.9 ||
-                                      (M <= 16 && tiles64 <= 512 &&
-                                       K < 4096));
-  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
-  p.bn = 64;
-  int slots = 512;
-  if (gated && M <= 64) {
-    if (N >= (p.bm == 16 ? 48000 : 36000)) p.bn = 256;
-    else if (N >= 16384 && !even &&
-             (p.bm == 64 ? N <= 32768 : fill_of(tiles64, 512) < 0.8))
-      p.bn = 128;
-  } else if (gated && M <= 128) {
-    p.bm = N >= 8192 ? 128 : 64;
-    p.bn = N >= 36000 ? 256 : N >= 16384 && N <= 32768 ? 128 : 64;
-  } else if (gated) {
-    p.bm = K >= 2 * N || N >= 16384 ? 256 : 128;
-    p.bn = p.bm == 128 ? 64 : N >= 36000 ? 256 : 128;
-  } else if (M <= 64) {
-    const bool small = weights < (p.bm == 16 ? 6L << 20 : 20L << 20);
-    if (small && tiles64 <= 256) slots = 256;
-    if (!small && !even) {
-      p.bn = 128;
-      if (p.bm > 16) {
-        slots = 256;
-        if (N >= 8192 && fill_of((N + 255) / 256, 256) >
-                             fill_of((N + 127) / 128, 256) + 0.1)
-          p.bn = 256;
-      }
-    }
-  } else if (M <= 128) {
-    slots = 256;
-    p.bn = N >= 36000 ? 256 : weights >= (20L << 20) ? 128 : 64;
-    if (p.bn == 64 && tiles64 <= 128 && fill_of(2 * tiles64, 256) >= 0.6)
-      p.bm = 64;
-  } else {
-    slots = 256;
-    if (N >= 16384 || (K >= 2 * N && N >= 5120)) {
-      p.bm = 256;
-      p.bn = 128;
-    } else if (N < 5120) {
-      const int tiles = (M + 63) / 64 * tiles64;
-      if (weights >= (12L << 20)) p.bn = 128;
-      else if (tiles <= 256 && fill_of(tiles, 256) >= 0.65) p.bm = 64;
-    }
-  }
+int compute_units() {
+  return at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+}
+
+Plan finish(Plan p, int M, int N, int K, int splits) {
+  const int stages = K / BK, per = (stages + splits - 1) / splits;
   p.nbm = (M + p.bm - 1) / p.bm;
   p.nbn = (N + p.bn - 1) / p.bn;
-  const int tiles = p.nbm * p.nbn, stages = K / BK;
-  int s = 1;
-  if (!gated) {
-    s = std::min(slots / tiles, MAX_SPLIT);
-    if (p.bm == 256 && tiles < 160) s = (384 + tiles - 1) / tiles;
-    if (tiles >= 28 && tiles <= 32) s = std::min(s, 8);
-    s = std::max(1, std::min(s, stages / 4));
-  }
-  const int per = (stages + s - 1) / s;
   p.k_slice = per * BK;
   p.splits = (stages + per - 1) / per;
+  return p;
+}
+
+// Rows 4 KB apart, and parts whose shares are, meet in the same channels of
+// memory: there fewer and narrower streams are the faster ones (us, four parts
+// of K 8192 / three: 64 x 8192 x 8192 39.9 / 33.6, 64 x 7168 x 8192 35.2 /
+// 32.5; two 64-column tiles a CU against one of 128, rows 8 KB apart: 48 x
+// 28672 x 4096 gated 46 / 49, 10 KB apart 66 / 57).
+bool far_apart(int values) { return values % 2048 == 0; }
+
+// From here on 64-column tiles of up to 64 rows are not left whole (17 x 16384
+// x 14336 92, in two parts 76).
+constexpr int DEEP = 12288;
+
+// Gated products are not split: the width whose tiles fill whole rounds of
+// workgroups (us). 64 columns with a tile a CU and no more (64 x 16384 x 3584
+// 23, 128 columns 33; 128 x 16384 x 2048 20, 25), then 128 until 64 nearly fill
+// two (64 x 22016 x 4096 44.5, 128 columns 38.2; 128 x 28672 x 4096 60, 50; 33
+// x 28672 x 4096 44, 48), 256 from 36000 columns on. Up to 16 rows 128 there,
+// 256 from 48000 unless rows are 4 KB apart (1 x 55296 x 5120 100 / 95, 1 x
+// 43008 x 4096 70 / 74, 1 x 57344 x 4096 81 / 97, 64 columns 87).
+Plan gated_plan(int M, int N, int K) {
+  const int cus = compute_units(), tiles64 = (N + 63) / 64;
+  const double fill = fill_of(tiles64, 2 * cus);
+  const bool far = far_apart(K);
+  Plan p;
+  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  p.bn = 64;
+  if (M <= 64) {
+    const double full = p.bm == 64 ? (far ? 0.85 : 0.9) : far ? 0.74 : 0.8;
+    const bool even =
+        fill >= full || (M <= 16 && tiles64 <= 2 * cus && K < 4096);
+    if (N >= 36000)
+      p.bn = p.bm > 16 || (N >= 48000 && !far) ? 256 : 128;
+    else if (tiles64 >= cus && tiles64 <= 2 * cus && !even)
+      p.bn = 128;
+  } else if (M <= 128) {
+    p.bm = N >= 8192 ? 128 : 64;
+    p.bn = N >= 36000 ? 256
+           : tiles64 > cus && tiles64 <= 2 * cus ? 128 : 64;
+  } else {
+    p.bm = K >= 2 * N || N >= 16384 ? 256 : 128;
+    p.bn = p.bm == 128 ? 64 : N >= 36000 ? 256 : 128;
+  }
+  return finish(p, M, N, K, 1);
+}
+
+// Products that may be split: in one round of a workgroup a CU, all there from
+// the start, along K into as many parts as fit that round. Rounding up instead
+// (to about 384 workgroups of 64 columns) left a second round nearly empty or
+// half the CUs with twice the work, and a second workgroup a CU doubles the
+// parts and brings no weight sooner. us in turn over weights that no cache
+// holds, with the norm or the bias behind them:
+//  * parts, rounded up / two a CU / one a CU: 1 x 5120 x 5120 17.1 / 15.8 /
+//    14.4, 16 x 2560 x 8192 16.2 / 16.4 / 14.0, 1 x 4608 x 14336 29.5 / 28.0 /
+//    26.3. Up to 16 rows take two where one leaves three tenths of the CUs
+//    idle (16 x 18432 x 14336 in one part 118, in three 97).
+//  * up to 64 rows: 64 columns below 20 M values (6 M for 16 rows; 64 x 4096 x
+//    4096 16.7 / 13.6, 32 x 3648 x 2048 9.3 / 8.0, 64 x 2560 x 2560 13.3 /
+//    10.9), where the most parts of 128 would leave a quarter of the CUs idle
+//    (32 x 768 x 27648 128 columns 19.3, 64 14.4), and where they fill a round
+//    of two a CU unsplit (32064 x 4096). Else 128 (1 x 6144 x 4096 11.8 / 10.0,
+//    64 x 5120 x 5120 23.2 / 20.2, 64 x 4096 x 14336 36.5 / 28.7), or 256 where
+//    they fill the chip better by a tenth (64 x 19008 x 5120 60 / 44). Beyond a
+//    round of two a CU 64 up to 16 rows (1 x 38016 x 4096 128 columns 71, 64
+//    59), else 256 (64 x 64128 x 5120 64 columns 140, 256 105).
+//  * up to 128 rows 128 x 128 from 20 M values on, one row block in place of
+//    two of 64: 128 x 6144 x 4096 21.6 / 16.4. Below, two row blocks of 64 x
+//    64 where they fill six tenths of the CUs (128 x 2048 x 2048 12.9 / 10.4,
+//    128 x 5120 x 2048 15.2 / 12.1, 128 x 3648 x 2048 13.8 / 11.5), else 128 x
+//    64: 128 x 4608 x 3584 at 144 tiles 13.7, 64 x 64 over 15.
+//  * up to 256 rows, narrow: below 12 M values 64 x 64 where they fill two
+//    thirds of the CUs (256 x 2048 x 2048 14.3 / 12.4, 160 x 3648 x 2048 15.1 /
+//    11.9), else 128 x 64 (256 x 2560 x 2048 9.8 / 8.9); above 128 x 128, but
+//    256 x 128 for few columns and long K (136 x 1536 x 14336 29.0 / 24.2).
+//    Rounding up stays for 256 x 128 tiles (160 x 19008 x 5120 58; unsplit 74).
+// From 16384 columns on the router has the library for more than 64 rows; only
+// a caller of the kernel itself gets there. A part has four stages at least on
+// average; the last may be shorter (17 stages: 5, 5, 5, 2).
+Plan parts_plan(int M, int N, int K) {
+  const int cus = compute_units(), stages = K / BK;
+  const long weights = (long)N * K;
+  const int tiles64 = (N + 63) / 64, tiles128 = (N + 127) / 128;
+  Plan p;
+  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  p.bn = 64;
+  if (M <= 64) {
+    const bool even = tiles64 >= cus && tiles64 <= 2 * cus && K < DEEP &&
+                      (fill_of(tiles64, 2 * cus) >=
+                           (far_apart(K) ? 0.74 : 0.9) ||
+                       (M <= 16 && K < 4096));
+    const bool small = weights < (p.bm == 16 ? 6L << 20 : 20L << 20) ||
+                       tiles128 * MAX_SPLIT < cus * 3 / 4;
+    if (tiles64 > 2 * cus) {
+      p.bn = p.bm == 16 ? 64 : 256;
+    } else if (!small && !even) {
+      p.bn = 128;
+      if (p.bm > 16 && N >= 8192 &&
+          fill_of((N + 255) / 256, cus) > fill_of(tiles128, cus) + 0.1)
+        p.bn = 256;
+    }
+  } else if (M <= 128) {
+    p.bn = N >= 36000 ? 256 : weights >= (20L << 20) ? 128 : 64;
+    if (p.bn == 64 && tiles64 <= cus / 2 && fill_of(2 * tiles64, cus) >= 0.6)
+      p.bm = 64;
+  } else if (N >= 16384 || (K >= 2 * N && N >= 5120) ||
+             (M <= 192 && K >= 5 * N && N > 1024 && N <= 2048)) {
+    p.bm = 256;
+    p.bn = 128;
+  } else if (N < 5120) {
+    const int tiles = (M + 63) / 64 * tiles64;
+    if (weights >= (12L << 20)) p.bn = 128;
+    else if (tiles <= cus && fill_of(tiles, cus) >= 0.65) p.bm = 64;
+  }
+  const int tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
+  int s = cus / tiles;
+  if (M <= 16 && s > 0 && fill_of(tiles, cus) < 0.7) s = 2 * cus / tiles;
+  if (p.bm == 256 && tiles < 160) s = (384 + tiles - 1) / tiles;
+  s = std::max(1, std::min(std::min(s, MAX_SPLIT), stages / 4));
+  if (M <= 64 && s > 2 && far_apart((stages + s - 1) / s * BK)) --s;
+  return finish(p, M, N, K, s);
+}
+
+// The plain product in one launch, 64 columns a tile, where that is quicker
+// than the parts and the launch that sums them; else no splits. Both sides from
+// what a stage, the weight's bytes and the parts' take (us, parts / one launch:
+// 64 x 12288 x 4096 29.6 / 25.0, 64 x 12288 x 2048 22.4 / 14.3, 16 x 16384 x
+// 1024 12.1 / 7.7, 128 x 7168 x 4096 25.8 / 22.4; the other way, 128 x 64 tiles
+// unsplit against parts of tile_gemm.hip: 192 x 8192 x 14336 112 / 68, 256 x
+// 7168 x 11008 81 / 66). Over 3682 sizes (up to 256 rows, 512 to 38016 columns,
+// K of 512 to 27648) it takes 0.89 of what rounding up took, which left 160
+// tiles of 64 columns and more whole, and is behind it by more than 8 % in
+// nine.
+Plan plain_plan(int M, int N, int K, int parts, bool tiled) {
+  const int cus = compute_units();
+  const double bytes = 2e-6 * N * K, sums = 8e-6 * parts * M * N;  // MB
+  // us beside what both take
+  const double split = tiled ? bytes / 5.5 + sums / 6 + 7
+                             : bytes / 6 + sums / (M <= 64 ? 4 : 3) + 2.5;
+  Plan p;
+  p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 || (M <= 128 && N < 8192) ? 64
+                                                                       : 128;
+  p.bn = 64;
+  p = finish(p, M, N, K, 1);
+  // a stage with a tile a CU, and with two
+  const int tiles = p.nbm * p.nbn;
+  const double few = p.bm == 16 ? 0.2 : p.bm == 32 ? 0.24 : 0.27;
+  const double one = M <= 64 ? few + 0.1 * tiles / cus
+                     : p.bm == 64 ? 0.31 : 0.46;
+  const double two = p.bm == 16 ? 0.6 : p.bm == 32 ? 0.65
+                     : p.bm == 64 ? 0.68 : M > 128 ? 0.8 : 0.92;
+  const double stage =
+      tiles <= cus ? one : two * std::max(1.0, tiles / (2.0 * cus));
+  if ((M <= 64 && K >= DEEP) || K / BK * stage >= split) p.splits = 0;
   return p;
 }
 
@@ -515,7 +584,7 @@ torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w) {
                w.size(1), bm, splits);
     return part;
   }
-  const Plan p = plan_for(M, N, w.size(1), false);
+  const Plan p = parts_plan(M, N, w.size(1));
   auto part = torch::empty({(long)p.splits, M, N},
                            x.options().dtype(at::kFloat));
   launch<PART>(p, part.data_ptr(), x, w, nullptr);
@@ -555,12 +624,15 @@ torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
   const void *bp = bias_ptr(bias, N);
   auto out = torch::empty({M, N}, x.options());
   if (M == 0) return out;
-  const Plan p = plan_for(M, N, w.size(1), false);
-  if (p.splits == 1) {
-    launch<PLAIN>(p, out.data_ptr(), x, w, bp);
-    return out;
+  Plan p = parts_plan(M, N, w.size(1));
+  int bm, tiled = 0;
+  if (x.is_contiguous()) tile_parts_plan(M, N, w.size(1), &bm, &tiled);
+  if (tiled > 0 || p.splits > 1) {
+    p = plain_plan(M, N, w.size(1), tiled > 0 ? tiled : p.splits, tiled > 0);
+    if (p.splits == 0) return parts_sum(stream_parts(x, w), bias);
   }
-  return parts_sum(stream_parts(x, w), bias);
+  launch<PLAIN>(p, out.data_ptr(), x, w, bp);
+  return out;
 }
 
 // silu(x w_gate^T) * (x w_up^T), w = gate rows, up rows
@@ -570,7 +642,7 @@ torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(N % 16 == 0);
   auto out = torch::empty({M, N / 2}, x.options());
   if (M == 0) return out;
-  launch<GATED>(plan_for(M, N, w.size(1), true), out.data_ptr(), x, w,
+  launch<GATED>(gated_plan(M, N, w.size(1)), out.data_ptr(), x, w,
                 nullptr);
   return out;
 }
