@@ -872,7 +872,8 @@ static torch::Tensor decode_rows(
               slots.scalar_type() == at::kLong && slots.is_contiguous() &&
               slots.numel() == B);
   TORCH_CHECK(block_table.scalar_type() == at::kInt &&
-              block_table.size(0) >= B && block_table.stride(1) == 1 &&
+              block_table.size(0) >= B &&
+              (block_table.size(1) <= 1 || block_table.stride(1) == 1) &&
               seq_lens.scalar_type() == at::kInt &&
               seq_lens.is_contiguous() && seq_lens.numel() >= B);
   TORCH_CHECK(arrived.is_cuda() && arrived.scalar_type() == at::kInt &&
