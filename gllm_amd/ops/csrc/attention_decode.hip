@@ -775,18 +775,25 @@ void launch_decode(torch::Tensor &out, const torch::Tensor &q,
                      zdim, order_above, rows)
   // A split's rows, partials and the join take 3 us, as long as a wave takes
   // for one or two tiles while most of the chip idles, for two to four in one
-  // round of workgroups and for six beside others (us, 40 heads on 8 of 128,
+  // round of workgroups and for six beside others; a sequence stays whole up
+  // to twice that in a round, and beyond up to eight tiles a wave, ten where
+  // the sequences by themselves nearly fill a round (us, 40 heads on 8 of 128,
   // every sequence over all splits / so: 4 of 520 to 1500 keys 17.7 / 15.2, 16
   // of 150 to 450 15.8 / 12.8, 12 of them 22.6 / 12.6, 12 of 520 to 1500 28.4 /
   // 21.2, 24 of 60 to 180 21.1 / 10.2, 31 of 150 to 450 25.8 / 14.7, 60 of 600
   // 40.2 / 30.5, 9 of 5400 46.9 / 43.8; 24 of 2700 to 7900 102.5 / 102.8. 24
   // tiles in one round: 8 of 520 to 1500 20.4 for 18.8; 16 beyond: 60 of 600
-  // 40.2). Rounded rows stand behind e4m3 products: there the count stays
-  // (splits_for).
+  // 40.2. Whole up to 24 / 32 / 40 / 48 tiles beyond a round: 24 of 1000 27.5 /
+  // 24.0 / 23.9 / 24.0, of 520 to 1500 31.5 / 31.5 / 34.0 / 28.0, 40 of 440 to
+  // 1270 44.3 / 44.0 / 39.7 / 39.8, of 770 to 2240 66.7 / 64.2 / 69.2 / 70.8,
+  // 60 of 520 to 1500 59.6 / 58.4 / 56.4 / 54.2, of 1150 to 3400 114.1 /
+  // 115.0 / 115.1 / 119.1). Rounded rows stand behind e4m3 products: there the
+  // count stays (splits_for).
   NewRows rows = fresh ? *fresh : NewRows{};
   if (fresh && !fresh->rows.rounded) {
     const long all = (long)B * Hkv * splits;
-    rows.whole = all <= ALONE ? 8 : all <= 2 * ALONE ? 16 : 24;
+    rows.whole = all <= ALONE ? 8 : all <= 2 * ALONE ? 16
+                 : 5L * B * Hkv >= 7 * ALONE ? 40 : 32;
     rows.least = all <= ALONE ? 4 : all <= 2 * ALONE ? 8 : 24;
   }
   if (fresh) { if (D <= 64) RUN(64, 64, true); else RUN(128, 128, true); }
