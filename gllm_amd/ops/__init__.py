@@ -1135,7 +1135,7 @@ def qkv_decode_ok(parts: torch.Tensor, k_cache: torch.Tensor,
     """Whether ``qkv_decode`` takes these rows and heads (with caches that
     ``qkv_rope_cache_ok`` takes) and is the faster form."""
     return parts.dim() == 3 and _gpu_kernels().qkv_decode_ok(
-        k_cache, k_cache, num_heads, parts.shape[1], rounded)
+        k_cache, num_heads, parts.shape[1], rounded)
 
 
 def qkv_decode(parts: torch.Tensor, bias, positions: torch.Tensor,

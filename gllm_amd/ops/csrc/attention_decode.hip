@@ -939,23 +939,23 @@ std::vector<torch::Tensor> qkv_decode_fp8(
   return {out, q, st};
 }
 
-// Whether qkv_decode takes heads of this geometry, and is the faster form: its
-// rows cost each workgroup a few us, which pays in up to two rounds of
-// workgroups; rounded, with all sequences in all splits, in one if they are
-// split. (us of an attention step, 40 heads on 8 of 128, two kernels or three /
-// this one: 1 sequence of 600 keys 13.9 / 12.8, 2 of 2400 19.4 / 18.1, 16 of 340
-// to 880 19.4 / 18.9, 24 of 150 to 450 21.5 / 13.5, of 2700 to 7900 102.3 /
-// 102.8, 32 of 520 to 1500 36.5 / 34.6, 60 of them 56.1 / 58.1, of 150 to 450
-// 30.2 / 21.2, 64 of 520 to 1500 54.8 / 51.5, 128 96.2 / 92.3; 14 on 2 of 64, 64
-// of 520 to 1500 17.0 / 15.5. Beyond: 256 of 150 to 450 65.2 / 67.1. Rounded: 24
-// of 150 to 450 in four splits 21.6 / 24.2.)
-bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
-                   long B, bool rounded) {
+// Whether qkv_decode takes heads of this geometry (caches of one shape), and
+// is the faster form: its rows cost each workgroup a few us, which pays in up
+// to two rounds of workgroups; rounded, with all sequences in all splits, in
+// one if they are split. (us of an attention step, 40 heads on 8 of 128, two
+// kernels or three / this one: 1 sequence of 600 keys 13.9 / 12.8, 2 of 2400
+// 19.4 / 18.1, 16 of 340 to 880 19.4 / 18.9, 24 of 150 to 450 21.5 / 13.5, of
+// 2700 to 7900 102.3 / 102.8, 32 of 520 to 1500 36.5 / 34.6, 60 of them 57.3 /
+// 56.4, of 150 to 450 30.2 / 21.2, 64 of 520 to 1500 54.8 / 51.5, 128 96.2 /
+// 92.3; 14 on 2 of 64, 64 of 520 to 1500 17.0 / 15.5. Long unequal sequences
+// lose by the join what the rest gains: 60 of 1150 to 3400 112.8 / 115.1.
+// Beyond: 256 of 150 to 450 65.2 / 67.1. Rounded: 24 of 150 to 450 in four
+// splits 21.6 / 24.2.)
+bool qkv_decode_ok(torch::Tensor k_cache, long Hq, long B, bool rounded) {
   const long Hkv = k_cache.size(2);
   const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
   const int splits = splits_for(k_cache, B);
-  return decode_rows_ok(k_cache, v_cache, Hq) &&
-         k_cache.sizes() == v_cache.sizes() &&
+  return decode_rows_ok(k_cache, k_cache, Hq) &&
          B * Hkv * splits <= (rounded && splits > 1 ? 2L : 4L) * cus;
 }
 

@@ -183,8 +183,7 @@ torch::Tensor stream_parts(torch::Tensor x, torch::Tensor w);
 torch::Tensor stream_add_norm(torch::Tensor x, torch::Tensor w,
                               torch::Tensor residual, torch::Tensor norm_w,
                               double eps);
-bool qkv_decode_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
-                   long B, bool rounded);
+bool qkv_decode_ok(torch::Tensor k_cache, long Hq, long B, bool rounded);
 torch::Tensor qkv_decode(torch::Tensor parts,
                          c10::optional<torch::Tensor> bias,
                          torch::Tensor positions, torch::Tensor cos_sin,

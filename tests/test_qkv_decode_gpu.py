@@ -124,7 +124,7 @@ def test_refusals():
     assert ops.qkv_decode_ok(s["parts"], s["k"], 8)
     assert not ops.qkv_decode_ok(s["parts"], s["k"], 34)  # group of 17
     many = s["parts"].expand(2, 2, -1).repeat(1, 600, 1)
-    assert not ops.qkv_decode_ok(many, s["k"], 8)  # more than two per CU
+    assert not ops.qkv_decode_ok(many, s["k"], 8)  # more than four per CU
     args = [s["parts"], s["bias"], s["positions"], s["cos_sin"], s["k"],
             s["v"], s["slots"], s["table"], s["lens"]]
     few = torch.zeros(3, dtype=torch.int32, device="cuda")
