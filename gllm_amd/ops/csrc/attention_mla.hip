@@ -20,7 +20,7 @@
 // dims, of ONE row; V is read transposed out of the key tile
 // (ds_read_tr16_b64).
 //  * up to 16 rows (decode): mla_decode_kernel, bound by memory.
-//  * prompts, more heads: a workgroup of four waves takes R = 4 row tiles of
+//  * prompts, more heads: a workgroup of four waves takes four row tiles of
 //    16 and walks tiles of 64 keys (147 KB: one workgroup per CU). Wave w
 //    scores row tile w against all 64 keys; the output is split by dims, so V
 //    is read once for 64 rows instead of once per row tile. Bound by LDS reads
@@ -45,6 +45,7 @@ typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 constexpr int BLOCK = 256;    // 4 waves
 constexpr int BKV = 64;       // keys of a tile
+constexpr int PROMPT_TILES = 4;  // row tiles of a workgroup: one a wave
 constexpr int DK = 576;       // latent dims (kv_lora 512 + rope 64)
 constexpr int DV = 512;
 constexpr int KT = DK / 32;   // score k-steps (18)
@@ -73,7 +74,7 @@ DEV_INLINE void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <int R, bool SPLIT>
+template <bool SPLIT>
 __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     __hip_bfloat16 *__restrict__ out,      // [T, H, DV] (SPLIT: unused)
     float *__restrict__ partial_out,       // [S, TH, DV] (SPLIT only)
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     const int *__restrict__ qsl,           // [B+1]
     int max_pages, int page_size, int H, float scale, int num_splits,
     long th_total) {
-  constexpr int BQ = R * 16;
+  constexpr int R = PROMPT_TILES, BQ = R * 16;
   constexpr int NF = 4;  // score fragments of a wave
   // the last row tiles see the most keys: they start first
   const int tile = gridDim.x - 1 - blockIdx.x;
@@ -558,8 +559,8 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(k_cache.is_contiguous() &&
               reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0);
-  const int R = max_query_len * H <= 16 ? 1 : 4;
-  const int BQ = R * 16;
+  const bool few = max_query_len * H <= 16;
+  const int BQ = (few ? 1 : PROMPT_TILES) * 16;
   const int tiles = (int)((max_query_len * H + BQ - 1) / BQ);
   const long th_total = T * H;
   auto stream = at::cuda::getCurrentCUDAStream();
@@ -593,13 +594,13 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
                      (int)block_table.stride(0), (int)k_cache.size(1), H,    \
                      (float)scale, splits, th_total)
   if (splits == 1) {
-    if (R == 1) RUN(mla_decode_kernel<false>);
-    else RUN(mla_attention_kernel<4, false>);
+    if (few) RUN(mla_decode_kernel<false>);
+    else RUN(mla_attention_kernel<false>);
     HIP_CHECK_KERNEL();
     return;
   }
-  if (R == 1) RUN(mla_decode_kernel<true>);
-  else RUN(mla_attention_kernel<4, true>);
+  if (few) RUN(mla_decode_kernel<true>);
+  else RUN(mla_attention_kernel<true>);
 #undef RUN
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((mla_merge_kernel), dim3((unsigned)th_total),
