@@ -243,7 +243,7 @@ __global__ __launch_bounds__(512) void stream_add_norm_kernel(
   shortx4 old[V] = {};
   float wv[V][4] = {};
   st_f4 v[V] = {};
-  if ((int)threadIdx.x * 4 < N) {
+  if (V > 1 || (int)threadIdx.x * 4 < N) {
     const float *p[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
