@@ -925,11 +925,13 @@ def skinny_gemm(x: torch.Tensor, w: torch.Tensor,
 def _use_skinny(M: int, N: int, K: int) -> bool:
     """Measured against hipBLASLt (us, stream / library): up to 64 rows
     the stream wins wherever the product is more than a few workgroups (64
-    x 5120 x 5120 20.6 / 24.6, 64 x 38016 x 5120 83 / 89, 64 x 5120 x 27648
-    63 / 159); above that the library is level or better on wide weights
-    (96 x 28672 x 4096 57.6 / 55.6, 256 x 38016 x 5120 139 / 109) and
-    worse on the rest (256 x 7168 x 5120 40 / 54, 256 x 5120 x 27648 110 /
-    266)."""
+    x 5120 x 5120 18.9 / 21.5, 64 x 38016 x 5120 84 / 90, 64 x 5120 x 27648
+    60 / 158); above that the library is level on wide weights (96 x 28672
+    x 4096 53.7 / 55.0, 128 x 19008 x 5120 53.4 / 51.8, 128 x 38016 x 5120
+    98 / 100) and, with 256 rows, ahead on the widest (28672 x 4096 82 /
+    70, 38016 x 5120 158 / 111; 19008 x 5120 69 / 80, 16384 x 4096 54.7 /
+    52.8), and it is behind on the rest (256 x 7168 x 5120 39 / 51, 256 x
+    5120 x 27648 84 / 265)."""
     if K % 64 != 0 or N < 512 or M > SKINNY_MAX_M or M == 0:
         return False
     import os

@@ -598,7 +598,7 @@ struct Plan {
 //    than 32 rows (64 x 28672 x 4096 28.6, 29.1).
 // K is split into about as many workgroups as the chip holds at once: 256 of
 // the 512-thread tiles, 448 of the others (1 x 7168 x 5120 4 parts 7.4, 3
-// 8.3), each part at least four stages long.
+// 8.3), each part four stages long on average (the last may be shorter).
 Plan plan_for(bool int4, int M, int N, int K, bool gated, int splits) {
   Plan p;
   const bool wide = N >= 16384, deep = K >= 2 * N;

@@ -811,18 +811,19 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w,
 // weight's bytes, else two of 128 rows with half the splits (us with the norm
 // that sums the parts, one / two: 256 x 5120 x 27648 81 / 95, 256 x 5120 x
 // 5120 44 / 36, 256 x 4096 x 14336 57 / 51, 136 x 7168 x 5120 37 / 38).
-// Against the stream (stream / this): 256 x 5120 x 27648 113 / 81, 256 x 7168
-// x 5120 48 / 42, 256 x 5120 x 5120 45 / 36, 160 x 6144 x 4096 37 / 31, 96 x
-// 5120 x 5120 31 / 28, 128 x 4096 x 14336 44 / 39; below 24 M weights its
-// short parts lose (256 x 4096 x 4096 28 / 28, 256 x 6144 x 2048 25 / 27), up
-// to 128 rows those of K below 4608 (128 x 6144 x 4096 27.7 / 29.6, 96 x 7680
-// x 3840 28 / 31, 128 x 8192 x 3584 25 / 31). Up to 64 rows only long streams
-// gain: 64 x 5120 x 27648 73 / 63, 40 x 10240 x 8192 42 / 38, but 64 x 4096 x
-// 14336 37 / 37, 64 x 7168 x 5120 28 / 31. Few columns leave CUs idle with 16
-// parts, the most (256 x 1024 x 28672 38 / 52, 160 x 2048 x 16384 28 / 35): it
-// takes 160 workgroups for a block of rows (256 x 2560 x 12800 51 / 37), 200
-// for half a one (96 x 3072 x 12288 with 192 29.6 / 31.9, 96 x 3584 x 8192
-// with 224 27.6 / 26.4).
+// Against the stream, with the norm (us, stream / this): 256 x 5120 x 27648
+// 117 / 95, 256 x 7168 x 5120 44.8 / 41.1, 256 x 5120 x 5120 42.7 / 34.1, 160
+// x 6144 x 4096 34.1 / 29.2, 192 x 5120 x 5120 40 / 32, 192 x 7168 x 5120 42.3
+// / 38.7; level with few columns and long K (256 x 4096 x 14336 48.2 / 49.5,
+// 256 x 2560 x 12800 36.1 / 37.6); below 24 M weights its short parts lose.
+// The lines up to 128 rows (K from 4608 on; up to 64 rows from 8192 on and 72 M
+// weights) were drawn where the stream of 64-column tiles fell behind; the
+// stream of 128-column tiles is level or ahead there (128 x 5120 x 27648 65.4 /
+// 64.0, 128 x 5120 x 5120 25.4 / 30.5, 128 x 7168 x 5120 29.7 / 33.7, 128 x
+// 4096 x 14336 34.0 / 39.3, 96 x 3584 x 8192 22.9 / 25.9, 64 x 5120 x 27648
+// 54.2 / 61.3, 40 x 8192 x 10240 35.5 / 41.8). Few columns leave CUs idle with
+// 16 parts, the most: it takes 160 workgroups for a block of rows, 200 for half
+// a one.
 void tile_parts_plan(long M, long N, long K, int *bm, int *splits) {
   *splits = 0;
   *bm = M > 128 ? 256 : 128;
