@@ -19,12 +19,16 @@
 // Scores are K Q^T and the output is O^T = V^T P^T, so a lane holds keys, then
 // dims, of ONE row; V is read transposed out of the key tile
 // (ds_read_tr16_b64).
-//  * up to 16 rows (decode): mla_decode_kernel, bound by memory.
-//  * prompts, more heads: a workgroup of four waves takes four row tiles of
-//    16 and walks tiles of 64 keys (147 KB: one workgroup per CU). Wave w
-//    scores row tile w against all 64 keys; the output is split by dims, so V
-//    is read once for 64 rows instead of once per row tile. Bound by LDS reads
-//    (K 295 KB + V 64 KB + P 32 KB a tile against 2176 cycles of products).
+//  * up to 16 rows and more workgroups than CUs (decode): mla_decode_kernel,
+//    bound by memory.
+//  * else a workgroup of four waves takes R row tiles of 16 and walks tiles of
+//    64 keys (147 KB: one workgroup per CU). R = 1 (up to 16 rows): wave w
+//    scores keys 16 w .. + 15, the row maxima and the weights pass through LDS,
+//    then wave w owns dims 128 w .. + 127 of the output. R = 4 (prompts, more
+//    heads): wave w scores row tile w against all 64 keys; the output is split
+//    by dims as well, so V is read once for 64 rows instead of once per row
+//    tile. Bound by LDS reads (K 295 KB + V 64 KB + P 32 KB a tile against 2176
+//    cycles of products).
 // 128 requests of 16 heads at 512 to 1536 keys (151 MB), us: element by
 // element and in one split 282; in tiles of 64 keys, one workgroup per CU, 52
 // + 6; of 32 keys, two per CU, 37 + 6. Prompts of 4096 tokens in four, 16
@@ -45,7 +49,6 @@ typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 constexpr int BLOCK = 256;    // 4 waves
 constexpr int BKV = 64;       // keys of a tile
-constexpr int PROMPT_TILES = 4;  // row tiles of a workgroup: one a wave
 constexpr int DK = 576;       // latent dims (kv_lora 512 + rope 64)
 constexpr int DV = 512;
 constexpr int KT = DK / 32;   // score k-steps (18)
@@ -74,7 +77,7 @@ DEV_INLINE void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <bool SPLIT>
+template <int R, bool SPLIT>
 __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     __hip_bfloat16 *__restrict__ out,      // [T, H, DV] (SPLIT: unused)
     float *__restrict__ partial_out,       // [S, TH, DV] (SPLIT only)
@@ -86,8 +89,8 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     const int *__restrict__ qsl,           // [B+1]
     int max_pages, int page_size, int H, float scale, int num_splits,
     long th_total) {
-  constexpr int R = PROMPT_TILES, BQ = R * 16;
-  constexpr int NF = 4;  // score fragments of a wave
+  constexpr int BQ = R * 16;
+  constexpr int NF = R == 1 ? 1 : 4;  // score fragments of a wave
   // the last row tiles see the most keys: they start first
   const int tile = gridDim.x - 1 - blockIdx.x;
   const int b = blockIdx.y;
@@ -124,7 +127,8 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
   __shared__ float s_a[4][16], s_b[4][16], s_m[4][16];
 
   // query fragments: column l16 = row, dims kt * 32 + lhi * 8
-  const int my_row = wave * 16 + l16;
+  const int my_tile = R == 1 ? 0 : wave;
+  const int my_row = my_tile * 16 + l16;
   mfma_bf8 qf[KT];
   {
     const __hip_bfloat16 *qp =
@@ -167,7 +171,7 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
         __builtin_amdgcn_global_load_lds(
             reinterpret_cast<const unsigned int *>(src[g] + c * 128),
             reinterpret_cast<unsigned int *>(dst + c * CB_B + g * 1024), 16,
-            0, 0);
+            0, R == 1 ? 2 : 0);
   };
 
   float m_run = -INFINITY, l_run = 0.f;
@@ -192,19 +196,22 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     }
     const char *kt_base = ring + slot * TILE_B;
 
-    // ---- scores: fragment f = keys f * 16 + lhi * 4 + r
-    mfma_f4 s[NF];
+    // ---- scores: fragment f = keys (R == 1 ? wave : f) * 16 + lhi * 4 + r
+    mfma_f4 s[NF][2];
 #pragma unroll
-    for (int f = 0; f < NF; ++f) s[f] = mfma_f4{0, 0, 0, 0};
+    for (int f = 0; f < NF; ++f)
+      s[f][0] = s[f][1] = mfma_f4{0, 0, 0, 0};
+    const int krow = (R == 1 ? wave * 16 : 0) + l16;
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const mfma_bf8 kf = *reinterpret_cast<const mfma_bf8 *>(
-            kt_base + (kt >> 1) * CB_B + (l16 + f * 16) * 128 +
-            (((kt & 1) * 64 + lhi * 16) ^ ((l16 & 7) << 4)));
-        s[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[kt], s[f], 0, 0,
-                                                       0);
+            kt_base + (kt >> 1) * CB_B + (krow + f * 16) * 128 +
+            (((kt & 1) * 64 + lhi * 16) ^ ((krow & 7) << 4)));
+        // (one fragment: two chains)
+        s[f][NF == 1 ? kt & 1 : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            kf, qf[kt], s[f][NF == 1 ? kt & 1 : 0], 0, 0, 0);
       }
     float mx = -INFINITY;
     float sv[NF][4];
@@ -212,13 +219,19 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int key = k0 + f * 16 + lhi * 4 + r;
-        const float x = s[f][r] * qscale;
+        const int key = k0 + (R == 1 ? wave : f) * 16 + lhi * 4 + r;
+        const float x = (s[f][0][r] + s[f][1][r]) * qscale;
         sv[f][r] = key < vis ? x : -INFINITY;
         mx = fmaxf(mx, sv[f][r]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (R == 1) {
+      if (lhi == 0) s_a[wave][l16] = mx;
+      lds_barrier();
+#pragma unroll
+      for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_a[w][l16]);
+    }
     // (a row may see nothing yet: a finite maximum keeps its weights at 0)
     const float m_new = fmaxf(fmaxf(m_run, mx), -1e30f);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -234,16 +247,17 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
         p[r] = bf16_bits(e);
       }
       *reinterpret_cast<shortx4 *>(
-          p_tile + my_row * P_ROW + (f * 16 + lhi * 4) * 2) = p;
+          p_tile + my_row * P_ROW +
+          ((R == 1 ? wave : f) * 16 + lhi * 4) * 2) = p;
     }
     l_run = l_run * alpha + sum;  // this lane's keys
-    if (lhi == 0) s_a[wave][l16] = alpha;
+    if (R > 1 && lhi == 0) s_a[wave][l16] = alpha;
     lds_barrier();
 
     // ---- output dims wave * 128 + nt * 16 .. of every row tile
     float al[R];
 #pragma unroll
-    for (int rt = 0; rt < R; ++rt) al[rt] = s_a[rt][l16];
+    for (int rt = 0; rt < R; ++rt) al[rt] = R == 1 ? alpha : s_a[rt][l16];
 #pragma unroll
     for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -292,7 +306,9 @@ __global__ __launch_bounds__(BLOCK, 1) void mla_attention_kernel(
   for (int rt = 0; rt < R; ++rt) {
     const int row = rt * 16 + l16;
     if (row >= rows_here) continue;
-    const float l = s_b[rt][l16];
+    const float l = R == 1 ? s_b[0][l16] + s_b[1][l16] + s_b[2][l16] +
+                                 s_b[3][l16]
+                           : s_b[rt][l16];
     const float m = s_m[rt][l16];
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const long at = row0 + row;
@@ -559,8 +575,8 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(k_cache.is_contiguous() &&
               reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0);
-  const bool few = max_query_len * H <= 16;
-  const int BQ = (few ? 1 : PROMPT_TILES) * 16;
+  const int R = max_query_len * H <= 16 ? 1 : 4;
+  const int BQ = R * 16;
   const int tiles = (int)((max_query_len * H + BQ - 1) / BQ);
   const long th_total = T * H;
   auto stream = at::cuda::getCurrentCUDAStream();
@@ -584,6 +600,13 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
     po = partial.data_ptr<float>();
     pl = lse.data_ptr<float>();
   }
+  // Two workgroups a CU hide each other's latencies; by itself one walks 64
+  // keys at a time (us: one sequence of 4000 keys and two rows 185, by 32 keys
+  // 241, 64 of 1000 74 / 92; decode, 4 of 4000 in 32 splits 23 / 24, 64 of 1000
+  // in eight 32 / 25).
+  const bool paired =
+      R == 1 && (long)B * splits > at::cuda::getCurrentDeviceProperties()
+                                       ->multiProcessorCount;
 #define RUN(...)                                                             \
   hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles, B, splits), dim3(BLOCK), 0,  \
                      stream, (__hip_bfloat16 *)out.data_ptr(), po, pl,       \
@@ -594,13 +617,15 @@ void mla_paged_attention(torch::Tensor out, torch::Tensor q,
                      (int)block_table.stride(0), (int)k_cache.size(1), H,    \
                      (float)scale, splits, th_total)
   if (splits == 1) {
-    if (few) RUN(mla_decode_kernel<false>);
-    else RUN(mla_attention_kernel<false>);
+    if (paired) RUN(mla_decode_kernel<false>);
+    else if (R == 1) RUN(mla_attention_kernel<1, false>);
+    else RUN(mla_attention_kernel<4, false>);
     HIP_CHECK_KERNEL();
     return;
   }
-  if (few) RUN(mla_decode_kernel<true>);
-  else RUN(mla_attention_kernel<true>);
+  if (paired) RUN(mla_decode_kernel<true>);
+  else if (R == 1) RUN(mla_attention_kernel<1, true>);
+  else RUN(mla_attention_kernel<4, true>);
 #undef RUN
   HIP_CHECK_KERNEL();
   hipLaunchKernelGGL((mla_merge_kernel), dim3((unsigned)th_total),
