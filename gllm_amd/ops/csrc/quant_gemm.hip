@@ -35,7 +35,9 @@
 // columns / this: 55296 x 5120 gated 45.9 / 41.1, 5120 x 27648 26.1 / 22.5,
 // 7168 x 5120 10.3 / 9.3; 64 rows 67.5 / 58.9, 38.1 / 34.5, 22.7 / 21.7; 1 row
 // 37.2 / 32.3, 19.2 / 17.8. Sixteen waves 40.8 / 23.2; three stages 42.2 /
-// 23.9.)
+// 23.9.) Up to 16 rows of weights below 20 M values have shares of a few stages:
+// three of them in flight, and no sums to join, are the faster there (parts, 1
+// row: 4096 x 3584 5.7, by pairs 6.2; 2560 x 4096 8 % less; 4096 x 5120 8 % more).
 //
 // (us, 29 rows; the kernels before these formed floats weight by weight and
 // did not fill the chip:) fp8 55296 x 5120 gated 46, 5120 x 27648 31; four
@@ -642,7 +644,8 @@ void launch(const Plan &p, const Fp8Out &fp8, bool int4, void *C, const void *X,
     else if (p.bm == 64 && p.bn == 256) RUN(INT4, 64, 256, 1, 4, 2, 2);
     else if (p.bm == 64) RUN(INT4, 64, 128, 2, 2, 2, 2);
     else if constexpr (FORM != GATED) {  // (gate and up tile in one wave)
-      if (p.bm == 16) RUN(INT4, 16, 64, 1, 2, 2, 2);
+      if (p.bm == 16 && (long)N * K < (20L << 20)) RUN(INT4, 16, 64, 1, 4, 3, 1);
+      else if (p.bm == 16) RUN(INT4, 16, 64, 1, 2, 2, 2);
       else RUN(INT4, 32, 64, 1, 2, 2, 2);
     }
   } else {
