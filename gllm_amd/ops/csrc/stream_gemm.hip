@@ -363,7 +363,7 @@ Plan finish(Plan p, int M, int N, int K, int splits) {
 bool far_apart(int values) { return values % 2048 == 0; }
 
 // From here on 64-column tiles of up to 64 rows are not left whole (17 x 16384
-// x 14336 92, in two parts 76).
+// x 14336 92, in two parts 76; 32 x 14336 x 11008 whole 65, 72).
 constexpr int DEEP = 12288;
 
 // Gated products are not split: the width whose tiles fill whole rounds of
@@ -489,7 +489,7 @@ Plan plain_plan(int M, int N, int K, int parts, bool tiled) {
   const int cus = compute_units();
   const double bytes = 2e-6 * N * K, sums = 8e-6 * parts * M * N;  // MB
   // us beside what both take
-  const double split = tiled ? bytes / 5.5 + sums / 6 + 7
+  const double split = tiled ? bytes / 5.5 + sums / 6 + 8
                              : bytes / 6 + sums / (M <= 64 ? 4 : 3) + 2.5;
   Plan p;
   p.bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 || (M <= 128 && N < 8192) ? 64
@@ -500,7 +500,7 @@ Plan plain_plan(int M, int N, int K, int parts, bool tiled) {
   const int tiles = p.nbm * p.nbn;
   const double few = p.bm == 16 ? 0.2 : p.bm == 32 ? 0.24 : 0.27;
   const double one = M <= 64 ? few + 0.1 * tiles / cus
-                     : p.bm == 64 ? 0.31 : 0.46;
+                     : p.bm == 64 ? 0.31 : tiled && M <= 128 ? 0.52 : 0.46;
   const double two = p.bm == 16 ? 0.6 : p.bm == 32 ? 0.65
                      : p.bm == 64 ? 0.68 : M > 128 ? 0.8 : 0.92;
   const double stage =
