@@ -141,11 +141,11 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 //           A = strict tril(beta_t exp(b_t - b_i) k_t k_i), T = (I + A)^-1 by
 //           blocks of 16 rows, X = T [beta B k | beta v] and att =
 //           tril(exp(b_t - b_i) q_t k_i). b is the running log decay.
-//   carry   one workgroup per (sequence, v-head, DVS value columns), chunk
+//   carry   one workgroup per (sequence, v-head, 16 value columns), chunk
 //           after chunk: U = X_v - X_k S^T, o = B q S^T + att U,
 //           S = B_last S + (exp(b_last - b) U)^T k, with its columns of S in
 //           accumulators and the next chunk's operands on their way into
-//           registers.
+//           the registers that this one has used.
 //
 // Keys, queries and values are bf16 and enter the matrix instructions as they
 // are, their norms as fp32 factors of the sums; an fp32 operand (T, X_k, att,
@@ -155,14 +155,19 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // Accumulation, T and the state stay fp32. Error of the state against 64
 // bits, 64 to 1500 tokens, weak and strong decay: 1.1e-7 to 5.2e-7 (1.7e-7 to
 // 5.3e-7 with fp32 instructions, mean 2.5e-7 against 2.9e-7).
-// 4096 tokens in four prompts, 16 heads of 128: 59 + 127 us (carry 145 with a
-// 64-bit address and a branch for each load, with stores inside the wait for
-// the next chunk's operands, and one sum after the other; 212 + 200 with fp32
-// instructions throughout and the triangular system solved column strip by
-// column strip; 922 for one kernel that did all of it chunk after chunk on a
-// workgroup per sequence, head and 64 columns). local is bound by its
-// stores (X, att: 105 MB); carry by the serial chain of the longest prompt, a
-// chunk's operands arriving (110 KB a workgroup) and two barriers.
+//
+// 4096 tokens in four prompts of 682 to 1365, 16 heads of 128: 48 + 68 us;
+// with the same results, of carry's 118 us 91 were left when its operands
+// stood in runs of 1 KB (see below; local 55 -> 48), 89 with 16 columns and
+// two workgroups a CU for 32 and one (the next chunk's operands in registers
+// that are free by then, 220 for 332: what follows a barrier or an LDS read
+// in one workgroup is hidden by the other), 75 with sequences spread over the
+// XCDs and 68 with the longest first. One prompt of 4096: 253 -> 152, 64 of
+// 16: 98 -> 73, 30 tokens beside 700 + 900 + 15: 135 -> 58. (Queries and keys
+// in rows of another stride, sums of att and state in turn: no faster.)
+// local is bound by its stores (X, att: 105 MB); carry by the chain of a
+// chunk: products of U, split, barrier, products of the state, split, barrier,
+// 2.4 us alone and 4 us for two on a CU.
 typedef __attribute__((ext_vector_type(4))) float gdn_f4;
 typedef __attribute__((ext_vector_type(8))) __bf16 gdn_bf8;
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
@@ -179,6 +184,19 @@ constexpr int AS = 68;    // LDS row of 64 floats: rows 4 banks apart
 constexpr int KB = 144;   // of 128 bf16, for transposed reads: 8 banks
 constexpr int SB = 136;   // of 128 bf16: 4 banks
 constexpr int UB = 72;    // of 64 bf16
+constexpr int DVS = 16;   // value columns of a workgroup of carry
+
+// What local leaves for carry stands as carry's waves take it, a block of 16
+// rows and a head after the other and in it the 16 bytes of lane 0, 1, .. of
+// each load: a load is one run of 1 KB. With rows of all heads side by side
+// it was 16 runs of 64 bytes 4 KB apart, which share a channel of the L2, and
+// local's stores 16 runs of 32 bytes.
+constexpr int XK = 16 * D;  // X_k, of 3 parts: columns ks * 32 .. at ks * 512
+constexpr int XV = 16 * D;  // X_v: value columns n * 16 .. at n * 256
+constexpr int AT = 16 * C;  // att, of 3 parts: columns kk * 32 .. at kk * 512
+// A sequence's first block there: blocks of 16 rows from row `start` on end
+// before the next sequence's begin, T / 16 + sequences in all.
+DEV_INLINE long first_block(int start, int seq) { return start / 16 + seq; }
 
 DEV_INLINE gdn_f4 mma4(float a, float b, gdn_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -248,21 +266,37 @@ struct Gates {
 };
 
 __global__ __launch_bounds__(512) void gdn_local_kernel(
-    short *__restrict__ wk,    // X_k, bf16 [3, T, Hv, D]
-    float *__restrict__ u0,    // X_v [T, Hv, D]
-    short *__restrict__ att,   // bf16 [3, T, Hv, C]
+    short *__restrict__ wk,    // X_k, bf16 [blocks, Hv, 3, XK]
+    float *__restrict__ u0,    // X_v [blocks, Hv, XV]
+    short *__restrict__ att,   // bf16 [blocks, Hv, 3, AT]
     float *__restrict__ scal,  // [3, T, Hv]: b, 1/|k|, scale/|q|
+    int *__restrict__ order,   // [B] sequences, the longest first
     const __hip_bfloat16 *__restrict__ q, const __hip_bfloat16 *__restrict__ k,
     const __hip_bfloat16 *__restrict__ v, long qk_stride, long v_stride,
     Gates gates, const int *__restrict__ qsl, long T, int Hk, int Hv,
     float scale) {
   const int seq = blockIdx.y, h = blockIdx.z;
+  if (blockIdx.x == 0 && h == 0) {
+    const int B = gridDim.y, own = qsl[seq + 1] - qsl[seq];
+    int rank = 0;
+    for (int j0 = 0; j0 < B; j0 += 512) {
+      const int j = min(j0 + (int)threadIdx.x, B - 1);
+      const int other = qsl[j + 1] - qsl[j];
+      rank += __syncthreads_count(j0 + (int)threadIdx.x < B &&
+                                  (other > own || (other == own && j < seq)));
+    }
+    if (threadIdx.x == 0) order[rank] = seq;
+  }
   const int start = qsl[seq] + blockIdx.x * C;
   const int len = min(C, qsl[seq + 1] - start);
   if (len <= 0) return;
   const int hk = h / (Hv / Hk);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lhi = lane >> 4;
+  // block R of the chunk: + R * Hv times a block's size
+  const long block =
+      (first_block(qsl[seq], seq) + blockIdx.x * (C / 16)) * Hv + h;
   __shared__ __attribute__((aligned(16))) short Kt[C * KB], Vt[C * KB];
   __shared__ __attribute__((aligned(16))) float Am[C * AS], Tm[C * AS];
   __shared__ __attribute__((aligned(16))) float bb[C], btv[C], rkv[C],
@@ -353,13 +387,15 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
       s[r] = i0 + r <= t ? __expf(bb[t] - bb[i0 + r]) * rqv[t] *
                                rkv[i0 + r] * s[r]
                          : 0.f;
-    if (t < len) {
+    if (R * 16 < len) {  // (rows past the end are zero)
       shortx4 p[3];
       split3(s, p);
 #pragma unroll
       for (int j = 0; j < 3; ++j)
         *reinterpret_cast<shortx4 *>(
-            att + ((j * T + start + t) * Hv + h) * C + i0) = p[j];
+            att + ((block + R * Hv) * 3 + j) * AT + (I >> 1) * 512 +
+            (((I & 1) * 2 + (lhi >> 1)) * 16 + l16) * 8 + (lhi & 1) * 4) =
+            p[j];
     }
   }
   __syncthreads();
@@ -409,7 +445,8 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
     }
     __syncthreads();
   }
-  // ---- X, transposed: waves 0..3 the keys' columns, 4..7 the values'
+  // ---- X: waves 0..3 the keys' columns (transposed: a lane has four of a
+  // row), 4..7 the values' (four rows of a column)
   const short *src = wave < 4 ? Kt : Vt;
   const float *fac = wave < 4 ? ck : btv;
   const int c0 = (wave & 3) * 32;
@@ -439,23 +476,25 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
 #pragma unroll
       for (int j = 2; j >= 0; --j)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) x[n] = mma32(cols[kk][n], tf[j], x[n]);
+        for (int n = 0; n < 2; ++n)
+          x[n] = wave < 4 ? mma32(cols[kk][n], tf[j], x[n])
+                          : mma32(tf[j], cols[kk][n], x[n]);
     }
-    const int t = R * 16 + l16;
-    if (t >= len) continue;
+    if (R * 16 >= len) break;  // (rows past the end are zero)
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      const int c = c0 + n * 16 + lhi * 4;
       if (wave < 4) {
         shortx4 p[3];
         split3(x[n], p);
 #pragma unroll
         for (int j = 0; j < 3; ++j)
           *reinterpret_cast<shortx4 *>(
-              wk + ((j * T + start + t) * Hv + h) * D + c) = p[j];
+              wk + ((block + R * Hv) * 3 + j) * XK + wave * 512 +
+              ((n * 2 + (lhi >> 1)) * 16 + l16) * 8 + (lhi & 1) * 4) = p[j];
       } else {
         *reinterpret_cast<gdn_f4 *>(
-            u0 + ((long)(start + t) * Hv + h) * D + c) = x[n];
+            u0 + (block + R * Hv) * XV + ((wave & 3) * 2 + n) * 256 +
+            lane * 4) = x[n];
       }
     }
   }
@@ -467,20 +506,23 @@ DEV_INLINE __amdgpu_buffer_rsrc_t rows_of(const T_ *p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, bytes, 0x00020000);
 }
 
-// DVS value columns of a (sequence, head)
-template <int DVS>
-__global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
+__global__ __launch_bounds__(256, 2) void gdn_carry_kernel(
     __hip_bfloat16 *__restrict__ o,  // [T, Hv, D]
     float *__restrict__ states,      // [slots, Hv, D, D], in place
     const short *__restrict__ wk, const float *__restrict__ u0,
     const short *__restrict__ att, const float *__restrict__ scal,
     const __hip_bfloat16 *__restrict__ q, const __hip_bfloat16 *__restrict__ k,
     long qk_stride, const long *__restrict__ slots,
-    const int *__restrict__ has_init, const int *__restrict__ qsl, long T,
-    int Hk, int Hv) {
-  constexpr int VT = DVS / 16;
-  static_assert(VT <= 2, "q S^T: a term of each column tile in turn, below");
-  const int seq = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
+    const int *__restrict__ has_init, const int *__restrict__ qsl,
+    const int *__restrict__ order, long T, int B, int Hk, int Hv,
+    bool snake) {
+  // workgroups go to the 8 XCDs in turn
+  const int turn = blockIdx.x >> 3, z = turn % (D / DVS);
+  const int pair = turn / (D / DVS) * 8 + (blockIdx.x & 7);
+  if (pair >= B * Hv) return;
+  int at_seq = pair / Hv;
+  if (snake && at_seq >= (B + 1) / 2) at_seq = B - 1 - (at_seq - (B + 1) / 2);
+  const int h = pair % Hv, seq = order[at_seq];
   const int begin = qsl[seq], end = qsl[seq + 1];
   if (begin >= end) return;
   const int hk = h / (Hv / Hk);
@@ -493,107 +535,103 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
   __shared__ __attribute__((aligned(16))) short Up[6][DVS * UB];
   __shared__ float sc[2][3][C];  // b, 1/|k|, scale/|q|
 
-  // S transposed: lane value column vt * 16 + l16, keys (wave * 2 + dt) * 16
-  // + lhi * 4 + r
+  // S transposed: lane value column l16, keys (wave * 2 + dt) * 16 + lhi * 4
+  // + r
   float *sg = states + ((slots[seq] * Hv + h) * D + z * DVS) * D;
-  gdn_f4 s[VT][2];
+  gdn_f4 s[2];
   const bool init = has_init[seq] != 0;
   auto put_state = [&]() {
 #pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
+    for (int dt = 0; dt < 2; ++dt) {
+      shortx4 p[3];
+      split3(s[dt], p);
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt) {
-        shortx4 p[3];
-        split3(s[vt][dt], p);
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          *reinterpret_cast<shortx4 *>(
-              Sp[j] + (vt * 16 + l16) * SB + (wave * 2 + dt) * 16 +
-              lhi * 4) = p[j];
-      }
+      for (int j = 0; j < 3; ++j)
+        *reinterpret_cast<shortx4 *>(Sp[j] + l16 * SB +
+                                     (wave * 2 + dt) * 16 + lhi * 4) = p[j];
+    }
   };
 #pragma unroll
-  for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-      s[vt][dt] = init ? *reinterpret_cast<const gdn_f4 *>(
-                             sg + (long)(vt * 16 + l16) * D +
-                             (wave * 2 + dt) * 16 + lhi * 4)
-                       : gdn_f4{0, 0, 0, 0};
+  for (int dt = 0; dt < 2; ++dt)
+    s[dt] = init ? *reinterpret_cast<const gdn_f4 *>(
+                       sg + l16 * D + (wave * 2 + dt) * 16 + lhi * 4)
+                 : gdn_f4{0, 0, 0, 0};
   put_state();
 
-  // operands of a chunk, on their way in registers
-  shortx8 wr[4][3], ar[2][3] = {}, qr[4], kr[4];
-  float ur[VT][4], sr;
+  // operands of a chunk; the next one's are on their way as soon as their
+  // registers are free: keys, then X and queries, then att
+  GdnFrag w[4][3], at[2][3] = {}, qf[4];
+  shortx8 kr[4];
+  gdn_f4 u;
+  float sr;
   // Rows of a chunk by descriptors that end with it (what lies past is zero):
   // addresses are a lane's fixed offsets, where 64 bits and a branch for each
   // load were a third of the loop's instructions.
   const int row_b = Hv * D * 2, key_b = (int)qk_stride * 2;
-  const int w_at = (wave * 16 + l16) * row_b + lhi * 16;
-  const int a_at = (wave * 16 + l16) * (Hv * C * 2) + lhi * 16;
   const int q_at = (wave * 16 + l16) * key_b + lhi * 16;
   const int k_at = (tid >> 4) * key_b + (tid & 15) * 16;
-  const int u_at = (wave * 16 + lhi * 4) * (row_b * 2) + l16 * 4;
   auto load16 = [](__amdgpu_buffer_rsrc_t r, int at) {
     return __builtin_bit_cast(
         shortx8, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
   };
-  auto fetch = [&](int start) {
+  // the wave's block of rows in the chunk at `start`
+  const long block0 = (first_block(begin, seq) + wave) * Hv + h;
+  auto block_of = [&](int start) {
+    return block0 + (long)((start - begin) / 16) * Hv;
+  };
+  auto fetch_keys = [&](int start) {
     const int len = min(C, end - start);
-    const __amdgpu_buffer_rsrc_t rq =
-        rows_of(q + start * qk_stride + hk * D, (len - 1) * key_b + D * 2);
     const __amdgpu_buffer_rsrc_t rk =
         rows_of(k + start * qk_stride + hk * D, (len - 1) * key_b + D * 2);
-    const __amdgpu_buffer_rsrc_t ru =
-        rows_of(u0 + ((long)start * Hv + h) * D + z * DVS,
-                (len - 1) * row_b * 2 + DVS * 4);
-    if (wave * 16 >= len) {
-      // no row of this wave (64 prompts of 16 rows, 16 heads: 118 us, 126
-      // with loads that all fall outside)
-      const shortx8 none = {};
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) wr[ks][j] = none;
-        ar[0][j] = ar[1][j] = none;
-      }
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) qr[ks] = none;
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ur[vt][r] = 0.f;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const __amdgpu_buffer_rsrc_t rw =
-            rows_of(wk + ((j * T + start) * Hv + h) * D,
-                    (len - 1) * row_b + D * 2);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) wr[ks][j] = load16(rw, w_at + ks * 64);
-      }
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) qr[ks] = load16(rq, q_at + ks * 64);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const __amdgpu_buffer_rsrc_t ra =
-            rows_of(att + ((j * T + start) * Hv + h) * C,
-                    ((len - 1) * Hv + 1) * C * 2);
-        ar[0][j] = load16(ra, a_at);
-        // (blocks past the diagonal's pair are never written, nor read)
-        if (wave >= 2) ar[1][j] = load16(ra, a_at + 64);
-      }
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          ur[vt][r] = __builtin_bit_cast(
-              float, __builtin_amdgcn_raw_buffer_load_b32(
-                         ru, u_at + r * row_b * 2 + vt * 64, 0, 0));
-    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) kr[j] = load16(rk, k_at + j * 16 * key_b);
     sr = scal[(min(wave, 2) * T + start + min(lane, len - 1)) * Hv + h];
+  };
+  auto fetch_rows = [&](int start) {
+    const int len = min(C, end - start);
+    if (wave * 16 >= len) {
+      // no row of this wave (loads that all fall outside: 7 % of 64 prompts
+      // of 16 rows)
+      const shortx8 none = {};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) w[ks][j].s = none;
+        qf[ks].s = none;
+      }
+      u = gdn_f4{0, 0, 0, 0};
+      return;
+    }
+    const long block = block_of(start);
+    const __amdgpu_buffer_rsrc_t rw = rows_of(wk + block * 3 * XK, 6 * XK);
+    const __amdgpu_buffer_rsrc_t ru =
+        rows_of(u0 + block * XV + z * 256, 1024);
+    const __amdgpu_buffer_rsrc_t rq =
+        rows_of(q + start * qk_stride + hk * D, (len - 1) * key_b + D * 2);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        w[ks][j].s = load16(rw, (j * XK + ks * 512) * 2 + lane * 16);
+      qf[ks].s = load16(rq, q_at + ks * 64);
+    }
+    u = __builtin_bit_cast(gdn_f4, load16(ru, lane * 16));
+  };
+  auto fetch_att = [&](int start) {
+    if (wave * 16 >= end - start) {
+      const shortx8 none = {};
+#pragma unroll
+      for (int j = 0; j < 3; ++j) at[0][j].s = at[1][j].s = none;
+      return;
+    }
+    const __amdgpu_buffer_rsrc_t ra =
+        rows_of(att + block_of(start) * 3 * AT, 6 * AT);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      at[0][j].s = load16(ra, j * AT * 2 + lane * 16);
+      // (blocks past the diagonal's pair are never written, nor read)
+      if (wave >= 2) at[1][j].s = load16(ra, (j * AT + 512) * 2 + lane * 16);
+    }
   };
   auto put_keys = [&](int buf) {
 #pragma unroll
@@ -604,45 +642,27 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     }
     if (wave < 3) sc[buf][wave][lane] = sr;
   };
-  fetch(begin);
+  fetch_keys(begin);
+  fetch_rows(begin);
+  fetch_att(begin);
   put_keys(0);
   __syncthreads();
   int cur = 0;
   for (int start = begin; start < end; start += C) {
     const int len = min(C, end - start);
-    GdnFrag w[4][3], at[2][3], qf[4];
-    gdn_f4 u[VT];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) w[ks][j].s = wr[ks][j];
-      qf[ks].s = qr[ks];
-    }
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) at[kk][j].s = ar[kk][j];
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-      u[vt] = gdn_f4{ur[vt][0], ur[vt][1], ur[vt][2], ur[vt][3]};
-    if (start + C < end) fetch(start + C);
+    const bool more = start + C < end;
+    if (more) fetch_keys(start + C);
 
     // ---- U = X_v - X_k S^T and q S^T, rows 16 w ..
-    gdn_f4 xs[VT], qs[VT];
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-      xs[vt] = qs[vt] = gdn_f4{0, 0, 0, 0};
-    // (one wave per SIMD: nothing else hides the latency of a chain of
-    // products or of an LDS read, so the sums take turns and fragments are
-    // read a step ahead)
-    GdnFrag sf[2][VT][3];
+    // (two waves per SIMD hide little of the latency of an LDS read, so
+    // fragments are read a step ahead)
+    gdn_f4 xs = {0, 0, 0, 0}, qs = {0, 0, 0, 0};
+    GdnFrag sf[2][3];
     auto read_state = [&](int ks) {
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          sf[ks & 1][vt][j].s = *reinterpret_cast<const shortx8 *>(
-              Sp[j] + (vt * 16 + l16) * SB + ks * 32 + lhi * 8);
+      for (int j = 0; j < 3; ++j)
+        sf[ks & 1][j].s = *reinterpret_cast<const shortx8 *>(
+            Sp[j] + l16 * SB + ks * 32 + lhi * 8);
     };
     read_state(0);
 #pragma unroll
@@ -651,12 +671,8 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < 6; ++i) {
-#pragma unroll
-        for (int vt = 0; vt < VT; ++vt) {
-          xs[vt] = mma32(w[ks][TERM_A[i]], sf[ks & 1][vt][TERM_B[i]], xs[vt]);
-          if (i % 2 == vt)
-            qs[vt] = mma32(qf[ks], sf[ks & 1][vt][2 - i / 2], qs[vt]);
-        }
+        xs = mma32(w[ks][TERM_A[i]], sf[ks & 1][TERM_B[i]], xs);
+        if (i % 2 == 0) qs = mma32(qf[ks], sf[ks & 1][2 - i / 2], qs);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -668,46 +684,39 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
       wc[r] = __expf(last - sc[cur][0][t]) * sc[cur][1][t];
       eb[r] = __expf(sc[cur][0][t]) * sc[cur][2][t];
     }
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt) {
-      u[vt] -= xs[vt];
-      qs[vt] *= eb;
+    u -= xs;
+    qs *= eb;
+    {
       shortx4 p[3], pw[3];
-      split3(u[vt], p);
-      split3(u[vt] * wc, pw);
-      const int at_u = (vt * 16 + l16) * UB + wave * 16 + lhi * 4;
+      split3(u, p);
+      split3(u * wc, pw);
+      const int at_u = l16 * UB + wave * 16 + lhi * 4;
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         *reinterpret_cast<shortx4 *>(Up[j] + at_u) = p[j];
         *reinterpret_cast<shortx4 *>(Up[3 + j] + at_u) = pw[j];
       }
     }
+    if (more) fetch_rows(start + C);
     __syncthreads();
     // ---- o = B q S^T + att U
-    GdnFrag uf[2][VT][3], kf[2][2], wf[2][VT][3];
+    GdnFrag uf[2][3], kf[2][2], wf[2][3];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          uf[kk][vt][j].s = *reinterpret_cast<const shortx8 *>(
-              Up[j] + (vt * 16 + l16) * UB + kk * 32 + lhi * 8);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {  // the state's, for below
+      for (int j = 0; j < 3; ++j)
+        uf[kk][j].s = *reinterpret_cast<const shortx8 *>(
+            Up[j] + l16 * UB + kk * 32 + lhi * 8);
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt)
         read_tr(kf[kk][dt], Kt[cur], KB, kk * 32, (wave * 2 + dt) * 16, l16,
                 lhi);
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
+      for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-          for (int half = 0; half < 2; ++half)
-            wf[kk][vt][j].h[half] = *reinterpret_cast<const shortx4 *>(
-                Up[3 + j] + (vt * 16 + l16) * UB + kk * 32 + half * 16 +
-                lhi * 4);
+        for (int half = 0; half < 2; ++half)
+          wf[kk][j].h[half] = *reinterpret_cast<const shortx4 *>(
+              Up[3 + j] + l16 * UB + kk * 32 + half * 16 + lhi * 4);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -715,48 +724,39 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
       if (kk > wave / 2) continue;
 #pragma unroll
       for (int i = 0; i < 6; ++i)
-#pragma unroll
-        for (int vt = 0; vt < VT; ++vt)
-          qs[vt] = mma32(at[kk][TERM_A[i]], uf[kk][vt][TERM_B[i]], qs[vt]);
+        qs = mma32(at[kk][TERM_A[i]], uf[kk][TERM_B[i]], qs);
     }
+    if (more) fetch_att(start + C);
     // (rows past the end fall outside: with a branch around each store the
     // wait for the next chunk's operands would be one for these stores too)
     const __amdgpu_buffer_rsrc_t ro =
         rows_of(o + ((long)start * Hv + h) * D + z * DVS,
                 (len - 1) * row_b + DVS * 2);
 #pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        __builtin_amdgcn_raw_buffer_store_b16(
-            __builtin_bit_cast(short, __float2bfloat16(qs[vt][r])), ro,
-            (wave * 16 + lhi * 4 + r) * row_b + l16 * 2 + vt * 32, 0, 0);
+    for (int r = 0; r < 4; ++r)
+      __builtin_amdgcn_raw_buffer_store_b16(
+          __builtin_bit_cast(short, __float2bfloat16(qs[r])), ro,
+          (wave * 16 + lhi * 4 + r) * row_b + l16 * 2, 0, 0);
     // ---- S = B_last S + (exp(b_last - b) U)^T k
     const float keep = __expf(last);
-#pragma unroll
-    for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt) s[vt][dt] *= keep;
+    s[0] *= keep;
+    s[1] *= keep;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int j = 2; j >= 0; --j)
-#pragma unroll
-        for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-          for (int dt = 0; dt < 2; ++dt)
-            s[vt][dt] = mma32(kf[kk][dt], wf[kk][vt][j], s[vt][dt]);
+      for (int j = 2; j >= 0; --j) {
+        s[0] = mma32(kf[kk][0], wf[kk][j], s[0]);
+        s[1] = mma32(kf[kk][1], wf[kk][j], s[1]);
+      }
     put_state();
-    if (start + C < end) put_keys(cur ^ 1);
+    if (more) put_keys(cur ^ 1);
     cur ^= 1;
     __syncthreads();  // S is there, this chunk's U and keys have been read
   }
 #pragma unroll
-  for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-      *reinterpret_cast<gdn_f4 *>(sg + (long)(vt * 16 + l16) * D +
-                                  (wave * 2 + dt) * 16 + lhi * 4) = s[vt][dt];
+  for (int dt = 0; dt < 2; ++dt)
+    *reinterpret_cast<gdn_f4 *>(sg + l16 * D + (wave * 2 + dt) * 16 +
+                                lhi * 4) = s[dt];
 }
 
 // ------------------------------------------------- one token per sequence
@@ -917,30 +917,31 @@ void run_chunks(torch::Tensor &o, const void *q, const void *k,
                 int max_len, int Hk, int Hv, double scale) {
   auto opts = states.options();
   auto bf = opts.dtype(at::kBFloat16);
-  auto wk = torch::empty({3, T, (long)Hv, (long)D}, bf);
-  auto u0 = torch::empty({T, (long)Hv, (long)D}, opts);
-  auto att = torch::empty({3, T, (long)Hv, (long)C}, bf);
+  const long blocks = T / 16 + B;
+  auto wk = torch::empty({blocks, (long)Hv, 3, (long)XK}, bf);
+  auto u0 = torch::empty({blocks, (long)Hv, (long)XV}, opts);
+  auto att = torch::empty({blocks, (long)Hv, 3, (long)AT}, bf);
   auto scal = torch::empty({3, T, (long)Hv}, opts);
+  auto order = torch::empty({(long)B}, opts.dtype(at::kInt));
   auto stream = at::cuda::getCurrentCUDAStream();
   hipLaunchKernelGGL(gdn_local_kernel, dim3((max_len + C - 1) / C, B, Hv),
                      dim3(512), 0, stream, (short *)wk.data_ptr(),
                      u0.data_ptr<float>(), (short *)att.data_ptr(),
-                     scal.data_ptr<float>(), (const __hip_bfloat16 *)q,
-                     (const __hip_bfloat16 *)k, (const __hip_bfloat16 *)v,
+                     scal.data_ptr<float>(), order.data_ptr<int>(),
+                     (const __hip_bfloat16 *)q, (const __hip_bfloat16 *)k,
+                     (const __hip_bfloat16 *)v,
                      qk_stride, v_stride, gates, qsl, T, Hk, Hv,
                      (float)scale);
   HIP_CHECK_KERNEL();
-#define RUN(DVS)                                                             \
-  hipLaunchKernelGGL((gdn_carry_kernel<DVS>), dim3(B, Hv, D / DVS),          \
-                     dim3(256), 0, stream, (__hip_bfloat16 *)o.data_ptr(),   \
-                     states.data_ptr<float>(), (const short *)wk.data_ptr(), \
-                     u0.data_ptr<float>(), (const short *)att.data_ptr(),    \
-                     scal.data_ptr<float>(), (const __hip_bfloat16 *)q,      \
-                     (const __hip_bfloat16 *)k, qk_stride, slots, has_init,  \
-                     qsl, T, Hk, Hv)
-  // (narrower columns shorten the serial chain as long as CUs are free)
-  if ((long)B * Hv * 4 < 256) RUN(16); else RUN(32);
-#undef RUN
+  const long pairs = (long)B * Hv;
+  hipLaunchKernelGGL(
+      gdn_carry_kernel, dim3((pairs + 7) / 8 * 8 * (D / DVS)), dim3(256), 0,
+      stream, (__hip_bfloat16 *)o.data_ptr(), states.data_ptr<float>(),
+      (const short *)wk.data_ptr(), u0.data_ptr<float>(),
+      (const short *)att.data_ptr(), scal.data_ptr<float>(),
+      (const __hip_bfloat16 *)q, (const __hip_bfloat16 *)k, qk_stride, slots,
+      has_init, qsl, order.data_ptr<int>(), T, B, Hk, Hv,
+      pairs * (D / DVS) <= 512);
   HIP_CHECK_KERNEL();
 }
 
