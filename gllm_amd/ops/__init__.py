@@ -664,7 +664,8 @@ def gdn_rows(qkvz: torch.Tensor, ba: torch.Tensor, conv_w: torch.Tensor,
     conv = causal_conv_silu(qkvz[:, :conv_dim], conv_w, conv_state, slots,
                             has_init, query_start_loc,
                             max_query_len=max_query_len)
-    A, dt = A_log.float(), dt_bias.float()
+    A = A_log.float()
+    dt = dt_bias if dt_bias.dtype == torch.bfloat16 else dt_bias.float()
     if carried:
         o = k.gdn_step(conv, ba, A, dt, state, slots, Hk, scale)
     else:

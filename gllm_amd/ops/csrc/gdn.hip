@@ -252,13 +252,15 @@ struct Gates {
   const __hip_bfloat16 *ba;         // rows of b | a
   long ba_stride;
   const float *A_log, *dt;          // [Hv]
+  const __hip_bfloat16 *dt16;       // or dt in 16 bits, where dt is null
   DEV_INLINE void at(long t, int h, int Hv, float &gv, float &bv) const {
     if (g) {
       gv = g[t * Hv + h];
       bv = beta[t * Hv + h];
       return;
     }
-    const float a = __bfloat162float(ba[t * ba_stride + Hv + h]) + dt[h];
+    const float a = __bfloat162float(ba[t * ba_stride + Hv + h]) +
+                    (dt ? dt[h] : __bfloat162float(dt16[h]));
     const float sp = a > 20.f ? a : log1pf(expf(a));
     gv = -expf(A_log[h]) * sp;
     bv = 1.f / (1.f + expf(-__bfloat162float(ba[t * ba_stride + h])));
@@ -970,7 +972,7 @@ void gdn_chunk_prefill(torch::Tensor o, torch::Tensor q, torch::Tensor k,
   auto ones = torch::ones({(long)B}, ints);
   auto slots = torch::arange((long)B, q.options().dtype(at::kLong));
   const Gates gates = {g.data_ptr<float>(), beta.data_ptr<float>(), nullptr,
-                       0, nullptr, nullptr};
+                       0, nullptr, nullptr, nullptr};
   run_chunks(o, q.data_ptr(), k.data_ptr(), v.data_ptr(), (long)Hk * D,
              (long)Hv * D, gates, states, slots.data_ptr<long>(),
              ones.data_ptr<int>(), qsl.data_ptr<int>(), (long)B * T, B, T,
@@ -992,15 +994,19 @@ Gates check_rows(const torch::Tensor &conv, const torch::Tensor &ba,
               ba.dim() == 2 && ba.stride(1) == 1 &&
               ba.size(0) == conv.size(0) && ba.size(1) == 2L * Hv);
   TORCH_CHECK(A_log.scalar_type() == at::kFloat && A_log.numel() == Hv &&
-              dt_bias.scalar_type() == at::kFloat && dt_bias.numel() == Hv &&
-              A_log.is_contiguous() && dt_bias.is_contiguous());
+              (dt_bias.scalar_type() == at::kFloat ||
+               dt_bias.scalar_type() == at::kBFloat16) &&
+              dt_bias.numel() == Hv && A_log.is_contiguous() &&
+              dt_bias.is_contiguous());
   TORCH_CHECK(states.dim() == 4 && states.is_contiguous() &&
               states.scalar_type() == at::kFloat && states.size(2) == D &&
               states.size(3) == D, "gdn: state [slots, Hv, 128, 128] fp32");
   TORCH_CHECK(slots.scalar_type() == at::kLong && slots.is_contiguous());
+  const bool wide = dt_bias.scalar_type() == at::kFloat;
   return {nullptr, nullptr, (const __hip_bfloat16 *)ba.data_ptr(),
           (long)ba.stride(0), A_log.data_ptr<float>(),
-          dt_bias.data_ptr<float>()};
+          wide ? dt_bias.data_ptr<float>() : nullptr,
+          wide ? nullptr : (const __hip_bfloat16 *)dt_bias.data_ptr()};
 }
 
 }  // namespace
