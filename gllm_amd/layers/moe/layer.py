@@ -135,12 +135,29 @@ class FusedMoE(nn.Module):
         return out
 
     def routed_add_norm(self, x: torch.Tensor, weights: torch.Tensor,
-                        ids: torch.Tensor, shared: Optional[torch.Tensor],
-                        residual: torch.Tensor, norm):
+                        ids: torch.Tensor, shared, residual: torch.Tensor,
+                        norm):
         """(norm(residual + (forward_routed(...) + shared)), that sum): one
         kernel behind the experts where nothing has to be reduced over
-        ranks first."""
+        ranks first. ``shared``: a tensor, a gated feed-forward of x (beside
+        the experts where that is the faster) or None."""
         one_rank = (get_ep_size() if self.use_ep else get_tp_size()) == 1
+        if isinstance(shared, nn.Module):
+            mlp = shared.weights_beside(x)
+            if (mlp is not None and one_rank and get_tp_size() == 1
+                    and self.activation == "silu_glu" and self._grouped(x)
+                    and ops.moe_add_norm_ok(x, None, residual, norm.scale())
+                    and ops.moe_shared_beside(x, self.w13_weight,
+                                              self.w2_weight, ids.shape[1],
+                                              *mlp)):
+                out = ops.fused_moe(
+                    x, self.w13_weight, self.w2_weight, weights, ids,
+                    expert_start=self.expert_start,
+                    num_global_experts=self.num_experts,
+                    add_norm=(None, residual, norm.scale(), norm.eps),
+                    shared_mlp=mlp)
+                return out, residual
+            shared = shared(x)
         if (one_rank and self._grouped(x)
                 and ops.moe_add_norm_ok(x, shared, residual, norm.scale())):
             out = ops.fused_moe(

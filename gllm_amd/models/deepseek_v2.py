@@ -355,10 +355,8 @@ class DeepseekMoE(nn.Module):
     def forward_add_norm(self, x, residual, norm):
         """(norm(residual + self(x)), that sum)."""
         weights, ids = self._route(self.gate(x))
-        shared = None if self.shared_experts is None \
-            else self.shared_experts(x)
-        return self.experts.routed_add_norm(x, weights, ids, shared,
-                                            residual, norm)
+        return self.experts.routed_add_norm(
+            x, weights, ids, self.shared_experts, residual, norm)
 
 
 class DeepseekDecoderLayer(nn.Module):

@@ -40,6 +40,15 @@ class DenseMLP(nn.Module):
     def forward(self, x):
         return self.down_proj(self.gate_up_proj.forward_silu(x))
 
+    def weights_beside(self, x):
+        """(gate over up rows, down weight) where these products of x may
+        run beside others, None for quantized weights or a bias."""
+        up, down = self.gate_up_proj, self.down_proj
+        if not (up.is_plain and down.is_plain) or up.bias is not None \
+                or down.bias is not None or x.dim() != 2:
+            return None
+        return up.weight, down.weight
+
     def forward_add_norm(self, x, residual, norm, fp8=False):
         """(norm(residual + self(x)), that sum); ``fp8``: see
         RowParallelLinear."""

@@ -250,7 +250,8 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
               num_global_experts: Optional[int] = None,
               activation: str = "silu_glu",
               act_args: tuple = (),
-              add_norm: Optional[tuple] = None) -> torch.Tensor:
+              add_norm: Optional[tuple] = None,
+              shared_mlp: Optional[tuple] = None) -> torch.Tensor:
     """Grouped-GEMM fused MoE on the gfx950 kernels (GPU, bf16).
     ``activation``: "silu_glu" (w13 = gate | up rows), "relu2"
     (ungated experts, w13 = up rows only, act = max(z, 0)^2) or
@@ -265,7 +266,10 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     run their TP/EP all-reduce on top). ``add_norm`` = (shared or None,
     residual, norm weight, eps): the output (+ shared) is added to the
     residual, in place, and the norm of that is returned (one kernel; see
-    ``moe_add_norm_ok``).
+    ``moe_add_norm_ok``). ``shared_mlp`` = (gate over up rows, down weight)
+    of a gated feed-forward that all rows pass: its output is the ``shared``
+    of ``add_norm``, its products run beside the experts' (see
+    ``moe_shared_beside``).
     """
     T, K = x.shape
     E_local, rows13, _ = w13.shape
@@ -284,18 +288,24 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
         # row block by the rows per expert: while an expert's weights are
         # the cost, one block holds the rows of all but the most popular
         # experts (csrc/moe_tiled.hip has times on both sides of each line)
-        block_m = (32 if rpe <= 12 else 64 if rpe <= 40
-                   else 128 if rpe <= 128 else 256)
+        block_m = _moe_block(rpe)
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
                                           block_m)
         act = torch.empty(rows, inter, dtype=x.dtype, device=dev)
         code = {"swiglu_clamp": 2, "relu2": 3}.get(activation, 1)
         limit, alpha = act_args if activation == "swiglu_clamp" \
             else (0.0, 0.0)
-        k.moe_gemm_tiled(act, x, w13, *tables, None, n_pairs, topk, block_m,
-                         code, limit, alpha)
-        k.moe_gemm_tiled(pair_out, act, w2, *tables, tw, n_pairs, topk,
-                         block_m, 0, 0.0, 0.0)
+        if shared_mlp is not None:
+            h = k.moe_gemm_tiled_shared(act, x, w13, *tables, None, n_pairs,
+                                        topk, block_m, 1, x, shared_mlp[0])
+            add_norm = (k.moe_gemm_tiled_shared(
+                pair_out, act, w2, *tables, tw, n_pairs, topk, block_m, 0, h,
+                shared_mlp[1]),) + add_norm[1:]
+        else:
+            k.moe_gemm_tiled(act, x, w13, *tables, None, n_pairs, topk,
+                             block_m, code, limit, alpha)
+            k.moe_gemm_tiled(pair_out, act, w2, *tables, tw, n_pairs, topk,
+                             block_m, 0, 0.0, 0.0)
     else:
         block_m = 16 if rpe < 12 else 32 if rpe < 40 else 64
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
@@ -317,6 +327,34 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     out = torch.empty(T, K, dtype=x.dtype, device=dev)
     k.moe_sum(out, pair_out, ids32, expert_start, E_local, topk)
     return out
+
+
+def _moe_block(rows_per_expert: float) -> int:
+    return (32 if rows_per_expert <= 12 else 64 if rows_per_expert <= 40
+            else 128 if rows_per_expert <= 128 else 256)
+
+
+def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
+                      topk: int, gate_up: torch.Tensor,
+                      down: torch.Tensor) -> bool:
+    """Whether ``fused_moe`` of gated experts runs a shared expert's products
+    beside theirs: up to 256 rows, where these are a few launches that wait for
+    weights (us of experts, sum and norm, apart / beside: 64 experts of 2048 x
+    1408, shared 2816, 1 row 53 / 45, 32 rows 203 / 194, 128 rows 214 / 207, 256
+    rows 241 / 231; 256 of 2048 x 512, shared 512, 8 rows 88 / 76, 128 rows 283 /
+    276; 64 of 7168 x 2048, shared 2048, 64 rows 897 / 887). Beyond, the tile
+    kernel serves all rows of a weight at once (420 rows 1244 / 1254), and a
+    shared expert of more than two routed ones has too long a K for a tile's
+    chain (16 of 4096 x 2048, shared 8192, 32 rows 215 / 241)."""
+    T, K = x.shape
+    inter = w2.shape[2]
+    ok = all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
+             and t.data_ptr() % 16 == 0 for t in (x, w13, w2, gate_up, down))
+    return (ok and 0 < T <= 256 and K % 64 == 0 and inter % 64 == 0
+            and down.shape[1] % 64 == 0 and down.shape[1] <= 2 * inter
+            and down.shape[0] == K
+            and gate_up.shape == (2 * down.shape[1], K)
+            and _moe_block(T * topk / max(1, w13.shape[0])) <= 128)
 
 
 def moe_add_norm_ok(x: torch.Tensor, shared: Optional[torch.Tensor],

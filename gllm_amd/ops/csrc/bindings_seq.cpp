@@ -205,6 +205,12 @@ void moe_gemm(torch::Tensor C, torch::Tensor A, torch::Tensor W,
               torch::Tensor n_post_pad,
               c10::optional<torch::Tensor> topk_weights, long n_pairs,
               long topk, long block_m, bool scatter);
+torch::Tensor moe_gemm_tiled_shared(
+    torch::Tensor C, torch::Tensor A, torch::Tensor W,
+    torch::Tensor sorted_ids, torch::Tensor expert_blocks,
+    torch::Tensor n_post_pad, c10::optional<torch::Tensor> topk_weights,
+    long n_pairs, long topk, long block_m, long act, torch::Tensor rows,
+    torch::Tensor w);
 void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
                     torch::Tensor sorted_ids, torch::Tensor expert_blocks,
                     torch::Tensor n_post_pad,
@@ -307,6 +313,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_and_mul", &silu_and_mul, "silu(x[:d]) * x[d:]");
   m.def("moe_align", &moe_align, "device-side moe_align_block_size");
   m.def("moe_gemm", &moe_gemm, "grouped MFMA GEMM over sorted pairs");
+  m.def("moe_gemm_tiled_shared", &moe_gemm_tiled_shared,
+        "moe_gemm_tiled with a shared expert's product beside it");
   m.def("moe_gemm_tiled", &moe_gemm_tiled,
         "grouped MFMA GEMM of wide tiles, activation in the epilogue");
   m.def("softmax_topk_rows", &softmax_topk_rows,

@@ -34,6 +34,10 @@
 //    64 rows per expert 375 + 192 us against 442 + 251 us (64 x 128) and
 //    475 + 379 us (256 x 256); 192 rows 287 + 182 us against 226 + 163 us
 //    for 256 x 256.
+// A shared expert's tiles come first in the same launch: they are the longest
+// of the second product, and what they wait for is hidden by the routed ones'.
+// (Two of 2048 x 1408 for 128 rows beside 64 routed ones, with sum and norm:
+// 214 us by launches of their own, 207 so; 32 rows 203, 194.)
 // Workgroups go to the eight dies in turn; each die gets a contiguous run
 // of tiles, row blocks fastest within groups, so that the tiles which
 // share weights meet in one L2.
@@ -66,8 +70,17 @@ DEV_INLINE short to_bf16(float v) {
   return __builtin_bit_cast(short, __float2bfloat16(v));
 }
 
+// An expert that all rows pass, of a size of its own and in row order, beside
+// the routed ones in the same launch.
+struct Shared {
+  __hip_bfloat16 *C;
+  const __hip_bfloat16 *A, *W;  // [rows, K], [N, K]
+  int rows, K, N, nbm, nbn;
+};
+
 // WM x WN waves share a BM x BN tile; a ring of ST stages of BK columns
-template <int BM, int BN, int WM, int WN, int ST, int AUX, int FORM, int ACT>
+template <int BM, int BN, int WM, int WN, int ST, int AUX, int FORM, int ACT,
+          bool SHARED = false>
 __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
     __hip_bfloat16 *__restrict__ C, const __hip_bfloat16 *__restrict__ A,
     const __hip_bfloat16 *__restrict__ W,  // [E_local, Nd, K]
@@ -75,7 +88,7 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
     const int *__restrict__ n_post_pad,
     const float *__restrict__ topk_w,  // [n_pairs] (SCATTER only, may be 0)
     int n_pairs, int K, int Nd, int topk, int nbn, float limit,
-    float alpha) {
+    float alpha, const Shared shared) {
   constexpr int THREADS = WM * WN * 64;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;  // 16 x 16 per wave
   constexpr int A_B = BM * ROW_B, STAGE = A_B + BN * ROW_B;
@@ -90,14 +103,35 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
   const int nblk = n_post_pad[0] / BM;
   const int total = nblk * nbn;
   const int pid = blockIdx.x;
-  if (pid >= total) return;
-  const int xcd = pid & 7, per = total >> 3;
-  const int t = xcd * per + min(xcd, total & 7) + (pid >> 3);
-  constexpr int GM = BM >= 256 ? 4 : 8;  // row blocks of a group
-  const int grp = t / (GM * nbn), in_g = t - grp * GM * nbn;
-  const int gm = min(GM, nblk - grp * GM);
-  const int mb = grp * GM + in_g % gm, nb = in_g / gm;
-  const int e = expert_blocks[mb];
+  const int xcd = pid & 7;
+  int t = pid >> 3, mb, nb, e = 0;
+  bool sh = false;  // a tile of the shared expert: each die's first ones
+  if (SHARED) {
+    const int s_total = shared.nbm * shared.nbn;
+    const int s0 = xcd * s_total >> 3, s1 = (xcd + 1) * s_total >> 3;
+    sh = t < s1 - s0;
+    if (sh) {
+      mb = (s0 + t) % shared.nbm;
+      nb = (s0 + t) / shared.nbm;
+      A = shared.A;
+      W = shared.W;
+      C = shared.C;
+      K = shared.K;
+      Nd = shared.N;
+    }
+    t -= s1 - s0;
+  }
+  if (!sh) {
+    const int per = total >> 3;
+    if (t >= per + (xcd < (total & 7))) return;
+    t += xcd * per + min(xcd, total & 7);
+    constexpr int GM = BM >= 256 ? 4 : 8;  // row blocks of a group
+    const int grp = t / (GM * nbn), in_g = t - grp * GM * nbn;
+    const int gm = min(GM, nblk - grp * GM);
+    mb = grp * GM + in_g % gm;
+    nb = in_g / gm;
+    e = expert_blocks[mb];
+  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, lhi = lane >> 4;
   const int wm = wave / WN, wn = wave % WN;
@@ -110,7 +144,9 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
   for (int j = 0; j < AL; ++j) {
     const int u = j * THREADS + tid, row = u >> 3;
     long r = g0 + row;  // (padding rows of a sorted buffer are not used)
-    if (FORM != SCATTER) {
+    if (sh) {
+      r = min(g0 + row, shared.rows - 1);
+    } else if (FORM != SCATTER) {
       const int pair = sorted_ids[g0 + row];
       r = pair < n_pairs ? pair / topk : 0;
     }
@@ -211,9 +247,9 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     const int g = g0 + (wm * MT + m) * 16 + l16;
-    const int pair = sorted_ids[g];
-    if (pair >= n_pairs) continue;
-    const float sc = FORM == SCATTER && topk_w ? topk_w[pair] : 1.f;
+    const int pair = sh ? g : sorted_ids[g];
+    if (pair >= (sh ? shared.rows : n_pairs)) continue;
+    const float sc = FORM == SCATTER && topk_w && !sh ? topk_w[pair] : 1.f;
     __hip_bfloat16 *crow = C + (long)(FORM == SCATTER ? pair : g) * I;
 #pragma unroll
     for (int n = 0; n < NT; n += FORM == GATED ? 2 : 1) {
@@ -251,12 +287,13 @@ __global__ __launch_bounds__(WM *WN * 64) void moe_tiled_kernel(
 
 // act: 0 none (scatter), 1 silu_glu, 2 clamped swiglu (limit, alpha), 3
 // relu^2. block_m: the row block of the tables, 32, 64, 128 or 256.
-void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
-                    torch::Tensor sorted_ids, torch::Tensor expert_blocks,
-                    torch::Tensor n_post_pad,
-                    c10::optional<torch::Tensor> topk_weights, long n_pairs,
-                    long topk, long block_m, long act, double limit,
-                    double alpha) {
+static void run_tiled(const torch::Tensor &C, const torch::Tensor &A,
+                      const torch::Tensor &W, const torch::Tensor &sorted_ids,
+                      const torch::Tensor &expert_blocks,
+                      const torch::Tensor &n_post_pad,
+                      const c10::optional<torch::Tensor> &topk_weights,
+                      long n_pairs, long topk, long block_m, long act,
+                      double limit, double alpha, Shared shared) {
   TORCH_CHECK(A.scalar_type() == at::kBFloat16 &&
               W.scalar_type() == at::kBFloat16 &&
               C.scalar_type() == at::kBFloat16);
@@ -287,7 +324,7 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
                 topk_weights->numel() >= n_pairs);
     tw = topk_weights->data_ptr<float>();
   }
-  if (block_m == 256 &&
+  if (!shared.C && block_m == 256 &&
       tile_gemm_grouped_ok(A.numel(), n_pairs, Nd, K, (int)act)) {
     tile_gemm_grouped(C.data_ptr(), A.data_ptr(), W.data_ptr(),
                       sorted_ids.data_ptr<int>(),
@@ -298,16 +335,23 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
     return;
   }
   auto stream = at::cuda::getCurrentCUDAStream();
-#define RUN(BM, BN, WM, WN, ST, AUX, FORM, ACT)                              \
+#define RUN(BM, BN, WM, WN, ST, AUX, FORM, ACT, ...)                         \
   do {                                                                       \
     const int nbn = ((FORM == GATED ? 2 * cols : cols) + BN - 1) / BN;       \
+    shared.nbm = (shared.rows + BM - 1) / BM;                                \
+    shared.nbn = (shared.N + BN - 1) / BN;                                   \
+    /* (a die has at most one tile of each kind more than another) */        \
+    const long tiles = max_blocks * nbn +                                    \
+                       (shared.C ? shared.nbm * shared.nbn + 8L : 0);        \
     hipLaunchKernelGGL(                                                      \
-        (moe_tiled_kernel<BM, BN, WM, WN, ST, AUX, FORM, ACT>),              \
-        dim3(max_blocks * nbn), dim3(WM * WN * 64), 0, stream,               \
+        (moe_tiled_kernel<BM, BN, WM, WN, ST, AUX, FORM, ACT                 \
+                          __VA_OPT__(,) __VA_ARGS__>),                       \
+        dim3((tiles + 7) / 8 * 8), dim3(WM * WN * 64), 0, stream,            \
         (__hip_bfloat16 *)C.data_ptr(), (const __hip_bfloat16 *)A.data_ptr(),\
         (const __hip_bfloat16 *)W.data_ptr(), sorted_ids.data_ptr<int>(),    \
         expert_blocks.data_ptr<int>(), n_post_pad.data_ptr<int>(), tw,       \
-        (int)n_pairs, K, Nd, (int)topk, nbn, (float)limit, (float)alpha);    \
+        (int)n_pairs, K, Nd, (int)topk, nbn, (float)limit, (float)alpha,     \
+        shared);                                                             \
   } while (0)
 #define FORMS(BM, BN, WM, WN, ST, AUX)                                       \
   do {                                                                       \
@@ -317,12 +361,63 @@ void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
     else if (act == RELU2) RUN(BM, BN, WM, WN, ST, AUX, PLAIN, RELU2);       \
     else TORCH_CHECK(false, "moe_gemm_tiled: act ", act);                    \
   } while (0)
-  if (block_m == 32) FORMS(32, 128, 1, 4, 4, 2);
+#define WITH(BM, BN, WM, WN, ST, AUX)                                        \
+  do {                                                                       \
+    if (act == NONE) RUN(BM, BN, WM, WN, ST, AUX, SCATTER, NONE, true);      \
+    else RUN(BM, BN, WM, WN, ST, AUX, GATED, SILU, true);                    \
+  } while (0)
+  if (shared.C && block_m == 32) WITH(32, 128, 1, 4, 4, 2);
+  else if (shared.C && block_m == 64) WITH(64, 128, 1, 4, 3, 2);
+  else if (shared.C) WITH(128, 128, 2, 2, 3, 0);
+  else if (block_m == 32) FORMS(32, 128, 1, 4, 4, 2);
   else if (block_m == 64) FORMS(64, 128, 1, 4, 3, 2);
   else if (block_m == 128) FORMS(128, 128, 2, 2, 3, 0);
   else if (block_m == 256) FORMS(256, 256, 2, 4, 2, 0);
   else TORCH_CHECK(false, "moe_gemm_tiled: block_m must be 32/64/128/256");
+#undef WITH
 #undef FORMS
 #undef RUN
   HIP_CHECK_KERNEL();
+}
+
+void moe_gemm_tiled(torch::Tensor C, torch::Tensor A, torch::Tensor W,
+                    torch::Tensor sorted_ids, torch::Tensor expert_blocks,
+                    torch::Tensor n_post_pad,
+                    c10::optional<torch::Tensor> topk_weights, long n_pairs,
+                    long topk, long block_m, long act, double limit,
+                    double alpha) {
+  run_tiled(C, A, W, sorted_ids, expert_blocks, n_post_pad, topk_weights,
+            n_pairs, topk, block_m, act, limit, alpha, Shared{});
+}
+
+// moe_gemm_tiled of act 1 or 0 with a shared expert's product beside it:
+// silu(gate) * up of all rows for w = gate rows over up rows, [rows, N / 2], or
+// rows w^T, [rows, N].
+torch::Tensor moe_gemm_tiled_shared(
+    torch::Tensor C, torch::Tensor A, torch::Tensor W,
+    torch::Tensor sorted_ids, torch::Tensor expert_blocks,
+    torch::Tensor n_post_pad, c10::optional<torch::Tensor> topk_weights,
+    long n_pairs, long topk, long block_m, long act, torch::Tensor rows,
+    torch::Tensor w) {
+  TORCH_CHECK((act == NONE || act == SILU) &&
+              (block_m == 32 || block_m == 64 || block_m == 128));
+  for (const auto *t : {&rows, &w})
+    TORCH_CHECK(t->is_cuda() && t->dim() == 2 && t->is_contiguous() &&
+                t->scalar_type() == at::kBFloat16 &&
+                reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0,
+                "moe_gemm_tiled_shared: 16 B aligned bf16 rows");
+  const long T = rows.size(0), K = rows.size(1), N = w.size(0);
+  const long cols = act == SILU ? N / 2 : N;
+  TORCH_CHECK(w.size(1) == K && K > 0 && K % BK == 0 && cols > 0 &&
+              cols % 8 == 0 && (act == NONE || N % 2 == 0) && T > 0 &&
+              T < 1L << 24 && N < 1L << 24,
+              "moe_gemm_tiled_shared: K a multiple of 64, columns of 8");
+  auto out = torch::empty({T, cols}, rows.options());
+  run_tiled(C, A, W, sorted_ids, expert_blocks, n_post_pad, topk_weights,
+            n_pairs, topk, block_m, act, 0.0, 0.0,
+            Shared{(__hip_bfloat16 *)out.data_ptr(),
+                   (const __hip_bfloat16 *)rows.data_ptr(),
+                   (const __hip_bfloat16 *)w.data_ptr(), (int)T, (int)K,
+                   (int)N, 0, 0});
+  return out;
 }
