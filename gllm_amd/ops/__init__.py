@@ -338,23 +338,38 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
                       topk: int, gate_up: torch.Tensor,
                       down: torch.Tensor) -> bool:
     """Whether ``fused_moe`` of gated experts runs a shared expert's products
-    beside theirs: up to 256 rows, where these are a few launches that wait for
-    weights (us of experts, sum and norm, apart / beside: 64 experts of 2048 x
-    1408, shared 2816, 1 row 53 / 45, 32 rows 203 / 194, 128 rows 214 / 207, 256
-    rows 241 / 231; 256 of 2048 x 512, shared 512, 8 rows 88 / 76, 128 rows 283 /
-    276; 64 of 7168 x 2048, shared 2048, 64 rows 897 / 887). Beyond, the tile
-    kernel serves all rows of a weight at once (420 rows 1244 / 1254), and a
-    shared expert of more than two routed ones has too long a K for a tile's
-    chain (16 of 4096 x 2048, shared 8192, 32 rows 215 / 241)."""
+    beside theirs (us of experts, sum and norm, apart / beside).
+    Up to 256 rows these are a few launches that wait for weights: 64 experts
+    of 2048 x 1408, shared 2816, 1 row 53 / 45, 32 rows 203 / 194, 128 rows 214 /
+    207, 256 rows 241 / 231; 256 of 2048 x 512, shared 512, 8 rows 88 / 76, 128
+    rows 283 / 276; 64 of 7168 x 2048, shared 2048, 64 rows 897 / 887. A shared
+    expert of more than two routed ones has too long a K for a tile's chain (16
+    of 4096 x 2048, shared 8192, 32 rows 215 / 241).
+    Beyond, they fill rounds of tiles that either would leave: rows of 2048 at
+    most, where rounds are short, and weights that are worth it (2048 x 1408 as
+    above, 320 rows 260 / 240, 1000 rows 364 / 344, 3000 rows 600 / 578, 4096 rows
+    661 / 624; 16 experts, shared 5632, 3000 rows 457 / 420; but 256 of 2048 x
+    512, 512 rows 322 / 329, 64 of 7168 x 2048, 4096 rows 3363 / 3530). Blocks
+    of 256 rows: level below 1536 and above 6144 rows (1400 rows 365 / 374, 8192
+    rows 1130 / 1152)."""
     T, K = x.shape
-    inter = w2.shape[2]
-    ok = all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
-             and t.data_ptr() % 16 == 0 for t in (x, w13, w2, gate_up, down))
-    return (ok and 0 < T <= 256 and K % 64 == 0 and inter % 64 == 0
-            and down.shape[1] % 64 == 0 and down.shape[1] <= 2 * inter
-            and down.shape[0] == K
-            and gate_up.shape == (2 * down.shape[1], K)
-            and _moe_block(T * topk / max(1, w13.shape[0])) <= 128)
+    inter, width = w2.shape[2], down.shape[1]
+    if not (all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
+                and t.data_ptr() % 16 == 0
+                for t in (x, w13, w2, gate_up, down))
+            and T > 0 and K % 64 == 0 and inter % 64 == 0 and width % 64 == 0
+            and down.shape[0] == K and gate_up.shape == (2 * width, K)):
+        return False
+    if T <= 256:
+        return width <= 2 * inter
+    if K > 2048 or width * K < 4 << 20:
+        return False
+    experts = max(1, w13.shape[0])
+    if _moe_block(T * topk / experts) < 256:
+        return width <= 2 * inter
+    # (offsets of tile_gemm.hip are 32 bits)
+    return (1536 <= T <= 6144 and 2 * max(inter, width) * K < 1 << 30
+            and (T * topk + 255 * experts) * max(inter, K) < 1 << 30)
 
 
 def moe_add_norm_ok(x: torch.Tensor, shared: Optional[torch.Tensor],

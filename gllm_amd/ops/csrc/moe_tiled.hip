@@ -324,14 +324,16 @@ static void run_tiled(const torch::Tensor &C, const torch::Tensor &A,
                 topk_weights->numel() >= n_pairs);
     tw = topk_weights->data_ptr<float>();
   }
-  if (!shared.C && block_m == 256 &&
+  if (block_m == 256 &&
       tile_gemm_grouped_ok(A.numel(), n_pairs, Nd, K, (int)act)) {
     tile_gemm_grouped(C.data_ptr(), A.data_ptr(), W.data_ptr(),
                       sorted_ids.data_ptr<int>(),
                       expert_blocks.data_ptr<int>(),
                       n_post_pad.data_ptr<int>(), tw, max_blocks, n_pairs,
                       topk, Nd, K, A.numel() / K, (int)act, (float)limit,
-                      (float)alpha);
+                      (float)alpha,
+                      TileShared{shared.C, shared.A, shared.W, shared.rows,
+                                 shared.K, shared.N});
     return;
   }
   auto stream = at::cuda::getCurrentCUDAStream();
@@ -399,8 +401,7 @@ torch::Tensor moe_gemm_tiled_shared(
     torch::Tensor n_post_pad, c10::optional<torch::Tensor> topk_weights,
     long n_pairs, long topk, long block_m, long act, torch::Tensor rows,
     torch::Tensor w) {
-  TORCH_CHECK((act == NONE || act == SILU) &&
-              (block_m == 32 || block_m == 64 || block_m == 128));
+  TORCH_CHECK(act == NONE || act == SILU);
   for (const auto *t : {&rows, &w})
     TORCH_CHECK(t->is_cuda() && t->dim() == 2 && t->is_contiguous() &&
                 t->scalar_type() == at::kBFloat16 &&
@@ -410,8 +411,12 @@ torch::Tensor moe_gemm_tiled_shared(
   const long cols = act == SILU ? N / 2 : N;
   TORCH_CHECK(w.size(1) == K && K > 0 && K % BK == 0 && cols > 0 &&
               cols % 8 == 0 && (act == NONE || N % 2 == 0) && T > 0 &&
-              T < 1L << 24 && N < 1L << 24,
+              T < 1L << 20 && N < 1L << 20 && N * K < 1L << 30,
               "moe_gemm_tiled_shared: K a multiple of 64, columns of 8");
+  TORCH_CHECK(block_m != 256 ||
+              tile_gemm_grouped_ok(A.numel(), n_pairs, W.size(1), W.size(2),
+                                   (int)act),
+              "moe_gemm_tiled_shared: operands below 2 GiB");
   auto out = torch::empty({T, cols}, rows.options());
   run_tiled(C, A, W, sorted_ids, expert_blocks, n_post_pad, topk_weights,
             n_pairs, topk, block_m, act, 0.0, 0.0,

@@ -36,6 +36,12 @@
 //    descriptor's bounds cut off, and a tile's first wait leaves the stores
 //    of the one before on their way (4 steps a tile before, 2.5 now).
 // A block of at most 128 rows runs half the products (waves of 64 x 128).
+// Beside a grouped product a plain one of the same form can take part in its
+// rounds (SHARED: a shared expert, rows in order): its tiles come first, spread
+// over the dies, and workgroups without one of the last of them take routed
+// tiles meanwhile. 4096 rows of 2048, 64 experts of 1408 and a shared one of
+// 2816: 661 us with sum and norm by launches of their own (352 and 128 tiles on
+// 256 CUs), 624 so.
 // Tiles of the last round are split along K when most CUs would idle
 // (plan_for); the fp32 parts are then joined by tile_sum_kernel in the order
 // of K. (us, before / now:) 4133 x 5120 x 27648 1448 (hipBLASLt) / 810; 4133
@@ -77,6 +83,11 @@ struct Args {
   const float *topk_w;
   int n_pairs, topk, a_bytes;
   float limit, alpha;
+  // grouped, with a product [s_rows, s_K] [s_N, s_K]^T beside it, a tile of
+  // which takes about s_slots times as long
+  __hip_bfloat16 *s_C;
+  const __hip_bfloat16 *s_A, *s_W;
+  int s_rows, s_K, s_N, s_nbm, s_nbn, s_group, s_slots;
 };
 
 #define RFL(x) __builtin_amdgcn_readfirstlane(x)
@@ -259,8 +270,9 @@ DEV_INLINE shortx8 results(const float *g, const float *u, float scale,
 }
 
 // ONCE: a weight row is read by one workgroup (non-temporal loads leave the
-// L2 to x)
-template <int FORM, int ACT, bool GROUPED, bool BIAS, bool ONCE = false>
+// L2 to x). SHARED (grouped, gated or scatter): the product beside
+template <int FORM, int ACT, bool GROUPED, bool BIAS, bool ONCE = false,
+          bool SHARED = false>
 __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   // two stages of x, then three of W
   __shared__ __attribute__((aligned(16))) char smem[5 * SLOT];
@@ -282,16 +294,58 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   const int step = gridDim.x >> 3;  // workgroups of a die
   const int w0 = (die * whole >> 3) + idx, w1 = (die + 1) * whole >> 3;
   const int p0 = (die * parts >> 3) + idx, p1 = (die + 1) * parts >> 3;
-  const int n_whole = RFL(max(0, (w1 - w0 + step - 1) / step));
-  const int items = RFL(n_whole + max(0, (p1 - p0 + step - 1) / step));
+  int n_whole = RFL(max(0, (w1 - w0 + step - 1) / step));
+  // SHARED: a die's tiles of the product beside are dealt out first; of the
+  // others a workgroup without one of the last `b` of these takes `lead` while
+  // those take theirs (`width` such workgroups a turn), then all take turns
+  int n_sh = 0, sh0 = 0, lead = 0, width = 0, b = 0, behind = 0;
+  if (SHARED) {
+    const int all = P.s_nbm * P.s_nbn;
+    sh0 = (die * all >> 3) + idx;
+    const int mine = ((die + 1) * all >> 3) - (die * all >> 3);
+    n_sh = RFL(max(0, (mine - idx + step - 1) / step));
+    b = mine % step;
+    if (b > 0) {
+      width = step - b;
+      behind = P.s_slots * width;
+      lead = idx >= b ? P.s_slots : 0;
+    }
+    const int n = w1 - (w0 - idx);  // the die's others
+    int first = 0;
+    if (lead > 0)
+      first = min(lead, max(0, (n - (idx - b) + width - 1) / width));
+    n_whole = RFL(first);
+    if (first == lead)
+      n_whole = RFL(first + max(0, (n - behind - idx + step - 1) / step));
+  }
+  const int items =
+      RFL(n_sh + n_whole + max(0, (p1 - p0 + step - 1) / step));
   if (items == 0) return;
   struct Item {
-    int mb, nb, k0, nk, part;
+    int mb, nb, k0, nk, part, sh;
   };
-  auto item_at = [&](int i) {
+  auto item_at = [&](int i) __attribute__((always_inline)) {
     Item it;
     int t;
-    if (i < n_whole) {
+    it.sh = SHARED && i < n_sh;
+    if (SHARED) {
+      it.k0 = 0;
+      it.part = -1;
+      if (it.sh) {
+        t = sh0 + i * step;
+        it.nk = P.s_K / BK;
+        const int g = t / (P.s_group * P.s_nbn), r0 = g * P.s_group;
+        const int in_g = t - r0 * P.s_nbn;
+        const int rows = min(P.s_group, P.s_nbm - r0);
+        it.nb = RFL(in_g / rows);
+        it.mb = RFL(r0 + in_g - it.nb * rows);
+        return it;
+      }
+      const int j = i - n_sh;
+      t = w0 - idx + (j < lead ? j * width + idx - b
+                               : behind + (j - lead) * step + idx);
+      it.nk = nkt;
+    } else if (i < n_whole) {
       t = w0 + i * step;
       it.k0 = 0;
       it.nk = nkt;
@@ -307,32 +361,42 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
     return it;
   };
   // at most 128 rows of the block are in use
-  auto is_half = [&](int mb) {
+  auto is_half = [&](const Item &it) __attribute__((always_inline)) {
+    if (SHARED && it.sh) return (int)(P.s_rows - it.mb * 256 <= 128);
     if (GROUPED)
-      return (int)(table_at(P.sorted_ids, mb * 256 + 128) >= P.n_pairs);
-    return (int)(min(P.bm, P.M - mb * P.bm) <= 128);
+      return (int)(table_at(P.sorted_ids, it.mb * 256 + 128) >= P.n_pairs);
+    return (int)(min(P.bm, P.M - it.mb * P.bm) <= 128);
   };
 
   // sources of this lane: LDS rows j * 32 + wave * 8 + sub, 16 B units
   // permuted by row & 7
   const int sub = lane >> 3, unit = ((lane & 7) ^ sub) * 16;
   int va[8], vw[8], ids[8];
+  auto a_rows = [&](int K) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int r = j * 32 + wave * 8 + sub, i = r & 15, n = r >> 4;
-    va[j] = r * K * 2 + unit;
-    // row i of fragment n: lane group i >> 2 holds its columns i & 3
-    int c;
-    if (FORM == GATED)
-      c = (n >> 2) * 32 + (i >> 2) * 8 + ((n >> 1) & 1) * 4 + (i & 3) +
-          (n & 1) * NC;
-    else
-      c = (n >> 1) * 32 + (i >> 2) * 8 + (n & 1) * 4 + (i & 3);
-    vw[j] = c * K * 2 + unit;
-  }
-  auto fetch_ids = [&](int i) {
+    for (int j = 0; j < 8; ++j)
+      va[j] = (j * 32 + wave * 8 + sub) * K * 2 + unit;
+  };
+  auto w_rows = [&](int K, int NC) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = j * 32 + wave * 8 + sub, i = r & 15, n = r >> 4;
+      // row i of fragment n: lane group i >> 2 holds its columns i & 3
+      int c;
+      if (FORM == GATED)
+        c = (n >> 2) * 32 + (i >> 2) * 8 + ((n >> 1) & 1) * 4 + (i & 3) +
+            (n & 1) * NC;
+      else
+        c = (n >> 1) * 32 + (i >> 2) * 8 + (n & 1) * 4 + (i & 3);
+      vw[j] = c * K * 2 + unit;
+    }
+  };
+  a_rows(K);
+  w_rows(K, NC);
+  auto fetch_ids = [&](int i) __attribute__((always_inline)) {
     if (i >= items) return;
     const Item it = item_at(i);
+    if (SHARED && it.sh) return;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       ids[j] = P.sorted_ids[it.mb * 256 + j * 32 + wave * 8 + sub];
@@ -341,13 +405,30 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   // item they read nothing
   __amdgpu_buffer_rsrc_t ra, rw;
   int li = -1, lleft = 0, lso = 0;
-  auto advance = [&]() {
+  auto advance = [&]() __attribute__((always_inline)) {
     if (lleft == 0) {
       ++li;
       if (li < items) {
         const Item it = item_at(li);
         lleft = it.nk;
         lso = it.k0 * ROW_B;
+        if (SHARED) {
+          if (it.sh) {
+            const int sk = P.s_K, at = it.nb * BC;
+            rw = rows_of(P.s_W + (long)at * sk,
+                         (FORM == GATED ? P.s_N - at : min(256, P.s_N - at)) *
+                             sk * 2);
+            ra = rows_of(P.s_A + (long)it.mb * 256 * sk,
+                         min(256, P.s_rows - it.mb * 256) * sk * 2);
+            a_rows(sk);
+            w_rows(sk, P.s_N >> 1);
+            if (GATHER) fetch_ids(li + 1);
+            --lleft;
+            return;
+          }
+          a_rows(K);
+          w_rows(K, NC);
+        }
         const __hip_bfloat16 *w = P.W;
         if (GROUPED) w += (long)table_at(P.expert_blocks, it.mb) * P.N * K;
         rw = rows_of(w + (long)it.nb * BC * K,
@@ -418,7 +499,7 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   __builtin_amdgcn_s_barrier();
 
   Item it = item_at(0);
-  int half = is_half(it.mb);
+  int half = is_half(it);
   int ab = a_base(half);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -429,10 +510,10 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
   int stores = 0;      // of the tile before, if this is a tile's first step
   for (int ci = 0; ci < items; ++ci) {
     const Item nx = item_at(min(ci + 1, items - 1));
-    const int next_half = is_half(nx.mb);
+    const int next_half = is_half(nx);
     const int next_ab = a_base(next_half);
     int row_id[8];
-    if (GROUPED) {
+    if (GROUPED && !(SHARED && it.sh)) {
 #pragma unroll
       for (int m = 0; m < 8; ++m)
         row_id[m] = P.sorted_ids[it.mb * 256 +
@@ -545,6 +626,9 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
       }
       // this lane's columns: 8 at c0 + 32 p
       constexpr int NP = BC / 64;
+      const bool sh = SHARED && it.sh;
+      const int NCi =
+          sh ? (FORM == GATED ? P.s_N >> 1 : P.s_N) : NC;
       const int c0 = it.nb * BC + wn * (BC / 2) + xhi * 8;
       float bias[NP][8];
       if (BIAS) {
@@ -556,7 +640,8 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
       if (FORM == SCATTER) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          sc[m] = P.topk_w ? P.topk_w[min(row_id[m], P.n_pairs - 1)] : 1.f;
+          sc[m] = P.topk_w && !sh ? P.topk_w[min(row_id[m], P.n_pairs - 1)]
+                                  : 1.f;
       }
       auto result = [&](auto mt_, auto pt) {
         constexpr int m = decltype(mt_)::value, p = decltype(pt)::value;
@@ -590,21 +675,23 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(const Args P) {
       // lies outside is not stored
       const int bm = GROUPED ? 256 : P.bm;
       const auto rc =
-          FORM == SCATTER
+          sh ? rows_of(P.s_C + (long)it.mb * 256 * NCi,
+                       min(256, P.s_rows - it.mb * 256) * NCi * 2)
+          : FORM == SCATTER
               ? rows_of(P.C, P.n_pairs * NC * 2)
               : rows_of(P.C + (long)it.mb * bm * NC,
                         (GROUPED ? 256 : min(bm, P.M - it.mb * bm)) * NC * 2);
       repeat<MT>([&](auto mt_) {
         constexpr int m = decltype(mt_)::value;
         ORDER;
-        const int row = FORM == SCATTER ? row_id[m] : r0 + m * 16;
-        const bool used = !GROUPED || row_id[m] < P.n_pairs;
-        const int at = (row * NC + c0) * 2;
+        const int row = FORM == SCATTER && !sh ? row_id[m] : r0 + m * 16;
+        const bool used = !GROUPED || sh || row_id[m] < P.n_pairs;
+        const int at = (row * NCi + c0) * 2;
         repeat<NP>([&](auto pt) {
           constexpr int p = decltype(pt)::value;
           const tg_u4 o = __builtin_bit_cast(tg_u4, result(mt_, pt));
           __builtin_amdgcn_raw_buffer_store_b128(
-              o, rc, used && c0 + p * 32 < NC ? at + p * 64 : 0x7ffffff0, 0,
+              o, rc, used && c0 + p * 32 < NCi ? at + p * 64 : 0x7ffffff0, 0,
               0);
         });
       });
@@ -891,7 +978,7 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
                        const int *n_post_pad, const float *topk_w,
                        long max_blocks, long n_pairs, long topk, long Nd,
                        long K, long a_rows, int act, float limit,
-                       float alpha) {
+                       float alpha, const TileShared &shared) {
   const bool gated = act == SILU || act == CLAMP;
   Args P{};
   P.C = (__hip_bfloat16 *)C;
@@ -914,11 +1001,33 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
   P.limit = limit;
   P.alpha = alpha;
   auto stream = at::cuda::getCurrentCUDAStream();
-  const dim3 grid(
-      std::min<long>((max_blocks * P.nbn + 7) / 8 * 8, compute_units()));
-#define RUN(FORM, ACT)                                                       \
-  hipLaunchKernelGGL((tile_gemm_kernel<FORM, ACT, true, false>), grid,       \
+  if (shared.C) {
+    P.s_C = (__hip_bfloat16 *)shared.C;
+    P.s_A = (const __hip_bfloat16 *)shared.A;
+    P.s_W = (const __hip_bfloat16 *)shared.W;
+    P.s_rows = shared.rows;
+    P.s_K = shared.K;
+    P.s_N = shared.N;
+    P.s_nbm = (shared.rows + 255) / 256;
+    P.s_nbn = ((gated ? shared.N / 2 : shared.N) + (gated ? 127 : 255)) /
+              (gated ? 128 : 256);
+    const int groups = (P.s_nbm + 7) / 8;
+    P.s_group = (P.s_nbm + groups - 1) / groups;
+    P.s_slots = std::max<long>(1, (shared.K + K / 2) / K);
+  }
+  const dim3 grid(std::min<long>(
+      (max_blocks * P.nbn + P.s_nbm * P.s_nbn + 7) / 8 * 8, compute_units()));
+#define RUN(FORM, ACT, ...)                                                  \
+  hipLaunchKernelGGL((tile_gemm_kernel<FORM, ACT, true, false                \
+                                       __VA_OPT__(,) __VA_ARGS__>), grid,    \
                      dim3(256), 0, stream, P)
+  if (shared.C) {
+    if (act == NONE) RUN(SCATTER, NONE, false, true);
+    else if (act == SILU) RUN(GATED, SILU, false, true);
+    else TORCH_CHECK(false, "moe_gemm_tiled_shared: act ", act);
+    HIP_CHECK_KERNEL();
+    return;
+  }
   if (act == NONE) RUN(SCATTER, NONE);
   else if (act == SILU) RUN(GATED, SILU);
   else if (act == CLAMP) RUN(GATED, CLAMP);

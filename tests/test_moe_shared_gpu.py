@@ -15,7 +15,11 @@ pytestmark = pytest.mark.gpu
     (49, 8, 2, 2048, 192, 384),     # just over: 64
     (161, 8, 2, 320, 128, 256),     # 128
     (256, 4, 2, 256, 64, 64),
-    (130, 64, 6, 128, 64, 128)])
+    (130, 64, 6, 128, 64, 128),
+    (260, 2, 1, 128, 64, 64),       # 256: a block of rows and four rows
+    (700, 4, 2, 128, 64, 192),      # a second product of thrice the K
+    (513, 2, 2, 320, 448, 1088),    # columns that end inside a tile
+    (2100, 8, 2, 1024, 512, 1024)])  # several tiles a workgroup
 def test_moe_shared(T, E, topk, H, I, S):
     from gllm_amd import ops
     gen = torch.Generator().manual_seed(T + S)
@@ -34,7 +38,6 @@ def test_moe_shared(T, E, topk, H, I, S):
     weights = torch.rand(T, topk, generator=gen) + 0.1
     norm_w = torch.rand(H, generator=gen) + 0.5
     dev = [t.cuda() for t in (x, w13, w2, weights, ids, up, down)]
-    assert ops.moe_shared_beside(dev[0], dev[1], dev[2], topk, *dev[5:])
     got_res = res.cuda()
     out = ops.fused_moe(*dev[:5], num_global_experts=E, add_norm=(
         None, got_res, norm_w.cuda(), 1e-6), shared_mlp=tuple(dev[5:]))
@@ -46,12 +49,11 @@ def test_moe_shared(T, E, topk, H, I, S):
 
     xd = x.double()
     want = res.double() + gated(xd, up, down)
-    for t in range(T):
-        for j in range(topk):
-            if ids[t, j] >= 0:
-                e = ids[t, j]
-                want[t] += weights[t, j].double() * gated(
-                    xd[t:t + 1], w13[e], w2[e])[0]
+    for e in range(E):
+        row, col = (ids == e).nonzero(as_tuple=True)
+        if len(row):
+            want.index_add_(0, row, gated(xd[row], w13[e], w2[e]) *
+                            weights[row, col].double()[:, None])
     # each term is rounded to bf16 once inside and once as it is stored, and
     # the stored sum once more: some 2^-8 of the terms' sizes, which are at
     # most a few times the row's
