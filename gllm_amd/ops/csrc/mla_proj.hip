@@ -3,9 +3,9 @@
 //
 //   mla_prepare   one workgroup per token: the latent row is RMS-normed, its
 //                 rotated part turned, both written to their slot of the
-//                 paged cache; the queries' rotated parts turned into the
-//                 attention's query rows
-//   mla_absorb    q_lat[t, h, :] = q_nope[t, h, :] W_uk[h]
+//                 paged cache; the queries' rotated parts turned
+//   mla_queries   the same into the attention's query rows, and beside it
+//                 q_lat[t, h, :] = q_nope[t, h, :] W_uk[h]
 //   mla_project   out[t, h, :] = o_lat[t, h, :] W_uv[h]^T
 //
 // Bound by launches and by fp32 copies where it was torch: three slices
@@ -13,8 +13,11 @@
 // batched products that converted their weights to fp32 in every layer (22
 // launches). The products take bf16 operands with fp32 sums: the same
 // products, exact in fp32.
-// A layer of 128 decoding requests, 16 heads: 5 + 5 + 8 us where these
-// launches took 105; of 4096 prompt tokens: 8 + 43 + 89 us for 390.
+// A layer of 128 decoding requests, 16 heads: 7 + 8 us where these launches
+// took 105 (rows and absorbed products, which need nothing of each other, by a
+// launch each: 5 + 5); of 4096 prompt tokens: 53 + 89 us for 390. (The products
+// from the parts of the split projection, without its sum: 2 us less at 128
+// rows, level at 64, 2 to 4 us more with few heads.)
 
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -63,8 +66,8 @@ DEV_INLINE void rotate8(const __hip_bfloat16 *src, __hip_bfloat16 *dst,
 // 4 waves: wave 0 the latent row, waves 1 to 3 the queries. PROMPT: the latent
 // goes to lat and pe too, and the queries are turned where they are.
 template <typename TW, bool PROMPT>
-__global__ __launch_bounds__(256) void mla_prepare_kernel(
-    __hip_bfloat16 *__restrict__ qf,        // [T, H, DK] (dims LORA..)
+DEV_INLINE void prepare_row(
+    const long t, __hip_bfloat16 *__restrict__ qf,  // [T, H, DK] (dims LORA..)
     __hip_bfloat16 *__restrict__ lat,       // [T, LORA]
     __hip_bfloat16 *__restrict__ pe,        // [T, ROPE]
     __hip_bfloat16 *__restrict__ k_cache,   // [slots, DK]
@@ -73,7 +76,6 @@ __global__ __launch_bounds__(256) void mla_prepare_kernel(
     const TW *__restrict__ norm_w, float eps,
     const long *__restrict__ positions, const float *__restrict__ cos_sin,
     const long *__restrict__ slots, int H) {
-  const long t = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float *cs = cos_sin + positions[t] * ROPE;
   if (wave == 0) {
@@ -101,17 +103,43 @@ __global__ __launch_bounds__(256) void mla_prepare_kernel(
   }
 }
 
-// Workgroup = 64 tokens (16 per wave), one head, 128 latent columns. The
-// weight block [128 k][128 columns] sits in LDS as two column blocks of
+template <typename TW>
+__global__ __launch_bounds__(256) void mla_prepare_kernel(
+    __hip_bfloat16 *__restrict__ lat, __hip_bfloat16 *__restrict__ pe,
+    __hip_bfloat16 *__restrict__ k_cache, __hip_bfloat16 *q, long q_stride,
+    const __hip_bfloat16 *__restrict__ kv, long kv_stride,
+    const TW *__restrict__ norm_w, float eps,
+    const long *__restrict__ positions, const float *__restrict__ cos_sin,
+    const long *__restrict__ slots, int H) {
+  prepare_row<TW, true>(blockIdx.x, nullptr, lat, pe, k_cache, q, q_stride,
+                        kv, kv_stride, norm_w, eps, positions, cos_sin, slots,
+                        H);
+}
+
+// A workgroup per 64 tokens (16 per wave), head and 128 latent columns, and
+// behind those one per token for its row. The weight block [128 k][128 columns] sits in LDS as two column blocks of
 // [128][128 B] (16 B units permuted by k & 7) and is read transposed; the
 // products are W^T q^T, so a lane holds four neighbouring columns of a token.
-__global__ __launch_bounds__(256) void mla_absorb_kernel(
-    __hip_bfloat16 *__restrict__ qf,       // [T, H, DK] (dims 0..LORA)
-    const __hip_bfloat16 *__restrict__ q, long q_stride,
+template <typename TW>
+__global__ __launch_bounds__(256) void mla_queries_kernel(
+    __hip_bfloat16 *__restrict__ qf,       // [T, H, DK]
+    __hip_bfloat16 *__restrict__ k_cache, __hip_bfloat16 *q, long q_stride,
+    const __hip_bfloat16 *__restrict__ kv, long kv_stride,
+    const TW *__restrict__ norm_w, float eps,
+    const long *__restrict__ positions, const float *__restrict__ cos_sin,
+    const long *__restrict__ slots,
     const __hip_bfloat16 *__restrict__ w,  // [H, WROWS, LORA]
     int T, int H) {
   __shared__ __attribute__((aligned(16))) char wt[NOPE * CHUNK * 2];
-  const int t0 = blockIdx.x * TOK, h = blockIdx.y, n0 = blockIdx.z * CHUNK;
+  const int tiles = (T + TOK - 1) / TOK, block = blockIdx.x;
+  if (block >= tiles * H * (LORA / CHUNK)) {
+    prepare_row<TW, false>(block - tiles * H * (LORA / CHUNK), qf, nullptr,
+                           nullptr, k_cache, q, q_stride, kv, kv_stride,
+                           norm_w, eps, positions, cos_sin, slots, H);
+    return;
+  }
+  const int t0 = block % tiles * TOK, h = block / tiles % H;
+  const int n0 = block / tiles / H * CHUNK;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int l16 = lane & 15, lhi = lane >> 4;
   const __hip_bfloat16 *wh = w + (long)h * WROWS * LORA + n0;
@@ -236,32 +264,6 @@ void check_rows(const torch::Tensor &q, const torch::Tensor &kv,
               "norm_w: fp32 or bf16");
 }
 
-// qf: the query rows of the absorbed form, nullptr for prompts
-void prepare(void *qf, void *lat, void *pe, torch::Tensor &q,
-             const torch::Tensor &kv, const torch::Tensor &norm_w, float eps,
-             const torch::Tensor &positions, const torch::Tensor &cos_sin,
-             const torch::Tensor &k_cache, const torch::Tensor &slots) {
-  const long T = q.size(0);
-  auto stream = at::cuda::getCurrentCUDAStream();
-#define PREP(TW, PROMPT)                                                     \
-  hipLaunchKernelGGL((mla_prepare_kernel<TW, PROMPT>), dim3(T), dim3(256),   \
-                     0, stream, (__hip_bfloat16 *)qf, (__hip_bfloat16 *)lat, \
-                     (__hip_bfloat16 *)pe,                                   \
-                     (__hip_bfloat16 *)k_cache.data_ptr(),                   \
-                     (__hip_bfloat16 *)q.data_ptr(), (long)q.stride(0),      \
-                     (const __hip_bfloat16 *)kv.data_ptr(),                  \
-                     (long)kv.stride(0), (const TW *)norm_w.data_ptr(), eps, \
-                     positions.data_ptr<long>(), cos_sin.data_ptr<float>(),  \
-                     slots.data_ptr<long>(), (int)(q.size(1) / QD))
-  const bool wide = norm_w.scalar_type() == at::kFloat;
-  if (qf && wide) PREP(float, false);
-  else if (qf) PREP(__hip_bfloat16, false);
-  else if (wide) PREP(float, true);
-  else PREP(__hip_bfloat16, true);
-#undef PREP
-  HIP_CHECK_KERNEL();
-}
-
 }  // namespace
 
 // w_kvb [H * 256, 512]; writes the cache rows of `slots`, returns the query
@@ -279,14 +281,22 @@ torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
               w_kvb.size(1) == LORA);
   auto qf = torch::empty({T, (long)H, (long)DK}, q.options());
   if (T == 0) return qf;
-  prepare(qf.data_ptr(), nullptr, nullptr, q, kv, norm_w, (float)eps,
-          positions, cos_sin, k_cache, slots);
-  hipLaunchKernelGGL(mla_absorb_kernel,
-                     dim3((T + TOK - 1) / TOK, H, LORA / CHUNK), dim3(256),
-                     0, at::cuda::getCurrentCUDAStream(),
-                     (__hip_bfloat16 *)qf.data_ptr(),
-                     (const __hip_bfloat16 *)q.data_ptr(), (long)q.stride(0),
-                     (const __hip_bfloat16 *)w_kvb.data_ptr(), (int)T, H);
+  const long blocks = (T + TOK - 1) / TOK * H * (LORA / CHUNK) + T;
+  TORCH_CHECK(blocks < 1L << 31);
+#define ROWS(TW)                                                             \
+  (__hip_bfloat16 *)k_cache.data_ptr(), (__hip_bfloat16 *)q.data_ptr(),      \
+      (long)q.stride(0), (const __hip_bfloat16 *)kv.data_ptr(),              \
+      (long)kv.stride(0), (const TW *)norm_w.data_ptr(), (float)eps,         \
+      positions.data_ptr<long>(), cos_sin.data_ptr<float>(),                 \
+      slots.data_ptr<long>()
+#define RUN(TW)                                                              \
+  hipLaunchKernelGGL((mla_queries_kernel<TW>), dim3(blocks), dim3(256), 0,   \
+                     at::cuda::getCurrentCUDAStream(),                       \
+                     (__hip_bfloat16 *)qf.data_ptr(), ROWS(TW),              \
+                     (const __hip_bfloat16 *)w_kvb.data_ptr(), (int)T, H)
+  if (norm_w.scalar_type() == at::kFloat) RUN(float);
+  else RUN(__hip_bfloat16);
+#undef RUN
   HIP_CHECK_KERNEL();
   return qf;
 }
@@ -302,9 +312,18 @@ std::vector<torch::Tensor> mla_prompt_rows(
   const long T = q.size(0);
   auto lat = torch::empty({T, (long)LORA}, q.options());
   auto pe = torch::empty({T, (long)ROPE}, q.options());
-  if (T > 0)
-    prepare(nullptr, lat.data_ptr(), pe.data_ptr(), q, kv, norm_w,
-            (float)eps, positions, cos_sin, k_cache, slots);
+  if (T == 0) return {lat, pe};
+#define RUN(TW)                                                              \
+  hipLaunchKernelGGL((mla_prepare_kernel<TW>), dim3(T), dim3(256), 0,        \
+                     at::cuda::getCurrentCUDAStream(),                       \
+                     (__hip_bfloat16 *)lat.data_ptr(),                       \
+                     (__hip_bfloat16 *)pe.data_ptr(), ROWS(TW),              \
+                     (int)(q.size(1) / QD))
+  if (norm_w.scalar_type() == at::kFloat) RUN(float);
+  else RUN(__hip_bfloat16);
+#undef RUN
+#undef ROWS
+  HIP_CHECK_KERNEL();
   return {lat, pe};
 }
 
