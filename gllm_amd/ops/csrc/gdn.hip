@@ -165,7 +165,9 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // XCDs and 68 with the longest first. One prompt of 4096: 253 -> 152, 64 of
 // 16: 98 -> 73, 30 tokens beside 700 + 900 + 15: 135 -> 58. (Queries and keys
 // in rows of another stride, sums of att and state in turn: no faster.)
-// local is bound by its stores (X, att: 105 MB); carry by the chain of a
+// local is bound by its chain of barriers and by its stores (X, att: 105 MB):
+// with 36 KB of LDS four workgroups a CU, 44 us where 73 KB and two took 52 (54
+// KB and three 46). carry is bound by the chain of a
 // chunk: products of U, split, barrier, products of the state, split, barrier,
 // 2.4 us alone and 4 us for two on a CU.
 typedef __attribute__((ext_vector_type(4))) float gdn_f4;
@@ -267,7 +269,7 @@ struct Gates {
   }
 };
 
-__global__ __launch_bounds__(512) void gdn_local_kernel(
+__global__ __launch_bounds__(512, 8) void gdn_local_kernel(
     short *__restrict__ wk,    // X_k, bf16 [blocks, Hv, 3, XK]
     float *__restrict__ u0,    // X_v [blocks, Hv, XV]
     short *__restrict__ att,   // bf16 [blocks, Hv, 3, AT]
@@ -299,13 +301,17 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
   // block R of the chunk: + R * Hv times a block's size
   const long block =
       (first_block(qsl[seq], seq) + blockIdx.x * (C / 16)) * Hv + h;
-  __shared__ __attribute__((aligned(16))) short Kt[C * KB], Vt[C * KB];
+  // (36 KB: four workgroups a CU. T takes the keys' place, whose columns X
+  // wants are in registers by then, and the values A's)
+  static_assert(C * SB * sizeof(short) == C * AS * sizeof(float));
   __shared__ __attribute__((aligned(16))) float Am[C * AS], Tm[C * AS];
+  short *Kt = reinterpret_cast<short *>(Tm);
+  short *Vt = reinterpret_cast<short *>(Am);
   __shared__ __attribute__((aligned(16))) float bb[C], btv[C], rkv[C],
       rqv[C], ck[C];
 
-  // ---- keys and values to LDS (rows past the end: the last one, factors
-  // 0), norms of keys and queries: 16 lanes per row
+  // ---- keys to LDS (rows past the end: the last one, factors 0), norms of
+  // keys and queries: 16 lanes per row
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int u = j * 512 + tid, t = u >> 4, c = (u & 15) * 8;
@@ -314,9 +320,7 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
         k + row * qk_stride + hk * D + c);
     const shortx8 qr = *reinterpret_cast<const shortx8 *>(
         q + row * qk_stride + hk * D + c);
-    *reinterpret_cast<shortx8 *>(Vt + t * KB + c) =
-        *reinterpret_cast<const shortx8 *>(v + row * v_stride + h * D + c);
-    *reinterpret_cast<shortx8 *>(Kt + t * KB + c) = kr;
+    *reinterpret_cast<shortx8 *>(Kt + t * SB + c) = kr;
     float kf[8], qf[8], nk = 0.f, nq = 0.f;
     unpack8<__hip_bfloat16>(kr, kf);
     unpack8<__hip_bfloat16>(qr, qf);
@@ -368,8 +372,8 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
       for (int ks = 0; ks < 4; ++ks) {
         GdnFrag ki, kt, qt;
         const int c = ks * 32 + lhi * 8;
-        ki.s = *reinterpret_cast<const shortx8 *>(Kt + (I * 16 + l16) * KB + c);
-        kt.s = *reinterpret_cast<const shortx8 *>(Kt + (R * 16 + l16) * KB + c);
+        ki.s = *reinterpret_cast<const shortx8 *>(Kt + (I * 16 + l16) * SB + c);
+        kt.s = *reinterpret_cast<const shortx8 *>(Kt + (R * 16 + l16) * SB + c);
         qt.s = *reinterpret_cast<const shortx8 *>(q + qrow * qk_stride +
                                                   hk * D + c);
         a = mma32(kt, ki, a);  // lane: i = l16, t = 4 lhi + r
@@ -381,7 +385,6 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
       const int t = R * 16 + lhi * 4 + r, i = I * 16 + l16;
       const float d = i < t ? __expf(bb[t] - bb[i]) : 0.f;
       Am[t * AS + i] = i < t ? btv[t] * d * rkv[t] * rkv[i] * a[r] : 0.f;
-      if (blk >= 10) Tm[t * AS + i] = 0.f;
     }
     const int t = R * 16 + l16, i0 = I * 16 + lhi * 4;
 #pragma unroll
@@ -400,8 +403,24 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
             p[j];
     }
   }
+  const int c0 = (wave & 3) * 32;
+  GdnFrag cols[2][2];
+  auto columns = [&](const short *src) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        read_tr(cols[kk][n], src, SB, kk * 32, c0 + n * 16, l16, lhi);
+  };
+  if (wave < 4) columns(Kt);
   __syncthreads();
   // ---- T: inverses of the diagonal blocks, a column per lane
+  if (wave >= 4 && wave < 6) {  // (0, 1) and (2, 3) are zero
+    const int R = (wave - 4) * 2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      Tm[(R * 16 + lhi * 4 + r) * AS + (R + 1) * 16 + l16] = 0.f;
+  }
   if (wave < 4) {
     float y[16];
 #pragma unroll
@@ -447,17 +466,19 @@ __global__ __launch_bounds__(512) void gdn_local_kernel(
     }
     __syncthreads();
   }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int u = j * 512 + tid;
+    const long row = start + min(u >> 4, len - 1);
+    *reinterpret_cast<shortx8 *>(Vt + (u >> 4) * SB + (u & 15) * 8) =
+        *reinterpret_cast<const shortx8 *>(v + row * v_stride + h * D +
+                                           (u & 15) * 8);
+  }
+  __syncthreads();
   // ---- X: waves 0..3 the keys' columns (transposed: a lane has four of a
   // row), 4..7 the values' (four rows of a column)
-  const short *src = wave < 4 ? Kt : Vt;
   const float *fac = wave < 4 ? ck : btv;
-  const int c0 = (wave & 3) * 32;
-  GdnFrag cols[2][2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-      read_tr(cols[kk][n], src, KB, kk * 32, c0 + n * 16, l16, lhi);
+  if (wave >= 4) columns(Vt);
 #pragma unroll
   for (int R = 0; R < 4; ++R) {
     gdn_f4 x[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
