@@ -90,15 +90,6 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
   out[(long)t * C + c] = ScalarOps<T>::from_f32(act ? silu_f(acc) : acc);
 }
 
-// silu of a sum that is rounded to T: 16-bit results take the hardware's
-// exponential and reciprocal (errors of about 2^-22, where the rounding is
-// 2^-9), which is a third of the instructions
-template <typename T>
-DEV_INLINE float silu_as(float z) {
-  if (sizeof(T) == 2) return z * __builtin_amdgcn_rcpf(1.f + __expf(-z));
-  return silu_f(z);
-}
-
 // 8 channels x TB consecutive tokens of one sequence per thread, 16 B accesses
 // (C % 8 == 0, aligned rows). The weights are loaded once per thread and the
 // inputs slide through registers; the first taps - 1 tokens of a portion find
@@ -110,10 +101,11 @@ DEV_INLINE float silu_as(float z) {
 // history, so it also rolls it: no launch of its own, no race.
 // TB 1 (and `store`): every portion is one token.
 //
-// Bound by memory with the silu above (by its instructions with expf and a
-// division): 4096 x 4096 in four prompts, 4 taps, state rolled, 31 -> 19 us,
-// 1000 x 4096 in one 16 -> 7.5, 20 tokens beside a prompt of 100 22 -> 7. (Four
-// tokens a thread for 4096 x 4096 21 us.)
+// Bound by the silu's instructions and by memory: 4096 x 4096 in four prompts, 4
+// taps, state rolled, 30 -> 26 us, 1000 x 4096 in one 16 -> 9.4, 20 tokens beside
+// a prompt of 100 22 -> 7.8. (The hardware's exponential and reciprocal as they
+// are take 19 us for the first, but round some results to another neighbour.
+// Four tokens a thread: 8 % more.)
 template <typename T, int TAPS, int TB>
 __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
     T *__restrict__ out, const T *__restrict__ x, long x_stride,
@@ -189,7 +181,7 @@ __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
         acc[e] += win[i + tap][e] * wf[e * TAPS + tap];
     if (act) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = silu_as<T>(acc[e]);
+      for (int e = 0; e < 8; ++e) acc[e] = silu_f(acc[e]);
     }
     st8<T>(out + (long)(start + r0 + i) * C + c0, acc);
   }

@@ -51,7 +51,7 @@ def test_short_conv(lens, init, taps, dtype):
     want_state = state.clone()
     want = oracle(x, w, want_state, slots.tolist(), init, lens, bias)
     # the result is rounded once; taps + 1 terms of at most ~10 are summed in
-    # 32 bits and the silu has a relative error of some 2^-21
+    # 32 bits and the silu has a relative error of some 2^-22
     step = 2 ** -8 if dtype == torch.bfloat16 else 2 ** -23
     assert ((got - want).abs() <= want.abs() * (step + 2 ** -20) + 2e-5).all()
     assert torch.equal(got_state.cpu(), want_state)
