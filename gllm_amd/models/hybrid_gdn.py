@@ -21,6 +21,7 @@ from typing import Iterable, List, Tuple
 import torch
 import torch.nn as nn
 
+from gllm_amd import ops
 from gllm_amd.layers.attention import Attention
 from gllm_amd.layers.embedding import ParallelLMHead, VocabParallelEmbedding
 from gllm_amd.layers.layernorm import GemmaRMSNorm, RMSNorm
@@ -325,7 +326,24 @@ class HybridFullAttention(nn.Module):
 
     def heads(self, positions, hidden, fctx):
         """The heads' outputs [T, heads * head_dim], before o_proj."""
-        qg, k, v = self.qkv_proj(hidden)
+        rows = self.qkv_proj.project(hidden)
+        qn, kn, rope = self.q_norm, self.k_norm, self.rotary_emb
+        if (not (self.gate or fctx.is_profile_run) and rows.is_cuda
+                and positions.dim() == 1 and qn.eps == kn.eps):
+            k_cache = fctx.k_caches[self.attn.layer_idx]
+            v_cache = fctx.v_caches[self.attn.layer_idx]
+            if (ops.qkv_rope_cache_ok(k_cache, v_cache, rope.cos_sin_cache,
+                                      rope.is_neox)
+                    and ops.qkv_norm_rope_cache_ok(
+                        rows, qn.scale(), kn.scale(), k_cache,
+                        rope.cos_sin_cache)):
+                q = ops.qkv_norm_rope_cache(
+                    rows, qn.scale(), kn.scale(), qn.eps, positions,
+                    rope.cos_sin_cache, k_cache, v_cache, fctx.slot_mapping,
+                    self.attn.num_heads)
+                return self.attn.attend(q, fctx)
+        proj = self.qkv_proj
+        qg, k, v = rows.split([proj.q_size, proj.kv_size, proj.kv_size], -1)
         T = hidden.shape[0]
         if self.gate:
             qg = qg.view(T, self.num_heads, 2 * self.head_dim)

@@ -1186,6 +1186,34 @@ def qkv_rope_cache(src: torch.Tensor, bias, positions: torch.Tensor,
                                      rounded)
 
 
+def qkv_norm_rope_cache_ok(src: torch.Tensor, q_w: torch.Tensor,
+                           k_w: torch.Tensor, k_cache: torch.Tensor,
+                           cos_sin: torch.Tensor) -> bool:
+    """Whether ``qkv_norm_rope_cache`` takes these, with caches that
+    ``qkv_rope_cache_ok`` takes."""
+    return (has_kernels() and src.dtype == torch.bfloat16 and src.dim() == 2
+            and src.stride(1) == 1 and src.stride(0) % 8 == 0
+            and k_cache.shape[3] <= 128 and cos_sin.shape[-1] % 16 == 0
+            and q_w.dtype == k_w.dtype
+            and q_w.dtype in (torch.bfloat16, torch.float32)
+            and all(t.is_contiguous() and t.numel() == k_cache.shape[3]
+                    for t in (q_w, k_w))
+            and all(t.data_ptr() % 16 == 0 for t in (src, q_w, k_w)))
+
+
+def qkv_norm_rope_cache(src: torch.Tensor, q_w: torch.Tensor,
+                        k_w: torch.Tensor, eps: float,
+                        positions: torch.Tensor, cos_sin: torch.Tensor,
+                        k_cache: torch.Tensor, v_cache: torch.Tensor,
+                        slot_mapping: torch.Tensor,
+                        num_heads: int) -> torch.Tensor:
+    """``qkv_rope_cache`` of bf16 rows with an RMS norm of each query and key
+    head in front of the rotation."""
+    return _gpu_kernels().qkv_norm_finish(src, q_w, k_w, eps, positions,
+                                          cos_sin, k_cache, v_cache,
+                                          slot_mapping, num_heads)
+
+
 def qkv_decode_ok(parts: torch.Tensor, k_cache: torch.Tensor,
                   num_heads: int, rounded: bool = False) -> bool:
     """Whether ``qkv_decode`` takes these rows and heads (with caches that

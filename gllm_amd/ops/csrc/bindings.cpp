@@ -20,6 +20,11 @@ void paged_attention_decode(torch::Tensor out, torch::Tensor q,
                             c10::optional<torch::Tensor> query_start_loc);
 bool decode_rows_ok(torch::Tensor k_cache, torch::Tensor v_cache, long Hq);
 torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
+torch::Tensor qkv_norm_finish(torch::Tensor src, torch::Tensor q_w,
+                              torch::Tensor k_w, double eps,
+                              torch::Tensor positions, torch::Tensor cos_sin,
+                              torch::Tensor k_cache, torch::Tensor v_cache,
+                              torch::Tensor slots, long Hq);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
@@ -229,6 +234,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_decode_ok", &qkv_decode_ok);
   m.def("qkv_decode", &qkv_decode,
         "bias, rotation, cache and decode attention of projection parts");
+  m.def("qkv_norm_finish", &qkv_norm_finish,
+        "qkv_finish of bf16 rows with a norm per head");
   m.def("qkv_finish", &qkv_finish,
         "bias, rotation, keys and values to the cache; queries");
   m.def("mla_paged_attention", &mla_paged_attention,
