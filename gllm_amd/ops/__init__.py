@@ -360,12 +360,17 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
             and T > 0 and K % 64 == 0 and inter % 64 == 0 and width % 64 == 0
             and down.shape[0] == K and gate_up.shape == (2 * width, K)):
         return False
+    experts = max(1, w13.shape[0])
+    block_m = _moe_block(T * topk / experts)
     if T <= 256:
-        return width <= 2 * inter
+        # (apart they are the streaming kernel's, and the second one's sums
+        # over shares of K are the same beside)
+        return (width <= 2 * inter and block_m < 256 and 2 * width >= 512
+                and _use_skinny(T, 512, K) and _use_skinny(T, K, width)
+                and _gpu_kernels().stream_slice(T, K, width) > 0)
     if K > 2048 or width * K < 4 << 20:
         return False
-    experts = max(1, w13.shape[0])
-    if _moe_block(T * topk / experts) < 256:
+    if block_m < 256:
         return width <= 2 * inter
     # (offsets of tile_gemm.hip are 32 bits)
     return (1536 <= T <= 6144 and 2 * max(inter, width) * K < 1 << 30

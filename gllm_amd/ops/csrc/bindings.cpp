@@ -25,6 +25,7 @@ torch::Tensor qkv_norm_finish(torch::Tensor src, torch::Tensor q_w,
                               torch::Tensor positions, torch::Tensor cos_sin,
                               torch::Tensor k_cache, torch::Tensor v_cache,
                               torch::Tensor slots, long Hq);
+long stream_slice(long M, long N, long K);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
@@ -222,6 +223,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "false = geometry not instantiated");
   m.def("resolve_tokens", &resolve_tokens,
         "token ids with places in the ring of sampled tokens");
+  m.def("stream_slice", &stream_slice,
+        "columns of K of one sum of stream_gemm's");
   m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
   m.def("tile_gemm", &tile_gemm, "x w^T + bias, or its gated form");
   m.def("tile_gemm_cost", &tile_gemm_cost,

@@ -173,6 +173,7 @@ void sigmoid_group_topk(torch::Tensor weights, torch::Tensor ids,
 // shared with the full extension (stream_gemm.hip, moe.hip,
 // elementwise.hip): what ops.linear / FusedMoE dispatch to in bf16
 torch::Tensor resolve_tokens(torch::Tensor tokens, torch::Tensor ring);
+long stream_slice(long M, long N, long K);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias);
 torch::Tensor stream_gemm_gated(torch::Tensor x, torch::Tensor w);
@@ -296,6 +297,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "sigmoid router with correction and group limits");
   m.def("resolve_tokens", &resolve_tokens,
         "token ids with places in the ring of sampled tokens");
+  m.def("stream_slice", &stream_slice,
+        "columns of K of one sum of stream_gemm's");
   m.def("stream_gemm", &stream_gemm, "x w^T + bias for at most 256 rows");
   m.def("tile_gemm", &tile_gemm, "x w^T + bias, or its gated form");
   m.def("tile_gemm_cost", &tile_gemm_cost,

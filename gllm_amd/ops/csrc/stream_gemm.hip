@@ -673,6 +673,29 @@ torch::Tensor parts_sum(torch::Tensor part,
   return out;
 }
 
+// How the plain product is formed: -1 by one launch of plan p, else by parts, of
+// tile_gemm.hip (their number) or of p (0).
+static int in_parts(int M, int N, int K, bool contiguous, Plan *p) {
+  int bm, tiled = 0;
+  *p = parts_plan(M, N, K);
+  if (contiguous) tile_parts_plan(M, N, K, &bm, &tiled);
+  if (tiled > 0 || p->splits > 1) {
+    const Plan one =
+        plain_plan(M, N, K, tiled > 0 ? tiled : p->splits, tiled > 0);
+    if (one.splits == 0) return tiled;
+    *p = one;
+  }
+  return -1;
+}
+
+long stream_slice(long M, long N, long K) {
+  TORCH_CHECK(M > 0 && M <= 256 && N > 0 && N < 1L << 20 && K > 0 &&
+              K % BK == 0 && K < 1L << 31, "stream_slice: no such product");
+  Plan p;
+  const int parts = in_parts(M, N, K, true, &p);
+  return parts < 0 ? K : parts > 0 ? 0 : p.k_slice;
+}
+
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> bias) {
   check_operands(x, w);
@@ -680,13 +703,9 @@ torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
   const void *bp = bias_ptr(bias, N);
   auto out = torch::empty({M, N}, x.options());
   if (M == 0) return out;
-  Plan p = parts_plan(M, N, w.size(1));
-  int bm, tiled = 0;
-  if (x.is_contiguous()) tile_parts_plan(M, N, w.size(1), &bm, &tiled);
-  if (tiled > 0 || p.splits > 1) {
-    p = plain_plan(M, N, w.size(1), tiled > 0 ? tiled : p.splits, tiled > 0);
-    if (p.splits == 0) return parts_sum(stream_parts(x, w), bias);
-  }
+  Plan p;
+  if (in_parts(M, N, w.size(1), x.is_contiguous(), &p) >= 0)
+    return parts_sum(stream_parts(x, w), bias);
   launch<PLAIN>(p, out.data_ptr(), x, w, bp);
   return out;
 }

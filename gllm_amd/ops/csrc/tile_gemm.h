@@ -22,3 +22,7 @@ void tile_gemm_grouped(void *C, const void *A, const void *W,
 void tile_parts_plan(long M, long N, long K, int *bm, int *splits);
 void tile_parts(float *part, const void *x, const void *w, long M, long N,
                 long K, int bm, int splits);
+
+// stream_gemm.hip: the columns of K that one fp32 sum of stream_gemm's covers
+// (the sums are added in the order of K), 0 where it takes tile_parts'
+long stream_slice(long M, long N, long K);
