@@ -360,7 +360,16 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
             and T > 0 and K % 64 == 0 and inter % 64 == 0 and width % 64 == 0
             and down.shape[0] == K and gate_up.shape == (2 * width, K)):
         return False
-    experts = max(1, w13.shape[0])
+    return _shared_beside(T, topk, max(1, w13.shape[0]), K, inter, width)
+
+
+def _shared_beside(T: int, topk: int, experts: int, K: int, inter: int,
+                   width: int) -> bool:
+    """The sizes of ``moe_shared_beside`` (rows, routed experts of K x inter,
+    a shared one of K x width)."""
+    # (what moe_gemm_tiled_shared takes of its two products)
+    if max(T, 2 * width, K) >= 1 << 20 or 2 * width * K >= 1 << 30:
+        return False
     block_m = _moe_block(T * topk / experts)
     if T <= 256:
         # (apart they are the streaming kernel's, and the second one's sums
@@ -373,8 +382,8 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     if block_m < 256:
         return width <= 2 * inter
     # (offsets of tile_gemm.hip are 32 bits)
-    return (1536 <= T <= 6144 and 2 * max(inter, width) * K < 1 << 30
-            and (T * topk + 255 * experts) * max(inter, K) < 1 << 30)
+    return (1536 <= T <= 6144 and 2 * inter * K < 1 << 30
+            and (T * topk + 256 * (experts + 1)) * max(inter, K) < 1 << 30)
 
 
 def moe_add_norm_ok(x: torch.Tensor, shared: Optional[torch.Tensor],
