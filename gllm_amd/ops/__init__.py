@@ -269,8 +269,12 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
     ``moe_add_norm_ok``). ``shared_mlp`` = (gate over up rows, down weight)
     of a gated feed-forward that all rows pass: its output is the ``shared``
     of ``add_norm``, its products run beside the experts' (see
-    ``moe_shared_beside``).
+    ``moe_shared_beside``) where these are on wide tiles.
     """
+    if shared_mlp is not None and (activation != "silu_glu" or add_norm is None
+                                   or add_norm[0] is not None):
+        raise ValueError("shared_mlp: beside gated experts, as the shared "
+                         "part of add_norm")
     T, K = x.shape
     E_local, rows13, _ = w13.shape
     inter = w2.shape[2]
@@ -307,6 +311,9 @@ def fused_moe(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
             k.moe_gemm_tiled(pair_out, act, w2, *tables, tw, n_pairs, topk,
                              block_m, 0, 0.0, 0.0)
     else:
+        if shared_mlp is not None:
+            add_norm = (linear(linear_silu(x, shared_mlp[0]),
+                               shared_mlp[1]),) + add_norm[1:]
         block_m = 16 if rpe < 12 else 32 if rpe < 40 else 64
         ids32, tables, rows = _moe_tables(topk_ids, E_local, expert_start,
                                           block_m)

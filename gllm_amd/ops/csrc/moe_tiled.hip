@@ -390,7 +390,7 @@ static void run_tiled(const torch::Tensor &C, const torch::Tensor &A,
   } while (0)
   if (shared.C && block_m == 32) WITH(32, 128, 1, 4, 4, 2);
   else if (shared.C && block_m == 64) WITH(64, 128, 1, 4, 3, 2);
-  else if (shared.C) WITH(128, 128, 2, 2, 3, 0);
+  else if (shared.C && block_m == 128) WITH(128, 128, 2, 2, 3, 0);
   else if (block_m == 32) FORMS(32, 128, 1, 4, 4, 2);
   else if (block_m == 64) FORMS(64, 128, 1, 4, 3, 2);
   else if (block_m == 128) FORMS(128, 128, 2, 2, 3, 0);
@@ -422,6 +422,9 @@ torch::Tensor moe_gemm_tiled_shared(
     long n_pairs, long topk, long block_m, long act, torch::Tensor rows,
     torch::Tensor w) {
   TORCH_CHECK(act == NONE || act == SILU);
+  TORCH_CHECK(block_m == 32 || block_m == 64 || block_m == 128 ||
+              block_m == 256,
+              "moe_gemm_tiled_shared: block_m must be 32/64/128/256");
   for (const auto *t : {&rows, &w})
     TORCH_CHECK(t->is_cuda() && t->dim() == 2 && t->is_contiguous() &&
                 t->scalar_type() == at::kBFloat16 &&

@@ -47,3 +47,32 @@ def test_beside_is_apart(T, E, topk, H, I, S):
         shared, want_res, norm_w, 1e-6))
     assert torch.equal(got_res, want_res)
     assert torch.equal(got, want)
+
+
+def test_where_there_are_no_wide_tiles():
+    """Widths that 64 does not divide: the shared expert's products apart."""
+    from gllm_amd import ops
+    x, w13, w2, weights, ids, up, down, res, norm_w = operands(
+        40, 8, 2, 72, 64, 128)
+    assert not ops.moe_shared_beside(x, w13, w2, 2, up, down)
+    got_res, want_res = res.clone(), res.clone()
+    got = ops.fused_moe(x, w13, w2, weights, ids, add_norm=(
+        None, got_res, norm_w, 1e-6), shared_mlp=(up, down))
+    want = ops.fused_moe(x, w13, w2, weights, ids, add_norm=(
+        ops.linear(ops.linear_silu(x, up), down), want_res, norm_w, 1e-6))
+    assert torch.equal(got_res, want_res)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("block_m", [16, 48, 512])
+def test_tables_of_another_block_are_refused(block_m):
+    """(on the host, ahead of any launch)"""
+    from gllm_amd import ops
+    x, w13, w2, weights, ids, up, down, res, norm_w = operands(
+        40, 8, 2, 128, 64, 128)
+    tables = [torch.zeros(n, dtype=torch.int32, device="cuda")
+              for n in (80 + 8 * block_m, 80 + 8, 1)]
+    act = x.new_empty(80 + 8 * block_m, 64)
+    with pytest.raises(RuntimeError, match="block_m"):
+        ops._gpu_kernels().moe_gemm_tiled_shared(
+            act, x, w13, *tables, None, 80, 2, block_m, 1, x, up)
