@@ -137,6 +137,9 @@ class GatedDeltaNet(nn.Module):
         """The gated heads [T, value_dim] before out_proj; None in a
         profile run (no state to work on)."""
         if fctx.is_profile_run or fctx.ssm_pool is None:
+            if fctx.largest_batch is not None and \
+                    self.head_k_dim == self.head_v_dim == 128:
+                ops.gdn_reserve(hidden, *fctx.largest_batch, self.tp_v)
             return None
         T = hidden.shape[0]
         k_tp = self.tp_k_heads * self.head_k_dim

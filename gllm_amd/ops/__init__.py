@@ -722,6 +722,14 @@ def gdn_rows_ok(qkvz: torch.Tensor, ba: torch.Tensor, conv_w: torch.Tensor,
             and qkvz.data_ptr() % 16 == 0 and norm_w.data_ptr() % 16 == 0)
 
 
+def gdn_reserve(like: torch.Tensor, rows: int, sequences: int, Hv: int):
+    """Takes from ``like``'s device what the recurrence of ``gdn_rows`` works
+    on for that many rows and sequences and gives it back (a profile run of a
+    layer whose state is not there yet)."""
+    if like.is_cuda and has_kernels():
+        _gpu_kernels().gdn_reserve(like, rows, sequences, Hv)
+
+
 def gdn_rows(qkvz: torch.Tensor, ba: torch.Tensor, conv_w: torch.Tensor,
              A_log: torch.Tensor, dt_bias: torch.Tensor,
              norm_w: torch.Tensor, eps: float, conv_state: torch.Tensor,

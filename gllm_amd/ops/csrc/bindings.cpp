@@ -167,6 +167,7 @@ void gdn_conv_update(torch::Tensor out, torch::Tensor x,
 void gdn_chunk_prefill(torch::Tensor o, torch::Tensor q, torch::Tensor k,
                        torch::Tensor v, torch::Tensor g, torch::Tensor beta,
                        torch::Tensor states, double scale);
+void gdn_reserve(torch::Tensor like, long T, long B, long Hv);
 torch::Tensor gdn_varlen(torch::Tensor conv, torch::Tensor ba,
                          torch::Tensor A_log, torch::Tensor dt_bias,
                          torch::Tensor states, torch::Tensor slots,
@@ -284,6 +285,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "batched causal-conv1d decode step w/ state roll");
   m.def("gdn_chunk_prefill", &gdn_chunk_prefill,
         "fused WY chunk-parallel gated delta rule prefill");
+  m.def("gdn_reserve", &gdn_reserve,
+        "takes and gives back the memory of a gdn_varlen call");
   m.def("gdn_varlen", &gdn_varlen,
         "ragged chunk-parallel gated delta rule");
   m.def("gdn_step", &gdn_step,

@@ -33,6 +33,9 @@ class ForwardContext:
     logits_indices: Optional[torch.Tensor] = None
     # profile/warmup run: attention may be skipped (no KV yet)
     is_profile_run: bool = False
+    # (rows, sequences) of the largest batch, in the profile run
+    largest_batch: Optional[tuple] = dataclasses.field(default=None,
+                                                       kw_only=True)
     # overlap mode: token ids contain negative ring placeholders
     has_placeholders: bool = False
     # hybrid GDN models: per-seq SSM state slots (core/ssm.py)

@@ -248,7 +248,8 @@ class ModelRunner:
             query_start_loc=torch.tensor([0, T], dtype=torch.int32,
                                          device=self.device),
             max_query_len=T, max_seq_len=T, k_caches=[], v_caches=[],
-            is_profile_run=True)
+            is_profile_run=True,
+            largest_batch=(cfg.maxp + cfg.maxd, cfg.maxd))
         fctx.logits_indices = torch.tensor([T - 1], device=self.device)
         with torch.no_grad():
             hidden, residual = self._stage_forward(input_ids, positions, fctx)
