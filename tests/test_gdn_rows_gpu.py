@@ -43,7 +43,7 @@ def oracle(conv, ba, z, A_log, dt, norm_w, state, slots, init, lens, Hk, Hv):
     ([1], [0]), ([1, 1, 1], [1, 1, 1]), ([1, 1], [1, 0]),
     ([63, 1, 64, 65, 2, 193], [0, 1, 1, 0, 0, 1]),
     ([15, 16, 17, 32, 33, 48, 49, 80], [1, 0] * 4),  # waves without rows
-    ([17] * 40, [1, 0] * 20)])     # (many sequences: wide columns)
+    ([17] * 40, [1, 0] * 20)])
 @pytest.mark.parametrize("Hk,Hv", [(2, 4), (3, 3)])
 def test_gdn_rows(lens, init, Hk, Hv):
     from gllm_amd import ops
