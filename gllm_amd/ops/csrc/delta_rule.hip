@@ -9,7 +9,8 @@
 //                      silu; the taps-1 inputs before a portion come from
 //                      the per-slot conv state
 //   conv_state_update  rolls the conv state to the portion's last inputs
-//                      (rows that are not whole 16 B vectors)
+//                      (rows that are not whole 16 B vectors,
+//                      few rows of many taps)
 //   delta_rule_varlen  per (sequence, value head): for each token
 //                        S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;
 //                        o = S^T q
@@ -91,27 +92,33 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
 }
 
 // 8 channels x TB consecutive tokens of one sequence per thread, 16 B accesses
-// (C % 8 == 0, aligned rows). The weights are loaded once per thread and the
-// inputs slide through registers; the first taps - 1 tokens of a portion find
-// their history in the per-slot state.
+// (C % 8 == 0, aligned rows). The weights are loaded once per thread, the first
+// taps - 1 tokens of a portion find their history in the per-slot state.
 //
 // A sequence's chunks of TB tokens begin at start / TB + sequence, which is
 // behind the last chunk of the one before, T / TB + B in all (some empty).
 // With TB >= TAPS - 1 the first chunk's thread alone reads a sequence's
-// history, so it also rolls it: no launch of its own, no race.
-// TB 1 (and `store`): every portion is one token.
+// history, so it also rolls it: no launch of its own, no race. So it does with
+// TB 1 where every portion is one token (`store`); TB 1 without leaves the
+// state to conv_state_update.
+// AHEAD: all inputs of a thread are loaded before its first sum. It is for
+// grids that leave SIMDs idle; else the inputs slide through a window of TAPS
+// rows, for whose registers more waves fit (bf16, 4 taps, eight tokens: 94 for
+// 150, 5 waves a SIMD for 3).
 //
-// Bound by the silu's instructions and by memory: 4096 x 4096 in four prompts, 4
-// taps, state rolled, 30 -> 26 us, 1000 x 4096 in one 16 -> 9.4, 20 tokens beside
-// a prompt of 100 22 -> 7.8. (The hardware's exponential and reciprocal as they
-// are take 19 us for the first, but round some results to another neighbour.
-// Four tokens a thread: 8 % more.)
-template <typename T, int TAPS, int TB>
+// Bound by the silu's instructions and by memory. 4096 channels of bf16, 4 taps
+// (us, with one token a thread in small batches and the state rolled by a launch
+// of its own / now): 4096 tokens in four prompts 31 / 25, 1000 in one 15 / 8.6,
+// 20 tokens beside a prompt of 100 21 / 7.2, 64 prompts of 16 37 / 11.6, 64
+// tokens 5.7 / 5.0; 8192 channels, eight prompts of 4096 322 / 270 (loaded ahead
+// 353). (The hardware's exponential and reciprocal as they are take 19 us for
+// the first, but round some results to another neighbour.)
+template <typename T, int TAPS, int TB, bool AHEAD>
 __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
     T *__restrict__ out, const T *__restrict__ x, long x_stride,
     const T *__restrict__ w, T *__restrict__ state,
     const long *__restrict__ slots, const int *__restrict__ has_init,
-    const int *__restrict__ qsl, int B, int C, int act, int n_tok,
+    const int *__restrict__ qsl, int B, int C, int act, int store, int n_tok,
     int n_chunks, const T *__restrict__ bias) {
   static_assert(TB == 1 || TB >= TAPS - 1, "one thread reads the history");
   const int nv = C / 8;
@@ -131,13 +138,14 @@ __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
   const int rows = b == B - 1 ? n_tok - start : n;
   // (an empty portion's only chunk still rolls its state)
   if (r0 >= rows && r0 > 0) return;
+  const bool init = has_init[b] != 0;
   T *st = state + ((long)slots[b] * C + c0) * (TAPS - 1);
   const T *xb = x + (long)start * x_stride + c0;
   // the input r rows into the portion, r >= 1 - TAPS
   auto input = [&](int r, float *v) {
     if (r >= 0) {
       ld8<T>(xb + (long)r * x_stride, v);
-    } else if (has_init[b] != 0) {
+    } else if (init) {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         v[e] = ScalarOps<T>::to_f32(st[e * (TAPS - 1) + TAPS - 1 + r]);
@@ -146,19 +154,8 @@ __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
       for (int e = 0; e < 8; ++e) v[e] = 0.f;
     }
   };
-  float win[TB + TAPS - 1][8];
-  if (rows > 0) {
-#pragma unroll
-    for (int i = 0; i < TB + TAPS - 1; ++i)
-      input(min(r0 + i - (TAPS - 1), rows - 1), win[i]);
-  }
-  float wf[8 * TAPS];  // [channel][tap], contiguous in memory
-#pragma unroll
-  for (int j = 0; j < TAPS; ++j) ld8<T>(w + (long)c0 * TAPS + j * 8, wf + j * 8);
-  float bf[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (bias) ld8<T>(bias + c0, bf);
-  if (TAPS > 1 && r0 == 0) {
-    // (16-bit values survive the trip through fp32 unchanged)
+  // (16-bit values survive the trip through fp32 unchanged)
+  auto roll = [&]() {
     float last[TAPS > 1 ? TAPS - 1 : 1][8];
 #pragma unroll
     for (int i = 0; i < TAPS - 1; ++i) input(n - (TAPS - 1) + i, last[i]);
@@ -167,10 +164,42 @@ __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         st[e * (TAPS - 1) + i] = ScalarOps<T>::from_f32(last[i][e]);
+  };
+  float win[AHEAD ? TB + TAPS - 1 : TAPS][8];
+  if (AHEAD) {
+    if (rows > 0) {
+#pragma unroll
+      for (int i = 0; i < TB + TAPS - 1; ++i)
+        input(min(r0 + i - (TAPS - 1), rows - 1), win[AHEAD ? i : 0]);
+    }
+    if (TAPS > 1 && r0 == 0) roll();
+  } else {
+#pragma unroll
+    for (int i = 1; i < TAPS; ++i) input(r0 + i - TAPS, win[i]);
   }
+  float wf[8 * TAPS];  // [channel][tap], contiguous in memory
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) ld8<T>(w + (long)c0 * TAPS + j * 8, wf + j * 8);
+  float bf[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (bias) ld8<T>(bias + c0, bf);
 #pragma unroll
   for (int i = 0; i < TB; ++i) {
-    if (r0 + i >= rows) return;
+    if (r0 + i >= rows) break;
+    if (!AHEAD) {
+#pragma unroll
+      for (int tap = 0; tap + 1 < TAPS; ++tap)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) win[tap][e] = win[tap + 1][e];
+      ld8<T>(xb + (long)(r0 + i) * x_stride, win[TAPS - 1]);
+      if (TB == 1 && store) {
+#pragma unroll
+        for (int tap = 1; tap < TAPS; ++tap)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            st[e * (TAPS - 1) + tap - 1] =
+                ScalarOps<T>::from_f32(win[tap][e]);
+      }
+    }
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = bf[e];
@@ -178,13 +207,14 @@ __global__ __launch_bounds__(256) void causal_conv_silu8_kernel(
     for (int tap = 0; tap < TAPS; ++tap)
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        acc[e] += win[i + tap][e] * wf[e * TAPS + tap];
+        acc[e] += win[(AHEAD ? i : 0) + tap][e] * wf[e * TAPS + tap];
     if (act) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[e] = silu_f(acc[e]);
     }
     st8<T>(out + (long)(start + r0 + i) * C + c0, acc);
   }
+  if (!AHEAD && TB > 1 && TAPS > 1 && r0 == 0) roll();
 }
 
 // grid (B, ceil(C / 256)); each thread owns one (sequence, channel) state
@@ -1354,21 +1384,27 @@ void causal_conv_silu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   // eight tokens per thread once that leaves enough workgroups
   const long work = T * (C / 8);
   const bool many = !store && work / 8 >= 512L * 256;
+  // ... one, and the state by a launch of its own, where with many taps of 32
+  // bits a thread's chain of sums takes longer than that launch (us, one /
+  // taps - 1: 120 x 4096 of 8 taps 14.0 / 17.2, of 6 10.8 / 11.9; 200 x 4096
+  // 16.7 / 17.4, 12.2 / 12.1; 400 x 4096 20.1 / 17.7, 15.7 / 12.6)
+  const bool single = !store && st == at::kFloat && taps > 5 &&
+                      T < (taps > 6 ? 384 : 160);
 #define CONV8(TT, TP)                                                        \
-  if (store) CONV8_TB(TT, TP, 1);                                            \
-  else if (many) CONV8_TB(TT, TP, 8);                                        \
-  else CONV8_TB(TT, TP, ((TP) <= 5 ? 4 : 8))
-#define CONV8_TB(TT, TP, TB)                                                 \
+  if (many) CONV8_TB(TT, TP, 8, false);                                      \
+  else if (store || single) CONV8_TB(TT, TP, 1, false);                      \
+  else CONV8_TB(TT, TP, ((TP) <= 5 ? 4 : (TP) - 1), true)
+#define CONV8_TB(TT, TP, TB, AHEAD)                                          \
   do {                                                                       \
     const long chunks = (TB) == 1 ? T : T / (TB) + B;                        \
-    hipLaunchKernelGGL((causal_conv_silu8_kernel<TT, TP, TB>),               \
+    hipLaunchKernelGGL((causal_conv_silu8_kernel<TT, TP, TB, AHEAD>),        \
                        dim3((chunks * (C / 8) + 255) / 256), dim3(256), 0,   \
                        stream, (TT *)out.data_ptr(),                         \
                        (const TT *)x.data_ptr(), (long)x.stride(0),          \
                        (const TT *)w.data_ptr(), (TT *)conv_state.data_ptr(), \
                        slots.data_ptr<long>(), has_init.data_ptr<int>(),     \
-                       query_start_loc.data_ptr<int>(), B, C, act, (int)T,   \
-                       (int)chunks, (const TT *)bp);                         \
+                       query_start_loc.data_ptr<int>(), B, C, act, store,    \
+                       (int)T, (int)chunks, (const TT *)bp);                 \
   } while (0)
 #define CONV8_T(TT)                                                          \
   switch (taps) {                                                            \
@@ -1392,7 +1428,7 @@ void causal_conv_silu(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                        slots.data_ptr<long>(), has_init.data_ptr<int>(),     \
                        query_start_loc.data_ptr<int>(), B, C, taps, act,     \
                        store, (const TT *)bp);                               \
-  if (taps > 1 && !store && !vec8)                                                    \
+  if (taps > 1 && !store && (!vec8 || single))                               \
     hipLaunchKernelGGL((conv_state_update_kernel<TT>), dim3(B, cy),          \
                        dim3(256), 0, stream, (TT *)conv_state.data_ptr(),    \
                        (const TT *)x.data_ptr(), (long)x.stride(0),          \
