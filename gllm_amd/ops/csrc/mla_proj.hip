@@ -4,7 +4,8 @@
 //   mla_prepare   one workgroup per token: the latent row is RMS-normed, its
 //                 rotated part turned, both written to their slot of the
 //                 paged cache; the queries' rotated parts turned
-//   mla_queries   the same into the attention's query rows, and beside it
+//   mla_queries   the same into the attention's query rows, and beside it (in
+//                 front of it where rows are many)
 //                 q_lat[t, h, :] = q_nope[t, h, :] W_uk[h]
 //   mla_project   out[t, h, :] = o_lat[t, h, :] W_uv[h]^T
 //
@@ -103,23 +104,25 @@ DEV_INLINE void prepare_row(
   }
 }
 
-template <typename TW>
+template <typename TW, bool PROMPT>
 __global__ __launch_bounds__(256) void mla_prepare_kernel(
-    __hip_bfloat16 *__restrict__ lat, __hip_bfloat16 *__restrict__ pe,
-    __hip_bfloat16 *__restrict__ k_cache, __hip_bfloat16 *q, long q_stride,
+    __hip_bfloat16 *__restrict__ qf, __hip_bfloat16 *__restrict__ lat,
+    __hip_bfloat16 *__restrict__ pe, __hip_bfloat16 *__restrict__ k_cache,
+    __hip_bfloat16 *q, long q_stride,
     const __hip_bfloat16 *__restrict__ kv, long kv_stride,
     const TW *__restrict__ norm_w, float eps,
     const long *__restrict__ positions, const float *__restrict__ cos_sin,
     const long *__restrict__ slots, int H) {
-  prepare_row<TW, true>(blockIdx.x, nullptr, lat, pe, k_cache, q, q_stride,
-                        kv, kv_stride, norm_w, eps, positions, cos_sin, slots,
-                        H);
+  prepare_row<TW, PROMPT>(blockIdx.x, qf, lat, pe, k_cache, q, q_stride, kv,
+                          kv_stride, norm_w, eps, positions, cos_sin, slots,
+                          H);
 }
 
 // A workgroup per 64 tokens (16 per wave), head and 128 latent columns, and
-// behind those one per token for its row. The weight block [128 k][128 columns] sits in LDS as two column blocks of
-// [128][128 B] (16 B units permuted by k & 7) and is read transposed; the
-// products are W^T q^T, so a lane holds four neighbouring columns of a token.
+// behind those (of a longer grid) one per token for its row. The weight block
+// [128 k][128 columns] sits in LDS as two column blocks of [128][128 B] (16 B
+// units permuted by k & 7) and is read transposed; the products are W^T q^T, so
+// a lane holds four neighbouring columns of a token.
 template <typename TW>
 __global__ __launch_bounds__(256) void mla_queries_kernel(
     __hip_bfloat16 *__restrict__ qf,       // [T, H, DK]
@@ -281,7 +284,14 @@ torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
               w_kvb.size(1) == LORA);
   auto qf = torch::empty({T, (long)H, (long)DK}, q.options());
   if (T == 0) return qf;
-  const long blocks = (T + TOK - 1) / TOK * H * (LORA / CHUNK) + T;
+  // The rows by a launch of their own where they are many: beside the products
+  // a row's workgroup holds LDS for the products too, and there is no longer a
+  // launch's time to save by it (us, apart / beside: 2 heads, 3000 rows 10.2 /
+  // 9.4, 4096 11.2 / 11.6, 16384 31.5 / 42.9; 16 heads, 4096 42.4 / 41.5, 8192
+  // 77.8 / 79.2, 16384 179 / 194; 32 heads, 4096 77.4 / 74.5, 8192 184 / 184).
+  const bool apart = T > (H < 8 ? 3072 : 4096);
+  const long blocks =
+      (T + TOK - 1) / TOK * H * (LORA / CHUNK) + (apart ? 0 : T);
   TORCH_CHECK(blocks < 1L << 31);
 #define ROWS(TW)                                                             \
   (__hip_bfloat16 *)k_cache.data_ptr(), (__hip_bfloat16 *)q.data_ptr(),      \
@@ -289,11 +299,18 @@ torch::Tensor mla_queries(torch::Tensor q, torch::Tensor kv,
       (long)kv.stride(0), (const TW *)norm_w.data_ptr(), (float)eps,         \
       positions.data_ptr<long>(), cos_sin.data_ptr<float>(),                 \
       slots.data_ptr<long>()
+  auto stream = at::cuda::getCurrentCUDAStream();
 #define RUN(TW)                                                              \
-  hipLaunchKernelGGL((mla_queries_kernel<TW>), dim3(blocks), dim3(256), 0,   \
-                     at::cuda::getCurrentCUDAStream(),                       \
-                     (__hip_bfloat16 *)qf.data_ptr(), ROWS(TW),              \
-                     (const __hip_bfloat16 *)w_kvb.data_ptr(), (int)T, H)
+  do {                                                                       \
+    if (apart)                                                               \
+      hipLaunchKernelGGL((mla_prepare_kernel<TW, false>), dim3(T),           \
+                         dim3(256), 0, stream,                               \
+                         (__hip_bfloat16 *)qf.data_ptr(), nullptr, nullptr,  \
+                         ROWS(TW), H);                                       \
+    hipLaunchKernelGGL((mla_queries_kernel<TW>), dim3(blocks), dim3(256), 0, \
+                       stream, (__hip_bfloat16 *)qf.data_ptr(), ROWS(TW),    \
+                       (const __hip_bfloat16 *)w_kvb.data_ptr(), (int)T, H); \
+  } while (0)
   if (norm_w.scalar_type() == at::kFloat) RUN(float);
   else RUN(__hip_bfloat16);
 #undef RUN
@@ -314,9 +331,9 @@ std::vector<torch::Tensor> mla_prompt_rows(
   auto pe = torch::empty({T, (long)ROPE}, q.options());
   if (T == 0) return {lat, pe};
 #define RUN(TW)                                                              \
-  hipLaunchKernelGGL((mla_prepare_kernel<TW>), dim3(T), dim3(256), 0,        \
+  hipLaunchKernelGGL((mla_prepare_kernel<TW, true>), dim3(T), dim3(256), 0,  \
                      at::cuda::getCurrentCUDAStream(),                       \
-                     (__hip_bfloat16 *)lat.data_ptr(),                       \
+                     nullptr, (__hip_bfloat16 *)lat.data_ptr(),              \
                      (__hip_bfloat16 *)pe.data_ptr(), ROWS(TW),              \
                      (int)(q.size(1) / QD))
   if (norm_w.scalar_type() == at::kFloat) RUN(float);
