@@ -13,6 +13,7 @@ through here. Dispatch rule:
 """
 
 import functools
+import math
 from typing import NamedTuple, Optional
 
 import torch
@@ -345,20 +346,8 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
                       topk: int, gate_up: torch.Tensor,
                       down: torch.Tensor) -> bool:
     """Whether ``fused_moe`` of gated experts runs a shared expert's products
-    beside theirs (us of experts, sum and norm, apart / beside).
-    Up to 256 rows these are a few launches that wait for weights: 64 experts
-    of 2048 x 1408, shared 2816, 1 row 53 / 45, 32 rows 203 / 194, 128 rows 214 /
-    207, 256 rows 241 / 231; 256 of 2048 x 512, shared 512, 8 rows 88 / 76, 128
-    rows 283 / 276; 64 of 7168 x 2048, shared 2048, 64 rows 897 / 887. A shared
-    expert of more than two routed ones has too long a K for a tile's chain (16
-    of 4096 x 2048, shared 8192, 32 rows 215 / 241).
-    Beyond, they fill rounds of tiles that either would leave: rows of 2048 at
-    most, where rounds are short, and weights that are worth it (2048 x 1408 as
-    above, 320 rows 260 / 240, 1000 rows 364 / 344, 3000 rows 600 / 578, 4096 rows
-    661 / 624; 16 experts, shared 5632, 3000 rows 457 / 420; but 256 of 2048 x
-    512, 512 rows 322 / 329, 64 of 7168 x 2048, 4096 rows 3363 / 3530). Blocks
-    of 256 rows: level below 1536 and above 6144 rows (1400 rows 365 / 374, 8192
-    rows 1130 / 1152)."""
+    beside theirs: where they are aligned bf16 and ``_shared_beside`` takes
+    their sizes."""
     T, K = x.shape
     inter, width = w2.shape[2], down.shape[1]
     if not (all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
@@ -372,25 +361,75 @@ def moe_shared_beside(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor,
 
 def _shared_beside(T: int, topk: int, experts: int, K: int, inter: int,
                    width: int) -> bool:
-    """The sizes of ``moe_shared_beside`` (rows, routed experts of K x inter,
-    a shared one of K x width)."""
+    """The sizes of ``moe_shared_beside``: rows, routed experts of K x inter,
+    a shared one of K x width (us of experts, sum and norm, apart / beside).
+    Up to 256 rows the products apart are a few launches that wait for
+    weights: 64 experts of 2048 x 1408, shared 2816, 1 row 53 / 45, 32 rows
+    203 / 194, 128 rows 214 / 207, 256 rows 241 / 231; 256 of 2048 x 512,
+    shared 512, 8 rows 88 / 76, 128 rows 283 / 276; 64 of 7168 x 2048, shared
+    2048, 64 rows 897 / 887. A shared expert wider than a routed one is a
+    longer chain of K in a tile of the second product than any of those beside
+    it, which they hide only while it is short (16 of 2048 x 3456, shared 5184,
+    27 rows 145 / 154; 8 of 4096 x 2368, shared 4736, 14 rows 104 / 113); in
+    blocks of 128 rows, of few experts, any chain has to be (8 of 4096 x 1856,
+    shared 1856, 79 rows 134 / 168; 4 of 2048 x 704, shared 704, 100 rows 61 /
+    47).
+    Beyond, they fill rounds of tiles that either would leave: rows of 2048 at
+    most, where rounds are short, and weights that are worth it (2048 x 1408 as
+    above, 320 rows 260 / 240, 1000 rows 364 / 344, 3000 rows 600 / 578, 4096
+    rows 661 / 624; 16 experts, shared 5632, 3000 rows 457 / 420; but 256 of
+    2048 x 512, 512 rows 322 / 329, 64 of 7168 x 2048, 4096 rows 3363 / 3530).
+    In blocks of less than 256 rows their tiles are slower than the library's
+    or tile_gemm.hip's by themselves, so they are to be few, of narrow experts
+    (32 of 2048 x 1088, shared 2176, 546 rows 176 / 146; 128 of 2048 x 1024,
+    shared 2048, 1407 rows 470 / 489; 64 of 2048 x 2304, shared 4608, 1303 rows
+    480 / 537). In blocks of 256 rows the rounds are counted: by themselves the
+    shared tiles take the part of a round that they fill, at least half of one,
+    and the routed ones whole rounds (8 of 2048 x 1856, shared 3712, 2498 rows
+    457 / 412; 8 of 2048 x 1216, shared 2432, 1653 rows 144 / 157). That holds
+    where most blocks have more than 128 rows, half of their products (32 of
+    2048 x 2368, shared 2368, 2195 rows, 137 an expert, 336 / 354), where the
+    shared products are a sixth of the routed ones or more (of 128 of 2048 x
+    2304, shared 2304, 8 a row, 3376 rows 1024 / 1070) and whole multiples of
+    theirs (4 of 2048 x 1728, shared 2560, 1566 rows 222 / 251), and from 1536
+    to 5120 rows (level beyond). Over 175 sizes of these blocks this takes 121,
+    in 0.92 of the time, three of them slower by 2 to 3 %."""
     # (what moe_gemm_tiled_shared takes of its two products)
     if max(T, 2 * width, K) >= 1 << 20 or 2 * width * K >= 1 << 30:
         return False
-    block_m = _moe_block(T * topk / experts)
+    per_expert = T * topk / experts
+    block_m = _moe_block(per_expert)
     if T <= 256:
+        short = (width <= inter and (block_m < 128 or inter <= 1024)
+                 or block_m < 128 and K <= 2048
+                 and width <= min(2 * inter, 3072))
         # (apart they are the streaming kernel's, and the second one's sums
         # over shares of K are the same beside)
-        return (width <= 2 * inter and block_m < 256 and 2 * width >= 512
+        return (short and block_m < 256 and 2 * width >= 512
                 and _use_skinny(T, 512, K) and _use_skinny(T, K, width)
                 and _gpu_kernels().stream_slice(T, K, width) > 0)
     if K > 2048 or width * K < 4 << 20:
         return False
     if block_m < 256:
-        return width <= 2 * inter
+        return (T <= 1024 and inter <= 1600 and width <= 2 * inter
+                and -(-T // block_m) * -(-width // 64) <= 384)
     # (offsets of tile_gemm.hip are 32 bits)
-    return (1536 <= T <= 6144 and 2 * inter * K < 1 << 30
-            and (T * topk + 256 * (experts + 1)) * max(inter, K) < 1 << 30)
+    if not (1536 <= T <= 5120 and per_expert >= 176
+            and width % inter == 0 and 6 * width >= topk * inter
+            and 2 * inter * K < 1 << 30
+            and (T * topk + 256 * (experts + 1)) * max(inter, K) < 1 << 30):
+        return False
+    cus = _compute_units()
+    rows, cols = -(-T // 256), -(-K // 256)
+    blocks = experts * (per_expert / 256 + 0.5)
+    up, down = rows * -(-width // 128), rows * cols
+    routed_up, routed_down = blocks * -(-inter // 128), blocks * cols
+    rounds = lambda tiles: math.ceil(tiles / cus)  # noqa: E731
+    apart = (K * (max(0.5, up / cus) + rounds(routed_up))
+             + width * max(0.5, down / cus) + inter * rounds(routed_down))
+    beside = K * rounds(up + routed_up) + max(
+        width, inter * rounds(down * width / inter + routed_down))
+    return beside < apart
 
 
 def moe_add_norm_ok(x: torch.Tensor, shared: Optional[torch.Tensor],

@@ -33,7 +33,7 @@ def operands(T, E, topk, H, I, S):
     (128, 64, 6, 2048, 1408, 2816),
     (129, 8, 2, 768, 1088, 2112),
     (256, 16, 2, 2048, 768, 1536),
-    (256, 32, 8, 4096, 320, 512)])
+    (256, 32, 8, 4096, 512, 512)])    # blocks of 128 rows
 def test_beside_is_apart(T, E, topk, H, I, S):
     from gllm_amd import ops
     x, w13, w2, weights, ids, up, down, res, norm_w = operands(

@@ -24,10 +24,12 @@ def layer(H, I, E, topk, n_shared):
 
 
 @pytest.mark.parametrize("T,beside", [
-    (5, True), (64, True), (200, True), (256, True),
-    (257, True), (500, True),      # blocks of 128 rows
+    (5, True), (64, True), (160, True),
+    (161, False), (256, False),    # blocks of 128 rows, a wider one beside
+    (257, True), (500, True),
     (700, False),                  # of 256 rows, too few of them
-    (1536, True), (2101, True)])   # of 256 rows
+    (1536, True), (1700, True),    # of 256
+    (2101, False)])                # a round more
 def test_layer(T, beside, monkeypatch):
     from gllm_amd import ops
     from gllm_amd.layers.layernorm import RMSNorm
