@@ -156,7 +156,7 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // bits, 64 to 1500 tokens, weak and strong decay: 1.1e-7 to 5.2e-7 (1.7e-7 to
 // 5.3e-7 with fp32 instructions, mean 2.5e-7 against 2.9e-7).
 //
-// 4096 tokens in four prompts of 682 to 1365, 16 heads of 128: 48 + 68 us;
+// 4096 tokens in four prompts of 682 to 1365, 16 heads of 128: 44 + 68 us;
 // with the same results, of carry's 118 us 91 were left when its operands
 // stood in runs of 1 KB (see below; local 55 -> 48), 89 with 16 columns and
 // two workgroups a CU for 32 and one (the next chunk's operands in registers
@@ -167,9 +167,12 @@ __global__ void rmsnorm_gated_kernel(__hip_bfloat16 *__restrict__ out,
 // in rows of another stride, sums of att and state in turn: no faster.)
 // local is bound by its chain of barriers and by its stores (X, att: 105 MB):
 // with 36 KB of LDS four workgroups a CU, 44 us where 73 KB and two took 52 (54
-// KB and three 46). carry is bound by the chain of a
-// chunk: products of U, split, barrier, products of the state, split, barrier,
-// 2.4 us alone and 4 us for two on a CU.
+// KB and three 46). carry is bound by what a CU takes in as much as by a
+// chunk's chain (products of U, split, barrier, products of the state, split,
+// barrier): 103 KB of operands a workgroup and chunk, the same for the eight of
+// a sequence and head, 0.87 GB in 7.6 million reads of the L2, five of six of
+// which hit. That is 49 KB a us and CU, 2.4 us a chunk alone and 4 us for two
+// workgroups on a CU.
 typedef __attribute__((ext_vector_type(4))) float gdn_f4;
 typedef __attribute__((ext_vector_type(8))) __bf16 gdn_bf8;
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
